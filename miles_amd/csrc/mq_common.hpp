@@ -116,6 +116,17 @@ __device__ __forceinline__ float recip_shared(float s) {
     const float e = __builtin_fmaf(-s, r, 1.0f);
     return __builtin_fmaf(e, r, r);
 }
+// The same for numerators of any 24-bit mantissa: one more correction step, so that the last one starts from a quotient
+// within one ulp of the true one, and then y = RN(1/s) gives the correctly rounded quotient (Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", 1990).  The residuals are exact while |w| >= 2^-102; below
+// that |w / s| < 2^-11 for every s of shared_div_ok, where the result is only within a few ulp: enough for a caller that
+// rounds it to e4m3 or e2m1, whose smallest non-zero codes start at 2^-10 and 2^-2.  Five instructions where the IEEE
+// division takes some thirteen.
+__device__ __forceinline__ float div24_by_shared(float w, float s, float y) {
+    const float q0 = w * y;
+    const float q1 = __builtin_fmaf(-__builtin_fmaf(q0, s, -w), y, q0);
+    return __builtin_fmaf(-__builtin_fmaf(q1, s, -w), y, q1);
+}
 // divisor range in which div_by_shared is used; outside it kernels fall back to operator/
 __device__ __forceinline__ bool shared_div_ok(float s) {
     uint32_t a = f2u(s) & 0x7FFFFFFFu;
@@ -234,6 +245,13 @@ __device__ __forceinline__ T* load_global_ptr(T* const* slot) {
 __device__ __forceinline__ u32x4 ld16_keep(const void* p) { return *reinterpret_cast<const u32x4*>(p); }
 __device__ __forceinline__ void st16(void* p, u32x4 v) { __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p)); }
 __device__ __forceinline__ void st8(void* p, u32x2 v) { __builtin_nontemporal_store(v, reinterpret_cast<u32x2*>(p)); }
+// The same at any element boundary (2-byte and 4-byte elements, byte-aligned stores): the target takes unaligned global
+// accesses, and the reduced alignment is part of the type, so the compiler may not assume more.  Without the non-temporal
+// hint: neighbouring workgroups share the lines at the ends of unaligned rows.
+typedef u32x4 u32x4_at2 __attribute__((aligned(2)));
+typedef u32x2 u32x2_at1 __attribute__((aligned(1)));
+__device__ __forceinline__ u32x4 ld16_at2(const void* p) { return *reinterpret_cast<const u32x4_at2*>(p); }
+__device__ __forceinline__ void st8_at1(void* p, u32x2 v) { *reinterpret_cast<u32x2_at1*>(p) = v; }
 __device__ __forceinline__ void st4(void* p, uint32_t v) { __builtin_nontemporal_store(v, reinterpret_cast<uint32_t*>(p)); }
 
 }  // namespace mq

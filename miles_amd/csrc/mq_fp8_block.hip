@@ -215,9 +215,165 @@ __global__ __launch_bounds__(kTileThreads) void fp8_block128_kernel(const Table 
     }
 }
 
+// 128x128 tiles of a matrix with unit column stride and nothing else: any row stride, any column count, rows at any element
+// boundary, fp32 as well as 16-bit.  The tile split is the fast kernel's (lane t: rows t/16 + 32 i, eight columns from
+// 8 (t%16)); loads and stores are the same 16 and 8 bytes, only unaligned.  Past the matrix's edge nothing is masked: the
+// last rows are read again, and a segment that would leave the row is moved back to end with it, so that the maximum sees
+// only the tile's own elements (a tile at least eight columns wide) and a byte that two lanes own is written twice with one
+// value.  Bound by the memory system, which takes unaligned rows at 4.9 TB/s (24 [4097, 4099] bf16 tensors, 3.3 with
+// non-temporal loads and 2.9 with non-temporal stores too) and aligned fp32 rows (LINES, non-temporal loads) at 5.8.  Twelve
+// [1545, 2563] bf16 tensors as one list: 779 us in the two-pass kernel below, one launch each; 72 us here, host included.
+template <int MODE, int DT, bool LINES>
+__global__ __launch_bounds__(kTileThreads) void fp8_block128_any_kernel(const TileTable tab) {
+    constexpr uint32_t kInfBits = DT == MQ_F32 ? 0x7F800000u : DT == MQ_F16 ? 0x7C00u : 0x7F80u;
+    constexpr uint32_t kSize = DT == MQ_F32 ? 4u : 2u;
+    constexpr int kF16 = DT == MQ_F16, kLoads = DT == MQ_F32 ? 2 : 1;
+    __shared__ uint32_t wave_amax[kTileWaves];
+    const int32_t x = blockIdx.x % kXcds, k = blockIdx.x / kXcds, run = k >> tab.chunk_shift;
+    const int32_t item = ((run * kXcds + x) << tab.chunk_shift) + (k - (run << tab.chunk_shift));
+    if (item >= tab.total) return;
+    const JobRef ref = find_job(tab, item);
+    const TileJob& job = tab.job[ref.ji];
+    const uint32_t tile = (uint32_t)(item - ref.start);
+    const uint32_t M = (uint32_t)job.M, K = (uint32_t)job.K, ldw = (uint32_t)job.ldw;
+    const uint32_t tiles_k = (K + kTile - 1) / kTile;
+    uint32_t ti = tile, tj = 0;
+    if (tiles_k > 1) {
+        ti = tile_div(tile, job.magic_k, job.shifts & 0xFFu);
+        tj = tile - ti * tiles_k;
+    }
+    const char* __restrict__ wt = (const char*)load_global_ptr(&job.w) + ((int64_t)ti * kTile * ldw + (int64_t)tj * kTile) * kSize;
+    uint8_t* __restrict__ qt = (uint8_t*)load_global_ptr(&job.q) + (int64_t)ti * kTile * K + (int64_t)tj * kTile;
+    float* __restrict__ tile_scales = load_global_ptr(&job.scale);
+    const uint32_t rows_left = M - ti * kTile, cols_left = K - tj * kTile;     // both at least 1
+
+    const uint32_t t = threadIdx.x, r0 = t >> 4, c0 = (t & 15u) * 8u;
+    const bool narrow = cols_left < 8u;                                        // uniform over the workgroup
+    const uint32_t c = narrow ? 0u : c0 + 8u <= cols_left ? c0 : cols_left - 8u;
+    u32x4 v[kRowsPerThread][kLoads];
+    if (!narrow) {
+#pragma unroll
+        for (int i = 0; i < kRowsPerThread; i++) {
+            const uint32_t r = r0 + kRowStep * i, rr = r < rows_left ? r : rows_left - 1u;
+#pragma unroll
+            for (int k = 0; k < kLoads; k++) {
+                const char* at = wt + ((rr * ldw + c) * kSize + 16u * k);
+                v[i][k] = LINES ? ld16(at) : ld16_at2(at);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < kRowsPerThread; i++) {
+            const uint32_t r = r0 + kRowStep * i, rr = r < rows_left ? r : rows_left - 1u;
+            uint32_t e[8];
+#pragma unroll
+            for (uint32_t j = 0; j < 8; j++) {
+                const char* at = wt + (rr * ldw + (j < cols_left ? j : cols_left - 1u)) * kSize;
+                e[j] = DT == MQ_F32 ? *(const uint32_t*)at : *(const uint16_t*)at;
+            }
+            if (DT == MQ_F32) {
+                v[i][0] = u32x4{e[0], e[1], e[2], e[3]};
+                v[i][kLoads - 1] = u32x4{e[4], e[5], e[6], e[7]};
+            } else {
+                v[i][0] = u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
+            }
+        }
+    }
+    // the eight elements of row segment i
+    auto element = [&](int i, int j) -> float {
+        if (DT == MQ_F32) return u2f(v[i][(j >> 2) & (kLoads - 1)][j & 3]);
+        const uint32_t pair = v[i][0][j >> 1];
+        return (j & 1) ? elem_hi<kF16>(pair) : elem_lo<kF16>(pair);
+    };
+    auto workgroup_max = [&](uint32_t m) {
+        m = wave_max(m);
+        if ((t & (kWave - 1)) == 0) wave_amax[t >> 6] = m;
+        __syncthreads();
+        m = 0;
+#pragma unroll
+        for (int k = 0; k < kTileWaves; k++) m = umax(m, wave_amax[k]);
+        return m;
+    };
+    uint32_t m = 0;
+#pragma unroll
+    for (int i = 0; i < kRowsPerThread; i++)
+#pragma unroll
+        for (int k = 0; k < kLoads; k++) {
+            const u32x4 x = v[i][k];
+            if (DT == MQ_F32)
+                m = umax(umax(umax(m, x.x & 0x7FFFFFFFu), umax(x.y & 0x7FFFFFFFu, x.z & 0x7FFFFFFFu)), x.w & 0x7FFFFFFFu);
+            else
+                m = max2_u16(max2_u16(m, max2_u16(abs2(x.x), abs2(x.y))), max2_u16(abs2(x.z), abs2(x.w)));
+        }
+    m = workgroup_max(DT == MQ_F32 ? m : hmax_u16(m));
+    const bool special = m >= kInfBits;      // an infinity or a NaN in the tile, as in the fast kernel
+    if (MODE == 1 && special) {
+        uint32_t finite = 0;
+#pragma unroll
+        for (int i = 0; i < kRowsPerThread; i++)
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const uint32_t a = f2u(element(i, j)) & 0x7FFFFFFFu;
+                finite = umax(finite, a > 0x7F800000u ? 0u : a);
+            }
+        __syncthreads();                     // every wavefront has read the first set of maxima
+        m = workgroup_max(finite);
+    }
+    const float amax = DT == MQ_F32 || (MODE == 1 && special) ? u2f(m) : elem_lo<kF16>(m);
+    float s;
+    if (MODE == 0) s = amax / kFp8Max;
+    else if (MODE == 1) s = (amax > 1e-10f ? amax : 1e-10f) / kFp8Max;
+    else s = special ? amax : ceil_pow2_scale((amax > 1e-4f ? amax : 1e-4f) / kFp8Max);
+    const float y = 1.0f / s;
+    if (t == 0) tile_scales[tile] = s;
+    const bool zero_tile = MODE == 0 && !(amax > 0.0f) && amax == amax;       // 0 / 0: the negative NaN code
+    // software arithmetic where the hardware conversion or the shared-divisor sequence do not hold: infinities, NaN,
+    // scales at the ends of the fp32 range
+    const bool plain = !special && (MODE != 0 || shared_div_ok(s));
+#pragma unroll
+    for (int i = 0; i < kRowsPerThread; i++) {
+        u32x2 o;
+        if (zero_tile) {
+            o = u32x2{0xFFFFFFFFu, 0xFFFFFFFFu};
+        } else if (plain) {
+            float f[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const float x = element(i, j);
+                f[j] = MODE != 0 ? x * y : DT == MQ_F32 ? div24_by_shared(x, s, y) : div_by_shared(x, s, y);
+            }
+            o.x = hw_e4m3x4(f[0], f[1], f[2], f[3]);       // at most 448 (1 + 2^-22): rounds to 448 by itself
+            o.y = hw_e4m3x4(f[4], f[5], f[6], f[7]);
+        } else {
+            uint32_t code[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const float x = element(i, j);
+                float p = MODE != 0 ? x * y : x / s;
+                if (MODE == 0) p = clamp_keep_nan(p, -kFp8Max, kFp8Max);                            // torch.clamp
+                else if (MODE == 1) p = __builtin_fminf(__builtin_fmaxf(p, -kFp8Max), kFp8Max);     // tl.clamp: NaN -> -448
+                code[j] = sw_e4m3fn(p);
+            }
+            o.x = code[0] | (code[1] << 8) | (code[2] << 16) | (code[3] << 24);
+            o.y = code[4] | (code[5] << 8) | (code[6] << 16) | (code[7] << 24);
+        }
+        const uint32_t r = r0 + kRowStep * i;
+        if (r >= rows_left || c0 >= cols_left) continue;
+        uint8_t* at = qt + (r * K + c);
+        if (!narrow) {
+            st8_at1(at, o);
+        } else {
+#pragma unroll
+            for (uint32_t j = 0; j < 7; j++)
+                if (j < cols_left) at[j] = (uint8_t)((j < 4 ? o.x : o.y) >> (8 * (j & 3)));
+        }
+    }
+}
+
 constexpr int kGenThreads = 256;
 // Any dtype, any strides, any block size: one workgroup per tile, two passes over the tile (the second
-// one is served by the caches).  Correctness path for shapes the fast kernel does not take.
+// one is served by the caches).  Correctness path for what the tile kernels do not take: other block sizes, column
+// strides, rows of 2^24 elements and more.
 template <int MODE>
 __global__ __launch_bounds__(kGenThreads) void fp8_block_generic_kernel(const void* __restrict__ w, int dtype,
                                                                          int64_t sxm, int64_t sxn,
@@ -557,6 +713,13 @@ bool mq_fp8_tile_fast_ok(const void* w, int dtype, int64_t sxm, int64_t sxn, con
            sxm < (1 << 24);
 }
 
+// the same tiles without the 16-byte alignment, and of fp32 matrices (fp8_block128_any_kernel)
+bool mq_fp8_tile_any_ok(const void* w, int dtype, int64_t sxm, int64_t sxn, int64_t M, int64_t K, int bm, int bk) {
+    // 127 rows of 2^24 two-byte (2^23 four-byte) elements are what a 32-bit byte offset covers
+    return dtype >= MQ_BF16 && dtype <= MQ_F32 && bm == kTile && bk == kTile && sxn == 1 && M <= 0x7FFFFFFF && K < (1 << 24) &&
+           sxm > 0 && sxm < (dtype == MQ_F32 ? 1 << 23 : 1 << 24) && ((uintptr_t)w % (dtype == MQ_F32 ? 4 : 2)) == 0;
+}
+
 // fills the division constants of a descriptor whose w, q, scale, ldw, M, K and row blocks are set; returns its tile count
 int64_t mq_fp8_tile_job_finish(TileJob& j) {
     const uint32_t tiles_k = (uint32_t)((j.K + kTile - 1) / kTile);
@@ -581,6 +744,14 @@ static void tile_launch(int mode, bool f16, dim3 grid, hipStream_t st, const Tab
     }
 }
 
+template <int DT, bool LINES>
+static void tile_any_launch(int mode, dim3 grid, hipStream_t st, const TileTable& tab) {
+    const dim3 blk(kTileThreads);
+    if (mode == 0) hipLaunchKernelGGL((fp8_block128_any_kernel<0, DT, LINES>), grid, blk, 0, st, tab);
+    else if (mode == 1) hipLaunchKernelGGL((fp8_block128_any_kernel<1, DT, LINES>), grid, blk, 0, st, tab);
+    else hipLaunchKernelGGL((fp8_block128_any_kernel<2, DT, LINES>), grid, blk, 0, st, tab);
+}
+
 // n finished descriptors in device memory, all of one 16-bit dtype; max_tiles: the largest tensor's tile count
 int mq_fp8_tile_launch_table(int mode, int dtype, const TileJob* device_jobs, int n, int64_t max_tiles, hipStream_t st) {
     if (n == 0 || max_tiles == 0) return MQ_OK;
@@ -590,9 +761,9 @@ int mq_fp8_tile_launch_table(int mode, int dtype, const TileJob* device_jobs, in
     return mq_check_launch("fp8 block quant");
 }
 
-// tab.job[i] filled by the caller (w, q, scale, ldw, M, K, row blocks), all of one 16-bit dtype; fills the division
-// constants and `end`, launches
-int mq_fp8_tile_launch_group(int mode, int dtype, TileTable& tab, hipStream_t st) {
+// tab.job[i] filled by the caller (w, q, scale, ldw, M, K, row blocks), all of one dtype; fills the division constants
+// and `end`, launches.  `aligned`: every tensor passed mq_fp8_tile_fast_ok, otherwise mq_fp8_tile_any_ok.
+int mq_fp8_tile_launch_group(int mode, int dtype, bool aligned, TileTable& tab, hipStream_t st) {
     int64_t tiles = 0;
     for (int i = 0; i < tab.n; i++) {
         tiles += mq_fp8_tile_job_finish(tab.job[i]);
@@ -601,7 +772,23 @@ int mq_fp8_tile_launch_group(int mode, int dtype, TileTable& tab, hipStream_t st
     }
     if (tiles == 0) return MQ_OK;
     seal_table(tab);
-    tile_launch(mode, dtype == MQ_F16, dim3((unsigned)xcd_grid(tiles)), st, tab);
+    if (aligned) {
+        tile_launch(mode, dtype == MQ_F16, dim3((unsigned)xcd_grid(tiles)), st, tab);
+        return mq_check_launch("fp8 block quant");
+    }
+    bool lines = dtype == MQ_F32;      // whole 128-byte lines per tile row (every segment inside its row as well: K % 8 == 0)
+    for (int i = 0; i < tab.n; i++)
+        lines &= ((uintptr_t)tab.job[i].w % 128) == 0 && tab.job[i].ldw % 32 == 0 && tab.job[i].K % 8 == 0;
+    // Neighbouring tiles of unaligned rows share lines, so the longer an XCD's runs of tiles are the better, as long as
+    // every XCD has several: 24 [4097, 4099] bf16 tensors 4.48 / 4.73 / 4.77 / 4.93 TB/s with runs of 8 / 16 / 32 / 64.
+    while (tab.chunk_shift < 6 && (tiles >> (tab.chunk_shift + 1)) >= 64) tab.chunk_shift++;
+    const int64_t gx = xcd_grid_chunked(tiles, 1ll << tab.chunk_shift);
+    if (gx >= 0x7FFFFFF0) return mq_fail(MQ_ERR_ARG, "too many tiles");
+    const dim3 grid((unsigned)gx);
+    if (dtype == MQ_BF16) tile_any_launch<MQ_BF16, false>(mode, grid, st, tab);
+    else if (dtype == MQ_F16) tile_any_launch<MQ_F16, false>(mode, grid, st, tab);
+    else if (lines) tile_any_launch<MQ_F32, true>(mode, grid, st, tab);
+    else tile_any_launch<MQ_F32, false>(mode, grid, st, tab);
     return mq_check_launch("fp8 block quant");
 }
 
@@ -611,11 +798,12 @@ static int fp8_block_launch(int mode, const void* w, int dtype, int64_t sxm, int
     if (M < 0 || K < 0 || bm <= 0 || bk <= 0) return mq_fail(MQ_ERR_ARG, "bad shape or block size");
     if (dtype < MQ_BF16 || dtype > MQ_F32) return mq_fail(MQ_ERR_ARG, "unsupported dtype");
     if (M == 0 || K == 0) return MQ_OK;
-    if (mq_fp8_tile_fast_ok(w, dtype, sxm, sxn, q, M, K, bm, bk)) {
+    const bool aligned = mq_fp8_tile_fast_ok(w, dtype, sxm, sxn, q, M, K, bm, bk);
+    if (aligned || mq_fp8_tile_any_ok(w, dtype, sxm, sxn, M, K, bm, bk)) {
         TileTable tab{};
         tab.n = 1;
         tab.job[0] = TileJob{w, q, scale, (int32_t)sxm, (int32_t)M, (int32_t)K, 0, 0, 0, 0, 0};
-        return mq_fp8_tile_launch_group(mode, dtype, tab, stream);
+        return mq_fp8_tile_launch_group(mode, dtype, aligned, tab, stream);
     }
     const int64_t tiles_m = (M + bm - 1) / bm, tiles_k = (K + bk - 1) / bk;
     const int64_t tiles = tiles_m * tiles_k;

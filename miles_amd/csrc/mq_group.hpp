@@ -78,6 +78,8 @@ struct TileTable {
     int32_t n;
     int32_t total;            // all work items of the launch
     int32_t end[kMaxGroup];   // running count of tiles: tensor i owns [end[i-1], end[i]); INT32_MAX past n
+    int32_t chunk_shift;      // kernel for any alignment: an XCD takes runs of 2^chunk_shift tiles
+    int32_t pad;
     TileJob job[kMaxGroup];
 };
 

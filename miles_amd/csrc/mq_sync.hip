@@ -19,7 +19,8 @@ using namespace mq;
 // grouped launchers implemented next to their kernels
 bool mq_fp8_tile_fast_ok(const void* w, int dtype, int64_t sxm, int64_t sxn, const void* q, int64_t M, int64_t K,
                          int bm, int bk);
-int mq_fp8_tile_launch_group(int mode, int dtype, TileTable& tab, hipStream_t st);
+bool mq_fp8_tile_any_ok(const void* w, int dtype, int64_t sxm, int64_t sxn, int64_t M, int64_t K, int bm, int bk);
+int mq_fp8_tile_launch_group(int mode, int dtype, bool aligned, TileTable& tab, hipStream_t st);
 int64_t mq_fp8_tile_job_finish(TileJob& j);
 int mq_fp8_tile_launch_table(int mode, int dtype, const TileJob* device_jobs, int n, int64_t max_tiles, hipStream_t st);
 bool mq_fp8_dequant_fast_ok(const void* x, const void* y, int64_t M, int64_t N, int block);
@@ -106,6 +107,16 @@ static bool job_fast(const mq_job& j) {
             return false;
     }
 }
+
+// FP8 tile jobs that the aligned kernel does not take still share grouped launches, of the kernel for any alignment and
+// for fp32 (row-blocked inputs are refused there)
+static bool job_tiles_any(const mq_job& j) {
+    return (j.kind == MQ_JOB_FP8_BLOCK || j.kind == MQ_JOB_FP8_BLOCKWISE_CAST || j.kind == MQ_JOB_FP8_BLOCK_POW2) &&
+           j.rows_per_block == 0 && mq_fp8_tile_any_ok(j.in, j.dtype, j.ld, 1, j.rows, j.cols, j.p0, j.p1);
+}
+// how a job runs: alone through its entry point, in grouped launches of the tuned kernels, or of the any-alignment ones
+enum JobPath { kSinglePath, kFastPath, kAnyPath };
+static JobPath job_path(const mq_job& j) { return job_fast(j) ? kFastPath : job_tiles_any(j) ? kAnyPath : kSinglePath; }
 
 static int64_t copy_dst_pitch(const mq_job& j);
 static int check_job(const mq_job& j) {
@@ -495,7 +506,8 @@ extern "C" int mq_run_jobs_tabled(const mq_job* jobs, int64_t n, const void* dev
             continue;
         }
         if (head.rows == 0 || head.cols == 0) { i++; continue; }
-        if (!job_fast(head)) {
+        const JobPath path = job_path(head);
+        if (path == kSinglePath) {
             if (head.rows_per_block != 0) return mq_fail(MQ_ERR_ARG, "row-blocked input must be 16-byte aligned, with fewer than 2^24 columns and a block stride below 2^31 elements");
             int rc = run_single(head, stream);
             if (rc) return rc;
@@ -505,7 +517,7 @@ extern "C" int mq_run_jobs_tabled(const mq_job* jobs, int64_t n, const void* dev
         // flat kinds run on a (largest tensor) x (tensors) grid: keep the padding of a group under 25 %
         const bool flat = head.kind != MQ_JOB_FP8_BLOCK && head.kind != MQ_JOB_FP8_BLOCKWISE_CAST &&
                           head.kind != MQ_JOB_FP8_BLOCK_POW2 && head.kind != MQ_JOB_COPY;
-        const bool tabled = table != nullptr && table_kind(head.kind);
+        const bool tabled = table != nullptr && table_kind(head.kind) && path == kFastPath;
         if (tabled && tile_kind(head.kind)) {
             // tile jobs of similar tile counts (an MoE layer's experts) beyond what the kernel arguments hold: one launch
             // on a (largest tile count) x (tensors) grid; mixed shapes keep the searched form below, 64 tensors at a time
@@ -531,7 +543,7 @@ extern "C" int mq_run_jobs_tabled(const mq_job* jobs, int64_t n, const void* dev
         }
         const int64_t group_cap = tabled && !tile_kind(head.kind) ? kTableGroup : kMaxGroup;
         int64_t j = i + 1, sum = head.rows * head.cols, mx = sum;
-        while (j < n && j - i < group_cap && same_group(head, jobs[j]) && job_fast(jobs[j]) && jobs[j].rows > 0 &&
+        while (j < n && j - i < group_cap && same_group(head, jobs[j]) && job_path(jobs[j]) == path && jobs[j].rows > 0 &&
                jobs[j].cols > 0) {
             const int64_t e = jobs[j].rows * jobs[j].cols;
             const int64_t nmx = e > mx ? e : mx;
@@ -558,7 +570,7 @@ extern "C" int mq_run_jobs_tabled(const mq_job* jobs, int64_t n, const void* dev
                     const mq_job& jb = jobs[i + t];
                     tab.job[t] = tile_entry(jb);
                 }
-                rc = mq_fp8_tile_launch_group(head.kind == MQ_JOB_FP8_BLOCK ? 0 : head.kind == MQ_JOB_FP8_BLOCKWISE_CAST ? 1 : 2, head.dtype, tab, st);
+                rc = mq_fp8_tile_launch_group(head.kind == MQ_JOB_FP8_BLOCK ? 0 : head.kind == MQ_JOB_FP8_BLOCKWISE_CAST ? 1 : 2, head.dtype, path == kFastPath, tab, st);
                 break;
             }
             case MQ_JOB_FP8_DEQUANT: {
