@@ -11,8 +11,8 @@ recorded (nothing has run yet: the quantizer calls only allocated their outputs 
     bucket or two of temporary outputs;
   * with `packed`, lays the bucket out as one flat transport payload instead (tensors back to back, no padding, the
     reference's `_flatten_weight_bucket` layout, protocols/broadcast.py:191-208): quantizer jobs are re-pointed at
-    their place in the payload, pass-through tensors get copy jobs, and a quantizer output whose place is not 16-byte
-    aligned keeps a buffer of its own behind the payload and is copied in;
+    their place in the payload, pass-through tensors get copy jobs, and a quantizer output whose place is not aligned for
+    its kernel (`_code_alignment`) keeps a buffer of its own behind the payload and is copied in;
   * leaves views of live parameter storage, declared constants and amax records (they carry state from one sync to
     the next) where they are.
 
@@ -45,6 +45,14 @@ class NotPackable(Exception):
 
 def _align(n: int, a: int = _SLOT_ALIGN) -> int:
     return (n + a - 1) // a * a
+
+
+def _code_alignment(kind: int) -> int:
+    """Bytes a quantizer's codes are aligned to when they are produced in place.  The packed INT4 kernels store one 32-bit
+    word per lane; the others keep to a 16-byte boundary, which covers the widest store.  (Every INT4 matrix is followed by
+    its 8-byte shape, so half of a payload's code tensors start 8 bytes off such a boundary: copied in, they cost the
+    sync of sixteen [2048, 7168] experts 175 us of device time on top of the quantizer's 263.)"""
+    return 4 if kind in (_lib.JOB_INT4_PACK, _lib.JOB_INT4_PACK_ASYM) else 16
 
 
 def _written_fields(kind: int) -> tuple[int, ...]:
@@ -291,9 +299,9 @@ class Placement:
                     jobs.add(ri)
                 continue
             hits = writers.get(old.data_ptr())
-            # codes written by a quantizer need their place on a 16-byte boundary for the tuned kernels (a row-blocked
-            # FP8 job has no other kernel at all); a place that follows, say, a 12-byte scale grid is filled by a copy
-            if hits and place % 16 and any(f == _F.OUT for _, f, _ in hits):
+            # codes written by a quantizer need their place on the tuned kernels' boundary (a row-blocked FP8 job has no
+            # other kernel at all); a place that follows, say, a 12-byte scale grid is filled by a copy
+            if hits and any(f == _F.OUT and place % _code_alignment(recorded[ri][_F.KIND]) for ri, f, _ in hits):
                 hits = None
             if hits:
                 for ri, f, s in hits:
