@@ -165,7 +165,7 @@ __global__ __launch_bounds__(256) void mxfp8_generic_kernel(const void* __restri
 using namespace mq;
 
 bool mq_mxfp8_fast_ok(const void* w, int dtype, const void* q) {
-    return ((uintptr_t)w % 16) == 0 && ((uintptr_t)q % (dtype == MQ_F32 ? 4 : 8)) == 0;
+    return dtype >= MQ_BF16 && dtype <= MQ_F32 && ((uintptr_t)w % 16) == 0 && ((uintptr_t)q % (dtype == MQ_F32 ? 4 : 8)) == 0;
 }
 
 template <class Table>
