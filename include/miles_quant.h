@@ -217,6 +217,16 @@ int mq_nvfp4_quant(const void* w, int dtype, const void* record, int n_sections,
 int mq_nvfp4_fold(void* record, int n_sections, int e4m3_max, void* stream);
 int mq_nvfp4_qdq(const void* x, int dtype, const float* amax, void* y, int64_t numel, int e4m3_max, int flags,
                  void* stream);
+/* The two passes -- amax, quantize-dequantize with it -- over a list of tensors of one dtype, in grouped launches.
+ * partial_maxima: device workspace of n * MQ_NVFP4_SECTION_WORDS 32-bit words, written before it is read.  Every tensor
+ * as for mq_nvfp4_qdq, none of them empty; x and y of one entry may not overlap any other entry's y. */
+typedef struct mq_fake_quant_item {
+    const void* x;
+    void* y;
+    int64_t numel;
+} mq_fake_quant_item;
+int mq_nvfp4_fake_quant(const mq_fake_quant_item* list, int64_t n, int dtype, void* partial_maxima, int e4m3_max, int flags,
+                        void* stream);
 
 /* Batched driver: runs a list of quantization jobs on one stream, in order, with the same results as calling
  * the single-tensor entry points one by one.  Consecutive jobs of the same kind are fused into grouped

@@ -47,6 +47,7 @@ SIGNATURES = {
     "mq_nvfp4_quant": [_vp, _i32, _vp, _i32, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _vp],
     "mq_nvfp4_fold": [_vp, _i32, _i32, _vp],
     "mq_nvfp4_qdq": [_vp, _i32, _vp, _vp, _i64, _i32, _i32, _vp],
+    "mq_nvfp4_fake_quant": [_vp, _i64, _i32, _vp, _i32, _i32, _vp],
     "mq_run_jobs": [_vp, _i64, _vp],
     "mq_tune_tile_launch_tiles": [_i64, _vp],
     "mq_job_table_fill": [_vp, _i64, _vp],

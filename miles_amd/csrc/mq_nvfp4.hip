@@ -174,26 +174,6 @@ __global__ __launch_bounds__(256) void nvfp4_fold_kernel(const Table tab, float 
 // error wins, ties go to map-to-6.  The error is an fp32 sum over the 16 elements in element order:
 //   default   | RN(RN(RN(value * f32(scale)) * amax) / (6 * e4m3_max)) - x |   (MQ_NVFP4_ERR_MSE: its square)
 //   ERR_FP16  | f32(RN_f16(f16(value) * f16(scale))) - RN(x * S_enc) |
-struct NvCandidate {
-    uint32_t sc;     // e4m3 byte
-    uint32_t word;   // this lane's eight codes
-    float s_f;       // f32(sc)
-};
-__device__ __forceinline__ NvCandidate nv_candidate(const float f[8], float s_hp, float s_dec) {
-    NvCandidate c;
-    c.sc = hw_e4m3x2<false>(__builtin_fminf(s_hp, kFp8Max), 0.0f, 0u) & 0xFFu;
-    c.s_f = hw_e4m3x2_decode<false>(c.sc).x;
-    // the refined hardware reciprocal where it equals the division, decided for the wavefront (see nvfp4_quant_units)
-    const float d = c.s_f * s_dec;
-    float inv;
-    if (__builtin_amdgcn_ballot_w64(!shared_div_ok(d)) == 0) inv = recip_shared(d);
-    else inv = __builtin_fminf(1.0f / d, kFltMax);
-    c.word = hw_e2m1x2<0>(f[0] * inv, f[1] * inv, 0u);
-    c.word = hw_e2m1x2<1>(f[2] * inv, f[3] * inv, c.word);
-    c.word = hw_e2m1x2<2>(f[4] * inv, f[5] * inv, c.word);
-    c.word = hw_e2m1x2<3>(f[6] * inv, f[7] * inv, c.word);
-    return c;
-}
 __device__ __forceinline__ void nv_decode8(uint32_t word, float q[8]) {
     const f32x2 a = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(word, 1.0f, 0), b = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(word, 1.0f, 1);
     const f32x2 c = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(word, 1.0f, 2), d = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(word, 1.0f, 3);
@@ -221,60 +201,30 @@ __device__ __forceinline__ float div_by_numer(float x, float d, float y) {
 }
 // error terms of this lane's eight elements; EM bit 0: squared error, bit 1: fp16 candidate error
 template <int EM, int FASTDIV>
-__device__ __forceinline__ void nv_error_terms(const float f[8], const NvCandidate& c, float amax, float enc, float denom, float denom_inv,
-                                               float term[8]) {
+__device__ __forceinline__ void nv_error_terms(const float f[8], uint32_t word, float s_f, float amax, float enc, float denom,
+                                               float denom_inv, float term[8]) {
     float q[8];
-    nv_decode8(c.word, q);
+    nv_decode8(word, q);
     // FASTDIV 2: every partial product of value x f32(scale) x amax is exact, one multiplication per element
-    const float scale_amax = c.s_f * amax;
+    const float scale_amax = s_f * amax;
 #pragma unroll
     for (int j = 0; j < 8; j++) {
         float diff;
         if (EM & 2) {
-            _Float16 h = (_Float16)q[j] * (_Float16)c.s_f;        // both factors exact in fp16; one fp16 rounding
+            _Float16 h = (_Float16)q[j] * (_Float16)s_f;        // both factors exact in fp16; one fp16 rounding
             float hf = (float)h;
             asm volatile("" : "+v"(hf));                          // keep the fp16 product a value of its own
             diff = hf - f[j] * enc;
         } else {
-            diff = div_by_numer<FASTDIV>(FASTDIV == 2 ? q[j] * scale_amax : (q[j] * c.s_f) * amax, denom, denom_inv) - f[j];
+            diff = div_by_numer<FASTDIV>(FASTDIV == 2 ? q[j] * scale_amax : (q[j] * s_f) * amax, denom, denom_inv) - f[j];
         }
         term[j] = (EM & 1) ? diff * diff : __builtin_fabsf(diff);
     }
 }
-// Sum of the block's sixteen terms in element order.  The even lane of the pair holds elements 0..7: its partial
-// sum from zero seeds the odd lane's accumulation, and the odd lane's total goes back to the even lane.
-__device__ __forceinline__ float nv_pair_error(const float term[8], bool odd_lane) {
-    float from_zero = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 8; j++) from_zero = from_zero + term[j];
-    float seeded = u2f(dpp_u32<kDppQuadXor1>(f2u(from_zero)));
-#pragma unroll
-    for (int j = 0; j < 8; j++) seeded = seeded + term[j];
-    const float partner_total = u2f(dpp_u32<kDppQuadXor1>(f2u(seeded)));
-    return odd_lane ? seeded : partner_total;
-}
-// the winning candidate for this lane's block; bmax is the block amax (pair-uniform)
-template <int EM, int FASTDIV>
-__device__ __forceinline__ NvCandidate nv_four_over_six(const float f[8], float bmax, float amax, const NvScales& gs,
-                                                        float denom, bool odd_lane) {
-    // bmax / 6: a bf16 numerator and a shared divisor, so the three-instruction sequence gives the IEEE quotient
-    // wherever its intermediates stay normal (decided for the wavefront; zero blocks and extreme maxima divide)
-    const bool plain_bmax = shared_div_ok(bmax);
-    const float s6_hp = (__builtin_amdgcn_ballot_w64(!plain_bmax) == 0 ? div_by_shared(bmax, 6.0f, 0x1.555556p-3f) : bmax / 6.0f) * gs.enc;
-    const float s4_hp = s6_hp * 1.5f;
-    const NvCandidate c4 = nv_candidate(f, s4_hp, gs.s_dec), c6 = nv_candidate(f, s6_hp, gs.s_dec);
-    float t4[8], t6[8];
-    const float denom_inv = 1.0f / denom;
-    nv_error_terms<EM, FASTDIV>(f, c4, amax, gs.enc, denom, denom_inv, t4);
-    nv_error_terms<EM, FASTDIV>(f, c6, amax, gs.enc, denom, denom_inv, t6);
-    const float e4 = nv_pair_error(t4, odd_lane), e6 = nv_pair_error(t6, odd_lane);
-    return e4 < e6 ? c4 : c6;
-}
-// ---- the same with one lane per block (the quantizer's form) ------------------------------------------------
-// With two lanes per block every block-level step (the two candidate scales, their reciprocals, the comparison) is
-// done twice, and the error sum, which has to run through the sixteen terms in element order, takes sixteen additions
-// in each lane of the pair.  The quantizer therefore regroups its data first: a lane ends up with the thirty-two
-// bytes of one whole block, and this kernel is bound by vector instructions, not by memory.
+// One lane works on one block.  With two lanes per block every block-level step (the two candidate scales, their
+// reciprocals, the comparison) is done twice, and the error sum, which has to run through the sixteen terms in element
+// order, takes sixteen additions in each lane of the pair.  The data is therefore regrouped first: a lane ends up with the
+// thirty-two bytes of one whole block, and the kernels are bound by vector instructions, not by memory.
 struct NvCandidate16 {
     uint32_t sc;        // e4m3 byte
     uint32_t lo, hi;    // codes of elements 0..7 and 8..15
@@ -319,12 +269,11 @@ template <int EM, int FASTDIV>
 __device__ __forceinline__ float nv_block_error(const float f[16], const NvCandidate16& c, float amax, float enc, float denom,
                                                 float denom_inv) {
     float term[8], error = 0.0f;
-    NvCandidate half{c.sc, c.lo, hw_e4m3x2_decode<false>(c.sc).x};
-    nv_error_terms<EM, FASTDIV>(f, half, amax, enc, denom, denom_inv, term);
+    const float s_f = hw_e4m3x2_decode<false>(c.sc).x;
+    nv_error_terms<EM, FASTDIV>(f, c.lo, s_f, amax, enc, denom, denom_inv, term);
 #pragma unroll
     for (int j = 0; j < 8; j++) error = error + term[j];
-    half.word = c.hi;
-    nv_error_terms<EM, FASTDIV>(f + 8, half, amax, enc, denom, denom_inv, term);
+    nv_error_terms<EM, FASTDIV>(f + 8, c.hi, s_f, amax, enc, denom, denom_inv, term);
 #pragma unroll
     for (int j = 0; j < 8; j++) error = error + term[j];
     return error;
@@ -398,10 +347,40 @@ __device__ __forceinline__ NvCandidate16 nv_four_over_six16(const float f[16], f
 // error mode of a flags word, as the EM template argument
 static inline int nv_error_mode(int flags) { return ((flags & MQ_NVFP4_ERR_MSE) ? 1 : 0) | ((flags & MQ_NVFP4_ERR_FP16) ? 2 : 0); }
 
+// The amax that a fake quantization of job.w works with: the caller's fp32 scalar (job.aux2), or the maximum of the
+// kSectionWords partial maxima an amax pass left in job.aux -- one per lane of the workgroup, so folding them here costs a
+// load and a reduction that overlap the data's loads, where a fold kernel costs a launch between the two passes.
+__device__ __forceinline__ float nv_fake_amax(const FlatJob& job, const int t) {
+    static_assert(kNvThreads == kSectionWords, "a partial maximum per lane");
+    if (job.aux2) return *(const float*)job.aux2;
+    __shared__ uint32_t part[kNvThreads / kWave];
+    const uint32_t m = wave_max(((const uint32_t*)job.aux)[t]);
+    if ((t & (kWave - 1)) == 0) part[t >> 6] = m;
+    __syncthreads();
+    return u2f(umax(umax(part[0], part[1]), umax(part[2], part[3])));
+}
+// eight values times a scale as a unit of 16-bit elements
+template <int F16>
+__device__ __forceinline__ u32x4 nv_scaled16(const float q[8], float scale) {
+    uint32_t p[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        float a = q[2 * i] * scale, b = q[2 * i + 1] * scale;
+        if (F16) {
+            asm volatile("" : "+v"(a), "+v"(b));     // keep the product apart from the conversion: a fused fma(.., +0) loses -0
+            p[i] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)a) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)b) << 16);
+        } else {
+            p[i] = hw_bf16x2(a, b);
+        }
+    }
+    return u32x4{p[0], p[1], p[2], p[3]};
+}
+
 // Four Over Six over kNvThreads * 2 units starting at `base`: loaded as the standard quantizer loads them (lane t takes
 // units t and kNvThreads + t, so a wavefront's loads are contiguous), then regrouped through LDS inside each wavefront so
 // that the even lane of a pair holds the block made of units 2p, 2p + 1 and the odd lane the block kNvThreads + 2p, + 1.
-// Returns the largest |element| of the lane's block (bf16 bits).
+// Returns the largest |element| of the lane's block (bf16 bits).  QDQ: job.q takes the dequantized values instead of the
+// codes, the amax is that of the fake quantization below, and the values go back through LDS to the lanes that loaded them.
 #ifndef MQ_NV_FOS_ROUNDS
 #define MQ_NV_FOS_ROUNDS 2
 #endif
@@ -411,8 +390,9 @@ static inline int nv_error_mode(int flags) { return ((flags & MQ_NVFP4_ERR_MSE) 
 constexpr int kFosRounds = MQ_NV_FOS_ROUNDS;
 // units a workgroup of the quantizer covers (FOS as in nvfp4_quant_units)
 constexpr int64_t nv_units_per_block(int fos) { return (int64_t)kNvThreads * kNvUnroll * (fos ? kFosRounds : 1); }
-template <int EM, int F16>
-__device__ __forceinline__ uint32_t nvfp4_fos_units(const FlatJob& job, const int64_t base, const int t, const float denom) {
+template <int EM, int F16, bool QDQ = false>
+__device__ __forceinline__ uint32_t nvfp4_fos_units(const FlatJob& job, const int64_t base, const int t, const float denom,
+                                                    const float inv_denom = 0.0f) {
     static_assert(kNvUnroll == 2, "the regrouping pairs the two units of a lane");
     constexpr uint32_t kPiece = kNvThreads * 2;
     __shared__ u32x4 stage[kPiece];
@@ -439,10 +419,16 @@ __device__ __forceinline__ uint32_t nvfp4_fos_units(const FlatJob& job, const in
             in[r][i] = ld16(w0 + (off < rem_all ? off : 0u) * 8u);
         }
     NvScales gs;
-    gs.enc_sixth = u2f(amax_bits[kRecEncSixth]);
-    gs.s_dec = u2f(amax_bits[kRecSDec]);
-    gs.enc = u2f(amax_bits[kRecEnc]);
-    const float amax = u2f(amax_bits[kRecAmax]);
+    float amax;
+    if (QDQ) {
+        amax = nv_fake_amax(job, t);
+        gs = nv_scales(amax, denom);
+    } else {
+        gs.enc_sixth = u2f(amax_bits[kRecEncSixth]);
+        gs.s_dec = u2f(amax_bits[kRecSDec]);
+        gs.enc = u2f(amax_bits[kRecEnc]);
+        amax = u2f(amax_bits[kRecAmax]);
+    }
     const int fastdiv = nv_fast_division(amax);
     // the error's divisor 6 * e4m3_max is one of two constants and the same for the whole launch: its reciprocal is
     // picked on the scalar unit
@@ -483,7 +469,25 @@ __device__ __forceinline__ uint32_t nvfp4_fos_units(const FlatJob& job, const in
         const NvCandidate16 c = fastdiv == 2   ? nv_four_over_six16<EM, 2>(f, bmax, amax, gs, denom, denom_inv, scale_table)
                                 : fastdiv == 1 ? nv_four_over_six16<EM, 1>(f, bmax, amax, gs, denom, denom_inv, scale_table)
                                                : nv_four_over_six16<EM, 0>(f, bmax, amax, gs, denom, denom_inv, scale_table);
-        if (first < rem) {      // the tensor is whole blocks: both units of a block are inside or outside
+        if (QDQ) {
+            const float final_scale = (hw_e4m3x2_decode<false>(c.sc).x * amax) * inv_denom;
+            float y[8];
+            nv_decode8(c.lo, y);
+            stage[first] = nv_scaled16<F16>(y, final_scale);
+            nv_decode8(c.hi, y);
+            stage[first + 1] = nv_scaled16<F16>(y, final_scale);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const uint32_t off = (uint32_t)t + i * kNvThreads;
+                const u32x4 o = stage[off];
+                if (off < rem) st16((uint16_t*)job.q + (base + r * kPiece + off) * 8, o);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        } else if (first < rem) {      // the tensor is whole blocks: both units of a block are inside or outside
             st8(q0 + r * kPiece + first, u32x2{c.lo, c.hi});      // `first` is even and `base` a multiple of the piece
             s80[(r * kPiece + first) >> 1] = (uint8_t)c.sc;
         }
@@ -682,82 +686,70 @@ __global__ __launch_bounds__(256) void nvfp4_quant_generic_kernel(const void* __
 
 // ---- fused quantize + dequantize (training-forward fake quantization) -------------------------------
 // Reference: miles/kernels/quant/nvfp4_qdq.py:877-890 (standard quantize), :993-1029 (dequantize), kernel :1067-1105.
-// Given the tensor amax (a device scalar): codes and block scale exactly as the quantizer above, then
+// Given the tensor amax: codes and block scale exactly as the quantizer above, then
 //   final = RN(RN(f32(s8) * amax) * f32(1 / (6 * e4m3_max)));  y = dtype(RN(e2m1_value * final))
-// Two lanes own one 1x16 block; nothing but x is read and nothing but y written.
-template <int DT, int FOS>
-__global__ __launch_bounds__(kNvThreads) void nvfp4_qdq_kernel(const uint16_t* __restrict__ x,
-                                                               const float* __restrict__ amax_ptr,
-                                                               uint16_t* __restrict__ y, int64_t total_units,
-                                                               float numer, float inv_numer, int chunk) {
+// Nothing but x (and the amax, see nv_fake_amax) is read and nothing but y written.  job: w = x, q = y, units.
+// Standard blocks: two lanes own one 1x16 block.  Four Over Six: nvfp4_fos_units.
+// Standard blocks are bound by HBM: sixteen [1536, 2048] weights in one launch 33 us (6.1 TB/s; one launch per weight 4.6 us
+// each).  Four Over Six is bound by vector instructions: four [4096, 7168] weights 77 us with a lane per block, 120 us with
+// two lanes per block and the exact error sums throughout.
+template <int FOS, int F16>
+__global__ __launch_bounds__(kNvThreads) void nvfp4_fake_kernel(const FlatTable tab, float numer, float inv_numer) {
+    const FlatJob job = flat_job(tab);
     const int t = threadIdx.x;
-    const int64_t unit = xcd_chunked_block(chunk) * kNvThreads + t;
-    const bool live = unit < total_units;
-    const u32x4 v = ld16(x + (live ? unit : total_units - 1) * 8);
-    const float amax = *amax_ptr;
-    const NvScales gs = nv_scales(amax, numer);
-    float f[8];
-    const uint32_t u[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        if (DT == MQ_BF16) { f[2 * i] = bf16_lo(u[i]); f[2 * i + 1] = bf16_hi(u[i]); }
-        else {
-            f[2 * i] = (float)__builtin_bit_cast(_Float16, (uint16_t)(u[i] & 0xFFFFu));
-            f[2 * i + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(u[i] >> 16));
-        }
-    }
-    uint32_t m = 0;
-#pragma unroll
-    for (int i = 0; i < 8; i++) m = umax(m, f2u(f[i]) & 0x7FFFFFFFu);
-    m = group_max2(m);
-    const float bmax = u2f(m);
-    const float s_hp = bmax == 0.0f ? 0.0f : bmax * gs.enc_sixth;
-    float s_f, q[8];
-    if (FOS) {
-        constexpr int EM = FOS > 0 ? FOS - 1 : 0;
-        const int fastdiv = nv_fast_division(amax);
-        const NvCandidate c = fastdiv == 2   ? nv_four_over_six<EM, 2>(f, bmax, amax, gs, numer, (t & 1) != 0)
-                              : fastdiv == 1 ? nv_four_over_six<EM, 1>(f, bmax, amax, gs, numer, (t & 1) != 0)
-                                             : nv_four_over_six<EM, 0>(f, bmax, amax, gs, numer, (t & 1) != 0);
-        s_f = c.s_f;
-        nv_decode8(c.word, q);
-    } else if (m < 0x7F800000u && s_hp == s_hp) {
-        const uint32_t sc = hw_e4m3x2<false>(__builtin_fminf(s_hp, kFp8Max), 0.0f, 0u) & 0xFFu;
-        s_f = hw_e4m3x2_decode<false>(sc).x;
-        const float inv = __builtin_fminf(1.0f / (s_f * gs.s_dec), kFltMax);
-        uint32_t word = hw_e2m1x2<0>(f[0] * inv, f[1] * inv, 0u);
-        word = hw_e2m1x2<1>(f[2] * inv, f[3] * inv, word);
-        word = hw_e2m1x2<2>(f[4] * inv, f[5] * inv, word);
-        word = hw_e2m1x2<3>(f[6] * inv, f[7] * inv, word);
-        const f32x2 a = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(word, 1.0f, 0), b = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(word, 1.0f, 1);
-        const f32x2 c = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(word, 1.0f, 2), d = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(word, 1.0f, 3);
-        q[0] = a.x; q[1] = a.y; q[2] = b.x; q[3] = b.y; q[4] = c.x; q[5] = c.y; q[6] = d.x; q[7] = d.y;
+    const int64_t base = flat_block(tab) * nv_units_per_block(FOS);
+    if (base >= job.units) return;
+    if constexpr (FOS != 0) {
+        nvfp4_fos_units<FOS - 1, F16, true>(job, base, t, numer, inv_numer);
     } else {
-        const uint32_t sc = sw_e4m3fn_sat(s_hp);
-        s_f = sw_e4m3fn_decode(sc);
-        const float inv = __builtin_fminf(1.0f / (s_f * gs.s_dec), kFltMax);
+        const int64_t left = job.units - base;
+        const uint32_t rem = left < kNvThreads * kNvUnroll ? (uint32_t)left : (uint32_t)(kNvThreads * kNvUnroll);
+        const uint16_t* __restrict__ x0 = (const uint16_t*)job.w + base * 8;
+        uint16_t* __restrict__ y0 = (uint16_t*)job.q + base * 8;
+        u32x4 v[kNvUnroll];
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const uint32_t c = sw_e2m1(f[j] * inv);
-            const float mag = (c & 7u) < 2u ? 0.5f * (float)(c & 7u) : u2f(0x3F000000u + ((c & 7u) << 22));
-            q[j] = (c & 8u) ? -mag : mag;
+        for (int i = 0; i < kNvUnroll; i++) {
+            const uint32_t off = (uint32_t)t + i * kNvThreads;
+            v[i] = ld16(x0 + (off < rem ? off : 0u) * 8u);      // a lane past the end reads the first unit again
         }
-    }
-    const float final_scale = (s_f * amax) * inv_numer;
+        const float amax = nv_fake_amax(job, t);
+        const NvScales gs = nv_scales(amax, numer);
 #pragma unroll
-    for (int j = 0; j < 8; j++) q[j] = q[j] * final_scale;
-    if (!live) return;
-    if (DT == MQ_BF16) {
-        st16(y + unit * 8, u32x4{hw_bf16x2(q[0], q[1]), hw_bf16x2(q[2], q[3]), hw_bf16x2(q[4], q[5]), hw_bf16x2(q[6], q[7])});
-    } else {
-        uint32_t p[4];
+        for (int i = 0; i < kNvUnroll; i++) {
+            const uint32_t off = (uint32_t)t + i * kNvThreads;
+            const float f[8] = {elem_lo<F16>(v[i].x), elem_hi<F16>(v[i].x), elem_lo<F16>(v[i].y), elem_hi<F16>(v[i].y),
+                                elem_lo<F16>(v[i].z), elem_hi<F16>(v[i].z), elem_lo<F16>(v[i].w), elem_hi<F16>(v[i].w)};
+            const uint32_t m2 = max2_u16(max2_u16(abs2(v[i].x), abs2(v[i].y)), max2_u16(abs2(v[i].z), abs2(v[i].w)));
+            const uint32_t mb = group_max2(hmax_u16(m2));
+            const float bmax = elem_lo<F16>(mb);
+            const float s_hp = bmax == 0.0f ? 0.0f : bmax * gs.enc_sixth;
+            float s_f, q[8];
+            if (mb < (F16 ? 0x7C00u : 0x7F80u) && s_hp == s_hp) {
+                const uint32_t sc = hw_e4m3x2<false>(__builtin_fminf(s_hp, kFp8Max), 0.0f, 0u) & 0xFFu;
+                s_f = hw_e4m3x2_decode<false>(sc).x;
+                const float d = s_f * gs.s_dec;
+                float inv;          // as in nvfp4_quant_units
+                if (__builtin_amdgcn_ballot_w64(!shared_div_ok(d)) == 0) inv = recip_shared(d);
+                else inv = __builtin_fminf(1.0f / d, kFltMax);
+                uint32_t word = hw_e2m1x2<0>(f[0] * inv, f[1] * inv, 0u);
+                word = hw_e2m1x2<1>(f[2] * inv, f[3] * inv, word);
+                word = hw_e2m1x2<2>(f[4] * inv, f[5] * inv, word);
+                word = hw_e2m1x2<3>(f[6] * inv, f[7] * inv, word);
+                nv_decode8(word, q);
+            } else {
+                const uint32_t sc = sw_e4m3fn_sat(s_hp);
+                s_f = sw_e4m3fn_decode(sc);
+                const float inv = __builtin_fminf(1.0f / (s_f * gs.s_dec), kFltMax);
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            float a = q[2 * i], b = q[2 * i + 1];
-            asm volatile("" : "+v"(a), "+v"(b));     // keep the product apart from the conversion: a fused fma(.., +0) loses -0
-            p[i] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)a) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)b) << 16);
+                for (int j = 0; j < 8; j++) {
+                    const uint32_t c = sw_e2m1(f[j] * inv);
+                    const float mag = (c & 7u) < 2u ? 0.5f * (float)(c & 7u) : u2f(0x3F000000u + ((c & 7u) << 22));
+                    q[j] = (c & 8u) ? -mag : mag;
+                }
+            }
+            const u32x4 o = nv_scaled16<F16>(q, (s_f * amax) * inv_numer);
+            if (off < rem) st16(y0 + off * 8u, o);
         }
-        st16(y + unit * 8, u32x4{p[0], p[1], p[2], p[3]});
     }
 }
 
@@ -907,6 +899,27 @@ extern "C" int mq_nvfp4_fold(void* record, int n_sections, int e4m3_max, void* s
     return mq_check_launch("nvfp4 fold");
 }
 
+template <int F16>
+static void nvfp4_fake_launch_dtype(const FlatTable& tab, int fos, float numer, float inv_numer, hipStream_t st) {
+    const dim3 grid((unsigned)tab.max_blocks, (unsigned)tab.n), blk(kNvThreads);
+    switch (fos) {
+        case 0: hipLaunchKernelGGL((nvfp4_fake_kernel<0, F16>), grid, blk, 0, st, tab, numer, inv_numer); break;
+        case 1: hipLaunchKernelGGL((nvfp4_fake_kernel<1, F16>), grid, blk, 0, st, tab, numer, inv_numer); break;
+        case 2: hipLaunchKernelGGL((nvfp4_fake_kernel<2, F16>), grid, blk, 0, st, tab, numer, inv_numer); break;
+        case 3: hipLaunchKernelGGL((nvfp4_fake_kernel<3, F16>), grid, blk, 0, st, tab, numer, inv_numer); break;
+        default: hipLaunchKernelGGL((nvfp4_fake_kernel<4, F16>), grid, blk, 0, st, tab, numer, inv_numer); break;
+    }
+}
+// tab.job[i]: w = x, q = y, units, and the amax (see nv_fake_amax)
+static int nvfp4_fake_launch(int dtype, FlatTable& tab, int e4m3_max, int flags, hipStream_t st) {
+    if (!flat_grid(tab, nv_units_per_block(flags & MQ_NVFP4_4OVER6))) return mq_fail(MQ_ERR_ARG, "tensor too large");
+    const float numer = (float)e4m3_max * 6.0f, inv_numer = (float)(1.0 / (double)(6 * e4m3_max));
+    const int fos = (flags & MQ_NVFP4_4OVER6) ? 1 + nv_error_mode(flags) : 0;
+    if (dtype == MQ_F16) nvfp4_fake_launch_dtype<1>(tab, fos, numer, inv_numer, st);
+    else nvfp4_fake_launch_dtype<0>(tab, fos, numer, inv_numer, st);
+    return mq_check_launch("nvfp4 fake quant");
+}
+
 extern "C" int mq_nvfp4_qdq(const void* x, int dtype, const float* amax, void* y, int64_t numel, int e4m3_max,
                             int flags, void* stream) {
     if (((!x || !y) && numel != 0) || !amax) return mq_fail(MQ_ERR_ARG, "null pointer");
@@ -916,28 +929,40 @@ extern "C" int mq_nvfp4_qdq(const void* x, int dtype, const float* amax, void* y
     if ((((uintptr_t)x | (uintptr_t)y) & 15) != 0) return mq_fail(MQ_ERR_ARG, "tensors must be 16-byte aligned");
     if (flags & ~(MQ_NVFP4_4OVER6 | MQ_NVFP4_ERR_MSE | MQ_NVFP4_ERR_FP16)) return mq_fail(MQ_ERR_ARG, "unknown NVFP4 flag");
     if (numel == 0) return MQ_OK;
-    const int64_t units = numel / 8;
-    int64_t blocks = (units + kNvThreads - 1) / kNvThreads;
-    const int chunk = (int)flat_chunk(blocks);
-    blocks = flat_padded(blocks, chunk);
-    if (blocks > 0x7FFFFFF0ll) return mq_fail(MQ_ERR_ARG, "tensor too large");
-    const float numer = (float)e4m3_max * 6.0f, inv_numer = (float)(1.0 / (double)(6 * e4m3_max));
-    const dim3 grid((unsigned)blocks), blk(kNvThreads);
-    hipStream_t st = (hipStream_t)stream;
-    const uint16_t* xi = (const uint16_t*)x;
-    uint16_t* yo = (uint16_t*)y;
-    const int fos = (flags & MQ_NVFP4_4OVER6) ? 1 + nv_error_mode(flags) : 0;
-#define MQ_QDQ_LAUNCH(DT, FOS) hipLaunchKernelGGL((nvfp4_qdq_kernel<DT, FOS>), grid, blk, 0, st, xi, amax, yo, units, numer, inv_numer, chunk)
-#define MQ_QDQ_SWITCH(DT)                           \
-    switch (fos) {                                  \
-        case 0: MQ_QDQ_LAUNCH(DT, 0); break;        \
-        case 1: MQ_QDQ_LAUNCH(DT, 1); break;        \
-        case 2: MQ_QDQ_LAUNCH(DT, 2); break;        \
-        case 3: MQ_QDQ_LAUNCH(DT, 3); break;        \
-        default: MQ_QDQ_LAUNCH(DT, 4); break;       \
+    FlatTable tab{};
+    tab.n = 1;
+    tab.job[0] = FlatJob{x, y, nullptr, nullptr, numel / 8, const_cast<float*>(amax), 0, 0};
+    return nvfp4_fake_launch(dtype, tab, e4m3_max, flags, (hipStream_t)stream);
+}
+
+extern "C" int mq_nvfp4_fake_quant(const mq_fake_quant_item* list, int64_t n, int dtype, void* partial_maxima, int e4m3_max,
+                                   int flags, void* stream) {
+    if (n < 0 || (n > 0 && (!list || !partial_maxima))) return mq_fail(MQ_ERR_ARG, "null pointer");
+    if (dtype != MQ_BF16 && dtype != MQ_F16) return mq_fail(MQ_ERR_ARG, "input must be bfloat16 or float16");
+    if (e4m3_max != 448 && e4m3_max != 256) return mq_fail(MQ_ERR_ARG, "e4m3_max must be 448 or 256");
+    if (flags & ~(MQ_NVFP4_4OVER6 | MQ_NVFP4_ERR_MSE | MQ_NVFP4_ERR_FP16)) return mq_fail(MQ_ERR_ARG, "unknown NVFP4 flag");
+    if (((uintptr_t)partial_maxima & 3) != 0) return mq_fail(MQ_ERR_ARG, "the partial maxima must be 4-byte aligned");
+    for (int64_t i = 0; i < n; i++) {
+        if (!list[i].x || !list[i].y || list[i].numel <= 0) return mq_fail(MQ_ERR_ARG, "empty tensor");
+        if (list[i].numel % 16 != 0) return mq_fail(MQ_ERR_ARG, "element count must be a multiple of 16");
+        if ((((uintptr_t)list[i].x | (uintptr_t)list[i].y) & 15) != 0) return mq_fail(MQ_ERR_ARG, "tensors must be 16-byte aligned");
     }
-    if (dtype == MQ_BF16) { MQ_QDQ_SWITCH(MQ_BF16) } else { MQ_QDQ_SWITCH(MQ_F16) }
-#undef MQ_QDQ_SWITCH
-#undef MQ_QDQ_LAUNCH
-    return mq_check_launch("nvfp4 qdq");
+    hipStream_t st = (hipStream_t)stream;
+    for (int64_t i = 0; i < n;) {
+        FlatTable tab{};
+        int64_t sum = 0, mx = 0;
+        for (; i < n && tab.n < kMaxGroup; i++) {
+            const int64_t e = list[i].numel, nmx = e > mx ? e : mx;
+            if (tab.n > 0 && nmx * (tab.n + 1) * 4 > (sum + e) * 5) break;       // padding of the 2-D grid under 25 %
+            sum += e;
+            mx = nmx;
+            // (the amax kernel takes the element count in `s`)
+            tab.job[tab.n++] = FlatJob{list[i].x, list[i].y, (void*)(uintptr_t)e, (uint32_t*)partial_maxima + i * kSectionWords,
+                                       e / 8, nullptr, 0, 0};
+        }
+        int rc = mq_nvfp4_amax_launch_group(dtype, tab, st);
+        if (rc == MQ_OK) rc = nvfp4_fake_launch(dtype, tab, e4m3_max, flags, st);
+        if (rc != MQ_OK) return rc;
+    }
+    return MQ_OK;
 }

@@ -10,6 +10,7 @@ second instantiation of the same kernel.
 
 from __future__ import annotations
 
+import ctypes
 import os
 from dataclasses import dataclass
 from enum import IntEnum
@@ -20,6 +21,7 @@ from miles_amd import _lib, launch
 
 _FP4_BLOCK_SIZE = 16
 
+_SECTION_WORDS = 256     # MQ_NVFP4_SECTION_WORDS: partial maxima of a tensor
 _RECORD_WORDS = 1280     # MQ_NVFP4_RECORD_WORDS; the folded amax sits in word 1024
 
 
@@ -113,15 +115,19 @@ def _validate_input(x: torch.Tensor, amax: torch.Tensor) -> None:
         raise TypeError("The per-tensor amax must contain exactly one FP32 value.")
 
 
+def _flags(config: NVFP4QDQConfig) -> int:
+    if not config.use_4over6:
+        return 0
+    return _lib.NVFP4_4OVER6 | (_lib.NVFP4_ERR_MSE if config.error_mode == NVFP4QDQErrorMode.MSE else 0) \
+        | (_lib.NVFP4_ERR_FP16 if config.error_use_fast_math else 0)
+
+
 def fused_nvfp4_qdq(x: torch.Tensor, amax: torch.Tensor, config: NVFP4QDQConfig | None = None) -> torch.Tensor:
     """Quantize to NVFP4 and dequantize again in registers; returns a detached tensor in the dtype of x."""
     if config is None:
         config = current_nvfp4_qdq_config()
     _validate_input(x, amax)
-    flags = 0
-    if config.use_4over6:
-        flags = _lib.NVFP4_4OVER6 | (_lib.NVFP4_ERR_MSE if config.error_mode == NVFP4QDQErrorMode.MSE else 0) \
-            | (_lib.NVFP4_ERR_FP16 if config.error_use_fast_math else 0)
+    flags = _flags(config)
     out = torch.empty_like(x)
     launch.note_direct_call()
     rc = _lib.load().mq_nvfp4_qdq(x.detach().data_ptr(), _lib.dtype_code(x, "fused_nvfp4_qdq"), amax.detach().data_ptr(),
@@ -130,24 +136,63 @@ def fused_nvfp4_qdq(x: torch.Tensor, amax: torch.Tensor, config: NVFP4QDQConfig 
     return out
 
 
+def _groupable(weights: list[torch.Tensor]) -> bool:
+    """Whether the list can share launches: what `_validate_input` accepts, of one dtype on one device."""
+    dtype, device = weights[0].dtype, weights[0].device
+    return (device.type == "cuda" and dtype in (torch.bfloat16, torch.float16)
+            and all(w.dtype == dtype and w.device == device and w.ndim == 2 and w.is_contiguous() and w.numel() > 0
+                    and w.shape[1] % _FP4_BLOCK_SIZE == 0 and w.data_ptr() % 16 == 0 for w in weights))
+
+
+def _images(weights: list[torch.Tensor], config: NVFP4QDQConfig) -> list[torch.Tensor]:
+    """amax and quantize-dequantize of tensors that `_groupable` accepts, in two grouped launches."""
+    with torch.no_grad():
+        outs = [torch.empty_like(w) for w in weights]
+    first = weights[0]
+    partials = torch.empty(len(weights) * _SECTION_WORDS, dtype=torch.int32, device=first.device)
+    items = []
+    for w, out in zip(weights, outs):
+        items += (w.data_ptr(), out.data_ptr(), w.numel())
+    launch.note_direct_call()
+    _lib.check(_lib.load().mq_nvfp4_fake_quant((ctypes.c_int64 * len(items))(*items), len(weights), _lib.DTYPE_CODE[first.dtype],
+                                               partials.data_ptr(), config.e4m3_max, _flags(config), _lib.stream_ptr(first.device)))
+    return outs
+
+
 class _QDQStraightThrough(torch.autograd.Function):
+    """A graph node per weight, whose image has been computed with those of its list (`images`: an iterator, so that the
+    image is this node's output and not one of its inputs)."""
+
     @staticmethod
-    def forward(ctx, x, amax, config):
-        return fused_nvfp4_qdq(x, amax, config)
+    def forward(ctx, x, images):
+        return next(images)
 
     @staticmethod
     def backward(ctx, grad_output):
-        return grad_output, None, None
+        return grad_output, None
+
+
+def fake_nvfp4_quantization_ste_list(weights: list[torch.Tensor], config: NVFP4QDQConfig) -> list[torch.Tensor] | None:
+    """`fake_nvfp4_quantization_ste` of every weight of a list that can share launches, or None if it cannot."""
+    if not weights or not _groupable(weights):
+        return None
+    images = iter(_images(weights, config))
+    outputs = [_QDQStraightThrough.apply(w, images) for w in weights]
+    for w, output in zip(weights, outputs):
+        if hasattr(w, "main_grad"):
+            output.main_grad = w.main_grad
+    return outputs
 
 
 def fake_nvfp4_quantization_ste(x: torch.Tensor, config: NVFP4QDQConfig | None = None) -> torch.Tensor:
     """NVFP4 QDQ forward, identity backward; a Megatron `main_grad` attribute follows the output."""
     if config is None:
         config = current_nvfp4_qdq_config()
-    output = _QDQStraightThrough.apply(x, compute_nvfp4_amax(x), config)
-    if hasattr(x, "main_grad"):
-        output.main_grad = x.main_grad
-    return output
+    outputs = fake_nvfp4_quantization_ste_list([x], config)
+    if outputs is None:
+        _validate_input(x, compute_nvfp4_amax(x))       # names what is wrong with x
+        raise ValueError(f"Fused NVFP4 QDQ does not support a tensor of shape {tuple(x.shape)} and type {x.dtype}.")
+    return outputs[0]
 
 
 __all__ = ["NVFP4QDQConfig", "NVFP4QDQErrorMode", "compute_nvfp4_amax", "current_nvfp4_qdq_config",

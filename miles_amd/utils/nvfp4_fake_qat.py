@@ -3,7 +3,7 @@
 Surface of the reference's miles/utils/nvfp4_fake_qat.py:10-23.  While the environment variable named by
 NVFP4_FAKE_QAT_FLAG is "1", `maybe_fake_quantize_nvfp4_weight_tensors` swaps every weight of the list it is given
 for its quantize-dequantize image (gradients pass straight through); the q-dq options are read from the environment
-once per call, not once per weight.  With any other value the caller gets its own list object back untouched.
+once per call, not once per weight, and weights of one dtype share two grouped launches.  With any other value the caller gets its own list object back untouched.
 """
 
 from __future__ import annotations
@@ -26,5 +26,8 @@ def maybe_fake_quantize_nvfp4_weight_tensors(weight_tensors: list[torch.Tensor])
         from miles_amd.kernels.quant import nvfp4_qdq as qdq
 
         options = qdq.current_nvfp4_qdq_config()
-        weight_tensors = [qdq.fake_nvfp4_quantization_ste(weight, options) for weight in weight_tensors]
+        weights = list(weight_tensors)
+        weight_tensors = qdq.fake_nvfp4_quantization_ste_list(weights, options)
+        if weight_tensors is None:      # of several kinds, or one that is refused: by itself
+            weight_tensors = [qdq.fake_nvfp4_quantization_ste(weight, options) for weight in weights]
     return weight_tensors
