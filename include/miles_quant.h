@@ -203,7 +203,8 @@ int mq_fp8_act_quant(const void* x, int dtype, void* y, void* scale, int64_t num
  *   MQ_NVFP4_ERR_FP16 uses the fp16 candidate-error form (NVTE_NVFP4_4OVER6_ERR_USE_FAST_MATH=1). */
 enum { MQ_NVFP4_4OVER6 = 1, MQ_NVFP4_ERR_MSE = 2, MQ_NVFP4_ERR_FP16 = 4,
        /* jobs of mq_run_jobs only: see the NVFP4 note there */
-       MQ_NVFP4_CARRY_AMAX = 8 };
+       MQ_NVFP4_CARRY_AMAX = 8,
+       MQ_NVFP4_NO_WAIT = 16 };
 int mq_fill_u32(void* p, uint32_t value, int64_t n, void* stream);
 int mq_nvfp4_amax(const void* w, int dtype, int64_t numel, void* record, int section, void* stream);
 int mq_nvfp4_quant(const void* w, int dtype, const void* record, int n_sections, void* q, void* block_scale,
@@ -290,7 +291,11 @@ int mq_nvfp4_fake_quant(const mq_fake_quant_item* list, int64_t n, int dtype, vo
  * (results are identical either way; a weight tensor's amax rarely moves between two syncs).  A tensor whose amax
  * changed on two submissions in a row is marked volatile in its record: on the next submission the single pass only
  * collects its amax and the second pass quantizes it (what the plain two-pass form costs), and it returns to the
- * single pass once its amax has stayed the same for one submission. */
+ * single pass once its amax has stayed the same for one submission.
+ * Without that flag, lists of 64 MB and more of bf16 or fp16 tensors with standard block scaling are read once as well when
+ * every record's tensors fit the chip's registers twice (20 MB on 256 CUs; 32 MB for one tensor at most): the workgroups
+ * of a record keep their share and wait for each other's maxima, for a bounded time, after which a second pass does
+ * what is left.  MQ_NVFP4_NO_WAIT in p1 sets that time to zero (it exists to test the second pass; results are the same). */
 enum {
     MQ_JOB_FP8_BLOCK = 0,
     MQ_JOB_FP8_BLOCKWISE_CAST = 1,

@@ -10,6 +10,7 @@
 // into the tensor's section of the amax record: plain stores, no atomics (thousands of agent-scope atomics
 // on one address serialise at ~8 ns each on this multi-XCD part) and nothing to clear.  A one-workgroup-per-
 // record fold kernel turns the partial maxima into the amax, S_enc/6, 1/S_enc and the published global scale.
+// Lists of tensors that fit the chip's registers a few at a time run in one pass instead (nvfp4_one_pass_kernel).
 // Pass 2 (mq_nvfp4_quant) reads those two factors with a scalar load; two lanes own one 16-element block
 // (16 bytes each), the block amax is one DPP step, and each lane emits four bytes of codes.  A gate/up pair
 // writes two sections of one record.
@@ -495,12 +496,50 @@ __device__ __forceinline__ uint32_t nvfp4_fos_units(const FlatJob& job, const in
     return seen;
 }
 
+// one 16-byte unit, half of a 1x16 block whose other half the neighbouring lane holds: the block's scale byte, the unit's
+// codes and the block maximum (a 16-bit pattern)
+struct NvUnitCodes {
+    uint32_t sc, word, mb;
+};
+template <int F16>
+__device__ __forceinline__ NvUnitCodes nvfp4_quant_unit(const u32x4 v, const NvScales& gs) {
+    constexpr uint32_t kInfBits = F16 ? 0x7C00u : 0x7F80u;
+    const uint32_t m2 = max2_u16(max2_u16(abs2(v.x), abs2(v.y)), max2_u16(abs2(v.z), abs2(v.w)));
+    const uint32_t mb = group_max2(hmax_u16(m2));
+    const float bmax = elem_lo<F16>(mb);
+    const float s_hp = bmax == 0.0f ? 0.0f : bmax * gs.enc_sixth;
+    const float f[8] = {elem_lo<F16>(v.x), elem_hi<F16>(v.x), elem_lo<F16>(v.y), elem_hi<F16>(v.y),
+                        elem_lo<F16>(v.z), elem_hi<F16>(v.z), elem_lo<F16>(v.w), elem_hi<F16>(v.w)};
+    uint32_t sc, word;
+    if (mb < kInfBits && s_hp == s_hp) {
+        sc = hw_e4m3x2<false>(__builtin_fminf(s_hp, kFp8Max), 0.0f, 0u) & 0xFFu;
+        const float s_f = hw_e4m3x2_decode<false>(sc).x;
+        // 1 / (block scale x global decode scale): the refined hardware reciprocal where it equals the division (every
+        // divisor in 2^-91 .. 2^90, far below FLT_MAX), decided for the wavefront; an all-zero block has divisor 0
+        const float d = s_f * gs.s_dec;
+        float inv;
+        if (__builtin_amdgcn_ballot_w64(!shared_div_ok(d)) == 0) inv = recip_shared(d);
+        else inv = __builtin_fminf(1.0f / d, kFltMax);
+        word = hw_e2m1x2<0>(f[0] * inv, f[1] * inv, 0u);
+        word = hw_e2m1x2<1>(f[2] * inv, f[3] * inv, word);
+        word = hw_e2m1x2<2>(f[4] * inv, f[5] * inv, word);
+        word = hw_e2m1x2<3>(f[6] * inv, f[7] * inv, word);
+    } else {
+        sc = sw_e4m3fn_sat(s_hp);
+        const float s_f = sw_e4m3fn_decode(sc);
+        const float inv = __builtin_fminf(1.0f / (s_f * gs.s_dec), kFltMax);
+        word = 0;
+#pragma unroll
+        for (int j = 0; j < 8; j++) word |= sw_e2m1(f[j] * inv) << (4 * j);
+    }
+    return NvUnitCodes{sc, word, mb};
+}
+
 // kNvThreads * kNvUnroll units starting at `base` of one tensor; returns the largest |element| this lane saw (bf16 bits)
 // FOS = 0: standard quantizer; FOS = 1 + error mode: Four Over Six
 template <int FOS, int F16>
 __device__ __forceinline__ uint32_t nvfp4_quant_units(const FlatJob& job, const int64_t base, const int t, const float denom) {
     if (FOS) return nvfp4_fos_units<(FOS > 0 ? FOS - 1 : 0), F16>(job, base, t, denom);
-    constexpr uint32_t kInfBits = F16 ? 0x7C00u : 0x7F80u;
     const uint16_t* __restrict__ w = (const uint16_t*)job.w;
     uint32_t* __restrict__ q = (uint32_t*)job.q;
     uint8_t* __restrict__ s8 = (uint8_t*)job.s;
@@ -522,44 +561,15 @@ __device__ __forceinline__ uint32_t nvfp4_quant_units(const FlatJob& job, const 
     gs.enc_sixth = u2f(amax_bits[kRecEncSixth]);
     gs.s_dec = u2f(amax_bits[kRecSDec]);
     gs.enc = u2f(amax_bits[kRecEnc]);
-    const float amax = u2f(amax_bits[kRecAmax]);
-    const int fastdiv = nv_fast_division(amax);
     uint32_t seen = 0;
 #pragma unroll
     for (int i = 0; i < kNvUnroll; i++) {
         const uint32_t off = (uint32_t)t + i * kNvThreads;
-        const uint32_t m2 = max2_u16(max2_u16(abs2(v[i].x), abs2(v[i].y)), max2_u16(abs2(v[i].z), abs2(v[i].w)));
-        const uint32_t mb = group_max2(hmax_u16(m2));
-        seen = umax(seen, mb);
-        const float bmax = elem_lo<F16>(mb);
-        const float s_hp = bmax == 0.0f ? 0.0f : bmax * gs.enc_sixth;
-        const float f[8] = {elem_lo<F16>(v[i].x), elem_hi<F16>(v[i].x), elem_lo<F16>(v[i].y), elem_hi<F16>(v[i].y),
-                            elem_lo<F16>(v[i].z), elem_hi<F16>(v[i].z), elem_lo<F16>(v[i].w), elem_hi<F16>(v[i].w)};
-        uint32_t sc, word;
-        if (mb < kInfBits && s_hp == s_hp) {
-            sc = hw_e4m3x2<false>(__builtin_fminf(s_hp, kFp8Max), 0.0f, 0u) & 0xFFu;
-            const float s_f = hw_e4m3x2_decode<false>(sc).x;
-            // 1 / (block scale x global decode scale): the refined hardware reciprocal where it equals the division (every
-            // divisor in 2^-91 .. 2^90, far below FLT_MAX), decided for the wavefront; an all-zero block has divisor 0
-            const float d = s_f * gs.s_dec;
-            float inv;
-            if (__builtin_amdgcn_ballot_w64(!shared_div_ok(d)) == 0) inv = recip_shared(d);
-            else inv = __builtin_fminf(1.0f / d, kFltMax);
-            word = hw_e2m1x2<0>(f[0] * inv, f[1] * inv, 0u);
-            word = hw_e2m1x2<1>(f[2] * inv, f[3] * inv, word);
-            word = hw_e2m1x2<2>(f[4] * inv, f[5] * inv, word);
-            word = hw_e2m1x2<3>(f[6] * inv, f[7] * inv, word);
-        } else {
-            sc = sw_e4m3fn_sat(s_hp);
-            const float s_f = sw_e4m3fn_decode(sc);
-            const float inv = __builtin_fminf(1.0f / (s_f * gs.s_dec), kFltMax);
-            word = 0;
-#pragma unroll
-            for (int j = 0; j < 8; j++) word |= sw_e2m1(f[j] * inv) << (4 * j);
-        }
+        const NvUnitCodes c = nvfp4_quant_unit<F16>(v[i], gs);
+        seen = umax(seen, c.mb);
         if (off < rem) {
-            st4(q0 + off, word);
-            if ((t & 1) == 0) s80[off >> 1] = (uint8_t)sc;
+            st4(q0 + off, c.word);
+            if ((t & 1) == 0) s80[off >> 1] = (uint8_t)c.sc;
         }
     }
     return seen;
@@ -618,6 +628,183 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
             atomicMax((uint32_t*)job.aux + job.section * kSectionWords + (blockIdx.x & (kSectionWords - 1)), f2u(elem_lo<F16>(m)));
         }
     }
+}
+
+// ---- one read of the tensor without an amax from before ----------------------------------------------------
+// The two-pass form reads every element twice, and at 6.8 TB/s its amax pass is 43 % of its time.  Here a workgroup keeps its
+// 64 KiB in registers (16 units per lane, 94 VGPRs, five workgroups per CU: 80 MB on the chip), publishes their maximum,
+// waits for the tensor's other workgroups and quantizes what it holds.  While one tensor waits for its last loads, the
+// workgroups of the next two are already loading.
+//   exchange: a workgroup stores its maximum (with kOneFull, so that it is never zero) into a 16-bit slot of its tensor's
+//     section; the record's first workgroup alone watches the slots and publishes the maximum of all of them in
+//     kOneWords words, each a line of its own, one of which every other workgroup watches with one request at a time.
+//     (With every workgroup watching all slots the polling itself filled the memory channels that hold them: 496 us
+//     instead of 240 on 32 x [2048, 7168].)  No counters, so no atomic read-modify-writes.
+//   every wait ends: after `polls` looks a workgroup leaves its part to the second pass (kRecRedo), the same kernel that
+//     re-quantizes tensors whose carried-over amax moved.  That happens when workgroups of one record cannot all be on
+//     the chip because something else occupies it; workgroups start in order of their ids, so otherwise the oldest
+//     unfinished tensor always gets there.
+// 32 x [2048, 7168] (940 MB of bf16, the four launches together): 312 us in two passes, 228 us this way (5.3 TB/s); the
+// same without the wait 198 us.  24 units per lane at four workgroups per CU: 239; 8 units in 512 lanes: 242.
+constexpr int kOneThreads = 256, kOneUnits = 16, kOneWavesPerSimd = 5;
+constexpr int64_t kOnePerBlock = kOneThreads * kOneUnits;
+constexpr int kOneSlots = 2 * kSectionWords;         // 16-bit slots of a section
+constexpr uint32_t kOneFull = 0x8000u;               // marks a slot or word that has been written
+constexpr int kOneWords = 7, kOneStride = 32, kRecOne = kRecAmax + 32;     // the published maximum, 128 bytes apart
+constexpr int kOneLeaderSleep = 1, kOneSleep = 12;   // between two looks, in units of 64 cycles
+
+__device__ __forceinline__ void agent_store(uint32_t* p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ void agent_store16(uint16_t* p, uint16_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ uint32_t agent_load(const uint32_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// one workgroup per tensor: no slot and no word written yet
+template <class Table>
+__global__ __launch_bounds__(256) void nvfp4_one_pass_clear_kernel(const Table tab) {
+    const FlatJob& job = tab.job[blockIdx.x];
+    uint32_t* rec = (uint32_t*)job.aux;
+    rec[job.section * kSectionWords + threadIdx.x] = 0;
+    if (job.section == 0 && threadIdx.x == 0) rec[kRecRedo] = 0;
+    if (job.section == 0 && threadIdx.x < kOneWords) rec[kRecOne + threadIdx.x * kOneStride] = 0;
+}
+
+// job as for the fold in MODE 1: section = place of the tensor inside its record, pad = tensors sharing it (neighbours)
+template <int F16, class Table>
+__global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_kernel(const Table tab, float numer, int polls) {
+    __shared__ uint32_t wave_seen[kOneThreads / 64], wave_late[kOneThreads / 64];
+    const FlatJob job = flat_job(tab);
+    const int t = threadIdx.x;
+    const int64_t block = flat_block(tab), base = block * kOnePerBlock;
+    if (base >= job.units) return;
+    const int64_t left = job.units - base;
+    const uint32_t rem = left < kOnePerBlock ? (uint32_t)left : (uint32_t)kOnePerBlock;
+    const uint16_t* __restrict__ w0 = (const uint16_t*)job.w + base * 8;
+    u32x4 v[kOneUnits];
+    const bool whole = rem == kOnePerBlock;
+    if (whole) {
+#pragma unroll
+        for (int i = 0; i < kOneUnits; i++) v[i] = ld16(w0 + i * kOneThreads * 8 + (uint32_t)t * 8u);
+    } else {
+#pragma unroll
+        for (int i = 0; i < kOneUnits; i++) {
+            const uint32_t off = (uint32_t)t + i * kOneThreads;
+            v[i] = ld16(w0 + (off < rem ? off : (off & 1u)) * 8u);      // a lane past the end reads the first block again
+        }
+    }
+    uint32_t m2 = 0;
+#pragma unroll
+    for (int i = 0; i < kOneUnits; i++)
+        m2 = max2_u16(m2, max2_u16(max2_u16(abs2(v[i].x), abs2(v[i].y)), max2_u16(abs2(v[i].z), abs2(v[i].w))));
+    uint32_t m = wave_max(hmax_u16(m2));
+    if ((t & 63) == 0) wave_seen[t >> 6] = m;
+    __syncthreads();
+    uint32_t* rec = (uint32_t*)job.aux;
+    if (t == 0) {
+        m = 0;
+#pragma unroll
+        for (int k = 0; k < kOneThreads / 64; k++) m = umax(m, wave_seen[k]);
+        agent_store16((uint16_t*)(rec + job.section * kSectionWords) + block, (uint16_t)(kOneFull | m));
+    }
+    m = 0;
+    bool late = false;
+    if (block == 0 && job.section == 0) {
+        // the record's first workgroup waits for every other one: a lane watches one word (two slots) of each section
+        for (int k = 0; k < job.pad; k++) {
+            const int64_t units = tab.job[blockIdx.y + k].units;
+            const int slots = (int)((units + kOnePerBlock - 1) / kOnePerBlock);
+            for (int word = t; word * 2 < slots; word += kOneThreads) {
+                const uint32_t need = word * 2 + 1 < slots ? 0x80008000u : 0x8000u;
+                uint32_t got = agent_load(rec + k * kSectionWords + word);
+                for (int n = 0; (got & need) != need && n < polls; n++) {
+                    __builtin_amdgcn_s_sleep(kOneLeaderSleep);
+                    got = agent_load(rec + k * kSectionWords + word);
+                }
+                late |= (got & need) != need;
+                m = umax(m, hmax_u16(abs2(got)));
+            }
+        }
+        __syncthreads();            // wave_seen has been read
+        m = wave_max(m);
+        const uint32_t any_late = __builtin_amdgcn_ballot_w64(late) != 0;
+        if ((t & 63) == 0) {
+            wave_seen[t >> 6] = m;
+            wave_late[t >> 6] = any_late;
+        }
+        __syncthreads();
+        m = 0;
+        uint32_t gave_up = 0;
+#pragma unroll
+        for (int k = 0; k < kOneThreads / 64; k++) {
+            m = umax(m, wave_seen[k]);
+            gave_up |= wave_late[k];
+        }
+        late = gave_up != 0;
+        if (t < kOneWords && !late) agent_store(rec + kRecOne + t * kOneStride, kOneFull | m);
+    } else {
+        if (t < 64) {
+            const uint32_t* word = rec + kRecOne + (blockIdx.x % kOneWords) * kOneStride;
+            uint32_t got = agent_load(word);
+            for (int n = 0; got == 0 && n < polls; n++) {
+                __builtin_amdgcn_s_sleep(kOneSleep);
+                got = agent_load(word);
+            }
+            if (t == 0) wave_late[0] = got;
+        }
+        __syncthreads();
+        m = wave_late[0];
+        late = m == 0;
+        m &= 0x7FFFu;
+    }
+    if (late) {
+        if (t == 0) rec[kRecRedo] = 1;
+        return;
+    }
+    const NvScales gs = nv_scales(elem_lo<F16>(m), numer);
+    uint32_t* __restrict__ q0 = (uint32_t*)job.q + base;
+    uint8_t* __restrict__ s80 = (uint8_t*)job.s + base / 2;
+#pragma unroll
+    for (int i = 0; i < kOneUnits; i++) {
+        const uint32_t off = (uint32_t)t + i * kOneThreads;
+        const NvUnitCodes c = nvfp4_quant_unit<F16>(v[i], gs);
+        if (whole || off < rem) {
+            st4(q0 + i * kOneThreads + (uint32_t)t, c.word);
+            if ((t & 1) == 0) (s80 + i * (kOneThreads / 2))[(uint32_t)t >> 1] = (uint8_t)c.sc;
+        }
+        __builtin_amdgcn_sched_barrier(0);      // one unit at a time: interleaved ones do not fit the registers
+    }
+}
+
+// What nvfp4_fold_kernel<1> does, from the 16-bit slots: amax, scales and published scales, slots cleared for a carried run.
+// kRecRedo stays as the workgroups left it.
+template <int F16, class Table>
+__global__ __launch_bounds__(256) void nvfp4_one_pass_finish_kernel(const Table tab, float numer, uint32_t* moved_counter, uint32_t* moved_mirror) {
+    __shared__ uint32_t lds4[4];
+    const int ji = blockIdx.x;
+    const FlatJob& job = tab.job[ji];
+    const int sections = job.pad;
+    amax_feedback_folded(moved_counter, moved_mirror, gridDim.x);
+    if (job.section != sections - 1) return;
+    uint32_t* rec = (uint32_t*)job.aux;
+    uint32_t m = 0;
+    for (int i = threadIdx.x; i < sections * kSectionWords; i += 256) {
+        m = umax(m, hmax_u16(abs2(rec[i])));
+        rec[i] = 0;
+    }
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) lds4[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    const float amax = elem_lo<F16>(umax(umax(lds4[0], lds4[1]), umax(lds4[2], lds4[3])));
+    const NvScales gs = nv_scales(amax, numer);
+    rec[kRecVolatile] = 0;
+    rec[kRecMovedRuns] = 0;
+    amax_feedback(moved_counter, rec[kRecAmax] != f2u(amax), (uint32_t)sections);
+    rec[kRecAmax] = f2u(amax);
+    rec[kRecEncSixth] = f2u(gs.enc_sixth);
+    rec[kRecSDec] = f2u(gs.s_dec);
+    rec[kRecEnc] = f2u(gs.enc);
+    const float published = nv_published_scale(amax, numer);
+    for (int k = 0; k < sections; k++)
+        if (tab.job[ji - k].aux2) *(float*)tab.job[ji - k].aux2 = published;
 }
 
 // software candidate of the one-lane-per-block kernel: codes of sixteen values and their error
@@ -842,6 +1029,56 @@ int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, in
     if (!flat_grid(ref, max_units, kNvThreads * kNvUnroll)) return mq_fail(MQ_ERR_ARG, "tensor too large");
     if (n == 0) return MQ_OK;
     return nvfp4_quant_launch(ref, n, e4m3_max, dtype == MQ_F16 ? kNvFlagF16 : 0, mode, st);
+}
+
+// Whether a chunk of NVFP4 jobs (standard scaling, packed kernels, no carried amax) takes the one-pass form.  `slots` is the
+// largest number of workgroups that share a record, `bytes` the input of the whole chunk.  All workgroups of a record
+// have to be on the chip together, and the records behind it should be loading meanwhile: half of what fits (640 workgroups,
+// 40 MB, on 256 CUs).  A pair of [2048, 7168] weights, 896 workgroups, gained less (313 -> 265 us for 16 pairs) and is one
+// busy neighbour away from waiting in vain, so it keeps two passes.  Short lists keep them as well, which then find their
+// second read in the memory-side cache and save two launches: 4 x [1537, 2064] (25 MB) 15 against 19 us, [4096, 4096]
+// (34 MB) 20 / 19, 16 x [1536, 2048] (100 MB) 39 / 34.
+constexpr int64_t kOneMinBytes = 64ll << 20;
+constexpr int kOnePolls = 256;         // looks of a waiting workgroup, 0.25 ms or more; a wait in a chunk like the above takes some 10
+bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes) {
+    int device = 0, cus = 0;
+    if (bytes < kOneMinBytes || max_units > kOneSlots * kOnePerBlock) return false;
+    if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return slots * 2 <= (int64_t)cus * kOneWavesPerSimd;       // a workgroup is one wavefront per SIMD
+}
+int64_t mq_nvfp4_one_pass_slots(int64_t units) { return (units + kOnePerBlock - 1) / kOnePerBlock; }
+
+// descriptors as for mode 1; `redo` and `one`: their grids for the second pass and for the one-pass kernel
+template <class Table, int F16>
+static int nvfp4_one_pass_launch_dtype(const Table& one, const Table& redo, int n, float numer, int polls, hipStream_t st) {
+    const dim3 folds((unsigned)n), blk(256);
+    hipLaunchKernelGGL((nvfp4_one_pass_clear_kernel<Table>), folds, blk, 0, st, one);
+    hipLaunchKernelGGL((nvfp4_one_pass_kernel<F16, Table>), dim3((unsigned)one.max_blocks, (unsigned)n), dim3(kOneThreads), 0, st, one, numer, polls);
+    hipLaunchKernelGGL((nvfp4_one_pass_finish_kernel<F16, Table>), folds, blk, 0, st, one, numer, mq_amax_feedback(), mq_amax_feedback_mirror());
+    const unsigned redo_blocks = redo.max_blocks < kSectionWords ? (unsigned)redo.max_blocks : (unsigned)kSectionWords;
+    hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<0, 2, Table, F16>), dim3(redo_blocks, (unsigned)n), dim3(kNvThreads), 0, st, redo, numer);
+    return mq_check_launch("nvfp4 quant (one pass)");
+}
+template <class Table>
+static int nvfp4_one_pass_launch(int dtype, const Table& one, const Table& redo, int n, int e4m3_max, int flags, hipStream_t st) {
+    const float numer = (float)e4m3_max * 6.0f;
+    const int polls = (flags & MQ_NVFP4_NO_WAIT) ? 0 : kOnePolls;
+    return dtype == MQ_F16 ? nvfp4_one_pass_launch_dtype<Table, 1>(one, redo, n, numer, polls, st)
+                           : nvfp4_one_pass_launch_dtype<Table, 0>(one, redo, n, numer, polls, st);
+}
+int mq_nvfp4_one_pass_launch_group(int dtype, const FlatTable& tab, int e4m3_max, int flags, hipStream_t st) {
+    FlatTable one = tab, redo = tab;
+    if (!flat_grid(one, kOnePerBlock) || !flat_grid(redo, kNvThreads * kNvUnroll)) return mq_fail(MQ_ERR_ARG, "tensor too large");
+    return nvfp4_one_pass_launch(dtype, one, redo, tab.n, e4m3_max, flags, st);
+}
+int mq_nvfp4_one_pass_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int e4m3_max, int flags,
+                                   hipStream_t st) {
+    FlatRef one{device_jobs, 0, 0}, redo{device_jobs, 0, 0};
+    if (!flat_grid(one, max_units, kOnePerBlock) || !flat_grid(redo, max_units, kNvThreads * kNvUnroll)) return mq_fail(MQ_ERR_ARG, "tensor too large");
+    return nvfp4_one_pass_launch(dtype, one, redo, n, e4m3_max, flags, st);
 }
 
 extern "C" int mq_nvfp4_amax(const void* w, int dtype, int64_t numel, void* record, int section, void* stream) {

@@ -32,6 +32,11 @@ int mq_int4_pack_launch_group(int dtype, FlatTable& tab, int group, hipStream_t 
 bool mq_nvfp4_fast_ok(const void* w, int dtype, const void* q);
 int mq_nvfp4_amax_launch_group(int dtype, FlatTable& tab, hipStream_t st);
 int mq_nvfp4_quant_launch_group(int dtype, FlatTable& tab, int e4m3_max, int flags, int mode, hipStream_t st);
+bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes);
+int64_t mq_nvfp4_one_pass_slots(int64_t units);
+int mq_nvfp4_one_pass_launch_group(int dtype, const FlatTable& tab, int e4m3_max, int flags, hipStream_t st);
+int mq_nvfp4_one_pass_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int e4m3_max, int flags,
+                                   hipStream_t st);
 bool mq_mxfp4_fast_ok(const void* w, int dtype, const void* packed, int group);
 int mq_mxfp4_launch_group(int dtype, FlatTable& tab, hipStream_t st);
 bool mq_fp8_tensor_fast_ok(const void* w, int dtype, const void* q, int64_t rows, int64_t cols, int64_t ld);
@@ -338,6 +343,9 @@ static int run_fp8_tensor(const mq_job* jobs, int64_t i, int64_t j, const FlatJo
     return MQ_OK;
 }
 
+// flags of an NVFP4 job that the driver acts on itself
+constexpr int kNvDriverFlags = MQ_NVFP4_CARRY_AMAX | MQ_NVFP4_NO_WAIT;
+
 // NVFP4 run [i, j): all jobs fast or not, processed as amax-phase then quantize-phase per chunk
 // (`table`: the device descriptors of jobs[0..), or null; n_all: length of the whole list, for the section lookup)
 static int run_nvfp4(const mq_job* jobs, int64_t n_all, int64_t i, int64_t j, const FlatJob* table, void* stream) {
@@ -392,11 +400,23 @@ static int run_nvfp4(const mq_job* jobs, int64_t n_all, int64_t i, int64_t j, co
             bool carry = true;
             for (int t = 0; t < n; t++) carry &= (jobs[i + t].p1 & MQ_NVFP4_CARRY_AMAX) != 0;
             int rc = MQ_OK;
+            int64_t max_units = 0, sum_units = 0, slots = 0, max_slots = 0;
+            bool empty = false;
+            for (int t = 0; t < n; t++) {
+                const int64_t u = jobs[i + t].rows * jobs[i + t].cols / 8;
+                empty |= u == 0;
+                max_units = u > max_units ? u : max_units;
+                sum_units += u;
+                slots = (section[t] == 0 ? 0 : slots) + mq_nvfp4_one_pass_slots(u);
+                max_slots = slots > max_slots ? slots : max_slots;
+            }
+            const bool one_pass = !carry && standard && !empty && mq_nvfp4_one_pass_ok(max_units, max_slots, sum_units * 16);
             if (from_table) {
-                int64_t max_units = 0;
-                for (int t = 0; t < n; t++) {
-                    const int64_t u = jobs[i + t].rows * jobs[i + t].cols / 8;
-                    max_units = u > max_units ? u : max_units;
+                if (one_pass) {
+                    rc = mq_nvfp4_one_pass_launch_table(jobs[i].dtype, table + i, n, max_units, jobs[i].p0, jobs[i].p1, st);
+                    if (rc) return rc;
+                    i = k;
+                    continue;
                 }
                 if (!carry) rc = mq_nvfp4_amax_launch_table(jobs[i].dtype, table + i, n, st);
                 if (rc) return rc;
@@ -407,7 +427,7 @@ static int run_nvfp4(const mq_job* jobs, int64_t n_all, int64_t i, int64_t j, co
             }
             FlatTable tab{};
             tab.n = n;
-            if (!carry) {
+            if (!carry && !one_pass) {
                 for (int t = 0; t < n; t++) {
                     const mq_job& jb = jobs[i + t];
                     const int64_t numel = jb.rows * jb.cols;
@@ -420,7 +440,8 @@ static int run_nvfp4(const mq_job* jobs, int64_t n_all, int64_t i, int64_t j, co
                 const mq_job& jb = jobs[i + t];
                 tab.job[t] = FlatJob{jb.in, jb.out, jb.scale, jb.aux, jb.rows * jb.cols / 8, jb.aux2, section[t], sections[t]};
             }
-            rc = mq_nvfp4_quant_launch_group(jobs[i].dtype, tab, jobs[i].p0, jobs[i].p1 & ~MQ_NVFP4_CARRY_AMAX, carry ? 2 : 1, st);
+            rc = one_pass ? mq_nvfp4_one_pass_launch_group(jobs[i].dtype, tab, jobs[i].p0, jobs[i].p1, st)
+                          : mq_nvfp4_quant_launch_group(jobs[i].dtype, tab, jobs[i].p0, jobs[i].p1 & ~kNvDriverFlags, carry ? 2 : 1, st);
             if (rc) return rc;
         } else {
             for (int t = 0; t < n; t++) {
@@ -431,7 +452,7 @@ static int run_nvfp4(const mq_job* jobs, int64_t n_all, int64_t i, int64_t j, co
             for (int t = 0; t < n; t++) {
                 const mq_job& jb = jobs[i + t];
                 int rc = mq_nvfp4_quant(jb.in, jb.dtype, jb.aux, sections[t], jb.out, jb.scale, (float*)jb.aux2, jb.rows,
-                                        jb.cols, jb.p0, jb.p1 & ~MQ_NVFP4_CARRY_AMAX, stream);
+                                        jb.cols, jb.p0, jb.p1 & ~kNvDriverFlags, stream);
                 if (rc) return rc;
             }
         }
