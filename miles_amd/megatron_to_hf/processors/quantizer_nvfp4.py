@@ -12,7 +12,7 @@ import re
 
 import torch
 
-from miles_amd.utils.nvfp4 import NVFP4_GROUP_SIZE, nvfp4_quantize_1d, nvfp4_quantize_1d_pair, nvfp4_quantize_stack
+from miles_amd.utils.nvfp4 import NVFP4_GROUP_SIZE, nvfp4_quantize_1d, nvfp4_quantize_1d_pair, stack_slices
 
 from ._names import in_bf16_head_or_tail, named_in_extra_high_precision, parse_layer_param
 
@@ -148,7 +148,8 @@ def quantize_nvfp4(weight: torch.Tensor):
         codes = torch.empty((n, rows, cols // 2), dtype=torch.uint8, device=weight.device)
         block_scale = torch.empty((n, rows, cols // NVFP4_GROUP_SIZE), dtype=torch.float8_e4m3fn, device=weight.device)
         global_scale = torch.empty((n,), dtype=torch.float32, device=weight.device)
-        nvfp4_quantize_stack(weight, codes, block_scale, global_scale)
+        for matrix, out in stack_slices(weight, codes, block_scale, global_scale):
+            nvfp4_quantize_1d(matrix, out=out)
         return codes, block_scale, global_scale
     if weight.dim() != 2:
         raise ValueError(f"Unsupported weight rank {weight.dim()} for NVFP4 quantization.")

@@ -69,41 +69,46 @@ def _alloc_outputs(w: torch.Tensor):
     return q, block_scale, global_scale
 
 
+class StackSlice(tuple):
+    """The outputs of one matrix of a stack, as `nvfp4_quantize_1d` takes them in `out`, with what the stack's matrices
+    share: the quantizer's options, and a slice of one allocation as the amax record.  (Made anew for every matrix they
+    took the host 300 us for thirty-two matrices, longer than the GPU needs to quantize them.)"""
+
+
+def stack_slices(stack: torch.Tensor, codes: torch.Tensor, block_scale: torch.Tensor, global_scale: torch.Tensor):
+    """(matrix, its `StackSlice`) for every matrix of [n, M, K] and stacked outputs shaped like the results, contiguous."""
+    options = _quantizer_options() if len(stack) else None
+    records = torch.empty((len(stack), AMAX_RECORD_WORDS), dtype=torch.int32, device=stack.device)
+    for w, *out, record in zip(stack.unbind(0), codes.unbind(0), block_scale.unbind(0), global_scale.unbind(0), records.unbind(0)):
+        out = StackSlice(out)
+        out.options, out.record = options, record
+        yield w, out
+
+
 def nvfp4_quantize_1d(weight: torch.Tensor, *, out=None) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """weight [M, K] -> (uint8 [M, K/2], float8_e4m3fn [M, K/16], float32 [] = weight_scale_2).
     `out` (not in the reference): three contiguous tensors of those shapes to write into, e.g. one matrix's slices
     of stacked outputs, so that a caller inside a deferred batch never has to read results before the batch runs."""
     _lib.require_gpu(weight, "nvfp4_quantize_1d")
-    e4m3_max, flags = _quantizer_options()
+    in_stack = type(out) is StackSlice
+    e4m3_max, flags = out.options if in_stack else _quantizer_options()
     w = weight.contiguous()
-    if w.shape[1] % NVFP4_GROUP_SIZE != 0:
-        raise ValueError(f"NVFP4 requires K divisible by {NVFP4_GROUP_SIZE}, got {w.shape[1]}.")
-    word = torch.empty(AMAX_RECORD_WORDS, dtype=torch.int32, device=w.device)   # written by the amax pass of the job driver
-    if out is None:
+    rows, cols = w.shape
+    if cols % NVFP4_GROUP_SIZE != 0:
+        raise ValueError(f"NVFP4 requires K divisible by {NVFP4_GROUP_SIZE}, got {cols}.")
+    # the amax record is written by the job driver
+    word = out.record if in_stack else torch.empty(AMAX_RECORD_WORDS, dtype=torch.int32, device=w.device)
+    if in_stack:
+        _lib.dtype_code(w, "nvfp4")
+    elif out is None:
         out = _alloc_outputs(w)
     else:
         _lib.dtype_code(w, "nvfp4")
         want = ((w.shape[0], w.shape[1] // 2), (w.shape[0], w.shape[1] // NVFP4_GROUP_SIZE), ())
         if any(tuple(t.shape) != shape or not t.is_contiguous() for t, shape in zip(out, want)):
             raise ValueError("nvfp4_quantize_1d: `out` tensors must be contiguous and shaped like the results")
-    launch.submit(_lib.JOB_NVFP4, w, out[0], out[1], word, out[2], w.shape[0], w.shape[1], w.shape[1], e4m3_max, flags)
+    launch.submit(_lib.JOB_NVFP4, w, out[0], out[1], word, out[2], rows, cols, cols, e4m3_max, flags)
     return out
-
-
-def nvfp4_quantize_stack(stack: torch.Tensor, codes: torch.Tensor, block_scale: torch.Tensor, global_scale: torch.Tensor) -> None:
-    """`nvfp4_quantize_1d` of every matrix of [n, M, K] into the slices of stacked outputs (contiguous, shaped like the
-    results; not in the reference).  What the matrices share -- options, checks, the amax records' memory -- is done once:
-    the calls one by one took the host 300 us for thirty-two matrices, longer than the GPU needs for them."""
-    n, rows, cols = stack.shape
-    if n == 0:
-        return
-    _lib.require_gpu(stack, "nvfp4_quantize_1d")
-    e4m3_max, flags = _quantizer_options()
-    _lib.dtype_code(stack, "nvfp4")
-    records = torch.empty((n, AMAX_RECORD_WORDS), dtype=torch.int32, device=stack.device)
-    for w, q, s, word, g in zip(stack.unbind(0), codes.unbind(0), block_scale.unbind(0), records.unbind(0), global_scale.unbind(0)):
-        w = w.contiguous()
-        launch.submit(_lib.JOB_NVFP4, w, q, s, word, g, rows, cols, cols, e4m3_max, flags)
 
 
 def nvfp4_quantize_1d_pair(first: torch.Tensor, second: torch.Tensor):
