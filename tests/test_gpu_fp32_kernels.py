@@ -81,3 +81,101 @@ def test_mxfp8_fp32_in_one_list_with_16_bit_tensors(oracle):
         for o in outs:
             for t in o:
                 t.view(torch.uint8).fill_(0x5A)
+
+
+# the largest magnitudes of a group decide how its codes are computed: near the top of the range, at the limit of the fused
+# form (2^90), and an overflowing sevenfold scale
+INT4_TOPS = [3.4028235e38, -3.4e38, 2.0**90, 2.0**90 * (1 + 2.0**-23), 1e-5, 7e-5, 2.0**-120]
+
+
+@pytest.mark.parametrize("group", [32, 64, 128])
+@pytest.mark.parametrize("shape", [(1, 128), (5, 384), (1, 2048), (3, 2176), (129, 2048), (513, 1024)])
+@pytest.mark.parametrize("specials", [False, True])
+def test_int4_pack_fp32(oracle, shape, group, specials):
+    from miles_amd.kernels.quant.int4_fake import pack_layer
+
+    w = fp32_case(shape, 20 + shape[1] + group)
+    # quotients at and next to a half: multiples of half a scale of 1 (group maximum 7), and their neighbours
+    w[0, :32] = torch.arange(-16, 16) * 0.5
+    w[0, 0] = 7.0
+    w[0, 1:32:3] = torch.nextafter(w[0, 1:32:3], torch.tensor(100.0))
+    if specials:
+        at = torch.rand(shape, generator=torch.Generator().manual_seed(shape[1])) < 0.002
+        values = torch.tensor(INT4_TOPS + [0.0, -0.0, 1e-45, float("inf"), -float("inf")])
+        w = torch.where(at, values[torch.randint(0, len(values), shape, generator=torch.Generator().manual_seed(group))], w)
+        w[-1, -group:] = 0
+    q, s, _ = pack_layer(w.to(DEV), group)
+    q_o, s_o, _ = oracle.pack_layer(w, group)
+    _assert_same(s, s_o, "scales")
+    _assert_same(q, q_o, "codes")
+
+
+@pytest.mark.parametrize("shape", FLAT_SHAPES)
+@pytest.mark.parametrize("specials", [False, True])
+def test_mxfp4_fp32(oracle, shape, specials):
+    from miles_amd.utils.mxfp4 import quantize_mxfp4
+
+    w = fp32_case(shape, 30 + shape[1], specials).nan_to_num(nan=1.0, posinf=float("inf"), neginf=-float("inf"))
+    # (the reference's scale byte for a NaN is an undefined float-to-integer conversion)
+    # every bound between two codes at a scale of 1 (group maximum 6), and its neighbours on both sides
+    bounds = torch.tensor([0.25, 0.75, 1.25, 1.75, 2.5, 3.5, 5.0])
+    row = torch.cat([bounds, torch.nextafter(bounds, torch.tensor(9.0)), torch.nextafter(bounds, torch.tensor(0.0)), -bounds])
+    w[0, :28], w[0, 28:32] = row, torch.tensor([6.0, -0.0, 0.0, -6.0])
+    q, s = quantize_mxfp4(w.to(DEV), 32)
+    q_o, s_o = oracle.quantize_mxfp4(w, 32)
+    _assert_same(s, s_o, "scales")
+    _assert_same(q, q_o, "codes")
+
+
+@pytest.mark.parametrize("shape", [(1, 16), (5, 48), (1, 2048), (3, 4112), (129, 2032), (513, 1024)])
+@pytest.mark.parametrize("mode", [None, "MAE", "MSE", "FP16"])
+def test_nvfp4_fp32(oracle, monkeypatch, shape, mode):
+    from miles_amd import _lib
+    from miles_amd.utils.nvfp4 import nvfp4_quantize_1d
+
+    e4m3_max, flags = 448, 0
+    if mode is not None:
+        monkeypatch.setenv("NVTE_NVFP4_4OVER6", "weights")
+        monkeypatch.setenv("NVTE_NVFP4_4OVER6_ERR_MODE", "MSE" if mode == "MSE" else "MAE")
+        monkeypatch.setenv("NVTE_NVFP4_4OVER6_ERR_USE_FAST_MATH", "1" if mode == "FP16" else "0")
+        e4m3_max = 256
+        flags = _lib.NVFP4_4OVER6 | (_lib.NVFP4_ERR_MSE if mode == "MSE" else 0) | (_lib.NVFP4_ERR_FP16 if mode == "FP16" else 0)
+    for case in range(3):
+        w = fp32_case(shape, 40 + shape[1] + case) * torch.logspace(0, -2, shape[1])
+        if case == 1:
+            w[:, : shape[1] // 16 // 2 * 16] = 0          # blocks of zeros
+        if case == 2:
+            w = torch.full(shape, 3e38) * torch.sign(w)   # an amax outside the range of the fast divisions
+        q, s, g = nvfp4_quantize_1d(w.to(DEV))
+        q_o, s_o, g_o = oracle.nvfp4_quantize_1d(w, e4m3_max=e4m3_max, flags=flags)
+        _assert_same(g.reshape(1), torch.as_tensor(g_o).reshape(1).float(), "global scale")
+        _assert_same(s, s_o, "scales")
+        _assert_same(q, q_o, "codes")
+
+
+@pytest.mark.parametrize("kind", ["int4", "mxfp4", "nvfp4"])
+def test_fp32_in_one_list_with_16_bit_tensors(oracle, kind):
+    """A recorded list of seventy-odd tensors (more than the kernel arguments of a launch hold), run twice."""
+    from miles_amd import launch
+    from miles_amd.kernels.quant.int4_fake import pack_layer
+    from miles_amd.utils.mxfp4 import quantize_mxfp4
+    from miles_amd.utils.nvfp4 import nvfp4_quantize_1d
+
+    here, there = {"int4": (lambda t: pack_layer(t, 32)[:2], lambda t: oracle.pack_layer(t, 32)[:2]),
+                   "mxfp4": (lambda t: quantize_mxfp4(t, 32), lambda t: oracle.quantize_mxfp4(t, 32)),
+                   "nvfp4": (lambda t: nvfp4_quantize_1d(t)[:2], lambda t: oracle.nvfp4_quantize_1d(t)[:2])}[kind]
+    tensors = [fp32_case((33, 160), 60 + i) for i in range(72)]
+    tensors[5], tensors[6] = tensors[5].bfloat16(), tensors[6].half()
+    dev = [t.to(DEV) for t in tensors]
+    with launch.recording() as batch:
+        outs = [here(t) for t in dev]
+    batch.freeze()
+    for rep in range(2):
+        batch.run()
+        torch.cuda.synchronize()
+        for i, t in enumerate(tensors):
+            for got, want, what in zip(outs[i], there(t), ("codes", "scales")):
+                _assert_same(got, want, f"tensor {i} ({t.dtype}) {what}, run {rep}")
+        for o in outs:
+            for t in o:
+                t.view(torch.uint8).fill_(0x5A)
