@@ -280,8 +280,8 @@ int mq_nvfp4_fake_quant(const mq_fake_quant_item* list, int64_t n, int dtype, vo
  * ld is the input row stride in elements for the two FP8 quantizers (column stride 1) and ignored elsewhere;
  * rows_per_block / block_stride describe a row-blocked input (see the struct).
  * The three FP8 tile kinds (FP8_BLOCK, FP8_BLOCKWISE_CAST, FP8_BLOCK_POW2), MXFP8, MXFP4, INT4_PACK, INT4_PACK_ASYM, FP8_TENSOR and NVFP4 run their tuned
- * kernels on bf16 and on fp16 inputs; consecutive jobs share a launch when they also share the input dtype (NVFP4 jobs
- * that share an amax record must have one dtype to take them).
+ * kernels on bf16 and on fp16 inputs, and all but INT4_PACK_ASYM and FP8_TENSOR on fp32 ones as well; consecutive jobs share a
+ * launch when they also share the input dtype (NVFP4 jobs that share an amax record must have one dtype to take them).
  * NVFP4: the driver reduces every job's tensor into a section of its record and then quantizes; jobs that
  * share one record (a gate/up pair; at most MQ_NVFP4_SECTIONS) must be adjacent in the list.
  * MQ_NVFP4_CARRY_AMAX in p1 of NVFP4 and FP8_TENSOR jobs (no counterpart in the reference): a caller that submits the

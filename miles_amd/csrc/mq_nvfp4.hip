@@ -72,6 +72,35 @@ __global__ __launch_bounds__(256) void nvfp4_amax_bf16_kernel(const Table tab) {
     if (t == 0) section[blockIdx.x] = f2u(elem_lo<F16>(umax(umax(wave_amax[0], wave_amax[1]), umax(wave_amax[2], wave_amax[3]))));
 }
 
+// fp32 input (units and the element count as above): 16-byte loads of four elements
+template <class Table>
+__global__ __launch_bounds__(256) void nvfp4_amax_f32_kernel(const Table tab) {
+    __shared__ uint32_t wave_amax[4];
+    const FlatJob job = flat_job(tab);
+    const float* __restrict__ w = (const float*)job.w;
+    const int64_t loads = job.units * 2, numel = std::is_same<Table, FlatRef>::value ? job.units * 8 : (int64_t)(uintptr_t)job.s;
+    const int t = threadIdx.x;
+    uint32_t m = 0;
+    for (int64_t base = (int64_t)blockIdx.x * (256 * kAmaxUnroll); base < loads; base += (int64_t)kSectionWords * 256 * kAmaxUnroll) {
+        u32x4 v[kAmaxUnroll];
+#pragma unroll
+        for (int i = 0; i < kAmaxUnroll; i++) {
+            const int64_t at = base + i * 256 + t;
+            v[i] = at < loads ? ld16(w + at * 4) : u32x4{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (int i = 0; i < kAmaxUnroll; i++)
+            m = umax(m, umax(umax(v[i].x & 0x7FFFFFFFu, v[i].y & 0x7FFFFFFFu), umax(v[i].z & 0x7FFFFFFFu, v[i].w & 0x7FFFFFFFu)));
+    }
+    if (blockIdx.x == 0 && t == 0)
+        for (int64_t i = loads * 4; i < numel; i++) m = umax(m, f2u(w[i]) & 0x7FFFFFFFu);
+    m = wave_max(m);
+    if ((t & 63) == 0) wave_amax[t >> 6] = m;
+    __syncthreads();
+    if (t == 0)
+        ((uint32_t*)job.aux + job.section * kSectionWords)[blockIdx.x] = umax(umax(wave_amax[0], wave_amax[1]), umax(wave_amax[2], wave_amax[3]));
+}
+
 __global__ __launch_bounds__(256) void nvfp4_amax_generic_kernel(const void* __restrict__ w, int dtype, int64_t numel,
                                                                  uint32_t* __restrict__ section) {
     __shared__ uint32_t wave_amax[4];
@@ -312,11 +341,12 @@ __device__ __forceinline__ float nv_block_error_estimate(const float f[16], cons
     }
     return sum;
 }
-template <int EM, int FASTDIV>
+template <int EM, int FASTDIV, bool F32 = false>
 __device__ __forceinline__ NvCandidate16 nv_four_over_six16(const float f[16], float bmax, float amax, const NvScales& gs,
                                                             float denom, float denom_inv, const NvScaleEntry* table) {
     const bool plain_bmax = shared_div_ok(bmax);
-    const float s6_hp = (__builtin_amdgcn_ballot_w64(!plain_bmax) == 0 ? div_by_shared(bmax, 6.0f, 0x1.555556p-3f) : bmax / 6.0f) * gs.enc;
+    // (an fp32 block's maximum has more bits than the shared-divisor sequence takes)
+    const float s6_hp = (!F32 && __builtin_amdgcn_ballot_w64(!plain_bmax) == 0 ? div_by_shared(bmax, 6.0f, 0x1.555556p-3f) : bmax / 6.0f) * gs.enc;
     const float s4_hp = s6_hp * 1.5f;
     const NvCandidate16 c4 = nv_candidate16(f, s4_hp, table), c6 = nv_candidate16(f, s6_hp, table);
     if ((EM == 0 || EM == 1) && FASTDIV == 2) {
@@ -807,6 +837,92 @@ __global__ __launch_bounds__(256) void nvfp4_one_pass_finish_kernel(const Table 
         if (tab.job[ji - k].aux2) *(float*)tab.job[ji - k].aux2 = published;
 }
 
+// fp32 input, the second pass of the two-pass form (the carried-over amax and the one-pass form are for 16-bit tensors).
+// Standard blocks: four elements per 16-byte load, four lanes a block, two bytes of codes per lane; bound by HBM, 8.56
+// bytes per element with the amax pass.  Four Over Six: a lane per block, 64 consecutive bytes each, and the exact error sums
+// (the estimate wants an amax of twelve significant bits); bound by vector instructions.
+// A stack of eight [2048, 4096] tensors: 92 us, Four Over Six 95 (769 and 762 in the element-wise kernels, a launch each).
+constexpr int kNvF32Loads = 2;                     // 16-byte loads per lane, standard blocks
+// 8-element units a workgroup covers
+constexpr int64_t nv_f32_units_per_block(int fos) { return fos ? kNvThreads * 2 : kNvThreads * kNvF32Loads / 2; }
+template <int FOS, class Table>
+__global__ __launch_bounds__(kNvThreads) void nvfp4_quant_f32_kernel(const Table tab, float denom) {
+    const FlatJob job = flat_job(tab);
+    const uint32_t t = threadIdx.x;
+    const int64_t first = flat_block(tab) * nv_f32_units_per_block(FOS);       // in 8-element units
+    if (first >= job.units) return;
+    const uint32_t* __restrict__ amax_bits = (const uint32_t*)job.aux;
+    NvScales gs;
+    gs.enc_sixth = u2f(amax_bits[kRecEncSixth]);
+    gs.s_dec = u2f(amax_bits[kRecSDec]);
+    gs.enc = u2f(amax_bits[kRecEnc]);
+    const float amax = u2f(amax_bits[kRecAmax]);
+    const float* __restrict__ w0 = (const float*)job.w + first * 8;
+    const int64_t left = (job.units - first) * 2;                              // 16-byte loads
+    if constexpr (FOS != 0) {
+        __shared__ NvScaleEntry scale_table[128];
+        constexpr int EM = FOS - 1;
+        const uint32_t rem = left < 4 * kNvThreads ? (uint32_t)left / 4 : (uint32_t)kNvThreads;      // blocks
+        const uint32_t at = t < rem ? t : 0u;
+        float f[16];
+        uint32_t mb = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const u32x4 v = ld16_keep(w0 + at * 16u + 4 * i);      // (each line is touched by four load instructions)
+            mb = umax(mb, umax(umax(v.x & 0x7FFFFFFFu, v.y & 0x7FFFFFFFu), umax(v.z & 0x7FFFFFFFu, v.w & 0x7FFFFFFFu)));
+            f[4 * i] = u2f(v.x); f[4 * i + 1] = u2f(v.y); f[4 * i + 2] = u2f(v.z); f[4 * i + 3] = u2f(v.w);
+        }
+        const float denom_inv = 1.0f / denom;
+        nv_fill_scale_table(scale_table, (int)t, amax, gs.s_dec, false, denom, denom_inv);
+        __syncthreads();
+        const NvCandidate16 c = nv_fast_division(amax) != 0 ? nv_four_over_six16<EM, 1, true>(f, u2f(mb), amax, gs, denom, denom_inv, scale_table)
+                                                            : nv_four_over_six16<EM, 0, true>(f, u2f(mb), amax, gs, denom, denom_inv, scale_table);
+        if (t < rem) {
+            ((uint32_t*)job.q + first)[2 * t] = c.lo;
+            ((uint32_t*)job.q + first)[2 * t + 1] = c.hi;
+            ((uint8_t*)job.s + first / 2)[t] = (uint8_t)c.sc;
+        }
+    } else {
+        constexpr uint32_t kPerBlock = kNvThreads * kNvF32Loads;
+        const uint32_t rem = left < kPerBlock ? (uint32_t)left : kPerBlock;
+        uint16_t* __restrict__ q0 = (uint16_t*)job.q + first * 2;
+        uint8_t* __restrict__ s80 = (uint8_t*)job.s + first / 2;
+        u32x4 v[kNvF32Loads];
+#pragma unroll
+        for (int i = 0; i < kNvF32Loads; i++) {
+            const uint32_t off = t + i * kNvThreads;
+            v[i] = off < rem ? ld16(w0 + off * 4u) : u32x4{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (int i = 0; i < kNvF32Loads; i++) {
+            const uint32_t off = t + i * kNvThreads;
+            const uint32_t mb = group_max4(umax(umax(v[i].x & 0x7FFFFFFFu, v[i].y & 0x7FFFFFFFu), umax(v[i].z & 0x7FFFFFFFu, v[i].w & 0x7FFFFFFFu)));
+            const float bmax = u2f(mb);
+            const float s_hp = bmax == 0.0f ? 0.0f : bmax * gs.enc_sixth;
+            const float f[4] = {u2f(v[i].x), u2f(v[i].y), u2f(v[i].z), u2f(v[i].w)};
+            uint32_t sc, word = 0;
+            if (mb < 0x7F800000u && s_hp == s_hp) {
+                sc = hw_e4m3x2<false>(__builtin_fminf(s_hp, kFp8Max), 0.0f, 0u) & 0xFFu;
+                const float d = hw_e4m3x2_decode<false>(sc).x * gs.s_dec;
+                float inv;          // as in nvfp4_quant_unit
+                if (__builtin_amdgcn_ballot_w64(!shared_div_ok(d)) == 0) inv = recip_shared(d);
+                else inv = __builtin_fminf(1.0f / d, kFltMax);
+                word = hw_e2m1x2<0>(f[0] * inv, f[1] * inv, word);
+                word = hw_e2m1x2<1>(f[2] * inv, f[3] * inv, word);
+            } else {
+                sc = sw_e4m3fn_sat(s_hp);
+                const float inv = __builtin_fminf(1.0f / (sw_e4m3fn_decode(sc) * gs.s_dec), kFltMax);
+#pragma unroll
+                for (int j = 0; j < 4; j++) word |= sw_e2m1(f[j] * inv) << (4 * j);
+            }
+            if (off < rem) {
+                __builtin_nontemporal_store((uint16_t)word, q0 + off);
+                if ((t & 3) == 0) s80[off >> 2] = (uint8_t)sc;
+            }
+        }
+    }
+}
+
 // software candidate of the one-lane-per-block kernel: codes of sixteen values and their error
 __device__ __forceinline__ float nv_candidate_sw(const float x[16], uint32_t sc, float amax, const NvScales& gs, float denom,
                                                  int flags, uint32_t codes[16]) {
@@ -945,16 +1061,18 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_fake_kernel(const FlatTable 
 using namespace mq;
 
 bool mq_nvfp4_fast_ok(const void* w, int dtype, const void* q) {
-    return (dtype == MQ_BF16 || dtype == MQ_F16) && ((uintptr_t)w % 16) == 0 && ((uintptr_t)q % 4) == 0;
+    return dtype >= MQ_BF16 && dtype <= MQ_F32 && ((uintptr_t)w % 16) == 0 && ((uintptr_t)q % 4) == 0;
 }
 
-// the 16-bit dtype of a launch's tensors rides in the flags word of the launch helpers below (not a public flag)
-constexpr int kNvFlagF16 = 1 << 30;
+// the dtype of a launch's tensors rides in the flags word of the launch helpers below (not public flags)
+constexpr int kNvFlagF16 = 1 << 30, kNvFlagF32 = 1 << 29;
+static int nv_dtype_flag(int dtype) { return dtype == MQ_F32 ? kNvFlagF32 : dtype == MQ_F16 ? kNvFlagF16 : 0; }
 
-// tab.job[i]: w, aux = amax record, section, units = numel / 8, s = (void*)numel; every tensor of the one 16-bit dtype
+// tab.job[i]: w, aux = amax record, section, units = numel / 8, s = (void*)numel; every tensor of the one dtype
 int mq_nvfp4_amax_launch_group(int dtype, FlatTable& tab, hipStream_t st) {
     const dim3 grid(kSectionWords, (unsigned)tab.n), blk(256);
-    if (dtype == MQ_F16) hipLaunchKernelGGL((nvfp4_amax_bf16_kernel<FlatTable, 1>), grid, blk, 0, st, tab);
+    if (dtype == MQ_F32) hipLaunchKernelGGL(nvfp4_amax_f32_kernel<FlatTable>, grid, blk, 0, st, tab);
+    else if (dtype == MQ_F16) hipLaunchKernelGGL((nvfp4_amax_bf16_kernel<FlatTable, 1>), grid, blk, 0, st, tab);
     else hipLaunchKernelGGL((nvfp4_amax_bf16_kernel<FlatTable, 0>), grid, blk, 0, st, tab);
     return mq_check_launch("nvfp4 amax");
 }
@@ -963,7 +1081,8 @@ int mq_nvfp4_amax_launch_table(int dtype, const FlatJob* device_jobs, int n, hip
     if (n == 0) return MQ_OK;
     const FlatRef ref{device_jobs, 0, 0};
     const dim3 grid(kSectionWords, (unsigned)n), blk(256);
-    if (dtype == MQ_F16) hipLaunchKernelGGL((nvfp4_amax_bf16_kernel<FlatRef, 1>), grid, blk, 0, st, ref);
+    if (dtype == MQ_F32) hipLaunchKernelGGL(nvfp4_amax_f32_kernel<FlatRef>, grid, blk, 0, st, ref);
+    else if (dtype == MQ_F16) hipLaunchKernelGGL((nvfp4_amax_bf16_kernel<FlatRef, 1>), grid, blk, 0, st, ref);
     else hipLaunchKernelGGL((nvfp4_amax_bf16_kernel<FlatRef, 0>), grid, blk, 0, st, ref);
     return mq_check_launch("nvfp4 amax");
 }
@@ -985,9 +1104,26 @@ static void launch_nvfp4_quant_dtype(const Table& tab, int flags, float numer, d
         }
     }
 }
+template <class Table>
+static void launch_nvfp4_quant_f32(const Table& tab, int flags, float numer, dim3 grid, hipStream_t st) {
+    const dim3 blk(kNvThreads);
+    const int fos = (flags & MQ_NVFP4_4OVER6) ? 1 + nv_error_mode(flags) : 0;
+    if constexpr (std::is_same<Table, FlatRef>::value) {
+        hipLaunchKernelGGL((nvfp4_quant_f32_kernel<0, Table>), grid, blk, 0, st, tab, numer);
+    } else {
+        switch (fos) {
+            case 0: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<0, Table>), grid, blk, 0, st, tab, numer); break;
+            case 1: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<1, Table>), grid, blk, 0, st, tab, numer); break;
+            case 2: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<2, Table>), grid, blk, 0, st, tab, numer); break;
+            case 3: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<3, Table>), grid, blk, 0, st, tab, numer); break;
+            default: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<4, Table>), grid, blk, 0, st, tab, numer); break;
+        }
+    }
+}
 template <int PASS, class Table>
 static void launch_nvfp4_quant(const Table& tab, int flags, float numer, dim3 grid, hipStream_t st) {
-    if (flags & kNvFlagF16) launch_nvfp4_quant_dtype<PASS, Table, 1>(tab, flags, numer, grid, st);
+    if (PASS == 0 && (flags & kNvFlagF32)) launch_nvfp4_quant_f32(tab, flags, numer, grid, st);
+    else if (flags & kNvFlagF16) launch_nvfp4_quant_dtype<PASS, Table, 1>(tab, flags, numer, grid, st);
     else launch_nvfp4_quant_dtype<PASS, Table, 0>(tab, flags, numer, grid, st);
 }
 
@@ -1016,19 +1152,21 @@ static int nvfp4_quant_launch(const Table& tab, int n, int e4m3_max, int flags, 
 // mode 0 (single calls): section = sections to fold; fold, then quantize.
 // mode 1 (job driver, after its amax launch): section = place of the tensor inside its record, pad = tensors sharing the
 //   record (adjacent entries); fold once per record, clear the sections, quantize.
+// (fp32 tensors take modes 0 and 1.)
 // mode 2 (job driver, carried-over amax; the sections were cleared by the previous sync's fold): quantize with the
 //   record's old scales while collecting the new partial maxima, fold and compare, quantize again where they differ.
 int mq_nvfp4_quant_launch_group(int dtype, FlatTable& tab, int e4m3_max, int flags, int mode, hipStream_t st) {
-    if (!flat_grid(tab, nv_units_per_block(flags & MQ_NVFP4_4OVER6))) return mq_fail(MQ_ERR_ARG, "tensor too large");
-    return nvfp4_quant_launch(tab, tab.n, e4m3_max, flags | (dtype == MQ_F16 ? kNvFlagF16 : 0), mode, st);
+    const int fos = flags & MQ_NVFP4_4OVER6;
+    if (!flat_grid(tab, dtype == MQ_F32 ? nv_f32_units_per_block(fos) : nv_units_per_block(fos))) return mq_fail(MQ_ERR_ARG, "tensor too large");
+    return nvfp4_quant_launch(tab, tab.n, e4m3_max, flags | nv_dtype_flag(dtype), mode, st);
 }
 // modes 1 and 2 over n descriptors of a device table (standard block scaling only); max_units: the largest tensor's units
 int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int e4m3_max, int mode,
                                 hipStream_t st) {
     FlatRef ref{device_jobs, 0, 0};
-    if (!flat_grid(ref, max_units, kNvThreads * kNvUnroll)) return mq_fail(MQ_ERR_ARG, "tensor too large");
+    if (!flat_grid(ref, max_units, dtype == MQ_F32 ? nv_f32_units_per_block(0) : kNvThreads * kNvUnroll)) return mq_fail(MQ_ERR_ARG, "tensor too large");
     if (n == 0) return MQ_OK;
-    return nvfp4_quant_launch(ref, n, e4m3_max, dtype == MQ_F16 ? kNvFlagF16 : 0, mode, st);
+    return nvfp4_quant_launch(ref, n, e4m3_max, nv_dtype_flag(dtype), mode, st);
 }
 
 // Whether a chunk of NVFP4 jobs (standard scaling, packed kernels, no carried amax) takes the one-pass form.  `slots` is the
@@ -1086,7 +1224,7 @@ extern "C" int mq_nvfp4_amax(const void* w, int dtype, int64_t numel, void* reco
     if (dtype < MQ_BF16 || dtype > MQ_F32 || numel < 0) return mq_fail(MQ_ERR_ARG, "bad argument");
     if (section < 0 || section >= MQ_NVFP4_SECTIONS) return mq_fail(MQ_ERR_ARG, "bad amax record section");
     hipStream_t st = (hipStream_t)stream;
-    if ((dtype == MQ_BF16 || dtype == MQ_F16) && ((uintptr_t)w % 16) == 0) {
+    if (((uintptr_t)w % 16) == 0) {
         FlatTable tab{};
         tab.n = 1;
         tab.job[0] = FlatJob{w, nullptr, (void*)(uintptr_t)numel, record, numel / 8, nullptr, section, 0};

@@ -374,7 +374,7 @@ static int run_nvfp4(const mq_job* jobs, int64_t n_all, int64_t i, int64_t j, co
             return k;
         };
         auto all_fast_in = [&](int64_t k) {
-            for (int64_t t = i; t < k; t++)       // (the packed kernels are compiled per 16-bit dtype: one per launch)
+            for (int64_t t = i; t < k; t++)       // (the packed kernels are compiled per dtype: one per launch)
                 if (!job_fast(jobs[t]) || jobs[t].dtype != jobs[i].dtype) return false;
             return true;
         };
@@ -397,7 +397,8 @@ static int run_nvfp4(const mq_job* jobs, int64_t n_all, int64_t i, int64_t j, co
         if (all_fast) {
             // MQ_NVFP4_CARRY_AMAX (set by a caller that replays this very list, records included, after a first plain
             // run): one pass with last sync's amax instead of the amax pass; every job of the chunk must ask for it
-            bool carry = true;
+            // (fp32 tensors have neither this form nor the one-pass form)
+            bool carry = jobs[i].dtype != MQ_F32;
             for (int t = 0; t < n; t++) carry &= (jobs[i + t].p1 & MQ_NVFP4_CARRY_AMAX) != 0;
             int rc = MQ_OK;
             int64_t max_units = 0, sum_units = 0, slots = 0, max_slots = 0;
@@ -410,7 +411,7 @@ static int run_nvfp4(const mq_job* jobs, int64_t n_all, int64_t i, int64_t j, co
                 slots = (section[t] == 0 ? 0 : slots) + mq_nvfp4_one_pass_slots(u);
                 max_slots = slots > max_slots ? slots : max_slots;
             }
-            const bool one_pass = !carry && standard && !empty && mq_nvfp4_one_pass_ok(max_units, max_slots, sum_units * 16);
+            const bool one_pass = !carry && standard && !empty && jobs[i].dtype != MQ_F32 && mq_nvfp4_one_pass_ok(max_units, max_slots, sum_units * 16);
             if (from_table) {
                 if (one_pass) {
                     rc = mq_nvfp4_one_pass_launch_table(jobs[i].dtype, table + i, n, max_units, jobs[i].p0, jobs[i].p1, st);
