@@ -252,6 +252,10 @@ typedef u32x4 u32x4_at2 __attribute__((aligned(2)));
 typedef u32x2 u32x2_at1 __attribute__((aligned(1)));
 __device__ __forceinline__ u32x4 ld16_at2(const void* p) { return *reinterpret_cast<const u32x4_at2*>(p); }
 __device__ __forceinline__ void st8_at1(void* p, u32x2 v) { *reinterpret_cast<u32x2_at1*>(p) = v; }
+typedef uint32_t u32_at1 __attribute__((aligned(1)));
+__device__ __forceinline__ u32x2 ld8_at1(const void* p) { return *reinterpret_cast<const u32x2_at1*>(p); }
+__device__ __forceinline__ void st4_at1(void* p, uint32_t v) { *reinterpret_cast<u32_at1*>(p) = v; }
+__device__ __forceinline__ void st16_at2(void* p, u32x4 v) { *reinterpret_cast<u32x4_at2*>(p) = v; }
 __device__ __forceinline__ void st4(void* p, uint32_t v) { __builtin_nontemporal_store(v, reinterpret_cast<uint32_t*>(p)); }
 
 }  // namespace mq

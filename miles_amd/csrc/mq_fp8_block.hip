@@ -598,6 +598,160 @@ __global__ __launch_bounds__(256) void fp8_tensor_quant_bf16_kernel(const uint16
     }
 }
 
+// ---- the same of any alignment, and of fp32 ----------------------------------------------------------------------
+// 16-byte loads at any element boundary (E elements: eight of a 16-bit dtype, four of fp32); the last unit of a row, or of
+// the tensor, is moved back to end with it, so that it codes a few elements a second time, to the same bytes.
+// HBM-bound; fp32 quotients come correctly rounded from div24_by_shared where that matters to an e4m3 code.  Eight tensors in
+// eight calls, three launches each per tensor and one per channel (the two element-wise passes before): per tensor
+// [2048, 4096] fp32 381 -> 173 us, [2049, 4099] bf16 379 -> 148; per channel 198 -> 118 and 209 -> 116, which is the host's
+// time for eight calls.
+template <int DT> constexpr int kUnitElems = DT == MQ_F32 ? 4 : 8;
+template <int DT>
+__device__ __forceinline__ u32x4 ld_unit(const void* p, int64_t elem) {
+    return DT == MQ_F32 ? ld16_at2((const float*)p + elem) : ld16_at2((const uint16_t*)p + elem);
+}
+// the largest magnitude of a unit: an fp32 pattern, or packed 16-bit patterns
+template <int DT>
+__device__ __forceinline__ uint32_t unit_max(uint32_t m, const u32x4 v) {
+    if (DT == MQ_F32)
+        return umax(m, umax(umax(v.x & 0x7FFFFFFFu, v.y & 0x7FFFFFFFu), umax(v.z & 0x7FFFFFFFu, v.w & 0x7FFFFFFFu)));
+    return max2_u16(m, max2_u16(max2_u16(abs2(v.x), abs2(v.y)), max2_u16(abs2(v.z), abs2(v.w))));
+}
+// what a lane collected with unit_max, as an fp32 pattern
+template <int DT>
+__device__ __forceinline__ uint32_t unit_max_f32(uint32_t m) {
+    return DT == MQ_F32 ? m : f2u(DT == MQ_F16 ? elem_lo<1>(hmax_u16(m)) : elem_lo<0>(hmax_u16(m)));
+}
+// codes of one unit; ROUNDED: the quotient is rounded to the dtype first (one scale for the whole tensor)
+template <int DT, bool ROUNDED>
+__device__ __forceinline__ void scaled_unit(const u32x4 v, float s, float y, bool fast_div, bool plain, uint8_t* __restrict__ q) {
+    constexpr int E = kUnitElems<DT>;
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    float f[E];
+#pragma unroll
+    for (int j = 0; j < E; j++) {
+        if (DT == MQ_F32) f[j] = u2f(w[j]);
+        else if (DT == MQ_F16) f[j] = (j & 1) ? elem_hi<1>(w[j / 2]) : elem_lo<1>(w[j / 2]);
+        else f[j] = (j & 1) ? elem_hi<0>(w[j / 2]) : elem_lo<0>(w[j / 2]);
+    }
+#pragma unroll
+    for (int j = 0; j < E; j++)
+        f[j] = !fast_div ? f[j] / s : DT == MQ_F32 ? div24_by_shared(f[j], s, y) : div_by_shared(f[j], s, y);
+    if (ROUNDED && DT != MQ_F32) {
+#pragma unroll
+        for (int j = 0; j < E; j += 2) {
+            if (DT == MQ_BF16 && plain) {
+                const uint32_t p = hw_bf16x2(f[j], f[j + 1]);
+                f[j] = bf16_lo(p);
+                f[j + 1] = bf16_hi(p);
+            } else {
+                f[j] = round_to_dtype(f[j], DT);
+                f[j + 1] = round_to_dtype(f[j + 1], DT);
+            }
+        }
+    }
+    u32x2 o = {0u, 0u};
+    if (plain) {
+        o.x = hw_e4m3x4(f[0], f[1], f[2], f[3]);
+        if (E == 8) o.y = hw_e4m3x4(f[E - 4], f[E - 3], f[E - 2], f[E - 1]);
+    } else {                                  // inf / NaN, or a zero scale: clamp and convert in software
+#pragma unroll
+        for (int j = 0; j < E; j++) {
+            const uint32_t c = sw_e4m3fn(clamp_keep_nan(f[j], -kFp8Max, kFp8Max)) << (8 * (j & 3));
+            if (j < 4) o.x |= c;
+            else o.y |= c;
+        }
+    }
+    if (E == 8) st8_at1(q, o);
+    else st4_at1(q, o.x);
+}
+// per channel: as fp8_channel_bf16_kernel, a row in the registers of ROWLANES lanes, up to UNITS units each
+template <int ROWLANES, int DT, int UNITS>
+__global__ __launch_bounds__(256) void fp8_channel_any_kernel(const void* __restrict__ w, int64_t ldw, int64_t K, int64_t M,
+                                                              float floor_v, uint8_t* __restrict__ q, float* __restrict__ scale, int chunk) {
+    __shared__ uint32_t wave_amax[4];
+    constexpr int kRows = 256 / ROWLANES, E = kUnitElems<DT>;
+    const int t = threadIdx.x, lane = t % ROWLANES;
+    const int64_t row = xcd_chunked_block(chunk) * kRows + t / ROWLANES;
+    const bool row_ok = row < M;
+    const int64_t src = (row_ok ? row : M - 1) * ldw;
+    const int units = (int)((K + E - 1) / E), last = (int)K - E;
+    u32x4 v[UNITS];
+    uint32_t m = 0;
+#pragma unroll
+    for (int u = 0; u < UNITS; u++) {
+        const int unit = lane + u * ROWLANES, at = unit * E < last ? unit * E : last;      // (lanes past the end read the last unit)
+        v[u] = u * ROWLANES < units ? ld_unit<DT>(w, src + at) : u32x4{0u, 0u, 0u, 0u};
+    }
+#pragma unroll
+    for (int u = 0; u < UNITS; u++) m = unit_max<DT>(m, v[u]);
+    m = wave_max(unit_max_f32<DT>(m));
+    if (ROWLANES == 256) {
+        if ((t & 63) == 0) wave_amax[t >> 6] = m;
+        __syncthreads();
+        m = umax(umax(wave_amax[0], wave_amax[1]), umax(wave_amax[2], wave_amax[3]));
+    }
+    float amax = u2f(m);
+    if (amax < floor_v) amax = floor_v;
+    const float s = amax / kFp8Max, y = 1.0f / s;
+    const bool fast_div = shared_div_ok(s), plain = m < 0x7F800000u && s > 0.0f;
+    if (!row_ok) return;
+    if (lane == 0) scale[row] = s;
+#pragma unroll
+    for (int u = 0; u < UNITS; u++) {
+        const int unit = lane + u * ROWLANES, at = unit * E < last ? unit * E : last;
+        if (unit < units) scaled_unit<DT, false>(v[u], s, y, fast_div, plain, q + row * K + at);
+    }
+}
+// per tensor: amax pass (one atomic max per workgroup on the fp32 pattern) and flat quantize pass over n contiguous elements
+constexpr int kTensorAnyLoads = 4, kTensorAnyUnits = 2;
+constexpr int kTensorAnyMaxBlocks = 512;      // of the amax pass: its atomics on one word follow each other at some 8 ns
+template <int DT>
+__global__ __launch_bounds__(256) void fp8_tensor_amax_any_kernel(const void* __restrict__ w, int64_t n, uint32_t* __restrict__ amax_bits) {
+    __shared__ uint32_t wave_amax[4];
+    constexpr int E = kUnitElems<DT>;
+    const int t = threadIdx.x;
+    const int64_t units = (n + E - 1) / E;
+    uint32_t m = 0;
+    for (int64_t base = (int64_t)blockIdx.x * (256 * kTensorAnyLoads); base < units; base += (int64_t)gridDim.x * (256 * kTensorAnyLoads)) {
+        u32x4 v[kTensorAnyLoads];
+#pragma unroll
+        for (int i = 0; i < kTensorAnyLoads; i++) {
+            const int64_t at = (base + i * 256 + t) * E;
+            v[i] = ld_unit<DT>(w, at < n - E ? at : n - E);
+        }
+#pragma unroll
+        for (int i = 0; i < kTensorAnyLoads; i++) m = unit_max<DT>(m, v[i]);
+    }
+    m = wave_max(unit_max_f32<DT>(m));
+    if ((t & 63) == 0) wave_amax[t >> 6] = m;
+    __syncthreads();
+    if (t == 0) atomicMax(amax_bits, umax(umax(wave_amax[0], wave_amax[1]), umax(wave_amax[2], wave_amax[3])));
+}
+template <int DT>
+__global__ __launch_bounds__(256) void fp8_tensor_quant_any_kernel(const void* __restrict__ w, int64_t n, const uint32_t* __restrict__ amax_bits,
+                                                                   float floor_v, uint8_t* __restrict__ q, float* __restrict__ scale, int chunk) {
+    constexpr int E = kUnitElems<DT>;
+    const int64_t base = xcd_chunked_block(chunk) * (256 * kTensorAnyUnits) + threadIdx.x;
+    u32x4 v[kTensorAnyUnits];
+#pragma unroll
+    for (int i = 0; i < kTensorAnyUnits; i++) {
+        const int64_t at = (base + i * 256) * E;
+        v[i] = ld_unit<DT>(w, at < n - E ? at : n - E);
+    }
+    const uint32_t abits = amax_bits[0];
+    float amax = u2f(abits);
+    if (amax < floor_v) amax = floor_v;
+    const float s = amax / kFp8Max, y = 1.0f / s;
+    const bool fast_div = shared_div_ok(s), plain = abits < 0x7F800000u && s > 0.0f;
+    if (base == 0) scale[0] = s;
+#pragma unroll
+    for (int i = 0; i < kTensorAnyUnits; i++) {
+        const int64_t at = (base + i * 256) * E;
+        if (at < n) scaled_unit<DT, true>(v[i], s, y, fast_div, plain, q + (at < n - E ? at : n - E));
+    }
+}
+
 __global__ void fill_u32_kernel(uint32_t* p, uint32_t v, int n) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
@@ -837,6 +991,41 @@ extern "C" int mq_fp8_block_quant_pow2(const void* w, int dtype, int64_t ldw, vo
     return fp8_block_launch(2, w, dtype, ldw, 1, q, scale, M, K, kTile, kTile, (hipStream_t)stream);
 }
 
+// the forms for any alignment and for fp32 (rows, or the whole tensor, of at least one unit)
+template <int DT>
+static bool fp8_scaled_any(const void* w, int64_t ldw, uint8_t* q, float* scale, uint32_t* amax_ws, int64_t M, int64_t K,
+                           int per_channel, float floor_v, hipStream_t st) {
+    constexpr int E = kUnitElems<DT>;
+    if ((uintptr_t)w % (DT == MQ_F32 ? 4 : 2) != 0) return false;
+    if (per_channel) {
+        const int64_t units = (K + E - 1) / E;
+        if (K < E || units > 256 * 16) return false;
+        // (a wavefront per row while that leaves a lane no more than four units, as for aligned rows; sixteen units a lane
+        // are 64 registers)
+        const bool four_rows = units <= 256;
+        const int64_t blocks = four_rows ? (M + 3) / 4 : M;
+        if (blocks > 0x7FFFF000ll) return false;          // (the grid is padded by up to 511 workgroups)
+        const int chunk = (int)flat_chunk(blocks);
+        const dim3 grid((unsigned)flat_padded(blocks, chunk)), blk(256);
+        if (four_rows) hipLaunchKernelGGL((fp8_channel_any_kernel<64, DT, 4>), grid, blk, 0, st, w, ldw, K, M, floor_v, q, scale, chunk);
+        else if (units <= 1024) hipLaunchKernelGGL((fp8_channel_any_kernel<256, DT, 4>), grid, blk, 0, st, w, ldw, K, M, floor_v, q, scale, chunk);
+        else if (units <= 2048) hipLaunchKernelGGL((fp8_channel_any_kernel<256, DT, 8>), grid, blk, 0, st, w, ldw, K, M, floor_v, q, scale, chunk);
+        else hipLaunchKernelGGL((fp8_channel_any_kernel<256, DT, 16>), grid, blk, 0, st, w, ldw, K, M, floor_v, q, scale, chunk);
+        return true;
+    }
+    const int64_t n = M * K, units = (n + E - 1) / E;
+    if ((ldw != K && M != 1) || n < E || units >= (1ll << 38)) return false;
+    const int64_t trips = (units + 256 * kTensorAnyLoads - 1) / (256 * kTensorAnyLoads);
+    hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, amax_ws, 0u, 1);
+    hipLaunchKernelGGL(fp8_tensor_amax_any_kernel<DT>, dim3((unsigned)(trips < kTensorAnyMaxBlocks ? trips : kTensorAnyMaxBlocks)), dim3(256), 0,
+                       st, w, n, amax_ws);
+    const int64_t blocks = (units + 256 * kTensorAnyUnits - 1) / (256 * kTensorAnyUnits);
+    const int chunk = (int)flat_chunk(blocks);
+    hipLaunchKernelGGL(fp8_tensor_quant_any_kernel<DT>, dim3((unsigned)flat_padded(blocks, chunk)), dim3(256), 0, st, w, n, amax_ws,
+                       floor_v, q, scale, chunk);
+    return true;
+}
+
 static int fp8_scaled_quant(const void* w, int dtype, int64_t ldw, void* q, float* scale, void* amax_ws, int64_t M,
                             int64_t K, int per_channel, float floor_in_dtype, void* stream) {
     if ((!w || !q) && M != 0 && K != 0) return mq_fail(MQ_ERR_ARG, "null pointer");
@@ -875,6 +1064,12 @@ static int fp8_scaled_quant(const void* w, int dtype, int64_t ldw, void* q, floa
                            (const uint32_t*)amax_ws, floor_in_dtype, (uint8_t*)q, scale, units, chunk);
         return mq_check_launch("fp8 scaled quant");
     }
+    uint32_t* ws = (uint32_t*)amax_ws;
+    if (dtype == MQ_F32  ? fp8_scaled_any<MQ_F32>(w, ldw, (uint8_t*)q, scale, ws, M, K, per_channel, floor_in_dtype, st)
+        : dtype == MQ_F16 ? fp8_scaled_any<MQ_F16>(w, ldw, (uint8_t*)q, scale, ws, M, K, per_channel, floor_in_dtype, st)
+                          : fp8_scaled_any<MQ_BF16>(w, ldw, (uint8_t*)q, scale, ws, M, K, per_channel, floor_in_dtype, st))
+        return mq_check_launch("fp8 scaled quant");
+    // rows of more than 4096 units or of less than one, strided tensors with one scale
     if (!per_channel) hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, (uint32_t*)amax_ws, 0u, 1);
     hipLaunchKernelGGL(fp8_row_amax_kernel, dim3((unsigned)M), dim3(256), 0, st, w, dtype, ldw, K,
                        (uint32_t*)amax_ws, per_channel);

@@ -45,6 +45,11 @@ def block_fp8(weight: torch.Tensor, block_size):
     return q, scale
 
 
+# clamp(min=1e-12) acts in the weight dtype (fp16 has no such value): the floor, and its fp32 bit pattern
+_FLOORS = {}
+for _dtype in (torch.bfloat16, torch.float16, torch.float32):
+    _floor = torch.tensor(1e-12, dtype=_dtype).float()
+    _FLOORS[_dtype] = float(_floor), int(_floor.view(torch.int32))
 _AMAX_RECORD_WORDS = 1280   # MQ_NVFP4_RECORD_WORDS: partial maxima of a tensor on the device, then its folded amax
 
 
@@ -59,11 +64,10 @@ def _scaled_fp8(weight: torch.Tensor, per_channel: bool):
     w = weight if weight.stride(1) == 1 else weight.contiguous()
     q = torch.empty((n, k), dtype=torch.float8_e4m3fn, device=w.device)
     scale = torch.empty((n, 1) if per_channel else (1,), dtype=torch.float32, device=w.device)
-    floor = float(torch.tensor(1e-12, dtype=w.dtype).float())  # clamp(min=1e-12) acts in the weight dtype
+    floor, floor_bits = _FLOORS.get(w.dtype, (0.0, 0))      # (another dtype is refused below)
     if not per_channel and w.dtype in (torch.bfloat16, torch.float16) and w.is_contiguous() and k % 8 == 0 and w.data_ptr() % 16 == 0:
         # a job of the batched driver (grouped launches, replayable): amax record as for NVFP4
         record = torch.empty(_AMAX_RECORD_WORDS, dtype=torch.int32, device=w.device)
-        floor_bits = int(torch.tensor(floor, dtype=torch.float32).view(torch.int32))
         launch.submit(_lib.JOB_FP8_TENSOR, w, q, scale, record, None, n, k, k, floor_bits, 0)
         return q, scale
     ws = torch.empty(max(n, 1), dtype=torch.int32, device=w.device)

@@ -101,3 +101,68 @@ def test_division_sequence_of_fp32_tiles(oracle):  # noqa: F811
     q_o, s_o = oracle.block_fp8(w, (128, 128))
     _assert_same(s, s_o, "scales")
     _assert_same(q, q_o, "codes")
+
+
+# shorter than a unit of either size, a unit and its neighbours, the register limits of the row kernels (256, 1024, 2048 and
+# 4096 units of four or eight elements) and past them
+ROW_WIDTHS = [1, 3, 4, 5, 7, 8, 9, 255, 1021, 1027, 2047, 2049, 4093, 4099, 8191, 8195, 16381, 16387, 32767, 32771]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("specials", [False, True])
+@pytest.mark.parametrize("strategy", ["channel", "tensor"])
+def test_scaled_rows_of_any_width(oracle, dtype, specials, strategy):  # noqa: F811
+    from miles_amd.tools.convert_hf_to_fp8 import quant_fp8
+
+    reference = oracle.channel_fp8 if strategy == "channel" else oracle.tensor_fp8
+    for i, cols in enumerate(ROW_WIDTHS):
+        wide = _matrix((5 + i % 3, cols + 3), dtype, 300 + i, specials).to(DEV)
+        wide[1] = 0
+        views = [wide[:, 3:].contiguous(), wide[:, 1:1 + cols]]      # contiguous rows; rows of a wider matrix off every boundary
+        flat = torch.empty(views[0].numel() + 1, dtype=dtype, device=DEV)
+        flat[1:] = views[0].reshape(-1)
+        views.append(flat[1:].view(views[0].shape))                  # contiguous, one element off the allocation's start
+        for v in views:
+            q, s = quant_fp8(v, strategy)
+            q_o, s_o = reference(v.cpu().contiguous())
+            what = f"{strategy} {dtype} {tuple(v.shape)} stride {v.stride(0)}"
+            _assert_same(_one_nan(s.view(torch.uint8)) if specials else s, _one_nan(s_o.view(torch.uint8)) if specials else s_o, what + " scales")
+            _assert_same(_one_nan(q), _one_nan(q_o), what + " codes")
+
+
+def test_tensor_scale_of_many_workgroups(oracle):  # noqa: F811
+    """Several trips of the amax pass, and the maximum in the last, moved-back unit."""
+    from miles_amd.tools.convert_hf_to_fp8 import tensor_fp8
+
+    for dtype in DTYPES:
+        w = _matrix((1021, 2053), dtype, 400, False)
+        w[-1, -1] = w.abs().max() * 2
+        q, s = tensor_fp8(w.to(DEV))
+        q_o, s_o = oracle.tensor_fp8(w)
+        _assert_same(s, s_o, f"{dtype} scale")
+        _assert_same(q, q_o, f"{dtype} codes")
+
+
+@pytest.mark.parametrize("block", [8, 32, 128])
+def test_dequantize_rows_of_any_width(oracle, block):  # noqa: F811
+    """One list of matrices from one unit to several tiles wide, codes at any byte, NaN codes and non-finite scales."""
+    from miles_amd import launch
+    from miles_amd.tools.fp8_cast_bf16 import weight_dequant
+
+    g = torch.Generator().manual_seed(block)
+    cases = []
+    for cols in [1, 7, 8, 9, 15, 17, 121, 127, 129, 135, 263, 1000, 2051]:
+        rows = 3 * block // 2 + 1
+        codes = torch.randint(0, 256, (rows, cols), generator=g, dtype=torch.uint8)
+        if cols % 2:
+            codes = torch.where(codes & 0x7F == 0x7F, codes & 0x3F, codes)
+        s = torch.exp2(torch.randint(-30, 30, (-(-rows // block), -(-cols // block)), generator=g).float()) * 1.37
+        if cols > 128:
+            s[0, 0], s[-1, -1] = float("inf"), float("nan")
+        flat = torch.zeros(codes.numel() + 3, dtype=torch.uint8, device=DEV)
+        flat[3:] = codes.reshape(-1).to(DEV)
+        cases.append((codes.view(torch.float8_e4m3fn), s, flat[3:].view(rows, cols).view(torch.float8_e4m3fn)))
+    with launch.deferred():
+        outs = [weight_dequant(x, s.to(DEV), block) for _codes, s, x in cases]
+    for (codes, s, _x), y in zip(cases, outs):
+        _assert_same(y, oracle.weight_dequant(codes, s, block), f"block {block} {tuple(codes.shape)}")
