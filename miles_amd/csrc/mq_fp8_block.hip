@@ -778,6 +778,7 @@ struct DequantJob {
     uint32_t magic, shift;   // floor(n / units_per_row) == (t + ((n - t) >> 1)) >> shift, t = mulhi(magic, n)
     int32_t block_shift;     // log2(block)
     int32_t tiles_n;
+    int32_t N;               // columns (the form for any alignment)
 };
 struct DequantTable {
     int32_t n;
@@ -841,6 +842,51 @@ __global__ __launch_bounds__(kDqThreads) void fp8_dequant_kernel(const DequantTa
         }
         st16(job.y + (int64_t)unit * 8, u32x4{o[0], o[1], o[2], o[3]});
     }
+}
+
+// Rows of any length >= 8 and any alignment: units_per_row = ceil(N / 8), and the last unit of a row is moved back to end with
+// the row, decoding a few codes a second time.  Such a unit may reach into two tiles, hence two scales.  Bound by HBM and, a
+// little, by the lines that neighbouring rows' units share.
+// Eight [2049, 4099] matrices as one job list: 40 us with the submission, 5.0 TB/s, what [2048, 4096] ones take (200 us in the
+// element-wise kernel, a launch each).
+__global__ __launch_bounds__(kDqThreads) void fp8_dequant_any_kernel(const DequantTable tab) {
+    const DequantJob& job = tab.job[blockIdx.y];
+    const int64_t base64 = xcd_chunked_block(tab.chunk) * kDqThreads;
+    if (base64 >= job.units) return;
+    const uint32_t unit = (uint32_t)base64 + threadIdx.x;
+    const uint32_t uc = unit < job.units ? unit : (uint32_t)base64;
+    const uint32_t th = __umulhi(job.magic, uc);
+    const uint32_t r = (th + ((uc - th) >> 1)) >> job.shift;
+    const uint32_t at = (uc - r * job.units_per_row) * 8u, last = (uint32_t)job.N - 8u;
+    const uint32_t c = at < last ? at : last;
+    const int64_t off = (int64_t)r * job.N + c;
+    const u32x2 in = ld8_at1(job.x + off);
+    const float* __restrict__ s = job.s + (int64_t)(r >> job.block_shift) * job.tiles_n;
+    const uint32_t tile = c >> job.block_shift;
+    const float s0 = s[tile], s1 = s[(c + 7u) >> job.block_shift];
+    const uint32_t split = ((tile + 1u) << job.block_shift) - c;      // elements of the first tile
+    if (unit >= job.units) return;
+    const uint32_t wd[2] = {in.x, in.y};
+    bool special = (f2u(s0) & 0x7F800000u) == 0x7F800000u || (f2u(s1) & 0x7F800000u) == 0x7F800000u;
+#pragma unroll
+    for (int k = 0; k < 2; k++) special |= (((wd[k] & 0x7F7F7F7Fu) + 0x01010101u) & 0x80808080u) != 0u;
+    uint32_t o[4];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const float sc[4] = {4u * k < split ? s0 : s1, 4u * k + 1u < split ? s0 : s1, 4u * k + 2u < split ? s0 : s1, 4u * k + 3u < split ? s0 : s1};
+        if (!special) {
+            const f32x2 a = hw_e4m3x2_decode<false>(wd[k]), b = hw_e4m3x2_decode<true>(wd[k]);
+            o[2 * k] = hw_bf16x2(a.x * sc[0], a.y * sc[1]);
+            o[2 * k + 1] = hw_bf16x2(b.x * sc[2], b.y * sc[3]);
+        } else {
+            uint32_t h[4];
+#pragma unroll
+            for (int b = 0; b < 4; b++) h[b] = sw_bf16(sw_e4m3fn_decode((wd[k] >> (8 * b)) & 0xFFu) * sc[b]);
+            o[2 * k] = h[0] | (h[1] << 16);
+            o[2 * k + 1] = h[2] | (h[3] << 16);
+        }
+    }
+    st16_at2(job.y + off, u32x4{o[0], o[1], o[2], o[3]});
 }
 
 __global__ __launch_bounds__(256) void fp8_dequant_generic_kernel(const uint8_t* __restrict__ x,
@@ -1138,7 +1184,14 @@ bool mq_fp8_dequant_fast_ok(const void* x, const void* y, int64_t M, int64_t N, 
            M * (N / 8) < 0xFFFFFFF0ll;
 }
 
-int mq_fp8_dequant_launch_group(const MqDequantArgs* a, int n, hipStream_t st) {
+// the same without the alignment: rows of nine codes and more (two units)
+bool mq_fp8_dequant_any_ok(const void* y, int64_t M, int64_t N, int block) {
+    const bool pow2 = block >= 8 && (block & (block - 1)) == 0;
+    return N >= 9 && N < (1ll << 31) && pow2 && ((uintptr_t)y % 2) == 0 && M * ((N + 7) / 8) < 0xFFFFFFF0ll;
+}
+
+// `aligned`: every tensor passed mq_fp8_dequant_fast_ok, otherwise mq_fp8_dequant_any_ok
+int mq_fp8_dequant_launch_group(const MqDequantArgs* a, int n, bool aligned, hipStream_t st) {
     DequantTable tab{};
     tab.n = n;
     int64_t mx = 0;
@@ -1147,8 +1200,9 @@ int mq_fp8_dequant_launch_group(const MqDequantArgs* a, int n, hipStream_t st) {
         j.x = (const uint8_t*)a[i].x;
         j.s = a[i].s;
         j.y = (uint16_t*)a[i].y;
-        j.units = (uint32_t)(a[i].M * (a[i].N / 8));
-        const uint32_t d = (uint32_t)(a[i].N / 8);   // >= 2
+        const uint32_t d = (uint32_t)((a[i].N + 7) / 8);   // >= 2
+        j.units = (uint32_t)(a[i].M * d);
+        j.N = (int32_t)a[i].N;
         j.units_per_row = d;
         uint32_t l = 0;
         while ((1ull << l) < d) l++;                 // ceil(log2 d) >= 1
@@ -1158,7 +1212,8 @@ int mq_fp8_dequant_launch_group(const MqDequantArgs* a, int n, hipStream_t st) {
         while ((1 << bs) < a[i].block) bs++;
         j.block_shift = bs;
         j.tiles_n = (int32_t)((a[i].N + a[i].block - 1) / a[i].block);
-        const int64_t b = ((int64_t)j.units + kDqThreads * kDqUnroll - 1) / (kDqThreads * kDqUnroll);
+        const int per_block = aligned ? kDqThreads * kDqUnroll : kDqThreads;
+        const int64_t b = ((int64_t)j.units + per_block - 1) / per_block;
         if (b > mx) mx = b;
     }
     if (mx == 0) return MQ_OK;
@@ -1166,7 +1221,8 @@ int mq_fp8_dequant_launch_group(const MqDequantArgs* a, int n, hipStream_t st) {
     mx = flat_padded(mx, chunk);
     tab.chunk = (int32_t)chunk;
     tab.max_blocks = (int32_t)mx;
-    hipLaunchKernelGGL(fp8_dequant_kernel, dim3((unsigned)mx, (unsigned)n), dim3(kDqThreads), 0, st, tab);
+    if (aligned) hipLaunchKernelGGL(fp8_dequant_kernel, dim3((unsigned)mx, (unsigned)n), dim3(kDqThreads), 0, st, tab);
+    else hipLaunchKernelGGL(fp8_dequant_any_kernel, dim3((unsigned)mx, (unsigned)n), dim3(kDqThreads), 0, st, tab);
     return mq_check_launch("fp8 block dequant");
 }
 
@@ -1224,9 +1280,10 @@ extern "C" int mq_fp8_block_dequant(const void* x, const float* s, void* y, int6
     const int64_t tiles_n = (N + block - 1) / block;
     if (tiles_n > 0x7FFFFFFF) return mq_fail(MQ_ERR_ARG, "too many tiles");
     hipStream_t st = (hipStream_t)stream;
-    if (mq_fp8_dequant_fast_ok(x, y, M, N, block)) {
+    const bool aligned = mq_fp8_dequant_fast_ok(x, y, M, N, block);
+    if (aligned || mq_fp8_dequant_any_ok(y, M, N, block)) {
         MqDequantArgs a{x, s, y, M, N, block};
-        return mq_fp8_dequant_launch_group(&a, 1, st);
+        return mq_fp8_dequant_launch_group(&a, 1, aligned, st);
     }
     int64_t blocks = (M * N + 255) / 256;
     if (blocks > mq_grid_cap()) blocks = mq_grid_cap();

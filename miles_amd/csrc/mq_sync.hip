@@ -24,7 +24,8 @@ int mq_fp8_tile_launch_group(int mode, int dtype, bool aligned, TileTable& tab, 
 int64_t mq_fp8_tile_job_finish(TileJob& j);
 int mq_fp8_tile_launch_table(int mode, int dtype, const TileJob* device_jobs, int n, int64_t max_tiles, hipStream_t st);
 bool mq_fp8_dequant_fast_ok(const void* x, const void* y, int64_t M, int64_t N, int block);
-int mq_fp8_dequant_launch_group(const MqDequantArgs* a, int n, hipStream_t st);
+bool mq_fp8_dequant_any_ok(const void* y, int64_t M, int64_t N, int block);
+int mq_fp8_dequant_launch_group(const MqDequantArgs* a, int n, bool aligned, hipStream_t st);
 bool mq_mxfp8_fast_ok(const void* w, int dtype, const void* q);
 int mq_mxfp8_launch_group(int dtype, FlatTable& tab, hipStream_t st);
 bool mq_int4_pack_fast_ok(const void* w, int dtype, int group);
@@ -113,15 +114,16 @@ static bool job_fast(const mq_job& j) {
     }
 }
 
-// FP8 tile jobs that the aligned kernel does not take still share grouped launches, of the kernel for any alignment and
-// for fp32 (row-blocked inputs are refused there)
-static bool job_tiles_any(const mq_job& j) {
+// FP8 tile jobs and dequantizations that the aligned kernels do not take still share grouped launches, of the kernels for any
+// alignment (and, for tiles, for fp32; row-blocked inputs are refused there)
+static bool job_any(const mq_job& j) {
+    if (j.kind == MQ_JOB_FP8_DEQUANT) return mq_fp8_dequant_any_ok(j.out, j.rows, j.cols, j.p0);
     return (j.kind == MQ_JOB_FP8_BLOCK || j.kind == MQ_JOB_FP8_BLOCKWISE_CAST || j.kind == MQ_JOB_FP8_BLOCK_POW2) &&
            j.rows_per_block == 0 && mq_fp8_tile_any_ok(j.in, j.dtype, j.ld, 1, j.rows, j.cols, j.p0, j.p1);
 }
 // how a job runs: alone through its entry point, in grouped launches of the tuned kernels, or of the any-alignment ones
 enum JobPath { kSinglePath, kFastPath, kAnyPath };
-static JobPath job_path(const mq_job& j) { return job_fast(j) ? kFastPath : job_tiles_any(j) ? kAnyPath : kSinglePath; }
+static JobPath job_path(const mq_job& j) { return job_fast(j) ? kFastPath : job_any(j) ? kAnyPath : kSinglePath; }
 
 static int64_t copy_dst_pitch(const mq_job& j);
 static int check_job(const mq_job& j) {
@@ -601,7 +603,7 @@ extern "C" int mq_run_jobs_tabled(const mq_job* jobs, int64_t n, const void* dev
                     const mq_job& jb = jobs[i + t];
                     a[t] = MqDequantArgs{jb.in, (const float*)jb.aux, jb.out, jb.rows, jb.cols, jb.p0};
                 }
-                rc = mq_fp8_dequant_launch_group(a, cnt, st);
+                rc = mq_fp8_dequant_launch_group(a, cnt, path == kFastPath, st);
                 break;
             }
             case MQ_JOB_MXFP8:
