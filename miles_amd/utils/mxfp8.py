@@ -59,9 +59,8 @@ def mxfp8_quantize(weight: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
 SOURCE_FP8_TILE = 128
 
 
-def _grids(weight: torch.Tensor, scale: torch.Tensor):
-    """(codes [B, N, K], tile-scale grid [B, >= ceil(N/128), >= ceil(K/128)] with unit column stride) of a source weight
-    [..., N, K] and its scale tensor; the grid may be larger than the weight needs (the reference crops it)."""
+def _check_grid(weight: torch.Tensor, scale: torch.Tensor):
+    """(N, K, tile rows, tile columns) of a source weight [..., N, K] that its scale grid covers."""
     _lib.require_gpu(weight, "FP8 source weight")
     _lib.require_gpu(scale, "FP8 source scale")
     if weight.dim() < 2 or scale.dim() != weight.dim() or weight.element_size() != 1:
@@ -71,6 +70,13 @@ def _grids(weight: torch.Tensor, scale: torch.Tensor):
     nt, kt = -(-n // SOURCE_FP8_TILE), -(-k // SOURCE_FP8_TILE)
     if scale.shape[-2] < nt or scale.shape[-1] < kt or scale.shape[:-2] != weight.shape[:-2]:
         raise ValueError(f"scale grid {tuple(scale.shape)} does not cover a weight of shape {tuple(weight.shape)}")
+    return n, k, nt, kt
+
+
+def _grids(weight: torch.Tensor, scale: torch.Tensor):
+    """(codes [B, N, K], tile-scale grid [B, >= ceil(N/128), >= ceil(K/128)] with unit column stride) of a source weight
+    [..., N, K] and its scale tensor; the grid may be larger than the weight needs (the reference crops it)."""
+    n, k, nt, kt = _check_grid(weight, scale)
     if scale.stride(-1) != 1 and scale.shape[-1] > 1:
         scale = scale.contiguous()
     batch = 1
@@ -138,10 +144,14 @@ def requantize_fp8_block_to_mxfp8(weight: torch.Tensor, scale: torch.Tensor) -> 
         raise ValueError(f"the FP8 to MXFP8 re-quantizer reads float8_e4m3fn codes, got {weight.dtype}")
     if scale.dtype != torch.float32:
         raise ValueError(f"expected fp32 tile scales, got {scale.dtype}")
-    w3, s3, nt, _kt = _grids(weight, scale)
-    n = w3.shape[-2]
+    n = _check_grid(weight, scale)[0]
     q = torch.empty(weight.shape, dtype=torch.float8_e4m3fn, device=weight.device)
     out_scale = torch.empty((*weight.shape[:-1], k // MXFP8_GROUP_SIZE), dtype=torch.uint8, device=weight.device)
+    if weight.dim() == 2 and weight.is_contiguous() and scale.is_contiguous() and weight.numel() > 0:
+        # one matrix as a checkpoint holds it: none of the views below, which take the host longer than the GPU needs
+        launch.submit(_lib.JOB_FP8_TO_MXFP8, weight, q, out_scale, scale, None, n, k, scale.shape[1])
+        return q, out_scale
+    w3, s3, nt, _kt = _grids(weight, scale)
     q3, o3 = q.view(w3.shape[0], n, k), out_scale.view(w3.shape[0], n, k // MXFP8_GROUP_SIZE)
     for b in range(w3.shape[0] if n and k else 0):
         launch.submit(_lib.JOB_FP8_TO_MXFP8, w3[b], q3[b], o3[b], s3[b], None, n, k,
