@@ -259,7 +259,7 @@ int mq_nvfp4_fake_quant(const mq_fake_quant_item* list, int64_t n, int dtype, vo
  *      16-byte aligned input; p0 = bit pattern of 1e-12 rounded to the weight dtype; p1 = 0 or MQ_NVFP4_CARRY_AMAX)
  *   MQ_JOB_INT4_PACK_ASYM       w             int32 words   scales (dtype) aux = uint8 zero points,    group, -
  *                                                                          aux2 = int32 packed_zp
- *     (mq_int4_group_quant_pack_asym; bf16 or fp16 tensors on a 16-byte boundary with groups of 32 / 64 / 128 share their two
+ *     (mq_int4_group_quant_pack_asym; tensors on a 16-byte boundary with groups of 32 / 64 / 128 share their two
  *      launches, codes and then packed zero points, with up to MQ_MAX_GROUP tensors)
  *     (mq_ue8m0_pack_scales with mn = rows, kb = cols, row_major = ld; its input is usually the scale output of an
  *      earlier job)
@@ -280,7 +280,7 @@ int mq_nvfp4_fake_quant(const mq_fake_quant_item* list, int64_t n, int dtype, vo
  * ld is the input row stride in elements for the two FP8 quantizers (column stride 1) and ignored elsewhere;
  * rows_per_block / block_stride describe a row-blocked input (see the struct).
  * The three FP8 tile kinds (FP8_BLOCK, FP8_BLOCKWISE_CAST, FP8_BLOCK_POW2), MXFP8, MXFP4, INT4_PACK, INT4_PACK_ASYM, FP8_TENSOR and NVFP4 run their tuned
- * kernels on bf16 and on fp16 inputs, and all but INT4_PACK_ASYM and FP8_TENSOR on fp32 ones as well; consecutive jobs share a
+ * kernels on bf16 and on fp16 inputs, and all but FP8_TENSOR on fp32 ones as well; consecutive jobs share a
  * launch when they also share the input dtype (NVFP4 jobs that share an amax record must have one dtype to take them).
  * NVFP4: the driver reduces every job's tensor into a section of its record and then quantizes; jobs that
  * share one record (a gate/up pair; at most MQ_NVFP4_SECTIONS) must be adjacent in the list.

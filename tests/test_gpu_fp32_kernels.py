@@ -110,6 +110,28 @@ def test_int4_pack_fp32(oracle, shape, group, specials):
     _assert_same(q, q_o, "codes")
 
 
+@pytest.mark.parametrize("group", [32, 64, 128])
+@pytest.mark.parametrize("shape", [(8, 128), (8, 384), (16, 4224), (136, 1024)])
+@pytest.mark.parametrize("specials", [False, True])
+def test_int4_pack_asym_fp32(oracle, shape, group, specials):
+    from miles_amd.kernels.quant.int4_fake import pack_layer
+
+    w = fp32_case(shape, 25 + shape[1] + group)
+    # quotients at and next to a half: multiples of half a scale of 1 (extrema -7 and 8), and their neighbours
+    w[0, :32] = torch.arange(-14, 18) * 0.5
+    w[0, 1:31:3] = torch.nextafter(w[0, 1:31:3], torch.tensor(100.0))
+    if specials:
+        w[1] += 1e4 * w[1].abs().max()        # minima far above zero and far below it: the zero point is clamped, codes carry
+        w[2] -= 1e4 * w[2].abs().max()
+        at = torch.rand(shape, generator=torch.Generator().manual_seed(shape[1])) < 0.002
+        values = torch.tensor(INT4_TOPS + [0.0, -0.0, 1e-45])
+        w = torch.where(at, values[torch.randint(0, len(values), shape, generator=torch.Generator().manual_seed(group))], w)
+        w[-1, -group:] = 0
+        w[-2, -group:] = 3.25
+    for got, want, what in zip(pack_layer(w.to(DEV), group, False), oracle.pack_layer(w, group, False), ("codes", "scales", "zero points")):
+        _assert_same(got, want, what)
+
+
 @pytest.mark.parametrize("shape", FLAT_SHAPES)
 @pytest.mark.parametrize("specials", [False, True])
 def test_mxfp4_fp32(oracle, shape, specials):
@@ -153,7 +175,7 @@ def test_nvfp4_fp32(oracle, monkeypatch, shape, mode):
         _assert_same(q, q_o, "codes")
 
 
-@pytest.mark.parametrize("kind", ["int4", "mxfp4", "nvfp4"])
+@pytest.mark.parametrize("kind", ["int4", "int4_asym", "mxfp4", "nvfp4"])
 def test_fp32_in_one_list_with_16_bit_tensors(oracle, kind):
     """A recorded list of seventy-odd tensors (more than the kernel arguments of a launch hold), run twice."""
     from miles_amd import launch
@@ -162,9 +184,10 @@ def test_fp32_in_one_list_with_16_bit_tensors(oracle, kind):
     from miles_amd.utils.nvfp4 import nvfp4_quantize_1d
 
     here, there = {"int4": (lambda t: pack_layer(t, 32)[:2], lambda t: oracle.pack_layer(t, 32)[:2]),
+                   "int4_asym": (lambda t: pack_layer(t, 32, False), lambda t: oracle.pack_layer(t, 32, False)),
                    "mxfp4": (lambda t: quantize_mxfp4(t, 32), lambda t: oracle.quantize_mxfp4(t, 32)),
                    "nvfp4": (lambda t: nvfp4_quantize_1d(t)[:2], lambda t: oracle.nvfp4_quantize_1d(t)[:2])}[kind]
-    tensors = [fp32_case((33, 160), 60 + i) for i in range(72)]
+    tensors = [fp32_case((40, 160), 60 + i) for i in range(72)]
     tensors[5], tensors[6] = tensors[5].bfloat16(), tensors[6].half()
     dev = [t.to(DEV) for t in tensors]
     with launch.recording() as batch:
