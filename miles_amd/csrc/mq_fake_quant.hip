@@ -11,7 +11,7 @@
 //   out = dtype(q * scale)
 // A power-of-two scale makes x / scale exact, so it is a multiplication by the reciprocal power.  The hardware
 // conversions saturate / round exactly as clamp-then-round does for the one or two ulp by which |x / scale| can
-// exceed the format maximum.  Lanes own 8 consecutive elements; 4 (or 2) neighbouring lanes form a block.
+// exceed the format maximum.  Lanes own 16 consecutive bytes; 4 (or 2) neighbouring lanes form a block, of fp32 twice as many.
 #include "mq_api_internal.hpp"
 #include "mq_common.hpp"
 #include "mq_group.hpp"
@@ -26,63 +26,64 @@ __device__ __forceinline__ float ceil_pow2_normal(float v) {   // v normal and p
     return u2f(((u >> 23) + ((u & 0x7FFFFFu) != 0)) << 23);
 }
 
-// MODE as above; LANES = lanes per block (4 for 1x32, 2 for 1x16)
+// MODE as above; E elements per lane, LANES lanes per block
 template <int DT, int MODE>
 __global__ __launch_bounds__(kFqThreads) void fake_quant_kernel(const void* __restrict__ x, void* __restrict__ y,
                                                                 int64_t units, int chunk) {
-    constexpr int LANES = MODE == 2 ? 2 : 4;
+    constexpr int E = kLaneElems<DT>, LANES = (MODE == 2 ? 16 : 32) / E;
     const int64_t unit = xcd_chunked_block(chunk) * kFqThreads + threadIdx.x;
     const bool live = unit < units;           // a block is a whole number of lanes: dead lanes never share one with live lanes
-    float f[8];
-    fq_load8<DT>(x, live ? unit : units - 1, f);
+    float f[E];
+    fq_load<DT>(x, live ? unit : units - 1, f);
     uint32_t m = 0;
 #pragma unroll
-    for (int i = 0; i < 8; i++) m = umax(m, f2u(f[i]) & 0x7FFFFFFFu);
-    m = LANES == 4 ? group_max4(m) : group_max2(m);
+    for (int i = 0; i < E; i++) m = umax(m, f2u(f[i]) & 0x7FFFFFFFu);
+    m = LANES == 8 ? group_max8(m) : LANES == 4 ? group_max4(m) : group_max2(m);
     const bool finite = m < 0x7F800000u;
-    float amax = u2f(m), scale, q[8];
+    float amax = u2f(m), scale, q[E];
     if (MODE == 2) {
         const float hp = __builtin_fminf(__builtin_fmaxf(amax * u2f(0x3E2AAAABu), 0.001953125f), 448.0f);
         scale = finite ? hw_e4m3x2_decode<false>(hw_e4m3x2<false>(hp, hp, 0u)).x : sw_e4m3fn_decode(sw_e4m3fn(hp));
         const float r = 1.0f / scale;
         const bool fast = DT != MQ_F32;       // 16-bit numerators: the shared-divisor sequence is the exact quotient
 #pragma unroll
-        for (int i = 0; i < 8; i++) q[i] = fast ? div_by_shared(f[i], scale, r) : f[i] / scale;
+        for (int i = 0; i < E; i++) q[i] = fast ? div_by_shared(f[i], scale, r) : f[i] / scale;
     } else {
         amax = __builtin_fmaxf(amax, MODE == 0 ? 1e-4f : u2f(0x01C00000u) /* 6 * 2^-126 */);
         scale = ceil_pow2_normal(amax * u2f(MODE == 0 ? 0x3B124925u : 0x3E2AAAABu));
         const float r = u2f(0x7F000000u - f2u(scale));      // 2^-k for scale = 2^k
 #pragma unroll
-        for (int i = 0; i < 8; i++) q[i] = f[i] * r;
+        for (int i = 0; i < E; i++) q[i] = f[i] * r;
     }
     if (MODE == 0) {
         if (finite) {
-            const uint32_t lo = hw_e4m3x4(q[0], q[1], q[2], q[3]), hi = hw_e4m3x4(q[4], q[5], q[6], q[7]);
-            const f32x2 a = hw_e4m3x2_decode<false>(lo), b = hw_e4m3x2_decode<true>(lo);
-            const f32x2 c = hw_e4m3x2_decode<false>(hi), d = hw_e4m3x2_decode<true>(hi);
-            q[0] = a.x; q[1] = a.y; q[2] = b.x; q[3] = b.y; q[4] = c.x; q[5] = c.y; q[6] = d.x; q[7] = d.y;
+#pragma unroll
+            for (int i = 0; i < E; i += 4) {
+                const uint32_t w = hw_e4m3x4(q[i], q[i + 1], q[i + 2], q[i + 3]);
+                const f32x2 a = hw_e4m3x2_decode<false>(w), b = hw_e4m3x2_decode<true>(w);
+                q[i] = a.x; q[i + 1] = a.y; q[i + 2] = b.x; q[i + 3] = b.y;
+            }
         } else {
 #pragma unroll
-            for (int i = 0; i < 8; i++) q[i] = sw_e4m3fn_decode(sw_e4m3fn_sat(q[i]));
+            for (int i = 0; i < E; i++) q[i] = sw_e4m3fn_decode(sw_e4m3fn_sat(q[i]));
         }
     } else {
-        const bool zero[8] = {q[0] == 0.0f, q[1] == 0.0f, q[2] == 0.0f, q[3] == 0.0f,
-                              q[4] == 0.0f, q[5] == 0.0f, q[6] == 0.0f, q[7] == 0.0f};
-        uint32_t w = 0;
-        w = hw_e2m1x2<0>(q[0], q[1], w);
-        w = hw_e2m1x2<1>(q[2], q[3], w);
-        w = hw_e2m1x2<2>(q[4], q[5], w);
-        w = hw_e2m1x2<3>(q[6], q[7], w);
-        const f32x2 a = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 0), b = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 1);
-        const f32x2 c = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 2), d = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 3);
-        q[0] = a.x; q[1] = a.y; q[2] = b.x; q[3] = b.y; q[4] = c.x; q[5] = c.y; q[6] = d.x; q[7] = d.y;
+        bool zero[E];
+#pragma unroll
+        for (int i = 0; i < E; i++) zero[i] = q[i] == 0.0f;
+#pragma unroll
+        for (int i = 0; i < E; i += 4) {
+            const uint32_t w = hw_e2m1x2<1>(q[i + 2], q[i + 3], hw_e2m1x2<0>(q[i], q[i + 1], 0u));
+            const f32x2 a = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 0), b = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 1);
+            q[i] = a.x; q[i + 1] = a.y; q[i + 2] = b.x; q[i + 3] = b.y;
+        }
         // an exact zero has sign 0 in the reference and comes out as +0; a negative value that rounds to zero keeps its sign
 #pragma unroll
-        for (int i = 0; i < 8; i++) q[i] = zero[i] ? 0.0f : q[i];
+        for (int i = 0; i < E; i++) q[i] = zero[i] ? 0.0f : q[i];
     }
 #pragma unroll
-    for (int i = 0; i < 8; i++) q[i] = q[i] * scale;
-    if (live) fq_store8<DT>(y, unit, q);
+    for (int i = 0; i < E; i++) q[i] = q[i] * scale;
+    if (live) fq_store<DT>(y, unit, q);
 }
 
 
@@ -260,8 +261,8 @@ extern "C" int mq_fake_quant(const void* x, int dtype, void* y, int64_t numel, i
                            (hipStream_t)stream, x, dtype, y, blocks, mode);
         return mq_check_launch("fake quant");
     }
-    const int64_t units = numel / 8;
-    if ((units + kFqThreads - 1) / kFqThreads > 0x7FFFFF00ll) return mq_fail(MQ_ERR_ARG, "tensor too large");
+    if ((numel / 8 + kFqThreads - 1) / kFqThreads > 0x7FFFFF00ll) return mq_fail(MQ_ERR_ARG, "tensor too large");
+    const int64_t units = numel / (dtype == MQ_F32 ? kLaneElems<MQ_F32> : kLaneElems<MQ_BF16>);
     hipStream_t st = (hipStream_t)stream;
     if (mode == 0) launch_fq<0>(x, dtype, y, units, st);
     else if (mode == 1) launch_fq<1>(x, dtype, y, units, st);

@@ -794,7 +794,7 @@ __global__ __launch_bounds__(256) void int4_zero_pack_group_kernel(const Table t
 // `out` holds the integer codes as values of the input dtype, `scale` (and `zero`) one value per block in that dtype.
 //   symmetric:  s = max(amax * f32(1/7), 1e-5);   out = rint(x / s)
 //   asymmetric: s = max((max - min) * f32(1/15), 1e-5);   z = min(max(-rint(min / s), +0), 15);   out = rint(x / s) + z
-// Lanes own 8 consecutive elements, G / 8 neighbouring lanes a block; x / s is the exact quotient (shared-divisor
+// Lanes own 16 consecutive bytes, the neighbouring lanes of G elements a block; x / s is the exact quotient (shared-divisor
 // sequence for 16-bit inputs, the sign of a -0 numerator put back; the division itself otherwise).
 template <int DT, int LANES, bool SYM>
 __global__ __launch_bounds__(kI4Threads) void int4_fake_rows_kernel(const void* __restrict__ x, void* __restrict__ out,
@@ -802,24 +802,25 @@ __global__ __launch_bounds__(kI4Threads) void int4_fake_rows_kernel(const void* 
                                                                     void* __restrict__ zero_out, int64_t units, int chunk) {
     const int64_t unit = xcd_chunked_block(chunk) * kI4Threads + threadIdx.x;
     const bool live = unit < units;            // a block is a whole number of lanes: dead lanes never share one with live lanes
-    float f[8], q[8];
-    fq_load8<DT>(x, live ? unit : units - 1, f);
+    constexpr int E = kLaneElems<DT>;
+    float f[E], q[E];
+    fq_load<DT>(x, live ? unit : units - 1, f);
     float mx, mn = 0.0f, s, zero = 0.0f;
     if (SYM) {
         mx = __builtin_fabsf(f[0]);
 #pragma unroll
-        for (int i = 1; i < 8; i++) mx = __builtin_fmaxf(mx, __builtin_fabsf(f[i]));
-        mx = mx != mx ? 0.0f : mx;             // eight NaNs in one lane: fmaxf over the group skips them
-        mx = u2f(seg_max<LANES>(f2u(mx)));     // non-negative floats order like their bit patterns
+        for (int i = 1; i < E; i++) mx = __builtin_fmaxf(mx, __builtin_fabsf(f[i]));
+        mx = mx != mx ? 0.0f : mx;             // a lane of NaNs: fmaxf over the group skips them
+        mx = u2f(seg_max32<LANES>(f2u(mx)));     // non-negative floats order like their bit patterns
         s = __builtin_fmaxf(mx * kSymCons, 1e-5f);
     } else {
         mx = mn = f[0];
 #pragma unroll
-        for (int i = 1; i < 8; i++) { mx = __builtin_fmaxf(mx, f[i]); mn = __builtin_fminf(mn, f[i]); }
-        mx = mx != mx ? -__builtin_inff() : mx;     // eight NaNs in one lane: the group reduction skips them
+        for (int i = 1; i < E; i++) { mx = __builtin_fmaxf(mx, f[i]); mn = __builtin_fminf(mn, f[i]); }
+        mx = mx != mx ? -__builtin_inff() : mx;     // a lane of NaNs: the group reduction skips them
         mn = mn != mn ? __builtin_inff() : mn;
-        mx = order_unkey(seg_max<LANES>(order_key(mx)));
-        mn = order_unkey(~seg_max<LANES>(~order_key(mn)));
+        mx = order_unkey(seg_max32<LANES>(order_key(mx)));
+        mn = order_unkey(~seg_max32<LANES>(~order_key(mn)));
         s = __builtin_fmaxf((mx - mn) * kAsymCons, 1e-5f);
         // max(-0, +0) is +0 in the reference's device code: adding +0 makes that explicit
         zero = __builtin_fminf(__builtin_fmaxf(-__builtin_rintf(mn / s), 0.0f), 15.0f) + 0.0f;
@@ -828,17 +829,17 @@ __global__ __launch_bounds__(kI4Threads) void int4_fake_rows_kernel(const void* 
     const float top = SYM ? mx : __builtin_fmaxf(__builtin_fabsf(mx), __builtin_fabsf(mn));
     if (DT != MQ_F32 && shared_div_ok(s) && top * y < 1e30f) {
 #pragma unroll
-        for (int i = 0; i < 8; i++) q[i] = __builtin_rintf(div_by_shared(f[i], s, y));
+        for (int i = 0; i < E; i++) q[i] = __builtin_rintf(div_by_shared(f[i], s, y));
     } else {
 #pragma unroll
-        for (int i = 0; i < 8; i++) q[i] = __builtin_rintf(f[i] / s);
+        for (int i = 0; i < E; i++) q[i] = __builtin_rintf(f[i] / s);
     }
     if (!SYM) {
 #pragma unroll
-        for (int i = 0; i < 8; i++) q[i] = q[i] + zero;
+        for (int i = 0; i < E; i++) q[i] = q[i] + zero;
     }
     if (!live) return;
-    fq_store8<DT>(out, unit, q);
+    fq_store<DT>(out, unit, q);
     if ((threadIdx.x & (LANES - 1)) == 0) {
         store_dtype(scale_out, unit / LANES, s, DT);
         if (!SYM) store_dtype(zero_out, unit / LANES, zero, DT);
@@ -950,8 +951,11 @@ static void launch_fake_rows_sym(const void* x, void* out, void* scale, void* ze
 template <int DT>
 static void launch_fake_rows_dt(const void* x, void* out, void* scale, void* zero, int64_t units, int lanes, bool sym,
                                 int chunk, unsigned blocks, hipStream_t st) {
+    if constexpr (DT == MQ_F32) {
+        if (lanes == 32) return launch_fake_rows_sym<DT, 32>(x, out, scale, zero, units, sym, chunk, blocks, st);
+    }
     if (lanes == 16) launch_fake_rows_sym<DT, 16>(x, out, scale, zero, units, sym, chunk, blocks, st);
-    else if (lanes == 8) launch_fake_rows_sym<DT, 8>(x, out, scale, zero, units, sym, chunk, blocks, st);
+    else if (DT == MQ_F32 || lanes == 8) launch_fake_rows_sym<DT, 8>(x, out, scale, zero, units, sym, chunk, blocks, st);
     else launch_fake_rows_sym<DT, 4>(x, out, scale, zero, units, sym, chunk, blocks, st);
 }
 static void launch_fake_rows(const void* x, int dtype, void* out, void* scale, void* zero, int64_t units, int lanes,
@@ -971,11 +975,12 @@ extern "C" int mq_int4_fake_quant(const void* x, int dtype, void* out, void* sca
     const bool rows_fast = block_m == 1 && (block_n == 32 || block_n == 64 || block_n == 128) &&
                            N % block_n == 0 && ((((uintptr_t)x | (uintptr_t)out)) & 15) == 0 && M * (N / 8) < (1ll << 38);
     if (rows_fast) {
-        const int64_t units = M * (N / 8);
+        const int elems = dtype == MQ_F32 ? kLaneElems<MQ_F32> : kLaneElems<MQ_BF16>;
+        const int64_t units = M * (N / elems);
         int64_t blocks = (units + kI4Threads - 1) / kI4Threads;
         const int chunk = (int)flat_chunk(blocks);
         blocks = flat_padded(blocks, chunk);
-        launch_fake_rows(x, dtype, out, scale, zero, units, block_n / 8, sym != 0, chunk, (unsigned)blocks, (hipStream_t)stream);
+        launch_fake_rows(x, dtype, out, scale, zero, units, block_n / elems, sym != 0, chunk, (unsigned)blocks, (hipStream_t)stream);
         return mq_check_launch("int4 fake quant");
     }
     const int64_t gpr = (N + block_n - 1) / block_n;

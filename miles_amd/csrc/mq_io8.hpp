@@ -1,5 +1,8 @@
-// Eight consecutive elements of a bf16 / fp16 / fp32 tensor as floats, and back: the per-lane unit of the row-wise
-// kernels (16 bytes of a 16-bit tensor, 32 bytes of an fp32 one).
+// Eight consecutive elements of a bf16 / fp16 / fp32 tensor as floats, and back (16 bytes of a 16-bit tensor, 32 bytes of an
+// fp32 one), and the 16-byte unit that row-wise kernels give a lane: eight elements of a 16-bit tensor, four of an fp32 one.
+// (With eight fp32 elements a lane, two loads and two stores 32 bytes apart, every instruction covers half of each of its
+// lines: on [16384, 4096] fp32 fake INT4 quantization ran at 5.0-5.1 TB/s, 6.4-6.5 with four, block fake quantization at
+// 5.3-5.4, 6.5 with four.)
 #pragma once
 #include "mq_api_internal.hpp"
 #include "mq_common.hpp"
@@ -44,6 +47,19 @@ __device__ __forceinline__ void fq_store8(void* y, int64_t unit, const float f[8
         }
         st16((uint16_t*)y + unit * 8, u32x4{p[0], p[1], p[2], p[3]});
     }
+}
+
+template <int DT> constexpr int kLaneElems = DT == MQ_F32 ? 4 : 8;
+template <int DT>
+__device__ __forceinline__ void fq_load(const void* x, int64_t unit, float f[]) {
+    if (DT != MQ_F32) return fq_load8<DT>(x, unit, f);
+    const u32x4 a = ld16((const float*)x + unit * 4);
+    f[0] = u2f(a.x); f[1] = u2f(a.y); f[2] = u2f(a.z); f[3] = u2f(a.w);
+}
+template <int DT>
+__device__ __forceinline__ void fq_store(void* y, int64_t unit, const float f[]) {
+    if (DT != MQ_F32) return fq_store8<DT>(y, unit, f);
+    st16((float*)y + unit * 4, u32x4{f2u(f[0]), f2u(f[1]), f2u(f[2]), f2u(f[3])});
 }
 
 }  // namespace mq

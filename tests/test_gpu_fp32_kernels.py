@@ -175,6 +175,34 @@ def test_nvfp4_fp32(oracle, monkeypatch, shape, mode):
         _assert_same(q, q_o, "codes")
 
 
+@pytest.mark.parametrize("shape", [(1, 32), (5, 96), (1, 1024), (1, 1056), (129, 2016)])
+@pytest.mark.parametrize("kind", ["fp8", "fp4", "kv"])
+def test_fake_quant_fp32(oracle, shape, kind):
+    """A workgroup covers 1024 elements, a lane four."""
+    from miles_amd.kernels.quant import fake_quant as fq
+
+    forward = {"fp8": fq.fake_quant_fp8_forward, "fp4": fq.fake_quant_fp4_forward, "kv": fq.fake_quant_compressed_kv_forward}[kind]
+    w = fp32_case(shape, 70 + shape[1])
+    w[0, :6] = torch.tensor([0.0, -0.0, 1e-45, -1e-45, 3e38, -1e-30])
+    _assert_same(forward(w.to(DEV)), oracle.fake_quant(w, {"kv": "compressed_kv"}.get(kind, kind)), kind)
+
+
+@pytest.mark.parametrize("shape", [(1, 128), (5, 384), (1, 1152), (129, 2048)])
+@pytest.mark.parametrize("group", [32, 64, 128])
+@pytest.mark.parametrize("sym", [True, False])
+def test_fake_int4_fp32(oracle, shape, group, sym):
+    from miles_amd.kernels.quant.int4_fake import fake_int4_quant_cuda
+
+    w = fp32_case(shape, 80 + shape[1] + group)
+    w[-1, :group] = 0
+    w[0, 1:5] = float("nan")           # a lane of NaNs, skipped by the extrema, in part of the groups
+    if group > 32:
+        w[0, 4:8] = float("nan")
+    got, want = fake_int4_quant_cuda(w.to(DEV), (1, group), sym), oracle.fake_int4_quant(w, (1, group), sym)
+    for a, b, what in list(zip(got, want, ("codes", "scales", "zero points")))[: 2 if sym else 3]:
+        _assert_same(a.nan_to_num(nan=77.0), b.nan_to_num(nan=77.0), what)
+
+
 @pytest.mark.parametrize("kind", ["int4", "int4_asym", "mxfp4", "nvfp4"])
 def test_fp32_in_one_list_with_16_bit_tensors(oracle, kind):
     """A recorded list of seventy-odd tensors (more than the kernel arguments of a launch hold), run twice."""
