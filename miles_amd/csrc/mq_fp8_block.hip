@@ -603,7 +603,7 @@ __global__ __launch_bounds__(256) void fp8_tensor_quant_bf16_kernel(const uint16
 // the tensor, is moved back to end with it, so that it codes a few elements a second time, to the same bytes.
 // HBM-bound; fp32 quotients come correctly rounded from div24_by_shared where that matters to an e4m3 code.  Eight tensors in
 // eight calls, three launches each per tensor and one per channel (the two element-wise passes before): per tensor
-// [2048, 4096] fp32 381 -> 173 us, [2049, 4099] bf16 379 -> 148; per channel 198 -> 118 and 209 -> 116, which is the host's
+// [2048, 4096] fp32 381 -> 149 us, [2049, 4099] bf16 379 -> 135; per channel 198 -> 118 and 209 -> 116, which is the host's
 // time for eight calls.
 template <int DT> constexpr int kUnitElems = DT == MQ_F32 ? 4 : 8;
 template <int DT>
@@ -705,9 +705,15 @@ __global__ __launch_bounds__(256) void fp8_channel_any_kernel(const void* __rest
 }
 // per tensor: amax pass (one atomic max per workgroup on the fp32 pattern) and flat quantize pass over n contiguous elements
 constexpr int kTensorAnyLoads = 4, kTensorAnyUnits = 2;
-constexpr int kTensorAnyMaxBlocks = 512;      // of the amax pass: its atomics on one word follow each other at some 8 ns
+// Partial maxima of the amax pass, which the quantize pass folds, a word per lane.  The atomics on one word follow each other at
+// some 8 ns, which 512 workgroups spend at the pass's end: [2048, 4096] fp32 12.5 us with one word, 9.1 to 9.6 with 64.  Those on
+// neighbouring words still meet in one line, so more workgroups pay off only where their loads gain more than that:
+// 512 / 1024 / 2048 of them take 9.6 / 11.1 / 13.6 us there (256: 9.7), but [8192, 16383] bf16 (268 MB) 52 / - / 46.
+// The line lies halfway, at 128 MB (8192 trips of a workgroup).  Looking at the word before the atomic: 13.8 us.
+constexpr int kTensorAnyWords = 64, kTensorAnyBlocks = 512, kTensorAnyManyBlocks = 2048, kTensorAnyManyTrips = 8192;
+static_assert(kTensorAnyWords == kWave, "a wavefront folds the partial maxima with one load");
 template <int DT>
-__global__ __launch_bounds__(256) void fp8_tensor_amax_any_kernel(const void* __restrict__ w, int64_t n, uint32_t* __restrict__ amax_bits) {
+__global__ __launch_bounds__(256) void fp8_tensor_amax_any_kernel(const void* __restrict__ w, int64_t n, uint32_t* __restrict__ amax_bits, uint32_t word_mask) {
     __shared__ uint32_t wave_amax[4];
     constexpr int E = kUnitElems<DT>;
     const int t = threadIdx.x;
@@ -726,11 +732,11 @@ __global__ __launch_bounds__(256) void fp8_tensor_amax_any_kernel(const void* __
     m = wave_max(unit_max_f32<DT>(m));
     if ((t & 63) == 0) wave_amax[t >> 6] = m;
     __syncthreads();
-    if (t == 0) atomicMax(amax_bits, umax(umax(wave_amax[0], wave_amax[1]), umax(wave_amax[2], wave_amax[3])));
+    if (t == 0) atomicMax(amax_bits + (blockIdx.x & word_mask), umax(umax(wave_amax[0], wave_amax[1]), umax(wave_amax[2], wave_amax[3])));
 }
 template <int DT>
 __global__ __launch_bounds__(256) void fp8_tensor_quant_any_kernel(const void* __restrict__ w, int64_t n, const uint32_t* __restrict__ amax_bits,
-                                                                   float floor_v, uint8_t* __restrict__ q, float* __restrict__ scale, int chunk) {
+                                                                   uint32_t word_mask, float floor_v, uint8_t* __restrict__ q, float* __restrict__ scale, int chunk) {
     constexpr int E = kUnitElems<DT>;
     const int64_t base = xcd_chunked_block(chunk) * (256 * kTensorAnyUnits) + threadIdx.x;
     u32x4 v[kTensorAnyUnits];
@@ -739,7 +745,7 @@ __global__ __launch_bounds__(256) void fp8_tensor_quant_any_kernel(const void* _
         const int64_t at = (base + i * 256) * E;
         v[i] = ld_unit<DT>(w, at < n - E ? at : n - E);
     }
-    const uint32_t abits = amax_bits[0];
+    const uint32_t abits = wave_max(amax_bits[threadIdx.x & word_mask]);
     float amax = u2f(abits);
     if (amax < floor_v) amax = floor_v;
     const float s = amax / kFp8Max, y = 1.0f / s;
@@ -1062,13 +1068,16 @@ static bool fp8_scaled_any(const void* w, int64_t ldw, uint8_t* q, float* scale,
     const int64_t n = M * K, units = (n + E - 1) / E;
     if ((ldw != K && M != 1) || n < E || units >= (1ll << 38)) return false;
     const int64_t trips = (units + 256 * kTensorAnyLoads - 1) / (256 * kTensorAnyLoads);
-    hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, amax_ws, 0u, 1);
-    hipLaunchKernelGGL(fp8_tensor_amax_any_kernel<DT>, dim3((unsigned)(trips < kTensorAnyMaxBlocks ? trips : kTensorAnyMaxBlocks)), dim3(256), 0,
-                       st, w, n, amax_ws);
+    // (the workspace holds a word per row, that of the static form 64 for a tensor)
+    const int words = M >= kTensorAnyWords ? kTensorAnyWords : 1;
+    const int64_t cap = words > 1 && trips > kTensorAnyManyTrips ? kTensorAnyManyBlocks : kTensorAnyBlocks;
+    const uint32_t word_mask = (uint32_t)words - 1u;
+    hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, amax_ws, 0u, words);
+    hipLaunchKernelGGL(fp8_tensor_amax_any_kernel<DT>, dim3((unsigned)(trips < cap ? trips : cap)), dim3(256), 0, st, w, n, amax_ws, word_mask);
     const int64_t blocks = (units + 256 * kTensorAnyUnits - 1) / (256 * kTensorAnyUnits);
     const int chunk = (int)flat_chunk(blocks);
     hipLaunchKernelGGL(fp8_tensor_quant_any_kernel<DT>, dim3((unsigned)flat_padded(blocks, chunk)), dim3(256), 0, st, w, n, amax_ws,
-                       floor_v, q, scale, chunk);
+                       word_mask, floor_v, q, scale, chunk);
     return true;
 }
 

@@ -143,6 +143,20 @@ def test_tensor_scale_of_many_workgroups(oracle):  # noqa: F811
         _assert_same(q, q_o, f"{dtype} codes")
 
 
+@pytest.mark.parametrize("shape,dtype", [((63, 1027), torch.float32), ((64, 1027), torch.float32), ((65, 515), torch.bfloat16),
+                                         ((64, 1), torch.float16), ((4097, 16387), torch.bfloat16)])
+def test_tensor_scale_of_many_partial_maxima(oracle, shape, dtype):  # noqa: F811
+    """The rows from which the amax pass has 64 words, and the size from which it has 2048 workgroups; the maximum comes last."""
+    from miles_amd.tools.convert_hf_to_fp8 import tensor_fp8
+
+    w = torch.randn(shape, generator=torch.Generator(device=DEV).manual_seed(7), device=DEV).to(dtype)
+    w[-1, -1] = -2 * w.abs().max()
+    q, s = tensor_fp8(w)
+    q_o, s_o = oracle.tensor_fp8(w.cpu())
+    _assert_same(s, s_o, f"{shape} {dtype} scale")
+    _assert_same(q, q_o, f"{shape} {dtype} codes")
+
+
 @pytest.mark.parametrize("block", [8, 32, 128])
 def test_dequantize_rows_of_any_width(oracle, block):  # noqa: F811
     """One list of matrices from one unit to several tiles wide, codes at any byte, NaN codes and non-finite scales."""
