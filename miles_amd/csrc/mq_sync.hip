@@ -156,6 +156,9 @@ static int check_job(const mq_job& j) {
         return mq_mxfp4_to_fp8_job(probe, j.in, j.aux, j.out, j.scale, j.rows, j.cols);
     }
     if (!empty && (j.kind == MQ_JOB_FP8_DEQUANT ? !j.aux : !j.scale)) return mq_fail(MQ_ERR_ARG, "job without a scale pointer");
+    // (the grouped kernels store a scale byte wherever a group starts: a last group that is cut short has none of its own)
+    if (j.kind == MQ_JOB_MXFP4 && !empty && (j.p0 <= 0 || (j.rows * j.cols) % j.p0 != 0 || (j.rows * j.cols) % 2 != 0))
+        return mq_fail(MQ_ERR_ARG, "element count must be a multiple of the group size and of 2");
     if (j.kind == MQ_JOB_NVFP4 && !j.aux) return mq_fail(MQ_ERR_ARG, "NVFP4 job without an amax record");
     if (j.kind == MQ_JOB_INT4_PACK_ASYM && !empty && (!j.aux || !j.aux2)) return mq_fail(MQ_ERR_ARG, "asymmetric INT4 job without zero-point outputs");
     if (j.kind == MQ_JOB_FP8_TENSOR) {

@@ -3,6 +3,7 @@
 import ctypes
 
 import pytest
+import torch
 
 from miles_amd import _lib
 
@@ -17,3 +18,27 @@ def test_unknown_dtype(kind, dtype):
     # (addresses that are aligned for every kernel and never read)
     job = (_lib.Job * 1)(_lib.Job(kind, dtype, 1 << 20, 1 << 21, 1 << 22, None, None, 256, 256, 256, block, block, 0, 0))
     assert _lib.load().mq_run_jobs(ctypes.byref(job), 1, None) == MQ_ERR_ARG
+
+
+def _addresses(nbytes):
+    """Three buffers of `nbytes` that a job may name: real ones where a GPU is visible, so that a job which is not refused
+    shows as a wrong answer and not as a fault; elsewhere numbers (aligned for every kernel) that nothing can read."""
+    if not torch.cuda.is_available():
+        return [None, 1 << 20, 1 << 21, 1 << 22]
+    keep = torch.zeros(3, nbytes, dtype=torch.uint8, device="cuda")
+    return [keep, *(row.data_ptr() for row in keep)]
+
+
+def _run(kind, dtype, rows, cols, p0, p1=0):
+    keep, inp, out, scale = _addresses(max(1 << 16, rows * cols * 8))
+    record = torch.zeros(1280, dtype=torch.int32, device="cuda" if keep is not None else "cpu")
+    job = (_lib.Job * 1)(_lib.Job(kind, dtype, inp, out, scale, record.data_ptr(), None, rows, cols, cols, p0, p1, 0, 0))
+    return _lib.load().mq_run_jobs(ctypes.byref(job), 1, None)
+
+
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+@pytest.mark.parametrize("rows, cols, group", [(1, 40, 32), (3, 16, 32), (5, 72, 32), (1, 33, 33), (3, 32, 64), (2, 32, 0)])
+def test_mxfp4_element_counts(dtype, rows, cols, group):
+    """Elements that are no whole number of groups, or odd in number: refused as mq_mxfp4_quant refuses them, whatever the
+    dtype and however the job would have been launched."""
+    assert _run(_lib.JOB_MXFP4, dtype, rows, cols, group) == MQ_ERR_ARG
