@@ -1064,10 +1064,6 @@ bool mq_nvfp4_fast_ok(const void* w, int dtype, const void* q) {
     return dtype >= MQ_BF16 && dtype <= MQ_F32 && ((uintptr_t)w % 16) == 0 && ((uintptr_t)q % 4) == 0;
 }
 
-// the dtype of a launch's tensors rides in the flags word of the launch helpers below (not public flags)
-constexpr int kNvFlagF16 = 1 << 30, kNvFlagF32 = 1 << 29;
-static int nv_dtype_flag(int dtype) { return dtype == MQ_F32 ? kNvFlagF32 : dtype == MQ_F16 ? kNvFlagF16 : 0; }
-
 // tab.job[i]: w, aux = amax record, section, units = numel / 8, s = (void*)numel; every tensor of the one dtype
 int mq_nvfp4_amax_launch_group(int dtype, FlatTable& tab, hipStream_t st) {
     const dim3 grid(kSectionWords, (unsigned)tab.n), blk(256);
@@ -1121,30 +1117,32 @@ static void launch_nvfp4_quant_f32(const Table& tab, int flags, float numer, dim
     }
 }
 template <int PASS, class Table>
-static void launch_nvfp4_quant(const Table& tab, int flags, float numer, dim3 grid, hipStream_t st) {
-    if (PASS == 0 && (flags & kNvFlagF32)) launch_nvfp4_quant_f32(tab, flags, numer, grid, st);
-    else if (flags & kNvFlagF16) launch_nvfp4_quant_dtype<PASS, Table, 1>(tab, flags, numer, grid, st);
+static void launch_nvfp4_quant(int dtype, const Table& tab, int flags, float numer, dim3 grid, hipStream_t st) {
+    // (fp32 has no instances of passes 1 and 2: nvfp4_quant_launch refuses mode 2 for it)
+    if (PASS == 0 && dtype == MQ_F32) launch_nvfp4_quant_f32(tab, flags, numer, grid, st);
+    else if (dtype == MQ_F16) launch_nvfp4_quant_dtype<PASS, Table, 1>(tab, flags, numer, grid, st);
     else launch_nvfp4_quant_dtype<PASS, Table, 0>(tab, flags, numer, grid, st);
 }
 
 // fold + quantize (+ second pass) over a table whose grid is known: tab.chunk / tab.max_blocks are set
 template <class Table>
-static int nvfp4_quant_launch(const Table& tab, int n, int e4m3_max, int flags, int mode, hipStream_t st) {
+static int nvfp4_quant_launch(int dtype, const Table& tab, int n, int e4m3_max, int flags, int mode, hipStream_t st) {
+    if (mode == 2 && dtype == MQ_F32) return mq_fail(MQ_ERR_ARG, "a carried-over amax is for bf16 and fp16 tensors");
     const float numer = (float)e4m3_max * 6.0f;
     const dim3 folds((unsigned)n), blk(256);
     const dim3 grid((unsigned)tab.max_blocks, (unsigned)n);
     if (mode == 2) {
-        if (tab.max_blocks > 0) launch_nvfp4_quant<1>(tab, flags, numer, grid, st);
+        if (tab.max_blocks > 0) launch_nvfp4_quant<1>(dtype, tab, flags, numer, grid, st);
         hipLaunchKernelGGL((nvfp4_fold_kernel<2, Table>), folds, blk, 0, st, tab, numer, mq_amax_feedback(), mq_amax_feedback_mirror());
         if (tab.max_blocks > 0) {
             const unsigned redo_blocks = tab.max_blocks < kSectionWords ? (unsigned)tab.max_blocks : (unsigned)kSectionWords;
-            launch_nvfp4_quant<2>(tab, flags, numer, dim3(redo_blocks, (unsigned)n), st);
+            launch_nvfp4_quant<2>(dtype, tab, flags, numer, dim3(redo_blocks, (unsigned)n), st);
         }
         return mq_check_launch("nvfp4 quant (carried-over amax)");
     }
     if (mode == 1) hipLaunchKernelGGL((nvfp4_fold_kernel<1, Table>), folds, blk, 0, st, tab, numer, mq_amax_feedback(), mq_amax_feedback_mirror());
     else hipLaunchKernelGGL((nvfp4_fold_kernel<0, Table>), folds, blk, 0, st, tab, numer, (uint32_t*)nullptr, (uint32_t*)nullptr);
-    if (tab.max_blocks > 0) launch_nvfp4_quant<0>(tab, flags, numer, grid, st);
+    if (tab.max_blocks > 0) launch_nvfp4_quant<0>(dtype, tab, flags, numer, grid, st);
     return mq_check_launch("nvfp4 quant");
 }
 
@@ -1158,7 +1156,7 @@ static int nvfp4_quant_launch(const Table& tab, int n, int e4m3_max, int flags, 
 int mq_nvfp4_quant_launch_group(int dtype, FlatTable& tab, int e4m3_max, int flags, int mode, hipStream_t st) {
     const int fos = flags & MQ_NVFP4_4OVER6;
     if (!flat_grid(tab, dtype == MQ_F32 ? nv_f32_units_per_block(fos) : nv_units_per_block(fos))) return mq_fail(MQ_ERR_ARG, "tensor too large");
-    return nvfp4_quant_launch(tab, tab.n, e4m3_max, flags | nv_dtype_flag(dtype), mode, st);
+    return nvfp4_quant_launch(dtype, tab, tab.n, e4m3_max, flags, mode, st);
 }
 // modes 1 and 2 over n descriptors of a device table (standard block scaling only); max_units: the largest tensor's units
 int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int e4m3_max, int mode,
@@ -1166,7 +1164,7 @@ int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, in
     FlatRef ref{device_jobs, 0, 0};
     if (!flat_grid(ref, max_units, dtype == MQ_F32 ? nv_f32_units_per_block(0) : kNvThreads * kNvUnroll)) return mq_fail(MQ_ERR_ARG, "tensor too large");
     if (n == 0) return MQ_OK;
-    return nvfp4_quant_launch(ref, n, e4m3_max, nv_dtype_flag(dtype), mode, st);
+    return nvfp4_quant_launch(dtype, ref, n, e4m3_max, 0, mode, st);
 }
 
 // Whether a chunk of NVFP4 jobs (standard scaling, packed kernels, no carried amax) takes the one-pass form.  `slots` is the

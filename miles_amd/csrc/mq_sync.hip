@@ -125,6 +125,10 @@ static bool job_any(const mq_job& j) {
 enum JobPath { kSinglePath, kFastPath, kAnyPath };
 static JobPath job_path(const mq_job& j) { return job_fast(j) ? kFastPath : job_any(j) ? kAnyPath : kSinglePath; }
 
+// flags of an NVFP4 job that the driver acts on itself, and those that mq_nvfp4_quant knows
+constexpr int kNvDriverFlags = MQ_NVFP4_CARRY_AMAX | MQ_NVFP4_NO_WAIT;
+constexpr int kNvQuantFlags = MQ_NVFP4_4OVER6 | MQ_NVFP4_ERR_MSE | MQ_NVFP4_ERR_FP16;
+
 static int64_t copy_dst_pitch(const mq_job& j);
 static int check_job(const mq_job& j) {
     if (j.kind < MQ_JOB_FP8_BLOCK || j.kind > MQ_JOB_MXFP4_DEQUANT) return mq_fail(MQ_ERR_ARG, "unknown job kind");
@@ -159,6 +163,7 @@ static int check_job(const mq_job& j) {
     // (the grouped kernels store a scale byte wherever a group starts: a last group that is cut short has none of its own)
     if (j.kind == MQ_JOB_MXFP4 && !empty && (j.p0 <= 0 || (j.rows * j.cols) % j.p0 != 0 || (j.rows * j.cols) % 2 != 0))
         return mq_fail(MQ_ERR_ARG, "element count must be a multiple of the group size and of 2");
+    if (j.kind == MQ_JOB_NVFP4 && (j.p1 & ~(kNvQuantFlags | kNvDriverFlags))) return mq_fail(MQ_ERR_ARG, "unknown NVFP4 flag");
     if (j.kind == MQ_JOB_NVFP4 && !j.aux) return mq_fail(MQ_ERR_ARG, "NVFP4 job without an amax record");
     if (j.kind == MQ_JOB_INT4_PACK_ASYM && !empty && (!j.aux || !j.aux2)) return mq_fail(MQ_ERR_ARG, "asymmetric INT4 job without zero-point outputs");
     if (j.kind == MQ_JOB_FP8_TENSOR) {
@@ -348,9 +353,6 @@ static int run_fp8_tensor(const mq_job* jobs, int64_t i, int64_t j, const FlatJo
     return MQ_OK;
 }
 
-// flags of an NVFP4 job that the driver acts on itself
-constexpr int kNvDriverFlags = MQ_NVFP4_CARRY_AMAX | MQ_NVFP4_NO_WAIT;
-
 // NVFP4 run [i, j): all jobs fast or not, processed as amax-phase then quantize-phase per chunk
 // (`table`: the device descriptors of jobs[0..), or null; n_all: length of the whole list, for the section lookup)
 static int run_nvfp4(const mq_job* jobs, int64_t n_all, int64_t i, int64_t j, const FlatJob* table, void* stream) {
@@ -384,7 +386,7 @@ static int run_nvfp4(const mq_job* jobs, int64_t n_all, int64_t i, int64_t j, co
             return true;
         };
         // a device table lifts the limit for standard block scaling when every job takes the packed kernels
-        const bool standard = (jobs[i].p1 & (MQ_NVFP4_4OVER6 | MQ_NVFP4_ERR_MSE | MQ_NVFP4_ERR_FP16)) == 0;
+        const bool standard = (jobs[i].p1 & kNvQuantFlags) == 0;
         int64_t k = form(table && standard ? kTableGroup : kMaxGroup);
         bool all_fast = all_fast_in(k);
         if (k - i > kMaxGroup && !all_fast) {

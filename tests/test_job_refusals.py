@@ -42,3 +42,11 @@ def test_mxfp4_element_counts(dtype, rows, cols, group):
     """Elements that are no whole number of groups, or odd in number: refused as mq_mxfp4_quant refuses them, whatever the
     dtype and however the job would have been launched."""
     assert _run(_lib.JOB_MXFP4, dtype, rows, cols, group) == MQ_ERR_ARG
+
+
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+@pytest.mark.parametrize("flag", [1 << 5, 1 << 28, 1 << 29, 1 << 30, -(1 << 31)])
+def test_nvfp4_unknown_flags(dtype, flag):
+    """Bits that mq_nvfp4_quant does not know: refused for jobs as well, never handed on to a kernel's launcher."""
+    assert _run(_lib.JOB_NVFP4, dtype, 16, 32, 448, flag) == MQ_ERR_ARG
+    assert _run(_lib.JOB_NVFP4, dtype, 16, 32, 448, flag | _lib.NVFP4_CARRY_AMAX | _lib.NVFP4_4OVER6) == MQ_ERR_ARG
