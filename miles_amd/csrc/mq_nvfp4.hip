@@ -875,8 +875,16 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_f32_kernel(const Table
         const float denom_inv = 1.0f / denom;
         nv_fill_scale_table(scale_table, (int)t, amax, gs.s_dec, false, denom, denom_inv);
         __syncthreads();
-        const NvCandidate16 c = nv_fast_division(amax) != 0 ? nv_four_over_six16<EM, 1, true>(f, u2f(mb), amax, gs, denom, denom_inv, scale_table)
-                                                            : nv_four_over_six16<EM, 0, true>(f, u2f(mb), amax, gs, denom, denom_inv, scale_table);
+        NvCandidate16 c = nv_fast_division(amax) != 0 ? nv_four_over_six16<EM, 1, true>(f, u2f(mb), amax, gs, denom, denom_inv, scale_table)
+                                                      : nv_four_over_six16<EM, 0, true>(f, u2f(mb), amax, gs, denom, denom_inv, scale_table);
+        // the hardware conversion hands a NaN's sign on; the code of a NaN is 7, as in the element-wise kernel
+        if (__builtin_amdgcn_ballot_w64(mb > 0x7F800000u) != 0) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                if (f[j] != f[j]) c.lo &= ~(8u << (4 * j));
+                if (f[8 + j] != f[8 + j]) c.hi &= ~(8u << (4 * j));
+            }
+        }
         if (t < rem) {
             ((uint32_t*)job.q + first)[2 * t] = c.lo;
             ((uint32_t*)job.q + first)[2 * t + 1] = c.hi;
