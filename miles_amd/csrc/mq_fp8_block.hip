@@ -622,9 +622,12 @@ template <int DT>
 __device__ __forceinline__ uint32_t unit_max_f32(uint32_t m) {
     return DT == MQ_F32 ? m : f2u(DT == MQ_F16 ? elem_lo<1>(hmax_u16(m)) : elem_lo<0>(hmax_u16(m)));
 }
-// codes of one unit; ROUNDED: the quotient is rounded to the dtype first (one scale for the whole tensor)
+// codes of one unit; ROUNDED: the quotient is rounded to the dtype first (one scale for the whole tensor).  `plain`: the
+// scale is in the range of the division sequence (shared_div_ok), so no element is infinite or NaN and no quotient exceeds
+// 448 by more than its rounding.  A zero, subnormal (a quotient by its few bits may be far above 448), huge or non-finite
+// scale takes divisions, the clamp and the software conversion.
 template <int DT, bool ROUNDED>
-__device__ __forceinline__ void scaled_unit(const u32x4 v, float s, float y, bool fast_div, bool plain, uint8_t* __restrict__ q) {
+__device__ __forceinline__ void scaled_unit(const u32x4 v, float s, float y, bool plain, uint8_t* __restrict__ q) {
     constexpr int E = kUnitElems<DT>;
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
     float f[E];
@@ -636,7 +639,7 @@ __device__ __forceinline__ void scaled_unit(const u32x4 v, float s, float y, boo
     }
 #pragma unroll
     for (int j = 0; j < E; j++)
-        f[j] = !fast_div ? f[j] / s : DT == MQ_F32 ? div24_by_shared(f[j], s, y) : div_by_shared(f[j], s, y);
+        f[j] = !plain ? f[j] / s : DT == MQ_F32 ? div24_by_shared(f[j], s, y) : div_by_shared(f[j], s, y);
     if (ROUNDED && DT != MQ_F32) {
 #pragma unroll
         for (int j = 0; j < E; j += 2) {
@@ -654,7 +657,7 @@ __device__ __forceinline__ void scaled_unit(const u32x4 v, float s, float y, boo
     if (plain) {
         o.x = hw_e4m3x4(f[0], f[1], f[2], f[3]);
         if (E == 8) o.y = hw_e4m3x4(f[E - 4], f[E - 3], f[E - 2], f[E - 1]);
-    } else {                                  // inf / NaN, or a zero scale: clamp and convert in software
+    } else {
 #pragma unroll
         for (int j = 0; j < E; j++) {
             const uint32_t c = sw_e4m3fn(clamp_keep_nan(f[j], -kFp8Max, kFp8Max)) << (8 * (j & 3));
@@ -694,13 +697,13 @@ __global__ __launch_bounds__(256) void fp8_channel_any_kernel(const void* __rest
     float amax = u2f(m);
     if (amax < floor_v) amax = floor_v;
     const float s = amax / kFp8Max, y = 1.0f / s;
-    const bool fast_div = shared_div_ok(s), plain = m < 0x7F800000u && s > 0.0f;
+    const bool plain = shared_div_ok(s);
     if (!row_ok) return;
     if (lane == 0) scale[row] = s;
 #pragma unroll
     for (int u = 0; u < UNITS; u++) {
         const int unit = lane + u * ROWLANES, at = unit * E < last ? unit * E : last;
-        if (unit < units) scaled_unit<DT, false>(v[u], s, y, fast_div, plain, q + row * K + at);
+        if (unit < units) scaled_unit<DT, false>(v[u], s, y, plain, q + row * K + at);
     }
 }
 // per tensor: amax pass (one atomic max per workgroup on the fp32 pattern) and flat quantize pass over n contiguous elements
@@ -749,12 +752,12 @@ __global__ __launch_bounds__(256) void fp8_tensor_quant_any_kernel(const void* _
     float amax = u2f(abits);
     if (amax < floor_v) amax = floor_v;
     const float s = amax / kFp8Max, y = 1.0f / s;
-    const bool fast_div = shared_div_ok(s), plain = abits < 0x7F800000u && s > 0.0f;
+    const bool plain = shared_div_ok(s);
     if (base == 0) scale[0] = s;
 #pragma unroll
     for (int i = 0; i < kTensorAnyUnits; i++) {
         const int64_t at = (base + i * 256) * E;
-        if (at < n) scaled_unit<DT, true>(v[i], s, y, fast_div, plain, q + (at < n - E ? at : n - E));
+        if (at < n) scaled_unit<DT, true>(v[i], s, y, plain, q + (at < n - E ? at : n - E));
     }
 }
 

@@ -180,3 +180,31 @@ def test_dequantize_rows_of_any_width(oracle, block):  # noqa: F811
         outs = [weight_dequant(x, s.to(DEV), block) for _codes, s, x in cases]
     for (codes, s, _x), y in zip(cases, outs):
         _assert_same(y, oracle.weight_dequant(codes, s, block), f"block {block} {tuple(codes.shape)}")
+
+
+@pytest.mark.parametrize("per_channel", [1, 0])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_scales_below_the_normal_range(oracle, dtype, per_channel):  # noqa: F811
+    """With a floor of zero (the entry point takes any) a row of subnormals has a scale that is rounded to a few units in the
+    last place, or to zero: quotients lie far above 448 and are clamped."""
+    from miles_amd import _lib
+
+    w = torch.zeros(8, 15, dtype=torch.float32)
+    for r, units in enumerate([1, 223, 225, 300, 650, 671, 1000, 5000]):
+        w[r] = torch.linspace(-1, 1, 15) * units * 2.0**-149
+    if dtype == torch.bfloat16:
+        w = w * 2.0**16
+    w = w.to(dtype)
+    for host in [w] if per_channel else [w[i:i + 1].contiguous() for i in range(8)]:
+        d = host.to(DEV)
+        q, s = torch.empty(host.shape, dtype=torch.uint8, device=DEV), torch.empty(len(host), device=DEV)
+        ws = torch.empty(8, dtype=torch.int32, device=DEV)
+        _lib.check(_lib.load().mq_fp8_scaled_quant(d.data_ptr(), _lib.DTYPE_CODE[dtype], 15, q.data_ptr(), s.data_ptr(), ws.data_ptr(),
+                                                   len(host), 15, per_channel, 0.0, _lib.stream_ptr(d.device)))
+        amax = host.float().abs().amax(1, keepdim=True)
+        scale = amax / 448
+        want = host.float() / scale
+        want = want.to(dtype).float() if not per_channel else want
+        want = want.clamp(-448, 448).to(torch.float8_e4m3fn)
+        _assert_same(s, scale.reshape(-1), "scales")
+        _assert_same(_one_nan(q.view(torch.float8_e4m3fn)), _one_nan(want), "codes")
