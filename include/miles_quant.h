@@ -295,7 +295,8 @@ int mq_nvfp4_fake_quant(const mq_fake_quant_item* list, int64_t n, int dtype, vo
  * Without that flag, lists of 64 MB and more of bf16 or fp16 tensors with standard block scaling are read once as well when
  * every record's tensors fit the chip's registers twice (20 MB on 256 CUs; 32 MB for one tensor at most): the workgroups
  * of a record keep their share and wait for each other's maxima, for a bounded time, after which a second pass does
- * what is left.  MQ_NVFP4_NO_WAIT in p1 sets that time to zero (it exists to test the second pass; results are the same). */
+ * what is left.  MQ_NVFP4_NO_WAIT in p1: a record's first workgroup, which collects the maxima, does not wait and tells the
+ * others so (it exists to test that exit and the second pass; results are the same). */
 enum {
     MQ_JOB_FP8_BLOCK = 0,
     MQ_JOB_FP8_BLOCKWISE_CAST = 1,

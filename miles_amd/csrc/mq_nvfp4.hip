@@ -670,18 +670,23 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
 //     kOneWords words, each a line of its own, one of which every other workgroup watches with one request at a time.
 //     (With every workgroup watching all slots the polling itself filled the memory channels that hold them: 496 us
 //     instead of 240 on 32 x [2048, 7168].)  No counters, so no atomic read-modify-writes.
-//   every wait ends: after `polls` looks a workgroup leaves its part to the second pass (kRecRedo), the same kernel that
+//   every wait ends: after kOnePolls looks a workgroup leaves its part to the second pass (kRecRedo), the same kernel that
 //     re-quantizes tensors whose carried-over amax moved.  That happens when workgroups of one record cannot all be on
 //     the chip because something else occupies it; workgroups start in order of their ids, so otherwise the oldest
-//     unfinished tensor always gets there.
+//     unfinished tensor always gets there.  A first workgroup that gives up publishes that (kOneGaveUp) in place of the
+//     maximum, and every workgroup that reads it leaves at once: a record that does not fit next to a busy neighbour costs
+//     one wait, not one for each batch of its workgroups that comes to the chip.  32 x [2048, 7168] beside a stream of
+//     [8192, 8192] matrix products: 2.5 ms, 3.0 without that word, 2.35 in two passes (beside one of copies 0.56, 0.56, 0.91).
 // 32 x [2048, 7168] (940 MB of bf16, the four launches together): 312 us in two passes, 228 us this way (5.3 TB/s); the
 // same without the wait 198 us.  24 units per lane at four workgroups per CU: 239; 8 units in 512 lanes: 242.
 constexpr int kOneThreads = 256, kOneUnits = 16, kOneWavesPerSimd = 5;
 constexpr int64_t kOnePerBlock = kOneThreads * kOneUnits;
 constexpr int kOneSlots = 2 * kSectionWords;         // 16-bit slots of a section
-constexpr uint32_t kOneFull = 0x8000u;               // marks a slot or word that has been written
+constexpr uint32_t kOneFull = 0x8000u;               // marks a slot or word that holds a maximum
+constexpr uint32_t kOneGaveUp = 0x10000u;            // in a word: the first workgroup has stopped waiting
 constexpr int kOneWords = 7, kOneStride = 32, kRecOne = kRecAmax + 32;     // the published maximum, 128 bytes apart
 constexpr int kOneLeaderSleep = 1, kOneSleep = 12;   // between two looks, in units of 64 cycles
+constexpr int kOnePolls = 256;                       // looks of a workgroup, 0.25 ms or more; undisturbed, some 10 are enough
 
 __device__ __forceinline__ void agent_store(uint32_t* p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void agent_store16(uint16_t* p, uint16_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -699,7 +704,7 @@ __global__ __launch_bounds__(256) void nvfp4_one_pass_clear_kernel(const Table t
 
 // job as for the fold in MODE 1: section = place of the tensor inside its record, pad = tensors sharing it (neighbours)
 template <int F16, class Table>
-__global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_kernel(const Table tab, float numer, int polls) {
+__global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_kernel(const Table tab, float numer, int first_polls) {
     __shared__ uint32_t wave_seen[kOneThreads / 64], wave_late[kOneThreads / 64];
     const FlatJob job = flat_job(tab);
     const int t = threadIdx.x;
@@ -744,7 +749,7 @@ __global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_
             for (int word = t; word * 2 < slots; word += kOneThreads) {
                 const uint32_t need = word * 2 + 1 < slots ? 0x80008000u : 0x8000u;
                 uint32_t got = agent_load(rec + k * kSectionWords + word);
-                for (int n = 0; (got & need) != need && n < polls; n++) {
+                for (int n = 0; (got & need) != need && n < first_polls; n++) {
                     __builtin_amdgcn_s_sleep(kOneLeaderSleep);
                     got = agent_load(rec + k * kSectionWords + word);
                 }
@@ -768,12 +773,12 @@ __global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_
             gave_up |= wave_late[k];
         }
         late = gave_up != 0;
-        if (t < kOneWords && !late) agent_store(rec + kRecOne + t * kOneStride, kOneFull | m);
+        if (t < kOneWords) agent_store(rec + kRecOne + t * kOneStride, late ? kOneGaveUp : kOneFull | m);
     } else {
         if (t < 64) {
             const uint32_t* word = rec + kRecOne + (blockIdx.x % kOneWords) * kOneStride;
             uint32_t got = agent_load(word);
-            for (int n = 0; got == 0 && n < polls; n++) {
+            for (int n = 0; got == 0 && n < kOnePolls; n++) {
                 __builtin_amdgcn_s_sleep(kOneSleep);
                 got = agent_load(word);
             }
@@ -781,7 +786,7 @@ __global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_
         }
         __syncthreads();
         m = wave_late[0];
-        late = m == 0;
+        late = (m & kOneFull) == 0;
         m &= 0x7FFFu;
     }
     if (late) {
@@ -1183,7 +1188,6 @@ int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, in
 // second read in the memory-side cache and save two launches: 4 x [1537, 2064] (25 MB) 15 against 19 us, [4096, 4096]
 // (34 MB) 20 / 19, 16 x [1536, 2048] (100 MB) 39 / 34.
 constexpr int64_t kOneMinBytes = 64ll << 20;
-constexpr int kOnePolls = 256;         // looks of a waiting workgroup, 0.25 ms or more; a wait in a chunk like the above takes some 10
 bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes) {
     int device = 0, cus = 0;
     if (bytes < kOneMinBytes || max_units > kOneSlots * kOnePerBlock) return false;
@@ -1197,10 +1201,10 @@ int64_t mq_nvfp4_one_pass_slots(int64_t units) { return (units + kOnePerBlock - 
 
 // descriptors as for mode 1; `redo` and `one`: their grids for the second pass and for the one-pass kernel
 template <class Table, int F16>
-static int nvfp4_one_pass_launch_dtype(const Table& one, const Table& redo, int n, float numer, int polls, hipStream_t st) {
+static int nvfp4_one_pass_launch_dtype(const Table& one, const Table& redo, int n, float numer, int first_polls, hipStream_t st) {
     const dim3 folds((unsigned)n), blk(256);
     hipLaunchKernelGGL((nvfp4_one_pass_clear_kernel<Table>), folds, blk, 0, st, one);
-    hipLaunchKernelGGL((nvfp4_one_pass_kernel<F16, Table>), dim3((unsigned)one.max_blocks, (unsigned)n), dim3(kOneThreads), 0, st, one, numer, polls);
+    hipLaunchKernelGGL((nvfp4_one_pass_kernel<F16, Table>), dim3((unsigned)one.max_blocks, (unsigned)n), dim3(kOneThreads), 0, st, one, numer, first_polls);
     hipLaunchKernelGGL((nvfp4_one_pass_finish_kernel<F16, Table>), folds, blk, 0, st, one, numer, mq_amax_feedback(), mq_amax_feedback_mirror());
     const unsigned redo_blocks = redo.max_blocks < kSectionWords ? (unsigned)redo.max_blocks : (unsigned)kSectionWords;
     hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<0, 2, Table, F16>), dim3(redo_blocks, (unsigned)n), dim3(kNvThreads), 0, st, redo, numer);
@@ -1209,9 +1213,9 @@ static int nvfp4_one_pass_launch_dtype(const Table& one, const Table& redo, int 
 template <class Table>
 static int nvfp4_one_pass_launch(int dtype, const Table& one, const Table& redo, int n, int e4m3_max, int flags, hipStream_t st) {
     const float numer = (float)e4m3_max * 6.0f;
-    const int polls = (flags & MQ_NVFP4_NO_WAIT) ? 0 : kOnePolls;
-    return dtype == MQ_F16 ? nvfp4_one_pass_launch_dtype<Table, 1>(one, redo, n, numer, polls, st)
-                           : nvfp4_one_pass_launch_dtype<Table, 0>(one, redo, n, numer, polls, st);
+    const int first_polls = (flags & MQ_NVFP4_NO_WAIT) ? 0 : kOnePolls;
+    return dtype == MQ_F16 ? nvfp4_one_pass_launch_dtype<Table, 1>(one, redo, n, numer, first_polls, st)
+                           : nvfp4_one_pass_launch_dtype<Table, 0>(one, redo, n, numer, first_polls, st);
 }
 int mq_nvfp4_one_pass_launch_group(int dtype, const FlatTable& tab, int e4m3_max, int flags, hipStream_t st) {
     FlatTable one = tab, redo = tab;

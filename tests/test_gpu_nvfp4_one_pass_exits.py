@@ -1,0 +1,48 @@
+"""What an amax record says after a list was read once: which form its tensors took, and how the waiting ended."""
+
+import pytest
+import torch
+
+from miles_amd import _lib, launch
+from miles_amd.utils.nvfp4 import nvfp4_quantize_1d, nvfp4_quantize_1d_pair
+
+pytestmark = pytest.mark.gpu
+FIRST_WORD, WORDS, STRIDE = 1056, 7, 32         # the words of a record that the waiting workgroups watch
+PUBLISHED, GAVE_UP = 0x8000, 0x10000
+
+
+def _run(tensors, pairs, flag=0):
+    """Outputs, and of every record the words watched and the one that asks for the second pass."""
+    with launch.recording() as batch:
+        if pairs:
+            got = [t for i in range(0, len(tensors), 2) for t in nvfp4_quantize_1d_pair(tensors[i], tensors[i + 1])]
+        else:
+            got = [nvfp4_quantize_1d(t) for t in tensors]
+    batch.replace_records([r[:batch.P1] + (r[batch.P1] | flag,) + r[batch.P1 + 1:] for r in batch.records])
+    records = batch.amax_records()
+    for r in records:
+        r.zero_()
+    batch.run()
+    words = torch.stack([r[FIRST_WORD:FIRST_WORD + WORDS * STRIDE:STRIDE] for r in records]).cpu()
+    redo = torch.stack([r[_lib.RECORD_REDO_WORD] for r in records]).cpu()
+    return got, words, redo
+
+
+def _tensors(n, rows, cols):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    return list((torch.randn(n, rows, cols, generator=g, device="cuda") * 0.02).bfloat16())
+
+
+@pytest.mark.parametrize("n, rows, cols, pairs", [(5, 1024, 7168, False), (70, 1031, 1040, False), (24, 768, 2048, True), (6, 1300, 7168, True)])
+def test_a_first_workgroup_that_gives_up_says_so(n, rows, cols, pairs):
+    """Every word that the other workgroups watch names the end of the wait, and the second pass quantizes the record."""
+    x = _tensors(n, rows, cols)
+    got, words, redo = _run(x, pairs, _lib.NVFP4_NO_WAIT)
+    assert (words == words[:, :1]).all()
+    gave_up = words[:, 0] == GAVE_UP
+    assert (gave_up | ((words[:, 0] & PUBLISHED) != 0)).all()       # (a first workgroup may find all others done already)
+    assert gave_up.any() and (redo[gave_up] == 1).all()
+    want = [t for i in range(0, n, 2) for t in nvfp4_quantize_1d_pair(x[i], x[i + 1])] if pairs else [nvfp4_quantize_1d(t) for t in x]
+    for one, ref in zip(got, want):
+        for a, b in zip(one, ref):
+            assert torch.equal(a.reshape(-1).view(torch.uint8), b.reshape(-1).view(torch.uint8))
