@@ -5,7 +5,7 @@ import ctypes
 import pytest
 import torch
 
-from miles_amd import _lib
+from miles_amd import _lib, launch
 
 MQ_ERR_ARG = -1
 KINDS = [_lib.JOB_MXFP8, _lib.JOB_FP8_BLOCK, _lib.JOB_FP8_BLOCKWISE_CAST, _lib.JOB_FP8_BLOCK_POW2]
@@ -50,3 +50,15 @@ def test_nvfp4_unknown_flags(dtype, flag):
     """Bits that mq_nvfp4_quant does not know: refused for jobs as well, never handed on to a kernel's launcher."""
     assert _run(_lib.JOB_NVFP4, dtype, 16, 32, 448, flag) == MQ_ERR_ARG
     assert _run(_lib.JOB_NVFP4, dtype, 16, 32, 448, flag | _lib.NVFP4_CARRY_AMAX | _lib.NVFP4_4OVER6) == MQ_ERR_ARG
+
+
+def test_tensors_off_the_gpu():
+    """A job that names host memory never reaches a stream: neither by itself nor from a batch."""
+    host = torch.zeros(32, 32, dtype=torch.bfloat16)
+    out, scale = torch.zeros(32, 32, dtype=torch.uint8), torch.zeros(32, 1, dtype=torch.uint8)
+    with pytest.raises(ValueError, match="cuda device"):
+        _lib.stream_ptr(host.device)
+    with pytest.raises(ValueError, match="cuda device"):
+        launch.submit(_lib.JOB_MXFP8, host, out, scale, None, None, 32, 32, 32)
+    with pytest.raises(ValueError, match="cuda device"), launch.deferred():
+        launch.submit(_lib.JOB_MXFP8, host, out, scale, None, None, 32, 32, 32)
