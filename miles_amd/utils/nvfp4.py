@@ -71,17 +71,22 @@ def _alloc_outputs(w: torch.Tensor):
 
 class StackSlice(tuple):
     """The outputs of one matrix of a stack, as `nvfp4_quantize_1d` takes them in `out`, with what the stack's matrices
-    share: the quantizer's options, and a slice of one allocation as the amax record.  (Made anew for every matrix they
-    took the host 300 us for thirty-two matrices, longer than the GPU needs to quantize them.)"""
+    share: the quantizer's options, a slice of one allocation as the amax record, and the check of the outputs, which
+    `stack_slices` makes once for all of them (`matrix`: the one they belong to).  (Made anew for every matrix they took
+    the host 300 us for thirty-two matrices, longer than the GPU needs to quantize them.)"""
 
 
 def stack_slices(stack: torch.Tensor, codes: torch.Tensor, block_scale: torch.Tensor, global_scale: torch.Tensor):
     """(matrix, its `StackSlice`) for every matrix of [n, M, K] and stacked outputs shaped like the results, contiguous."""
+    n, rows, cols = stack.shape
+    want = ((n, rows, cols // 2), (n, rows, cols // NVFP4_GROUP_SIZE), (n,))
+    if any(tuple(t.shape) != shape or not t.is_contiguous() for t, shape in zip((codes, block_scale, global_scale), want)):
+        raise ValueError("stack_slices: the outputs must be contiguous and shaped like the results")
     options = _quantizer_options() if len(stack) else None
     records = torch.empty((len(stack), AMAX_RECORD_WORDS), dtype=torch.int32, device=stack.device)
     for w, *out, record in zip(stack.unbind(0), codes.unbind(0), block_scale.unbind(0), global_scale.unbind(0), records.unbind(0)):
         out = StackSlice(out)
-        out.options, out.record = options, record
+        out.options, out.record, out.matrix = options, record, w
         yield w, out
 
 
@@ -91,6 +96,8 @@ def nvfp4_quantize_1d(weight: torch.Tensor, *, out=None) -> tuple[torch.Tensor, 
     of stacked outputs, so that a caller inside a deferred batch never has to read results before the batch runs."""
     _lib.require_gpu(weight, "nvfp4_quantize_1d")
     in_stack = type(out) is StackSlice
+    if in_stack and weight is not out.matrix:
+        raise ValueError("nvfp4_quantize_1d: `out` belongs to another matrix of a stack")
     e4m3_max, flags = out.options if in_stack else _quantizer_options()
     w = weight.contiguous()
     rows, cols = w.shape

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from miles_amd import _lib, launch
+from miles_amd.utils import nvfp4
 
 MQ_ERR_ARG = -1
 KINDS = [_lib.JOB_MXFP8, _lib.JOB_FP8_BLOCK, _lib.JOB_FP8_BLOCKWISE_CAST, _lib.JOB_FP8_BLOCK_POW2]
@@ -62,3 +63,31 @@ def test_tensors_off_the_gpu():
         launch.submit(_lib.JOB_MXFP8, host, out, scale, None, None, 32, 32, 32)
     with pytest.raises(ValueError, match="cuda device"), launch.deferred():
         launch.submit(_lib.JOB_MXFP8, host, out, scale, None, None, 32, 32, 32)
+
+
+def _stacked(n, rows, cols):
+    return (torch.zeros(n, rows, cols // 2, dtype=torch.uint8), torch.zeros(n, rows, cols // 16, dtype=torch.float8_e4m3fn), torch.zeros(n))
+
+
+@pytest.mark.parametrize("wrong", range(4))
+def test_outputs_of_a_stack(wrong):
+    """Stacked outputs are checked like a single matrix's, and a slice of them serves its own matrix only."""
+    stack, (codes, scales, top) = torch.zeros(3, 8, 32), _stacked(3, 8, 32)
+    if wrong == 0:
+        codes = codes[:, :4]
+    elif wrong == 1:
+        scales = scales[:, :, :1]
+    elif wrong == 2:
+        top = top[:2]
+    else:
+        codes = codes.transpose(0, 1).contiguous().transpose(0, 1)
+    with pytest.raises(ValueError, match="shaped like the results"):
+        next(nvfp4.stack_slices(stack, codes, scales, top))
+
+
+@pytest.mark.gpu
+def test_a_slice_of_a_stack_serves_its_own_matrix():
+    stack = torch.zeros(3, 8, 32, device="cuda", dtype=torch.bfloat16)
+    _matrix, out = next(nvfp4.stack_slices(stack, *(t.cuda() for t in _stacked(3, 8, 32))))
+    with pytest.raises(ValueError, match="another matrix"):
+        nvfp4.nvfp4_quantize_1d(torch.zeros(16, 32, device="cuda", dtype=torch.bfloat16), out=out)
