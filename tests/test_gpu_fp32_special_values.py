@@ -1,4 +1,4 @@
-"""Infinities and NaN of either sign in fp32 weights: the tuned kernels against the element-wise ones, which a tensor off a
+"""Infinities and NaN of either sign, in fp32 tensors: the tuned kernels against the element-wise ones, which a tensor off a
 16-byte boundary takes, byte for byte; where the reference defines the result, against the oracle as well."""
 
 import pytest
@@ -65,3 +65,69 @@ def test_nvfp4(oracle, monkeypatch, shape, mode, nan):  # noqa: F811
         _assert_same(g.reshape(1), torch.as_tensor(g_o).reshape(1).float(), "global scale")
         _assert_same(s, s_o, "scales")
         _assert_same(q, q_o, "codes")
+
+
+@pytest.mark.parametrize("shape", [(8, 128), (16, 4224), (136, 1024)])
+@pytest.mark.parametrize("group", [32, 64, 128])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_int4(oracle, shape, group, symmetric):  # noqa: F811
+    """NaN (skipped by the extrema, code by code 8 or 0) and infinities send a wavefront through the chain as written, next
+    to groups that keep the fused form."""
+    from miles_amd.kernels.quant.int4_fake import pack_layer
+
+    x = _with_specials(shape, 920 + shape[1] + group)
+    outs = _both(lambda w: [t for t in pack_layer(w, group, symmetric) if t is not None], x, f"group {group}")
+    # the oracle where a group is finite, or holds NaN but not only NaN, among which the reference's fmaxf picks the rest
+    want = oracle.pack_layer(x, group, symmetric)
+    grouped = x.view(shape[0], -1, group)
+    finite = torch.isfinite(grouped).all(-1)
+    _assert_same(outs[1].cpu()[finite], want[1][finite], "scales of finite groups")
+    words = finite.repeat_interleave(group // 8, 1)
+    _assert_same(outs[0].cpu()[words], want[0][words], "codes of finite groups")
+    assert 0 < int(finite.sum()) < finite.numel()
+
+
+@pytest.mark.parametrize("shape", [(1, 128), (5, 384), (129, 2016), (513, 1024)])
+def test_mx_formats(shape):
+    from miles_amd.utils.mxfp4 import quantize_mxfp4
+    from miles_amd.utils.mxfp8 import mxfp8_quantize
+
+    x = _with_specials(shape, 940 + shape[1])
+    _both(lambda w: quantize_mxfp4(w, 32), x, "mxfp4")
+    _both(mxfp8_quantize, x, "mxfp8")
+
+
+@pytest.mark.parametrize("group", [32, 64, 128])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_fake_int4(group, symmetric):
+    from miles_amd.kernels.quant.int4_fake import fake_int4_quant_cuda
+
+    # (a NaN result carries the sign and payload its operands happen to give it)
+    _both(lambda w: [t.nan_to_num(nan=77.0) for t in fake_int4_quant_cuda(w, (1, group), symmetric)[: 2 if symmetric else 3]],
+          _with_specials((129, 2048), 960 + group), f"group {group}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("four_over_six", [False, True])
+def test_lists_of_16_bit_weights(oracle, dtype, four_over_six):  # noqa: F811
+    """NVFP4 fake quantization of lists: an infinite weight against the oracle, a NaN makes every result of its weight NaN and
+    of no other."""
+    from miles_amd import _lib
+    from miles_amd.kernels.quant import nvfp4_qdq as m
+
+    cfg = m.NVFP4QDQConfig(four_over_six, 256 if four_over_six else 448)
+    weights = []
+    for i, shape in enumerate([(3, 48), (129, 1040), (130, 1040), (1, 8208), (5, 2736)]):
+        w = (fp32_case(shape, 980 + i) * 2.0**-12).to(dtype)
+        if i % 2:
+            w[0, 5], w[-1, -1] = float("inf"), -float("inf")
+        if i == 2:
+            w[-1, 3] = float("nan")
+        weights.append(w)
+    got = m.fake_nvfp4_quantization_ste_list([w.to(DEV) for w in weights], cfg)
+    for i, (y, w) in enumerate(zip(got, weights)):
+        if i == 2:
+            assert torch.isnan(y).all()
+            continue
+        want = oracle.fused_nvfp4_qdq(w, e4m3_max=cfg.e4m3_max, flags=_lib.NVFP4_4OVER6 if four_over_six else 0)
+        _assert_same(y.nan_to_num(nan=77.0), want.nan_to_num(nan=77.0), f"weight {i}")

@@ -46,3 +46,15 @@ def test_a_first_workgroup_that_gives_up_says_so(n, rows, cols, pairs):
     for one, ref in zip(got, want):
         for a, b in zip(one, ref):
             assert torch.equal(a.reshape(-1).view(torch.uint8), b.reshape(-1).view(torch.uint8))
+
+
+@pytest.mark.parametrize("n, rows, cols, pairs, one_pass", [
+    (5, 1024, 7168, False, True), (3, 2048, 8192, False, True), (2, 2048, 8208, False, False), (70, 1031, 1040, False, True),
+    (1100, 1, 256 * 16 * 8 + 16, False, True), (2200, 1, 256 * 16 * 8, False, True),
+    (24, 768, 2048, True, True), (6, 1300, 7168, True, True), (4, 2048, 7168, True, False)])
+def test_lists_that_are_read_once(n, rows, cols, pairs, one_pass):
+    """The lists that the comparison with single calls takes, and two that keep two passes: a tensor past a section's slots, a
+    pair of more workgroups than may share a record.  With the chip to itself no workgroup waits in vain."""
+    _got, words, redo = _run(_tensors(n, rows, cols), pairs)
+    assert (((words & PUBLISHED) != 0) if one_pass else (words == 0)).all()
+    assert (redo == 0).all()
