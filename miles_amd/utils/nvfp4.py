@@ -100,7 +100,7 @@ def nvfp4_quantize_1d(weight: torch.Tensor, *, out=None) -> tuple[torch.Tensor, 
         raise ValueError("nvfp4_quantize_1d: `out` belongs to another matrix of a stack")
     e4m3_max, flags = out.options if in_stack else _quantizer_options()
     w = weight.contiguous()
-    rows, cols = w.shape
+    rows, cols = w.shape[0], w.shape[1]
     if cols % NVFP4_GROUP_SIZE != 0:
         raise ValueError(f"NVFP4 requires K divisible by {NVFP4_GROUP_SIZE}, got {cols}.")
     # the amax record is written by the job driver

@@ -89,3 +89,10 @@ def test_a_slice_of_a_stack_serves_its_own_matrix():
     _matrix, out = next(nvfp4.stack_slices(stack, *(t.cuda() for t in _stacked(3, 8, 32))))
     with pytest.raises(ValueError, match="another matrix"):
         nvfp4.nvfp4_quantize_1d(torch.zeros(16, 32, device="cuda", dtype=torch.bfloat16), out=out)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape, error", [((16,), IndexError), ((2, 16, 32), ValueError), ((16, 24), ValueError)])
+def test_nvfp4_weights_of_another_rank(shape, error):
+    with pytest.raises(error):
+        nvfp4.nvfp4_quantize_1d(torch.zeros(shape, device="cuda", dtype=torch.bfloat16))
