@@ -187,11 +187,13 @@ int mq_fp8_act_quant(const void* x, int dtype, void* y, void* scale, int64_t num
 
 /* NVFP4                                              miles/utils/nvfp4.py:54-114
  * The global amax travels on the device in an "amax record": MQ_NVFP4_RECORD_WORDS uint32 words made of
- * MQ_NVFP4_SECTIONS sections of MQ_NVFP4_SECTION_WORDS partial maxima (float bit patterns).  Each tensor that
+ * MQ_NVFP4_SECTIONS sections of MQ_NVFP4_SECTION_WORDS partial maxima (float bit patterns; jobs that are read
+ * once, see the note at mq_run_jobs, keep 16-bit patterns of their tensors' dtype there while they run).  Each tensor that
  * shares the amax writes ONE whole section (no atomics, nothing to clear beforehand); the amax is the maximum
  * over the first n_sections sections.  A single tensor uses section 0 with n_sections = 1; a gate/up pair
  * uses sections 0 and 1 with n_sections = 2 (nvfp4.py:100-103).  The words after the last section hold the
- * folded amax and the two scale factors derived from it (written by mq_nvfp4_quant).
+ * folded amax and the two scale factors derived from it (written by mq_nvfp4_quant); the job driver uses all of them, up
+ * to MQ_NVFP4_RECORD_WORDS (5 KiB in all).
  * mq_nvfp4_amax: record section <- partial maxima of |w| (every word of the section is written).
  * mq_nvfp4_quant: folds the record, then quantizes: w [M,K] contiguous, K % 16 == 0; q [M,K/2] (element 2i in
  *   the low nibble);
@@ -292,11 +294,12 @@ int mq_nvfp4_fake_quant(const mq_fake_quant_item* list, int64_t n, int dtype, vo
  * changed on two submissions in a row is marked volatile in its record: on the next submission the single pass only
  * collects its amax and the second pass quantizes it (what the plain two-pass form costs), and it returns to the
  * single pass once its amax has stayed the same for one submission.
- * Without that flag, lists of 64 MB and more of bf16 or fp16 tensors with standard block scaling are read once as well when
- * every record's tensors fit the chip's registers twice (20 MB on 256 CUs; 32 MB for one tensor at most): the workgroups
- * of a record keep their share and wait for each other's maxima, for a bounded time, after which a second pass does
- * what is left.  MQ_NVFP4_NO_WAIT in p1: a record's first workgroup, which collects the maxima, does not wait and tells the
- * others so (it exists to test that exit and the second pass; results are the same). */
+ * Without that flag, bf16 or fp16 tensors with standard block scaling are read once as well when the tensors of a grouped
+ * launch are 64 MB and more and every record's tensors fit the chip's registers twice (640 workgroups of 64 KiB, 40 MB, on
+ * 256 CUs; a single tensor 32 MB at most).  A grouped launch holds MQ_MAX_GROUP tensors, or with a device table
+ * MQ_TABLE_GROUP.  The workgroups of a record keep their share and wait for each other's maxima, for a bounded time, after
+ * which a second pass does what is left.  MQ_NVFP4_NO_WAIT in p1: a record's first workgroup, which collects the maxima,
+ * does not wait and tells the others so (it exists to test that exit and the second pass; results are the same). */
 enum {
     MQ_JOB_FP8_BLOCK = 0,
     MQ_JOB_FP8_BLOCKWISE_CAST = 1,

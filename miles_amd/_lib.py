@@ -115,16 +115,19 @@ def check(rc: int, exc=MilesQuantError) -> None:
         raise exc(load().mq_last_error().decode() or f"libmiles_quant error {rc}")
 
 
+# the GPUs by their device (reading the type of a torch.device costs 0.2 us, twice this lookup)
+_GPU_INDEX = {torch.device("cuda", i): i for i in range(64)}
+
+
 def stream_ptr(device: torch.device | None = None) -> int:
     """The handle of the current stream (`torch.cuda.current_stream(device).cuda_stream` without making a Stream object of
     it, which costs 1.9 us, a fifth of the smallest calls); a device that has no streams is refused, as there."""
-    if device is None:
-        index = None
-    elif device.type == "cuda":
-        index = device.index
-    else:
-        raise ValueError(f"Expected a cuda device, but got: {device}")
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    index = _GPU_INDEX.get(device)
+    if index is None:
+        if device is not None and device.type != "cuda":
+            raise ValueError(f"Expected a cuda device, but got: {device}")
+        index = torch.cuda.current_device() if device is None or device.index is None else device.index
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def require_gpu(t: torch.Tensor, what: str) -> None:

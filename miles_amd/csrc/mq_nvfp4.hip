@@ -685,6 +685,7 @@ constexpr int kOneSlots = 2 * kSectionWords;         // 16-bit slots of a sectio
 constexpr uint32_t kOneFull = 0x8000u;               // marks a slot or word that holds a maximum
 constexpr uint32_t kOneGaveUp = 0x10000u;            // in a word: the first workgroup has stopped waiting
 constexpr int kOneWords = 7, kOneStride = 32, kRecOne = kRecAmax + 32;     // the published maximum, 128 bytes apart
+static_assert(kRecOne + (kOneWords - 1) * kOneStride < MQ_NVFP4_RECORD_WORDS, "the published words lie inside the record");
 constexpr int kOneLeaderSleep = 1, kOneSleep = 12;   // between two looks, in units of 64 cycles
 constexpr int kOnePolls = 256;                       // looks of a workgroup, 0.25 ms or more; undisturbed, some 10 are enough
 

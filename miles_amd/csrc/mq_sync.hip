@@ -291,8 +291,8 @@ static int64_t tile_run_end(const mq_job* jobs, int64_t i, int64_t j, int64_t ti
 }
 
 static bool same_group(const mq_job& a, const mq_job& b) {
-    // the quantizer kernels are compiled per 16-bit input dtype; the other kinds' fast paths take one dtype, or any
-    // (copies)
+    // the quantizer kernels are compiled per input dtype (bf16, fp16, fp32); the other kinds' fast paths take one dtype, or
+    // any (copies)
     const bool per_dtype = tile_kind(a.kind) || a.kind == MQ_JOB_MXFP8 || a.kind == MQ_JOB_MXFP4 || a.kind == MQ_JOB_INT4_PACK ||
                            a.kind == MQ_JOB_INT4_PACK_ASYM || a.kind == MQ_JOB_INT4_UNPACK;
     return a.kind == b.kind && a.p0 == b.p0 && a.p1 == b.p1 && (!per_dtype || a.dtype == b.dtype);

@@ -3,7 +3,8 @@
 Surface of the reference's miles/utils/nvfp4_fake_qat.py:10-23.  While the environment variable named by
 NVFP4_FAKE_QAT_FLAG is "1", `maybe_fake_quantize_nvfp4_weight_tensors` swaps every weight of the list it is given
 for its quantize-dequantize image (gradients pass straight through); the q-dq options are read from the environment
-once per call, not once per weight, and weights of one dtype share two grouped launches.  With any other value the caller gets its own list object back untouched.
+once per call, not once per weight, and weights of one dtype share two grouped launches.  With any other value the
+caller gets its own list object back untouched.
 """
 
 from __future__ import annotations
