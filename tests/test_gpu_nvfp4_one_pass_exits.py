@@ -58,3 +58,28 @@ def test_lists_that_are_read_once(n, rows, cols, pairs, one_pass):
     _got, words, redo = _run(_tensors(n, rows, cols), pairs)
     assert (((words & PUBLISHED) != 0) if one_pass else (words == 0)).all()
     assert (redo == 0).all()
+
+
+def test_two_streams_at_once():
+    """Two lists whose workgroups compete for the chip: whoever waits in vain leaves its record to the second pass, and every
+    byte is that of a single call."""
+    lists = [_tensors(12, 2048, 7168), [t * 3 for t in _tensors(9, 2048, 8192)]]
+    streams = [torch.cuda.Stream() for _ in lists]
+    batches, outs = [], []
+    for x in lists:
+        with launch.recording() as batch:
+            outs.append([nvfp4_quantize_1d(t) for t in x])
+        batch.freeze()
+        batches.append(batch)
+    want = [[nvfp4_quantize_1d(t) for t in x] for x in lists]
+    torch.cuda.synchronize()
+    for rep in range(4):
+        for batch, stream in zip(batches, streams):
+            batch.run(stream.cuda_stream)
+        torch.cuda.synchronize()
+        for got, ref in zip(outs, want):
+            for one, two in zip(got, ref):
+                for a, b in zip(one, two):
+                    assert torch.equal(a.reshape(-1).view(torch.uint8), b.reshape(-1).view(torch.uint8))
+                    a.reshape(-1).view(torch.uint8).fill_(0xA5)
+        torch.cuda.synchronize()
