@@ -520,7 +520,7 @@ __device__ __forceinline__ void seg_extrema(float& mx, float& mn) {
 #undef MQ_EXTREMA_FIRST
 #undef MQ_EXTREMA_STEP
 // job: w, q = packed codes, s = scales, aux = zero points (one byte per group, read again by the zero-point packer),
-// aux2 = packed zero points, units, section = groups per row
+// aux2 = packed zero points, units, section = groups per row, pad = rows / 8
 //
 // Every group first runs the fused form as one straight instruction stream: scale and zero point from the group's
 // extrema, codes = rint(x / s) + z through the shared-divisor sequence.  The form is final when the scale is in the
@@ -718,74 +718,64 @@ __global__ __launch_bounds__(kI4Threads) void int4_pack_asym_f32_kernel(const Ta
 }
 
 // packed_zp[g, j] = sum_i zero[8j+i, g] << 4*order[i], order = {0,4,1,5,2,6,3,7}   (py:249-254)
-// `zero` is [rows, groups_per_row] bytes and the packed words are its transpose, eight rows to a word.  A workgroup
-// takes a tile of 256 rows x 64 groups through LDS: the bytes are read along the rows (neighbouring lanes, neighbouring
-// bytes) and the words written along j (32 consecutive words of one group per half wavefront).
-constexpr int kZpRows = 256, kZpCols = 64, kZpPitch = kZpCols + 4;
+// `zero` is [rows, groups_per_row] bytes and the packed words are its transpose, eight rows to a word.  A workgroup takes
+// a tile of 256 rows x 16 groups: a lane makes two words, whose sixteen byte loads it issues together (sixteen lanes read
+// neighbouring bytes of a row, whatever the number of groups), and the words go through LDS so that 32 consecutive ones of
+// a group are written by neighbouring lanes.  The bytes are few and still cached: what counts is one memory round trip per
+// workgroup and enough workgroups.  (In tiles of 64 groups, with a loop over the rows where four groups did not fill a
+// word: [352, 3968] 18.7 -> 2.4 us, 174 matrices with 10 and 14 groups a row 21.0 -> 5.5, four [4096, 8192] 4.3 -> 4.4.)
+constexpr int kZpRows = 256, kZpCols = 16, kZpWords = kZpRows / 8, kZpPitch = kZpWords + 1;
+static_assert(kZpWords * kZpCols == 2 * 256, "two words per lane");
 __host__ __device__ __forceinline__ int64_t int4_zero_tiles(int64_t rows8, int64_t groups_per_row) {
-    return ((rows8 * 8 + kZpRows - 1) / kZpRows) * ((groups_per_row + kZpCols - 1) / kZpCols);
+    return ((rows8 + kZpWords - 1) / kZpWords) * ((groups_per_row + kZpCols - 1) / kZpCols);
 }
 __device__ __forceinline__ void int4_zero_pack_tile(const uint8_t* __restrict__ zero, uint32_t* __restrict__ packed_zp,
-                                                    const int64_t rows8, const int64_t groups_per_row, const int64_t tile,
-                                                    uint8_t* lds) {
-    const int64_t col_tiles = (groups_per_row + kZpCols - 1) / kZpCols;
-    const int64_t row0 = (tile / col_tiles) * kZpRows, g0 = (tile % col_tiles) * kZpCols;
-    const int64_t rows = rows8 * 8;
-    const int t = threadIdx.x;
-    if ((groups_per_row & 3) == 0 && ((uintptr_t)zero & 3) == 0) {
-        // four bytes per lane and every load of the tile issued before the first is used: one memory round trip
-        const int c = (t & 15) * 4;
-        const bool col_live = g0 + c < groups_per_row;
-        uint32_t v[kZpRows / 16];
+                                                    const int64_t rows8, const uint32_t groups_per_row, const uint32_t tile,
+                                                    uint32_t* lds) {
+    const uint32_t col_tiles = (groups_per_row + kZpCols - 1) / kZpCols, row_tile = tile / col_tiles;
+    const uint32_t g0 = (tile - row_tile * col_tiles) * kZpCols, t = threadIdx.x;
+    const int64_t j0 = (int64_t)row_tile * kZpWords;
+    const uint32_t words = rows8 - j0 < kZpWords ? (uint32_t)(rows8 - j0) : (uint32_t)kZpWords;      // of each group, at least 1
+    {
+        const uint32_t g = t % kZpCols;
+        // (lanes past the tensor's edge read its last group or rows again)
+        const uint8_t* __restrict__ src = zero + j0 * 8 * groups_per_row + (g0 + g < groups_per_row ? g0 + g : groups_per_row - 1);
+        uint8_t b[2][8];
 #pragma unroll
-        for (int i = 0; i < kZpRows / 16; i++) {
-            const int r = (t >> 4) + 16 * i;
-            const bool live = col_live && row0 + r < rows;
-            v[i] = live ? *(const uint32_t*)(zero + (row0 + r) * groups_per_row + g0 + c) : 0u;
+        for (int h = 0; h < 2; h++) {
+            const uint32_t j = t / kZpCols + 16 * h, jj = j < words ? j : words - 1;
+#pragma unroll
+            for (int k = 0; k < 8; k++) b[h][k] = src[(int64_t)(jj * 8 + k) * groups_per_row];
         }
 #pragma unroll
-        for (int i = 0; i < kZpRows / 16; i++) *(uint32_t*)(lds + ((t >> 4) + 16 * i) * kZpPitch + c) = v[i];
-    } else {
-        const int c = t & (kZpCols - 1);
-        const bool col_live = g0 + c < groups_per_row;
-#pragma unroll 8
-        for (int r = t / kZpCols; r < kZpRows; r += 256 / kZpCols) {
-            const bool live = col_live && row0 + r < rows;
-            lds[r * kZpPitch + c] = live ? zero[(row0 + r) * groups_per_row + g0 + c] : (uint8_t)0;
+        for (int h = 0; h < 2; h++) {
+            uint32_t word = 0;
+#pragma unroll
+            for (int k = 0; k < 8; k++) word += (uint32_t)b[h][k] << (4 * ((k >> 1) + 4 * (k & 1)));
+            lds[g * kZpPitch + t / kZpCols + 16 * h] = word;
         }
     }
     __syncthreads();
-    const int j = t & (kZpRows / 8 - 1);
-    const int64_t jj = row0 / 8 + j;
-    if (jj >= rows8) return;
 #pragma unroll
-    for (int g = t / (kZpRows / 8); g < kZpCols; g += 256 / (kZpRows / 8)) {
-        if (g0 + g >= groups_per_row) break;
-        uint32_t word = 0;
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            const int nib = (k >> 1) + 4 * (k & 1);
-            word += (uint32_t)lds[(j * 8 + k) * kZpPitch + g] << (4 * nib);
-        }
-        packed_zp[(g0 + g) * rows8 + jj] = word;
+    for (int h = 0; h < 2; h++) {
+        const uint32_t j = t % kZpWords, g = t / kZpWords + h * (kZpCols / 2);
+        if (j < words && g0 + g < groups_per_row) packed_zp[(int64_t)(g0 + g) * rows8 + j0 + j] = lds[g * kZpPitch + j];
     }
 }
 __global__ __launch_bounds__(256) void int4_zero_pack_kernel(const uint8_t* __restrict__ zero,
-                                                             uint32_t* __restrict__ packed_zp, int64_t M,
-                                                             int64_t groups_per_row) {
-    __shared__ __align__(4) uint8_t lds[kZpRows * kZpPitch];
-    int4_zero_pack_tile(zero, packed_zp, M / 8, groups_per_row, blockIdx.x, lds);
+                                                             uint32_t* __restrict__ packed_zp, int64_t rows8,
+                                                             uint32_t groups_per_row) {
+    __shared__ uint32_t lds[kZpCols * kZpPitch];
+    int4_zero_pack_tile(zero, packed_zp, rows8, groups_per_row, blockIdx.x, lds);
 }
-// the zero points of a group of tensors (descriptors as for int4_pack_asym_bf16_kernel): blockIdx.y selects the tensor;
-// a tensor of `units` 16-byte units has units / units_per_group groups, groups_per_row of them in each row
+// the zero points of a group of tensors (descriptors as for int4_pack_asym_bf16_kernel): blockIdx.y selects the tensor
 template <class Table>
-__global__ __launch_bounds__(256) void int4_zero_pack_group_kernel(const Table tab, int units_per_group) {
-    __shared__ __align__(4) uint8_t lds[kZpRows * kZpPitch];
-    const FlatJob& job = flat_job(tab);
-    const int64_t groups_per_row = job.section;
-    if (groups_per_row <= 0) return;
-    const int64_t rows8 = job.units / units_per_group / groups_per_row / 8;
-    if (blockIdx.x >= int4_zero_tiles(rows8, groups_per_row)) return;
+__global__ __launch_bounds__(256) void int4_zero_pack_group_kernel(const Table tab) {
+    __shared__ uint32_t lds[kZpCols * kZpPitch];
+    const FlatJob job = flat_job(tab);
+    const int64_t rows8 = job.pad;
+    const uint32_t groups_per_row = (uint32_t)job.section;
+    if (job.section <= 0 || blockIdx.x >= int4_zero_tiles(rows8, groups_per_row)) return;
     int4_zero_pack_tile((const uint8_t*)job.aux, (uint32_t*)job.aux2, rows8, groups_per_row, blockIdx.x, lds);
 }
 
@@ -1080,7 +1070,7 @@ static int int4_pack_asym_launch(int dtype, const Table& tab, int n, int64_t max
     }
     int rc = mq_check_launch("int4 asymmetric pack");
     if (rc != MQ_OK) return rc;
-    hipLaunchKernelGGL(int4_zero_pack_group_kernel<Table>, dim3((unsigned)max_tiles, (unsigned)n), dim3(256), 0, st, tab, group / 8);
+    hipLaunchKernelGGL(int4_zero_pack_group_kernel<Table>, dim3((unsigned)max_tiles, (unsigned)n), dim3(256), 0, st, tab);
     return mq_check_launch("int4 zero-point pack");
 }
 int mq_int4_pack_asym_launch_group(int dtype, FlatTable& tab, int group, hipStream_t st) {
@@ -1090,7 +1080,7 @@ int mq_int4_pack_asym_launch_group(int dtype, FlatTable& tab, int group, hipStre
     for (int i = 0; i < tab.n; i++) {
         const int64_t gpr = tab.job[i].section;
         if (gpr <= 0) continue;
-        const int64_t tiles = int4_zero_tiles(tab.job[i].units / (group / 8) / gpr / 8, gpr);
+        const int64_t tiles = int4_zero_tiles(tab.job[i].pad, gpr);
         max_tiles = tiles > max_tiles ? tiles : max_tiles;
     }
     if (max_tiles >= 0x7FFFFFFF) return mq_fail(MQ_ERR_ARG, "tensor too large");
@@ -1121,7 +1111,7 @@ extern "C" int mq_int4_group_quant_pack_asym(const void* w, int dtype, int32_t* 
     if (mq_int4_pack_asym_fast_ok(w, dtype, group, M)) {
         FlatTable tab{};
         tab.n = 1;
-        tab.job[0] = FlatJob{w, packed, scale, zero, M * (K / 8), packed_zp, (int32_t)gpr, 0};
+        tab.job[0] = FlatJob{w, packed, scale, zero, M * (K / 8), packed_zp, (int32_t)gpr, (int32_t)(M / 8)};
         return mq_int4_pack_asym_launch_group(dtype, tab, group, st);
     } else if (dtype == MQ_BF16)
         hipLaunchKernelGGL(int4_pack_asym_kernel<MQ_BF16>, dim3((unsigned)blocks), dim3(256), 0, st, w, (uint32_t*)packed, scale, zero, groups, wpg, aligned);
@@ -1133,7 +1123,7 @@ extern "C" int mq_int4_group_quant_pack_asym(const void* w, int dtype, int32_t* 
     if (rc != MQ_OK) return rc;
     const int64_t zblocks = int4_zero_tiles(M / 8, gpr);
     if (zblocks >= 0x7FFFFFFF) return mq_fail(MQ_ERR_ARG, "tensor too large");
-    hipLaunchKernelGGL(int4_zero_pack_kernel, dim3((unsigned)zblocks), dim3(256), 0, st, zero, (uint32_t*)packed_zp, M, gpr);
+    hipLaunchKernelGGL(int4_zero_pack_kernel, dim3((unsigned)zblocks), dim3(256), 0, st, zero, (uint32_t*)packed_zp, M / 8, (uint32_t)gpr);
     return mq_check_launch("int4 zero-point pack");
 }
 

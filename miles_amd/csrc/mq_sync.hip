@@ -250,8 +250,9 @@ static TileJob tile_entry(const mq_job& jb) {
 #endif
 static int64_t tiles_of(const mq_job& jb) { return ((jb.rows + 127) / 128) * ((jb.cols + 127) / 128); }
 static FlatJob flat_entry(const mq_job& jb) {
-    if (jb.kind == MQ_JOB_INT4_PACK_ASYM)       // zero points, packed zero points, groups per row
-        return FlatJob{jb.in, jb.out, jb.scale, jb.aux, jb.rows * jb.cols / 8, jb.aux2, jb.p0 > 0 ? (int32_t)(jb.cols / jb.p0) : 0, 0};
+    if (jb.kind == MQ_JOB_INT4_PACK_ASYM)       // zero points, packed zero points, groups per row, words of zero points per group
+        return FlatJob{jb.in, jb.out, jb.scale, jb.aux, jb.rows * jb.cols / 8, jb.aux2, jb.p0 > 0 ? (int32_t)(jb.cols / jb.p0) : 0,
+                       (int32_t)(jb.rows / 8)};
     if (jb.kind == MQ_JOB_FP8_TENSOR)           // amax record, one section
         return FlatJob{jb.in, jb.out, jb.scale, jb.aux, jb.rows * jb.cols / 8, nullptr, 0, 1};
     return FlatJob{jb.in, jb.out, jb.scale, nullptr, jb.rows * jb.cols / 8, nullptr, 0, 0};
