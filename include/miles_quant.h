@@ -351,8 +351,8 @@ int mq_tune_tile_launch_tiles(int64_t tiles, int64_t* previous);
  * hold MQ_MAX_GROUP descriptors at most; a model of thousands of small tensors (the 18 432 expert matrices of a
  * Qwen3-30B-A3B sync, 3 MB each) then drains and refills the chip every 64 tensors.  With a table a launch of the
  * MXFP8, MXFP4, INT4 (symmetric and asymmetric), NVFP4 (standard block scaling), per-tensor FP8 and 128x128 FP8 jobs
- * covers up to MQ_TABLE_GROUP tensors of similar size; every other job kind, Four Over Six NVFP4 jobs and FP8 jobs of
- * mixed shapes run as in mq_run_jobs.
+ * covers up to MQ_TABLE_GROUP tensors of similar size, and one of copy jobs as many independent runs of up to 64 KiB;
+ * every other job kind, Four Over Six NVFP4 jobs and FP8 jobs of mixed shapes run as in mq_run_jobs.
  * mq_job_table_fill writes n entries of MQ_JOB_TABLE_ENTRY_BYTES bytes into host memory, entry i for jobs[i]; the
  * caller copies them to device memory (any 8-byte aligned address) and passes that address, together with the same
  * jobs, to mq_run_jobs_tabled.  A call may cover a sub-range of the list: pass jobs + k, n' and the address of entry k.

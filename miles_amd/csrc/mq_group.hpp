@@ -261,7 +261,11 @@ struct CopyJob {      // rows of `bytes` bytes each (one row: a plain run), chun
     int64_t bytes;
     int64_t src_pitch, dst_pitch;
     int32_t chunks_per_row;
-    int32_t pad;
+    int32_t chunks;           // of all rows
+};
+struct CopyTableEntry {      // in a device table, whose entries are of one size for every kind
+    CopyJob job;
+    int64_t unused;
 };
 struct CopyTable {
     int32_t n;

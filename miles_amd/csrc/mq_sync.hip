@@ -7,6 +7,7 @@
 #include <atomic>
 #include <vector>
 
+#include <stdint.h>
 #include <stdlib.h>
 #include <string.h>
 
@@ -66,7 +67,9 @@ int mq_int4_unpack_launch_group(int scale_dtype, FlatTable& tab, hipStream_t st)
 bool mq_mxfp4_dequant_fast_ok(const void* packed, const void* y, int64_t bytes, int group);
 FlatJob mq_mxfp4_dequant_entry(const void* packed, const void* scale, void* y, int64_t bytes, int group);
 int mq_mxfp4_dequant_launch_group(FlatTable& tab, hipStream_t st);
+int64_t mq_copy_job_finish(CopyJob& job, int64_t rows);
 int mq_copy_launch_group(CopyTable& tab, hipStream_t st);
+int mq_copy_launch_table(const CopyTableEntry* device_jobs, int n, int64_t max_chunks, hipStream_t st);
 int mq_copy_launch_run(const void* src, void* dst, int64_t bytes, hipStream_t st);
 
 // Upper bound on the input bytes of one NVFP4 group (amax launch + fold + quantize launch).  Measured on
@@ -219,7 +222,8 @@ static int run_single(const mq_job& j, void* stream) {
 
 static_assert(kMaxGroup == MQ_MAX_GROUP, "the public group size must match the launch tables");
 static_assert(sizeof(FlatJob) == MQ_JOB_TABLE_ENTRY_BYTES && sizeof(TileJob) == MQ_JOB_TABLE_ENTRY_BYTES &&
-              kTableGroup == MQ_TABLE_GROUP, "the public table entry must match FlatJob and TileJob");
+              sizeof(CopyTableEntry) == MQ_JOB_TABLE_ENTRY_BYTES && kTableGroup == MQ_TABLE_GROUP,
+              "the public table entry must match the descriptors");
 
 // job kinds whose grouped launch can read its descriptors from a device table: the flat kernels and the FP8 tile kernel
 static bool tile_kind(int kind) {
@@ -307,6 +311,20 @@ static int64_t copy_dst_pitch(const mq_job& j) { return j.block_stride != 0 ? j.
 static uintptr_t copy_span(const mq_job& j, int64_t pitch) {
     return (uintptr_t)(j.rows > 1 ? (j.rows - 1) * pitch + j.cols : j.rows * j.cols);
 }
+// a long aligned run streams best from a launch of its own; everything else shares grouped launches
+static bool copy_one_run(const mq_job& j) { return j.rows == 1 || (j.ld == j.cols && copy_dst_pitch(j) == j.cols); }
+static bool copy_alone(const mq_job& j) {
+    return copy_one_run(j) && (((uintptr_t)j.in | (uintptr_t)j.out) & 15) == 0 && j.rows * j.cols >= (64 << 20);
+}
+// the descriptor of a job that is not empty; its chunk count is `chunks` (-1: more than a launch can have)
+static CopyJob copy_entry(const mq_job& j, int64_t& chunks) {
+    const bool one = copy_one_run(j);
+    CopyJob e{(const uint8_t*)j.in, (uint8_t*)j.out, one ? j.rows * j.cols : j.cols, one ? 0 : j.ld, one ? 0 : copy_dst_pitch(j), 0, 0};
+    chunks = mq_copy_job_finish(e, one ? 1 : j.rows);
+    return e;
+}
+// runs of at most this many chunks (64 KiB) share a launch over a device table, whose grid is as wide as the longest of them
+constexpr int64_t kCopyTableChunks = 4;
 static bool copy_depends_on_group(const mq_job* jobs, int64_t first, int64_t candidate) {
     const mq_job& c = jobs[candidate];
     const uintptr_t cin = (uintptr_t)c.in, cout = (uintptr_t)c.out;
@@ -320,6 +338,29 @@ static bool copy_depends_on_group(const mq_job* jobs, int64_t first, int64_t can
     }
     return false;
 }
+
+// Where the copy jobs of a group write, as one interval, and how near to it they read on either side.  A job that keeps the
+// interval free of every source and writes outside it depends on none of the group.  (Records that are packed into a payload
+// have sources of their own and ascending destinations, so that hundreds of them are admitted without comparing each with
+// every other.)
+struct CopyRanges {
+    uintptr_t out_lo = UINTPTR_MAX, out_hi = 0, below = 0, above = UINTPTR_MAX;     // below: the last end of a source in front of the interval
+    static uintptr_t in_end(const mq_job& j) { return (uintptr_t)j.in + copy_span(j, j.ld); }
+    static uintptr_t out_end(const mq_job& j) { return (uintptr_t)j.out + copy_span(j, copy_dst_pitch(j)); }
+    uintptr_t low(const mq_job& j) const { return (uintptr_t)j.out < out_lo ? (uintptr_t)j.out : out_lo; }
+    uintptr_t high(const mq_job& j) const { return out_end(j) > out_hi ? out_end(j) : out_hi; }
+    bool independent(const mq_job& j) const {
+        const uintptr_t lo = low(j), hi = high(j);
+        return ((uintptr_t)j.out >= out_hi || out_end(j) <= out_lo) && (in_end(j) <= lo || (uintptr_t)j.in >= hi) && below <= lo && above >= hi;
+    }
+    void add(const mq_job& j) {
+        out_lo = low(j);
+        out_hi = high(j);
+        if (in_end(j) <= out_lo) below = in_end(j) > below ? in_end(j) : below;
+        else if ((uintptr_t)j.in >= out_hi) above = (uintptr_t)j.in < above ? (uintptr_t)j.in : above;
+        else below = UINTPTR_MAX;       // a source inside: nothing more is independent at a glance
+    }
+};
 
 // per-tensor FP8 run [i, j): chunks of up to kMaxGroup tensors of similar size with the same floor and flags
 // (`table`: the device descriptors of jobs[0..), or null)
@@ -478,6 +519,10 @@ extern "C" int mq_job_table_fill(const mq_job* jobs, int64_t n, void* host_table
             TileJob e = tile_entry(jobs[i]);
             mq_fp8_tile_job_finish(e);
             memcpy(slot, &e, sizeof(e));
+        } else if (jobs[i].kind == MQ_JOB_COPY) {
+            int64_t chunks;
+            const CopyTableEntry e{copy_entry(jobs[i], chunks), 0};
+            memcpy(slot, &e, sizeof(e));
         } else if (jobs[i].kind == MQ_JOB_NVFP4) {
             const mq_job& jb = jobs[i];
             int section, sections;
@@ -571,14 +616,38 @@ extern "C" int mq_run_jobs_tabled(const mq_job* jobs, int64_t n, const void* dev
                 continue;
             }
         }
+        CopyRanges copied;
+        if (head.kind == MQ_JOB_COPY && table) {
+            // short independent runs (the shape records of a packed payload) beyond what the kernel arguments hold
+            int64_t j = i, mx = 0;
+            while (j < n && j - i < kTableGroup && jobs[j].kind == MQ_JOB_COPY && jobs[j].rows > 0 && jobs[j].cols > 0 &&
+                   copied.independent(jobs[j])) {
+                int64_t chunks;
+                copy_entry(jobs[j], chunks);
+                if (chunks < 0 || chunks > kCopyTableChunks) break;
+                mx = chunks > mx ? chunks : mx;
+                copied.add(jobs[j++]);
+            }
+            if (j - i > kMaxGroup) {
+                int rc = mq_copy_launch_table((const CopyTableEntry*)table + i, (int)(j - i), mx, st);
+                if (rc) return rc;
+                i = j;
+                continue;
+            }
+            copied = CopyRanges{};
+        }
         const int64_t group_cap = tabled && !tile_kind(head.kind) ? kTableGroup : kMaxGroup;
         int64_t j = i + 1, sum = head.rows * head.cols, mx = sum;
+        if (head.kind == MQ_JOB_COPY) copied.add(head);
         while (j < n && j - i < group_cap && same_group(head, jobs[j]) && job_path(jobs[j]) == path && jobs[j].rows > 0 &&
                jobs[j].cols > 0) {
             const int64_t e = jobs[j].rows * jobs[j].cols;
             const int64_t nmx = e > mx ? e : mx;
             if (flat && nmx * (j - i + 1) * 4 > (sum + e) * 5) break;
-            if (head.kind == MQ_JOB_COPY && copy_depends_on_group(jobs, i, j)) break;
+            if (head.kind == MQ_JOB_COPY) {
+                if (!copied.independent(jobs[j]) && copy_depends_on_group(jobs, i, j)) break;
+                copied.add(jobs[j]);
+            }
             sum += e;
             mx = nmx;
             j++;
@@ -672,17 +741,16 @@ extern "C" int mq_run_jobs_tabled(const mq_job* jobs, int64_t n, const void* dev
                 break;
             }
             case MQ_JOB_COPY: {
-                // long aligned runs stream best from a launch of their own; everything else shares one grouped launch
                 CopyTable tab{};
                 for (int t = 0; t < cnt && rc == MQ_OK; t++) {
                     const mq_job& jb = jobs[i + t];
-                    const int64_t bytes = jb.rows * jb.cols;
-                    const bool aligned = (((uintptr_t)jb.in | (uintptr_t)jb.out) & 15) == 0;
-                    const bool one_run = jb.rows == 1 || (jb.ld == jb.cols && copy_dst_pitch(jb) == jb.cols);
-                    if (one_run && aligned && bytes >= (64 << 20)) rc = mq_copy_launch_run(jb.in, jb.out, bytes, st);
-                    else if (one_run) tab.job[tab.n++] = CopyJob{(const uint8_t*)jb.in, (uint8_t*)jb.out, bytes, 0, 0, 1, 0};
-                    else tab.job[tab.n++] = CopyJob{(const uint8_t*)jb.in, (uint8_t*)jb.out, jb.cols, jb.ld, copy_dst_pitch(jb),
-                                                    (int32_t)jb.rows, 0};
+                    if (copy_alone(jb)) {
+                        rc = mq_copy_launch_run(jb.in, jb.out, jb.rows * jb.cols, st);
+                        continue;
+                    }
+                    int64_t chunks;
+                    tab.job[tab.n++] = copy_entry(jb, chunks);
+                    if (chunks < 0) rc = mq_fail(MQ_ERR_ARG, "copy group too large");
                 }
                 if (rc == MQ_OK && tab.n > 0) rc = mq_copy_launch_group(tab, st);
                 break;

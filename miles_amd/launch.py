@@ -170,9 +170,10 @@ class JobBatch:
     def held(self) -> list[torch.Tensor]:
         return self._keep
 
-    # job kinds whose grouped launches can take their descriptors from a device table (mq_run_jobs_tabled)
+    # job kinds whose grouped launches can take their descriptors from a device table (mq_run_jobs_tabled); copies take
+    # one that is there, and are not worth making one for
     _TABLE_KINDS = (_lib.JOB_MXFP8, _lib.JOB_MXFP4, _lib.JOB_INT4_PACK, _lib.JOB_INT4_PACK_ASYM, _lib.JOB_FP8_BLOCK,
-                    _lib.JOB_FP8_BLOCKWISE_CAST, _lib.JOB_FP8_BLOCK_POW2, _lib.JOB_NVFP4, _lib.JOB_FP8_TENSOR)
+                    _lib.JOB_FP8_BLOCKWISE_CAST, _lib.JOB_FP8_BLOCK_POW2, _lib.JOB_NVFP4, _lib.JOB_FP8_TENSOR, _lib.JOB_COPY)
 
     def freeze(self):
         """Materialise the ctypes job array (done once; `run` can then be repeated).  A list with more jobs of a
@@ -185,7 +186,7 @@ class JobBatch:
             self._array = arr
             self._array_plain = None
             self._table = None
-            if self.device is not None and sum(r[self.KIND] in self._TABLE_KINDS for r in self._records) > _lib.MAX_GROUP:
+            if self.device is not None and sum(r[self.KIND] in self._TABLE_KINDS and r[self.KIND] != _lib.JOB_COPY for r in self._records) > _lib.MAX_GROUP:
                 host = torch.empty(len(self._records) * _lib.TABLE_ENTRY_BYTES, dtype=torch.uint8)
                 _lib.check(_lib.load().mq_job_table_fill(arr, len(self._records), host.data_ptr()))
                 self._table = host.to(self.device)
