@@ -279,7 +279,12 @@ int mq_nvfp4_fake_quant(const mq_fake_quant_item* list, int64_t n, int dtype, vo
  *      scale dtype share launches of up to MQ_MAX_GROUP tensors: a checkpoint shard's experts unpacked together)
  *   MQ_JOB_MXFP4_DEQUANT        e2m1 pairs    bf16          -              aux = E8M0 bytes (in)       group, -
  *     (mq_mxfp4_dequant with bytes = rows * cols / 2; jobs of one group size share launches the same way)
- * ld is the input row stride in elements for the two FP8 quantizers (column stride 1) and ignored elsewhere;
+ *   MQ_JOB_FP8_SCALED           w[rows,cols]  e4m3          fp32           aux = workspace             floor bits, per_channel
+ *     (mq_fp8_scaled_quant with per_channel = p1, 0 or 1, and the floor's bit pattern in p0, for any dtype, row stride ld and
+ *      alignment; no amax is carried over.  The workspace, MQ_FP8_SCALED_WORDS words and at least one per row, may be NULL
+ *      with per_channel where a row has one to 4096 16-byte units, the last one possibly cut short.  Jobs of one dtype and of
+ *      similar size share launches of up to MQ_MAX_GROUP tensors)
+ * ld is the input row stride in elements for the FP8 quantizers (column stride 1) and ignored elsewhere;
  * rows_per_block / block_stride describe a row-blocked input (see the struct).
  * The three FP8 tile kinds (FP8_BLOCK, FP8_BLOCKWISE_CAST, FP8_BLOCK_POW2), MXFP8, MXFP4, INT4_PACK, INT4_PACK_ASYM, FP8_TENSOR and NVFP4 run their tuned
  * kernels on bf16 and on fp16 inputs, and all but FP8_TENSOR on fp32 ones as well; consecutive jobs share a
@@ -317,8 +322,10 @@ enum {
     MQ_JOB_FP8_TO_MXFP8 = 13,
     MQ_JOB_E8M0_EXPAND = 14,
     MQ_JOB_INT4_UNPACK = 15,
-    MQ_JOB_MXFP4_DEQUANT = 16
+    MQ_JOB_MXFP4_DEQUANT = 16,
+    MQ_JOB_FP8_SCALED = 17
 };
+#define MQ_FP8_SCALED_WORDS 256
 typedef struct mq_job {
     int32_t kind;
     int32_t dtype;

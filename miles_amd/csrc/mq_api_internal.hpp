@@ -24,6 +24,15 @@ struct MqDequantArgs {
     int block;
 };
 
+struct MqScaledArgs {      // one tensor of the per-channel / per-tensor FP8 quantizers
+    const void* w;
+    void* q;
+    float* scale;
+    uint32_t* maxima;      // per tensor: words for the partial maxima
+    int64_t ldw, M, K;
+    float floor_v;
+};
+
 struct MqRescaleArgs {
     const void* x;
     const float* s;

@@ -249,6 +249,7 @@ __device__ __forceinline__ void st8(void* p, u32x2 v) { __builtin_nontemporal_st
 // accesses, and the reduced alignment is part of the type, so the compiler may not assume more.  Without the non-temporal
 // hint: neighbouring workgroups share the lines at the ends of unaligned rows.
 typedef u32x4 u32x4_at2 __attribute__((aligned(2)));
+typedef u32x4 u32x4_at4 __attribute__((aligned(4)));
 typedef u32x2 u32x2_at1 __attribute__((aligned(1)));
 __device__ __forceinline__ u32x4 ld16_at2(const void* p) { return *reinterpret_cast<const u32x4_at2*>(p); }
 __device__ __forceinline__ void st8_at1(void* p, u32x2 v) { *reinterpret_cast<u32x2_at1*>(p) = v; }

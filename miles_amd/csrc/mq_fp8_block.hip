@@ -470,145 +470,21 @@ __global__ __launch_bounds__(256) void fp8_row_quant_kernel(const void* __restri
         q[r * K + c] = (uint8_t)sw_e4m3fn(v);
     }
 }
-// bf16 fast paths of the two.  The quotient x / s is the exact one (shared-divisor sequence, which keeps the sign of a
-// -0 numerator; the division itself when s leaves the guarded range).
-//
-// per channel: a row lives in the registers of ROWLANES lanes (up to 8 sixteen-byte units each), so it is read once:
-// amax across the lanes, one scale, codes.  ROWLANES = 64: four rows per workgroup, no LDS; 256: one row.
-template <int ROWLANES, int F16>
-__global__ __launch_bounds__(256) void fp8_channel_bf16_kernel(const uint16_t* __restrict__ w, int64_t ldw, int64_t K,
-                                                               int64_t M, float floor_v, uint8_t* __restrict__ q,
-                                                               float* __restrict__ scale, int chunk) {
-    __shared__ uint32_t wave_amax[4];
-    constexpr int kRows = 256 / ROWLANES, kMaxUnits = 8;
-    const int t = threadIdx.x, lane = t % ROWLANES;
-    // an XCD takes runs of consecutive rows, as the flat kernels take runs of consecutive blocks
-    const int64_t row = xcd_chunked_block(chunk) * kRows + t / ROWLANES;
-    const int64_t units = K / 8;
-    const bool row_ok = row < M;
-    const uint16_t* __restrict__ src = w + (row_ok ? row : M - 1) * ldw;
-    u32x4 v[kMaxUnits];
-    uint32_t m2 = 0;
-#pragma unroll
-    for (int u = 0; u < kMaxUnits; u++) {
-        const int64_t unit = lane + (int64_t)u * ROWLANES;
-        v[u] = unit < units ? ld16(src + unit * 8) : u32x4{0u, 0u, 0u, 0u};
-        m2 = max2_u16(m2, max2_u16(max2_u16(abs2(v[u].x), abs2(v[u].y)), max2_u16(abs2(v[u].z), abs2(v[u].w))));
-    }
-    uint32_t m = wave_max(hmax_u16(m2));
-    if (ROWLANES == 256) {
-        if ((t & 63) == 0) wave_amax[t >> 6] = m;
-        __syncthreads();
-        m = umax(umax(wave_amax[0], wave_amax[1]), umax(wave_amax[2], wave_amax[3]));
-    }
-    float amax = elem_lo<F16>(m);
-    if (amax < floor_v) amax = floor_v;
-    const float s = amax / kFp8Max, y = 1.0f / s;
-    const bool fast_div = shared_div_ok(s);
-    // the hardware conversion takes finite quotients: an infinity or a NaN in the row, or a zero scale (fp16 has no
-    // 1e-12 floor, so a row of zeros divides 0 by 0), goes through the software conversion
-    const bool plain = m < (F16 ? 0x7C00u : 0x7F80u) && s > 0.0f;
-    if (!row_ok) return;
-    if (lane == 0) scale[row] = s;
-#pragma unroll
-    for (int u = 0; u < kMaxUnits; u++) {
-        const int64_t unit = lane + (int64_t)u * ROWLANES;
-        if (unit >= units) continue;
-        float f[8] = {elem_lo<F16>(v[u].x), elem_hi<F16>(v[u].x), elem_lo<F16>(v[u].y), elem_hi<F16>(v[u].y),
-                      elem_lo<F16>(v[u].z), elem_hi<F16>(v[u].z), elem_lo<F16>(v[u].w), elem_hi<F16>(v[u].w)};
-#pragma unroll
-        for (int j = 0; j < 8; j++) f[j] = fast_div ? div_by_shared(f[j], s, y) : f[j] / s;
-        u32x2 o;
-        if (plain) {
-            o.x = hw_e4m3x4(f[0], f[1], f[2], f[3]);
-            o.y = hw_e4m3x4(f[4], f[5], f[6], f[7]);
-        } else {                                  // inf / NaN in the row: clamp and convert in software
-            uint32_t c[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++) c[j] = sw_e4m3fn(clamp_keep_nan(f[j], -kFp8Max, kFp8Max));
-            o.x = c[0] | (c[1] << 8) | (c[2] << 16) | (c[3] << 24);
-            o.y = c[4] | (c[5] << 8) | (c[6] << 16) | (c[7] << 24);
-        }
-        st8(q + row * K + unit * 8, o);
-    }
-}
-
-// per tensor, pass 1: every workgroup strides over 8 KiB pieces and ends with one atomic max on the bf16 amax
-__global__ __launch_bounds__(256) void fp8_tensor_amax_bf16_kernel(const uint16_t* __restrict__ w, int64_t units,
-                                                                   uint32_t* __restrict__ amax_bits) {
-    __shared__ uint32_t wave_amax[4];
-    const int t = threadIdx.x;
-    uint32_t m2 = 0;
-    for (int64_t base = (int64_t)blockIdx.x * 512; base < units; base += (int64_t)gridDim.x * 512) {
-        const int64_t a = base + t, b = base + 256 + t;
-        const u32x4 va = a < units ? ld16(w + a * 8) : u32x4{0u, 0u, 0u, 0u};
-        const u32x4 vb = b < units ? ld16(w + b * 8) : u32x4{0u, 0u, 0u, 0u};
-        m2 = max2_u16(m2, max2_u16(max2_u16(abs2(va.x), abs2(va.y)), max2_u16(abs2(va.z), abs2(va.w))));
-        m2 = max2_u16(m2, max2_u16(max2_u16(abs2(vb.x), abs2(vb.y)), max2_u16(abs2(vb.z), abs2(vb.w))));
-    }
-    const uint32_t m = wave_max(hmax_u16(m2));
-    if ((t & 63) == 0) wave_amax[t >> 6] = m;
-    __syncthreads();
-    if (t == 0) atomicMax(amax_bits, umax(umax(wave_amax[0], wave_amax[1]), umax(wave_amax[2], wave_amax[3])) << 16);
-}
-// per tensor, pass 2: flat.  torch divides by a zero-dimensional scale in the weight's dtype, so the quotient is
-// rounded to bf16 before it is clamped and converted.
-__global__ __launch_bounds__(256) void fp8_tensor_quant_bf16_kernel(const uint16_t* __restrict__ w,
-                                                                    const uint32_t* __restrict__ amax_bits, float floor_v,
-                                                                    uint8_t* __restrict__ q, float* __restrict__ scale,
-                                                                    int64_t units, int chunk) {
-    const int64_t base = xcd_chunked_block(chunk) * 512 + threadIdx.x;
-    u32x4 v[2];
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int64_t unit = base + i * 256;
-        v[i] = ld16(w + (unit < units ? unit : units - 1) * 8);
-    }
-    const uint32_t abits = amax_bits[0];
-    float amax = u2f(abits);
-    if (amax < floor_v) amax = floor_v;
-    const float s = amax / kFp8Max, y = 1.0f / s;
-    const bool fast_div = shared_div_ok(s);
-    if (base == 0) scale[0] = s;
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int64_t unit = base + i * 256;
-        float f[8] = {bf16_lo(v[i].x), bf16_hi(v[i].x), bf16_lo(v[i].y), bf16_hi(v[i].y),
-                      bf16_lo(v[i].z), bf16_hi(v[i].z), bf16_lo(v[i].w), bf16_hi(v[i].w)};
-#pragma unroll
-        for (int j = 0; j < 8; j++) f[j] = fast_div ? div_by_shared(f[j], s, y) : f[j] / s;
-#pragma unroll
-        for (int j = 0; j < 8; j += 2) {           // the rounding to bf16
-            const uint32_t p = hw_bf16x2(f[j], f[j + 1]);
-            f[j] = bf16_lo(p);
-            f[j + 1] = bf16_hi(p);
-        }
-        u32x2 o;
-        if (abits < 0x7F800000u) {
-            o.x = hw_e4m3x4(f[0], f[1], f[2], f[3]);
-            o.y = hw_e4m3x4(f[4], f[5], f[6], f[7]);
-        } else {
-            uint32_t c[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++) c[j] = sw_e4m3fn(clamp_keep_nan(f[j], -kFp8Max, kFp8Max));
-            o.x = c[0] | (c[1] << 8) | (c[2] << 16) | (c[3] << 24);
-            o.y = c[4] | (c[5] << 8) | (c[6] << 16) | (c[7] << 24);
-        }
-        if (unit < units) st8(q + unit * 8, o);
-    }
-}
-
-// ---- the same of any alignment, and of fp32 ----------------------------------------------------------------------
-// 16-byte loads at any element boundary (E elements: eight of a 16-bit dtype, four of fp32); the last unit of a row, or of
-// the tensor, is moved back to end with it, so that it codes a few elements a second time, to the same bytes.
-// HBM-bound; fp32 quotients come correctly rounded from div24_by_shared where that matters to an e4m3 code.  Eight tensors in
-// eight calls, three launches each per tensor and one per channel (the two element-wise passes before): per tensor
-// [2048, 4096] fp32 381 -> 149 us, [2049, 4099] bf16 379 -> 135; per channel 198 -> 118 and 209 -> 116, which is the host's
-// time for eight calls.
+// ---- rows, and whole tensors, of 16-byte units -------------------------------------------------------------------
+// What the two passes above do, from 16-byte loads (E elements: eight of a 16-bit dtype, four of fp32), for up to 64 tensors
+// a launch.  LINES: aligned units, streamed with non-temporal accesses.  Otherwise any element boundary: the
+// last unit of a row, or of the tensor, is moved back to end with it, so that it codes a few elements a second time, to the
+// same bytes.  HBM-bound.  The quotient x / s is the exact one (shared-divisor sequence, which keeps the sign of a -0
+// numerator; the division itself when s leaves the guarded range); fp32 quotients come correctly rounded from
+// div24_by_shared where that matters to an e4m3 code.
+// Four tensors in one list against a launch (per channel) or three (per tensor) each, us of the kernels: per channel [4096,
+// 8192] bf16 72 -> 61 (6.6 TB/s), fp32 129 -> 108 (6.2), [4095, 8191] bf16 90 -> 74, [1024, 2048] bf16 16.8 -> 6.0; per tensor
+// [4096, 8192] fp32 218 -> 179, [4095, 8191] bf16 138 -> 104, [1024, 2048] fp32 39 -> 16.
 template <int DT> constexpr int kUnitElems = DT == MQ_F32 ? 4 : 8;
-template <int DT>
+template <int DT, bool LINES>
 __device__ __forceinline__ u32x4 ld_unit(const void* p, int64_t elem) {
-    return DT == MQ_F32 ? ld16_at2((const float*)p + elem) : ld16_at2((const uint16_t*)p + elem);
+    const char* at = (const char*)p + elem * (DT == MQ_F32 ? 4 : 2);
+    return LINES ? ld16(at) : ld16_at2(at);
 }
 // the largest magnitude of a unit: an fp32 pattern, or packed 16-bit patterns
 template <int DT>
@@ -626,7 +502,7 @@ __device__ __forceinline__ uint32_t unit_max_f32(uint32_t m) {
 // scale is in the range of the division sequence (shared_div_ok), so no element is infinite or NaN and no quotient exceeds
 // 448 by more than its rounding.  A zero, subnormal (a quotient by its few bits may be far above 448), huge or non-finite
 // scale takes divisions, the clamp and the software conversion.
-template <int DT, bool ROUNDED>
+template <int DT, bool ROUNDED, bool LINES>
 __device__ __forceinline__ void scaled_unit(const u32x4 v, float s, float y, bool plain, uint8_t* __restrict__ q) {
     constexpr int E = kUnitElems<DT>;
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
@@ -665,26 +541,46 @@ __device__ __forceinline__ void scaled_unit(const u32x4 v, float s, float y, boo
             else o.y |= c;
         }
     }
-    if (E == 8) st8_at1(q, o);
+    if (LINES && E == 8) st8(q, u32x2{o.x, o.y});
+    else if (LINES) st4(q, o.x);
+    else if (E == 8) st8_at1(q, u32x2{o.x, o.y});
     else st4_at1(q, o.x);
 }
-// per channel: as fp8_channel_bf16_kernel, a row in the registers of ROWLANES lanes, up to UNITS units each
-template <int ROWLANES, int DT, int UNITS>
-__global__ __launch_bounds__(256) void fp8_channel_any_kernel(const void* __restrict__ w, int64_t ldw, int64_t K, int64_t M,
-                                                              float floor_v, uint8_t* __restrict__ q, float* __restrict__ scale, int chunk) {
+struct ChannelJob {
+    const void* w;
+    uint8_t* q;
+    float* scale;
+    int64_t ldw;
+    int32_t K, M;
+    float floor_v;
+    int32_t pad;
+};
+struct ChannelTable {
+    int32_t n, chunk, max_blocks, pad;      // grid: max_blocks workgroups (a multiple of 8 * chunk) x n tensors
+    ChannelJob job[kMaxGroup];
+};
+// per channel: a row lives in the registers of ROWLANES lanes (up to UNITS units each), so it is read once: amax across the
+// lanes, one scale, codes.  ROWLANES = 64: four rows per workgroup, no LDS; 256: one row.  An XCD takes runs of consecutive
+// rows, as the flat kernels take runs of consecutive blocks.
+template <int ROWLANES, int DT, int UNITS, bool LINES>
+__global__ __launch_bounds__(256) void fp8_channel_kernel(const ChannelTable tab) {
     __shared__ uint32_t wave_amax[4];
     constexpr int kRows = 256 / ROWLANES, E = kUnitElems<DT>;
-    const int t = threadIdx.x, lane = t % ROWLANES;
-    const int64_t row = xcd_chunked_block(chunk) * kRows + t / ROWLANES;
-    const bool row_ok = row < M;
-    const int64_t src = (row_ok ? row : M - 1) * ldw;
-    const int units = (int)((K + E - 1) / E), last = (int)K - E;
+    const ChannelJob& job = tab.job[blockIdx.y];
+    const void* __restrict__ w = load_global_ptr(&job.w);
+    uint8_t* __restrict__ q = load_global_ptr(&job.q);
+    const int t = threadIdx.x, lane = t % ROWLANES, K = job.K;
+    const int64_t block = xcd_chunked_block(tab.chunk), row = block * kRows + t / ROWLANES;
+    if (block * kRows >= job.M) return;
+    const bool row_ok = row < job.M;
+    const int64_t src = (row_ok ? row : job.M - 1) * job.ldw;
+    const int units = (K + E - 1) / E, last = K - E;
     u32x4 v[UNITS];
     uint32_t m = 0;
 #pragma unroll
     for (int u = 0; u < UNITS; u++) {
         const int unit = lane + u * ROWLANES, at = unit * E < last ? unit * E : last;      // (lanes past the end read the last unit)
-        v[u] = u * ROWLANES < units ? ld_unit<DT>(w, src + at) : u32x4{0u, 0u, 0u, 0u};
+        v[u] = u * ROWLANES < units ? ld_unit<DT, LINES>(w, src + at) : u32x4{0u, 0u, 0u, 0u};
     }
 #pragma unroll
     for (int u = 0; u < UNITS; u++) m = unit_max<DT>(m, v[u]);
@@ -695,69 +591,106 @@ __global__ __launch_bounds__(256) void fp8_channel_any_kernel(const void* __rest
         m = umax(umax(wave_amax[0], wave_amax[1]), umax(wave_amax[2], wave_amax[3]));
     }
     float amax = u2f(m);
-    if (amax < floor_v) amax = floor_v;
+    if (amax < job.floor_v) amax = job.floor_v;
     const float s = amax / kFp8Max, y = 1.0f / s;
     const bool plain = shared_div_ok(s);
     if (!row_ok) return;
-    if (lane == 0) scale[row] = s;
+    if (lane == 0) load_global_ptr(&job.scale)[row] = s;
 #pragma unroll
     for (int u = 0; u < UNITS; u++) {
         const int unit = lane + u * ROWLANES, at = unit * E < last ? unit * E : last;
-        if (unit < units) scaled_unit<DT, false>(v[u], s, y, plain, q + row * K + at);
+        if (unit < units) scaled_unit<DT, false, LINES>(v[u], s, y, plain, q + row * K + at);
     }
 }
-// per tensor: amax pass (one atomic max per workgroup on the fp32 pattern) and flat quantize pass over n contiguous elements
-constexpr int kTensorAnyLoads = 4, kTensorAnyUnits = 2;
-// Partial maxima of the amax pass, which the quantize pass folds, a word per lane.  The atomics on one word follow each other at
-// some 8 ns, which 512 workgroups spend at the pass's end: [2048, 4096] fp32 12.5 us with one word, 9.1 to 9.6 with 64.  Those on
-// neighbouring words still meet in one line, so more workgroups pay off only where their loads gain more than that:
-// 512 / 1024 / 2048 of them take 9.6 / 11.1 / 13.6 us there (256: 9.7), but [8192, 16383] bf16 (268 MB) 52 / - / 46.
-// The line lies halfway, at 128 MB (8192 trips of a workgroup).  Looking at the word before the atomic: 13.8 us.
-constexpr int kTensorAnyWords = 64, kTensorAnyBlocks = 512, kTensorAnyManyBlocks = 2048, kTensorAnyManyTrips = 8192;
-static_assert(kTensorAnyWords == kWave, "a wavefront folds the partial maxima with one load");
-template <int DT>
-__global__ __launch_bounds__(256) void fp8_tensor_amax_any_kernel(const void* __restrict__ w, int64_t n, uint32_t* __restrict__ amax_bits, uint32_t word_mask) {
-    __shared__ uint32_t wave_amax[4];
+struct ScaledJob {
+    const void* w;
+    uint8_t* q;
+    float* scale;
+    uint32_t* maxima;       // of the amax pass, ScaledTable::words of them
+    int64_t n;              // elements
+    float floor_v;
+    int32_t pad;
+};
+struct ScaledTable {
+    int32_t n, chunk, max_blocks;
+    int32_t words;          // partial maxima of a tensor: a power of two, at most kScaledWords
+    int32_t amax_blocks;    // workgroups of the amax pass for each tensor
+    int32_t pad;
+    ScaledJob job[kMaxGroup];
+};
+// per tensor: an amax pass over n contiguous elements, and a flat quantize pass that folds the partial maxima by itself, under
+// its loads.  The maxima are read by every workgroup of the second pass, so they are few: a workgroup of the amax pass is 1024
+// lanes, 64 of them cover a tensor where eight share a launch, and a wavefront folds 64 words with one load.  (256 words, read
+// by each wavefront: four [4096, 8192] fp32 111 us in the second pass instead of 101.)  As jobs a workgroup of the amax
+// pass has a word of its own; the direct calls have fewer words than workgroups, cleared beforehand, and take the maximum
+// atomically, at some 8 ns each.
+constexpr int kScaledLoads = 4, kScaledUnits = 2, kAmaxThreads = 1024, kScaledWords = 256, kDirectWords = 64, kDirectBlocks = 256;
+template <int DT, bool LINES>
+__global__ __launch_bounds__(kAmaxThreads) void fp8_scaled_amax_kernel(const ScaledTable tab) {
+    __shared__ uint32_t wave_amax[kAmaxThreads / kWave];
     constexpr int E = kUnitElems<DT>;
+    const ScaledJob& job = tab.job[blockIdx.y];
+    const void* __restrict__ w = load_global_ptr(&job.w);
     const int t = threadIdx.x;
-    const int64_t units = (n + E - 1) / E;
+    const int64_t n = job.n, units = (n + E - 1) / E, last = LINES ? n / E * E - E : n - E;      // of the units that lanes past the end read again
     uint32_t m = 0;
-    for (int64_t base = (int64_t)blockIdx.x * (256 * kTensorAnyLoads); base < units; base += (int64_t)gridDim.x * (256 * kTensorAnyLoads)) {
-        u32x4 v[kTensorAnyLoads];
+    for (int64_t base = (int64_t)blockIdx.x * (kAmaxThreads * kScaledLoads); base < units; base += (int64_t)gridDim.x * (kAmaxThreads * kScaledLoads)) {
+        u32x4 v[kScaledLoads];
 #pragma unroll
-        for (int i = 0; i < kTensorAnyLoads; i++) {
-            const int64_t at = (base + i * 256 + t) * E;
-            v[i] = ld_unit<DT>(w, at < n - E ? at : n - E);
+        for (int i = 0; i < kScaledLoads; i++) {
+            const int64_t at = (base + i * kAmaxThreads + t) * E;
+            v[i] = ld_unit<DT, LINES>(w, at < last ? at : last);
         }
 #pragma unroll
-        for (int i = 0; i < kTensorAnyLoads; i++) m = unit_max<DT>(m, v[i]);
+        for (int i = 0; i < kScaledLoads; i++) m = unit_max<DT>(m, v[i]);
     }
+    if (LINES && last + E < n && blockIdx.x == 0 && t == 0) m = unit_max<DT>(m, ld_unit<DT, false>(w, n - E));
     m = wave_max(unit_max_f32<DT>(m));
     if ((t & 63) == 0) wave_amax[t >> 6] = m;
     __syncthreads();
-    if (t == 0) atomicMax(amax_bits + (blockIdx.x & word_mask), umax(umax(wave_amax[0], wave_amax[1]), umax(wave_amax[2], wave_amax[3])));
-}
-template <int DT>
-__global__ __launch_bounds__(256) void fp8_tensor_quant_any_kernel(const void* __restrict__ w, int64_t n, const uint32_t* __restrict__ amax_bits,
-                                                                   uint32_t word_mask, float floor_v, uint8_t* __restrict__ q, float* __restrict__ scale, int chunk) {
-    constexpr int E = kUnitElems<DT>;
-    const int64_t base = xcd_chunked_block(chunk) * (256 * kTensorAnyUnits) + threadIdx.x;
-    u32x4 v[kTensorAnyUnits];
+    if (t != 0) return;
+    m = 0;
 #pragma unroll
-    for (int i = 0; i < kTensorAnyUnits; i++) {
+    for (int k = 0; k < kAmaxThreads / kWave; k++) m = umax(m, wave_amax[k]);
+    uint32_t* __restrict__ word = load_global_ptr(&job.maxima) + (blockIdx.x & (uint32_t)(tab.words - 1));
+    if (tab.amax_blocks > tab.words) atomicMax(word, m);
+    else *word = m;
+}
+template <int DT, bool LINES>
+__global__ __launch_bounds__(256) void fp8_scaled_quant_kernel(const ScaledTable tab) {
+    __shared__ uint32_t wave_amax[4];
+    constexpr int E = kUnitElems<DT>;
+    const ScaledJob& job = tab.job[blockIdx.y];
+    const void* __restrict__ w = load_global_ptr(&job.w);
+    const uint32_t* __restrict__ maxima = load_global_ptr(&job.maxima);
+    uint8_t* __restrict__ q = load_global_ptr(&job.q);
+    const int64_t n = job.n, first = xcd_chunked_block(tab.chunk) * (256 * kScaledUnits), base = first + threadIdx.x;
+    if (first * E >= n) return;
+    const int64_t last = LINES ? n / E * E - E : n - E;
+    u32x4 v[kScaledUnits];
+#pragma unroll
+    for (int i = 0; i < kScaledUnits; i++) {
         const int64_t at = (base + i * 256) * E;
-        v[i] = ld_unit<DT>(w, at < n - E ? at : n - E);
+        v[i] = ld_unit<DT, LINES>(w, at < last ? at : last);
     }
-    const uint32_t abits = wave_max(amax_bits[threadIdx.x & word_mask]);
-    float amax = u2f(abits);
-    if (amax < floor_v) amax = floor_v;
+    static_assert(kScaledWords <= 256, "a word per lane");
+    uint32_t m = wave_max(maxima[threadIdx.x & (uint32_t)(tab.words - 1)]);
+    if (tab.words > kWave) {
+        if ((threadIdx.x & 63) == 0) wave_amax[threadIdx.x >> 6] = m;
+        __syncthreads();
+        m = umax(umax(wave_amax[0], wave_amax[1]), umax(wave_amax[2], wave_amax[3]));
+    }
+    float amax = u2f(m);
+    if (amax < job.floor_v) amax = job.floor_v;
     const float s = amax / kFp8Max, y = 1.0f / s;
     const bool plain = shared_div_ok(s);
-    if (base == 0) scale[0] = s;
+    if (base == 0) *load_global_ptr(&job.scale) = s;
 #pragma unroll
-    for (int i = 0; i < kTensorAnyUnits; i++) {
+    for (int i = 0; i < kScaledUnits; i++) {
         const int64_t at = (base + i * 256) * E;
-        if (at < n) scaled_unit<DT, true>(v[i], s, y, plain, q + (at < n - E ? at : n - E));
+        if (!LINES && at < n) scaled_unit<DT, true, false>(v[i], s, y, plain, q + (at < last ? at : last));
+        else if (LINES && at <= last) scaled_unit<DT, true, true>(v[i], s, y, plain, q + at);
+        else if (LINES && at < n) scaled_unit<DT, true, false>(ld_unit<DT, false>(w, n - E), s, y, plain, q + (n - E));      // the tail
     }
 }
 
@@ -1046,42 +979,96 @@ extern "C" int mq_fp8_block_quant_pow2(const void* w, int dtype, int64_t ldw, vo
     return fp8_block_launch(2, w, dtype, ldw, 1, q, scale, M, K, kTile, kTile, (hipStream_t)stream);
 }
 
-// the forms for any alignment and for fp32 (rows, or the whole tensor, of at least one unit)
-template <int DT>
-static bool fp8_scaled_any(const void* w, int64_t ldw, uint8_t* q, float* scale, uint32_t* amax_ws, int64_t M, int64_t K,
-                           int per_channel, float floor_v, hipStream_t st) {
-    constexpr int E = kUnitElems<DT>;
-    if ((uintptr_t)w % (DT == MQ_F32 ? 4 : 2) != 0) return false;
-    if (per_channel) {
-        const int64_t units = (K + E - 1) / E;
-        if (K < E || units > 256 * 16) return false;
-        // (a wavefront per row while that leaves a lane no more than four units, as for aligned rows; sixteen units a lane
-        // are 64 registers)
-        const bool four_rows = units <= 256;
-        const int64_t blocks = four_rows ? (M + 3) / 4 : M;
-        if (blocks > 0x7FFFF000ll) return false;          // (the grid is padded by up to 511 workgroups)
-        const int chunk = (int)flat_chunk(blocks);
-        const dim3 grid((unsigned)flat_padded(blocks, chunk)), blk(256);
-        if (four_rows) hipLaunchKernelGGL((fp8_channel_any_kernel<64, DT, 4>), grid, blk, 0, st, w, ldw, K, M, floor_v, q, scale, chunk);
-        else if (units <= 1024) hipLaunchKernelGGL((fp8_channel_any_kernel<256, DT, 4>), grid, blk, 0, st, w, ldw, K, M, floor_v, q, scale, chunk);
-        else if (units <= 2048) hipLaunchKernelGGL((fp8_channel_any_kernel<256, DT, 8>), grid, blk, 0, st, w, ldw, K, M, floor_v, q, scale, chunk);
-        else hipLaunchKernelGGL((fp8_channel_any_kernel<256, DT, 16>), grid, blk, 0, st, w, ldw, K, M, floor_v, q, scale, chunk);
-        return true;
+// How the rows of a tensor are held (fp8_channel_kernel): lanes per row and units per lane, and whether the rows are whole
+// aligned units.  A wavefront per row while that leaves a lane no more than four units; sixteen units a lane are 64
+// registers.  0: rows of less than a unit or of more than 4096, which take the element-wise kernels.
+enum ChannelForm { kChannelNone = 0, kChannel64x4 = 1, kChannel256x4, kChannel256x8, kChannel256x16, kChannelLines = 8 };
+int mq_fp8_channel_form(const void* w, int dtype, int64_t ldw, const void* q, int64_t M, int64_t K) {
+    if (dtype < MQ_BF16 || dtype > MQ_F32 || M <= 0 || M > 0x7FFFFFFF) return kChannelNone;
+    const int64_t E = dtype == MQ_F32 ? 4 : 8, units = (K + E - 1) / E;
+    if (K < E || units > 256 * 16 || (uintptr_t)w % (dtype == MQ_F32 ? 4 : 2) != 0) return kChannelNone;
+    const int64_t blocks = units <= 256 ? (M + 3) / 4 : M;
+    if (blocks > 0x7FFFF000ll) return kChannelNone;          // (the grid is padded by up to 511 workgroups)
+    const bool lines = K % E == 0 && ldw % E == 0 && (uintptr_t)w % 16 == 0 && (uintptr_t)q % E == 0;
+    return (units <= 256 ? kChannel64x4 : units <= 1024 ? kChannel256x4 : units <= 2048 ? kChannel256x8 : kChannel256x16) | (lines ? kChannelLines : 0);
+}
+int64_t mq_fp8_channel_blocks(int form, int64_t M) { return (form & ~kChannelLines) == kChannel64x4 ? (M + 3) / 4 : M; }
+template <int DT, bool LINES>
+static void channel_launch(int form, const ChannelTable& tab, hipStream_t st) {
+    const dim3 grid((unsigned)tab.max_blocks, (unsigned)tab.n), blk(256);
+    switch (form) {
+        case kChannel64x4: hipLaunchKernelGGL((fp8_channel_kernel<64, DT, 4, LINES>), grid, blk, 0, st, tab); break;
+        case kChannel256x4: hipLaunchKernelGGL((fp8_channel_kernel<256, DT, 4, LINES>), grid, blk, 0, st, tab); break;
+        case kChannel256x8: hipLaunchKernelGGL((fp8_channel_kernel<256, DT, 8, LINES>), grid, blk, 0, st, tab); break;
+        default: hipLaunchKernelGGL((fp8_channel_kernel<256, DT, 16, LINES>), grid, blk, 0, st, tab); break;
     }
-    const int64_t n = M * K, units = (n + E - 1) / E;
-    if ((ldw != K && M != 1) || n < E || units >= (1ll << 38)) return false;
-    const int64_t trips = (units + 256 * kTensorAnyLoads - 1) / (256 * kTensorAnyLoads);
-    // (the workspace holds a word per row, that of the static form 64 for a tensor)
-    const int words = M >= kTensorAnyWords ? kTensorAnyWords : 1;
-    const int64_t cap = words > 1 && trips > kTensorAnyManyTrips ? kTensorAnyManyBlocks : kTensorAnyBlocks;
-    const uint32_t word_mask = (uint32_t)words - 1u;
-    hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, amax_ws, 0u, words);
-    hipLaunchKernelGGL(fp8_tensor_amax_any_kernel<DT>, dim3((unsigned)(trips < cap ? trips : cap)), dim3(256), 0, st, w, n, amax_ws, word_mask);
-    const int64_t blocks = (units + 256 * kTensorAnyUnits - 1) / (256 * kTensorAnyUnits);
-    const int chunk = (int)flat_chunk(blocks);
-    hipLaunchKernelGGL(fp8_tensor_quant_any_kernel<DT>, dim3((unsigned)flat_padded(blocks, chunk)), dim3(256), 0, st, w, n, amax_ws,
-                       word_mask, floor_v, q, scale, chunk);
-    return true;
+}
+// n <= kMaxGroup tensors of one dtype and one form
+int mq_fp8_channel_launch_group(int dtype, int form, const MqScaledArgs* a, int n, hipStream_t st) {
+    ChannelTable tab{};
+    tab.n = n;
+    int64_t mx = 0;
+    for (int i = 0; i < n; i++) {
+        tab.job[i] = ChannelJob{a[i].w, (uint8_t*)a[i].q, a[i].scale, a[i].ldw, (int32_t)a[i].K, (int32_t)a[i].M, a[i].floor_v, 0};
+        const int64_t blocks = mq_fp8_channel_blocks(form, a[i].M);
+        mx = blocks > mx ? blocks : mx;
+    }
+    tab.chunk = (int32_t)flat_chunk(mx);
+    tab.max_blocks = (int32_t)flat_padded(mx, tab.chunk);
+    const bool lines = (form & kChannelLines) != 0;
+    form &= ~kChannelLines;
+    if (dtype == MQ_F32) lines ? channel_launch<MQ_F32, true>(form, tab, st) : channel_launch<MQ_F32, false>(form, tab, st);
+    else if (dtype == MQ_F16) lines ? channel_launch<MQ_F16, true>(form, tab, st) : channel_launch<MQ_F16, false>(form, tab, st);
+    else lines ? channel_launch<MQ_BF16, true>(form, tab, st) : channel_launch<MQ_BF16, false>(form, tab, st);
+    return mq_check_launch("fp8 per-channel quant");
+}
+
+// one scale for a contiguous tensor: 1 from aligned addresses (only a tail of less than a unit is not), 2 from any others; 0:
+// not for these kernels
+int mq_fp8_scaled_form(const void* w, int dtype, int64_t ldw, const void* q, int64_t M, int64_t K) {
+    if (dtype < MQ_BF16 || dtype > MQ_F32 || M <= 0 || M > 0x7FFFFFFF || (ldw != K && M != 1)) return 0;
+    const int64_t E = dtype == MQ_F32 ? 4 : 8, n = M * K;
+    if (n < E || (n + E - 1) / E >= (1ll << 38) || (uintptr_t)w % (dtype == MQ_F32 ? 4 : 2) != 0) return 0;
+    return (uintptr_t)w % 16 == 0 && (uintptr_t)q % E == 0 ? 1 : 2;
+}
+template <int DT, bool LINES>
+static void scaled_launch(const ScaledTable& tab, hipStream_t st) {
+    hipLaunchKernelGGL((fp8_scaled_amax_kernel<DT, LINES>), dim3((unsigned)tab.amax_blocks, (unsigned)tab.n), dim3(kAmaxThreads), 0, st, tab);
+    hipLaunchKernelGGL((fp8_scaled_quant_kernel<DT, LINES>), dim3((unsigned)tab.max_blocks, (unsigned)tab.n), dim3(256), 0, st, tab);
+}
+// n <= kMaxGroup tensors of one dtype and one form, each with `words` words for its partial maxima (a power of two; fewer than
+// kScaledWords: cleared first)
+int mq_fp8_scaled_launch_group(int dtype, int form, const MqScaledArgs* a, int n, int words, hipStream_t st) {
+    ScaledTable tab{};
+    tab.n = n;
+    const int64_t E = dtype == MQ_F32 ? 4 : 8;
+    int64_t units = 0;
+    for (int i = 0; i < n; i++) {
+        const int64_t numel = a[i].M * a[i].K, u = (numel + E - 1) / E;
+        tab.job[i] = ScaledJob{a[i].w, (uint8_t*)a[i].q, a[i].scale, a[i].maxima, numel, a[i].floor_v, 0};
+        units = u > units ? u : units;
+    }
+    const int64_t trips = (units + kAmaxThreads * kScaledLoads - 1) / (kAmaxThreads * kScaledLoads);
+    if (words >= kScaledWords) {
+        // what the chip holds (two workgroups per CU) from all tensors together, but not fewer than 64 for each, and no more
+        // than it has trips
+        int blocks = kScaledWords;
+        while (blocks > 1 && ((blocks > 64 && blocks * n > 512) || blocks / 2 >= trips)) blocks /= 2;
+        tab.words = tab.amax_blocks = blocks;
+    } else {
+        tab.words = words;
+        tab.amax_blocks = (int32_t)(trips < kDirectBlocks ? trips : kDirectBlocks);
+        for (int i = 0; i < n; i++) hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, a[i].maxima, 0u, words);
+    }
+    const int64_t blocks = (units + 256 * kScaledUnits - 1) / (256 * kScaledUnits), chunk = flat_chunk(blocks);
+    if (flat_padded(blocks, chunk) >= 0x7FFFFFF0) return mq_fail(MQ_ERR_ARG, "tensor too large");
+    tab.chunk = (int32_t)chunk;
+    tab.max_blocks = (int32_t)flat_padded(blocks, chunk);
+    const bool lines = form == 1;
+    if (dtype == MQ_F32) lines ? scaled_launch<MQ_F32, true>(tab, st) : scaled_launch<MQ_F32, false>(tab, st);
+    else if (dtype == MQ_F16) lines ? scaled_launch<MQ_F16, true>(tab, st) : scaled_launch<MQ_F16, false>(tab, st);
+    else lines ? scaled_launch<MQ_BF16, true>(tab, st) : scaled_launch<MQ_BF16, false>(tab, st);
+    return mq_check_launch("fp8 scaled quant");
 }
 
 static int fp8_scaled_quant(const void* w, int dtype, int64_t ldw, void* q, float* scale, void* amax_ws, int64_t M,
@@ -1092,41 +1079,15 @@ static int fp8_scaled_quant(const void* w, int dtype, int64_t ldw, void* q, floa
     if (M == 0 || K == 0) return MQ_OK;
     if (M > 0x7FFFFFFF) return mq_fail(MQ_ERR_ARG, "too many rows");
     hipStream_t st = (hipStream_t)stream;
-    const bool aligned16 = (dtype == MQ_BF16 || dtype == MQ_F16) && K % 8 == 0 && ldw % 8 == 0 && ((uintptr_t)w % 16) == 0 &&
-                           ((uintptr_t)q % 8) == 0;
-    const bool aligned = aligned16 && dtype == MQ_BF16;
-    if (aligned16 && per_channel && K / 8 <= 2048) {
-        const uint16_t* wi = (const uint16_t*)w;
-        const bool four_rows = K / 8 <= 256;
-        const int64_t blocks = four_rows ? (M + 3) / 4 : M;
-        const int chunk = (int)flat_chunk(blocks);
-        const dim3 grid((unsigned)flat_padded(blocks, chunk)), blk(256);
-        if (dtype == MQ_F16) {
-            if (four_rows) hipLaunchKernelGGL((fp8_channel_bf16_kernel<64, 1>), grid, blk, 0, st, wi, ldw, K, M, floor_in_dtype, (uint8_t*)q, scale, chunk);
-            else hipLaunchKernelGGL((fp8_channel_bf16_kernel<256, 1>), grid, blk, 0, st, wi, ldw, K, M, floor_in_dtype, (uint8_t*)q, scale, chunk);
-        } else {
-            if (four_rows) hipLaunchKernelGGL((fp8_channel_bf16_kernel<64, 0>), grid, blk, 0, st, wi, ldw, K, M, floor_in_dtype, (uint8_t*)q, scale, chunk);
-            else hipLaunchKernelGGL((fp8_channel_bf16_kernel<256, 0>), grid, blk, 0, st, wi, ldw, K, M, floor_in_dtype, (uint8_t*)q, scale, chunk);
-        }
-        return mq_check_launch("fp8 scaled quant");
+    const MqScaledArgs one{w, q, scale, (uint32_t*)amax_ws, ldw, M, K, floor_in_dtype};
+    if (per_channel) {
+        const int form = mq_fp8_channel_form(w, dtype, ldw, q, M, K);
+        if (form) return mq_fp8_channel_launch_group(dtype, form, &one, 1, st);
+    } else {
+        // (the workspace holds a word per row, that of the static form 64 for a tensor)
+        const int form = mq_fp8_scaled_form(w, dtype, ldw, q, M, K);
+        if (form) return mq_fp8_scaled_launch_group(dtype, form, &one, 1, M >= kDirectWords ? kDirectWords : 1, st);
     }
-    if (aligned && !per_channel && ldw == K && M * (K / 8) < (1ll << 38)) {
-        const int64_t units = M * (K / 8);
-        int64_t blocks = (units + 511) / 512;
-        hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, (uint32_t*)amax_ws, 0u, 1);
-        hipLaunchKernelGGL(fp8_tensor_amax_bf16_kernel, dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(256), 0, st,
-                           (const uint16_t*)w, units, (uint32_t*)amax_ws);
-        const int chunk = (int)flat_chunk(blocks);
-        blocks = flat_padded(blocks, chunk);
-        hipLaunchKernelGGL(fp8_tensor_quant_bf16_kernel, dim3((unsigned)blocks), dim3(256), 0, st, (const uint16_t*)w,
-                           (const uint32_t*)amax_ws, floor_in_dtype, (uint8_t*)q, scale, units, chunk);
-        return mq_check_launch("fp8 scaled quant");
-    }
-    uint32_t* ws = (uint32_t*)amax_ws;
-    if (dtype == MQ_F32  ? fp8_scaled_any<MQ_F32>(w, ldw, (uint8_t*)q, scale, ws, M, K, per_channel, floor_in_dtype, st)
-        : dtype == MQ_F16 ? fp8_scaled_any<MQ_F16>(w, ldw, (uint8_t*)q, scale, ws, M, K, per_channel, floor_in_dtype, st)
-                          : fp8_scaled_any<MQ_BF16>(w, ldw, (uint8_t*)q, scale, ws, M, K, per_channel, floor_in_dtype, st))
-        return mq_check_launch("fp8 scaled quant");
     // rows of more than 4096 units or of less than one, strided tensors with one scale
     if (!per_channel) hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, (uint32_t*)amax_ws, 0u, 1);
     hipLaunchKernelGGL(fp8_row_amax_kernel, dim3((unsigned)M), dim3(256), 0, st, w, dtype, ldw, K,

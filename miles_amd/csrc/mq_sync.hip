@@ -45,6 +45,11 @@ bool mq_fp8_tensor_fast_ok(const void* w, int dtype, const void* q, int64_t rows
 int mq_fp8_tensor_launch_group(int dtype, FlatTable& tab, float floor_v, bool carry, hipStream_t st);
 int mq_fp8_tensor_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, float floor_v, bool carry,
                                hipStream_t st);
+int mq_fp8_channel_form(const void* w, int dtype, int64_t ldw, const void* q, int64_t M, int64_t K);
+int64_t mq_fp8_channel_blocks(int form, int64_t M);
+int mq_fp8_channel_launch_group(int dtype, int form, const MqScaledArgs* a, int n, hipStream_t st);
+int mq_fp8_scaled_form(const void* w, int dtype, int64_t ldw, const void* q, int64_t M, int64_t K);
+int mq_fp8_scaled_launch_group(int dtype, int form, const MqScaledArgs* a, int n, int words, hipStream_t st);
 int mq_nvfp4_amax_launch_table(int dtype, const FlatJob* device_jobs, int n, hipStream_t st);
 int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int e4m3_max, int mode,
                                 hipStream_t st);
@@ -134,7 +139,7 @@ constexpr int kNvQuantFlags = MQ_NVFP4_4OVER6 | MQ_NVFP4_ERR_MSE | MQ_NVFP4_ERR_
 
 static int64_t copy_dst_pitch(const mq_job& j);
 static int check_job(const mq_job& j) {
-    if (j.kind < MQ_JOB_FP8_BLOCK || j.kind > MQ_JOB_MXFP4_DEQUANT) return mq_fail(MQ_ERR_ARG, "unknown job kind");
+    if (j.kind < MQ_JOB_FP8_BLOCK || j.kind > MQ_JOB_FP8_SCALED) return mq_fail(MQ_ERR_ARG, "unknown job kind");
     if (j.rows < 0 || j.cols < 0) return mq_fail(MQ_ERR_ARG, "job with a negative shape");
     const bool empty = j.rows == 0 || j.cols == 0;       // an empty tensor has no address
     if ((!j.in || !j.out) && !empty) return mq_fail(MQ_ERR_ARG, "job with a null tensor pointer");
@@ -161,6 +166,14 @@ static int check_job(const mq_job& j) {
         if (j.rows_per_block != 0) return mq_fail(MQ_ERR_ARG, "bad MXFP4 to FP8 job");
         RecodeJob probe;
         return mq_mxfp4_to_fp8_job(probe, j.in, j.aux, j.out, j.scale, j.rows, j.cols);
+    }
+    if (j.kind == MQ_JOB_FP8_SCALED) {
+        if (j.rows_per_block != 0 || (j.p1 & ~1) != 0) return mq_fail(MQ_ERR_ARG, "bad FP8 job");
+        if (empty) return MQ_OK;
+        if (j.dtype < MQ_BF16 || j.dtype > MQ_F32) return mq_fail(MQ_ERR_ARG, "bad argument");
+        if (!j.scale || (!j.aux && !(j.p1 && mq_fp8_channel_form(j.in, j.dtype, j.ld, j.out, j.rows, j.cols))))
+            return mq_fail(MQ_ERR_ARG, "FP8 job without a scale pointer or a workspace");
+        return MQ_OK;
     }
     if (!empty && (j.kind == MQ_JOB_FP8_DEQUANT ? !j.aux : !j.scale)) return mq_fail(MQ_ERR_ARG, "job without a scale pointer");
     // (the grouped kernels store a scale byte wherever a group starts: a last group that is cut short has none of its own)
@@ -395,6 +408,49 @@ static int run_fp8_tensor(const mq_job* jobs, int64_t i, int64_t j, const FlatJo
     return MQ_OK;
 }
 
+// per-channel or per-tensor FP8 jobs [i, j) of any alignment and dtype: groups of one form and dtype, of similar size
+static float scaled_floor(const mq_job& j) {
+    float v;
+    memcpy(&v, &j.p0, 4);
+    return v;
+}
+static int run_fp8_scaled(const mq_job* jobs, int64_t i, int64_t j, void* stream) {
+    static_assert(MQ_FP8_SCALED_WORDS == 256, "kScaledWords: a word for each workgroup of the amax pass");
+    auto form_of = [](const mq_job& b) {
+        return b.p1 ? mq_fp8_channel_form(b.in, b.dtype, b.ld, b.out, b.rows, b.cols) : mq_fp8_scaled_form(b.in, b.dtype, b.ld, b.out, b.rows, b.cols);
+    };
+    while (i < j) {
+        const mq_job& head = jobs[i];
+        if (head.rows == 0 || head.cols == 0) { i++; continue; }
+        const int form = form_of(head);
+        int rc;
+        if (form == 0) {
+            rc = mq_fp8_scaled_quant(head.in, head.dtype, head.ld, head.out, (float*)head.scale, head.aux, head.rows, head.cols, head.p1,
+                                     scaled_floor(head), stream);
+            if (rc) return rc;
+            i++;
+            continue;
+        }
+        MqScaledArgs a[kMaxGroup];
+        int64_t k = i, sum = 0, mx = 0;
+        for (; k < j && k - i < kMaxGroup; k++) {
+            const mq_job& b = jobs[k];
+            if (b.rows == 0 || b.cols == 0 || b.p1 != head.p1 || b.dtype != head.dtype || form_of(b) != form) break;
+            // workgroups (per channel) or elements: padding of the 2-D grid under 25 %
+            const int64_t e = b.p1 ? mq_fp8_channel_blocks(form, b.rows) : b.rows * b.cols, nmx = e > mx ? e : mx;
+            if (k > i && nmx * (k - i + 1) * 4 > (sum + e) * 5) break;
+            sum += e;
+            mx = nmx;
+            a[k - i] = MqScaledArgs{b.in, b.out, (float*)b.scale, (uint32_t*)b.aux, b.ld, b.rows, b.cols, scaled_floor(b)};
+        }
+        rc = head.p1 ? mq_fp8_channel_launch_group(head.dtype, form, a, (int)(k - i), (hipStream_t)stream)
+                     : mq_fp8_scaled_launch_group(head.dtype, form, a, (int)(k - i), MQ_FP8_SCALED_WORDS, (hipStream_t)stream);
+        if (rc) return rc;
+        i = k;
+    }
+    return MQ_OK;
+}
+
 // NVFP4 run [i, j): all jobs fast or not, processed as amax-phase then quantize-phase per chunk
 // (`table`: the device descriptors of jobs[0..), or null; n_all: length of the whole list, for the section lookup)
 static int run_nvfp4(const mq_job* jobs, int64_t n_all, int64_t i, int64_t j, const FlatJob* table, void* stream) {
@@ -572,10 +628,12 @@ extern "C" int mq_run_jobs_tabled(const mq_job* jobs, int64_t n, const void* dev
     int64_t i = 0;
     while (i < n) {
         const mq_job& head = jobs[i];
-        if (head.kind == MQ_JOB_NVFP4 || head.kind == MQ_JOB_FP8_TENSOR) {
+        if (head.kind == MQ_JOB_NVFP4 || head.kind == MQ_JOB_FP8_TENSOR || head.kind == MQ_JOB_FP8_SCALED) {
             int64_t j = i + 1;
             while (j < n && jobs[j].kind == head.kind) j++;
-            int rc = head.kind == MQ_JOB_NVFP4 ? run_nvfp4(jobs, n, i, j, table, stream) : run_fp8_tensor(jobs, i, j, table, stream);
+            int rc = head.kind == MQ_JOB_NVFP4        ? run_nvfp4(jobs, n, i, j, table, stream)
+                     : head.kind == MQ_JOB_FP8_TENSOR ? run_fp8_tensor(jobs, i, j, table, stream)
+                                                      : run_fp8_scaled(jobs, i, j, stream);
             if (rc) return rc;
             i = j;
             continue;

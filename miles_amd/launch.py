@@ -94,6 +94,7 @@ class JobBatch:
         self._table = None      # device copy of the launch descriptors (see freeze)
         self.device = None
         self.direct_calls = 0   # kernels launched inside the block without going through the job list
+        self.kept = False       # made by `recording()`: its caller runs it, perhaps again and again
         self.constants: set[int] = set()   # addresses of result tensors whose contents never depend on the weights
 
     def __len__(self) -> int:
@@ -243,6 +244,12 @@ def active_batch() -> JobBatch | None:
     return getattr(_state, "batch", None)
 
 
+def records_for_replay() -> bool:
+    """Whether jobs are being recorded for a caller that keeps the list and may run it again (`recording()`)."""
+    batch = active_batch()
+    return batch is not None and batch.kept
+
+
 @contextlib.contextmanager
 def deferred():
     """Record the quantizer calls made inside the block and submit them together on exit.
@@ -270,6 +277,7 @@ def recording():
     if active_batch() is not None:
         raise _lib.MilesQuantError("recording() cannot start inside another batch")
     batch = JobBatch()
+    batch.kept = True
     _state.batch = batch
     try:
         yield batch
@@ -295,14 +303,18 @@ def note_constant(t: torch.Tensor) -> None:
 
 
 def submit(kind, inp: torch.Tensor, out: torch.Tensor, scale, aux, aux2, rows, cols, ld, p0=0, p1=0,
-           rows_per_block=0, block_stride=0, dtype=None) -> None:
+           rows_per_block=0, block_stride=0, dtype=None, replayable=True) -> None:
     """Run (or record) one job.  Tensor arguments may be None where the job kind has no such operand; `dtype` is the
-    job's dtype code where that is not the input tensor's (the scales' dtype of an INT4 unpacking job)."""
+    job's dtype code where that is not the input tensor's (the scales' dtype of an INT4 unpacking job).  A job that is not
+    `replayable` joins the list of a `deferred()` block only; inside `recording()` it runs at once, as a direct call."""
     rec = (kind, _lib.DTYPE_CODE.get(inp.dtype, 0) if dtype is None else dtype, inp.data_ptr(), out.data_ptr(),
            scale.data_ptr() if scale is not None else None, aux.data_ptr() if aux is not None else None,
            aux2.data_ptr() if aux2 is not None else None, rows, cols, ld, p0, p1, rows_per_block, block_stride)
     keep = [t for t in (inp, out, scale, aux, aux2) if t is not None]
     batch = active_batch()
+    if batch is not None and batch.kept and not replayable:
+        batch.direct_calls += 1
+        batch = None
     if batch is not None:
         if batch.device is None:
             batch.device = inp.device

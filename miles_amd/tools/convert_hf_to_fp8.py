@@ -45,11 +45,9 @@ def block_fp8(weight: torch.Tensor, block_size):
     return q, scale
 
 
-# clamp(min=1e-12) acts in the weight dtype (fp16 has no such value): the floor, and its fp32 bit pattern
-_FLOORS = {}
-for _dtype in (torch.bfloat16, torch.float16, torch.float32):
-    _floor = torch.tensor(1e-12, dtype=_dtype).float()
-    _FLOORS[_dtype] = float(_floor), int(_floor.view(torch.int32))
+# clamp(min=1e-12) acts in the weight dtype (fp16 has no such value): the fp32 bit pattern of that floor
+_FLOORS = {dtype: int(torch.tensor(1e-12, dtype=dtype).float().view(torch.int32))
+           for dtype in (torch.bfloat16, torch.float16, torch.float32)}
 _AMAX_RECORD_WORDS = 1280   # MQ_NVFP4_RECORD_WORDS: partial maxima of a tensor on the device, then its folded amax
 
 
@@ -64,18 +62,20 @@ def _scaled_fp8(weight: torch.Tensor, per_channel: bool):
     w = weight if weight.stride(1) == 1 else weight.contiguous()
     q = torch.empty((n, k), dtype=torch.float8_e4m3fn, device=w.device)
     scale = torch.empty((n, 1) if per_channel else (1,), dtype=torch.float32, device=w.device)
-    floor, floor_bits = _FLOORS.get(w.dtype, (0.0, 0))      # (another dtype is refused below)
-    if not per_channel and w.dtype in (torch.bfloat16, torch.float16) and w.is_contiguous() and k % 8 == 0 and w.data_ptr() % 16 == 0:
-        # a job of the batched driver (grouped launches, replayable): amax record as for NVFP4
+    floor_bits = _FLOORS.get(w.dtype, 0)      # (another dtype is refused below)
+    if (not per_channel and launch.records_for_replay() and w.dtype in (torch.bfloat16, torch.float16) and w.is_contiguous()
+            and k % 8 == 0 and w.data_ptr() % 16 == 0):
+        # a list that may run again: with an amax record, as for NVFP4, so that later runs read the tensor once
         record = torch.empty(_AMAX_RECORD_WORDS, dtype=torch.int32, device=w.device)
         launch.submit(_lib.JOB_FP8_TENSOR, w, q, scale, record, None, n, k, k, floor_bits, 0)
         return q, scale
-    ws = torch.empty(max(n, 1), dtype=torch.int32, device=w.device)
-    launch.note_direct_call()
-    rc = _lib.load().mq_fp8_scaled_quant(w.data_ptr(), _lib.dtype_code(w, "fp8"), w.stride(0), q.data_ptr(),
-                                         scale.data_ptr(), ws.data_ptr(), n, k, int(per_channel), floor,
-                                         _lib.stream_ptr(w.device))
-    _lib.check(rc)
+    _lib.dtype_code(w, "fp8")
+    unit = 4 if w.dtype == torch.float32 else 8
+    ws = None
+    if not per_channel or not unit <= k <= 4096 * unit:     # rows of 16-byte units are held in registers
+        ws = torch.empty(max(n, _lib.FP8_SCALED_WORDS), dtype=torch.int32, device=w.device)
+    launch.submit(_lib.JOB_FP8_SCALED, w, q, scale, ws, None, n, k, w.stride(0), floor_bits, int(per_channel),
+                  replayable=False)
     return q, scale
 
 

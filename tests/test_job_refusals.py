@@ -96,3 +96,14 @@ def test_a_slice_of_a_stack_serves_its_own_matrix():
 def test_nvfp4_weights_of_another_rank(shape, error):
     with pytest.raises(error):
         nvfp4.nvfp4_quantize_1d(torch.zeros(shape, device="cuda", dtype=torch.bfloat16))
+
+
+@pytest.mark.parametrize("dtype, cols, p1, workspace, rows_per_block", [
+    (3, 64, 1, True, 0), (-1, 64, 0, True, 0), (0, 64, 2, True, 0), (0, 64, 1, True, 128), (0, 64, 0, False, 0), (0, 7, 1, False, 0),
+    (2, 3, 1, False, 0), (2, 16388, 1, False, 0)])
+def test_scaled_fp8_jobs(dtype, cols, p1, workspace, rows_per_block):
+    """An unknown dtype or flag, row blocks, and a missing workspace where a row is not held in registers."""
+    keep, inp, out, scale = _addresses(1 << 16)
+    aux = scale if workspace else None
+    job = (_lib.Job * 1)(_lib.Job(_lib.JOB_FP8_SCALED, dtype, inp, out, scale, aux, None, 2, cols, cols, 0, p1, rows_per_block, 0))
+    assert _lib.load().mq_run_jobs(ctypes.byref(job), 1, None) == MQ_ERR_ARG
