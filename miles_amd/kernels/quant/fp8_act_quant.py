@@ -12,6 +12,7 @@ from __future__ import annotations
 import torch
 
 from miles_amd import _lib, launch
+from miles_amd._host import native
 
 ACT_ROUND_SCALE, ACT_SCALE_E8M0, ACT_INPLACE = 1, 2, 4     # flags of mq_fp8_act_quant
 
@@ -38,6 +39,10 @@ def act_quant(x: torch.Tensor, block_size: int = 128, scale_fmt: str | None = No
         raise ValueError("float8_e8m0fnu scales need scale_fmt (power-of-two scales)")
     flags = (ACT_ROUND_SCALE if scale_fmt is not None else 0) | (ACT_SCALE_E8M0 if e8m0 else 0)
     z = x.contiguous()
+    if not inplace and not torch.compiler.is_dynamo_compiling():
+        made = native.act_quant(z, block_size, flags, scale_dtype)
+        if made is not None:
+            return made
     s = z.new_empty(*z.size()[:-1], n // block_size, dtype=scale_dtype)
     if inplace:
         _run(z, z, s, block_size, flags | ACT_INPLACE)
@@ -72,4 +77,11 @@ class DeepSeekV4LinearQATFunc(torch.autograd.Function):
         return grad_kv, None
 
 
-fp8_simulate_qat = DeepSeekV4LinearQATFunc.apply
+def fp8_simulate_qat(*args):
+    """`DeepSeekV4LinearQATFunc.apply(kv, block_size=128)`, for an ordinary tensor with its graph node made in native code."""
+    if 0 < len(args) < 3 and not torch.compiler.is_dynamo_compiling():
+        out = native.simulate(args[0], *args[1:], ACT_ROUND_SCALE | ACT_INPLACE) if len(args) == 2 else \
+            native.simulate(args[0], 128, ACT_ROUND_SCALE | ACT_INPLACE)
+        if out is not None:
+            return out
+    return DeepSeekV4LinearQATFunc.apply(*args)

@@ -10,6 +10,7 @@ from __future__ import annotations
 import torch
 
 from miles_amd import _lib, launch
+from miles_amd._host import native
 
 
 def fake_int4_quant_cuda(x: torch.Tensor, block_size, sym: bool):
@@ -24,11 +25,15 @@ def fake_int4_quant_cuda(x: torch.Tensor, block_size, sym: bool):
     if (block_m * block_n) % 32 != 0:
         raise RuntimeError(f"block_m * block_n ({block_m * block_n}) must be divisible by 32. "
                            f"But got a {block_m}x{block_n} block.")
+    if not torch.compiler.is_dynamo_compiling():
+        made = native.int4_fake(x, block_m, block_n, bool(sym))      # (`zero` is left unwritten in symmetric mode, as in the reference)
+        if made is not None:
+            return made
     M, N = x.shape
     xc = x.contiguous()
     out = torch.empty_like(xc)
     scale = torch.empty((-(-M // block_m), -(-N // block_n)), dtype=x.dtype, device=x.device)
-    zero = torch.empty_like(scale)  # left unwritten in symmetric mode, as in the reference
+    zero = torch.empty_like(scale)
     launch.note_direct_call()
     rc = _lib.load().mq_int4_fake_quant(xc.data_ptr(), _lib.dtype_code(x, "fake_int4_quant_cuda"), out.data_ptr(),
                                         scale.data_ptr(), zero.data_ptr(), M, N, block_m, block_n, int(bool(sym)),
@@ -56,11 +61,8 @@ def pack_layer(weight: torch.Tensor, group_size: int, sym: bool = True):
     if K % group_size != 0 or K % 8 != 0:
         raise RuntimeError(f"shape {tuple(weight.shape)} is not divisible into groups of {group_size} and words of 8")
     w = weight.contiguous()
-    packed = torch.empty((M, K // 8), dtype=torch.int32, device=w.device)
-    scale = torch.empty((M, K // group_size), dtype=w.dtype, device=w.device)
     _lib.dtype_code(w, "pack_layer")
-    launch.submit(_lib.JOB_INT4_PACK, w, packed, scale, None, None, M, K, K, int(group_size), 0)
-    return packed, scale, None
+    return *launch.produce(_lib.JOB_INT4_PACK, w, M, K, K, int(group_size), 0, (torch.int32, M, K // 8), (w.dtype, M, K // group_size)), None
 
 
 def _pack_layer_asym(weight: torch.Tensor, group_size: int):
@@ -70,10 +72,7 @@ def _pack_layer_asym(weight: torch.Tensor, group_size: int):
                            f"words of 8 and zero-point words of 8 rows")
     w = weight.contiguous()
     groups = K // group_size
-    packed = torch.empty((M, K // 8), dtype=torch.int32, device=w.device)
-    scale = torch.empty((M, groups), dtype=w.dtype, device=w.device)
-    zero = torch.empty((M, groups), dtype=torch.uint8, device=w.device)
-    packed_zp = torch.empty((groups, M // 8), dtype=torch.int32, device=w.device)
     _lib.dtype_code(w, "pack_layer")
-    launch.submit(_lib.JOB_INT4_PACK_ASYM, w, packed, scale, zero, packed_zp, M, K, K, int(group_size), 0)
+    packed, scale, _zero, packed_zp = launch.produce(_lib.JOB_INT4_PACK_ASYM, w, M, K, K, int(group_size), 0, (torch.int32, M, K // 8),
+                                                     (w.dtype, M, groups), (torch.uint8, M, groups), (torch.int32, groups, M // 8))
     return packed, scale, packed_zp

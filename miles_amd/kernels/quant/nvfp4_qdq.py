@@ -18,6 +18,7 @@ from enum import IntEnum
 import torch
 
 from miles_amd import _lib, launch
+from miles_amd._host import native
 
 _FP4_BLOCK_SIZE = 16
 
@@ -174,10 +175,14 @@ class _QDQStraightThrough(torch.autograd.Function):
 
 def fake_nvfp4_quantization_ste_list(weights: list[torch.Tensor], config: NVFP4QDQConfig) -> list[torch.Tensor] | None:
     """`fake_nvfp4_quantization_ste` of every weight of a list that can share launches, or None if it cannot."""
-    if not weights or not _groupable(weights):
-        return None
-    images = iter(_images(weights, config))
-    outputs = [_QDQStraightThrough.apply(w, images) for w in weights]
+    outputs = None
+    if type(config) is NVFP4QDQConfig and not torch.compiler.is_dynamo_compiling():      # ordinary tensors: images and graph nodes, one for each weight, in native code
+        outputs = native.nvfp4_images(weights, _FP4_BLOCK_SIZE, _SECTION_WORDS, config.e4m3_max, _flags(config))
+    if outputs is None:
+        if not weights or not _groupable(weights):
+            return None
+        images = iter(_images(weights, config))
+        outputs = [_QDQStraightThrough.apply(w, images) for w in weights]
     for w, output in zip(weights, outputs):
         if hasattr(w, "main_grad"):
             output.main_grad = w.main_grad

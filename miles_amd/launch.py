@@ -17,6 +17,7 @@ import threading
 import torch
 
 from miles_amd import _lib
+from miles_amd._host import native
 
 _state = threading.local()
 
@@ -85,8 +86,9 @@ class JobBatch:
     """An ordered list of mq_job records plus the tensors they reference."""
 
     def __init__(self) -> None:
-        self._records: list[tuple] = []
-        self._keep: list[torch.Tensor] = []
+        self._list: list[tuple] = []
+        self._held: list[torch.Tensor] = []
+        self._recorder = None      # of a `deferred()` block: jobs recorded in native code, behind those of the list
         self._array = None
         self._array_plain = None   # the same list without MQ_NVFP4_CARRY_AMAX (see carry_amax)
         self._feedback: _AmaxFeedback | None = None
@@ -98,7 +100,27 @@ class JobBatch:
         self.constants: set[int] = set()   # addresses of result tensors whose contents never depend on the weights
 
     def __len__(self) -> int:
-        return len(self._records)
+        return len(self._list) + (len(self._recorder) if self._recorder is not None else 0)
+
+    def _absorb(self) -> None:
+        """Take over what native code has recorded, so that the list is in the order of the calls."""
+        if self._recorder is not None and len(self._recorder):
+            records, held, index = self._recorder.take()
+            self._list.extend(records)
+            self._held.extend(held)
+            self._array = None
+            if self.device is None:
+                self.device = torch.device("cuda", index)
+
+    @property
+    def _records(self) -> list[tuple]:
+        self._absorb()
+        return self._list
+
+    @property
+    def _keep(self) -> list[torch.Tensor]:
+        self._absorb()
+        return self._held
 
     def add(self, kind, dtype, inp, out, scale, aux, aux2, rows, cols, ld, p0, p1, rows_per_block=0,
             block_stride=0, keep=()) -> None:
@@ -118,9 +140,10 @@ class JobBatch:
     def replace_records(self, records: list[tuple], keep: list[torch.Tensor] | None = None) -> None:
         """Swap in an edited job list (a planner re-pointing outputs, adding copy jobs); `keep` replaces the tensors
         the batch holds alive."""
-        self._records = list(records)
+        self._absorb()
+        self._list = list(records)
         if keep is not None:
-            self._keep = list(keep)
+            self._held = list(keep)
         self._array = None
 
     def carry_amax(self, adaptive: bool = True) -> int:
@@ -143,8 +166,8 @@ class JobBatch:
         kinds = {_lib.JOB_FP8_TENSOR} | ({_lib.JOB_NVFP4} if nv_fit else set())
         flagged = sum(r[self.KIND] in kinds for r in self._records)
         if flagged:
-            self._records = [r[: self.P1] + (r[self.P1] | _lib.NVFP4_CARRY_AMAX,) + r[self.P1 + 1:]
-                             if r[self.KIND] in kinds else r for r in self._records]
+            self._list = [r[: self.P1] + (r[self.P1] | _lib.NVFP4_CARRY_AMAX,) + r[self.P1 + 1:]
+                          if r[self.KIND] in kinds else r for r in self._records]
             self._array = None
             self._array_plain = None
             if adaptive and self.device is not None and self.device.type == "cuda":
@@ -199,7 +222,13 @@ class JobBatch:
         tabled = self._table is not None and self._records[index][self.KIND] in self._TABLE_KINDS
         return _lib.TABLE_GROUP if tabled else _lib.MAX_GROUP
 
+    _TABLE_MASK = sum(1 << kind for kind in _TABLE_KINDS if kind != _lib.JOB_COPY)
+
     def run(self, stream: int | None = None) -> None:
+        recorder = self._recorder
+        if recorder is not None and not self._list and stream is None and recorder.count(self._TABLE_MASK) <= _lib.MAX_GROUP:
+            recorder.run()          # the list is whole as it is, and too short for a device table
+            return
         self.run_range(0, len(self._records), stream)
 
     def run_range(self, start: int, stop: int, stream: int | None = None) -> None:
@@ -250,24 +279,31 @@ def records_for_replay() -> bool:
     return batch is not None and batch.kept
 
 
-@contextlib.contextmanager
-def deferred():
+class deferred:
     """Record the quantizer calls made inside the block and submit them together on exit.
 
     Inside an enclosing `deferred()` / `recording()` block this is a pass-through: the jobs join the outer
     batch and run when that one does.
     """
-    outer = active_batch()
-    if outer is not None:
-        yield outer
-        return
-    batch = JobBatch()
-    _state.batch = batch
-    try:
-        yield batch
-    finally:
-        _state.batch = None
-    batch.run()
+
+    def __enter__(self) -> JobBatch:
+        outer = active_batch()
+        self._own = None if outer is not None else JobBatch()
+        if self._own is None:
+            return outer
+        self._own._recorder = native.Recorder()
+        native.enter(self._own._recorder)
+        _state.batch = self._own
+        return self._own
+
+    def __exit__(self, kind, value, traceback) -> bool:
+        batch, self._own = self._own, None
+        if batch is not None:
+            _state.batch = None
+            native.leave()
+            if kind is None:
+                batch.run()
+        return False
 
 
 @contextlib.contextmanager
@@ -278,11 +314,13 @@ def recording():
         raise _lib.MilesQuantError("recording() cannot start inside another batch")
     batch = JobBatch()
     batch.kept = True
+    native.enter(None)
     _state.batch = batch
     try:
         yield batch
     finally:
         _state.batch = None
+        native.leave()
 
 
 def note_direct_call() -> None:
@@ -307,6 +345,8 @@ def submit(kind, inp: torch.Tensor, out: torch.Tensor, scale, aux, aux2, rows, c
     """Run (or record) one job.  Tensor arguments may be None where the job kind has no such operand; `dtype` is the
     job's dtype code where that is not the input tensor's (the scales' dtype of an INT4 unpacking job).  A job that is not
     `replayable` joins the list of a `deferred()` block only; inside `recording()` it runs at once, as a direct call."""
+    if native.submit(kind, dtype, inp, out, scale, aux, aux2, rows, cols, ld, p0, p1, rows_per_block, block_stride):
+        return
     rec = (kind, _lib.DTYPE_CODE.get(inp.dtype, 0) if dtype is None else dtype, inp.data_ptr(), out.data_ptr(),
            scale.data_ptr() if scale is not None else None, aux.data_ptr() if aux is not None else None,
            aux2.data_ptr() if aux2 is not None else None, rows, cols, ld, p0, p1, rows_per_block, block_stride)
@@ -322,3 +362,16 @@ def submit(kind, inp: torch.Tensor, out: torch.Tensor, scale, aux, aux2, rows, c
         return
     one = (_lib.Job * 1)(_lib.Job(*rec))
     _lib.check(_lib.load().mq_run_jobs(one, 1, _lib.stream_ptr(inp.device)))
+
+
+def produce(kind, inp: torch.Tensor, rows, cols, ld, p0, p1, out, scale=None, aux=None, aux2=None, *, aux_in=None, dtype=None,
+            replayable=True) -> tuple[torch.Tensor, ...]:
+    """Make the outputs of one job, given as `(dtype, *sizes)`, run or record it (`submit`), and return them.  `aux_in`: an
+    input tensor in the place of `aux`."""
+    made = native.produce(kind, dtype, inp, aux_in, rows, cols, ld, p0, p1, out, scale, aux, aux2)
+    if made is not None:
+        return made
+    tensors = [None if spec is None else torch.empty(spec[1:], dtype=spec[0], device=inp.device) for spec in (out, scale, aux, aux2)]
+    submit(kind, inp, tensors[0], tensors[1], tensors[2] if aux_in is None else aux_in, tensors[3], rows, cols, ld, p0, p1,
+           dtype=dtype, replayable=replayable)
+    return tuple(t for t in tensors if t is not None)

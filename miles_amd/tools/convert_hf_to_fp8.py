@@ -38,11 +38,9 @@ def block_fp8(weight: torch.Tensor, block_size):
     bn, bk = int(block_size[0]), int(block_size[1])
     n, k = weight.shape
     w = weight if weight.stride(1) == 1 else weight.contiguous()
-    q = torch.empty((n, k), dtype=torch.float8_e4m3fn, device=w.device)
-    scale = torch.empty((ceildiv(n, bn), ceildiv(k, bk)), dtype=torch.float32, device=w.device)
     _lib.dtype_code(w, "block_fp8")
-    launch.submit(_lib.JOB_FP8_BLOCK, w, q, scale, None, None, n, k, w.stride(0), bn, bk)
-    return q, scale
+    return launch.produce(_lib.JOB_FP8_BLOCK, w, n, k, w.stride(0), bn, bk, (torch.float8_e4m3fn, n, k),
+                          (torch.float32, ceildiv(n, bn), ceildiv(k, bk)))
 
 
 # clamp(min=1e-12) acts in the weight dtype (fp16 has no such value): the fp32 bit pattern of that floor
@@ -60,23 +58,19 @@ def _scaled_fp8(weight: torch.Tensor, per_channel: bool):
     if per_channel and k == 0:
         raise RuntimeError("amax(): Expected reduction dim 1 to have non-zero size.")
     w = weight if weight.stride(1) == 1 else weight.contiguous()
-    q = torch.empty((n, k), dtype=torch.float8_e4m3fn, device=w.device)
-    scale = torch.empty((n, 1) if per_channel else (1,), dtype=torch.float32, device=w.device)
+    codes, scales = (torch.float8_e4m3fn, n, k), (torch.float32, n, 1) if per_channel else (torch.float32, 1)
     floor_bits = _FLOORS.get(w.dtype, 0)      # (another dtype is refused below)
     if (not per_channel and launch.records_for_replay() and w.dtype in (torch.bfloat16, torch.float16) and w.is_contiguous()
             and k % 8 == 0 and w.data_ptr() % 16 == 0):
         # a list that may run again: with an amax record, as for NVFP4, so that later runs read the tensor once
-        record = torch.empty(_AMAX_RECORD_WORDS, dtype=torch.int32, device=w.device)
-        launch.submit(_lib.JOB_FP8_TENSOR, w, q, scale, record, None, n, k, k, floor_bits, 0)
-        return q, scale
+        return launch.produce(_lib.JOB_FP8_TENSOR, w, n, k, k, floor_bits, 0, codes, scales, (torch.int32, _AMAX_RECORD_WORDS))[:2]
     _lib.dtype_code(w, "fp8")
     unit = 4 if w.dtype == torch.float32 else 8
     ws = None
     if not per_channel or not unit <= k <= 4096 * unit:     # rows of 16-byte units are held in registers
-        ws = torch.empty(max(n, _lib.FP8_SCALED_WORDS), dtype=torch.int32, device=w.device)
-    launch.submit(_lib.JOB_FP8_SCALED, w, q, scale, ws, None, n, k, w.stride(0), floor_bits, int(per_channel),
-                  replayable=False)
-    return q, scale
+        ws = (torch.int32, max(n, _lib.FP8_SCALED_WORDS))
+    return launch.produce(_lib.JOB_FP8_SCALED, w, n, k, w.stride(0), floor_bits, int(per_channel), codes, scales, ws,
+                          replayable=False)[:2]
 
 
 def channel_fp8(weight: torch.Tensor):

@@ -52,11 +52,9 @@ def _dequantize_tensor(weight_packed: torch.Tensor, weight_scale: torch.Tensor, 
         scale = scale.unsqueeze(1)
     if K % group_size != 0 or scale.numel() != M * (K // group_size):
         raise ValueError(f"Scale shape {tuple(scale.shape)} incompatible with weight shape {shape}")
-    out = torch.empty((M, K), dtype=torch.bfloat16, device=packed.device)
     # a job of the batched driver: inside `launch.deferred()` the experts of a whole shard share grouped launches
-    launch.submit(_lib.JOB_INT4_UNPACK, packed, out, None, scale, None, M, K, K, int(group_size),
-                  dtype=_lib.dtype_code(scale, "_dequantize_tensor"))
-    return out
+    return launch.produce(_lib.JOB_INT4_UNPACK, packed, M, K, K, int(group_size), 0, (torch.bfloat16, M, K), aux_in=scale,
+                          dtype=_lib.dtype_code(scale, "_dequantize_tensor"))[0]
 
 
 _PROJECTIONS = ("gate_proj", "up_proj", "down_proj")

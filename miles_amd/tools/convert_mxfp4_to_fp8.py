@@ -37,11 +37,9 @@ def cast_e2m1fn_to_e4m3fn(x: torch.Tensor, scale: torch.Tensor) -> tuple[torch.T
     packed, sbytes = x.contiguous(), scale.contiguous().view(torch.uint8)
     if packed.data_ptr() % 16:        # the kernel reads whole 16-byte pieces: a view that starts mid-allocation is moved first
         packed = packed.clone()
-    y = torch.empty((out_dim, in_dim), dtype=torch.float8_e4m3fn, device=x.device)
-    tile_scale = torch.empty((out_dim // 128, in_dim // 128), dtype=torch.float32, device=x.device)
     # a job of the batched driver: inside `launch.deferred()` the casts of a whole shard share grouped launches
-    launch.submit(_lib.JOB_MXFP4_TO_FP8, packed, y, tile_scale, sbytes, None, out_dim, in_dim, in_dim)
-    return y, tile_scale
+    return launch.produce(_lib.JOB_MXFP4_TO_FP8, packed, out_dim, in_dim, in_dim, 0, 0, (torch.float8_e4m3fn, out_dim, in_dim),
+                          (torch.float32, out_dim // 128, in_dim // 128), aux_in=sbytes)
 
 
 def _copy_side_files(model_dir: Path, save_dir: Path) -> None:

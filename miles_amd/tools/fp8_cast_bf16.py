@@ -33,9 +33,7 @@ def weight_dequant(x: torch.Tensor, s: torch.Tensor, block_size: int = 128) -> t
     if s.dtype != torch.float32:
         raise _lib.MilesQuantError(f"weight_dequant expects float32 scales, got {s.dtype}")
     M, N = x.size()
-    y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
-    launch.submit(_lib.JOB_FP8_DEQUANT, x, y, None, s, None, M, N, N, int(block_size), 0)
-    return y
+    return launch.produce(_lib.JOB_FP8_DEQUANT, x, M, N, N, int(block_size), 0, (torch.bfloat16, M, N), aux_in=s)[0]
 
 
 def main(fp8_path, bf16_path, remap=lambda name: name, device="cuda"):

@@ -22,11 +22,9 @@ def quantize_mxfp4(weight: torch.Tensor, group_size: int):
     w = weight.contiguous()
     k = w.shape[-1]
     rows = w.numel() // k if k else 0
-    packed = torch.empty((*w.shape[:-1], k // 2), dtype=torch.uint8, device=w.device)
-    scale = torch.empty((*w.shape[:-1], k // group_size), dtype=torch.uint8, device=w.device)
     _lib.dtype_code(w, "quantize_mxfp4")
-    launch.submit(_lib.JOB_MXFP4, w, packed, scale, None, None, rows, k, k, int(group_size), 0)
-    return packed, scale
+    return launch.produce(_lib.JOB_MXFP4, w, rows, k, k, int(group_size), 0, (torch.uint8, *w.shape[:-1], k // 2),
+                          (torch.uint8, *w.shape[:-1], k // group_size))
 
 
 def dequantize_mxfp4(weight_packed: torch.Tensor, weight_scale: torch.Tensor, group_size: int) -> torch.Tensor:
@@ -42,8 +40,8 @@ def dequantize_mxfp4(weight_packed: torch.Tensor, weight_scale: torch.Tensor, gr
     numel = packed.numel() * 2
     assert numel % group_size == 0
     assert scale.numel() == numel // group_size
-    out = torch.empty((*packed.shape[:-1], packed.shape[-1] * 2), dtype=torch.bfloat16, device=packed.device)
+    sizes = (*packed.shape[:-1], packed.shape[-1] * 2)
+    if not numel:
+        return torch.empty(sizes, dtype=torch.bfloat16, device=packed.device)
     # a job of the batched driver: inside `launch.deferred()` the tensors of a whole shard share grouped launches
-    if numel:
-        launch.submit(_lib.JOB_MXFP4_DEQUANT, packed, out, None, scale, None, 1, numel, numel, int(group_size))
-    return out
+    return launch.produce(_lib.JOB_MXFP4_DEQUANT, packed, 1, numel, numel, int(group_size), 0, (torch.bfloat16, *sizes), aux_in=scale)[0]

@@ -48,11 +48,9 @@ def mxfp8_quantize(weight: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     _lib.require_gpu(weight, "mxfp8_quantize")
     w = weight.contiguous()
     rows = w.numel() // k if k else 0
-    q = torch.empty(w.shape, dtype=torch.float8_e4m3fn, device=w.device)
-    scale = torch.empty((*w.shape[:-1], k // MXFP8_GROUP_SIZE), dtype=torch.uint8, device=w.device)
     _lib.dtype_code(w, "mxfp8_quantize")
-    launch.submit(_lib.JOB_MXFP8, w, q, scale, None, None, rows, k, k)
-    return q, scale
+    return launch.produce(_lib.JOB_MXFP8, w, rows, k, k, 0, 0, (torch.float8_e4m3fn, *w.shape),
+                          (torch.uint8, *w.shape[:-1], k // MXFP8_GROUP_SIZE))
 
 
 # ---- FP8 128x128 block-scaled sources (tools/convert_hf_to_mxfp8.py:56-102,180-195) ---------------------------------
@@ -145,12 +143,12 @@ def requantize_fp8_block_to_mxfp8(weight: torch.Tensor, scale: torch.Tensor) -> 
     if scale.dtype != torch.float32:
         raise ValueError(f"expected fp32 tile scales, got {scale.dtype}")
     n = _check_grid(weight, scale)[0]
-    q = torch.empty(weight.shape, dtype=torch.float8_e4m3fn, device=weight.device)
-    out_scale = torch.empty((*weight.shape[:-1], k // MXFP8_GROUP_SIZE), dtype=torch.uint8, device=weight.device)
     if weight.dim() == 2 and weight.is_contiguous() and scale.is_contiguous() and weight.numel() > 0:
         # one matrix as a checkpoint holds it: none of the views below, which take the host longer than the GPU needs
-        launch.submit(_lib.JOB_FP8_TO_MXFP8, weight, q, out_scale, scale, None, n, k, scale.shape[1])
-        return q, out_scale
+        return launch.produce(_lib.JOB_FP8_TO_MXFP8, weight, n, k, scale.shape[1], 0, 0, (torch.float8_e4m3fn, n, k),
+                              (torch.uint8, n, k // MXFP8_GROUP_SIZE), aux_in=scale)
+    q = torch.empty(weight.shape, dtype=torch.float8_e4m3fn, device=weight.device)
+    out_scale = torch.empty((*weight.shape[:-1], k // MXFP8_GROUP_SIZE), dtype=torch.uint8, device=weight.device)
     w3, s3, nt, _kt = _grids(weight, scale)
     q3, o3 = q.view(w3.shape[0], n, k), out_scale.view(w3.shape[0], n, k // MXFP8_GROUP_SIZE)
     for b in range(w3.shape[0] if n and k else 0):

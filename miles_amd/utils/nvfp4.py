@@ -103,14 +103,16 @@ def nvfp4_quantize_1d(weight: torch.Tensor, *, out=None) -> tuple[torch.Tensor, 
     rows, cols = w.shape[0], w.shape[1]
     if cols % NVFP4_GROUP_SIZE != 0:
         raise ValueError(f"NVFP4 requires K divisible by {NVFP4_GROUP_SIZE}, got {cols}.")
-    # the amax record is written by the job driver
+    _lib.dtype_code(w, "nvfp4")
+    if out is None:
+        rows, cols = w.shape
+        # (the amax record, third, is written by the job driver)
+        q, block_scale, _record, global_scale = launch.produce(
+            _lib.JOB_NVFP4, w, rows, cols, cols, e4m3_max, flags, (torch.uint8, rows, cols // 2),
+            (torch.float8_e4m3fn, rows, cols // NVFP4_GROUP_SIZE), (torch.int32, AMAX_RECORD_WORDS), (torch.float32,))
+        return q, block_scale, global_scale
     word = out.record if in_stack else torch.empty(AMAX_RECORD_WORDS, dtype=torch.int32, device=w.device)
-    if in_stack:
-        _lib.dtype_code(w, "nvfp4")
-    elif out is None:
-        out = _alloc_outputs(w)
-    else:
-        _lib.dtype_code(w, "nvfp4")
+    if not in_stack:
         want = ((w.shape[0], w.shape[1] // 2), (w.shape[0], w.shape[1] // NVFP4_GROUP_SIZE), ())
         if any(tuple(t.shape) != shape or not t.is_contiguous() for t, shape in zip(out, want)):
             raise ValueError("nvfp4_quantize_1d: `out` tensors must be contiguous and shaped like the results")

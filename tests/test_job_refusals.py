@@ -107,3 +107,17 @@ def test_scaled_fp8_jobs(dtype, cols, p1, workspace, rows_per_block):
     aux = scale if workspace else None
     job = (_lib.Job * 1)(_lib.Job(_lib.JOB_FP8_SCALED, dtype, inp, out, scale, aux, None, 2, cols, cols, 0, p1, rows_per_block, 0))
     assert _lib.load().mq_run_jobs(ctypes.byref(job), 1, None) == MQ_ERR_ARG
+
+
+def test_the_native_layer_leaves_host_tensors_to_python():
+    """Not on the GPU: every entry of the native layer hands the call back."""
+    from miles_amd._host import native
+
+    x = torch.zeros(4, 32, dtype=torch.bfloat16)
+    assert native.submit(_lib.JOB_MXFP8, None, x, x, x, None, None, 4, 32, 32, 0, 0, 0, 0) is False
+    assert native.produce(_lib.JOB_MXFP8, None, x, None, 4, 32, 32, 0, 0, (torch.uint8, 4, 32), (torch.uint8, 4, 1), None, None) is None
+    assert native.act_quant(x, 32, 0, torch.float32) is None and native.fake_quant(x, 0, 32) is None
+    assert native.simulate(x, 32, 0) is None and native.nvfp4_images([x], 16, 256, 448, 0) is None
+    assert native.nvfp4_images([None], 16, 256, 448, 0) is None and native.fake_quant(None, 0, 32) is None
+    with launch.deferred() as batch:
+        assert len(batch) == 0 and batch.records == []
