@@ -154,7 +154,7 @@ __global__ __launch_bounds__(kFtThreads) void fp8_tensor_quant_kernel(const Tabl
 using namespace mq;
 
 int mq_nvfp4_amax_launch_group(int dtype, FlatTable& tab, hipStream_t st);
-int mq_nvfp4_amax_launch_table(int dtype, const FlatJob* device_jobs, int n, hipStream_t st);
+int mq_nvfp4_amax_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, hipStream_t st);
 
 bool mq_fp8_tensor_fast_ok(const void* w, int dtype, const void* q, int64_t rows, int64_t cols, int64_t ld) {
     return (dtype == MQ_BF16 || dtype == MQ_F16) && cols % 8 == 0 && ld == cols && ((uintptr_t)w % 16) == 0 && ((uintptr_t)q % 8) == 0 &&
@@ -203,7 +203,7 @@ int mq_fp8_tensor_launch_table(int dtype, const FlatJob* device_jobs, int n, int
                                hipStream_t st) {
     if (n == 0) return MQ_OK;
     if (!carry) {
-        int rc = mq_nvfp4_amax_launch_table(dtype, device_jobs, n, st);
+        int rc = mq_nvfp4_amax_launch_table(dtype, device_jobs, n, max_units, st);
         if (rc) return rc;
     }
     FlatRef ref{device_jobs, 0, 0};

@@ -8,12 +8,12 @@
 //
 // Pass 1 (mq_nvfp4_amax): 256 workgroups per tensor stream its elements and each writes one partial maximum
 // into the tensor's section of the amax record: plain stores, no atomics (thousands of agent-scope atomics
-// on one address serialise at ~8 ns each on this multi-XCD part) and nothing to clear.  A one-workgroup-per-
-// record fold kernel turns the partial maxima into the amax, S_enc/6, 1/S_enc and the published global scale.
+// on one address serialise at ~8 ns each on this multi-XCD part) and nothing to clear.
 // Lists of tensors that fit the chip's registers a few at a time run in one pass instead (nvfp4_one_pass_kernel).
-// Pass 2 (mq_nvfp4_quant) reads those two factors with a scalar load; two lanes own one 16-element block
-// (16 bytes each), the block amax is one DPP step, and each lane emits four bytes of codes.  A gate/up pair
-// writes two sections of one record.
+// Pass 2 (mq_nvfp4_quant): every workgroup turns the partial maxima into the amax, S_enc/6 and 1/S_enc while its loads are
+// under way, and each tensor's first one publishes the global scale; two lanes own one 16-element block (16 bytes each), the
+// block amax is one DPP step, and each lane emits four bytes of codes.  A gate/up pair writes two sections of one record.
+// (A launch of its own for the fold took 4.2 us: four [1077, 64] tensors 12.8 -> 8.1 us for the two passes.)
 #include <type_traits>
 
 #include "mq_api_internal.hpp"
@@ -38,11 +38,17 @@ static_assert(kSectionWords == MQ_NVFP4_SECTION_WORDS && kRecordSections == MQ_N
 #endif
 constexpr int kAmaxUnroll = MQ_AMAX_UNROLL;             // 16-byte units per lane per loop trip
 
-// grid (kSectionWords, tensors): workgroup b of a tensor strides over its 16 KiB chunks and writes word b of
-// the section.  job.units counts whole 16-byte units; job.s carries the element count for the sub-unit tail.
+// grid (up to kSectionWords, tensors): workgroup b of a tensor strides over its 16 KiB chunks and writes word b of
+// the section.  A launch whose largest tensor has fewer chunks takes that many workgroups, which write a zero into the
+// words nobody owns (amax_section_store): fifty-nine tensors of 17 chunks 8.7 us with 256 workgroups each, 5.1 with 17.
+// job.units counts whole 16-byte units; job.s carries the element count for the sub-unit tail.
 // (descriptors of a device table are in the quantizer's form, whose tensors are whole units: no tail, and job.s is the
 // block-scale pointer there)
 // (16-bit inputs, bf16 or fp16: the maximum is taken on the absolute bit patterns and converted to the fp32 pattern once)
+__device__ __forceinline__ void amax_section_store(uint32_t* __restrict__ section, int t, uint32_t m) {
+    const uint32_t word = blockIdx.x + (uint32_t)t * gridDim.x;
+    if (word < (uint32_t)kSectionWords) section[word] = t == 0 ? m : 0u;
+}
 template <class Table, int F16>
 __global__ __launch_bounds__(256) void nvfp4_amax_bf16_kernel(const Table tab) {
     __shared__ uint32_t wave_amax[4];
@@ -52,7 +58,7 @@ __global__ __launch_bounds__(256) void nvfp4_amax_bf16_kernel(const Table tab) {
     const int64_t n16 = job.units, numel = std::is_same<Table, FlatRef>::value ? n16 * 8 : (int64_t)(uintptr_t)job.s;
     const int t = threadIdx.x;
     uint32_t m2 = 0;
-    for (int64_t base = (int64_t)blockIdx.x * (256 * kAmaxUnroll); base < n16; base += (int64_t)kSectionWords * 256 * kAmaxUnroll) {
+    for (int64_t base = (int64_t)blockIdx.x * (256 * kAmaxUnroll); base < n16; base += (int64_t)gridDim.x * 256 * kAmaxUnroll) {
         u32x4 v[kAmaxUnroll];
 #pragma unroll
         for (int i = 0; i < kAmaxUnroll; i++) {
@@ -69,7 +75,7 @@ __global__ __launch_bounds__(256) void nvfp4_amax_bf16_kernel(const Table tab) {
     m = wave_max(m);
     if ((t & 63) == 0) wave_amax[t >> 6] = m;
     __syncthreads();
-    if (t == 0) section[blockIdx.x] = f2u(elem_lo<F16>(umax(umax(wave_amax[0], wave_amax[1]), umax(wave_amax[2], wave_amax[3]))));
+    amax_section_store(section, t, f2u(elem_lo<F16>(umax(umax(wave_amax[0], wave_amax[1]), umax(wave_amax[2], wave_amax[3])))));
 }
 
 // fp32 input (units and the element count as above): 16-byte loads of four elements
@@ -81,7 +87,7 @@ __global__ __launch_bounds__(256) void nvfp4_amax_f32_kernel(const Table tab) {
     const int64_t loads = job.units * 2, numel = std::is_same<Table, FlatRef>::value ? job.units * 8 : (int64_t)(uintptr_t)job.s;
     const int t = threadIdx.x;
     uint32_t m = 0;
-    for (int64_t base = (int64_t)blockIdx.x * (256 * kAmaxUnroll); base < loads; base += (int64_t)kSectionWords * 256 * kAmaxUnroll) {
+    for (int64_t base = (int64_t)blockIdx.x * (256 * kAmaxUnroll); base < loads; base += (int64_t)gridDim.x * 256 * kAmaxUnroll) {
         u32x4 v[kAmaxUnroll];
 #pragma unroll
         for (int i = 0; i < kAmaxUnroll; i++) {
@@ -97,8 +103,8 @@ __global__ __launch_bounds__(256) void nvfp4_amax_f32_kernel(const Table tab) {
     m = wave_max(m);
     if ((t & 63) == 0) wave_amax[t >> 6] = m;
     __syncthreads();
-    if (t == 0)
-        ((uint32_t*)job.aux + job.section * kSectionWords)[blockIdx.x] = umax(umax(wave_amax[0], wave_amax[1]), umax(wave_amax[2], wave_amax[3]));
+    amax_section_store((uint32_t*)job.aux + job.section * kSectionWords, t,
+                       umax(umax(wave_amax[0], wave_amax[1]), umax(wave_amax[2], wave_amax[3])));
 }
 
 __global__ __launch_bounds__(256) void nvfp4_amax_generic_kernel(const void* __restrict__ w, int dtype, int64_t numel,
@@ -141,15 +147,78 @@ constexpr int kRecEncSixth = kRecAmax + 1;                     // S_enc * (1/6)
 constexpr int kRecSDec = kRecAmax + 2;                         // 1 / S_enc
 constexpr int kRecEnc = kRecAmax + 3;                          // S_enc
 
+// The tail of a record and the published scales, from the folded amax.
+__device__ __forceinline__ void nv_record_tail(uint32_t* rec, float amax, const NvScales& gs) {
+    rec[kRecAmax] = f2u(amax);
+    rec[kRecEncSixth] = f2u(gs.enc_sixth);
+    rec[kRecSDec] = f2u(gs.s_dec);
+    rec[kRecEnc] = f2u(gs.enc);
+}
+// What a plain run (no carried-over amax) leaves behind, by one lane of every tensor's first workgroup: its own published
+// scale, and for the last tensor of a record (job.section its place there, job.pad the number of tensors that share the
+// record) the record's tail and state words.
+__device__ __forceinline__ void nv_publish_plain(const FlatJob& job, float amax, const NvScales& gs, float numer, uint32_t* moved_counter) {
+    if (job.aux2) *(float*)job.aux2 = nv_published_scale(amax, numer);
+    if (job.section != job.pad - 1) return;
+    uint32_t* rec = (uint32_t*)job.aux;
+    amax_feedback(moved_counter, rec[kRecAmax] != f2u(amax), (uint32_t)job.pad);
+    rec[kRecVolatile] = 0;
+    rec[kRecMovedRuns] = 0;
+    nv_record_tail(rec, amax, gs);
+}
+// an amax and its scales, as the quantizing code below asks for them once its loads are issued
+struct NvAmaxScales {
+    float amax;
+    NvScales gs;
+};
+__device__ __forceinline__ float uniform_f(float v) { return u2f((uint32_t)__builtin_amdgcn_readfirstlane((int)f2u(v))); }
+__device__ __forceinline__ NvAmaxScales nv_record_scales(const FlatJob& job) {
+    const uint32_t* __restrict__ rec = (const uint32_t*)job.aux;
+    return NvAmaxScales{u2f(rec[kRecAmax]), NvScales{u2f(rec[kRecEncSixth]), u2f(rec[kRecSDec]), u2f(rec[kRecEnc])}};
+}
+// The same from the partial maxima of an amax pass, folded by every workgroup of the pass behind it while its data is under
+// way: a launch between the two passes that did it took 4.2 us, and the host's part of one.  Only the first wavefront folds
+// and divides (four words a lane and section), the others wait for its four values in LDS: Four Over Six is bound by vector
+// instructions, and some sixty of them in every wavefront cost it a tenth (fifty [616, 1584] tensors 24.5 us with the scales
+// read from a record, 30.0 folded by all four wavefronts, 27.3 by one).  Scalar registers hold the result, where values read
+// from a record are.
+__device__ __forceinline__ uint32_t nv_wave_fold(const uint32_t* __restrict__ words, int sections, int lane) {
+    uint32_t m = 0;
+    for (int k = 0; k < sections; k++) {
+        const u32x4 v = *reinterpret_cast<const u32x4_at4*>(words + k * kSectionWords + lane * 4);
+        m = umax(m, umax(umax(v.x, v.y), umax(v.z, v.w)));
+    }
+    return wave_max(m);
+}
+template <class AmaxBits>
+__device__ __forceinline__ NvAmaxScales nv_shared_scales(const int t, float numer, AmaxBits first_wave_bits) {
+    static_assert(kSectionWords == 4 * kWave, "a wavefront takes a section in one load");
+    __shared__ float shared[4];
+    if (t < kWave) {
+        const float amax = u2f(first_wave_bits());
+        const NvScales gs = nv_scales(amax, numer);
+        shared[0] = amax;
+        shared[1] = gs.enc_sixth;
+        shared[2] = gs.s_dec;
+        shared[3] = gs.enc;
+    }
+    __syncthreads();
+    return NvAmaxScales{uniform_f(shared[0]), NvScales{uniform_f(shared[1]), uniform_f(shared[2]), uniform_f(shared[3])}};
+}
+
+// A partial maximum that the single pass of a carried run has collected: the amax pass of a plain run leaves its own in the
+// same words, without the mark and below every word with it, so the sections need no clearing between the two.
+constexpr uint32_t kCarriedMark = 0x80000000u;
+
 // Fold kernel, one workgroup per tensor.
-// MODE 0 (single calls): fold the first job.section sections of the record and publish the scales.  Tensors that share
-//   a record compute the same values and write them twice.
-// MODE 1 / 2 (the job driver): job.section is the tensor's place inside its record and job.pad the number of tensors
-//   sharing it; they sit next to each other in the table.  Only the workgroup of the last one works: it folds all their
-//   sections, writes every one's global scale and then clears the sections, so that the next sync may collect its
-//   partial maxima with atomic max (see the carried-over amax below).  MODE 2 additionally checks the amax and scales
-//   the record held before against the new ones: all four words equal means the codes just written with the old values
-//   are final (kRecRedo = 0); otherwise the new values are stored and kRecRedo = 1 asks for a second quantization.
+// MODE 0 (mq_nvfp4_fold, and single calls outside the packed kernels): fold the first job.section sections of the record
+//   and publish the scales.  Tensors that share a record compute the same values and write them twice.
+// MODE 2 (the job driver, after the single pass of a carried run): job.section is the tensor's place inside its record and
+//   job.pad the number of tensors sharing it; they sit next to each other in the table.  Only the workgroup of the last one
+//   works: it folds what the run left in all their sections (kCarriedMark), writes every one's global scale and clears the
+//   sections for the next run.  It checks the amax and scales the record held before against the new ones: all four words
+//   equal means the codes just written with the old values are final (kRecRedo = 0); otherwise the new values are stored
+//   and kRecRedo = 1 asks for a second quantization.
 //   A record whose amax moved on two syncs in a row is marked volatile (kRecVolatile): on the next carried sync the
 //   single pass only collects its partial maxima (no codes are written with an amax that is likely stale again) and the
 //   second pass quantizes it with the fresh amax -- the cost of the plain two-pass form, instead of two full
@@ -164,12 +233,14 @@ __global__ __launch_bounds__(256) void nvfp4_fold_kernel(const Table tab, float 
     if (MODE != 0 && job.section != job.pad - 1) return;
     uint32_t* rec = (uint32_t*)job.aux;
     uint32_t m = 0;
-    for (int i = threadIdx.x; i < sections * kSectionWords; i += 256) m = umax(m, rec[i]);
+    for (int i = threadIdx.x; i < sections * kSectionWords; i += 256) {
+        const uint32_t word = rec[i];
+        m = umax(m, MODE == 0 ? word : (word & kCarriedMark) != 0 ? word & ~kCarriedMark : 0u);
+        if (MODE != 0) rec[i] = 0;
+    }
     m = wave_max(m);
     if ((threadIdx.x & 63) == 0) lds4[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (MODE != 0)
-        for (int i = threadIdx.x; i < sections * kSectionWords; i += 256) rec[i] = 0;
     if (threadIdx.x == 0) {
         const float amax = u2f(umax(umax(lds4[0], lds4[1]), umax(lds4[2], lds4[3])));
         const NvScales gs = nv_scales(amax, numer);
@@ -178,16 +249,8 @@ __global__ __launch_bounds__(256) void nvfp4_fold_kernel(const Table tab, float 
                                  rec[kRecSDec] == f2u(gs.s_dec) && rec[kRecEnc] == f2u(gs.enc));
             amax_record_after_carried_run(rec, moved);
             amax_feedback(moved_counter, moved, (uint32_t)sections);
-        } else if (MODE == 1) {
-            rec[kRecRedo] = 0;
-            rec[kRecVolatile] = 0;
-            rec[kRecMovedRuns] = 0;
-            amax_feedback(moved_counter, rec[kRecAmax] != f2u(amax), (uint32_t)sections);
         }
-        rec[kRecAmax] = f2u(amax);
-        rec[kRecEncSixth] = f2u(gs.enc_sixth);
-        rec[kRecSDec] = f2u(gs.s_dec);
-        rec[kRecEnc] = f2u(gs.enc);
+        nv_record_tail(rec, amax, gs);
         const float published = nv_published_scale(amax, numer);
         if (MODE == 0) {
             if (job.aux2) *(float*)job.aux2 = published;
@@ -378,17 +441,12 @@ __device__ __forceinline__ NvCandidate16 nv_four_over_six16(const float f[16], f
 // error mode of a flags word, as the EM template argument
 static inline int nv_error_mode(int flags) { return ((flags & MQ_NVFP4_ERR_MSE) ? 1 : 0) | ((flags & MQ_NVFP4_ERR_FP16) ? 2 : 0); }
 
-// The amax that a fake quantization of job.w works with: the caller's fp32 scalar (job.aux2), or the maximum of the
-// kSectionWords partial maxima an amax pass left in job.aux -- one per lane of the workgroup, so folding them here costs a
-// load and a reduction that overlap the data's loads, where a fold kernel costs a launch between the two passes.
-__device__ __forceinline__ float nv_fake_amax(const FlatJob& job, const int t) {
-    static_assert(kNvThreads == kSectionWords, "a partial maximum per lane");
-    if (job.aux2) return *(const float*)job.aux2;
-    __shared__ uint32_t part[kNvThreads / kWave];
-    const uint32_t m = wave_max(((const uint32_t*)job.aux)[t]);
-    if ((t & (kWave - 1)) == 0) part[t >> 6] = m;
-    __syncthreads();
-    return u2f(umax(umax(part[0], part[1]), umax(part[2], part[3])));
+// The amax and scales that a fake quantization of job.w works with: the caller's fp32 scalar (job.aux2), or the maximum of
+// the kSectionWords partial maxima an amax pass left in job.aux.
+__device__ __forceinline__ NvAmaxScales nv_fake_scales(const FlatJob& job, const int t, float numer) {
+    return nv_shared_scales(t, numer, [&] {
+        return job.aux2 ? *(const uint32_t*)job.aux2 : nv_wave_fold((const uint32_t*)job.aux, 1, t);
+    });
 }
 // eight values times a scale as a unit of 16-bit elements
 template <int F16>
@@ -421,9 +479,9 @@ __device__ __forceinline__ u32x4 nv_scaled16(const float q[8], float scale) {
 constexpr int kFosRounds = MQ_NV_FOS_ROUNDS;
 // units a workgroup of the quantizer covers (FOS as in nvfp4_quant_units)
 constexpr int64_t nv_units_per_block(int fos) { return (int64_t)kNvThreads * kNvUnroll * (fos ? kFosRounds : 1); }
-template <int EM, int F16, bool QDQ = false>
+template <int EM, int F16, bool QDQ, class Scales>
 __device__ __forceinline__ uint32_t nvfp4_fos_units(const FlatJob& job, const int64_t base, const int t, const float denom,
-                                                    const float inv_denom = 0.0f) {
+                                                    const float inv_denom, Scales scales) {
     static_assert(kNvUnroll == 2, "the regrouping pairs the two units of a lane");
     constexpr uint32_t kPiece = kNvThreads * 2;
     __shared__ u32x4 stage[kPiece];
@@ -431,7 +489,6 @@ __device__ __forceinline__ uint32_t nvfp4_fos_units(const FlatJob& job, const in
     const uint16_t* __restrict__ w = (const uint16_t*)job.w;
     uint32_t* __restrict__ q = (uint32_t*)job.q;
     uint8_t* __restrict__ s8 = (uint8_t*)job.s;
-    const uint32_t* __restrict__ amax_bits = (const uint32_t*)job.aux;
     const int64_t left = job.units - base;
     const uint32_t rem_all = left < kPiece * kFosRounds ? (uint32_t)left : kPiece * kFosRounds;
     const uint16_t* __restrict__ w0 = w + base * 8;
@@ -449,17 +506,9 @@ __device__ __forceinline__ uint32_t nvfp4_fos_units(const FlatJob& job, const in
             const uint32_t off = r * kPiece + (uint32_t)t + i * kNvThreads;
             in[r][i] = ld16(w0 + (off < rem_all ? off : 0u) * 8u);
         }
-    NvScales gs;
-    float amax;
-    if (QDQ) {
-        amax = nv_fake_amax(job, t);
-        gs = nv_scales(amax, denom);
-    } else {
-        gs.enc_sixth = u2f(amax_bits[kRecEncSixth]);
-        gs.s_dec = u2f(amax_bits[kRecSDec]);
-        gs.enc = u2f(amax_bits[kRecEnc]);
-        amax = u2f(amax_bits[kRecAmax]);
-    }
+    const NvAmaxScales known = scales();
+    const NvScales gs = known.gs;
+    const float amax = known.amax;
     const int fastdiv = nv_fast_division(amax);
     // the error's divisor 6 * e4m3_max is one of two constants and the same for the whole launch: its reciprocal is
     // picked on the scalar unit
@@ -567,13 +616,12 @@ __device__ __forceinline__ NvUnitCodes nvfp4_quant_unit(const u32x4 v, const NvS
 
 // kNvThreads * kNvUnroll units starting at `base` of one tensor; returns the largest |element| this lane saw (bf16 bits)
 // FOS = 0: standard quantizer; FOS = 1 + error mode: Four Over Six
-template <int FOS, int F16>
-__device__ __forceinline__ uint32_t nvfp4_quant_units(const FlatJob& job, const int64_t base, const int t, const float denom) {
-    if (FOS) return nvfp4_fos_units<(FOS > 0 ? FOS - 1 : 0), F16>(job, base, t, denom);
+template <int FOS, int F16, class Scales>
+__device__ __forceinline__ uint32_t nvfp4_quant_units(const FlatJob& job, const int64_t base, const int t, const float denom, Scales scales) {
+    if (FOS) return nvfp4_fos_units<(FOS > 0 ? FOS - 1 : 0), F16, false>(job, base, t, denom, 0.0f, scales);
     const uint16_t* __restrict__ w = (const uint16_t*)job.w;
     uint32_t* __restrict__ q = (uint32_t*)job.q;
     uint8_t* __restrict__ s8 = (uint8_t*)job.s;
-    const uint32_t* __restrict__ amax_bits = (const uint32_t*)job.aux;
     const int64_t total_units = job.units;
     // everything a lane adds to the workgroup's (uniform) base addresses is a 32-bit offset
     const int64_t left = total_units - base;
@@ -587,10 +635,7 @@ __device__ __forceinline__ uint32_t nvfp4_quant_units(const FlatJob& job, const 
         const uint32_t off = (uint32_t)t + i * kNvThreads;
         v[i] = off < rem ? ld16(w0 + off * 8u) : u32x4{0u, 0u, 0u, 0u};
     }
-    NvScales gs;
-    gs.enc_sixth = u2f(amax_bits[kRecEncSixth]);
-    gs.s_dec = u2f(amax_bits[kRecSDec]);
-    gs.enc = u2f(amax_bits[kRecEnc]);
+    const NvScales gs = scales().gs;
     uint32_t seen = 0;
 #pragma unroll
     for (int i = 0; i < kNvUnroll; i++) {
@@ -624,9 +669,10 @@ __device__ __forceinline__ uint32_t nvfp4_amax_units(const FlatJob& job, const i
 // PASS 1 quantizes with those in a single read of the tensor and collects this sync's partial maxima on the way (one
 // atomic max per workgroup into the tensor's section, cleared by the previous fold); the fold kernel then compares, and
 // PASS 2, a small grid striding over the blocks, quantizes again only the tensors whose amax did change.
-// PASS 0 is the second pass of the plain two-pass form (amax kernel, fold, quantize).
+// PASS 0 is the second pass of the plain two-pass form (amax kernel, then this): every workgroup folds the partial maxima,
+// and the first one of each tensor publishes what comes of them, also for a tensor without elements.
 template <int FOS, int PASS, class Table, int F16>
-__global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Table tab, float denom) {
+__global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Table tab, float denom, uint32_t* moved_counter, uint32_t* moved_mirror) {
     const FlatJob job = flat_job(tab);       // a copy in registers: a descriptor in device memory must not be re-read after the stores
     const int t = threadIdx.x;
     constexpr int64_t kPerBlock = nv_units_per_block(FOS);
@@ -635,17 +681,32 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
         // an XCD takes a run of consecutive blocks in every trip of the grid, as the flat grids do (second pass 2 pct faster)
         const int64_t first = xcd_chunked_block(gridDim.x == kSectionWords ? kSectionWords / kXcds : tab.chunk);
         for (int64_t base = first * kPerBlock; base < job.units; base += (int64_t)gridDim.x * kPerBlock)
-            nvfp4_quant_units<FOS, F16>(job, base, t, denom);
+            nvfp4_quant_units<FOS, F16>(job, base, t, denom, [&] { return nv_record_scales(job); });
         return;
     }
     const int64_t base = flat_block(tab) * kPerBlock;
+    if (PASS == 0) {
+        if (base >= job.units && base > 0) return;
+        if (base == 0 && blockIdx.y == 0) amax_feedback_folded(moved_counter, moved_mirror, gridDim.y);
+        auto fold = [&] {
+            const NvAmaxScales a = nv_shared_scales(t, denom, [&] { return nv_wave_fold((const uint32_t*)job.aux, job.pad, t); });
+            if (base == 0 && t == 0) {
+                ((uint32_t*)job.aux)[kRecRedo] = 0;
+                nv_publish_plain(job, a.amax, a.gs, denom, moved_counter);
+            }
+            return a;
+        };
+        if (job.units == 0) fold();
+        else nvfp4_quant_units<FOS, F16>(job, base, t, denom, fold);
+        return;
+    }
     if (base >= job.units) return;
     uint32_t seen;
     if (PASS == 1 && ((const uint32_t*)job.aux)[kRecVolatile] != 0) {
         seen = 0;
         for (int64_t piece = base; piece < base + kPerBlock && piece < job.units; piece += kNvThreads * kNvUnroll)
             seen = umax(seen, nvfp4_amax_units(job, piece, t));
-    } else seen = nvfp4_quant_units<FOS, F16>(job, base, t, denom);
+    } else seen = nvfp4_quant_units<FOS, F16>(job, base, t, denom, [&] { return nv_record_scales(job); });
     if (PASS == 1) {
         __shared__ uint32_t wave_seen[kNvThreads / 64];
         seen = wave_max(seen);
@@ -655,7 +716,7 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
             uint32_t m = 0;
 #pragma unroll
             for (int k = 0; k < kNvThreads / 64; k++) m = umax(m, wave_seen[k]);
-            atomicMax((uint32_t*)job.aux + job.section * kSectionWords + (blockIdx.x & (kSectionWords - 1)), f2u(elem_lo<F16>(m)));
+            atomicMax((uint32_t*)job.aux + job.section * kSectionWords + (blockIdx.x & (kSectionWords - 1)), kCarriedMark | f2u(elem_lo<F16>(m)));
         }
     }
 }
@@ -677,7 +738,7 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
 //     maximum, and every workgroup that reads it leaves at once: a record that does not fit next to a busy neighbour costs
 //     one wait, not one for each batch of its workgroups that comes to the chip.  32 x [2048, 7168] beside a stream of
 //     [8192, 8192] matrix products: 2.5 ms, 3.0 without that word, 2.35 in two passes (beside one of copies 0.56, 0.56, 0.91).
-// 32 x [2048, 7168] (940 MB of bf16, the four launches together): 312 us in two passes, 228 us this way (5.3 TB/s); the
+// 32 x [2048, 7168] (940 MB of bf16, all launches together): 318 us in two passes, 230 us this way (5.3 TB/s); the
 // same without the wait 198 us.  24 units per lane at four workgroups per CU: 239; 8 units in 512 lanes: 242.
 constexpr int kOneThreads = 256, kOneUnits = 16, kOneWavesPerSimd = 5;
 constexpr int64_t kOnePerBlock = kOneThreads * kOneUnits;
@@ -686,6 +747,7 @@ constexpr uint32_t kOneFull = 0x8000u;               // marks a slot or word tha
 constexpr uint32_t kOneGaveUp = 0x10000u;            // in a word: the first workgroup has stopped waiting
 constexpr int kOneWords = 7, kOneStride = 32, kRecOne = kRecAmax + 32;     // the published maximum, 128 bytes apart
 static_assert(kRecOne + (kOneWords - 1) * kOneStride < MQ_NVFP4_RECORD_WORDS, "the published words lie inside the record");
+constexpr int kRecReaders = kRecMovedRuns + 1;       // workgroups of the finish that have read the slots of a record left to it
 constexpr int kOneLeaderSleep = 1, kOneSleep = 12;   // between two looks, in units of 64 cycles
 constexpr int kOnePolls = 256;                       // looks of a workgroup, 0.25 ms or more; undisturbed, some 10 are enough
 
@@ -699,7 +761,7 @@ __global__ __launch_bounds__(256) void nvfp4_one_pass_clear_kernel(const Table t
     const FlatJob& job = tab.job[blockIdx.x];
     uint32_t* rec = (uint32_t*)job.aux;
     rec[job.section * kSectionWords + threadIdx.x] = 0;
-    if (job.section == 0 && threadIdx.x == 0) rec[kRecRedo] = 0;
+    if (job.section == 0 && threadIdx.x == 0) rec[kRecRedo] = rec[kRecReaders] = 0;
     if (job.section == 0 && threadIdx.x < kOneWords) rec[kRecOne + threadIdx.x * kOneStride] = 0;
 }
 
@@ -809,38 +871,45 @@ __global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_
     }
 }
 
-// What nvfp4_fold_kernel<1> does, from the 16-bit slots: amax, scales and published scales, slots cleared for a carried run.
-// kRecRedo stays as the workgroups left it.
+// Behind the one-pass kernel: quantizes the records that were left to it and publishes every record's amax, scales and
+// published scales.  grid (up to kSectionWords, tensors).  The slots are cleared for a carried run (their marks would pass for
+// kCarriedMark): of a finished record, whose amax its first workgroup has published, by the tensor's first workgroup here; of
+// one left to this pass, where every workgroup folds the slots, by the last one to have read them.
+// kRecRedo stays as the one-pass kernel left it.  (One launch of 4.3 us for the two of 4.3 us each that did this.)
 template <int F16, class Table>
-__global__ __launch_bounds__(256) void nvfp4_one_pass_finish_kernel(const Table tab, float numer, uint32_t* moved_counter, uint32_t* moved_mirror) {
-    __shared__ uint32_t lds4[4];
-    const int ji = blockIdx.x;
-    const FlatJob& job = tab.job[ji];
-    const int sections = job.pad;
-    amax_feedback_folded(moved_counter, moved_mirror, gridDim.x);
-    if (job.section != sections - 1) return;
+__global__ __launch_bounds__(kNvThreads) void nvfp4_one_pass_finish_kernel(const Table tab, float numer, uint32_t* moved_counter, uint32_t* moved_mirror) {
+    const FlatJob job = flat_job(tab);
+    const int t = threadIdx.x;
     uint32_t* rec = (uint32_t*)job.aux;
-    uint32_t m = 0;
-    for (int i = threadIdx.x; i < sections * kSectionWords; i += 256) {
-        m = umax(m, hmax_u16(abs2(rec[i])));
-        rec[i] = 0;
+    const bool redo = rec[kRecRedo] != 0;
+    if (blockIdx.x != 0 && !redo) return;
+    if (blockIdx.x == 0 && blockIdx.y == 0) amax_feedback_folded(moved_counter, moved_mirror, gridDim.y);
+    uint32_t bits;
+    if (!redo) {
+        bits = rec[kRecOne] & ~kOneFull;
+        rec[job.section * kSectionWords + t] = 0;
+    } else {
+        __shared__ uint32_t part[kNvThreads / kWave], readers;
+        bits = 0;
+        for (int k = 0; k < job.pad; k++) bits = umax(bits, hmax_u16(abs2(rec[k * kSectionWords + t])));
+        bits = wave_max(bits);
+        if ((t & (kWave - 1)) == 0) part[t >> 6] = bits;
+        __syncthreads();
+        bits = umax(umax(part[0], part[1]), umax(part[2], part[3]));
+        if (t == 0) readers = atomicAdd(rec + kRecReaders, 1u);
+        __syncthreads();
+        if (readers + 1 == gridDim.x * (uint32_t)job.pad)
+            for (int k = 0; k < job.pad; k++) rec[k * kSectionWords + t] = 0;
     }
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) lds4[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    const float amax = elem_lo<F16>(umax(umax(lds4[0], lds4[1]), umax(lds4[2], lds4[3])));
-    const NvScales gs = nv_scales(amax, numer);
-    rec[kRecVolatile] = 0;
-    rec[kRecMovedRuns] = 0;
-    amax_feedback(moved_counter, rec[kRecAmax] != f2u(amax), (uint32_t)sections);
-    rec[kRecAmax] = f2u(amax);
-    rec[kRecEncSixth] = f2u(gs.enc_sixth);
-    rec[kRecSDec] = f2u(gs.s_dec);
-    rec[kRecEnc] = f2u(gs.enc);
-    const float published = nv_published_scale(amax, numer);
-    for (int k = 0; k < sections; k++)
-        if (tab.job[ji - k].aux2) *(float*)tab.job[ji - k].aux2 = published;
+    const float amax = elem_lo<F16>(bits);
+    const NvAmaxScales a{amax, nv_scales(amax, numer)};
+    if (blockIdx.x == 0 && t == 0) nv_publish_plain(job, a.amax, a.gs, numer, moved_counter);
+    if (!redo) return;
+    // an XCD takes a run of consecutive blocks in every trip of the grid, as in the second pass of a carried run
+    constexpr int64_t kPerBlock = nv_units_per_block(0);
+    const int64_t first = xcd_chunked_block(gridDim.x == kSectionWords ? kSectionWords / kXcds : tab.chunk);
+    for (int64_t base = first * kPerBlock; base < job.units; base += (int64_t)gridDim.x * kPerBlock)
+        nvfp4_quant_units<0, F16>(job, base, t, numer, [&] { return a; });
 }
 
 // fp32 input, the second pass of the two-pass form (the carried-over amax and the one-pass form are for 16-bit tensors).
@@ -852,17 +921,24 @@ constexpr int kNvF32Loads = 2;                     // 16-byte loads per lane, st
 // 8-element units a workgroup covers
 constexpr int64_t nv_f32_units_per_block(int fos) { return fos ? kNvThreads * 2 : kNvThreads * kNvF32Loads / 2; }
 template <int FOS, class Table>
-__global__ __launch_bounds__(kNvThreads) void nvfp4_quant_f32_kernel(const Table tab, float denom) {
+__global__ __launch_bounds__(kNvThreads) void nvfp4_quant_f32_kernel(const Table tab, float denom, uint32_t* moved_counter, uint32_t* moved_mirror) {
     const FlatJob job = flat_job(tab);
     const uint32_t t = threadIdx.x;
     const int64_t first = flat_block(tab) * nv_f32_units_per_block(FOS);       // in 8-element units
-    if (first >= job.units) return;
-    const uint32_t* __restrict__ amax_bits = (const uint32_t*)job.aux;
-    NvScales gs;
-    gs.enc_sixth = u2f(amax_bits[kRecEncSixth]);
-    gs.s_dec = u2f(amax_bits[kRecSDec]);
-    gs.enc = u2f(amax_bits[kRecEnc]);
-    const float amax = u2f(amax_bits[kRecAmax]);
+    if (first >= job.units && first > 0) return;
+    if (first == 0 && blockIdx.y == 0) amax_feedback_folded(moved_counter, moved_mirror, gridDim.y);
+    auto fold = [&] {           // as in PASS 0 of the 16-bit kernel
+        const NvAmaxScales a = nv_shared_scales((int)t, denom, [&] { return nv_wave_fold((const uint32_t*)job.aux, job.pad, (int)t); });
+        if (first == 0 && t == 0) {
+            ((uint32_t*)job.aux)[kRecRedo] = 0;
+            nv_publish_plain(job, a.amax, a.gs, denom, moved_counter);
+        }
+        return a;
+    };
+    if (job.units == 0) {
+        fold();
+        return;
+    }
     const float* __restrict__ w0 = (const float*)job.w + first * 8;
     const int64_t left = (job.units - first) * 2;                              // 16-byte loads
     if constexpr (FOS != 0) {
@@ -878,7 +954,9 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_f32_kernel(const Table
             mb = umax(mb, umax(umax(v.x & 0x7FFFFFFFu, v.y & 0x7FFFFFFFu), umax(v.z & 0x7FFFFFFFu, v.w & 0x7FFFFFFFu)));
             f[4 * i] = u2f(v.x); f[4 * i + 1] = u2f(v.y); f[4 * i + 2] = u2f(v.z); f[4 * i + 3] = u2f(v.w);
         }
-        const float denom_inv = 1.0f / denom;
+        const NvAmaxScales known = fold();
+        const NvScales gs = known.gs;
+        const float amax = known.amax, denom_inv = 1.0f / denom;
         nv_fill_scale_table(scale_table, (int)t, amax, gs.s_dec, false, denom, denom_inv);
         __syncthreads();
         NvCandidate16 c = nv_fast_division(amax) != 0 ? nv_four_over_six16<EM, 1, true>(f, u2f(mb), amax, gs, denom, denom_inv, scale_table)
@@ -907,6 +985,7 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_f32_kernel(const Table
             const uint32_t off = t + i * kNvThreads;
             v[i] = off < rem ? ld16(w0 + off * 4u) : u32x4{0u, 0u, 0u, 0u};
         }
+        const NvScales gs = fold().gs;
 #pragma unroll
         for (int i = 0; i < kNvF32Loads; i++) {
             const uint32_t off = t + i * kNvThreads;
@@ -1017,7 +1096,7 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_fake_kernel(const FlatTable 
     const int64_t base = flat_block(tab) * nv_units_per_block(FOS);
     if (base >= job.units) return;
     if constexpr (FOS != 0) {
-        nvfp4_fos_units<FOS - 1, F16, true>(job, base, t, numer, inv_numer);
+        nvfp4_fos_units<FOS - 1, F16, true>(job, base, t, numer, inv_numer, [&] { return nv_fake_scales(job, t, numer); });
     } else {
         const int64_t left = job.units - base;
         const uint32_t rem = left < kNvThreads * kNvUnroll ? (uint32_t)left : (uint32_t)(kNvThreads * kNvUnroll);
@@ -1029,8 +1108,9 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_fake_kernel(const FlatTable 
             const uint32_t off = (uint32_t)t + i * kNvThreads;
             v[i] = ld16(x0 + (off < rem ? off : 0u) * 8u);      // a lane past the end reads the first unit again
         }
-        const float amax = nv_fake_amax(job, t);
-        const NvScales gs = nv_scales(amax, numer);
+        const NvAmaxScales known = nv_fake_scales(job, t, numer);
+        const float amax = known.amax;
+        const NvScales gs = known.gs;
 #pragma unroll
         for (int i = 0; i < kNvUnroll; i++) {
             const uint32_t off = (uint32_t)t + i * kNvThreads;
@@ -1079,18 +1159,25 @@ bool mq_nvfp4_fast_ok(const void* w, int dtype, const void* q) {
 }
 
 // tab.job[i]: w, aux = amax record, section, units = numel / 8, s = (void*)numel; every tensor of the one dtype
+static unsigned amax_blocks(int dtype, int64_t max_units) {
+    const int64_t chunks = (max_units * (dtype == MQ_F32 ? 2 : 1) + 256 * kAmaxUnroll - 1) / (256 * kAmaxUnroll);
+    return (unsigned)(chunks < 1 ? 1 : chunks < kSectionWords ? chunks : kSectionWords);
+}
 int mq_nvfp4_amax_launch_group(int dtype, FlatTable& tab, hipStream_t st) {
-    const dim3 grid(kSectionWords, (unsigned)tab.n), blk(256);
+    int64_t max_units = 0;
+    for (int i = 0; i < tab.n; i++) max_units = tab.job[i].units > max_units ? tab.job[i].units : max_units;
+    const dim3 grid(amax_blocks(dtype, max_units), (unsigned)tab.n), blk(256);
     if (dtype == MQ_F32) hipLaunchKernelGGL(nvfp4_amax_f32_kernel<FlatTable>, grid, blk, 0, st, tab);
     else if (dtype == MQ_F16) hipLaunchKernelGGL((nvfp4_amax_bf16_kernel<FlatTable, 1>), grid, blk, 0, st, tab);
     else hipLaunchKernelGGL((nvfp4_amax_bf16_kernel<FlatTable, 0>), grid, blk, 0, st, tab);
     return mq_check_launch("nvfp4 amax");
 }
-// the same over n descriptors of a device table (the quantizer's form: whole units, section = place inside the record)
-int mq_nvfp4_amax_launch_table(int dtype, const FlatJob* device_jobs, int n, hipStream_t st) {
+// the same over n descriptors of a device table (the quantizer's form: whole units, section = place inside the record);
+// max_units: the largest tensor's units
+int mq_nvfp4_amax_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, hipStream_t st) {
     if (n == 0) return MQ_OK;
     const FlatRef ref{device_jobs, 0, 0};
-    const dim3 grid(kSectionWords, (unsigned)n), blk(256);
+    const dim3 grid(amax_blocks(dtype, max_units), (unsigned)n), blk(256);
     if (dtype == MQ_F32) hipLaunchKernelGGL(nvfp4_amax_f32_kernel<FlatRef>, grid, blk, 0, st, ref);
     else if (dtype == MQ_F16) hipLaunchKernelGGL((nvfp4_amax_bf16_kernel<FlatRef, 1>), grid, blk, 0, st, ref);
     else hipLaunchKernelGGL((nvfp4_amax_bf16_kernel<FlatRef, 0>), grid, blk, 0, st, ref);
@@ -1098,47 +1185,50 @@ int mq_nvfp4_amax_launch_table(int dtype, const FlatJob* device_jobs, int n, hip
 }
 
 template <int PASS, class Table, int F16>
-static void launch_nvfp4_quant_dtype(const Table& tab, int flags, float numer, dim3 grid, hipStream_t st) {
+static void launch_nvfp4_quant_dtype(const Table& tab, int flags, float numer, bool counted, dim3 grid, hipStream_t st) {
     const dim3 blk(kNvThreads);
+    uint32_t *const moved = counted ? mq_amax_feedback() : nullptr, *const mirror = mq_amax_feedback_mirror();
     // Four Over Six keeps to launches of kernel-argument tables (its five error modes are not built in the other form)
     const int fos = (flags & MQ_NVFP4_4OVER6) ? 1 + nv_error_mode(flags) : 0;
     if constexpr (std::is_same<Table, FlatRef>::value) {
-        hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<0, PASS, Table, F16>), grid, blk, 0, st, tab, numer);
+        hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<0, PASS, Table, F16>), grid, blk, 0, st, tab, numer, moved, mirror);
     } else {
         switch (fos) {
-            case 0: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<0, PASS, Table, F16>), grid, blk, 0, st, tab, numer); break;
-            case 1: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<1, PASS, Table, F16>), grid, blk, 0, st, tab, numer); break;
-            case 2: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<2, PASS, Table, F16>), grid, blk, 0, st, tab, numer); break;
-            case 3: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<3, PASS, Table, F16>), grid, blk, 0, st, tab, numer); break;
-            default: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<4, PASS, Table, F16>), grid, blk, 0, st, tab, numer); break;
+            case 0: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<0, PASS, Table, F16>), grid, blk, 0, st, tab, numer, moved, mirror); break;
+            case 1: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<1, PASS, Table, F16>), grid, blk, 0, st, tab, numer, moved, mirror); break;
+            case 2: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<2, PASS, Table, F16>), grid, blk, 0, st, tab, numer, moved, mirror); break;
+            case 3: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<3, PASS, Table, F16>), grid, blk, 0, st, tab, numer, moved, mirror); break;
+            default: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<4, PASS, Table, F16>), grid, blk, 0, st, tab, numer, moved, mirror); break;
         }
     }
 }
 template <class Table>
-static void launch_nvfp4_quant_f32(const Table& tab, int flags, float numer, dim3 grid, hipStream_t st) {
+static void launch_nvfp4_quant_f32(const Table& tab, int flags, float numer, bool counted, dim3 grid, hipStream_t st) {
     const dim3 blk(kNvThreads);
+    uint32_t *const moved = counted ? mq_amax_feedback() : nullptr, *const mirror = mq_amax_feedback_mirror();
     const int fos = (flags & MQ_NVFP4_4OVER6) ? 1 + nv_error_mode(flags) : 0;
     if constexpr (std::is_same<Table, FlatRef>::value) {
-        hipLaunchKernelGGL((nvfp4_quant_f32_kernel<0, Table>), grid, blk, 0, st, tab, numer);
+        hipLaunchKernelGGL((nvfp4_quant_f32_kernel<0, Table>), grid, blk, 0, st, tab, numer, moved, mirror);
     } else {
         switch (fos) {
-            case 0: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<0, Table>), grid, blk, 0, st, tab, numer); break;
-            case 1: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<1, Table>), grid, blk, 0, st, tab, numer); break;
-            case 2: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<2, Table>), grid, blk, 0, st, tab, numer); break;
-            case 3: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<3, Table>), grid, blk, 0, st, tab, numer); break;
-            default: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<4, Table>), grid, blk, 0, st, tab, numer); break;
+            case 0: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<0, Table>), grid, blk, 0, st, tab, numer, moved, mirror); break;
+            case 1: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<1, Table>), grid, blk, 0, st, tab, numer, moved, mirror); break;
+            case 2: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<2, Table>), grid, blk, 0, st, tab, numer, moved, mirror); break;
+            case 3: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<3, Table>), grid, blk, 0, st, tab, numer, moved, mirror); break;
+            default: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<4, Table>), grid, blk, 0, st, tab, numer, moved, mirror); break;
         }
     }
 }
+// counted: pass 0 adds to the counters of the call's feedback (in a carried run the fold does)
 template <int PASS, class Table>
-static void launch_nvfp4_quant(int dtype, const Table& tab, int flags, float numer, dim3 grid, hipStream_t st) {
+static void launch_nvfp4_quant(int dtype, const Table& tab, int flags, float numer, bool counted, dim3 grid, hipStream_t st) {
     // (fp32 has no instances of passes 1 and 2: nvfp4_quant_launch refuses mode 2 for it)
-    if (PASS == 0 && dtype == MQ_F32) launch_nvfp4_quant_f32(tab, flags, numer, grid, st);
-    else if (dtype == MQ_F16) launch_nvfp4_quant_dtype<PASS, Table, 1>(tab, flags, numer, grid, st);
-    else launch_nvfp4_quant_dtype<PASS, Table, 0>(tab, flags, numer, grid, st);
+    if (PASS == 0 && dtype == MQ_F32) launch_nvfp4_quant_f32(tab, flags, numer, counted, grid, st);
+    else if (dtype == MQ_F16) launch_nvfp4_quant_dtype<PASS, Table, 1>(tab, flags, numer, counted, grid, st);
+    else launch_nvfp4_quant_dtype<PASS, Table, 0>(tab, flags, numer, counted, grid, st);
 }
 
-// fold + quantize (+ second pass) over a table whose grid is known: tab.chunk / tab.max_blocks are set
+// quantize (carried run: and fold, and second pass) over a table whose grid is known: tab.chunk / tab.max_blocks are set
 template <class Table>
 static int nvfp4_quant_launch(int dtype, const Table& tab, int n, int e4m3_max, int flags, int mode, hipStream_t st) {
     if (mode == 2 && dtype == MQ_F32) return mq_fail(MQ_ERR_ARG, "a carried-over amax is for bf16 and fp16 tensors");
@@ -1146,27 +1236,25 @@ static int nvfp4_quant_launch(int dtype, const Table& tab, int n, int e4m3_max, 
     const dim3 folds((unsigned)n), blk(256);
     const dim3 grid((unsigned)tab.max_blocks, (unsigned)n);
     if (mode == 2) {
-        if (tab.max_blocks > 0) launch_nvfp4_quant<1>(dtype, tab, flags, numer, grid, st);
+        if (tab.max_blocks > 0) launch_nvfp4_quant<1>(dtype, tab, flags, numer, false, grid, st);
         hipLaunchKernelGGL((nvfp4_fold_kernel<2, Table>), folds, blk, 0, st, tab, numer, mq_amax_feedback(), mq_amax_feedback_mirror());
         if (tab.max_blocks > 0) {
             const unsigned redo_blocks = tab.max_blocks < kSectionWords ? (unsigned)tab.max_blocks : (unsigned)kSectionWords;
-            launch_nvfp4_quant<2>(dtype, tab, flags, numer, dim3(redo_blocks, (unsigned)n), st);
+            launch_nvfp4_quant<2>(dtype, tab, flags, numer, false, dim3(redo_blocks, (unsigned)n), st);
         }
         return mq_check_launch("nvfp4 quant (carried-over amax)");
     }
-    if (mode == 1) hipLaunchKernelGGL((nvfp4_fold_kernel<1, Table>), folds, blk, 0, st, tab, numer, mq_amax_feedback(), mq_amax_feedback_mirror());
-    else hipLaunchKernelGGL((nvfp4_fold_kernel<0, Table>), folds, blk, 0, st, tab, numer, (uint32_t*)nullptr, (uint32_t*)nullptr);
-    if (tab.max_blocks > 0) launch_nvfp4_quant<0>(dtype, tab, flags, numer, grid, st);
+    // (a list of empty tensors still has its scales published, by the first workgroup of each)
+    launch_nvfp4_quant<0>(dtype, tab, flags, numer, mode == 1, dim3(grid.x > 0 ? grid.x : 1u, grid.y), st);
     return mq_check_launch("nvfp4 quant");
 }
 
 // tab.job[i]: w, q, s = block scales, aux = amax record, aux2 = fp32 global scale out (may be null), units = numel / 8.
-// mode 0 (single calls): section = sections to fold; fold, then quantize.
-// mode 1 (job driver, after its amax launch): section = place of the tensor inside its record, pad = tensors sharing the
-//   record (adjacent entries); fold once per record, clear the sections, quantize.
+// section = place of the tensor inside its record, pad = tensors sharing the record (adjacent entries).
+// mode 0 (single calls) and 1 (job driver), after the amax pass: quantize; mode 1 is counted in the call's feedback.
 // (fp32 tensors take modes 0 and 1.)
-// mode 2 (job driver, carried-over amax; the sections were cleared by the previous sync's fold): quantize with the
-//   record's old scales while collecting the new partial maxima, fold and compare, quantize again where they differ.
+// mode 2 (job driver, carried-over amax): quantize with the record's old scales while collecting the new partial maxima,
+//   fold and compare, quantize again where they differ.
 int mq_nvfp4_quant_launch_group(int dtype, FlatTable& tab, int e4m3_max, int flags, int mode, hipStream_t st) {
     const int fos = flags & MQ_NVFP4_4OVER6;
     if (!flat_grid(tab, dtype == MQ_F32 ? nv_f32_units_per_block(fos) : nv_units_per_block(fos))) return mq_fail(MQ_ERR_ARG, "tensor too large");
@@ -1185,9 +1273,10 @@ int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, in
 // largest number of workgroups that share a record, `bytes` the input of the whole chunk.  All workgroups of a record
 // have to be on the chip together, and the records behind it should be loading meanwhile: half of what fits (640 workgroups,
 // 40 MB, on 256 CUs).  A pair of [2048, 7168] weights, 896 workgroups, gained less (313 -> 265 us for 16 pairs) and is one
-// busy neighbour away from waiting in vain, so it keeps two passes.  Short lists keep them as well, which then find their
-// second read in the memory-side cache and save two launches: 4 x [1537, 2064] (25 MB) 15 against 19 us, [4096, 4096]
-// (34 MB) 20 / 19, 16 x [1536, 2048] (100 MB) 39 / 34.
+// busy neighbour away from waiting in vain, so it keeps two passes.  Short lists keep them as well, which then find part of
+// their second read in the memory-side cache and save a launch (us, two passes / one): 4 x [1537, 2064] (25 MB) 14 / 18,
+// 4 x [2048, 4096] (67 MB) 26 / 24, 18 x [1420, 1520] (78 MB) 30 / 33, 16 x [1536, 2048] (100 MB) 37 / 34,
+// 48 x [1536, 2048] (302 MB) 105 / 77.
 constexpr int64_t kOneMinBytes = 64ll << 20;
 bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes) {
     int device = 0, cus = 0;
@@ -1206,9 +1295,9 @@ static int nvfp4_one_pass_launch_dtype(const Table& one, const Table& redo, int 
     const dim3 folds((unsigned)n), blk(256);
     hipLaunchKernelGGL((nvfp4_one_pass_clear_kernel<Table>), folds, blk, 0, st, one);
     hipLaunchKernelGGL((nvfp4_one_pass_kernel<F16, Table>), dim3((unsigned)one.max_blocks, (unsigned)n), dim3(kOneThreads), 0, st, one, numer, first_polls);
-    hipLaunchKernelGGL((nvfp4_one_pass_finish_kernel<F16, Table>), folds, blk, 0, st, one, numer, mq_amax_feedback(), mq_amax_feedback_mirror());
     const unsigned redo_blocks = redo.max_blocks < kSectionWords ? (unsigned)redo.max_blocks : (unsigned)kSectionWords;
-    hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<0, 2, Table, F16>), dim3(redo_blocks, (unsigned)n), dim3(kNvThreads), 0, st, redo, numer);
+    hipLaunchKernelGGL((nvfp4_one_pass_finish_kernel<F16, Table>), dim3(redo_blocks, (unsigned)n), dim3(kNvThreads), 0, st, redo, numer,
+                       mq_amax_feedback(), mq_amax_feedback_mirror());
     return mq_check_launch("nvfp4 quant (one pass)");
 }
 template <class Table>
@@ -1260,7 +1349,7 @@ extern "C" int mq_nvfp4_quant(const void* w, int dtype, const void* record, int 
     if (blocks16 == 0 || mq_nvfp4_fast_ok(w, dtype, q)) {
         FlatTable tab{};
         tab.n = 1;
-        tab.job[0] = FlatJob{w, q, block_scale, const_cast<void*>(record), blocks16 * 2, global_scale, n_sections, 0};
+        tab.job[0] = FlatJob{w, q, block_scale, const_cast<void*>(record), blocks16 * 2, global_scale, n_sections - 1, n_sections};
         return mq_nvfp4_quant_launch_group(blocks16 == 0 ? MQ_BF16 : dtype, tab, e4m3_max, flags, 0, st);
     }
     FlatTable fold{};

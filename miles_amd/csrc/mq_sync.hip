@@ -50,7 +50,7 @@ int64_t mq_fp8_channel_blocks(int form, int64_t M);
 int mq_fp8_channel_launch_group(int dtype, int form, const MqScaledArgs* a, int n, hipStream_t st);
 int mq_fp8_scaled_form(const void* w, int dtype, int64_t ldw, const void* q, int64_t M, int64_t K);
 int mq_fp8_scaled_launch_group(int dtype, int form, const MqScaledArgs* a, int n, int words, hipStream_t st);
-int mq_nvfp4_amax_launch_table(int dtype, const FlatJob* device_jobs, int n, hipStream_t st);
+int mq_nvfp4_amax_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, hipStream_t st);
 int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int e4m3_max, int mode,
                                 hipStream_t st);
 int mq_mxfp8_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, hipStream_t st);
@@ -524,7 +524,7 @@ static int run_nvfp4(const mq_job* jobs, int64_t n_all, int64_t i, int64_t j, co
                     i = k;
                     continue;
                 }
-                if (!carry) rc = mq_nvfp4_amax_launch_table(jobs[i].dtype, table + i, n, st);
+                if (!carry) rc = mq_nvfp4_amax_launch_table(jobs[i].dtype, table + i, n, max_units, st);
                 if (rc) return rc;
                 rc = mq_nvfp4_quant_launch_table(jobs[i].dtype, table + i, n, max_units, jobs[i].p0, carry ? 2 : 1, st);
                 if (rc) return rc;
