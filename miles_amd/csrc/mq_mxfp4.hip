@@ -551,10 +551,16 @@ int mq_mxfp4_to_fp8_job(RecodeJob& job, const void* packed, const void* scale, v
     }
     return MQ_OK;
 }
+constexpr int64_t kTileRecodeUnits = 1ll << 21;       // 16-element units, see below
 int mq_mxfp4_to_fp8_launch_group(const RecodeTable& tab, hipStream_t st) {
-    // two tensors and more share the two launches of the flat form; a single call keeps the one launch of the tile form
-    // (2 % faster alone: the second launch's start costs more than the write pattern)
-    bool flat = tab.n > 1;
+    // Long lists take the two launches of the flat form; a single tensor (2 % faster alone) and lists of up to 2^25 elements
+    // the one launch of the tile form: the second launch's start costs them more than the write pattern.  Device time in us,
+    // flat / tile: two [384, 1408] 8.3 / 3.6, two [1024, 5376] 8.6 / 6.3, four [2048, 2048] 8.9 / 7.2, eight of them (2^25)
+    // 11.0 / 11.2, 32 [4096, 256] (2^25) 12.2 / 11.6; three [4096, 4096] 13.3 / 16.3, 24 [256, 8192] 14.2 / 17.2, eight
+    // [2048, 7168] 34 / 34.  (On the host a launch less: two [1024, 5376] 13.9 -> 11.7 with the submission.)
+    int64_t units = 0;
+    for (int i = 0; i < tab.n; i++) units += tab.job[i].units;
+    bool flat = tab.n > 1 && units > kTileRecodeUnits;
     int64_t bands = 0, blocks = 0;
     for (int i = 0; i < tab.n; i++) {
         const RecodeJob& j = tab.job[i];
