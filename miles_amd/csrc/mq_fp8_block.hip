@@ -217,17 +217,22 @@ __global__ __launch_bounds__(kTileThreads) void fp8_block128_kernel(const Table 
 
 // 128x128 tiles of a matrix with unit column stride and nothing else: any row stride, any column count, rows at any element
 // boundary, fp32 as well as 16-bit.  The tile split is the fast kernel's (lane t: rows t/16 + 32 i, eight columns from
-// 8 (t%16)); loads and stores are the same 16 and 8 bytes, only unaligned.  Past the matrix's edge nothing is masked: the
-// last rows are read again, and a segment that would leave the row is moved back to end with it, so that the maximum sees
-// only the tile's own elements (a tile at least eight columns wide) and a byte that two lanes own is written twice with one
-// value.  Bound by the memory system, which takes unaligned rows at 4.9 TB/s (24 [4097, 4099] bf16 tensors, 3.3 with
-// non-temporal loads and 2.9 with non-temporal stores too) and aligned fp32 rows (LINES, non-temporal loads) at 5.8.  Twelve
+// 8 (t%16)); loads and stores are the same 16 and 8 bytes, only unaligned.  fp32: rows t/32 + 16 i, four columns from
+// 4 (t%32), so that a load instruction takes whole lines there as well (eight columns from two loads, each of half of every
+// line: two [4096, 8192] tensors 63.7 us, 55.0 this way; with non-temporal stores of the four bytes 57.5).  Past the
+// matrix's edge nothing is masked: the last rows are read again, and a segment that would leave the row is moved back to end
+// with it, so that the maximum sees only the tile's own elements (a tile at least a segment wide) and a byte that two lanes
+// own is written twice with one value.  Bound by the memory system, which takes unaligned rows at 4.9 TB/s (24 [4097, 4099] bf16 tensors, 3.3 with
+// non-temporal loads and 2.9 with non-temporal stores too) and aligned fp32 rows (LINES, non-temporal loads) at 6.1.  Twelve
 // [1545, 2563] bf16 tensors as one list: 779 us in the two-pass kernel below, one launch each; 72 us here, host included.
 template <int MODE, int DT, bool LINES>
 __global__ __launch_bounds__(kTileThreads) void fp8_block128_any_kernel(const TileTable tab) {
     constexpr uint32_t kInfBits = DT == MQ_F32 ? 0x7F800000u : DT == MQ_F16 ? 0x7C00u : 0x7F80u;
     constexpr uint32_t kSize = DT == MQ_F32 ? 4u : 2u;
-    constexpr int kF16 = DT == MQ_F16, kLoads = DT == MQ_F32 ? 2 : 1;
+    constexpr int kF16 = DT == MQ_F16;
+    // a lane's segment is one 16-byte load: eight columns, or four fp32 ones
+    constexpr uint32_t kCols = DT == MQ_F32 ? 4u : 8u, kRowLanes = kTile / kCols, kStep = kTileThreads / kRowLanes;
+    constexpr int kRows = kTile / kStep;
     __shared__ uint32_t wave_amax[kTileWaves];
     const int32_t x = blockIdx.x % kXcds, k = blockIdx.x / kXcds, run = k >> tab.chunk_shift;
     const int32_t item = ((run * kXcds + x) << tab.chunk_shift) + (k - (run << tab.chunk_shift));
@@ -247,42 +252,35 @@ __global__ __launch_bounds__(kTileThreads) void fp8_block128_any_kernel(const Ti
     float* __restrict__ tile_scales = load_global_ptr(&job.scale);
     const uint32_t rows_left = M - ti * kTile, cols_left = K - tj * kTile;     // both at least 1
 
-    const uint32_t t = threadIdx.x, r0 = t >> 4, c0 = (t & 15u) * 8u;
-    const bool narrow = cols_left < 8u;                                        // uniform over the workgroup
-    const uint32_t c = narrow ? 0u : c0 + 8u <= cols_left ? c0 : cols_left - 8u;
-    u32x4 v[kRowsPerThread][kLoads];
+    const uint32_t t = threadIdx.x, r0 = t / kRowLanes, c0 = (t % kRowLanes) * kCols;
+    const bool narrow = cols_left < kCols;                                     // uniform over the workgroup
+    const uint32_t c = narrow ? 0u : c0 + kCols <= cols_left ? c0 : cols_left - kCols;
+    u32x4 v[kRows];
     if (!narrow) {
 #pragma unroll
-        for (int i = 0; i < kRowsPerThread; i++) {
-            const uint32_t r = r0 + kRowStep * i, rr = r < rows_left ? r : rows_left - 1u;
-#pragma unroll
-            for (int k = 0; k < kLoads; k++) {
-                const char* at = wt + ((rr * ldw + c) * kSize + 16u * k);
-                v[i][k] = LINES ? ld16(at) : ld16_at2(at);
-            }
+        for (int i = 0; i < kRows; i++) {
+            const uint32_t r = r0 + kStep * i, rr = r < rows_left ? r : rows_left - 1u;
+            const char* at = wt + (rr * ldw + c) * kSize;
+            v[i] = LINES ? ld16(at) : ld16_at2(at);
         }
     } else {
 #pragma unroll
-        for (int i = 0; i < kRowsPerThread; i++) {
-            const uint32_t r = r0 + kRowStep * i, rr = r < rows_left ? r : rows_left - 1u;
+        for (int i = 0; i < kRows; i++) {
+            const uint32_t r = r0 + kStep * i, rr = r < rows_left ? r : rows_left - 1u;
             uint32_t e[8];
 #pragma unroll
-            for (uint32_t j = 0; j < 8; j++) {
+            for (uint32_t j = 0; j < kCols; j++) {
                 const char* at = wt + (rr * ldw + (j < cols_left ? j : cols_left - 1u)) * kSize;
                 e[j] = DT == MQ_F32 ? *(const uint32_t*)at : *(const uint16_t*)at;
             }
-            if (DT == MQ_F32) {
-                v[i][0] = u32x4{e[0], e[1], e[2], e[3]};
-                v[i][kLoads - 1] = u32x4{e[4], e[5], e[6], e[7]};
-            } else {
-                v[i][0] = u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
-            }
+            if (DT == MQ_F32) v[i] = u32x4{e[0], e[1], e[2], e[3]};
+            else v[i] = u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
         }
     }
-    // the eight elements of row segment i
+    // the kCols elements of row segment i
     auto element = [&](int i, int j) -> float {
-        if (DT == MQ_F32) return u2f(v[i][(j >> 2) & (kLoads - 1)][j & 3]);
-        const uint32_t pair = v[i][0][j >> 1];
+        if (DT == MQ_F32) return u2f(v[i][j & 3]);
+        const uint32_t pair = v[i][(j >> 1) & 3];
         return (j & 1) ? elem_hi<kF16>(pair) : elem_lo<kF16>(pair);
     };
     auto workgroup_max = [&](uint32_t m) {
@@ -296,23 +294,21 @@ __global__ __launch_bounds__(kTileThreads) void fp8_block128_any_kernel(const Ti
     };
     uint32_t m = 0;
 #pragma unroll
-    for (int i = 0; i < kRowsPerThread; i++)
-#pragma unroll
-        for (int k = 0; k < kLoads; k++) {
-            const u32x4 x = v[i][k];
-            if (DT == MQ_F32)
-                m = umax(umax(umax(m, x.x & 0x7FFFFFFFu), umax(x.y & 0x7FFFFFFFu, x.z & 0x7FFFFFFFu)), x.w & 0x7FFFFFFFu);
-            else
-                m = max2_u16(max2_u16(m, max2_u16(abs2(x.x), abs2(x.y))), max2_u16(abs2(x.z), abs2(x.w)));
-        }
+    for (int i = 0; i < kRows; i++) {
+        const u32x4 x = v[i];
+        if (DT == MQ_F32)
+            m = umax(umax(umax(m, x.x & 0x7FFFFFFFu), umax(x.y & 0x7FFFFFFFu, x.z & 0x7FFFFFFFu)), x.w & 0x7FFFFFFFu);
+        else
+            m = max2_u16(max2_u16(m, max2_u16(abs2(x.x), abs2(x.y))), max2_u16(abs2(x.z), abs2(x.w)));
+    }
     m = workgroup_max(DT == MQ_F32 ? m : hmax_u16(m));
     const bool special = m >= kInfBits;      // an infinity or a NaN in the tile, as in the fast kernel
     if (MODE == 1 && special) {
         uint32_t finite = 0;
 #pragma unroll
-        for (int i = 0; i < kRowsPerThread; i++)
+        for (int i = 0; i < kRows; i++)
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
+            for (uint32_t j = 0; j < kCols; j++) {
                 const uint32_t a = f2u(element(i, j)) & 0x7FFFFFFFu;
                 finite = umax(finite, a > 0x7F800000u ? 0u : a);
             }
@@ -331,41 +327,42 @@ __global__ __launch_bounds__(kTileThreads) void fp8_block128_any_kernel(const Ti
     // scales at the ends of the fp32 range
     const bool plain = !special && (MODE != 0 || shared_div_ok(s));
 #pragma unroll
-    for (int i = 0; i < kRowsPerThread; i++) {
-        u32x2 o;
+    for (int i = 0; i < kRows; i++) {
+        uint32_t o[kCols / 4];
         if (zero_tile) {
-            o = u32x2{0xFFFFFFFFu, 0xFFFFFFFFu};
-        } else if (plain) {
-            float f[8];
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
+            for (uint32_t j = 0; j < kCols; j += 4) o[j / 4] = 0xFFFFFFFFu;
+        } else if (plain) {
+            float f[kCols];
+#pragma unroll
+            for (uint32_t j = 0; j < kCols; j++) {
                 const float x = element(i, j);
                 f[j] = MODE != 0 ? x * y : DT == MQ_F32 ? div24_by_shared(x, s, y) : div_by_shared(x, s, y);
             }
-            o.x = hw_e4m3x4(f[0], f[1], f[2], f[3]);       // at most 448 (1 + 2^-22): rounds to 448 by itself
-            o.y = hw_e4m3x4(f[4], f[5], f[6], f[7]);
-        } else {
-            uint32_t code[8];
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
+            for (uint32_t j = 0; j < kCols; j += 4)       // at most 448 (1 + 2^-22): rounds to 448 by itself
+                o[j / 4] = hw_e4m3x4(f[j], f[j + 1], f[j + 2], f[j + 3]);
+        } else {
+#pragma unroll
+            for (uint32_t j = 0; j < kCols; j++) {
                 const float x = element(i, j);
                 float p = MODE != 0 ? x * y : x / s;
                 if (MODE == 0) p = clamp_keep_nan(p, -kFp8Max, kFp8Max);                            // torch.clamp
                 else if (MODE == 1) p = __builtin_fminf(__builtin_fmaxf(p, -kFp8Max), kFp8Max);     // tl.clamp: NaN -> -448
-                code[j] = sw_e4m3fn(p);
+                const uint32_t code = sw_e4m3fn(p) << (8 * (j & 3));
+                o[j / 4] = (j & 3) == 0 ? code : o[j / 4] | code;
             }
-            o.x = code[0] | (code[1] << 8) | (code[2] << 16) | (code[3] << 24);
-            o.y = code[4] | (code[5] << 8) | (code[6] << 16) | (code[7] << 24);
         }
-        const uint32_t r = r0 + kRowStep * i;
+        const uint32_t r = r0 + kStep * i;
         if (r >= rows_left || c0 >= cols_left) continue;
         uint8_t* at = qt + (r * K + c);
         if (!narrow) {
-            st8_at1(at, o);
+            if (kCols == 8) st8_at1(at, u32x2{o[0], o[kCols / 4 - 1]});
+            else st4_at1(at, o[0]);
         } else {
 #pragma unroll
-            for (uint32_t j = 0; j < 7; j++)
-                if (j < cols_left) at[j] = (uint8_t)((j < 4 ? o.x : o.y) >> (8 * (j & 3)));
+            for (uint32_t j = 0; j < kCols - 1; j++)
+                if (j < cols_left) at[j] = (uint8_t)(o[j / 4] >> (8 * (j & 3)));
         }
     }
 }
