@@ -723,7 +723,7 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
 
 // ---- one read of the tensor without an amax from before ----------------------------------------------------
 // The two-pass form reads every element twice, and at 6.8 TB/s its amax pass is 43 % of its time.  Here a workgroup keeps its
-// 64 KiB in registers (16 units per lane, 94 VGPRs, five workgroups per CU: 80 MB on the chip), publishes their maximum,
+// 64 KiB in registers (16 units per lane, 93 VGPRs, five workgroups per CU: 80 MB on the chip), publishes their maximum,
 // waits for the tensor's other workgroups and quantizes what it holds.  While one tensor waits for its last loads, the
 // workgroups of the next two are already loading.
 //   exchange: a workgroup stores its maximum (with kOneFull, so that it is never zero) into a 16-bit slot of its tensor's
@@ -738,8 +738,10 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
 //     maximum, and every workgroup that reads it leaves at once: a record that does not fit next to a busy neighbour costs
 //     one wait, not one for each batch of its workgroups that comes to the chip.  32 x [2048, 7168] beside a stream of
 //     [8192, 8192] matrix products: 2.5 ms, 3.0 without that word, 2.35 in two passes (beside one of copies 0.56, 0.56, 0.91).
-// 32 x [2048, 7168] (940 MB of bf16, all launches together): 318 us in two passes, 230 us this way (5.3 TB/s); the
-// same without the wait 198 us.  24 units per lane at four workgroups per CU: 239; 8 units in 512 lanes: 242.
+// 32 x [2048, 7168] (940 MB of bf16, all launches together): 318 us in two passes, 226 us this way (5.4 TB/s; 234 with the
+// block maxima taken after the wait, a range test and a branch to the software forms in each unit).  24 units per lane at
+// four workgroups per CU were 5 % slower, 8 units in 512 lanes 6 %, six workgroups per CU (20 registers spilled) 38 %; two
+// units stored together, eight bytes a lane, 2 % slower here and 2 % faster on 18 x [1420, 1520].
 constexpr int kOneThreads = 256, kOneUnits = 16, kOneWavesPerSimd = 5;
 constexpr int64_t kOnePerBlock = kOneThreads * kOneUnits;
 constexpr int kOneSlots = 2 * kSectionWords;         // 16-bit slots of a section
@@ -765,7 +767,24 @@ __global__ __launch_bounds__(256) void nvfp4_one_pass_clear_kernel(const Table t
     if (job.section == 0 && threadIdx.x < kOneWords) rec[kRecOne + threadIdx.x * kOneStride] = 0;
 }
 
-// job as for the fold in MODE 1: section = place of the tensor inside its record, pad = tensors sharing it (neighbours)
+// maximum of the block that a lane's unit and its neighbour's make up (16-bit pattern)
+__device__ __forceinline__ uint32_t nv_block_max(const u32x4 v) {
+    return group_max2(hmax_u16(max2_u16(max2_u16(abs2(v.x), abs2(v.y)), max2_u16(abs2(v.z), abs2(v.w)))));
+}
+// nvfp4_quant_unit for finite elements and 1 / S_enc in 2^-82 .. 2^81: a block scale is 0 or in 2^-9 .. 448, so the divisor of
+// every block with a scale is in the range of recip_shared; the others have the largest reciprocal, as 1 / 0 is cut to it
+template <int F16>
+__device__ __forceinline__ NvUnitCodes nv_plain_unit(const u32x4 v, const uint32_t mb, const NvScales& gs) {
+    const uint32_t sc = hw_e4m3x2<false>(__builtin_fminf(elem_lo<F16>(mb) * gs.enc_sixth, kFp8Max), 0.0f, 0u) & 0xFFu;
+    const float inv = sc == 0u ? kFltMax : recip_shared(hw_e4m3x2_decode<false>(sc).x * gs.s_dec);
+    uint32_t word = hw_e2m1x2<0>(elem_lo<F16>(v.x) * inv, elem_hi<F16>(v.x) * inv, 0u);
+    word = hw_e2m1x2<1>(elem_lo<F16>(v.y) * inv, elem_hi<F16>(v.y) * inv, word);
+    word = hw_e2m1x2<2>(elem_lo<F16>(v.z) * inv, elem_hi<F16>(v.z) * inv, word);
+    word = hw_e2m1x2<3>(elem_lo<F16>(v.w) * inv, elem_hi<F16>(v.w) * inv, word);
+    return NvUnitCodes{sc, word, mb};
+}
+
+// job as for the quantize pass: section = place of the tensor inside its record, pad = tensors sharing it (neighbours)
 template <int F16, class Table>
 __global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_kernel(const Table tab, float numer, int first_polls) {
     __shared__ uint32_t wave_seen[kOneThreads / 64], wave_late[kOneThreads / 64];
@@ -788,10 +807,13 @@ __global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_
             v[i] = ld16(w0 + (off < rem ? off : (off & 1u)) * 8u);      // a lane past the end reads the first block again
         }
     }
-    uint32_t m2 = 0;
+    // the block maxima, two to a register: what does not depend on the amax is done before the wait for it
+    uint32_t maxima[kOneUnits / 2], m2 = 0;
 #pragma unroll
-    for (int i = 0; i < kOneUnits; i++)
-        m2 = max2_u16(m2, max2_u16(max2_u16(abs2(v[i].x), abs2(v[i].y)), max2_u16(abs2(v[i].z), abs2(v[i].w))));
+    for (int i = 0; i < kOneUnits; i += 2) {
+        maxima[i / 2] = nv_block_max(v[i]) | (nv_block_max(v[i + 1]) << 16);
+        m2 = max2_u16(m2, maxima[i / 2]);
+    }
     uint32_t m = wave_max(hmax_u16(m2));
     if ((t & 63) == 0) wave_seen[t >> 6] = m;
     __syncthreads();
@@ -852,17 +874,20 @@ __global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_
         late = (m & kOneFull) == 0;
         m &= 0x7FFFu;
     }
-    if (late) {
+    const NvScales gs = nv_scales(elem_lo<F16>(m), numer);
+    // Tensors with an infinity or a NaN, or with a scale at the ends of the fp32 range, are left to the finish as well: its
+    // code has the software forms, which here, in sixteen copies, were 8 700 instructions in the way of the 2 000 that run.
+    const uint32_t dec = f2u(gs.s_dec);
+    if (late || m >= (F16 ? 0x7C00u : 0x7F80u) || !(dec >= 0x16800000u /* 2^-82 */ && dec <= 0x68000000u /* 2^81 */)) {
         if (t == 0) rec[kRecRedo] = 1;
         return;
     }
-    const NvScales gs = nv_scales(elem_lo<F16>(m), numer);
     uint32_t* __restrict__ q0 = (uint32_t*)job.q + base;
     uint8_t* __restrict__ s80 = (uint8_t*)job.s + base / 2;
 #pragma unroll
     for (int i = 0; i < kOneUnits; i++) {
         const uint32_t off = (uint32_t)t + i * kOneThreads;
-        const NvUnitCodes c = nvfp4_quant_unit<F16>(v[i], gs);
+        const NvUnitCodes c = nv_plain_unit<F16>(v[i], (maxima[i / 2] >> (16 * (i & 1))) & 0xFFFFu, gs);
         if (whole || off < rem) {
             st4(q0 + i * kOneThreads + (uint32_t)t, c.word);
             if ((t & 1) == 0) (s80 + i * (kOneThreads / 2))[(uint32_t)t >> 1] = (uint8_t)c.sc;

@@ -66,3 +66,32 @@ def test_read_once_then_smaller_weights(no_wait):
                 nvfp4_quantize_1d(x[5])]
         for i, (one, ref) in enumerate(zip(got, want)):
             _same(one, [t.cpu() for t in ref], f"run {run}, tensor {i}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_read_once_with_extreme_tensors(dtype):
+    """What the kernel that reads a tensor once leaves to the launch behind it: scales at the ends of the fp32 range,
+    infinities, NaN.  Its neighbours in the list stay where they are."""
+    g = torch.Generator(device="cuda").manual_seed(4)
+    x = torch.randn(8, 1024, 7168, generator=g, device="cuda").to(dtype)
+    left = [2, 4]
+    x[2, 17, 40] = float("inf")
+    x[4, 1023, 7167] = float("nan")
+    x[6].zero_()
+    if dtype == torch.bfloat16:
+        left += [1, 5, 7]
+        x[1] = (x[1].float() * 1e-30).bfloat16()
+        x[5] = (x[5].float() * 1e-40).bfloat16()           # subnormal elements
+        x[7] = (x[7].float() * 5e37).bfloat16()
+        x[7].clamp_(-3e38, 3e38)
+    with launch.recording() as batch:
+        got = [nvfp4_quantize_1d(w) for w in x]
+    for run in range(2):
+        if run == 1:
+            batch.carry_amax(adaptive=False)
+        batch.run()
+        if run == 0:
+            redo = [int(r[_lib.RECORD_REDO_WORD]) for r in batch.amax_records()]
+            assert redo == [int(i in left) for i in range(8)]        # (1e-30, 1e-40 and 3e38, over 2688: outside 2^-82 .. 2^81)
+        for i, one in enumerate(got):
+            _same(one, [t.cpu() for t in nvfp4_quantize_1d(x[i])], f"run {run}, tensor {i}")
