@@ -738,8 +738,9 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
 //     maximum, and every workgroup that reads it leaves at once: a record that does not fit next to a busy neighbour costs
 //     one wait, not one for each batch of its workgroups that comes to the chip.  32 x [2048, 7168] beside a stream of
 //     [8192, 8192] matrix products: 2.5 ms, 3.0 without that word, 2.35 in two passes (beside one of copies 0.56, 0.56, 0.91).
-// 32 x [2048, 7168] (940 MB of bf16, all launches together): 318 us in two passes, 226 us this way (5.4 TB/s; 234 with the
-// block maxima taken after the wait, a range test and a branch to the software forms in each unit).  24 units per lane at
+// 32 x [2048, 7168] (940 MB of bf16, all launches together): 318 us in two passes, 218 us this way (5.55 TB/s; 226 with a
+// block's scale computed in both lanes that hold it and its byte stored under a mask, 234 with the block maxima taken after the
+// wait and a range test and a branch to the software forms in each unit).  24 units per lane at
 // four workgroups per CU were 5 % slower, 8 units in 512 lanes 6 %, six workgroups per CU (20 registers spilled) 38 %; two
 // units stored together, eight bytes a lane, 2 % slower here and 2 % faster on 18 x [1420, 1520].
 constexpr int kOneThreads = 256, kOneUnits = 16, kOneWavesPerSimd = 5;
@@ -771,17 +772,35 @@ __global__ __launch_bounds__(256) void nvfp4_one_pass_clear_kernel(const Table t
 __device__ __forceinline__ uint32_t nv_block_max(const u32x4 v) {
     return group_max2(hmax_u16(max2_u16(max2_u16(abs2(v.x), abs2(v.y)), max2_u16(abs2(v.z), abs2(v.w)))));
 }
-// nvfp4_quant_unit for finite elements and 1 / S_enc in 2^-82 .. 2^81: a block scale is 0 or in 2^-9 .. 448, so the divisor of
-// every block with a scale is in the range of recip_shared; the others have the largest reciprocal, as 1 / 0 is cut to it
+// The scale byte and the factor of a block with finite elements, for 1 / S_enc in 2^-82 .. 2^81: a block scale is 0 or in
+// 2^-9 .. 448, so the divisor of every block with a scale is in the range of recip_shared.  For a divisor of zero that gives
+// NaN, and the minimum with the largest factor is that factor, as for 1 / 0.
+struct NvPlainScale {
+    uint32_t sc;        // (only the low byte)
+    float inv;
+};
+__device__ __forceinline__ NvPlainScale nv_plain_scale(const float bmax, const NvScales& gs) {
+    uint32_t any;
+    asm("" : "=v"(any));      // the bytes above are never read: nothing to clear before
+    NvPlainScale s;
+    s.sc = hw_e4m3x2<false>(__builtin_fminf(bmax * gs.enc_sixth, kFp8Max), 0.0f, any);
+    s.inv = __builtin_fminf(recip_shared(hw_e4m3x2_decode<false>(s.sc).x * gs.s_dec), kFltMax);
+    return s;
+}
 template <int F16>
-__device__ __forceinline__ NvUnitCodes nv_plain_unit(const u32x4 v, const uint32_t mb, const NvScales& gs) {
-    const uint32_t sc = hw_e4m3x2<false>(__builtin_fminf(elem_lo<F16>(mb) * gs.enc_sixth, kFp8Max), 0.0f, 0u) & 0xFFu;
-    const float inv = sc == 0u ? kFltMax : recip_shared(hw_e4m3x2_decode<false>(sc).x * gs.s_dec);
-    uint32_t word = hw_e2m1x2<0>(elem_lo<F16>(v.x) * inv, elem_hi<F16>(v.x) * inv, 0u);
+__device__ __forceinline__ uint32_t nv_plain_codes(const u32x4 v, const float inv) {
+    uint32_t word;
+    asm("" : "=v"(word));      // the four conversions write all of it
+    word = hw_e2m1x2<0>(elem_lo<F16>(v.x) * inv, elem_hi<F16>(v.x) * inv, word);
     word = hw_e2m1x2<1>(elem_lo<F16>(v.y) * inv, elem_hi<F16>(v.y) * inv, word);
     word = hw_e2m1x2<2>(elem_lo<F16>(v.z) * inv, elem_hi<F16>(v.z) * inv, word);
-    word = hw_e2m1x2<3>(elem_lo<F16>(v.w) * inv, elem_hi<F16>(v.w) * inv, word);
-    return NvUnitCodes{sc, word, mb};
+    return hw_e2m1x2<3>(elem_lo<F16>(v.w) * inv, elem_hi<F16>(v.w) * inv, word);
+}
+// the value that the even / the odd lane of each pair holds
+template <int ODD>
+__device__ __forceinline__ float pair_lane(const float v) {
+    const int bits = (int)f2u(v);
+    return u2f((uint32_t)__builtin_amdgcn_update_dpp(bits, bits, ODD ? 0xF5 /* 1, 1, 3, 3 */ : 0xA0 /* 0, 0, 2, 2 */, 0xF, 0xF, true));
 }
 
 // job as for the quantize pass: section = place of the tensor inside its record, pad = tensors sharing it (neighbours)
@@ -882,18 +901,26 @@ __global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_
         if (t == 0) rec[kRecRedo] = 1;
         return;
     }
+    // Both lanes of a pair hold the maxima of the same blocks: of two units the even lane takes the first one's scale and the
+    // odd lane the second one's, so that a scale is computed once and every lane stores a byte.
+    const uint32_t odd = (uint32_t)t & 1u;
     uint32_t* __restrict__ q0 = (uint32_t*)job.q + base;
     uint8_t* __restrict__ s80 = (uint8_t*)job.s + base / 2;
+    auto quantize = [&](auto full) {
 #pragma unroll
-    for (int i = 0; i < kOneUnits; i++) {
-        const uint32_t off = (uint32_t)t + i * kOneThreads;
-        const NvUnitCodes c = nv_plain_unit<F16>(v[i], (maxima[i / 2] >> (16 * (i & 1))) & 0xFFFFu, gs);
-        if (whole || off < rem) {
-            st4(q0 + i * kOneThreads + (uint32_t)t, c.word);
-            if ((t & 1) == 0) (s80 + i * (kOneThreads / 2))[(uint32_t)t >> 1] = (uint8_t)c.sc;
+        for (int i = 0; i < kOneUnits; i += 2) {
+            const uint32_t two = maxima[i / 2];
+            const NvPlainScale s = nv_plain_scale(odd ? elem_hi<F16>(two) : elem_lo<F16>(two), gs);
+            const uint32_t word0 = nv_plain_codes<F16>(v[i], pair_lane<0>(s.inv)), word1 = nv_plain_codes<F16>(v[i + 1], pair_lane<1>(s.inv));
+            const uint32_t off = (uint32_t)t + i * kOneThreads;
+            if (full || off < rem) st4(q0 + off, word0);
+            if (full || off + kOneThreads < rem) st4(q0 + off + kOneThreads, word1);
+            if (full || off + odd * kOneThreads < rem) s80[(off >> 1) + odd * (kOneThreads / 2)] = (uint8_t)s.sc;
+            __builtin_amdgcn_sched_barrier(0);      // two units at a time: more do not fit the registers
         }
-        __builtin_amdgcn_sched_barrier(0);      // one unit at a time: interleaved ones do not fit the registers
-    }
+    };
+    if (whole) quantize(std::true_type{});
+    else quantize(std::false_type{});
 }
 
 // Behind the one-pass kernel: quantizes the records that were left to it and publishes every record's amax, scales and

@@ -95,3 +95,21 @@ def test_read_once_with_extreme_tensors(dtype):
             assert redo == [int(i in left) for i in range(8)]        # (1e-30, 1e-40 and 3e38, over 2688: outside 2^-82 .. 2^81)
         for i, one in enumerate(got):
             _same(one, [t.cpu() for t in nvfp4_quantize_1d(x[i])], f"run {run}, tensor {i}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows, cols", [(1037, 3680), (1024, 4096), (1, 16 * 262147)])
+def test_read_once_with_empty_blocks(rows, cols, dtype):
+    """Blocks of zeros and blocks whose scale rounds to zero have the largest factor; the last workgroup's piece is cut off at
+    the first or the second of two units."""
+    g = torch.Generator(device="cuda").manual_seed(6)
+    x = (torch.randn(10, rows * cols // 16, 16, generator=g, device="cuda") * 0.02).to(dtype)
+    x[:, 5::11] = 0.0
+    x[:, 7::13] *= 2.0 ** -14
+    x[:, ::17, 3] *= -0.0
+    x[:, -1, 15] = torch.arange(1.0, 11.0, device="cuda").to(dtype)
+    x = x.view(10, rows, cols)
+    with launch.deferred():
+        got = [nvfp4_quantize_1d(w) for w in x]
+    for i, one in enumerate(got):
+        _same(one, [t.cpu() for t in nvfp4_quantize_1d(x[i])], f"tensor {i}")
