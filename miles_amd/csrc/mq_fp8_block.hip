@@ -478,10 +478,10 @@ __global__ __launch_bounds__(256) void fp8_row_quant_kernel(const void* __restri
 // 8192] bf16 72 -> 61 (6.6 TB/s), fp32 129 -> 108 (6.2), [4095, 8191] bf16 90 -> 74, [1024, 2048] bf16 16.8 -> 6.0; per tensor
 // [4096, 8192] fp32 218 -> 179, [4095, 8191] bf16 138 -> 104, [1024, 2048] fp32 39 -> 16.
 template <int DT> constexpr int kUnitElems = DT == MQ_F32 ? 4 : 8;
-template <int DT, bool LINES>
+template <int DT, bool LINES, bool KEEP = false>
 __device__ __forceinline__ u32x4 ld_unit(const void* p, int64_t elem) {
     const char* at = (const char*)p + elem * (DT == MQ_F32 ? 4 : 2);
-    return LINES ? ld16(at) : ld16_at2(at);
+    return !LINES ? ld16_at2(at) : KEEP ? ld16_keep(at) : ld16(at);
 }
 // the largest magnitude of a unit: an fp32 pattern, or packed 16-bit patterns
 template <int DT>
@@ -621,8 +621,15 @@ struct ScaledTable {
 // by each wavefront: four [4096, 8192] fp32 111 us in the second pass instead of 101.)  As jobs a workgroup of the amax
 // pass has a word of its own; the direct calls have fewer words than workgroups, cleared beforehand, and take the maximum
 // atomically, at some 8 ns each.
-constexpr int kScaledLoads = 4, kScaledUnits = 2, kAmaxThreads = 1024, kScaledWords = 256, kDirectWords = 64, kDirectBlocks = 256;
-template <int DT, bool LINES>
+constexpr int kScaledLoads = 4, kScaledUnits = 4, kScaledShortUnits = 2, kAmaxThreads = 1024, kScaledWords = 256, kDirectWords = 64, kDirectBlocks = 256;
+// KEEP of the four loads of a trip are left in the memory-side cache for the quantize pass (kept_quarters; unaligned loads
+// carry no hint and stay there anyway).
+// A lane of the quantize pass takes four units, which is what gains by that cache (two: four [4096, 8192] bf16 62.5 us against
+// 56.4, without the cache 63.5 and 63.9); of a list under 8 MiB, two, which leaves it twice the workgroups (two [512, 1024]
+// 3.5 us, 4.4 with four).  Both passes together, us, before and after: four [4096, 8192] bf16 105 -> 100, fp32 179 -> 171,
+// two [4095, 8191] 55.4 -> 53.2, eight [2198, 1333] 25.6 -> 22.9.
+constexpr int64_t kScaledLongList = (8ll << 20) / 16;       // units of a list
+template <int DT, bool LINES, int KEEP>
 __global__ __launch_bounds__(kAmaxThreads) void fp8_scaled_amax_kernel(const ScaledTable tab) {
     __shared__ uint32_t wave_amax[kAmaxThreads / kWave];
     constexpr int E = kUnitElems<DT>;
@@ -633,8 +640,14 @@ __global__ __launch_bounds__(kAmaxThreads) void fp8_scaled_amax_kernel(const Sca
     uint32_t m = 0;
     for (int64_t base = (int64_t)blockIdx.x * (kAmaxThreads * kScaledLoads); base < units; base += (int64_t)gridDim.x * (kAmaxThreads * kScaledLoads)) {
         u32x4 v[kScaledLoads];
+        // (a loop for each kind: loads that one loop chooses between lose the hint)
 #pragma unroll
-        for (int i = 0; i < kScaledLoads; i++) {
+        for (int i = 0; i < KEEP; i++) {
+            const int64_t at = (base + i * kAmaxThreads + t) * E;
+            v[i] = ld_unit<DT, LINES, true>(w, at < last ? at : last);
+        }
+#pragma unroll
+        for (int i = KEEP; i < kScaledLoads; i++) {
             const int64_t at = (base + i * kAmaxThreads + t) * E;
             v[i] = ld_unit<DT, LINES>(w, at < last ? at : last);
         }
@@ -653,7 +666,7 @@ __global__ __launch_bounds__(kAmaxThreads) void fp8_scaled_amax_kernel(const Sca
     if (tab.amax_blocks > tab.words) atomicMax(word, m);
     else *word = m;
 }
-template <int DT, bool LINES>
+template <int DT, bool LINES, int UNITS>
 __global__ __launch_bounds__(256) void fp8_scaled_quant_kernel(const ScaledTable tab) {
     __shared__ uint32_t wave_amax[4];
     constexpr int E = kUnitElems<DT>;
@@ -661,12 +674,12 @@ __global__ __launch_bounds__(256) void fp8_scaled_quant_kernel(const ScaledTable
     const void* __restrict__ w = load_global_ptr(&job.w);
     const uint32_t* __restrict__ maxima = load_global_ptr(&job.maxima);
     uint8_t* __restrict__ q = load_global_ptr(&job.q);
-    const int64_t n = job.n, first = xcd_chunked_block(tab.chunk) * (256 * kScaledUnits), base = first + threadIdx.x;
+    const int64_t n = job.n, first = xcd_chunked_block(tab.chunk) * (256 * UNITS), base = first + threadIdx.x;
     if (first * E >= n) return;
     const int64_t last = LINES ? n / E * E - E : n - E;
-    u32x4 v[kScaledUnits];
+    u32x4 v[UNITS];
 #pragma unroll
-    for (int i = 0; i < kScaledUnits; i++) {
+    for (int i = 0; i < UNITS; i++) {
         const int64_t at = (base + i * 256) * E;
         v[i] = ld_unit<DT, LINES>(w, at < last ? at : last);
     }
@@ -683,7 +696,7 @@ __global__ __launch_bounds__(256) void fp8_scaled_quant_kernel(const ScaledTable
     const bool plain = shared_div_ok(s);
     if (base == 0) *load_global_ptr(&job.scale) = s;
 #pragma unroll
-    for (int i = 0; i < kScaledUnits; i++) {
+    for (int i = 0; i < UNITS; i++) {
         const int64_t at = (base + i * 256) * E;
         if (!LINES && at < n) scaled_unit<DT, true, false>(v[i], s, y, plain, q + (at < last ? at : last));
         else if (LINES && at <= last) scaled_unit<DT, true, true>(v[i], s, y, plain, q + at);
@@ -1029,9 +1042,13 @@ int mq_fp8_scaled_form(const void* w, int dtype, int64_t ldw, const void* q, int
     return (uintptr_t)w % 16 == 0 && (uintptr_t)q % E == 0 ? 1 : 2;
 }
 template <int DT, bool LINES>
-static void scaled_launch(const ScaledTable& tab, hipStream_t st) {
-    hipLaunchKernelGGL((fp8_scaled_amax_kernel<DT, LINES>), dim3((unsigned)tab.amax_blocks, (unsigned)tab.n), dim3(kAmaxThreads), 0, st, tab);
-    hipLaunchKernelGGL((fp8_scaled_quant_kernel<DT, LINES>), dim3((unsigned)tab.max_blocks, (unsigned)tab.n), dim3(256), 0, st, tab);
+static void scaled_launch(const ScaledTable& tab, int keep, bool whole, hipStream_t st) {
+    const dim3 amax((unsigned)tab.amax_blocks, (unsigned)tab.n), quant((unsigned)tab.max_blocks, (unsigned)tab.n);
+    if (!LINES || keep == 4) hipLaunchKernelGGL((fp8_scaled_amax_kernel<DT, LINES, 4>), amax, dim3(kAmaxThreads), 0, st, tab);
+    else if (keep == 2) hipLaunchKernelGGL((fp8_scaled_amax_kernel<DT, LINES, LINES ? 2 : 4>), amax, dim3(kAmaxThreads), 0, st, tab);
+    else hipLaunchKernelGGL((fp8_scaled_amax_kernel<DT, LINES, LINES ? 0 : 4>), amax, dim3(kAmaxThreads), 0, st, tab);
+    if (whole) hipLaunchKernelGGL((fp8_scaled_quant_kernel<DT, LINES, kScaledUnits>), quant, dim3(256), 0, st, tab);
+    else hipLaunchKernelGGL((fp8_scaled_quant_kernel<DT, LINES, kScaledShortUnits>), quant, dim3(256), 0, st, tab);
 }
 // n <= kMaxGroup tensors of one dtype and one form, each with `words` words for its partial maxima (a power of two; fewer than
 // kScaledWords: cleared first)
@@ -1039,9 +1056,10 @@ int mq_fp8_scaled_launch_group(int dtype, int form, const MqScaledArgs* a, int n
     ScaledTable tab{};
     tab.n = n;
     const int64_t E = dtype == MQ_F32 ? 4 : 8;
-    int64_t units = 0;
+    int64_t units = 0, all = 0;
     for (int i = 0; i < n; i++) {
         const int64_t numel = a[i].M * a[i].K, u = (numel + E - 1) / E;
+        all += u;
         tab.job[i] = ScaledJob{a[i].w, (uint8_t*)a[i].q, a[i].scale, a[i].maxima, numel, a[i].floor_v, 0};
         units = u > units ? u : units;
     }
@@ -1057,14 +1075,16 @@ int mq_fp8_scaled_launch_group(int dtype, int form, const MqScaledArgs* a, int n
         tab.amax_blocks = (int32_t)(trips < kDirectBlocks ? trips : kDirectBlocks);
         for (int i = 0; i < n; i++) hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, a[i].maxima, 0u, words);
     }
-    const int64_t blocks = (units + 256 * kScaledUnits - 1) / (256 * kScaledUnits), chunk = flat_chunk(blocks);
+    const bool whole = all >= kScaledLongList;
+    const int64_t block = 256 * (whole ? kScaledUnits : kScaledShortUnits), blocks = (units + block - 1) / block, chunk = flat_chunk(blocks);
     if (flat_padded(blocks, chunk) >= 0x7FFFFFF0) return mq_fail(MQ_ERR_ARG, "tensor too large");
     tab.chunk = (int32_t)chunk;
     tab.max_blocks = (int32_t)flat_padded(blocks, chunk);
     const bool lines = form == 1;
-    if (dtype == MQ_F32) lines ? scaled_launch<MQ_F32, true>(tab, st) : scaled_launch<MQ_F32, false>(tab, st);
-    else if (dtype == MQ_F16) lines ? scaled_launch<MQ_F16, true>(tab, st) : scaled_launch<MQ_F16, false>(tab, st);
-    else lines ? scaled_launch<MQ_BF16, true>(tab, st) : scaled_launch<MQ_BF16, false>(tab, st);
+    const int keep = kept_quarters(all * 16);
+    if (dtype == MQ_F32) lines ? scaled_launch<MQ_F32, true>(tab, keep, whole, st) : scaled_launch<MQ_F32, false>(tab, keep, whole, st);
+    else if (dtype == MQ_F16) lines ? scaled_launch<MQ_F16, true>(tab, keep, whole, st) : scaled_launch<MQ_F16, false>(tab, keep, whole, st);
+    else lines ? scaled_launch<MQ_BF16, true>(tab, keep, whole, st) : scaled_launch<MQ_BF16, false>(tab, keep, whole, st);
     return mq_check_launch("fp8 scaled quant");
 }
 

@@ -195,6 +195,14 @@ inline bool flat_grid(FlatRef& ref, int64_t max_units, int64_t per_block) {
     return mx < 0x7FFFFFF0;
 }
 
+// How many of every four loads the first of two passes over `bytes` of input issues without the non-temporal hint, which
+// leaves their lines in the 256 MB memory-side cache for the second pass (a second pass keeps the hint, and its stores too).
+// Four of four make the first pass 6 % slower, two of four do not, and the second one finds what fits: all of a list of that
+// size, half of a longer one, nothing of a list several times as long.  Device time of both passes, us, with 0 / 2 / 4 of four:
+// fake quantization of six [4096, 4096] (201 MB) 97 / 90 / 89, of four [4096, 7168] with Four Over Six (235 MB) 114 / 110 / 107;
+// NVFP4 of 403 MB 139 / 133 / 140, of 537 MB fp32 168 / 162 / 175, of 940 MB 311 / 312 / 326, of 1.9 GB 615 / 625 / 654.
+inline int kept_quarters(int64_t bytes) { return bytes <= (256ll << 20) ? 4 : bytes <= (768ll << 20) ? 2 : 0; }
+
 // one MXFP4 tensor re-coded as FP8 with 128 x 128 scales: a workgroup takes a pair of tiles, neighbours along `in`
 struct RecodeJob {
     const uint8_t* packed;    // [out, in / 2] e2m1 pairs

@@ -33,15 +33,13 @@ static_assert(kSectionWords == MQ_NVFP4_SECTION_WORDS && kRecordSections == MQ_N
 #ifndef MQ_AMAX_UNROLL
 #define MQ_AMAX_UNROLL 4
 #endif
-#ifndef MQ_AMAX_NT
-#define MQ_AMAX_NT 1
-#endif
 constexpr int kAmaxUnroll = MQ_AMAX_UNROLL;             // 16-byte units per lane per loop trip
 
 // grid (up to kSectionWords, tensors): workgroup b of a tensor strides over its 16 KiB chunks and writes word b of
 // the section.  A launch whose largest tensor has fewer chunks takes that many workgroups, which write a zero into the
 // words nobody owns (amax_section_store): fifty-nine tensors of 17 chunks 8.7 us with 256 workgroups each, 5.1 with 17.
 // job.units counts whole 16-byte units; job.s carries the element count for the sub-unit tail.
+// KEEP of a lane's four loads are left in the memory-side cache for the pass behind (kept_quarters).
 // (descriptors of a device table are in the quantizer's form, whose tensors are whole units: no tail, and job.s is the
 // block-scale pointer there)
 // (16-bit inputs, bf16 or fp16: the maximum is taken on the absolute bit patterns and converted to the fp32 pattern once)
@@ -49,7 +47,7 @@ __device__ __forceinline__ void amax_section_store(uint32_t* __restrict__ sectio
     const uint32_t word = blockIdx.x + (uint32_t)t * gridDim.x;
     if (word < (uint32_t)kSectionWords) section[word] = t == 0 ? m : 0u;
 }
-template <class Table, int F16>
+template <class Table, int F16, int KEEP>
 __global__ __launch_bounds__(256) void nvfp4_amax_bf16_kernel(const Table tab) {
     __shared__ uint32_t wave_amax[4];
     const FlatJob job = flat_job(tab);       // a copy in registers: a descriptor in device memory must not be re-read after the stores
@@ -60,10 +58,16 @@ __global__ __launch_bounds__(256) void nvfp4_amax_bf16_kernel(const Table tab) {
     uint32_t m2 = 0;
     for (int64_t base = (int64_t)blockIdx.x * (256 * kAmaxUnroll); base < n16; base += (int64_t)gridDim.x * 256 * kAmaxUnroll) {
         u32x4 v[kAmaxUnroll];
+        // (a loop for each kind: loads that one loop chooses between lose the hint)
 #pragma unroll
-        for (int i = 0; i < kAmaxUnroll; i++) {
+        for (int i = 0; i < KEEP; i++) {
             const int64_t unit = base + i * 256 + t;
-            v[i] = unit < n16 ? (MQ_AMAX_NT ? ld16(w + unit * 8) : ld16_keep(w + unit * 8)) : u32x4{0u, 0u, 0u, 0u};
+            v[i] = unit < n16 ? ld16_keep(w + unit * 8) : u32x4{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (int i = KEEP; i < kAmaxUnroll; i++) {
+            const int64_t unit = base + i * 256 + t;
+            v[i] = unit < n16 ? ld16(w + unit * 8) : u32x4{0u, 0u, 0u, 0u};
         }
 #pragma unroll
         for (int i = 0; i < kAmaxUnroll; i++)
@@ -79,7 +83,7 @@ __global__ __launch_bounds__(256) void nvfp4_amax_bf16_kernel(const Table tab) {
 }
 
 // fp32 input (units and the element count as above): 16-byte loads of four elements
-template <class Table>
+template <class Table, int KEEP>
 __global__ __launch_bounds__(256) void nvfp4_amax_f32_kernel(const Table tab) {
     __shared__ uint32_t wave_amax[4];
     const FlatJob job = flat_job(tab);
@@ -90,7 +94,12 @@ __global__ __launch_bounds__(256) void nvfp4_amax_f32_kernel(const Table tab) {
     for (int64_t base = (int64_t)blockIdx.x * (256 * kAmaxUnroll); base < loads; base += (int64_t)gridDim.x * 256 * kAmaxUnroll) {
         u32x4 v[kAmaxUnroll];
 #pragma unroll
-        for (int i = 0; i < kAmaxUnroll; i++) {
+        for (int i = 0; i < KEEP; i++) {
+            const int64_t at = base + i * 256 + t;
+            v[i] = at < loads ? ld16_keep(w + at * 4) : u32x4{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (int i = KEEP; i < kAmaxUnroll; i++) {
             const int64_t at = base + i * 256 + t;
             v[i] = at < loads ? ld16(w + at * 4) : u32x4{0u, 0u, 0u, 0u};
         }
@@ -738,7 +747,7 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
 //     maximum, and every workgroup that reads it leaves at once: a record that does not fit next to a busy neighbour costs
 //     one wait, not one for each batch of its workgroups that comes to the chip.  32 x [2048, 7168] beside a stream of
 //     [8192, 8192] matrix products: 2.5 ms, 3.0 without that word, 2.35 in two passes (beside one of copies 0.56, 0.56, 0.91).
-// 32 x [2048, 7168] (940 MB of bf16, all launches together): 318 us in two passes, 218 us this way (5.55 TB/s; 226 with a
+// 32 x [2048, 7168] (940 MB of bf16, all launches together): 311 us in two passes, 218 us this way (5.55 TB/s; 226 with a
 // block's scale computed in both lanes that hold it and its byte stored under a mask, 234 with the block maxima taken after the
 // wait and a range test and a branch to the software forms in each unit).  24 units per lane at
 // four workgroups per CU were 5 % slower, 8 units in 512 lanes 6 %, six workgroups per CU (20 registers spilled) 38 %; two
@@ -1215,25 +1224,37 @@ static unsigned amax_blocks(int dtype, int64_t max_units) {
     const int64_t chunks = (max_units * (dtype == MQ_F32 ? 2 : 1) + 256 * kAmaxUnroll - 1) / (256 * kAmaxUnroll);
     return (unsigned)(chunks < 1 ? 1 : chunks < kSectionWords ? chunks : kSectionWords);
 }
-int mq_nvfp4_amax_launch_group(int dtype, FlatTable& tab, hipStream_t st) {
-    int64_t max_units = 0;
-    for (int i = 0; i < tab.n; i++) max_units = tab.job[i].units > max_units ? tab.job[i].units : max_units;
-    const dim3 grid(amax_blocks(dtype, max_units), (unsigned)tab.n), blk(256);
-    if (dtype == MQ_F32) hipLaunchKernelGGL(nvfp4_amax_f32_kernel<FlatTable>, grid, blk, 0, st, tab);
-    else if (dtype == MQ_F16) hipLaunchKernelGGL((nvfp4_amax_bf16_kernel<FlatTable, 1>), grid, blk, 0, st, tab);
-    else hipLaunchKernelGGL((nvfp4_amax_bf16_kernel<FlatTable, 0>), grid, blk, 0, st, tab);
+template <int KEEP, class Table>
+static void launch_nvfp4_amax_kept(int dtype, const Table& tab, dim3 grid, hipStream_t st) {
+    const dim3 blk(256);
+    if (dtype == MQ_F32) hipLaunchKernelGGL((nvfp4_amax_f32_kernel<Table, KEEP>), grid, blk, 0, st, tab);
+    else if (dtype == MQ_F16) hipLaunchKernelGGL((nvfp4_amax_bf16_kernel<Table, 1, KEEP>), grid, blk, 0, st, tab);
+    else hipLaunchKernelGGL((nvfp4_amax_bf16_kernel<Table, 0, KEEP>), grid, blk, 0, st, tab);
+}
+// max_units: the largest tensor's units; all_units: of all n tensors
+template <class Table>
+static int launch_nvfp4_amax(int dtype, const Table& tab, int n, int64_t max_units, int64_t all_units, hipStream_t st) {
+    const dim3 grid(amax_blocks(dtype, max_units), (unsigned)n);
+    switch (kept_quarters(all_units * (dtype == MQ_F32 ? 32 : 16))) {
+        case 4: launch_nvfp4_amax_kept<4>(dtype, tab, grid, st); break;
+        case 2: launch_nvfp4_amax_kept<2>(dtype, tab, grid, st); break;
+        default: launch_nvfp4_amax_kept<0>(dtype, tab, grid, st); break;
+    }
     return mq_check_launch("nvfp4 amax");
+}
+int mq_nvfp4_amax_launch_group(int dtype, FlatTable& tab, hipStream_t st) {
+    int64_t max_units = 0, all_units = 0;
+    for (int i = 0; i < tab.n; i++) {
+        max_units = tab.job[i].units > max_units ? tab.job[i].units : max_units;
+        all_units += tab.job[i].units;
+    }
+    return launch_nvfp4_amax(dtype, tab, tab.n, max_units, all_units, st);
 }
 // the same over n descriptors of a device table (the quantizer's form: whole units, section = place inside the record);
 // max_units: the largest tensor's units
 int mq_nvfp4_amax_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, hipStream_t st) {
     if (n == 0) return MQ_OK;
-    const FlatRef ref{device_jobs, 0, 0};
-    const dim3 grid(amax_blocks(dtype, max_units), (unsigned)n), blk(256);
-    if (dtype == MQ_F32) hipLaunchKernelGGL(nvfp4_amax_f32_kernel<FlatRef>, grid, blk, 0, st, ref);
-    else if (dtype == MQ_F16) hipLaunchKernelGGL((nvfp4_amax_bf16_kernel<FlatRef, 1>), grid, blk, 0, st, ref);
-    else hipLaunchKernelGGL((nvfp4_amax_bf16_kernel<FlatRef, 0>), grid, blk, 0, st, ref);
-    return mq_check_launch("nvfp4 amax");
+    return launch_nvfp4_amax(dtype, FlatRef{device_jobs, 0, 0}, n, max_units, max_units * n, st);
 }
 
 template <int PASS, class Table, int F16>
@@ -1325,10 +1346,9 @@ int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, in
 // largest number of workgroups that share a record, `bytes` the input of the whole chunk.  All workgroups of a record
 // have to be on the chip together, and the records behind it should be loading meanwhile: half of what fits (640 workgroups,
 // 40 MB, on 256 CUs).  A pair of [2048, 7168] weights, 896 workgroups, gained less (313 -> 265 us for 16 pairs) and is one
-// busy neighbour away from waiting in vain, so it keeps two passes.  Short lists keep them as well, which then find part of
-// their second read in the memory-side cache and save a launch (us, two passes / one): 4 x [1537, 2064] (25 MB) 14 / 18,
-// 4 x [2048, 4096] (67 MB) 26 / 24, 18 x [1420, 1520] (78 MB) 30 / 33, 16 x [1536, 2048] (100 MB) 37 / 34,
-// 48 x [1536, 2048] (302 MB) 105 / 77.
+// busy neighbour away from waiting in vain, so it keeps two passes.  Short lists keep them as well, which then find their second
+// read in the memory-side cache and save a launch (us, two passes / one): 4 x [1537, 2064] (25 MB) 15 / 18, 4 x [2048, 4096]
+// (67 MB) 27 / 24, 18 x [1420, 1520] (78 MB) 33 / 30, 16 x [1536, 2048] (100 MB) 39 / 33, 48 x [1536, 2048] (302 MB) 105 / 73.
 constexpr int64_t kOneMinBytes = 64ll << 20;
 bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes) {
     int device = 0, cus = 0;
