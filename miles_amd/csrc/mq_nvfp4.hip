@@ -6,7 +6,7 @@
 //              inv = min(1 / (f32(s8) * S_dec), FLT_MAX);  code = sat_e2m1(x * inv)
 //   published global scale: 1 / min(e4m3_max*6/amax, FLT_MAX) with only the ==0 repair (nvfp4.py:19-39)
 //
-// Pass 1 (mq_nvfp4_amax): 256 workgroups per tensor stream its elements and each writes one partial maximum
+// Pass 1 (mq_nvfp4_amax): up to 256 workgroups per tensor stream its elements and each writes one partial maximum
 // into the tensor's section of the amax record: plain stores, no atomics (thousands of agent-scope atomics
 // on one address serialise at ~8 ns each on this multi-XCD part) and nothing to clear.
 // Lists of tensors that fit the chip's registers a few at a time run in one pass instead (nvfp4_one_pass_kernel).
@@ -1147,9 +1147,9 @@ __global__ __launch_bounds__(256) void nvfp4_quant_generic_kernel(const void* __
 //   final = RN(RN(f32(s8) * amax) * f32(1 / (6 * e4m3_max)));  y = dtype(RN(e2m1_value * final))
 // Nothing but x (and the amax, see nv_fake_amax) is read and nothing but y written.  job: w = x, q = y, units.
 // Standard blocks: two lanes own one 1x16 block.  Four Over Six: nvfp4_fos_units.
-// Standard blocks are bound by HBM: sixteen [1536, 2048] weights in one launch 33 us (6.1 TB/s; one launch per weight 4.6 us
-// each).  Four Over Six is bound by vector instructions: four [4096, 7168] weights 77 us with a lane per block, 120 us with
-// two lanes per block and the exact error sums throughout.
+// Both are bound by memory, the reads by the memory-side cache where the amax pass left its input there: sixteen [1536, 2048]
+// weights in one launch 28.4 us (33 from HBM; one launch per weight 4.6 us each), four [4096, 7168] with Four Over Six 67 us
+// (78 from HBM; 120 with two lanes per block and the exact error sums throughout, where vector instructions were the bound).
 template <int FOS, int F16>
 __global__ __launch_bounds__(kNvThreads) void nvfp4_fake_kernel(const FlatTable tab, float numer, float inv_numer) {
     const FlatJob job = flat_job(tab);
