@@ -161,9 +161,12 @@ PyObject* scope_leave(PyObject*, PyObject*) {
     Py_RETURN_NONE;
 }
 
+// false, and no error set, for what is no integer of 64 bits: the call goes back to Python
 bool integer(PyObject* o, int64_t& v) {
     v = PyLong_AsLongLong(o);
-    return !(v == -1 && PyErr_Occurred());
+    if (v != -1 || !PyErr_Occurred()) return true;
+    PyErr_Clear();
+    return false;
 }
 // Records the job or runs it; false with the error set if it is refused.
 bool place(const mq_job& job, const at::Tensor& in, const at::Tensor* const* named, int n) {
@@ -201,10 +204,10 @@ PyObject* submit(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!named[0]) Py_RETURN_FALSE;
     int64_t v[9];
     for (int i = 0; i < 7; i++)
-        if (!integer(a[7 + i], v[i])) return nullptr;
-    if (!integer(a[0], v[7])) return nullptr;
+        if (!integer(a[7 + i], v[i])) Py_RETURN_FALSE;
+    if (!integer(a[0], v[7])) Py_RETURN_FALSE;
     if (a[1] == Py_None) v[8] = dtype_code(in->scalar_type()) < 0 ? 0 : dtype_code(in->scalar_type());
-    else if (!integer(a[1], v[8])) return nullptr;
+    else if (!integer(a[1], v[8])) Py_RETURN_FALSE;
     const mq_job job{(int32_t)v[7], (int32_t)v[8], in->data_ptr(), data(named[0]), data(named[1]), data(named[2]), data(named[3]),
                      v[0], v[1], v[2], (int32_t)v[3], (int32_t)v[4], v[5], v[6]};
     if (!place(job, *in, named, 4)) return nullptr;
@@ -218,10 +221,7 @@ struct Spec {
     c10::SmallVector<int64_t, 4> sizes;
 };
 bool spec_of(PyObject* o, Spec& s) {
-    if (!PyTuple_Check(o) || PyTuple_GET_SIZE(o) < 1 || !THPDtype_Check(PyTuple_GET_ITEM(o, 0))) {
-        PyErr_SetString(PyExc_TypeError, "produce: an output is (dtype, *sizes)");
-        return false;
-    }
+    if (!PyTuple_Check(o) || PyTuple_GET_SIZE(o) < 1 || !THPDtype_Check(PyTuple_GET_ITEM(o, 0))) return false;
     s.dtype = ((THPDtype*)PyTuple_GET_ITEM(o, 0))->scalar_type;
     for (Py_ssize_t i = 1; i < PyTuple_GET_SIZE(o); i++) {
         int64_t v;
@@ -242,16 +242,16 @@ PyObject* produce(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (a[3] != Py_None && !(aux_in = ordinary(a[3]))) Py_RETURN_NONE;
     int64_t v[7];
     for (int i = 0; i < 5; i++)
-        if (!integer(a[4 + i], v[i])) return nullptr;
-    if (!integer(a[0], v[5])) return nullptr;
+        if (!integer(a[4 + i], v[i])) Py_RETURN_NONE;
+    if (!integer(a[0], v[5])) Py_RETURN_NONE;
     if (a[1] == Py_None) v[6] = dtype_code(in->scalar_type()) < 0 ? 0 : dtype_code(in->scalar_type());
-    else if (!integer(a[1], v[6])) return nullptr;
+    else if (!integer(a[1], v[6])) Py_RETURN_NONE;
     Spec spec[4];
     bool make[4];
     int count = 0;
     for (int i = 0; i < 4; i++) {
         make[i] = a[9 + i] != Py_None;
-        if (make[i] && !spec_of(a[9 + i], spec[i])) return nullptr;
+        if (make[i] && !spec_of(a[9 + i], spec[i])) Py_RETURN_NONE;
         count += make[i];
     }
     at::Tensor made[4];
@@ -283,7 +283,7 @@ PyObject* act_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const at::Tensor* x = ordinary(a[0]);
     int64_t block, flags;
     if (!x || listing() || !ordinary_moment() || !x->is_contiguous() || x->dim() == 0 || dtype_code(x->scalar_type()) < 0) Py_RETURN_NONE;
-    if (!integer(a[1], block) || !integer(a[2], flags)) return nullptr;
+    if (!integer(a[1], block) || !integer(a[2], flags)) Py_RETURN_NONE;
     if (block <= 0 || block > 0x7FFFFFFF || x->size(-1) % block != 0 || !THPDtype_Check(a[3])) Py_RETURN_NONE;
     c10::SmallVector<int64_t, 4> sizes(x->sizes().begin(), x->sizes().end());
     sizes.back() /= block;
@@ -323,7 +323,7 @@ PyObject* fake_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const at::Tensor* x = ordinary(a[0]);
     int64_t mode, block;
     if (listing() || !ordinary_moment() || !imageable(x) || dtype_code(x->scalar_type()) < 0) Py_RETURN_NONE;
-    if (!integer(a[1], mode) || !integer(a[2], block)) return nullptr;
+    if (!integer(a[1], mode) || !integer(a[2], block)) Py_RETURN_NONE;
     if (block <= 0 || x->size(-1) % block != 0) Py_RETURN_NONE;
     at::Tensor y;
     int rc;
@@ -344,7 +344,7 @@ PyObject* simulate(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const at::Tensor* x = ordinary(a[0]);
     int64_t block, flags;
     if (listing() || !ordinary_moment() || !imageable(x) || dtype_code(x->scalar_type()) < 0) Py_RETURN_NONE;
-    if (!integer(a[1], block) || !integer(a[2], flags)) return nullptr;
+    if (!integer(a[1], block) || !integer(a[2], flags)) Py_RETURN_NONE;
     if (block <= 0 || block > 0x7FFFFFFF || x->size(-1) % block != 0) Py_RETURN_NONE;
     c10::SmallVector<int64_t, 4> sizes(x->sizes().begin(), x->sizes().end());
     sizes.back() /= block;
@@ -365,10 +365,10 @@ PyObject* simulate(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // 16-bit dtype, one device, contiguous, whole blocks, 16-byte aligned), a node for each, or None
 PyObject* nvfp4_images(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    if (n != 5 || !PyList_Check(a[0])) return PyErr_Format(PyExc_TypeError, "nvfp4_images: a list and 4 numbers");
-    if (listing() || !ordinary_moment()) Py_RETURN_NONE;
+    if (n != 5) return PyErr_Format(PyExc_TypeError, "nvfp4_images: 5 arguments");
+    if (!PyList_Check(a[0]) || listing() || !ordinary_moment()) Py_RETURN_NONE;
     int64_t block, words, e4m3_max, flags;
-    if (!integer(a[1], block) || !integer(a[2], words) || !integer(a[3], e4m3_max) || !integer(a[4], flags)) return nullptr;
+    if (!integer(a[1], block) || !integer(a[2], words) || !integer(a[3], e4m3_max) || !integer(a[4], flags)) Py_RETURN_NONE;
     std::vector<at::Tensor> weights, images;
     std::vector<mq_fake_quant_item> items;
     for (Py_ssize_t i = 0; i < PyList_GET_SIZE(a[0]); i++) {
@@ -409,7 +409,7 @@ PyObject* int4_fake(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const at::Tensor* x = ordinary(a[0]);
     int64_t bm, bn, sym;
     if (!x || listing() || !ordinary_moment() || x->dim() != 2 || !x->is_contiguous() || dtype_code(x->scalar_type()) < 0) Py_RETURN_NONE;
-    if (!integer(a[1], bm) || !integer(a[2], bn) || !integer(a[3], sym)) return nullptr;
+    if (!integer(a[1], bm) || !integer(a[2], bn) || !integer(a[3], sym)) Py_RETURN_NONE;
     if (bm <= 0 || bn <= 0 || bm > 0x7FFFFFFF || bn > 0x7FFFFFFF) Py_RETURN_NONE;
     at::Tensor y, s, z;
     int rc;
