@@ -279,14 +279,22 @@ def records_for_replay() -> bool:
     return batch is not None and batch.kept
 
 
-class deferred:
+class deferred(contextlib.ContextDecorator):
     """Record the quantizer calls made inside the block and submit them together on exit.
 
     Inside an enclosing `deferred()` / `recording()` block this is a pass-through: the jobs join the outer
-    batch and run when that one does.
+    batch and run when that one does.  As a decorator it makes every call of the function such a block.
     """
 
+    _entered = False
+
+    def _recreate_cm(self) -> deferred:
+        return deferred()       # (threads, and a function that calls itself, may be in several at a time)
+
     def __enter__(self) -> JobBatch:
+        if self._entered:
+            raise RuntimeError("a deferred() block is entered once")
+        self._entered = True
         outer = active_batch()
         self._own = None if outer is not None else JobBatch()
         if self._own is None:

@@ -1,8 +1,11 @@
 """Forms of a call that the host layer does not take itself: each is answered, or refused, as the Python path does it."""
 
+import threading
+
 import pytest
 import torch
 
+from miles_amd import launch
 from miles_amd._host import native
 from miles_amd.kernels.quant import fp8_act_quant as aq
 from miles_amd.kernels.quant import nvfp4_qdq as nq
@@ -39,3 +42,49 @@ def test_the_block_size_is_taken_or_refused_as_in_python(block):
             return type(e)
 
     assert answer(aq.fp8_simulate_qat) == answer(aq.DeepSeekV4LinearQATFunc.apply)
+
+
+def test_deferred_decorates_a_function():
+    """Every call has a block of its own: calls inside join it, threads do not, and it is gone afterwards."""
+    @launch.deferred()
+    def call(depth, seen):
+        batch = launch.active_batch()
+        seen.append(batch)
+        if depth:
+            call(depth - 1, seen)
+        if depth == 7:
+            raise KeyError
+        assert launch.active_batch() is batch
+        return len(batch)
+
+    seen = []
+    assert call.__name__ == "call" and call(1, seen) == 0 and call(0, seen) == 0
+    assert seen[0] is seen[1] is not seen[2] and None not in seen and launch.active_batch() is None
+    with pytest.raises(KeyError):
+        call(7, [])
+    assert launch.active_batch() is None
+    both = threading.Barrier(2, timeout=30)
+    found = []
+
+    @launch.deferred()
+    def meet():
+        both.wait()
+        found.append(launch.active_batch())
+        both.wait()
+
+    threads = [threading.Thread(target=meet) for _ in range(2)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert len(found) == 2 and found[0] is not found[1] and None not in found
+
+
+def test_a_deferred_block_is_entered_once():
+    block = launch.deferred()
+    with block as outer:
+        with pytest.raises((RuntimeError, AttributeError)), block:
+            pass
+        assert launch.active_batch() is outer
+    assert launch.active_batch() is None
+    with pytest.raises((RuntimeError, AttributeError)), block:
+        pass
+    assert launch.active_batch() is None
