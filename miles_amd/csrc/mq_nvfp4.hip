@@ -10,10 +10,11 @@
 // into the tensor's section of the amax record: plain stores, no atomics (thousands of agent-scope atomics
 // on one address serialise at ~8 ns each on this multi-XCD part) and nothing to clear.
 // Lists of tensors that fit the chip's registers a few at a time run in one pass instead (nvfp4_one_pass_kernel).
-// Pass 2 (mq_nvfp4_quant): every workgroup turns the partial maxima into the amax, S_enc/6 and 1/S_enc while its loads are
-// under way, and each tensor's first one publishes the global scale; two lanes own one 16-element block (16 bytes each), the
-// block amax is one DPP step, and each lane emits four bytes of codes.  A gate/up pair writes two sections of one record.
-// (A launch of its own for the fold took 4.2 us: four [1077, 64] tensors 12.8 -> 8.1 us for the two passes.)
+// Pass 2 (mq_nvfp4_quant): the partial maxima become the amax, S_enc/6 and 1/S_enc, and each tensor's global scale is
+// published: in short passes by every workgroup while its loads are under way (a launch of its own for the fold took 4.2 us:
+// four [1077, 64] tensors 12.8 -> 8.1 us for the two passes), in long ones by a launch in front (nv_published).  Two lanes own
+// one 16-element block (16 bytes each), the block amax is one DPP step, and each lane emits four bytes of codes.  A gate/up
+// pair writes two sections of one record.
 #include <type_traits>
 
 #include "mq_api_internal.hpp"
@@ -186,7 +187,7 @@ __device__ __forceinline__ NvAmaxScales nv_record_scales(const FlatJob& job) {
     return NvAmaxScales{u2f(rec[kRecAmax]), NvScales{u2f(rec[kRecEncSixth]), u2f(rec[kRecSDec]), u2f(rec[kRecEnc])}};
 }
 // The same from the partial maxima of an amax pass, folded by every workgroup of the pass behind it while its data is under
-// way: a launch between the two passes that did it took 4.2 us, and the host's part of one.  Only the first wavefront folds
+// way: a launch between the two passes that did it took 4.2 us, and the host's part of one (long passes: nv_published).  Only the first wavefront folds
 // and divides (four words a lane and section), the others wait for its four values in LDS: Four Over Six is bound by vector
 // instructions, and some sixty of them in every wavefront cost it a tenth (fifty [616, 1584] tensors 24.5 us with the scales
 // read from a record, 30.0 folded by all four wavefronts, 27.3 by one).  Scalar registers hold the result, where values read
@@ -268,6 +269,18 @@ __global__ __launch_bounds__(256) void nvfp4_fold_kernel(const Table tab, float 
                 if (tab.job[ji - k].aux2) *(float*)tab.job[ji - k].aux2 = published;
         }
     }
+}
+
+// Publish kernel, one wavefront per tensor, grid (1, tensors): what every workgroup of a plain run's quantize pass does by
+// itself where the pass is short (nv_shared_scales) is done once here, and the pass reads the record.
+template <class Table>
+__global__ __launch_bounds__(kWave) void nvfp4_publish_kernel(const Table tab, float numer, uint32_t* moved_counter, uint32_t* moved_mirror) {
+    const FlatJob job = flat_job(tab);
+    if (blockIdx.y == 0) amax_feedback_folded(moved_counter, moved_mirror, gridDim.y);
+    const float amax = u2f(nv_wave_fold((const uint32_t*)job.aux, job.pad, (int)threadIdx.x));
+    if (threadIdx.x != 0) return;
+    ((uint32_t*)job.aux)[kRecRedo] = 0;
+    nv_publish_plain(job, amax, nv_scales(amax, numer), numer, moved_counter);
 }
 
 // ---- Four Over Six block scaling (miles/kernels/quant/nvfp4_qdq.py:893-990) --------------------------------
@@ -680,6 +693,7 @@ __device__ __forceinline__ uint32_t nvfp4_amax_units(const FlatJob& job, const i
 // PASS 2, a small grid striding over the blocks, quantizes again only the tensors whose amax did change.
 // PASS 0 is the second pass of the plain two-pass form (amax kernel, then this): every workgroup folds the partial maxima,
 // and the first one of each tensor publishes what comes of them, also for a tensor without elements.
+// PASS 3 is the same behind nvfp4_publish_kernel.
 template <int FOS, int PASS, class Table, int F16>
 __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Table tab, float denom, uint32_t* moved_counter, uint32_t* moved_mirror) {
     const FlatJob job = flat_job(tab);       // a copy in registers: a descriptor in device memory must not be re-read after the stores
@@ -710,6 +724,10 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
         return;
     }
     if (base >= job.units) return;
+    if (PASS == 3) {
+        nvfp4_quant_units<FOS, F16>(job, base, t, denom, [&] { return nv_record_scales(job); });
+        return;
+    }
     uint32_t seen;
     if (PASS == 1 && ((const uint32_t*)job.aux)[kRecVolatile] != 0) {
         seen = 0;
@@ -981,14 +999,15 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_one_pass_finish_kernel(const
 constexpr int kNvF32Loads = 2;                     // 16-byte loads per lane, standard blocks
 // 8-element units a workgroup covers
 constexpr int64_t nv_f32_units_per_block(int fos) { return fos ? kNvThreads * 2 : kNvThreads * kNvF32Loads / 2; }
-template <int FOS, class Table>
+template <int FOS, int PASS, class Table>
 __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_f32_kernel(const Table tab, float denom, uint32_t* moved_counter, uint32_t* moved_mirror) {
     const FlatJob job = flat_job(tab);
     const uint32_t t = threadIdx.x;
     const int64_t first = flat_block(tab) * nv_f32_units_per_block(FOS);       // in 8-element units
-    if (first >= job.units && first > 0) return;
-    if (first == 0 && blockIdx.y == 0) amax_feedback_folded(moved_counter, moved_mirror, gridDim.y);
-    auto fold = [&] {           // as in PASS 0 of the 16-bit kernel
+    if (first >= job.units && (PASS == 3 || first > 0)) return;
+    if (PASS == 0 && first == 0 && blockIdx.y == 0) amax_feedback_folded(moved_counter, moved_mirror, gridDim.y);
+    auto fold = [&] {           // as in PASS 0 and PASS 3 of the 16-bit kernel
+        if (PASS == 3) return nv_record_scales(job);
         const NvAmaxScales a = nv_shared_scales((int)t, denom, [&] { return nv_wave_fold((const uint32_t*)job.aux, job.pad, (int)t); });
         if (first == 0 && t == 0) {
             ((uint32_t*)job.aux)[kRecRedo] = 0;
@@ -1275,20 +1294,20 @@ static void launch_nvfp4_quant_dtype(const Table& tab, int flags, float numer, b
         }
     }
 }
-template <class Table>
+template <int PASS, class Table>
 static void launch_nvfp4_quant_f32(const Table& tab, int flags, float numer, bool counted, dim3 grid, hipStream_t st) {
     const dim3 blk(kNvThreads);
     uint32_t *const moved = counted ? mq_amax_feedback() : nullptr, *const mirror = mq_amax_feedback_mirror();
     const int fos = (flags & MQ_NVFP4_4OVER6) ? 1 + nv_error_mode(flags) : 0;
     if constexpr (std::is_same<Table, FlatRef>::value) {
-        hipLaunchKernelGGL((nvfp4_quant_f32_kernel<0, Table>), grid, blk, 0, st, tab, numer, moved, mirror);
+        hipLaunchKernelGGL((nvfp4_quant_f32_kernel<0, PASS, Table>), grid, blk, 0, st, tab, numer, moved, mirror);
     } else {
         switch (fos) {
-            case 0: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<0, Table>), grid, blk, 0, st, tab, numer, moved, mirror); break;
-            case 1: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<1, Table>), grid, blk, 0, st, tab, numer, moved, mirror); break;
-            case 2: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<2, Table>), grid, blk, 0, st, tab, numer, moved, mirror); break;
-            case 3: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<3, Table>), grid, blk, 0, st, tab, numer, moved, mirror); break;
-            default: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<4, Table>), grid, blk, 0, st, tab, numer, moved, mirror); break;
+            case 0: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<0, PASS, Table>), grid, blk, 0, st, tab, numer, moved, mirror); break;
+            case 1: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<1, PASS, Table>), grid, blk, 0, st, tab, numer, moved, mirror); break;
+            case 2: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<2, PASS, Table>), grid, blk, 0, st, tab, numer, moved, mirror); break;
+            case 3: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<3, PASS, Table>), grid, blk, 0, st, tab, numer, moved, mirror); break;
+            default: hipLaunchKernelGGL((nvfp4_quant_f32_kernel<4, PASS, Table>), grid, blk, 0, st, tab, numer, moved, mirror); break;
         }
     }
 }
@@ -1296,14 +1315,40 @@ static void launch_nvfp4_quant_f32(const Table& tab, int flags, float numer, boo
 template <int PASS, class Table>
 static void launch_nvfp4_quant(int dtype, const Table& tab, int flags, float numer, bool counted, dim3 grid, hipStream_t st) {
     // (fp32 has no instances of passes 1 and 2: nvfp4_quant_launch refuses mode 2 for it)
-    if (PASS == 0 && dtype == MQ_F32) launch_nvfp4_quant_f32(tab, flags, numer, counted, grid, st);
-    else if (dtype == MQ_F16) launch_nvfp4_quant_dtype<PASS, Table, 1>(tab, flags, numer, counted, grid, st);
+    if constexpr (PASS == 0 || PASS == 3) {
+        if (dtype == MQ_F32) {
+            launch_nvfp4_quant_f32<PASS>(tab, flags, numer, counted, grid, st);
+            return;
+        }
+    }
+    if (dtype == MQ_F16) launch_nvfp4_quant_dtype<PASS, Table, 1>(tab, flags, numer, counted, grid, st);
     else launch_nvfp4_quant_dtype<PASS, Table, 0>(tab, flags, numer, counted, grid, st);
 }
 
+// Whether a plain run's amax is folded by a launch between the two passes (nvfp4_publish_kernel), or by every workgroup of the
+// second one.  The launch takes 1 to 2 us; what it saves grows with the pass and with the sections of a record.  `sections`:
+// of all n tensors' records, `bytes`: of their elements.  Device time of both passes in us, folded in the pass / by the launch:
+//   gate and up in pairs, bf16: 2 x [2048, 7168] (59 MB) 25.1 / 25.6, 4 of them 44.3 / 43.7, 16 of them 168 / 158, 64 of them
+//     (1.9 GB) 646 / 615; fp32: 34 MB 16.6 / 17.3, 67 MB 26.8 / 27.0, 117 MB 42.1 / 41.2, 470 MB 156 / 148, 940 MB 314 / 293.
+//     (A pair folds two sections, a quarter of the bytes that a workgroup quantizes.)
+//   Four Over Six of 16-bit tensors, bound by vector instructions: 34 MB 19.7 / 20.9, 51 MB 25.7 / 26.0, 67 MB 34.5 / 34.1,
+//     134 MB 53.6 / 52.3, 268 MB 102.6 / 99.1, 470 MB 181 / 170, 1.9 GB 705 / 654.
+//   Four Over Six of fp32 tensors, as long as the second pass finds all of its input in the memory-side cache: 78 MB 34.1 / 34.8
+//     (in pairs 35.8 / 35.3), 117 MB 46.3 / 46.2 (47.6 / 46.3), 235 MB 85.4 / 83.9 (86.8 / 84.0), 268 MB 112 / 111; but 403 MB
+//     143.0 / 143.1, 470 MB 169 / 173 (170 / 173), 604 MB 207 / 211.
+//   one section per record, standard scaling: fp32 67 MB 25.5 / 27.1, 470 MB 147 / 148, 2.1 GB 667 / 663; bf16 tensors too large
+//     to be read once, [5120, 8192] 36.1 / 37.3, two [8192, 8192] 92.8 / 92.3, eight 355 / 359: folded in the pass.
+constexpr int64_t kPublishMinBytes = 64ll << 20;
+static bool nv_published(int dtype, bool four_over_six, int64_t sections, int64_t n, int64_t bytes) {
+    if (bytes < kPublishMinBytes) return false;
+    const bool paired = sections * 2 >= n * 3;       // half of the tensors at least
+    if (!four_over_six) return paired;
+    return dtype != MQ_F32 || (kept_quarters(bytes) == 4 && (paired || bytes >= 2 * kPublishMinBytes));
+}
 // quantize (carried run: and fold, and second pass) over a table whose grid is known: tab.chunk / tab.max_blocks are set
+// (all_units: of all n tensors; sections: of their records)
 template <class Table>
-static int nvfp4_quant_launch(int dtype, const Table& tab, int n, int e4m3_max, int flags, int mode, hipStream_t st) {
+static int nvfp4_quant_launch(int dtype, const Table& tab, int n, int64_t all_units, int64_t sections, int e4m3_max, int flags, int mode, hipStream_t st) {
     if (mode == 2 && dtype == MQ_F32) return mq_fail(MQ_ERR_ARG, "a carried-over amax is for bf16 and fp16 tensors");
     const float numer = (float)e4m3_max * 6.0f;
     const dim3 folds((unsigned)n), blk(256);
@@ -1316,6 +1361,12 @@ static int nvfp4_quant_launch(int dtype, const Table& tab, int n, int e4m3_max, 
             launch_nvfp4_quant<2>(dtype, tab, flags, numer, false, dim3(redo_blocks, (unsigned)n), st);
         }
         return mq_check_launch("nvfp4 quant (carried-over amax)");
+    }
+    if (nv_published(dtype, (flags & MQ_NVFP4_4OVER6) != 0, sections, n, all_units * (dtype == MQ_F32 ? 32 : 16))) {
+        hipLaunchKernelGGL((nvfp4_publish_kernel<Table>), dim3(1, (unsigned)n), dim3(kWave), 0, st, tab, numer,
+                           mode == 1 ? mq_amax_feedback() : nullptr, mq_amax_feedback_mirror());
+        launch_nvfp4_quant<3>(dtype, tab, flags, numer, false, grid, st);
+        return mq_check_launch("nvfp4 quant");
     }
     // (a list of empty tensors still has its scales published, by the first workgroup of each)
     launch_nvfp4_quant<0>(dtype, tab, flags, numer, mode == 1, dim3(grid.x > 0 ? grid.x : 1u, grid.y), st);
@@ -1331,15 +1382,21 @@ static int nvfp4_quant_launch(int dtype, const Table& tab, int n, int e4m3_max, 
 int mq_nvfp4_quant_launch_group(int dtype, FlatTable& tab, int e4m3_max, int flags, int mode, hipStream_t st) {
     const int fos = flags & MQ_NVFP4_4OVER6;
     if (!flat_grid(tab, dtype == MQ_F32 ? nv_f32_units_per_block(fos) : nv_units_per_block(fos))) return mq_fail(MQ_ERR_ARG, "tensor too large");
-    return nvfp4_quant_launch(dtype, tab, tab.n, e4m3_max, flags, mode, st);
+    int64_t all_units = 0, sections = 0;
+    for (int i = 0; i < tab.n; i++) {
+        all_units += tab.job[i].units;
+        sections += tab.job[i].pad;
+    }
+    return nvfp4_quant_launch(dtype, tab, tab.n, all_units, sections, e4m3_max, flags, mode, st);
 }
-// modes 1 and 2 over n descriptors of a device table (standard block scaling only); max_units: the largest tensor's units
-int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int e4m3_max, int mode,
-                                hipStream_t st) {
+// modes 1 and 2 over n descriptors of a device table (standard block scaling only); max_units: the largest tensor's units,
+// sections: of all tensors' records
+int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int64_t sections, int e4m3_max,
+                                int mode, hipStream_t st) {
     FlatRef ref{device_jobs, 0, 0};
     if (!flat_grid(ref, max_units, dtype == MQ_F32 ? nv_f32_units_per_block(0) : kNvThreads * kNvUnroll)) return mq_fail(MQ_ERR_ARG, "tensor too large");
     if (n == 0) return MQ_OK;
-    return nvfp4_quant_launch(dtype, ref, n, e4m3_max, 0, mode, st);
+    return nvfp4_quant_launch(dtype, ref, n, max_units * n, sections, e4m3_max, 0, mode, st);
 }
 
 // Whether a chunk of NVFP4 jobs (standard scaling, packed kernels, no carried amax) takes the one-pass form.  `slots` is the

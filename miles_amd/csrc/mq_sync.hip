@@ -51,8 +51,8 @@ int mq_fp8_channel_launch_group(int dtype, int form, const MqScaledArgs* a, int 
 int mq_fp8_scaled_form(const void* w, int dtype, int64_t ldw, const void* q, int64_t M, int64_t K);
 int mq_fp8_scaled_launch_group(int dtype, int form, const MqScaledArgs* a, int n, int words, hipStream_t st);
 int mq_nvfp4_amax_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, hipStream_t st);
-int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int e4m3_max, int mode,
-                                hipStream_t st);
+int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int64_t sections, int e4m3_max,
+                                int mode, hipStream_t st);
 int mq_mxfp8_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, hipStream_t st);
 int mq_mxfp4_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, hipStream_t st);
 int mq_int4_pack_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int group, hipStream_t st);
@@ -506,13 +506,14 @@ static int run_nvfp4(const mq_job* jobs, int64_t n_all, int64_t i, int64_t j, co
             bool carry = jobs[i].dtype != MQ_F32;
             for (int t = 0; t < n; t++) carry &= (jobs[i + t].p1 & MQ_NVFP4_CARRY_AMAX) != 0;
             int rc = MQ_OK;
-            int64_t max_units = 0, sum_units = 0, slots = 0, max_slots = 0;
+            int64_t max_units = 0, sum_units = 0, slots = 0, max_slots = 0, all_sections = 0;
             bool empty = false;
             for (int t = 0; t < n; t++) {
                 const int64_t u = jobs[i + t].rows * jobs[i + t].cols / 8;
                 empty |= u == 0;
                 max_units = u > max_units ? u : max_units;
                 sum_units += u;
+                all_sections += sections[t];
                 slots = (section[t] == 0 ? 0 : slots) + mq_nvfp4_one_pass_slots(u);
                 max_slots = slots > max_slots ? slots : max_slots;
             }
@@ -526,7 +527,7 @@ static int run_nvfp4(const mq_job* jobs, int64_t n_all, int64_t i, int64_t j, co
                 }
                 if (!carry) rc = mq_nvfp4_amax_launch_table(jobs[i].dtype, table + i, n, max_units, st);
                 if (rc) return rc;
-                rc = mq_nvfp4_quant_launch_table(jobs[i].dtype, table + i, n, max_units, jobs[i].p0, carry ? 2 : 1, st);
+                rc = mq_nvfp4_quant_launch_table(jobs[i].dtype, table + i, n, max_units, all_sections, jobs[i].p0, carry ? 2 : 1, st);
                 if (rc) return rc;
                 i = k;
                 continue;
