@@ -295,7 +295,10 @@ __global__ __launch_bounds__(kTileThreads) void fp8_block128_any_kernel(const Ti
     uint32_t m = 0;
 #pragma unroll
     for (int i = 0; i < kRows; i++) {
-        const u32x4 x = v[i];
+        u32x4 x = v[i];
+        // (a copy: the magnitudes of all 32 elements would otherwise be kept for MODE 1's second look at them, 82 registers
+        // instead of 50 and two workgroups per compute unit instead of four: 24 [200000, 32] tensors 272 us instead of 169)
+        if (MODE == 1 && DT == MQ_F32) asm("" : "+v"(x));
         if (DT == MQ_F32)
             m = umax(umax(umax(m, x.x & 0x7FFFFFFFu), umax(x.y & 0x7FFFFFFFu, x.z & 0x7FFFFFFFu)), x.w & 0x7FFFFFFFu);
         else
@@ -896,12 +899,15 @@ static void tile_launch(int mode, bool f16, dim3 grid, hipStream_t st, const Tab
     }
 }
 
+// Dynamic LDS that leaves a compute unit (160 KB) two workgroups.  Their registers are enough for four, which fill the memory
+// system best unless a launch reads more lines at a time than it keeps open; see mq_fp8_tile_launch_group.
+constexpr unsigned kTwoPerCu = 56u << 10;
 template <int DT, bool LINES>
-static void tile_any_launch(int mode, dim3 grid, hipStream_t st, const TileTable& tab) {
+static void tile_any_launch(int mode, dim3 grid, unsigned lds, hipStream_t st, const TileTable& tab) {
     const dim3 blk(kTileThreads);
-    if (mode == 0) hipLaunchKernelGGL((fp8_block128_any_kernel<0, DT, LINES>), grid, blk, 0, st, tab);
-    else if (mode == 1) hipLaunchKernelGGL((fp8_block128_any_kernel<1, DT, LINES>), grid, blk, 0, st, tab);
-    else hipLaunchKernelGGL((fp8_block128_any_kernel<2, DT, LINES>), grid, blk, 0, st, tab);
+    if (mode == 0) hipLaunchKernelGGL((fp8_block128_any_kernel<0, DT, LINES>), grid, blk, lds, st, tab);
+    else if (mode == 1) hipLaunchKernelGGL((fp8_block128_any_kernel<1, DT, LINES>), grid, blk, lds, st, tab);
+    else hipLaunchKernelGGL((fp8_block128_any_kernel<2, DT, LINES>), grid, blk, lds, st, tab);
 }
 
 // n finished descriptors in device memory, all of one 16-bit dtype; max_tiles: the largest tensor's tile count
@@ -929,18 +935,29 @@ int mq_fp8_tile_launch_group(int mode, int dtype, bool aligned, TileTable& tab, 
         return mq_check_launch("fp8 block quant");
     }
     bool lines = dtype == MQ_F32;      // whole 128-byte lines per tile row (every segment inside its row as well: K % 8 == 0)
-    for (int i = 0; i < tab.n; i++)
+    int64_t narrowest = INT64_MAX;
+    for (int i = 0; i < tab.n; i++) {
         lines &= ((uintptr_t)tab.job[i].w % 128) == 0 && tab.job[i].ldw % 32 == 0 && tab.job[i].K % 8 == 0;
+        narrowest = tab.job[i].K < narrowest ? tab.job[i].K : narrowest;
+    }
     // Neighbouring tiles of unaligned rows share lines, so the longer an XCD's runs of tiles are the better, as long as
     // every XCD has several: 24 [4097, 4099] bf16 tensors 4.48 / 4.73 / 4.77 / 4.93 TB/s with runs of 8 / 16 / 32 / 64.
     while (tab.chunk_shift < 6 && (tiles >> (tab.chunk_shift + 1)) >= 64) tab.chunk_shift++;
     const int64_t gx = xcd_grid_chunked(tiles, 1ll << tab.chunk_shift);
     if (gx >= 0x7FFFFFF0) return mq_fail(MQ_ERR_ARG, "too many tiles");
     const dim3 grid((unsigned)gx);
-    if (dtype == MQ_BF16) tile_any_launch<MQ_BF16, false>(mode, grid, st, tab);
-    else if (dtype == MQ_F16) tile_any_launch<MQ_F16, false>(mode, grid, st, tab);
-    else if (lines) tile_any_launch<MQ_F32, true>(mode, grid, st, tab);
-    else tile_any_launch<MQ_F32, false>(mode, grid, st, tab);
+    // The blockwise cast of long fp32 lists takes two workgroups per compute unit instead of four (us, four / two).
+    // Unaligned rows, from 4096 tiles of 64 KB and 512 columns on: [4095, 8191] one 34.7 / 35.9, two 71 / 66, eight 286 / 240;
+    // [4097, 2051] four 36.1 / 37.2, eight 69 / 66, 32 of them 268 / 240; [8193, 515] 8 of them 37.8 / 38.4, 16 72.9 / 71.2, 64
+    // 267 / 249; but [16385, 259] 16 of them 73 / 75, [32769, 131] 31 of them 151 / 162, [65537, 67] 31 of them 118 / 139.
+    // Aligned rows, from 16384 tiles and 32768 columns on: [1024, 32768] two 61 / 63, four 120 / 119, eight 242 / 229,
+    // [8192, 32768] 240 / 229; but [4096, 8192] eight 220 / 225, [16384, 128] 64 of them 116 / 119.
+    const bool long_list = lines ? tiles >= 16384 && narrowest >= 32768 : tiles >= 4096 && narrowest >= 512;
+    const unsigned lds = mode == 1 && dtype == MQ_F32 && long_list ? kTwoPerCu : 0u;
+    if (dtype == MQ_BF16) tile_any_launch<MQ_BF16, false>(mode, grid, lds, st, tab);
+    else if (dtype == MQ_F16) tile_any_launch<MQ_F16, false>(mode, grid, lds, st, tab);
+    else if (lines) tile_any_launch<MQ_F32, true>(mode, grid, lds, st, tab);
+    else tile_any_launch<MQ_F32, false>(mode, grid, lds, st, tab);
     return mq_check_launch("fp8 block quant");
 }
 

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from miles_amd import launch
+from miles_amd.kernels.quant.fp8_blockwise import fp8_blockwise_cast
 from tests.test_gpu_any_alignment_kernels import _matrix, _one_nan, _quantizers
 from tests.test_gpu_fp32_kernels import DEV, _assert_same, oracle  # noqa: F401
 
@@ -28,3 +29,25 @@ def test_fp32_tile_widths(oracle, specials, offset):  # noqa: F811
             q_o, s_o = ref(host)
             _assert_same(s, s_o, f"{name} scales {tuple(host.shape)}")
             _assert_same(_one_nan(q), _one_nan(q_o), f"{name} codes {tuple(host.shape)}")
+
+
+# (tiles, columns): around the lists from which on the cast takes two workgroups per compute unit, unaligned rows and whole lines
+@pytest.mark.parametrize("rows, cols, tensors", [(4095, 8191, 2), (3968, 8191, 2), (65536, 515, 2), (65536, 509, 2), (8192, 32768, 1), (8064, 32768, 1)])
+def test_long_lists_are_their_bands(rows, cols, tensors):
+    """Each tile is by itself: a long list gives what its bands of 1024 rows give in calls of their own, infinities and NaN
+    in some tiles included."""
+    weights = []
+    for i in range(tensors):
+        g = torch.Generator(device=DEV).manual_seed(i)
+        w = torch.randn(rows, cols, generator=g, device=DEV)
+        w[5 + 128 * i, 7] = float("inf")
+        w[rows - 1, cols - 1] = float("nan")
+        w[640:768, 128:256] = 0.0
+        weights.append(w)
+    with launch.deferred():
+        whole = [fp8_blockwise_cast(w) for w in weights]
+    for w, (q, s) in zip(weights, whole):
+        for r in range(0, rows, 1024):
+            q1, s1 = fp8_blockwise_cast(w[r:r + 1024])
+            assert torch.equal(q[r:r + 1024].view(torch.uint8), q1.view(torch.uint8)), f"codes from row {r}"
+            assert torch.equal(s[r // 128:r // 128 + 8].view(torch.int32), s1.view(torch.int32)), f"scales from row {r}"
