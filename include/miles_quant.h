@@ -370,10 +370,10 @@ int mq_job_table_fill(const mq_job* jobs, int64_t n, void* host_table);
 int mq_run_jobs_tabled(const mq_job* jobs, int64_t n, const void* device_table, void* stream);
 
 /* mq_run_jobs_tabled that also reports how many amax records moved (no counterpart in the reference).  device_moved
- * points to two uint32 in device memory, counters that the call never clears: every fold of NVFP4 or per-tensor FP8 amax
- * records made by the call adds the number of tensors it folded to word 1, and to word 0 the number of those whose
+ * points to two uint32 in device memory, counters that the call never clears: every launch of the call that finishes
+ * NVFP4 or per-tensor FP8 amax records adds the number of their tensors to word 1, and to word 0 the number of those whose
  * record held another amax before.  host_mirror (may be NULL) points to two uint32 of pinned host memory (hipHostMalloc;
- * anything else is refused): every fold launch first refreshes them with the counters as the launches before it left
+ * anything else is refused): every such launch first refreshes them with the counters as the launches before it left
  * them, so that the host can read them at any time without a copy, an event or a wait.  The mirror must stay allocated
  * until every submitted call that named it has finished on the GPU: the kernels store through its address.
  * When most tensors keep moving from one submission to the next -- where MQ_NVFP4_CARRY_AMAX costs a second pass over

@@ -7,9 +7,9 @@
 
 int mq_fail(int code, const char* msg);
 int mq_check_launch(const char* what);
-// Device counters that the amax fold kernels of the running mq_run_jobs_feedback call add to, and the device-visible
-// address of the host mirror they refresh (both null outside such a call): set on entry, cleared on return, per host
-// thread.
+// Device counters that the kernels which finish amax records add to in the running mq_run_jobs_feedback call, and the
+// device-visible address of the host mirror they refresh (both null outside such a call): set on entry, cleared on return,
+// per host thread.
 uint32_t* mq_amax_feedback();
 uint32_t* mq_amax_feedback_mirror();
 void mq_set_amax_feedback(uint32_t* device_counter, uint32_t* mirror);

@@ -242,13 +242,14 @@ __device__ __forceinline__ void amax_record_after_carried_run(uint32_t* rec, boo
     rec[kRecMovedRuns] = runs;
     rec[kRecVolatile] = runs >= 2u ? 1u : 0u;
 }
-// A fold launched by the job driver also tells its caller how many tensors' records held another amax before, and how
-// many tensors it folded (two counters in device memory that only ever grow: a copy taken at any time gives a
-// consistent rate): a caller whose every amax keeps moving can then submit the plain two-pass form.
+// The launch of the job driver that finishes a list's records -- a fold, nvfp4_publish_kernel, or the quantize pass of a plain
+// run itself -- also tells its caller how many tensors' records held another amax before, and how many tensors it finished
+// (two counters in device memory that only ever grow: a copy taken at any time gives a consistent rate): a caller whose every
+// amax keeps moving can then submit the plain two-pass form.
 __device__ __forceinline__ void amax_feedback(uint32_t* counter, bool moved, uint32_t tensors) {
     if (counter && moved) atomicAdd(counter, tensors);
 }
-// Once per fold launch: first the two counters as the launches before left them (a consistent pair) go to the caller's
+// Once per such launch: first the two counters as the launches before left them (a consistent pair) go to the caller's
 // host-visible mirror, if the call named one (a kernel argument: the host checked that it is pinned memory), then this
 // launch's tensors are added to the second counter.
 __device__ __forceinline__ void amax_feedback_folded(uint32_t* counter, uint32_t* mirror_words, uint32_t tensors) {

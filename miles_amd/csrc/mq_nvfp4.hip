@@ -1164,7 +1164,7 @@ __global__ __launch_bounds__(256) void nvfp4_quant_generic_kernel(const void* __
 // Reference: miles/kernels/quant/nvfp4_qdq.py:877-890 (standard quantize), :993-1029 (dequantize), kernel :1067-1105.
 // Given the tensor amax: codes and block scale exactly as the quantizer above, then
 //   final = RN(RN(f32(s8) * amax) * f32(1 / (6 * e4m3_max)));  y = dtype(RN(e2m1_value * final))
-// Nothing but x (and the amax, see nv_fake_amax) is read and nothing but y written.  job: w = x, q = y, units.
+// Nothing but x (and the amax, see nv_fake_scales) is read and nothing but y written.  job: w = x, q = y, units.
 // Standard blocks: two lanes own one 1x16 block.  Four Over Six: nvfp4_fos_units.
 // Both are bound by memory, the reads by the memory-side cache where the amax pass left its input there: sixteen [1536, 2048]
 // weights in one launch 28.4 us (33 from HBM; one launch per weight 4.6 us each), four [4096, 7168] with Four Over Six 67 us
@@ -1514,7 +1514,7 @@ static void nvfp4_fake_launch_dtype(const FlatTable& tab, int fos, float numer, 
         default: hipLaunchKernelGGL((nvfp4_fake_kernel<4, F16>), grid, blk, 0, st, tab, numer, inv_numer); break;
     }
 }
-// tab.job[i]: w = x, q = y, units, and the amax (see nv_fake_amax)
+// tab.job[i]: w = x, q = y, units, and the amax (see nv_fake_scales)
 static int nvfp4_fake_launch(int dtype, FlatTable& tab, int e4m3_max, int flags, hipStream_t st) {
     if (!flat_grid(tab, nv_units_per_block(flags & MQ_NVFP4_4OVER6))) return mq_fail(MQ_ERR_ARG, "tensor too large");
     const float numer = (float)e4m3_max * 6.0f, inv_numer = (float)(1.0 / (double)(6 * e4m3_max));

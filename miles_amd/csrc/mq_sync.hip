@@ -77,9 +77,11 @@ int mq_copy_launch_group(CopyTable& tab, hipStream_t st);
 int mq_copy_launch_table(const CopyTableEntry* device_jobs, int n, int64_t max_chunks, hipStream_t st);
 int mq_copy_launch_run(const void* src, void* dst, int64_t bytes, hipStream_t st);
 
-// Upper bound on the input bytes of one NVFP4 group (amax launch + fold + quantize launch).  Measured on
-// MI355X the second read of a tensor gains nothing from the memory-side cache at any group size, so groups
-// are as large as the 64-tensor table allows: fewer launch boundaries.
+// Upper bound on the input bytes of one NVFP4 group (its amax launch, a publishing launch where nv_published says so, its
+// quantize launch): none but the table's.  The second read of a group that fits the memory-side cache comes from there
+// (kept_quarters), but cutting a long list into such groups costs more in launch boundaries than that: in groups of any
+// size / 400 MB / 200 MB, bf16 pairs of 470 MB 155 / 162 / 171 us, of 1.9 GB 617 / 645 / 688, Four Over Six of 940 MB
+// 327 / 342 / 369, fp32 of 1.9 GB 584 / 592 / 617.
 #ifndef MQ_NV_GROUP_MB
 #define MQ_NV_GROUP_MB (1 << 20)
 #endif
@@ -603,7 +605,7 @@ extern "C" int mq_run_jobs_feedback(const mq_job* jobs, int64_t n, const void* d
     if (host_mirror && !device_moved) return mq_fail(MQ_ERR_ARG, "a feedback mirror needs the device counters it mirrors");
     uint32_t* mirror = nullptr;
     if (host_mirror) {
-        // the fold kernels store through this address: it has to be host memory the GPU can write (pinned, mapped)
+        // the kernels that finish the records store through this address: it has to be host memory the GPU can write (pinned, mapped)
         hipPointerAttribute_t attr;
         if (hipPointerGetAttributes(&attr, host_mirror) != hipSuccess || attr.type != hipMemoryTypeHost || !attr.devicePointer) {
             (void)hipGetLastError();

@@ -25,13 +25,14 @@ _state = threading.local()
 class _AmaxFeedback:
     """What share of the amax records moved in the syncs the GPU has finished, read without ever waiting for it.
 
-    The folds of a `mq_run_jobs_feedback` call add to two device counters that only grow -- tensors whose record held
-    another amax before, and tensors folded -- and every fold launch first mirrors the pair into two pinned words (their
-    address travels with every call, as a host argument), so the host reads them with no copy, no event and no wait.  At the start of a submission: when more than half of the tensors
-    folded since the last reading had moved, the list is submitted in the plain two-pass form (the carried-over amax
-    would cost every such tensor a second pass), until they hold again."""
+    The launches of a `mq_run_jobs_feedback` call that finish amax records (a fold, the publishing launch, or the quantize
+    pass itself) add to two device counters that only grow -- tensors whose record held another amax before, and tensors
+    finished -- and each first mirrors the pair into two pinned words (their address travels with every call, as a host
+    argument), so the host reads them with no copy, no event and no wait.  At the start of a submission: when more than
+    half of the tensors finished since the last reading had moved, the list is submitted in the plain two-pass form (the
+    carried-over amax would cost every such tensor a second pass), until they hold again."""
 
-    # The GPU writes the mirror words whenever a fold runs, possibly after the batch that named them is gone: they come
+    # The GPU writes the mirror words whenever records are finished, possibly after the batch that named them is gone: they come
     # from one pinned block that lives as long as the process and is never handed back to torch's host allocator.  A
     # slot re-used while an old sync still runs can at worst mislead one choice between two forms with equal results.
     _POOL_SLOTS = 1024
