@@ -899,9 +899,9 @@ static void tile_launch(int mode, bool f16, dim3 grid, hipStream_t st, const Tab
     }
 }
 
-// Dynamic LDS that leaves a compute unit (160 KB) two workgroups.  Their registers are enough for four, which fill the memory
-// system best unless a launch reads more lines at a time than it keeps open; see mq_fp8_tile_launch_group.
-constexpr unsigned kTwoPerCu = 56u << 10;
+// Dynamic LDS that leaves a compute unit (160 KB) two workgroups, or three.  Their registers are enough for four, which fill
+// the memory system best unless a launch reads more lines at a time than it keeps open; see mq_fp8_tile_launch_group.
+constexpr unsigned kTwoPerCu = 56u << 10, kThreePerCu = 44u << 10;
 template <int DT, bool LINES>
 static void tile_any_launch(int mode, dim3 grid, unsigned lds, hipStream_t st, const TileTable& tab) {
     const dim3 blk(kTileThreads);
@@ -935,10 +935,14 @@ int mq_fp8_tile_launch_group(int mode, int dtype, bool aligned, TileTable& tab, 
         return mq_check_launch("fp8 block quant");
     }
     bool lines = dtype == MQ_F32;      // whole 128-byte lines per tile row (every segment inside its row as well: K % 8 == 0)
-    int64_t narrowest = INT64_MAX;
+    int64_t elems = 0, narrowest = INT64_MAX;
+    bool slim = false;                 // few columns, the last few of them with tiles of their own
     for (int i = 0; i < tab.n; i++) {
-        lines &= ((uintptr_t)tab.job[i].w % 128) == 0 && tab.job[i].ldw % 32 == 0 && tab.job[i].K % 8 == 0;
-        narrowest = tab.job[i].K < narrowest ? tab.job[i].K : narrowest;
+        const TileJob& j = tab.job[i];
+        lines &= ((uintptr_t)j.w % 128) == 0 && j.ldw % 32 == 0 && j.K % 8 == 0;
+        elems += (int64_t)j.M * j.K;
+        narrowest = j.K < narrowest ? j.K : narrowest;
+        slim |= j.K < 4 * kTile && (j.K - 1) % kTile < 32;
     }
     // Neighbouring tiles of unaligned rows share lines, so the longer an XCD's runs of tiles are the better, as long as
     // every XCD has several: 24 [4097, 4099] bf16 tensors 4.48 / 4.73 / 4.77 / 4.93 TB/s with runs of 8 / 16 / 32 / 64.
@@ -946,14 +950,24 @@ int mq_fp8_tile_launch_group(int mode, int dtype, bool aligned, TileTable& tab, 
     const int64_t gx = xcd_grid_chunked(tiles, 1ll << tab.chunk_shift);
     if (gx >= 0x7FFFFFF0) return mq_fail(MQ_ERR_ARG, "too many tiles");
     const dim3 grid((unsigned)gx);
-    // The blockwise cast of long fp32 lists takes two workgroups per compute unit instead of four (us, four / two).
-    // Unaligned rows, from 4096 tiles of 64 KB and 512 columns on: [4095, 8191] one 34.7 / 35.9, two 71 / 66, eight 286 / 240;
-    // [4097, 2051] four 36.1 / 37.2, eight 69 / 66, 32 of them 268 / 240; [8193, 515] 8 of them 37.8 / 38.4, 16 72.9 / 71.2, 64
-    // 267 / 249; but [16385, 259] 16 of them 73 / 75, [32769, 131] 31 of them 151 / 162, [65537, 67] 31 of them 118 / 139.
-    // Aligned rows, from 16384 tiles and 32768 columns on: [1024, 32768] two 61 / 63, four 120 / 119, eight 242 / 229,
-    // [8192, 32768] 240 / 229; but [4096, 8192] eight 220 / 225, [16384, 128] 64 of them 116 / 119.
-    const bool long_list = lines ? tiles >= 16384 && narrowest >= 32768 : tiles >= 4096 && narrowest >= 512;
-    const unsigned lds = mode == 1 && dtype == MQ_F32 && long_list ? kTwoPerCu : 0u;
+    // The blockwise cast of long fp32 lists takes two or three workgroups per compute unit instead of four, whose tiles outgrow
+    // an XCD's L2 before the neighbours have read the lines they share (us, four / three / two):
+    //   unaligned rows of more than a tile, from 160 MiB on two: [4095, 8191] two 71 / 68 / 66, eight 286 / 259 / 240; [4097, 2051]
+    //     eight 69 / 67 / 66, 32 of them 268 / 250 / 240; 268 MB of 195 columns 88 / 78 / 73, of 451 79 / 74 / 72, of 705 78 / 70 /
+    //     67, 184 MB of 195 columns 60.2 / 53.7 / 51.1, of 1031 48.7 / 47.7 / 46.6 (but 268 MB of 250 columns 68 / 66 / 69, of 509
+    //     66 / 65 / 68); three where they are slim: 268 MB of 129 columns 79 / 73 / 85, of 145 87 / 77 / 86, of 259 70 / 69 / 72;
+    //   from 96 MiB on three: 134 MB of 145 columns 45 / 41 / 45, of 195 44 / 40 / 40, of 257 37.5 / 37.0 / 37.9, of 1163 37.5 / 36.2 /
+    //     36.7, [4095, 8191] 34.7 / 34.2 / 35.9; up to two tiles wide from 48 MiB on: 67 MB of 145 columns 24.6 / 23.5 / 24.8, of 195
+    //     24.1 / 23.2 / 22.6, but of 270 21.0 / 21.7 / 21.8, of 771 21.2 / 21.8 / 21.8;
+    //   up to a tile wide always four: [65537, 67] 15 of them 59 / 60 / 69;
+    //   whole lines, from 16384 tiles and 32768 columns on, two: [1024, 32768] four 120 / 119 / 119, eight 242 / 242 / 229; but
+    //     [4096, 8192] eight 220 / 221 / 225, [16384, 128] 64 of them 116 / 118 / 119.
+    unsigned lds = 0;
+    if (mode == 1 && dtype == MQ_F32) {
+        const int64_t mib = (elems * 4) >> 20;
+        if (lines) lds = tiles >= 16384 && narrowest >= 32768 ? kTwoPerCu : 0u;
+        else if (narrowest > kTile) lds = mib >= 160 && !slim ? kTwoPerCu : mib >= (narrowest <= 2 * kTile ? 48 : 96) ? kThreePerCu : 0u;
+    }
     if (dtype == MQ_BF16) tile_any_launch<MQ_BF16, false>(mode, grid, lds, st, tab);
     else if (dtype == MQ_F16) tile_any_launch<MQ_F16, false>(mode, grid, lds, st, tab);
     else if (lines) tile_any_launch<MQ_F32, true>(mode, grid, lds, st, tab);

@@ -31,8 +31,10 @@ def test_fp32_tile_widths(oracle, specials, offset):  # noqa: F811
             _assert_same(_one_nan(q), _one_nan(q_o), f"{name} codes {tuple(host.shape)}")
 
 
-# (tiles, columns): around the lists from which on the cast takes two workgroups per compute unit, unaligned rows and whole lines
-@pytest.mark.parametrize("rows, cols, tensors", [(4095, 8191, 2), (3968, 8191, 2), (65536, 515, 2), (65536, 509, 2), (8192, 32768, 1), (8064, 32768, 1)])
+# around the lists from which on the cast takes two or three workgroups per compute unit, unaligned rows and whole lines
+@pytest.mark.parametrize("rows, cols, tensors", [
+    (4095, 8191, 2), (3200, 8191, 1), (3072, 8191, 1), (65536, 515, 2), (65536, 509, 2), (8192, 32768, 1), (8064, 32768, 1),
+    (32769, 131, 13), (32769, 131, 4), (32769, 131, 2), (16385, 195, 17), (65536, 129, 2), (262144, 125, 2)])
 def test_long_lists_are_their_bands(rows, cols, tensors):
     """Each tile is by itself: a long list gives what its bands of 1024 rows give in calls of their own, infinities and NaN
     in some tiles included."""
