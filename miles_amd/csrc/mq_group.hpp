@@ -144,8 +144,8 @@ constexpr int kTableGroup = 8192;         // tensors per launch of the device-ta
 // the descriptor of this workgroup's tensor, copied into registers (a descriptor in device memory must not be read
 // again after the kernel's own stores) with its pointers loaded as global ones (see load_global_ptr)
 template <class Table>
-__device__ __forceinline__ FlatJob flat_job(const Table& tab) {
-    const FlatJob& src = tab.job[blockIdx.y];
+__device__ __forceinline__ FlatJob flat_job_at(const Table& tab, const uint32_t row) {
+    const FlatJob& src = tab.job[row];
     FlatJob j;
     j.w = load_global_ptr(&src.w);
     j.q = load_global_ptr(&src.q);
@@ -157,6 +157,8 @@ __device__ __forceinline__ FlatJob flat_job(const Table& tab) {
     j.pad = src.pad;
     return j;
 }
+template <class Table>
+__device__ __forceinline__ FlatJob flat_job(const Table& tab) { return flat_job_at(tab, blockIdx.y); }
 template <class Table>
 __device__ __forceinline__ int64_t flat_block(const Table& tab) { return xcd_chunked_block(tab.chunk); }
 // largest chunk of the form 2^a or 3 * 2^a (up to MQ_FLAT_CHUNK) whose grid padding stays under 3 % of `blocks` workgroups

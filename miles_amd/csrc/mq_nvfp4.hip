@@ -758,18 +758,25 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
 //     kOneWords words, each a line of its own, one of which every other workgroup watches with one request at a time.
 //     (With every workgroup watching all slots the polling itself filled the memory channels that hold them: 496 us
 //     instead of 240 on 32 x [2048, 7168].)  No counters, so no atomic read-modify-writes.
-//   every wait ends: after kOnePolls looks a workgroup leaves its part to the second pass (kRecRedo), the same kernel that
-//     re-quantizes tensors whose carried-over amax moved.  That happens when workgroups of one record cannot all be on
+//   every wait ends: after kOnePolls looks the first workgroup of a record publishes that it has given up (kOneGaveUp) in place
+//     of the maximum, and every workgroup that reads it leaves: that happens when workgroups of one record cannot all be on
 //     the chip because something else occupies it; workgroups start in order of their ids, so otherwise the oldest
-//     unfinished tensor always gets there.  A first workgroup that gives up publishes that (kOneGaveUp) in place of the
-//     maximum, and every workgroup that reads it leaves at once: a record that does not fit next to a busy neighbour costs
+//     unfinished tensor always gets there.  A record that does not fit next to a busy neighbour so costs
 //     one wait, not one for each batch of its workgroups that comes to the chip.  32 x [2048, 7168] beside a stream of
-//     [8192, 8192] matrix products: 2.5 ms, 3.0 without that word, 2.35 in two passes (beside one of copies 0.56, 0.56, 0.91).
-// 32 x [2048, 7168] (940 MB of bf16, all launches together): 311 us in two passes, 218 us this way (5.55 TB/s; 226 with a
+//     [8192, 8192] matrix products: 1.0 ms, of copies 0.37 (1.8 and 0.37 with what is left in a launch behind, which
+//     starts when the neighbour makes room).
+//   what is left: rows of workgroups behind those of the tensors (nv_one_rest), which start when all of these have, read every
+//     record's word and quantize what its own workgroups did not.  (As a launch behind this one they cost 4.5 us.)
+// 32 x [2048, 7168] (940 MB of bf16, all launches together): 311 us in two passes, 214 us this way (5.6 TB/s; 217 with what
+// is left in a launch behind, where 28 x [528, 3088] took 32.5 us and now 29, 48 x [1536, 2048] 73 and now 68; 226 with a
 // block's scale computed in both lanes that hold it and its byte stored under a mask, 234 with the block maxima taken after the
 // wait and a range test and a branch to the software forms in each unit).  24 units per lane at
 // four workgroups per CU were 5 % slower, 8 units in 512 lanes 6 %, six workgroups per CU (20 registers spilled) 38 %; two
 // units stored together, eight bytes a lane, 2 % slower here and 2 % faster on 18 x [1420, 1520].
+// What bounds it: so many long-lived workgroups stream at 5.8 TB/s even if nobody waits for anybody (206 of the kernel's
+// 209 us), where two units a lane stream at 6.9.  Two, four or six units a lane more, held in LDS, 222 to 234 us; four loads in flight
+// at a time 225 to 236; a tensor's units dealt to its workgroups in turn 222; plain stores 220; starting the first
+// workgroups of a CU one after the other, no difference.
 constexpr int kOneThreads = 256, kOneUnits = 16, kOneWavesPerSimd = 5;
 constexpr int64_t kOnePerBlock = kOneThreads * kOneUnits;
 constexpr int kOneSlots = 2 * kSectionWords;         // 16-bit slots of a section
@@ -777,9 +784,10 @@ constexpr uint32_t kOneFull = 0x8000u;               // marks a slot or word tha
 constexpr uint32_t kOneGaveUp = 0x10000u;            // in a word: the first workgroup has stopped waiting
 constexpr int kOneWords = 7, kOneStride = 32, kRecOne = kRecAmax + 32;     // the published maximum, 128 bytes apart
 static_assert(kRecOne + (kOneWords - 1) * kOneStride < MQ_NVFP4_RECORD_WORDS, "the published words lie inside the record");
-constexpr int kRecReaders = kRecMovedRuns + 1;       // workgroups of the finish that have read the slots of a record left to it
+constexpr int kRecReaders = kRecMovedRuns + 1;       // workgroups of the rows behind that have read the slots of a record left to them
 constexpr int kOneLeaderSleep = 1, kOneSleep = 12;   // between two looks, in units of 64 cycles
-constexpr int kOnePolls = 256;                       // looks of a workgroup, 0.25 ms or more; undisturbed, some 10 are enough
+constexpr int kOnePolls = 256;                       // looks of a first workgroup, 0.25 ms or more; undisturbed, some 10 are enough
+constexpr int kOnePatience = 1 << 16;                // of those that watch its word, which it writes in any case, 60 ms or more
 
 __device__ __forceinline__ void agent_store(uint32_t* p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void agent_store16(uint16_t* p, uint16_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -791,7 +799,7 @@ __global__ __launch_bounds__(256) void nvfp4_one_pass_clear_kernel(const Table t
     const FlatJob& job = tab.job[blockIdx.x];
     uint32_t* rec = (uint32_t*)job.aux;
     rec[job.section * kSectionWords + threadIdx.x] = 0;
-    if (job.section == 0 && threadIdx.x == 0) rec[kRecRedo] = rec[kRecReaders] = 0;
+    if (job.section == 0 && threadIdx.x == 0) rec[kRecReaders] = 0;
     if (job.section == 0 && threadIdx.x < kOneWords) rec[kRecOne + threadIdx.x * kOneStride] = 0;
 }
 
@@ -830,12 +838,132 @@ __device__ __forceinline__ float pair_lane(const float v) {
     return u2f((uint32_t)__builtin_amdgcn_update_dpp(bits, bits, ODD ? 0xF5 /* 1, 1, 3, 3 */ : 0xA0 /* 0, 0, 2, 2 */, 0xF, 0xF, true));
 }
 
-// job as for the quantize pass: section = place of the tensor inside its record, pad = tensors sharing it (neighbours)
+// the maximum over the workgroup of what its lanes have (CALL: one number for each place that takes one, which has words of its own)
+template <int CALL>
+__device__ __forceinline__ uint32_t nv_one_max(uint32_t m, const int t) {
+    __shared__ uint32_t part[kOneThreads / kWave];
+    m = wave_max(m);
+    if ((t & (kWave - 1)) == 0) part[t / kWave] = m;
+    __syncthreads();
+    m = 0;
+#pragma unroll
+    for (int k = 0; k < kOneThreads / kWave; k++) m = umax(m, part[k]);
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)m);
+}
+// What this lane sees of a record's slots, a word (two slots) of each section, as soon as they are all written; `late` if that
+// took more than `polls` looks.  row: of the record's first tensor.
+template <class Table>
+__device__ __forceinline__ uint32_t nv_one_collect(const Table& tab, const uint32_t row, const uint32_t* rec, const int tensors_of_it, const int t,
+                                                   const int polls, bool& late) {
+    uint32_t m = 0;
+    for (int k = 0; k < tensors_of_it; k++) {
+        const int64_t units = tab.job[row + k].units;
+        const int slots = (int)((units + kOnePerBlock - 1) / kOnePerBlock);
+        for (int word = t; word * 2 < slots; word += kOneThreads) {
+            const uint32_t need = word * 2 + 1 < slots ? 0x80008000u : 0x8000u;
+            uint32_t got = agent_load(rec + k * kSectionWords + word);
+            for (int n = 0; (got & need) != need && n < polls; n++) {
+                __builtin_amdgcn_s_sleep(kOneLeaderSleep);
+                got = agent_load(rec + k * kSectionWords + word);
+            }
+            late |= (got & need) != need;
+            m = umax(m, hmax_u16(abs2(got)));
+        }
+    }
+    return m;
+}
+// The record's published word for the whole workgroup, or 0 if its first workgroup has not come to write it in
+// `patience` looks.
+__device__ __forceinline__ uint32_t nv_one_watch(const uint32_t* word, const int t, const int patience) {
+    __shared__ uint32_t seen;
+    if (t < kWave) {
+        uint32_t got = agent_load(word);
+        for (int n = 0; got == 0 && n < patience; n++) {
+            __builtin_amdgcn_s_sleep(kOneSleep);
+            got = agent_load(word);
+        }
+        if (t == 0) seen = got;
+    }
+    __syncthreads();
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)seen);
+}
+// the same from the elements: for who has watched in vain
+template <class Table>
+__device__ __forceinline__ uint32_t nv_one_scan(const Table& tab, const uint32_t row, const int tensors_of_it, const int t) {
+    uint32_t m2 = 0;
+    for (int k = 0; k < tensors_of_it; k++) {
+        const uint16_t* __restrict__ w = (const uint16_t*)load_global_ptr(&tab.job[row + k].w);
+        const int64_t units = tab.job[row + k].units;
+        for (int64_t u = t; u < units; u += kOneThreads) {
+            const u32x4 v = ld16(w + u * 8);
+            m2 = max2_u16(m2, max2_u16(max2_u16(abs2(v.x), abs2(v.y)), max2_u16(abs2(v.z), abs2(v.w))));
+        }
+    }
+    return nv_one_max<2>(hmax_u16(m2), t);
+}
+// Tensors with an infinity or a NaN, or with a scale at the ends of the fp32 range, are left as well: the code behind
+// has the software forms, which here, in sixteen copies, were 8 700 instructions in the way of the 2 000 that run.
+template <int F16>
+__device__ __forceinline__ bool nv_one_leaves(const uint32_t m, const NvScales& gs) {
+    const uint32_t dec = f2u(gs.s_dec);
+    return m >= (F16 ? 0x7C00u : 0x7F80u) || !(dec >= 0x16800000u /* 2^-82 */ && dec <= 0x68000000u /* 2^81 */);
+}
+
+// Rows behind the tensors', `workers` workgroups to a tensor: they quantize the records that were left.  They come to the chip
+// when every workgroup of the tensors has, most of which are done, and of a record that is done there is its word to read.
+// The slots of a record whose first workgroup has given up, which every worker folds, are cleared by the last one to have read
+// them (a carried run would take their marks for kCarriedMark).
 template <int F16, class Table>
-__global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_kernel(const Table tab, float numer, int first_polls) {
-    __shared__ uint32_t wave_seen[kOneThreads / 64], wave_late[kOneThreads / 64];
-    const FlatJob job = flat_job(tab);
+__device__ __forceinline__ void nv_one_rest(const Table& tab, const uint32_t tensors, const uint32_t workers, const int patience, const int t, float numer,
+                                            uint32_t* moved_counter) {
+    __shared__ uint32_t readers;
+    const uint32_t id = (blockIdx.y - tensors) * gridDim.x + blockIdx.x, worker = id / tensors, row = id - worker * tensors;
+    if (worker >= workers) return;
+    const FlatJob job = flat_job_at(tab, row);
+    uint32_t* rec = (uint32_t*)job.aux;
+    const uint32_t got = nv_one_watch(rec + kRecOne + (id % kOneWords) * kOneStride, t, patience);
+    const bool gave_up = got == kOneGaveUp;
+    uint32_t m = got & 0x7FFFu;
+    bool late = got == 0;
+    if (gave_up) m = nv_one_max<1>(nv_one_collect(tab, row - job.section, rec, job.pad, t, patience, late), t);
+    if (__syncthreads_or(late)) m = nv_one_scan(tab, row - job.section, job.pad, t);
+    const float amax = elem_lo<F16>(m);
+    const NvAmaxScales a{amax, nv_scales(amax, numer)};
+    if ((got & kOneFull) != 0 && !nv_one_leaves<F16>(m, a.gs)) return;
+    if (gave_up) {
+        if (t == 0) readers = atomicAdd(rec + kRecReaders, 1u);
+        __syncthreads();
+        if (readers + 1 == workers * (uint32_t)job.pad)
+            for (int k = 0; k < job.pad; k++) rec[k * kSectionWords + t] = 0;
+    }
+    if ((got & kOneFull) == 0 && worker == 0 && t == 0) nv_publish_plain(job, a.amax, a.gs, numer, moved_counter);
+    constexpr int64_t kPerBlock = nv_units_per_block(0);
+    for (int64_t base = worker * kPerBlock; base < job.units; base += workers * kPerBlock)
+        nvfp4_quant_units<0, F16>(job, base, t, numer, [&] { return a; });
+}
+// By a record's first workgroup, when it has nothing else to do: the record of a maximum that it has published, for all
+// tensors that share it; the slots, which nobody reads any more, are cleared for a carried run.
+template <class Table>
+__device__ __forceinline__ void nv_one_settle(const Table& tab, const FlatJob& job, const int t, float amax, const NvScales& gs, float numer,
+                                              const bool left, uint32_t* moved_counter) {
+    uint32_t* rec = (uint32_t*)job.aux;
+    for (int k = 0; k < job.pad; k++) rec[k * kSectionWords + t] = 0;
+    if (t != 0) return;
+    rec[kRecRedo] = left;
+    for (int k = 0; k < job.pad; k++) nv_publish_plain(flat_job_at(tab, blockIdx.y + k), amax, gs, numer, moved_counter);
+}
+
+// job as for the quantize pass: section = place of the tensor inside its record, pad = tensors sharing it (neighbours)
+// grid (workgroups of the largest tensor, tensors + rows behind)
+template <int F16, class Table>
+__global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_kernel(const Table tab, float numer, int first_polls, int patience, uint32_t tensors,
+                                                                                       uint32_t workers, uint32_t* moved_counter, uint32_t* moved_mirror) {
     const int t = threadIdx.x;
+    if (blockIdx.y >= tensors) {
+        nv_one_rest<F16>(tab, tensors, workers, patience, t, numer, moved_counter);
+        return;
+    }
+    const FlatJob job = flat_job(tab);
     const int64_t block = flat_block(tab), base = block * kOnePerBlock;
     if (base >= job.units) return;
     const int64_t left = job.units - base;
@@ -858,137 +986,56 @@ __global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_
 #pragma unroll
     for (int i = 0; i < kOneUnits; i += 2) {
         maxima[i / 2] = nv_block_max(v[i]) | (nv_block_max(v[i + 1]) << 16);
+        if constexpr (std::is_same<Table, FlatRef>::value) asm("" : "+v"(maxima[i / 2]));      // (else its halves are kept as well, in scratch memory)
         m2 = max2_u16(m2, maxima[i / 2]);
     }
-    uint32_t m = wave_max(hmax_u16(m2));
-    if ((t & 63) == 0) wave_seen[t >> 6] = m;
-    __syncthreads();
+    uint32_t m = nv_one_max<0>(hmax_u16(m2), t);
     uint32_t* rec = (uint32_t*)job.aux;
-    if (t == 0) {
-        m = 0;
-#pragma unroll
-        for (int k = 0; k < kOneThreads / 64; k++) m = umax(m, wave_seen[k]);
-        agent_store16((uint16_t*)(rec + job.section * kSectionWords) + block, (uint16_t)(kOneFull | m));
-    }
-    m = 0;
-    bool late = false;
-    if (block == 0 && job.section == 0) {
-        // the record's first workgroup waits for every other one: a lane watches one word (two slots) of each section
-        for (int k = 0; k < job.pad; k++) {
-            const int64_t units = tab.job[blockIdx.y + k].units;
-            const int slots = (int)((units + kOnePerBlock - 1) / kOnePerBlock);
-            for (int word = t; word * 2 < slots; word += kOneThreads) {
-                const uint32_t need = word * 2 + 1 < slots ? 0x80008000u : 0x8000u;
-                uint32_t got = agent_load(rec + k * kSectionWords + word);
-                for (int n = 0; (got & need) != need && n < first_polls; n++) {
-                    __builtin_amdgcn_s_sleep(kOneLeaderSleep);
-                    got = agent_load(rec + k * kSectionWords + word);
-                }
-                late |= (got & need) != need;
-                m = umax(m, hmax_u16(abs2(got)));
-            }
+    if (t == 0) agent_store16((uint16_t*)(rec + job.section * kSectionWords) + block, (uint16_t)(kOneFull | m));
+    const bool first = block == 0 && job.section == 0;
+    if (first) {
+        // the record's first workgroup waits for every other one
+        bool late = false;
+        m = nv_one_max<1>(nv_one_collect(tab, blockIdx.y, rec, job.pad, t, first_polls, late), t);
+        const bool gave_up = __syncthreads_or(late);
+        if (t < kOneWords) agent_store(rec + kRecOne + t * kOneStride, gave_up ? kOneGaveUp : kOneFull | m);
+        if (blockIdx.y == 0) amax_feedback_folded(moved_counter, moved_mirror, tensors);
+        if (gave_up) {
+            if (t == 0) rec[kRecRedo] = 1;
+            return;
         }
-        __syncthreads();            // wave_seen has been read
-        m = wave_max(m);
-        const uint32_t any_late = __builtin_amdgcn_ballot_w64(late) != 0;
-        if ((t & 63) == 0) {
-            wave_seen[t >> 6] = m;
-            wave_late[t >> 6] = any_late;
-        }
-        __syncthreads();
-        m = 0;
-        uint32_t gave_up = 0;
-#pragma unroll
-        for (int k = 0; k < kOneThreads / 64; k++) {
-            m = umax(m, wave_seen[k]);
-            gave_up |= wave_late[k];
-        }
-        late = gave_up != 0;
-        if (t < kOneWords) agent_store(rec + kRecOne + t * kOneStride, late ? kOneGaveUp : kOneFull | m);
     } else {
-        if (t < 64) {
-            const uint32_t* word = rec + kRecOne + (blockIdx.x % kOneWords) * kOneStride;
-            uint32_t got = agent_load(word);
-            for (int n = 0; got == 0 && n < kOnePolls; n++) {
-                __builtin_amdgcn_s_sleep(kOneSleep);
-                got = agent_load(word);
-            }
-            if (t == 0) wave_late[0] = got;
-        }
-        __syncthreads();
-        m = wave_late[0];
-        late = (m & kOneFull) == 0;
+        m = nv_one_watch(rec + kRecOne + (blockIdx.x % kOneWords) * kOneStride, t, patience);
+        if (m == 0) m = kOneFull | nv_one_scan(tab, blockIdx.y - job.section, job.pad, t);
+        if ((m & kOneFull) == 0) return;
         m &= 0x7FFFu;
     }
-    const NvScales gs = nv_scales(elem_lo<F16>(m), numer);
-    // Tensors with an infinity or a NaN, or with a scale at the ends of the fp32 range, are left to the finish as well: its
-    // code has the software forms, which here, in sixteen copies, were 8 700 instructions in the way of the 2 000 that run.
-    const uint32_t dec = f2u(gs.s_dec);
-    if (late || m >= (F16 ? 0x7C00u : 0x7F80u) || !(dec >= 0x16800000u /* 2^-82 */ && dec <= 0x68000000u /* 2^81 */)) {
-        if (t == 0) rec[kRecRedo] = 1;
-        return;
-    }
-    // Both lanes of a pair hold the maxima of the same blocks: of two units the even lane takes the first one's scale and the
-    // odd lane the second one's, so that a scale is computed once and every lane stores a byte.
-    const uint32_t odd = (uint32_t)t & 1u;
-    uint32_t* __restrict__ q0 = (uint32_t*)job.q + base;
-    uint8_t* __restrict__ s80 = (uint8_t*)job.s + base / 2;
-    auto quantize = [&](auto full) {
+    const float amax = elem_lo<F16>(m);
+    const NvScales scales = nv_scales(amax, numer), gs{uniform_f(scales.enc_sixth), uniform_f(scales.s_dec), uniform_f(scales.enc)};
+    const bool leaves = nv_one_leaves<F16>(m, gs);
+    if (!leaves) {
+        // Both lanes of a pair hold the maxima of the same blocks: of two units the even lane takes the first one's scale and the
+        // odd lane the second one's, so that a scale is computed once and every lane stores a byte.
+        const uint32_t odd = (uint32_t)t & 1u;
+        uint32_t* __restrict__ q0 = (uint32_t*)job.q + base;
+        uint8_t* __restrict__ s80 = (uint8_t*)job.s + base / 2;
+        auto quantize = [&](auto full) {
 #pragma unroll
-        for (int i = 0; i < kOneUnits; i += 2) {
-            const uint32_t two = maxima[i / 2];
-            const NvPlainScale s = nv_plain_scale(odd ? elem_hi<F16>(two) : elem_lo<F16>(two), gs);
-            const uint32_t word0 = nv_plain_codes<F16>(v[i], pair_lane<0>(s.inv)), word1 = nv_plain_codes<F16>(v[i + 1], pair_lane<1>(s.inv));
-            const uint32_t off = (uint32_t)t + i * kOneThreads;
-            if (full || off < rem) st4(q0 + off, word0);
-            if (full || off + kOneThreads < rem) st4(q0 + off + kOneThreads, word1);
-            if (full || off + odd * kOneThreads < rem) s80[(off >> 1) + odd * (kOneThreads / 2)] = (uint8_t)s.sc;
-            __builtin_amdgcn_sched_barrier(0);      // two units at a time: more do not fit the registers
-        }
-    };
-    if (whole) quantize(std::true_type{});
-    else quantize(std::false_type{});
-}
-
-// Behind the one-pass kernel: quantizes the records that were left to it and publishes every record's amax, scales and
-// published scales.  grid (up to kSectionWords, tensors).  The slots are cleared for a carried run (their marks would pass for
-// kCarriedMark): of a finished record, whose amax its first workgroup has published, by the tensor's first workgroup here; of
-// one left to this pass, where every workgroup folds the slots, by the last one to have read them.
-// kRecRedo stays as the one-pass kernel left it.  (One launch of 4.3 us for the two of 4.3 us each that did this.)
-template <int F16, class Table>
-__global__ __launch_bounds__(kNvThreads) void nvfp4_one_pass_finish_kernel(const Table tab, float numer, uint32_t* moved_counter, uint32_t* moved_mirror) {
-    const FlatJob job = flat_job(tab);
-    const int t = threadIdx.x;
-    uint32_t* rec = (uint32_t*)job.aux;
-    const bool redo = rec[kRecRedo] != 0;
-    if (blockIdx.x != 0 && !redo) return;
-    if (blockIdx.x == 0 && blockIdx.y == 0) amax_feedback_folded(moved_counter, moved_mirror, gridDim.y);
-    uint32_t bits;
-    if (!redo) {
-        bits = rec[kRecOne] & ~kOneFull;
-        rec[job.section * kSectionWords + t] = 0;
-    } else {
-        __shared__ uint32_t part[kNvThreads / kWave], readers;
-        bits = 0;
-        for (int k = 0; k < job.pad; k++) bits = umax(bits, hmax_u16(abs2(rec[k * kSectionWords + t])));
-        bits = wave_max(bits);
-        if ((t & (kWave - 1)) == 0) part[t >> 6] = bits;
-        __syncthreads();
-        bits = umax(umax(part[0], part[1]), umax(part[2], part[3]));
-        if (t == 0) readers = atomicAdd(rec + kRecReaders, 1u);
-        __syncthreads();
-        if (readers + 1 == gridDim.x * (uint32_t)job.pad)
-            for (int k = 0; k < job.pad; k++) rec[k * kSectionWords + t] = 0;
+            for (int i = 0; i < kOneUnits; i += 2) {
+                const uint32_t two = maxima[i / 2];
+                const NvPlainScale s = nv_plain_scale(odd ? elem_hi<F16>(two) : elem_lo<F16>(two), gs);
+                const uint32_t word0 = nv_plain_codes<F16>(v[i], pair_lane<0>(s.inv)), word1 = nv_plain_codes<F16>(v[i + 1], pair_lane<1>(s.inv));
+                const uint32_t off = (uint32_t)t + i * kOneThreads;
+                if (full || off < rem) st4(q0 + off, word0);
+                if (full || off + kOneThreads < rem) st4(q0 + off + kOneThreads, word1);
+                if (full || off + odd * kOneThreads < rem) s80[(off >> 1) + odd * (kOneThreads / 2)] = (uint8_t)s.sc;
+                __builtin_amdgcn_sched_barrier(0);      // two units at a time: more do not fit the registers
+            }
+        };
+        if (whole) quantize(std::true_type{});
+        else quantize(std::false_type{});
     }
-    const float amax = elem_lo<F16>(bits);
-    const NvAmaxScales a{amax, nv_scales(amax, numer)};
-    if (blockIdx.x == 0 && t == 0) nv_publish_plain(job, a.amax, a.gs, numer, moved_counter);
-    if (!redo) return;
-    // an XCD takes a run of consecutive blocks in every trip of the grid, as in the second pass of a carried run
-    constexpr int64_t kPerBlock = nv_units_per_block(0);
-    const int64_t first = xcd_chunked_block(gridDim.x == kSectionWords ? kSectionWords / kXcds : tab.chunk);
-    for (int64_t base = first * kPerBlock; base < job.units; base += (int64_t)gridDim.x * kPerBlock)
-        nvfp4_quant_units<0, F16>(job, base, t, numer, [&] { return a; });
+    if (first) nv_one_settle(tab, job, t, amax, gs, numer, leaves, moved_counter);
 }
 
 // fp32 input, the second pass of the two-pass form (the carried-over amax and the one-pass form are for 16-bit tensors).
@@ -1403,10 +1450,12 @@ int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, in
 // largest number of workgroups that share a record, `bytes` the input of the whole chunk.  All workgroups of a record
 // have to be on the chip together, and the records behind it should be loading meanwhile: half of what fits (640 workgroups,
 // 40 MB, on 256 CUs).  A pair of [2048, 7168] weights, 896 workgroups, gained less (313 -> 265 us for 16 pairs) and is one
-// busy neighbour away from waiting in vain, so it keeps two passes.  Short lists keep them as well, which then find their second
-// read in the memory-side cache and save a launch (us, two passes / one): 4 x [1537, 2064] (25 MB) 15 / 18, 4 x [2048, 4096]
-// (67 MB) 27 / 24, 18 x [1420, 1520] (78 MB) 33 / 30, 16 x [1536, 2048] (100 MB) 39 / 33, 48 x [1536, 2048] (302 MB) 105 / 73.
-constexpr int64_t kOneMinBytes = 64ll << 20;
+// busy neighbour away from waiting in vain, so it keeps two passes.  Short lists keep them as well: they find their second
+// read in the memory-side cache, and the launch that clears the slots takes what is left of the gain (us, two passes / one): 4 x
+// [256, 1024] (2 MB) 6.5 / 8.8, 2 x [1024, 2048] 8.3 / 9.9, 4 of them (17 MB) 10.8 / 11.3, 1 x [2048, 4096] (17 MB) 11.5 / 11.1,
+// 4 x [1537, 2064] (25 MB) 14.2 / 13.3, 1 x [2048, 7168] (29 MB) 16.3 / 13.9, 8 x [1024, 2048] (34 MB) 16.2 / 14.8, 2 x [2048, 7168] (59 MB)
+// 24.0 / 19.0.
+constexpr int64_t kOneMinBytes = 24ll << 20;
 bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes) {
     int device = 0, cus = 0;
     if (bytes < kOneMinBytes || max_units > kOneSlots * kOnePerBlock) return false;
@@ -1418,34 +1467,41 @@ bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes) {
 }
 int64_t mq_nvfp4_one_pass_slots(int64_t units) { return (units + kOnePerBlock - 1) / kOnePerBlock; }
 
-// descriptors as for mode 1; `redo` and `one`: their grids for the second pass and for the one-pass kernel
+// workgroups behind the tensors' own, for each of n tensors of at most max_units: 64 of a list of 32 tensors (the launch has
+// 0.4 ns for one that finds nothing to do), and enough to fill half of the chip for one that is left
+constexpr int kOneWorkers = 2048;
+static uint32_t nv_one_workers(int n, int64_t max_units) {
+    const int64_t blocks = (max_units + nv_units_per_block(0) - 1) / nv_units_per_block(0);
+    int64_t workers = kOneWorkers / n;
+    workers = workers < 16 ? 16 : workers > kSectionWords ? kSectionWords : workers;
+    return (uint32_t)(workers < blocks ? workers : blocks);
+}
+// descriptors as for mode 1
 template <class Table, int F16>
-static int nvfp4_one_pass_launch_dtype(const Table& one, const Table& redo, int n, float numer, int first_polls, hipStream_t st) {
-    const dim3 folds((unsigned)n), blk(256);
-    hipLaunchKernelGGL((nvfp4_one_pass_clear_kernel<Table>), folds, blk, 0, st, one);
-    hipLaunchKernelGGL((nvfp4_one_pass_kernel<F16, Table>), dim3((unsigned)one.max_blocks, (unsigned)n), dim3(kOneThreads), 0, st, one, numer, first_polls);
-    const unsigned redo_blocks = redo.max_blocks < kSectionWords ? (unsigned)redo.max_blocks : (unsigned)kSectionWords;
-    hipLaunchKernelGGL((nvfp4_one_pass_finish_kernel<F16, Table>), dim3(redo_blocks, (unsigned)n), dim3(kNvThreads), 0, st, redo, numer,
+static int nvfp4_one_pass_launch_dtype(const Table& tab, int n, int64_t max_units, float numer, int first_polls, int patience, hipStream_t st) {
+    const uint32_t workers = nv_one_workers(n, max_units), blocks = (uint32_t)tab.max_blocks;
+    const dim3 grid(blocks, (unsigned)(n + ((int64_t)n * workers + blocks - 1) / blocks));
+    hipLaunchKernelGGL((nvfp4_one_pass_clear_kernel<Table>), dim3((unsigned)n), dim3(256), 0, st, tab);
+    hipLaunchKernelGGL((nvfp4_one_pass_kernel<F16, Table>), grid, dim3(kOneThreads), 0, st, tab, numer, first_polls, patience, (uint32_t)n, workers,
                        mq_amax_feedback(), mq_amax_feedback_mirror());
     return mq_check_launch("nvfp4 quant (one pass)");
 }
 template <class Table>
-static int nvfp4_one_pass_launch(int dtype, const Table& one, const Table& redo, int n, int e4m3_max, int flags, hipStream_t st) {
+static int nvfp4_one_pass_launch(int dtype, const Table& tab, int n, int64_t max_units, int e4m3_max, int flags, hipStream_t st) {
     const float numer = (float)e4m3_max * 6.0f;
-    const int first_polls = (flags & MQ_NVFP4_NO_WAIT) ? 0 : kOnePolls;
-    return dtype == MQ_F16 ? nvfp4_one_pass_launch_dtype<Table, 1>(one, redo, n, numer, first_polls, st)
-                           : nvfp4_one_pass_launch_dtype<Table, 0>(one, redo, n, numer, first_polls, st);
+    const int first_polls = (flags & MQ_NVFP4_NO_WAIT) ? 0 : kOnePolls, patience = (flags & MQ_NVFP4_NO_PATIENCE) ? 0 : kOnePatience;
+    return dtype == MQ_F16 ? nvfp4_one_pass_launch_dtype<Table, 1>(tab, n, max_units, numer, first_polls, patience, st)
+                           : nvfp4_one_pass_launch_dtype<Table, 0>(tab, n, max_units, numer, first_polls, patience, st);
 }
-int mq_nvfp4_one_pass_launch_group(int dtype, const FlatTable& tab, int e4m3_max, int flags, hipStream_t st) {
-    FlatTable one = tab, redo = tab;
-    if (!flat_grid(one, kOnePerBlock) || !flat_grid(redo, kNvThreads * kNvUnroll)) return mq_fail(MQ_ERR_ARG, "tensor too large");
-    return nvfp4_one_pass_launch(dtype, one, redo, tab.n, e4m3_max, flags, st);
+int mq_nvfp4_one_pass_launch_group(int dtype, FlatTable& tab, int64_t max_units, int e4m3_max, int flags, hipStream_t st) {
+    if (!flat_grid(tab, kOnePerBlock)) return mq_fail(MQ_ERR_ARG, "tensor too large");
+    return nvfp4_one_pass_launch(dtype, tab, tab.n, max_units, e4m3_max, flags, st);
 }
 int mq_nvfp4_one_pass_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int e4m3_max, int flags,
                                    hipStream_t st) {
-    FlatRef one{device_jobs, 0, 0}, redo{device_jobs, 0, 0};
-    if (!flat_grid(one, max_units, kOnePerBlock) || !flat_grid(redo, max_units, kNvThreads * kNvUnroll)) return mq_fail(MQ_ERR_ARG, "tensor too large");
-    return nvfp4_one_pass_launch(dtype, one, redo, n, e4m3_max, flags, st);
+    FlatRef ref{device_jobs, 0, 0};
+    if (!flat_grid(ref, max_units, kOnePerBlock)) return mq_fail(MQ_ERR_ARG, "tensor too large");
+    return nvfp4_one_pass_launch(dtype, ref, n, max_units, e4m3_max, flags, st);
 }
 
 extern "C" int mq_nvfp4_amax(const void* w, int dtype, int64_t numel, void* record, int section, void* stream) {

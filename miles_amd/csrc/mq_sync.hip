@@ -36,7 +36,7 @@ int mq_nvfp4_amax_launch_group(int dtype, FlatTable& tab, hipStream_t st);
 int mq_nvfp4_quant_launch_group(int dtype, FlatTable& tab, int e4m3_max, int flags, int mode, hipStream_t st);
 bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes);
 int64_t mq_nvfp4_one_pass_slots(int64_t units);
-int mq_nvfp4_one_pass_launch_group(int dtype, const FlatTable& tab, int e4m3_max, int flags, hipStream_t st);
+int mq_nvfp4_one_pass_launch_group(int dtype, FlatTable& tab, int64_t max_units, int e4m3_max, int flags, hipStream_t st);
 int mq_nvfp4_one_pass_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int e4m3_max, int flags,
                                    hipStream_t st);
 bool mq_mxfp4_fast_ok(const void* w, int dtype, const void* packed, int group);
@@ -136,7 +136,7 @@ enum JobPath { kSinglePath, kFastPath, kAnyPath };
 static JobPath job_path(const mq_job& j) { return job_fast(j) ? kFastPath : job_any(j) ? kAnyPath : kSinglePath; }
 
 // flags of an NVFP4 job that the driver acts on itself, and those that mq_nvfp4_quant knows
-constexpr int kNvDriverFlags = MQ_NVFP4_CARRY_AMAX | MQ_NVFP4_NO_WAIT;
+constexpr int kNvDriverFlags = MQ_NVFP4_CARRY_AMAX | MQ_NVFP4_NO_WAIT | MQ_NVFP4_NO_PATIENCE;
 constexpr int kNvQuantFlags = MQ_NVFP4_4OVER6 | MQ_NVFP4_ERR_MSE | MQ_NVFP4_ERR_FP16;
 
 static int64_t copy_dst_pitch(const mq_job& j);
@@ -549,7 +549,7 @@ static int run_nvfp4(const mq_job* jobs, int64_t n_all, int64_t i, int64_t j, co
                 const mq_job& jb = jobs[i + t];
                 tab.job[t] = FlatJob{jb.in, jb.out, jb.scale, jb.aux, jb.rows * jb.cols / 8, jb.aux2, section[t], sections[t]};
             }
-            rc = one_pass ? mq_nvfp4_one_pass_launch_group(jobs[i].dtype, tab, jobs[i].p0, jobs[i].p1, st)
+            rc = one_pass ? mq_nvfp4_one_pass_launch_group(jobs[i].dtype, tab, max_units, jobs[i].p0, jobs[i].p1, st)
                           : mq_nvfp4_quant_launch_group(jobs[i].dtype, tab, jobs[i].p0, jobs[i].p1 & ~kNvDriverFlags, carry ? 2 : 1, st);
             if (rc) return rc;
         } else {

@@ -1,0 +1,60 @@
+"""NVFP4 lists that are read once: the rows of workgroups behind the tensors', which quantize what was left, and workgroups that
+do not wait for the word of a record's first one."""
+
+import pytest
+import torch
+
+from miles_amd import _lib, launch
+from miles_amd.utils.nvfp4 import nvfp4_quantize_1d, nvfp4_quantize_1d_pair
+
+pytestmark = pytest.mark.gpu
+
+
+def _same(got, want, what):
+    for a, b in zip(got, want):
+        a, b = (t.contiguous().reshape(-1).view(torch.uint8) for t in (a, b))
+        assert torch.equal(a, b), what
+
+
+@pytest.mark.parametrize("flag", [0, _lib.NVFP4_NO_WAIT, _lib.NVFP4_NO_PATIENCE, _lib.NVFP4_NO_WAIT | _lib.NVFP4_NO_PATIENCE])
+@pytest.mark.parametrize("n, rows, cols, pairs", [
+    (3, 1024, 11184, False),            # few tensors: as many workers as a section has words
+    (9, 512, 7216, False),              # ragged last workgroup
+    (128, 16, 16384, False),            # more tensors than one launch of 64, workers bounded by a tensor's blocks
+    (140, 257, 1040, False),            # over a device table
+    (24, 768, 2048, True),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_what_is_left_and_the_records_behind_it(n, rows, cols, pairs, dtype, flag):
+    g = torch.Generator(device="cuda").manual_seed(n + cols)
+    x = (torch.randn(n, rows, cols, generator=g, device="cuda") * 0.02).to(dtype)
+    x[0, 0, 3] = float("inf")                           # left whatever the waits do, and the last one too
+    x[n - 1, rows - 1, cols - 1] = float("nan")
+    if n > 3:
+        x[2].zero_()
+    with launch.recording() as batch:
+        if pairs:
+            got = [t for i in range(0, n, 2) for t in nvfp4_quantize_1d_pair(x[i], x[i + 1])]
+        else:
+            got = [nvfp4_quantize_1d(t) for t in x]
+    batch.replace_records([r[:batch.P1] + (r[batch.P1] | flag,) + r[batch.P1 + 1:] for r in batch.records])
+    if n == 140:
+        batch.freeze()
+    for record in batch.amax_records():
+        record.fill_(-1)                                # whatever was in this memory
+    for run in range(3):
+        if run == 1 and flag != _lib.NVFP4_NO_WAIT | _lib.NVFP4_NO_PATIENCE:
+            batch.carry_amax(adaptive=False)            # the records serve a carried run
+        if run == 2:
+            x[1, 0, 0] = 1e3
+        for one in got:
+            for t in one:
+                t.view(torch.uint8).fill_(0xA5) if t.dim() else t.fill_(-1.0)
+        batch.run()
+        check = range(0, n, 2) if pairs else range(n) if n < 20 else [0, 1, 2, n // 2, n - 2, n - 1]
+        for i in check:
+            if pairs:
+                for one, ref in zip(got[i:i + 2], nvfp4_quantize_1d_pair(x[i], x[i + 1])):
+                    _same(one, ref, f"run {run}, tensor {i}")
+            else:
+                _same(got[i], nvfp4_quantize_1d(x[i]), f"run {run}, tensor {i}")
