@@ -206,8 +206,7 @@ int mq_fp8_act_quant(const void* x, int dtype, void* y, void* scale, int64_t num
 enum { MQ_NVFP4_4OVER6 = 1, MQ_NVFP4_ERR_MSE = 2, MQ_NVFP4_ERR_FP16 = 4,
        /* jobs of mq_run_jobs only: see the NVFP4 note there */
        MQ_NVFP4_CARRY_AMAX = 8,
-       MQ_NVFP4_NO_WAIT = 16,
-       MQ_NVFP4_NO_PATIENCE = 32 };
+       MQ_NVFP4_NO_WAIT = 16 };
 int mq_fill_u32(void* p, uint32_t value, int64_t n, void* stream);
 int mq_nvfp4_amax(const void* w, int dtype, int64_t numel, void* record, int section, void* stream);
 int mq_nvfp4_quant(const void* w, int dtype, const void* record, int n_sections, void* q, void* block_scale,
@@ -305,8 +304,7 @@ int mq_nvfp4_fake_quant(const mq_fake_quant_item* list, int64_t n, int dtype, vo
  * 256 CUs; a single tensor 32 MB at most).  A grouped launch holds MQ_MAX_GROUP tensors, or with a device table
  * MQ_TABLE_GROUP.  The workgroups of a record keep their share and wait for each other's maxima, for a bounded time, after
  * which workgroups behind them in the same launch do what is left.  MQ_NVFP4_NO_WAIT in p1: a record's first workgroup, which
- * collects the maxima, does not wait and tells the others so; MQ_NVFP4_NO_PATIENCE: the others don't wait for what the first one
- * has to say and read the tensors for it (both exist to test how the waits end; results are the same). */
+ * collects the maxima, does not wait and tells the others so (it exists to test that exit and what follows; results are the same). */
 enum {
     MQ_JOB_FP8_BLOCK = 0,
     MQ_JOB_FP8_BLOCKWISE_CAST = 1,

@@ -16,6 +16,7 @@ SIGNATURES = {
     "mqp_selftest_convert": [_vp, _vp],
     "mqp_selftest_reciprocal": [_vp, _vp],
     "mqp_copy_bytes": [_vp, _vp, _i64, _vp],
+    "mqp_nvfp4_one_pass": [_vp, _i32, _i32, _i32, _vp],
     "mqp_stream_probe": [_i32, _vp, _vp, _i64, _i64, _vp],
 }
 FLAT_2_1, FLAT_1_2, LOOP_2_1, TILE_2_1, TILE_READ, TILE_WRITE = range(6)      # MQP_* shapes of mqp_stream_probe

@@ -39,8 +39,8 @@ FLAGS = [
 ]
 
 
-def _link(target: str, sources: list[str], verbose: bool) -> None:
-    cmd = ["hipcc", *FLAGS, "-o", target, *(os.path.join(CSRC, s) for s in sources)]
+def _link(target: str, sources: list[str], verbose: bool, libraries: tuple[str, ...] = ()) -> None:
+    cmd = ["hipcc", *FLAGS, "-o", target, *(os.path.join(CSRC, s) for s in sources), *libraries]
     if verbose:
         print(" ".join(cmd))
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
@@ -71,7 +71,7 @@ def build(verbose: bool = False) -> str:
     os.makedirs(LIB_DIR, exist_ok=True)
     _link(LIB_PATH, SOURCES, verbose)
     _link_host(verbose)
-    _link(PROBES_LIB_PATH, PROBE_SOURCES, verbose)
+    _link(PROBES_LIB_PATH, PROBE_SOURCES, verbose, (f"-L{LIB_DIR}", "-l:libmiles_quant.so", "-Wl,-rpath,$ORIGIN"))
     return LIB_PATH
 
 

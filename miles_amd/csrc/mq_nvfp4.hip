@@ -1487,21 +1487,25 @@ static int nvfp4_one_pass_launch_dtype(const Table& tab, int n, int64_t max_unit
     return mq_check_launch("nvfp4 quant (one pass)");
 }
 template <class Table>
-static int nvfp4_one_pass_launch(int dtype, const Table& tab, int n, int64_t max_units, int e4m3_max, int flags, hipStream_t st) {
+static int nvfp4_one_pass_launch(int dtype, const Table& tab, int n, int64_t max_units, int e4m3_max, int first_polls, int patience, hipStream_t st) {
     const float numer = (float)e4m3_max * 6.0f;
-    const int first_polls = (flags & MQ_NVFP4_NO_WAIT) ? 0 : kOnePolls, patience = (flags & MQ_NVFP4_NO_PATIENCE) ? 0 : kOnePatience;
     return dtype == MQ_F16 ? nvfp4_one_pass_launch_dtype<Table, 1>(tab, n, max_units, numer, first_polls, patience, st)
                            : nvfp4_one_pass_launch_dtype<Table, 0>(tab, n, max_units, numer, first_polls, patience, st);
 }
-int mq_nvfp4_one_pass_launch_group(int dtype, FlatTable& tab, int64_t max_units, int e4m3_max, int flags, hipStream_t st) {
+static int nv_one_polls(int flags) { return (flags & MQ_NVFP4_NO_WAIT) ? 0 : kOnePolls; }
+// (with limits of its own for the waits: for the tests of how they end)
+int mq_nvfp4_one_pass_launch_waits(int dtype, FlatTable& tab, int64_t max_units, int e4m3_max, int first_polls, int patience, hipStream_t st) {
     if (!flat_grid(tab, kOnePerBlock)) return mq_fail(MQ_ERR_ARG, "tensor too large");
-    return nvfp4_one_pass_launch(dtype, tab, tab.n, max_units, e4m3_max, flags, st);
+    return nvfp4_one_pass_launch(dtype, tab, tab.n, max_units, e4m3_max, first_polls, patience, st);
+}
+int mq_nvfp4_one_pass_launch_group(int dtype, FlatTable& tab, int64_t max_units, int e4m3_max, int flags, hipStream_t st) {
+    return mq_nvfp4_one_pass_launch_waits(dtype, tab, max_units, e4m3_max, nv_one_polls(flags), kOnePatience, st);
 }
 int mq_nvfp4_one_pass_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int e4m3_max, int flags,
                                    hipStream_t st) {
     FlatRef ref{device_jobs, 0, 0};
     if (!flat_grid(ref, max_units, kOnePerBlock)) return mq_fail(MQ_ERR_ARG, "tensor too large");
-    return nvfp4_one_pass_launch(dtype, ref, n, max_units, e4m3_max, flags, st);
+    return nvfp4_one_pass_launch(dtype, ref, n, max_units, e4m3_max, nv_one_polls(flags), kOnePatience, st);
 }
 
 extern "C" int mq_nvfp4_amax(const void* w, int dtype, int64_t numel, void* record, int section, void* stream) {

@@ -136,7 +136,7 @@ enum JobPath { kSinglePath, kFastPath, kAnyPath };
 static JobPath job_path(const mq_job& j) { return job_fast(j) ? kFastPath : job_any(j) ? kAnyPath : kSinglePath; }
 
 // flags of an NVFP4 job that the driver acts on itself, and those that mq_nvfp4_quant knows
-constexpr int kNvDriverFlags = MQ_NVFP4_CARRY_AMAX | MQ_NVFP4_NO_WAIT | MQ_NVFP4_NO_PATIENCE;
+constexpr int kNvDriverFlags = MQ_NVFP4_CARRY_AMAX | MQ_NVFP4_NO_WAIT;
 constexpr int kNvQuantFlags = MQ_NVFP4_4OVER6 | MQ_NVFP4_ERR_MSE | MQ_NVFP4_ERR_FP16;
 
 static int64_t copy_dst_pitch(const mq_job& j);

@@ -1,10 +1,12 @@
 """NVFP4 lists that are read once: the rows of workgroups behind the tensors', which quantize what was left, and workgroups that
 do not wait for the word of a record's first one."""
 
+import ctypes
+
 import pytest
 import torch
 
-from miles_amd import _lib, launch
+from miles_amd import _lib, _probes, launch
 from miles_amd.utils.nvfp4 import nvfp4_quantize_1d, nvfp4_quantize_1d_pair
 
 pytestmark = pytest.mark.gpu
@@ -16,7 +18,7 @@ def _same(got, want, what):
         assert torch.equal(a, b), what
 
 
-@pytest.mark.parametrize("flag", [0, _lib.NVFP4_NO_WAIT, _lib.NVFP4_NO_PATIENCE, _lib.NVFP4_NO_WAIT | _lib.NVFP4_NO_PATIENCE])
+@pytest.mark.parametrize("flag", [0, _lib.NVFP4_NO_WAIT])
 @pytest.mark.parametrize("n, rows, cols, pairs", [
     (3, 1024, 11184, False),            # few tensors: as many workers as a section has words
     (9, 512, 7216, False),              # ragged last workgroup
@@ -43,7 +45,7 @@ def test_what_is_left_and_the_records_behind_it(n, rows, cols, pairs, dtype, fla
     for record in batch.amax_records():
         record.fill_(-1)                                # whatever was in this memory
     for run in range(3):
-        if run == 1 and flag != _lib.NVFP4_NO_WAIT | _lib.NVFP4_NO_PATIENCE:
+        if run == 1:
             batch.carry_amax(adaptive=False)            # the records serve a carried run
         if run == 2:
             x[1, 0, 0] = 1e3
@@ -58,3 +60,21 @@ def test_what_is_left_and_the_records_behind_it(n, rows, cols, pairs, dtype, fla
                     _same(one, ref, f"run {run}, tensor {i}")
             else:
                 _same(got[i], nvfp4_quantize_1d(x[i]), f"run {run}, tensor {i}")
+
+
+@pytest.mark.parametrize("first_polls", [0, 256])
+@pytest.mark.parametrize("n, rows, cols", [(1, 2048, 8192), (5, 512, 7216), (64, 3, 16384)])
+def test_workgroups_that_wait_for_nobody(n, rows, cols, first_polls):
+    """Whoever finds no word yet takes the maximum from the tensor, those behind as well: every byte as in a single call."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = (torch.randn(n, rows, cols, generator=g, device="cuda") * 0.02).bfloat16()
+    x[n // 2, 0, 3] = float("inf")
+    with launch.recording() as batch:
+        got = [nvfp4_quantize_1d(t) for t in x]
+    for one in got:
+        for t in one:
+            t.view(torch.uint8).fill_(0xA5) if t.dim() else t.fill_(-1.0)
+    stream = torch.cuda.current_stream().cuda_stream
+    _probes.check(_probes.load().mqp_nvfp4_one_pass(ctypes.byref(batch.freeze()), n, first_polls, 0, stream))
+    for i in range(n):
+        _same(got[i], nvfp4_quantize_1d(x[i]), f"tensor {i}")
