@@ -3,12 +3,15 @@
 // A call on a small tensor is bound by the host.  Written in Python, a converted matrix cost 6 us -- two allocations, the
 // record of its job as a tuple and again as a ctypes structure, the reference that keeps each tensor alive -- and a
 // straight-through node of torch.autograd.Function 41 us forward and backward, for a kernel of 3 us.  The functions here do
-// the same with the same torch calls (at::empty, the current stream, a graph node) and record or submit the same mq_job.
+// the same with the same torch calls (an allocation, the current stream, a graph node) and record or submit the same mq_job;
+// for the quantizers that converters call on every matrix, the checks and sizes as well.
 //
 // They take ordinary tensors only: of class Tensor or Parameter, dense, on the GPU, with no mode, transform, tracer or
 // forward-mode level active that would have to see the operation.  For anything else they return None (or False) and the
 // caller goes on in Python, which is where every argument is checked and every refusal is worded.
+#include <ATen/Context.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
@@ -51,6 +54,19 @@ const at::Tensor* ordinary(PyObject* o) {
 }
 hipStream_t stream_of(const at::Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 int dtype_code(at::ScalarType t) { return t == at::kBFloat16 ? MQ_BF16 : t == at::kHalf ? MQ_F16 : t == at::kFloat ? MQ_F32 : -1; }
+
+// at::empty on the device of `like`, without the dispatcher (0.3 us a call), whose modes and transforms no ordinary moment has;
+// where uninitialised memory is to be filled, that is the dispatched function's business
+at::Tensor make(at::IntArrayRef sizes, at::ScalarType dtype, const at::Tensor& like) {
+    if (at::globalContext().deterministicAlgorithms()) return at::empty(sizes, like.options().dtype(dtype).requires_grad(false));
+    return at::Tensor(at::detail::empty_cuda(sizes, dtype, like.device(), c10::nullopt));
+}
+
+// at::empty_like of a tensor whose memory is one run
+at::Tensor make_like(const at::Tensor& x) {
+    at::Tensor y = make(x.sizes(), x.scalar_type(), x);
+    return y.strides() == x.strides() ? y : at::empty_like(x);      // (dimensions of size 1 have any stride)
+}
 
 PyObject* failed() {
     PyErr_SetString(g_error ? g_error : PyExc_RuntimeError, mq_last_error());
@@ -168,12 +184,12 @@ bool integer(PyObject* o, int64_t& v) {
     PyErr_Clear();
     return false;
 }
-// Records the job or runs it; false with the error set if it is refused.
-bool place(const mq_job& job, const at::Tensor& in, const at::Tensor* const* named, int n) {
+// Records the jobs, which name `in` and `named`, or runs them; false with the error set if they are refused.
+bool place(const mq_job* jobs, size_t count, const at::Tensor& in, const at::Tensor* const* named, int n) {
     if (t_scope.recorder) {
         Recorder& r = *t_scope.recorder;
         if (r.jobs->empty() && r.device < 0) r.device = in.device().index();
-        r.jobs->push_back(job);
+        r.jobs->insert(r.jobs->end(), jobs, jobs + count);
         r.held->push_back(in);
         for (int i = 0; i < n; i++)
             if (named[i]) r.held->push_back(*named[i]);
@@ -183,7 +199,7 @@ bool place(const mq_job& job, const at::Tensor& in, const at::Tensor* const* nam
     {
         hipStream_t stream = stream_of(in);
         pybind11::gil_scoped_release no_gil;
-        rc = mq_run_jobs(&job, 1, stream);
+        rc = mq_run_jobs(jobs, (int64_t)count, stream);
     }
     if (rc != MQ_OK) failed();
     return rc == MQ_OK;
@@ -210,7 +226,7 @@ PyObject* submit(PyObject*, PyObject* const* a, Py_ssize_t n) {
     else if (!integer(a[1], v[8])) Py_RETURN_FALSE;
     const mq_job job{(int32_t)v[7], (int32_t)v[8], in->data_ptr(), data(named[0]), data(named[1]), data(named[2]), data(named[3]),
                      v[0], v[1], v[2], (int32_t)v[3], (int32_t)v[4], v[5], v[6]};
-    if (!place(job, *in, named, 4)) return nullptr;
+    if (!place(&job, 1, *in, named, 4)) return nullptr;
     Py_RETURN_TRUE;
     END_HANDLE_TH_ERRORS
 }
@@ -230,6 +246,30 @@ bool spec_of(PyObject* o, Spec& s) {
     }
     return true;
 }
+// Makes the outputs that `make` names, places the job on them (`aux_in` in the place of aux) and returns those that `kept` names.
+PyObject* made_by(mq_job job, const at::Tensor& in, const at::Tensor* aux_in, const Spec (&spec)[4], const bool (&making)[4], const bool (&kept)[4]) {
+    at::Tensor made[4];
+    {
+        pybind11::gil_scoped_release no_gil;      // (the allocator may wait for another thread)
+        for (int i = 0; i < 4; i++)
+            if (making[i]) made[i] = make(spec[i].sizes, spec[i].dtype, in);
+    }
+    const at::Tensor* named[4] = {making[0] ? &made[0] : nullptr, making[1] ? &made[1] : nullptr, aux_in ? aux_in : making[2] ? &made[2] : nullptr,
+                                  making[3] ? &made[3] : nullptr};
+    job.in = in.data_ptr();
+    job.out = data(named[0]);
+    job.scale = data(named[1]);
+    job.aux = data(named[2]);
+    job.aux2 = data(named[3]);
+    if (!place(&job, 1, in, named, 4)) return nullptr;
+    int count = 0;
+    for (int i = 0; i < 4; i++) count += kept[i];
+    Owned result = owned(PyTuple_New(count));
+    if (!result) return nullptr;
+    for (int i = 0, at = 0; i < 4; i++)
+        if (kept[i]) PyTuple_SET_ITEM(result.ptr(), at++, THPVariable_Wrap(std::move(made[i])));
+    return result.release().ptr();
+}
 // produce(kind, dtype | None, in, aux_in | None, rows, cols, ld, p0, p1, out, scale, aux, aux2) -> the tensors made, or None
 // `out` .. `aux2` are (dtype, *sizes) or None; `aux_in` is a tensor that takes the place of `aux` in the job.
 PyObject* produce(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -247,29 +287,206 @@ PyObject* produce(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (a[1] == Py_None) v[6] = dtype_code(in->scalar_type()) < 0 ? 0 : dtype_code(in->scalar_type());
     else if (!integer(a[1], v[6])) Py_RETURN_NONE;
     Spec spec[4];
-    bool make[4];
-    int count = 0;
+    bool making[4];
     for (int i = 0; i < 4; i++) {
-        make[i] = a[9 + i] != Py_None;
-        if (make[i] && !spec_of(a[9 + i], spec[i])) Py_RETURN_NONE;
-        count += make[i];
+        making[i] = a[9 + i] != Py_None;
+        if (making[i] && !spec_of(a[9 + i], spec[i])) Py_RETURN_NONE;
     }
-    at::Tensor made[4];
+    return made_by(mq_job{(int32_t)v[5], (int32_t)v[6], nullptr, nullptr, nullptr, nullptr, nullptr, v[0], v[1], v[2], (int32_t)v[3], (int32_t)v[4], 0, 0},
+                   *in, aux_in, spec, making, making);
+    END_HANDLE_TH_ERRORS
+}
+
+// ---- whole quantizers: the checks, sizes and job of one matrix ---------------------------------------------------------
+// Each takes the usual form of its argument (see `plain`) and answers None for every other one, and for whatever it would
+// have to refuse: the Python function goes on then, with the same job for what it accepts.  A recorded call, us, in
+// Python and here: block FP8 3.6 / 1.8, MXFP8 3.6 / 1.7, INT4 3.4 / 1.9, with zero points 5.5 / 3.1, FP8 back to bf16 2.4 / 1.1, most of
+// what is left its allocations; a stack of NVFP4 matrices, for each of them, 3.4 / 0.1.
+bool recordable() { return !t_scope.recording && ordinary_moment(); }
+// an ordinary tensor with elements whose memory is one run
+const at::Tensor* plain(PyObject* o) {
+    const at::Tensor* t = ordinary(o);
+    return t && t->numel() > 0 && t->is_contiguous() ? t : nullptr;
+}
+const at::Tensor* plain_weight(PyObject* o) {
+    const at::Tensor* t = plain(o);
+    return t && t->dim() > 0 && dtype_code(t->scalar_type()) >= 0 ? t : nullptr;
+}
+// an ordinary weight matrix with elements, its rows any distance apart
+const at::Tensor* weight_rows(PyObject* o) {
+    const at::Tensor* t = ordinary(o);
+    return t && t->dim() == 2 && t->numel() > 0 && t->stride(1) == 1 && dtype_code(t->scalar_type()) >= 0 ? t : nullptr;
+}
+bool positive(PyObject* o, int64_t& v) { return integer(o, v) && v > 0 && v <= 0x7FFFFFFF; }
+// the sizes of t with the last one replaced
+c10::SmallVector<int64_t, 4> sizes_to(const at::Tensor& t, int64_t last) {
+    c10::SmallVector<int64_t, 4> sizes(t.sizes().begin(), t.sizes().end());
+    sizes.back() = last;
+    return sizes;
+}
+mq_job job_of(int kind, int dtype, int64_t rows, int64_t cols, int64_t ld, int64_t p0 = 0, int64_t p1 = 0) {
+    return mq_job{kind, dtype, nullptr, nullptr, nullptr, nullptr, nullptr, rows, cols, ld, (int32_t)p0, (int32_t)p1, 0, 0};
+}
+constexpr bool kOne[4] = {true, false, false, false}, kTwo[4] = {true, true, false, false}, kThree[4] = {true, true, true, false},
+               kFour[4] = {true, true, true, true}, kPackedZeros[4] = {true, true, false, true};
+
+// block_fp8(weight, block_size)
+PyObject* block_fp8(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    const at::Tensor* w = n == 2 && recordable() ? weight_rows(a[0]) : nullptr;
+    int64_t bn, bk;
+    if (!w || !(PyList_CheckExact(a[1]) || PyTuple_CheckExact(a[1])) || PySequence_Fast_GET_SIZE(a[1]) < 2) Py_RETURN_NONE;
+    if (!positive(PySequence_Fast_GET_ITEM(a[1], 0), bn) || !positive(PySequence_Fast_GET_ITEM(a[1], 1), bk)) Py_RETURN_NONE;
+    const int64_t N = w->size(0), K = w->size(1);
+    const Spec spec[4] = {{at::kFloat8_e4m3fn, {N, K}}, {at::kFloat, {(N + bn - 1) / bn, (K + bk - 1) / bk}}};
+    return made_by(job_of(MQ_JOB_FP8_BLOCK, dtype_code(w->scalar_type()), N, K, w->stride(0), bn, bk), *w, nullptr, spec, kTwo, kTwo);
+    END_HANDLE_TH_ERRORS
+}
+// scaled_fp8(weight, per_channel, floor bits of bf16, of fp16, of fp32)
+PyObject* scaled_fp8(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    const at::Tensor* w = n == 5 && recordable() ? weight_rows(a[0]) : nullptr;
+    int64_t per_channel, floor_bits[3];
+    if (!w || !integer(a[1], per_channel)) Py_RETURN_NONE;
+    for (int i = 0; i < 3; i++)
+        if (!integer(a[2 + i], floor_bits[i])) Py_RETURN_NONE;
+    const int code = dtype_code(w->scalar_type());
+    const int64_t N = w->size(0), K = w->size(1), unit = code == MQ_F32 ? 4 : 8;
+    const bool held = per_channel && K >= unit && K <= 4096 * unit;      // rows of 16-byte units are held in registers: no workspace
+    Spec spec[4] = {{at::kFloat8_e4m3fn, {N, K}}, {at::kFloat, {1}}, {at::kInt, {N > MQ_FP8_SCALED_WORDS ? N : MQ_FP8_SCALED_WORDS}}};
+    if (per_channel) spec[1].sizes = {N, 1};
+    const int64_t bits = floor_bits[code == MQ_BF16 ? 0 : code == MQ_F16 ? 1 : 2];
+    return made_by(job_of(MQ_JOB_FP8_SCALED, code, N, K, w->stride(0), bits, per_channel != 0), *w, nullptr, spec, held ? kTwo : kThree, kTwo);
+    END_HANDLE_TH_ERRORS
+}
+// mxfp8(weight)
+PyObject* mxfp8(PyObject*, PyObject* o) {
+    HANDLE_TH_ERRORS
+    const at::Tensor* w = recordable() ? plain_weight(o) : nullptr;
+    if (!w || w->size(-1) % 32 != 0) Py_RETURN_NONE;
+    const int64_t K = w->size(-1);
+    const Spec spec[4] = {{at::kFloat8_e4m3fn, sizes_to(*w, K)}, {at::kByte, sizes_to(*w, K / 32)}};
+    return made_by(job_of(MQ_JOB_MXFP8, dtype_code(w->scalar_type()), w->numel() / K, K, K), *w, nullptr, spec, kTwo, kTwo);
+    END_HANDLE_TH_ERRORS
+}
+// mxfp4(weight, group)
+PyObject* mxfp4(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    const at::Tensor* w = n == 2 && recordable() ? plain_weight(a[0]) : nullptr;
+    int64_t group;
+    if (!w || !positive(a[1], group) || w->size(-1) % group != 0 || w->size(-1) % 2 != 0) Py_RETURN_NONE;
+    const int64_t K = w->size(-1);
+    const Spec spec[4] = {{at::kByte, sizes_to(*w, K / 2)}, {at::kByte, sizes_to(*w, K / group)}};
+    return made_by(job_of(MQ_JOB_MXFP4, dtype_code(w->scalar_type()), w->numel() / K, K, K, group), *w, nullptr, spec, kTwo, kTwo);
+    END_HANDLE_TH_ERRORS
+}
+// int4(weight, group, symmetric) -> (words, scales) or (words, scales, packed zero points)
+PyObject* int4(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    const at::Tensor* w = n == 3 && recordable() ? plain_weight(a[0]) : nullptr;
+    int64_t group;
+    if (!w || w->dim() != 2 || !positive(a[1], group) || !PyBool_Check(a[2])) Py_RETURN_NONE;
+    const bool symmetric = a[2] == Py_True;
+    const int64_t M = w->size(0), K = w->size(1), groups = K / group;
+    if (K % group != 0 || K % 8 != 0 || (!symmetric && (group % 8 != 0 || M % 8 != 0))) Py_RETURN_NONE;
+    const Spec spec[4] = {{at::kInt, {M, K / 8}}, {w->scalar_type(), {M, groups}}, {at::kByte, {M, groups}}, {at::kInt, {groups, M / 8}}};
+    return made_by(job_of(symmetric ? MQ_JOB_INT4_PACK : MQ_JOB_INT4_PACK_ASYM, dtype_code(w->scalar_type()), M, K, K, group), *w, nullptr, spec,
+                   symmetric ? kTwo : kFour, symmetric ? kTwo : kPackedZeros);
+    END_HANDLE_TH_ERRORS
+}
+// fp8_dequant(codes, scales, block) -> (values,)
+PyObject* fp8_dequant(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    const at::Tensor *x = n == 3 && recordable() ? plain(a[0]) : nullptr, *s = x ? plain(a[1]) : nullptr;
+    int64_t block;
+    if (!s || x->scalar_type() != at::kFloat8_e4m3fn || x->dim() != 2 || s->dim() != 2 || s->scalar_type() != at::kFloat || !positive(a[2], block))
+        Py_RETURN_NONE;
+    const int64_t M = x->size(0), N = x->size(1);
+    const Spec spec[4] = {{at::kBFloat16, {M, N}}};
+    return made_by(job_of(MQ_JOB_FP8_DEQUANT, 0, M, N, N, block), *x, s, spec, kOne, kOne);
+    END_HANDLE_TH_ERRORS
+}
+// mxfp4_dequant(codes, scales, group) -> (values,)
+PyObject* mxfp4_dequant(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    const at::Tensor *x = n == 3 && recordable() ? plain(a[0]) : nullptr, *s = x ? plain(a[1]) : nullptr;
+    int64_t group;
+    if (!s || x->dim() == 0 || x->scalar_type() != at::kByte || s->scalar_type() != at::kByte || s->device() != x->device() || !positive(a[2], group))
+        Py_RETURN_NONE;
+    const int64_t numel = x->numel() * 2;
+    if (numel % group != 0 || s->numel() != numel / group) Py_RETURN_NONE;
+    const Spec spec[4] = {{at::kBFloat16, sizes_to(*x, x->size(-1) * 2)}};
+    return made_by(job_of(MQ_JOB_MXFP4_DEQUANT, 0, 1, numel, numel, group), *x, s, spec, kOne, kOne);
+    END_HANDLE_TH_ERRORS
+}
+// fp8_to_mxfp8(codes, tile scales)
+PyObject* fp8_to_mxfp8(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    const at::Tensor *x = n == 2 && recordable() ? plain(a[0]) : nullptr, *s = x ? plain(a[1]) : nullptr;
+    if (!s || x->dim() != 2 || s->dim() != 2 || s->scalar_type() != at::kFloat || (x->scalar_type() != at::kFloat8_e4m3fn && x->scalar_type() != at::kByte))
+        Py_RETURN_NONE;
+    const int64_t N = x->size(0), K = x->size(1);
+    if (K % 32 != 0 || s->size(0) < (N + 127) / 128 || s->size(1) < (K + 127) / 128) Py_RETURN_NONE;
+    const Spec spec[4] = {{at::kFloat8_e4m3fn, {N, K}}, {at::kByte, {N, K / 32}}};
+    return made_by(job_of(MQ_JOB_FP8_TO_MXFP8, 0, N, K, s->size(1)), *x, s, spec, kTwo, kTwo);
+    END_HANDLE_TH_ERRORS
+}
+// mxfp4_to_fp8(codes, scale bytes)
+PyObject* mxfp4_to_fp8(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    const at::Tensor *x = n == 2 && recordable() ? plain(a[0]) : nullptr, *s = x ? plain(a[1]) : nullptr;
+    if (!s || x->dim() != 2 || s->dim() != 2 || x->scalar_type() != at::kChar || s->element_size() != 1 || (uintptr_t)x->data_ptr() % 16 != 0)
+        Py_RETURN_NONE;
+    const int64_t M = x->size(0), K = x->size(1) * 2;
+    if (M % 128 != 0 || K % 128 != 0 || s->size(0) != M || s->size(1) != K / 32) Py_RETURN_NONE;
+    const Spec spec[4] = {{at::kFloat8_e4m3fn, {M, K}}, {at::kFloat, {M / 128, K / 128}}};
+    return made_by(job_of(MQ_JOB_MXFP4_TO_FP8, 0, M, K, K), *x, s, spec, kTwo, kTwo);
+    END_HANDLE_TH_ERRORS
+}
+// int4_unpack(words, scales, (rows, columns), group) -> (values,)
+PyObject* int4_unpack(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    const at::Tensor *x = n == 4 && recordable() ? plain(a[0]) : nullptr, *s = x ? plain(a[1]) : nullptr;
+    int64_t M, K, group;
+    if (!s || x->dim() != 2 || x->scalar_type() != at::kInt || dtype_code(s->scalar_type()) < 0 || s->dim() == 0) Py_RETURN_NONE;
+    if (!PyTuple_CheckExact(a[2]) || PyTuple_GET_SIZE(a[2]) != 2 || !positive(PyTuple_GET_ITEM(a[2], 0), M) || !positive(PyTuple_GET_ITEM(a[2], 1), K) ||
+        !positive(a[3], group))
+        Py_RETURN_NONE;
+    if (x->size(0) != M || x->size(1) != (K + 7) / 8 || K % group != 0 || s->numel() != M * (K / group)) Py_RETURN_NONE;
+    const Spec spec[4] = {{at::kBFloat16, {M, K}}};
+    return made_by(job_of(MQ_JOB_INT4_UNPACK, dtype_code(s->scalar_type()), M, K, K, group), *x, s, spec, kOne, kOne);
+    END_HANDLE_TH_ERRORS
+}
+// nvfp4_stack(weights [n, M, K], e4m3_max, flags, words of a record) -> (codes, block scales, global scales): a job for each
+// matrix, all in one list
+PyObject* nvfp4_stack(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    const at::Tensor* w = n == 4 && recordable() ? plain_weight(a[0]) : nullptr;
+    int64_t e4m3_max, flags, words;
+    if (!w || w->dim() != 3 || w->size(2) % 16 != 0 || !integer(a[1], e4m3_max) || !integer(a[2], flags) || !positive(a[3], words)) Py_RETURN_NONE;
+    const int64_t count = w->size(0), M = w->size(1), K = w->size(2);
+    at::Tensor q, s, g, records;
+    std::vector<mq_job> jobs;
     {
-        pybind11::gil_scoped_release no_gil;      // (the allocator may wait for another thread)
-        for (int i = 0; i < 4; i++)
-            if (make[i]) made[i] = at::empty(spec[i].sizes, in->options().dtype(spec[i].dtype).requires_grad(false));
+        pybind11::gil_scoped_release no_gil;
+        q = make({count, M, K / 2}, at::kByte, *w);
+        s = make({count, M, K / 16}, at::kFloat8_e4m3fn, *w);
+        g = make({count}, at::kFloat, *w);
+        records = make({count, words}, at::kInt, *w);
+        jobs.reserve((size_t)count);
+        for (int64_t i = 0; i < count; i++) {
+            mq_job job = job_of(MQ_JOB_NVFP4, dtype_code(w->scalar_type()), M, K, K, e4m3_max, flags);
+            job.in = (const char*)w->data_ptr() + i * M * K * w->element_size();
+            job.out = (char*)q.data_ptr() + i * M * (K / 2);
+            job.scale = (char*)s.data_ptr() + i * M * (K / 16);
+            job.aux = (char*)records.data_ptr() + i * words * 4;
+            job.aux2 = (char*)g.data_ptr() + i * 4;
+            jobs.push_back(job);
+        }
     }
-    const at::Tensor* named[4] = {make[0] ? &made[0] : nullptr, make[1] ? &made[1] : nullptr, aux_in ? aux_in : make[2] ? &made[2] : nullptr,
-                                  make[3] ? &made[3] : nullptr};
-    const mq_job job{(int32_t)v[5], (int32_t)v[6], in->data_ptr(), data(named[0]), data(named[1]), data(named[2]), data(named[3]),
-                     v[0], v[1], v[2], (int32_t)v[3], (int32_t)v[4], 0, 0};
-    if (!place(job, *in, named, 4)) return nullptr;
-    Owned result = owned(PyTuple_New(count));
-    if (!result) return nullptr;
-    for (int i = 0, at = 0; i < 4; i++)
-        if (make[i]) PyTuple_SET_ITEM(result.ptr(), at++, THPVariable_Wrap(std::move(made[i])));
-    return result.release().ptr();
+    const at::Tensor* const named[4] = {&q, &s, &records, &g};
+    if (!place(jobs.data(), jobs.size(), *w, named, 4)) return nullptr;
+    return Py_BuildValue("(NNN)", THPVariable_Wrap(std::move(q)), THPVariable_Wrap(std::move(s)), THPVariable_Wrap(std::move(g)));
     END_HANDLE_TH_ERRORS
 }
 
@@ -291,9 +508,8 @@ PyObject* act_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
     int rc;
     {
         pybind11::gil_scoped_release no_gil;
-        const auto options = x->options().requires_grad(false);
-        s = at::empty(sizes, options.dtype(((THPDtype*)a[3])->scalar_type));
-        y = at::empty(x->sizes(), options.dtype(at::kFloat8_e4m3fn));
+        s = make(sizes, ((THPDtype*)a[3])->scalar_type, *x);
+        y = make(x->sizes(), at::kFloat8_e4m3fn, *x);
         rc = mq_fp8_act_quant(x->data_ptr(), dtype_code(x->scalar_type()), y.data_ptr(), s.data_ptr(), x->numel(), (int)block, (int)flags, stream_of(*x));
     }
     if (rc != MQ_OK) return failed();
@@ -330,7 +546,7 @@ PyObject* fake_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
     {
         pybind11::gil_scoped_release no_gil;
         at::NoGradGuard no_grad;
-        y = at::empty_like(*x);
+        y = make_like(*x);
         rc = mq_fake_quant(x->data_ptr(), dtype_code(x->scalar_type()), y.data_ptr(), x->numel(), (int)mode, stream_of(*x));
     }
     if (rc != MQ_OK) return failed();
@@ -353,8 +569,8 @@ PyObject* simulate(PyObject*, PyObject* const* a, Py_ssize_t n) {
     {
         pybind11::gil_scoped_release no_gil;
         at::NoGradGuard no_grad;
-        y = at::empty_like(*x);
-        const at::Tensor s = at::empty(sizes, x->options().dtype(at::kFloat).requires_grad(false));
+        y = make_like(*x);
+        const at::Tensor s = make(sizes, at::kFloat, *x);
         rc = mq_fp8_act_quant(x->data_ptr(), dtype_code(x->scalar_type()), y.data_ptr(), s.data_ptr(), x->numel(), (int)block, (int)flags, stream_of(*x));
     }
     if (rc != MQ_OK) return failed();
@@ -387,10 +603,10 @@ PyObject* nvfp4_images(PyObject*, PyObject* const* a, Py_ssize_t n) {
         images.reserve(weights.size());
         items.reserve(weights.size());
         for (const at::Tensor& w : weights) {
-            images.push_back(at::empty_like(w));
+            images.push_back(make_like(w));
             items.push_back(mq_fake_quant_item{w.data_ptr(), images.back().data_ptr(), w.numel()});
         }
-        const at::Tensor partials = at::empty({(int64_t)weights.size() * words}, weights[0].options().dtype(at::kInt).requires_grad(false));
+        const at::Tensor partials = make({(int64_t)weights.size() * words}, at::kInt, weights[0]);
         rc = mq_nvfp4_fake_quant(items.data(), (int64_t)items.size(), dtype_code(weights[0].scalar_type()), partials.data_ptr(), (int)e4m3_max,
                                  (int)flags, stream_of(weights[0]));
     }
@@ -417,9 +633,9 @@ PyObject* int4_fake(PyObject*, PyObject* const* a, Py_ssize_t n) {
         pybind11::gil_scoped_release no_gil;
         at::NoGradGuard no_grad;
         const int64_t M = x->size(0), N = x->size(1);
-        y = at::empty_like(*x);
-        s = at::empty({(M + bm - 1) / bm, (N + bn - 1) / bn}, x->options().requires_grad(false));
-        z = at::empty_like(s);
+        y = make_like(*x);
+        s = make({(M + bm - 1) / bm, (N + bn - 1) / bn}, x->scalar_type(), *x);
+        z = make(s.sizes(), x->scalar_type(), *x);
         rc = mq_int4_fake_quant(x->data_ptr(), dtype_code(x->scalar_type()), y.data_ptr(), s.data_ptr(), z.data_ptr(), M, N, (int)bm, (int)bn,
                                 (int)sym, stream_of(*x));
     }
@@ -442,6 +658,17 @@ PyMethodDef methods[] = {{"set_error", set_error, METH_O, nullptr},
                          {"leave", scope_leave, METH_NOARGS, nullptr},
                          {"submit", (PyCFunction)(void*)submit, METH_FASTCALL, nullptr},
                          {"produce", (PyCFunction)(void*)produce, METH_FASTCALL, nullptr},
+                         {"block_fp8", (PyCFunction)(void*)block_fp8, METH_FASTCALL, nullptr},
+                         {"scaled_fp8", (PyCFunction)(void*)scaled_fp8, METH_FASTCALL, nullptr},
+                         {"mxfp8", mxfp8, METH_O, nullptr},
+                         {"mxfp4", (PyCFunction)(void*)mxfp4, METH_FASTCALL, nullptr},
+                         {"int4", (PyCFunction)(void*)int4, METH_FASTCALL, nullptr},
+                         {"fp8_dequant", (PyCFunction)(void*)fp8_dequant, METH_FASTCALL, nullptr},
+                         {"mxfp4_dequant", (PyCFunction)(void*)mxfp4_dequant, METH_FASTCALL, nullptr},
+                         {"fp8_to_mxfp8", (PyCFunction)(void*)fp8_to_mxfp8, METH_FASTCALL, nullptr},
+                         {"mxfp4_to_fp8", (PyCFunction)(void*)mxfp4_to_fp8, METH_FASTCALL, nullptr},
+                         {"int4_unpack", (PyCFunction)(void*)int4_unpack, METH_FASTCALL, nullptr},
+                         {"nvfp4_stack", (PyCFunction)(void*)nvfp4_stack, METH_FASTCALL, nullptr},
                          {"act_quant", (PyCFunction)(void*)act_quant, METH_FASTCALL, nullptr},
                          {"fake_quant", (PyCFunction)(void*)fake_quant, METH_FASTCALL, nullptr},
                          {"simulate", (PyCFunction)(void*)simulate, METH_FASTCALL, nullptr},

@@ -52,6 +52,9 @@ def pack_layer(weight: torch.Tensor, group_size: int, sym: bool = True):
     and the scales directly.  With sym=False the third result is the AWQ-ordered int32 [K/group_size, M/8]
     zero-point tensor; with sym=True it is None.
     """
+    made = native.int4(weight, group_size, sym)
+    if made is not None:
+        return (*made, None) if sym else made
     _lib.require_gpu(weight, "pack_layer")
     if weight.dim() != 2:
         raise RuntimeError("Input must be 2D")

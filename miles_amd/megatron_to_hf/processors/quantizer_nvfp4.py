@@ -12,7 +12,8 @@ import re
 
 import torch
 
-from miles_amd.utils.nvfp4 import NVFP4_GROUP_SIZE, nvfp4_quantize_1d, nvfp4_quantize_1d_pair, stack_slices
+from miles_amd._host import native
+from miles_amd.utils.nvfp4 import AMAX_RECORD_WORDS, NVFP4_GROUP_SIZE, _quantizer_options, nvfp4_quantize_1d, nvfp4_quantize_1d_pair, stack_slices
 
 from ._names import in_bf16_head_or_tail, named_in_extra_high_precision, parse_layer_param
 
@@ -145,6 +146,10 @@ def quantize_nvfp4(weight: torch.Tensor):
         n, rows, cols = weight.shape
         if cols % NVFP4_GROUP_SIZE:
             raise ValueError(f"NVFP4 requires K divisible by {NVFP4_GROUP_SIZE}, got {cols}.")
+        if n:
+            made = native.nvfp4_stack(weight, *_quantizer_options(), AMAX_RECORD_WORDS)
+            if made is not None:
+                return made
         codes = torch.empty((n, rows, cols // 2), dtype=torch.uint8, device=weight.device)
         block_scale = torch.empty((n, rows, cols // NVFP4_GROUP_SIZE), dtype=torch.float8_e4m3fn, device=weight.device)
         global_scale = torch.empty((n,), dtype=torch.float32, device=weight.device)

@@ -18,6 +18,7 @@ from concurrent.futures import ThreadPoolExecutor
 import torch
 
 from miles_amd import _lib, launch
+from miles_amd._host import native
 from miles_amd.tools import _checkpoint as ckpt
 
 FP8_INFO = torch.finfo(torch.float8_e4m3fn)
@@ -34,6 +35,9 @@ def block_fp8(weight: torch.Tensor, block_size):
     Per (zero-padded) tile: scale = amax / 448 with a true division, q = e4m3(clamp(w / scale, +-448)).
     An all-zero tile keeps the reference's CPU result: scale 0 and every byte 0xFF.
     """
+    made = native.block_fp8(weight, block_size)
+    if made is not None:
+        return made
     _lib.require_gpu(weight, "block_fp8")
     bn, bk = int(block_size[0]), int(block_size[1])
     n, k = weight.shape
@@ -46,10 +50,14 @@ def block_fp8(weight: torch.Tensor, block_size):
 # clamp(min=1e-12) acts in the weight dtype (fp16 has no such value): the fp32 bit pattern of that floor
 _FLOORS = {dtype: int(torch.tensor(1e-12, dtype=dtype).float().view(torch.int32))
            for dtype in (torch.bfloat16, torch.float16, torch.float32)}
+_FLOOR_BITS = tuple(_FLOORS.values())
 _AMAX_RECORD_WORDS = 1280   # MQ_NVFP4_RECORD_WORDS: partial maxima of a tensor on the device, then its folded amax
 
 
 def _scaled_fp8(weight: torch.Tensor, per_channel: bool):
+    made = native.scaled_fp8(weight, per_channel, *_FLOOR_BITS)
+    if made is not None:
+        return made
     _lib.require_gpu(weight, "channel_fp8" if per_channel else "tensor_fp8")
     n, k = weight.shape
     # the reference reduces with weight.abs().max() / .amax(dim=1): torch refuses a reduction over nothing

@@ -21,6 +21,7 @@ import torch
 from safetensors.torch import safe_open, save_file
 
 from miles_amd import _lib, launch
+from miles_amd._host import native
 
 
 def _load_config(model_dir: str, config_path: str | None) -> tuple[int, int, int]:
@@ -34,6 +35,10 @@ def _load_config(model_dir: str, config_path: str | None) -> tuple[int, int, int
 
 def _dequantize_tensor(weight_packed: torch.Tensor, weight_scale: torch.Tensor, weight_shape, group_size: int) -> torch.Tensor:
     """int32 [M, ceil(K/8)] codes + [M, K/group_size] scales -> bfloat16 [M, K] = bf16((code - 8) * f32(scale))."""
+    # a job of the batched driver: inside `launch.deferred()` the experts of a whole shard share grouped launches
+    made = native.int4_unpack(weight_packed, weight_scale, weight_shape, group_size)
+    if made is not None:
+        return made[0]
     if isinstance(weight_shape, torch.Tensor):
         shape = tuple(int(v) for v in weight_shape.view(-1).tolist())
     else:
@@ -52,7 +57,6 @@ def _dequantize_tensor(weight_packed: torch.Tensor, weight_scale: torch.Tensor, 
         scale = scale.unsqueeze(1)
     if K % group_size != 0 or scale.numel() != M * (K // group_size):
         raise ValueError(f"Scale shape {tuple(scale.shape)} incompatible with weight shape {shape}")
-    # a job of the batched driver: inside `launch.deferred()` the experts of a whole shard share grouped launches
     return launch.produce(_lib.JOB_INT4_UNPACK, packed, M, K, K, int(group_size), 0, (torch.bfloat16, M, K), aux_in=scale,
                           dtype=_lib.dtype_code(scale, "_dequantize_tensor"))[0]
 

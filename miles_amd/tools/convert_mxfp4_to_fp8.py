@@ -22,11 +22,16 @@ from safetensors import safe_open
 from safetensors.torch import load_file, save_file
 
 from miles_amd import _lib, launch
+from miles_amd._host import native
 
 
 def cast_e2m1fn_to_e4m3fn(x: torch.Tensor, scale: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """int8 [out, in/2] (two e2m1 codes per byte, even element low) + E8M0 scales [out, in/32]
     -> (float8_e4m3fn [out, in], float32 [out/128, in/128])."""
+    # a job of the batched driver: inside `launch.deferred()` the casts of a whole shard share grouped launches
+    made = native.mxfp4_to_fp8(x, scale)
+    if made is not None:
+        return made
     assert x.dtype == torch.int8 and x.ndim == 2
     out_dim, in_dim = x.size(0), x.size(1) * 2
     assert out_dim % 128 == 0 and in_dim % 128 == 0
@@ -37,7 +42,6 @@ def cast_e2m1fn_to_e4m3fn(x: torch.Tensor, scale: torch.Tensor) -> tuple[torch.T
     packed, sbytes = x.contiguous(), scale.contiguous().view(torch.uint8)
     if packed.data_ptr() % 16:        # the kernel reads whole 16-byte pieces: a view that starts mid-allocation is moved first
         packed = packed.clone()
-    # a job of the batched driver: inside `launch.deferred()` the casts of a whole shard share grouped launches
     return launch.produce(_lib.JOB_MXFP4_TO_FP8, packed, out_dim, in_dim, in_dim, 0, 0, (torch.float8_e4m3fn, out_dim, in_dim),
                           (torch.float32, out_dim // 128, in_dim // 128), aux_in=sbytes)
 

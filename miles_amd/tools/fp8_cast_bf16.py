@@ -19,6 +19,7 @@ import torch
 from safetensors.torch import load_file, save_file
 
 from miles_amd import _lib, launch
+from miles_amd._host import native
 
 
 def weight_dequant(x: torch.Tensor, s: torch.Tensor, block_size: int = 128) -> torch.Tensor:
@@ -27,6 +28,9 @@ def weight_dequant(x: torch.Tensor, s: torch.Tensor, block_size: int = 128) -> t
     The reference allocates the output in the default dtype, which its tool sets to bfloat16 before the
     first call (tools/fp8_cast_bf16.py:44); this function always writes bfloat16.
     """
+    made = native.fp8_dequant(x, s, block_size)
+    if made is not None:
+        return made[0]
     assert x.is_contiguous() and s.is_contiguous()
     assert x.dim() == 2 and s.dim() == 2
     _lib.require_gpu(x, "weight_dequant")

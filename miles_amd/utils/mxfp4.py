@@ -10,12 +10,16 @@ from __future__ import annotations
 import torch
 
 from miles_amd import _lib, launch
+from miles_amd._host import native
 
 _E2M1_VALUES = (0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0)
 
 
 def quantize_mxfp4(weight: torch.Tensor, group_size: int):
     """weight [..., K] -> (uint8 [..., K/2], two codes per byte, even element low; uint8 E8M0 [..., K/group_size])."""
+    made = native.mxfp4(weight, group_size)
+    if made is not None:
+        return made
     assert weight.shape[-1] % group_size == 0
     assert weight.shape[-1] % 2 == 0
     _lib.require_gpu(weight, "quantize_mxfp4")
@@ -29,6 +33,10 @@ def quantize_mxfp4(weight: torch.Tensor, group_size: int):
 
 def dequantize_mxfp4(weight_packed: torch.Tensor, weight_scale: torch.Tensor, group_size: int) -> torch.Tensor:
     """(uint8 [..., K/2], uint8 E8M0 scales, group_size) -> bfloat16 [..., K]."""
+    # a job of the batched driver: inside `launch.deferred()` the tensors of a whole shard share grouped launches
+    made = native.mxfp4_dequant(weight_packed, weight_scale, group_size)
+    if made is not None:
+        return made[0]
     assert weight_packed.dtype == torch.uint8
     assert weight_scale.dtype == torch.uint8
     assert group_size > 0
@@ -43,5 +51,4 @@ def dequantize_mxfp4(weight_packed: torch.Tensor, weight_scale: torch.Tensor, gr
     sizes = (*packed.shape[:-1], packed.shape[-1] * 2)
     if not numel:
         return torch.empty(sizes, dtype=torch.bfloat16, device=packed.device)
-    # a job of the batched driver: inside `launch.deferred()` the tensors of a whole shard share grouped launches
     return launch.produce(_lib.JOB_MXFP4_DEQUANT, packed, 1, numel, numel, int(group_size), 0, (torch.bfloat16, *sizes), aux_in=scale)[0]

@@ -11,6 +11,7 @@ from __future__ import annotations
 import torch
 
 from miles_amd import _lib, launch
+from miles_amd._host import native
 
 MXFP8_GROUP_SIZE = 32
 
@@ -42,6 +43,9 @@ def should_use_mxfp8(name: str, shape: tuple[int, ...], dtype: torch.dtype, *,
 
 def mxfp8_quantize(weight: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """weight [..., K] -> (float8_e4m3fn, same shape; uint8 E8M0 scales [..., K/32], compact, unswizzled)."""
+    made = native.mxfp8(weight)
+    if made is not None:
+        return made
     k = weight.shape[-1]
     if k % MXFP8_GROUP_SIZE != 0:
         raise ValueError(f"Last dim {k} must be divisible by {MXFP8_GROUP_SIZE} for MXFP8.")
@@ -135,6 +139,9 @@ def requantize_fp8_block_to_mxfp8(weight: torch.Tensor, scale: torch.Tensor) -> 
     """FP8 codes [..., N, K] with fp32 128x128 tile scales -> (float8_e4m3fn [..., N, K], uint8 [..., N, K/32]): the
     result of `mxfp8_quantize(block_quant_dequant(weight, scale, [128, 128], torch.float32))` (:187-190) without the fp32
     tensor ever reaching memory."""
+    made = native.fp8_to_mxfp8(weight, scale)
+    if made is not None:
+        return made
     k = weight.shape[-1]
     if k % MXFP8_GROUP_SIZE != 0:
         raise ValueError(f"Last dim {k} must be divisible by {MXFP8_GROUP_SIZE} for MXFP8.")
@@ -144,7 +151,6 @@ def requantize_fp8_block_to_mxfp8(weight: torch.Tensor, scale: torch.Tensor) -> 
         raise ValueError(f"expected fp32 tile scales, got {scale.dtype}")
     n = _check_grid(weight, scale)[0]
     if weight.dim() == 2 and weight.is_contiguous() and scale.is_contiguous() and weight.numel() > 0:
-        # one matrix as a checkpoint holds it: none of the views below, which take the host longer than the GPU needs
         return launch.produce(_lib.JOB_FP8_TO_MXFP8, weight, n, k, scale.shape[1], 0, 0, (torch.float8_e4m3fn, n, k),
                               (torch.uint8, n, k // MXFP8_GROUP_SIZE), aux_in=scale)
     q = torch.empty(weight.shape, dtype=torch.float8_e4m3fn, device=weight.device)
