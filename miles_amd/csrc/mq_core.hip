@@ -4,6 +4,7 @@
 
 #include "mq_api_internal.hpp"
 #include "mq_common.hpp"
+#include "mq_copy.hpp"
 #include "mq_group.hpp"
 
 static thread_local char g_err[256] = "";
@@ -38,38 +39,6 @@ __global__ void fill_u32_n_kernel(uint32_t* p, uint32_t v, int64_t n) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (; i < n; i += stride) p[i] = v;
-}
-// Grouped byte copies: a workgroup moves one 16 KiB chunk (four 16-byte units per lane) of one of the launch's runs.
-// Runs whose pointers are 16-byte aligned use 16-byte accesses, the bytes behind the last whole unit a lane each; the others
-// go byte by byte.  The runs of a sync are mostly records of a few bytes, where the launch is bound by its chain of memory
-// round trips (descriptor, source): with the tail in one lane's loop, a byte after the other, 18 records of 8 bytes took
-// 4.4 us, now 3.2.
-constexpr int kCopyUnits = 4;
-constexpr int kCopyChunk = kCopyUnits * 4096;
-__device__ __forceinline__ void copy_chunk(const CopyJob& job, const int32_t local) {
-    const int32_t row = local / job.chunks_per_row;
-    const int64_t off0 = (int64_t)(local - row * job.chunks_per_row) * kCopyChunk, bytes = job.bytes;
-    const uint8_t* __restrict__ src = (const uint8_t*)load_global_ptr(&job.src) + row * job.src_pitch;
-    uint8_t* __restrict__ dst = (uint8_t*)load_global_ptr(&job.dst) + row * job.dst_pitch;
-    const bool aligned = (((uintptr_t)src | (uintptr_t)dst) & 15) == 0;
-    const int64_t stop = off0 + kCopyChunk < bytes ? off0 + kCopyChunk : bytes;
-    if (aligned) {
-        u32x4 v[kCopyUnits];
-#pragma unroll
-        for (int u = 0; u < kCopyUnits; u++) {
-            const int64_t o = off0 + (u * 256 + threadIdx.x) * 16;
-            if (o + 16 <= stop) v[u] = ld16(src + o);
-        }
-        const int64_t tail = stop & ~(int64_t)15;       // a chunk starts at a whole unit
-        if (tail + threadIdx.x < stop) dst[tail + threadIdx.x] = src[tail + threadIdx.x];
-#pragma unroll
-        for (int u = 0; u < kCopyUnits; u++) {
-            const int64_t o = off0 + (u * 256 + threadIdx.x) * 16;
-            if (o + 16 <= stop) st16(dst + o, v[u]);
-        }
-    } else {
-        for (int64_t b = off0 + threadIdx.x; b < stop; b += 256) dst[b] = src[b];
-    }
 }
 __global__ __launch_bounds__(256) void copy_group_kernel(const CopyTable tab) {
     const JobRef r = find_job(tab, blockIdx.x);

@@ -19,6 +19,7 @@
 // exactly rounded) and rint + the +8 offset are one fp32 add of 1.5*2^23 + 8.
 #include "mq_api_internal.hpp"
 #include "mq_common.hpp"
+#include "mq_copy.hpp"
 #include "mq_group.hpp"
 #include "mq_io8.hpp"
 
@@ -94,10 +95,11 @@ __device__ __forceinline__ void int4_pack_chain_unit(const u32x4 v, const int64_
 // tensor's dtype being the identity on the codes: proved for bf16 scales, and checked over every fp16 scale from the
 // floor fp16(1e-5) up (all 31 576 patterns x the fifteen codes): it fails only where 7 x scale overflows, which needs a
 // group maximum of 65504, the largest fp16.
-template <int LANES, class Table, int F16>
-__global__ __launch_bounds__(kI4Threads) void int4_pack_bf16_kernel(const Table tab) {
+template <int LANES, class Table, int F16, class R>
+__global__ __launch_bounds__(kI4Threads) void int4_pack_bf16_kernel(const Table tab, const R riders) {
+    if (ride_along(riders)) return;
     constexpr uint32_t kTopBits = F16 ? 0x7BFFu : 0x7F7Fu;      // the largest finite value; infinities and NaN lie above
-    const FlatJob& job = flat_job(tab);
+    const FlatJob& job = flat_job_at(tab, tensor_row(riders));
     const uint16_t* __restrict__ w = (const uint16_t*)job.w;
     uint32_t* __restrict__ packed = (uint32_t*)job.q;
     uint16_t* __restrict__ scale = (uint16_t*)job.s;
@@ -180,9 +182,10 @@ __device__ __forceinline__ uint32_t seg_max32(uint32_t v) {
     v = group_max16(v);
     return umax(v, (uint32_t)__shfl_xor((int)v, 16, 64));
 }
-template <int LANES, class Table>
-__global__ __launch_bounds__(kI4Threads) void int4_pack_f32_kernel(const Table tab) {
-    const FlatJob job = flat_job(tab);
+template <int LANES, class Table, class R>
+__global__ __launch_bounds__(kI4Threads) void int4_pack_f32_kernel(const Table tab, const R riders) {
+    if (ride_along(riders)) return;
+    const FlatJob job = flat_job_at(tab, tensor_row(riders));
     const uint32_t t = threadIdx.x;
     constexpr uint32_t kPerBlock = kI4Threads * kI4F32Loads;
     const int64_t base = flat_block(tab) * kPerBlock, total = job.units * 2;
@@ -769,10 +772,11 @@ __global__ __launch_bounds__(256) void int4_zero_pack_kernel(const uint8_t* __re
     int4_zero_pack_tile(zero, packed_zp, rows8, groups_per_row, blockIdx.x, lds);
 }
 // the zero points of a group of tensors (descriptors as for int4_pack_asym_bf16_kernel): blockIdx.y selects the tensor
-template <class Table>
-__global__ __launch_bounds__(256) void int4_zero_pack_group_kernel(const Table tab) {
+template <class Table, class R>
+__global__ __launch_bounds__(256) void int4_zero_pack_group_kernel(const Table tab, const R riders) {
+    if (ride_along(riders)) return;
     __shared__ uint32_t lds[kZpCols * kZpPitch];
-    const FlatJob job = flat_job(tab);
+    const FlatJob job = flat_job_at(tab, tensor_row(riders));
     const int64_t rows8 = job.pad;
     const uint32_t groups_per_row = (uint32_t)job.section;
     if (job.section <= 0 || blockIdx.x >= int4_zero_tiles(rows8, groups_per_row)) return;
@@ -988,37 +992,37 @@ bool mq_int4_pack_fast_ok(const void* w, int dtype, int group) {
 // 8-element units a workgroup of the symmetric packers covers
 static int64_t int4_pack_units(int dtype) { return dtype == MQ_F32 ? kI4Threads * kI4F32Loads / 2 : kI4Threads * kI4Unroll; }
 
-template <class Table>
-static void int4_pack_launch(int dtype, int group, dim3 grid, hipStream_t st, const Table& tab) {
+template <class Table, class R>
+static void int4_pack_launch(int dtype, int group, dim3 grid, hipStream_t st, const Table& tab, const R& riders) {
     const dim3 blk(kI4Threads);
     if (dtype == MQ_F32) {
-        if (group == 128) hipLaunchKernelGGL((int4_pack_f32_kernel<32, Table>), grid, blk, 0, st, tab);
-        else if (group == 64) hipLaunchKernelGGL((int4_pack_f32_kernel<16, Table>), grid, blk, 0, st, tab);
-        else hipLaunchKernelGGL((int4_pack_f32_kernel<8, Table>), grid, blk, 0, st, tab);
+        if (group == 128) hipLaunchKernelGGL((int4_pack_f32_kernel<32, Table, R>), grid, blk, 0, st, tab, riders);
+        else if (group == 64) hipLaunchKernelGGL((int4_pack_f32_kernel<16, Table, R>), grid, blk, 0, st, tab, riders);
+        else hipLaunchKernelGGL((int4_pack_f32_kernel<8, Table, R>), grid, blk, 0, st, tab, riders);
     } else if (dtype == MQ_F16) {
-        if (group == 128) hipLaunchKernelGGL((int4_pack_bf16_kernel<16, Table, 1>), grid, blk, 0, st, tab);
-        else if (group == 64) hipLaunchKernelGGL((int4_pack_bf16_kernel<8, Table, 1>), grid, blk, 0, st, tab);
-        else hipLaunchKernelGGL((int4_pack_bf16_kernel<4, Table, 1>), grid, blk, 0, st, tab);
+        if (group == 128) hipLaunchKernelGGL((int4_pack_bf16_kernel<16, Table, 1, R>), grid, blk, 0, st, tab, riders);
+        else if (group == 64) hipLaunchKernelGGL((int4_pack_bf16_kernel<8, Table, 1, R>), grid, blk, 0, st, tab, riders);
+        else hipLaunchKernelGGL((int4_pack_bf16_kernel<4, Table, 1, R>), grid, blk, 0, st, tab, riders);
     } else {
-        if (group == 128) hipLaunchKernelGGL((int4_pack_bf16_kernel<16, Table, 0>), grid, blk, 0, st, tab);
-        else if (group == 64) hipLaunchKernelGGL((int4_pack_bf16_kernel<8, Table, 0>), grid, blk, 0, st, tab);
-        else hipLaunchKernelGGL((int4_pack_bf16_kernel<4, Table, 0>), grid, blk, 0, st, tab);
+        if (group == 128) hipLaunchKernelGGL((int4_pack_bf16_kernel<16, Table, 0, R>), grid, blk, 0, st, tab, riders);
+        else if (group == 64) hipLaunchKernelGGL((int4_pack_bf16_kernel<8, Table, 0, R>), grid, blk, 0, st, tab, riders);
+        else hipLaunchKernelGGL((int4_pack_bf16_kernel<4, Table, 0, R>), grid, blk, 0, st, tab, riders);
     }
 }
 
 // every tensor of a launch has the one dtype
-int mq_int4_pack_launch_group(int dtype, FlatTable& tab, int group, hipStream_t st) {
+int mq_int4_pack_launch_group(int dtype, FlatTable& tab, int group, const RiderArgs& riders, hipStream_t st) {
     if (!flat_grid(tab, int4_pack_units(dtype))) return mq_fail(MQ_ERR_ARG, "tensor too large");
     if (tab.max_blocks == 0) return MQ_OK;
-    int4_pack_launch(dtype, group, dim3((unsigned)tab.max_blocks, (unsigned)tab.n), st, tab);
+    with_riders(riders, tab.n, tab.max_blocks, [&](unsigned rows, const auto& r) { int4_pack_launch(dtype, group, dim3((unsigned)tab.max_blocks, rows), st, tab, r); });
     return mq_check_launch("int4 pack");
 }
 
-int mq_int4_pack_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int group, hipStream_t st) {
+int mq_int4_pack_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int group, const RiderArgs& riders, hipStream_t st) {
     FlatRef ref{device_jobs, 0, 0};
     if (!flat_grid(ref, max_units, int4_pack_units(dtype))) return mq_fail(MQ_ERR_ARG, "tensor too large");
     if (ref.max_blocks == 0 || n == 0) return MQ_OK;
-    int4_pack_launch(dtype, group, dim3((unsigned)ref.max_blocks, (unsigned)n), st, ref);
+    with_riders(riders, n, ref.max_blocks, [&](unsigned rows, const auto& r) { int4_pack_launch(dtype, group, dim3((unsigned)ref.max_blocks, rows), st, ref, r); });
     return mq_check_launch("int4 pack");
 }
 
@@ -1034,7 +1038,7 @@ extern "C" int mq_int4_group_quant_pack(const void* w, int dtype, int32_t* packe
         FlatTable tab{};
         tab.n = 1;
         tab.job[0] = FlatJob{w, packed, scale, nullptr, units, nullptr, 0, 0};
-        return mq_int4_pack_launch_group(dtype, tab, group, st);
+        return mq_int4_pack_launch_group(dtype, tab, group, RiderArgs{}, st);
     }
     int64_t blocks = (units + 255) / 256;
     if (blocks > mq_grid_cap()) blocks = mq_grid_cap();
@@ -1051,9 +1055,10 @@ bool mq_int4_pack_asym_fast_ok(const void* w, int dtype, int group, int64_t M) {
 int64_t mq_int4_zero_tiles(int64_t rows, int64_t cols, int group) { return int4_zero_tiles(rows / 8, cols / group); }
 
 // The two launches of an asymmetric pack for a group of tensors: codes + scales + zero points, then the zero points
-// packed eight rows to a word.  max_tiles: the most tiles the second launch has to cover in one tensor.
+// packed eight rows to a word (copies that ride along, with the second).  max_tiles: the most tiles the second launch has to
+// cover in one tensor.
 template <class Table>
-static int int4_pack_asym_launch(int dtype, const Table& tab, int n, int64_t max_tiles, int group, hipStream_t st) {
+static int int4_pack_asym_launch(int dtype, const Table& tab, int n, int64_t max_tiles, int group, const RiderArgs& riders, hipStream_t st) {
     const dim3 grid((unsigned)tab.max_blocks, (unsigned)n), blk(kI4Threads);
     if (dtype == MQ_F32) {
         if (group == 128) hipLaunchKernelGGL((int4_pack_asym_f32_kernel<16, Table>), grid, blk, 0, st, tab);
@@ -1070,10 +1075,12 @@ static int int4_pack_asym_launch(int dtype, const Table& tab, int n, int64_t max
     }
     int rc = mq_check_launch("int4 asymmetric pack");
     if (rc != MQ_OK) return rc;
-    hipLaunchKernelGGL(int4_zero_pack_group_kernel<Table>, dim3((unsigned)max_tiles, (unsigned)n), dim3(256), 0, st, tab);
+    with_riders(riders, n, max_tiles, [&](unsigned rows, const auto& r) {
+        hipLaunchKernelGGL((int4_zero_pack_group_kernel<Table, std::decay_t<decltype(r)>>), dim3((unsigned)max_tiles, rows), dim3(256), 0, st, tab, r);
+    });
     return mq_check_launch("int4 zero-point pack");
 }
-int mq_int4_pack_asym_launch_group(int dtype, FlatTable& tab, int group, hipStream_t st) {
+int mq_int4_pack_asym_launch_group(int dtype, FlatTable& tab, int group, const RiderArgs& riders, hipStream_t st) {
     if (!flat_grid(tab, kI4Threads * kI4Unroll)) return mq_fail(MQ_ERR_ARG, "tensor too large");
     if (tab.max_blocks == 0) return MQ_OK;
     int64_t max_tiles = 1;
@@ -1084,15 +1091,15 @@ int mq_int4_pack_asym_launch_group(int dtype, FlatTable& tab, int group, hipStre
         max_tiles = tiles > max_tiles ? tiles : max_tiles;
     }
     if (max_tiles >= 0x7FFFFFFF) return mq_fail(MQ_ERR_ARG, "tensor too large");
-    return int4_pack_asym_launch(dtype, tab, tab.n, max_tiles, group, st);
+    return int4_pack_asym_launch(dtype, tab, tab.n, max_tiles, group, riders, st);
 }
 // max_units: the largest tensor's 16-byte units; max_zero_tiles: the largest mq_int4_zero_tiles of the tensors
 int mq_int4_pack_asym_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int64_t max_zero_tiles,
-                                   int group, hipStream_t st) {
+                                   int group, const RiderArgs& riders, hipStream_t st) {
     FlatRef ref{device_jobs, 0, 0};
     if (!flat_grid(ref, max_units, kI4Threads * kI4Unroll) || max_zero_tiles >= 0x7FFFFFFF) return mq_fail(MQ_ERR_ARG, "tensor too large");
     if (ref.max_blocks == 0 || n == 0) return MQ_OK;
-    return int4_pack_asym_launch(dtype, ref, n, max_zero_tiles < 1 ? 1 : max_zero_tiles, group, st);
+    return int4_pack_asym_launch(dtype, ref, n, max_zero_tiles < 1 ? 1 : max_zero_tiles, group, riders, st);
 }
 
 extern "C" int mq_int4_group_quant_pack_asym(const void* w, int dtype, int32_t* packed, void* scale, uint8_t* zero,
@@ -1112,7 +1119,7 @@ extern "C" int mq_int4_group_quant_pack_asym(const void* w, int dtype, int32_t* 
         FlatTable tab{};
         tab.n = 1;
         tab.job[0] = FlatJob{w, packed, scale, zero, M * (K / 8), packed_zp, (int32_t)gpr, (int32_t)(M / 8)};
-        return mq_int4_pack_asym_launch_group(dtype, tab, group, st);
+        return mq_int4_pack_asym_launch_group(dtype, tab, group, RiderArgs{}, st);
     } else if (dtype == MQ_BF16)
         hipLaunchKernelGGL(int4_pack_asym_kernel<MQ_BF16>, dim3((unsigned)blocks), dim3(256), 0, st, w, (uint32_t*)packed, scale, zero, groups, wpg, aligned);
     else if (dtype == MQ_F16)

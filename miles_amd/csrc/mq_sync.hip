@@ -13,6 +13,7 @@
 
 #include "mq_api_internal.hpp"
 #include "mq_common.hpp"
+#include "mq_copy.hpp"
 #include "mq_group.hpp"
 
 using namespace mq;
@@ -30,7 +31,7 @@ int mq_fp8_dequant_launch_group(const MqDequantArgs* a, int n, bool aligned, hip
 bool mq_mxfp8_fast_ok(const void* w, int dtype, const void* q);
 int mq_mxfp8_launch_group(int dtype, FlatTable& tab, hipStream_t st);
 bool mq_int4_pack_fast_ok(const void* w, int dtype, int group);
-int mq_int4_pack_launch_group(int dtype, FlatTable& tab, int group, hipStream_t st);
+int mq_int4_pack_launch_group(int dtype, FlatTable& tab, int group, const RiderArgs& riders, hipStream_t st);
 bool mq_nvfp4_fast_ok(const void* w, int dtype, const void* q);
 int mq_nvfp4_amax_launch_group(int dtype, FlatTable& tab, hipStream_t st);
 int mq_nvfp4_quant_launch_group(int dtype, FlatTable& tab, int e4m3_max, int flags, int mode, hipStream_t st);
@@ -55,11 +56,11 @@ int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, in
                                 int mode, hipStream_t st);
 int mq_mxfp8_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, hipStream_t st);
 int mq_mxfp4_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, hipStream_t st);
-int mq_int4_pack_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int group, hipStream_t st);
+int mq_int4_pack_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int group, const RiderArgs& riders, hipStream_t st);
 bool mq_int4_pack_asym_fast_ok(const void* w, int dtype, int group, int64_t M);
-int mq_int4_pack_asym_launch_group(int dtype, FlatTable& tab, int group, hipStream_t st);
+int mq_int4_pack_asym_launch_group(int dtype, FlatTable& tab, int group, const RiderArgs& riders, hipStream_t st);
 int mq_int4_pack_asym_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int64_t max_zero_tiles, int group,
-                                   hipStream_t st);
+                                   const RiderArgs& riders, hipStream_t st);
 int64_t mq_int4_zero_tiles(int64_t rows, int64_t cols, int group);
 int mq_mxfp4_to_fp8_job(RecodeJob& job, const void* packed, const void* scale, void* y, void* tile_scale, int64_t out_dim,
                         int64_t in_dim);
@@ -376,6 +377,62 @@ struct CopyRanges {
         else below = UINTPTR_MAX;       // a source inside: nothing more is independent at a glance
     }
 };
+
+// Whether runs a[0..) and b[0..), each of them in ascending order and apart from one another, are apart from each other
+// (false as well for what is in no such order).
+struct Span {
+    uintptr_t lo, hi;
+};
+static bool ascending_apart(const std::vector<Span>& a, const std::vector<Span>& b) {
+    for (const std::vector<Span>* v : {&a, &b})
+        for (size_t i = 1; i < v->size(); i++)
+            if ((*v)[i].lo < (*v)[i - 1].hi) return false;
+    for (size_t i = 0, k = 0; i < a.size() && k < b.size();) {
+        if (a[i].hi <= b[k].lo) i++;
+        else if (b[k].hi <= a[i].lo) k++;
+        else return false;
+    }
+    return true;
+}
+static Span hull(const std::vector<Span>& v) {
+    Span h{UINTPTR_MAX, 0};
+    for (const Span& s : v) h = Span{s.lo < h.lo ? s.lo : h.lo, s.hi > h.hi ? s.hi : h.hi};
+    return h;
+}
+static bool apart(const Span& a, const Span& b) { return a.hi <= b.lo || b.hi <= a.lo; }
+// How many of the copy jobs at `j` can ride along with the INT4 jobs [i, j) in front of them, at most `cap`: short runs that
+// depend neither on one another nor on those jobs.  Of the shape records of a packed payload, which stand between its codes and
+// scales in the order of the jobs, that is seen in one pass; what is in no such order keeps a launch of its own.
+static int64_t int4_riders(const mq_job* jobs, int64_t n, int64_t i, int64_t j, int64_t cap) {
+    int64_t k = j;
+    CopyRanges copied;
+    std::vector<Span> to, from;
+    for (; k < n && k - j < cap && jobs[k].kind == MQ_JOB_COPY && jobs[k].rows > 0 && jobs[k].cols > 0 && copy_one_run(jobs[k]) &&
+           jobs[k].rows * jobs[k].cols <= kRiderChunks * kCopyChunk && copied.independent(jobs[k]); k++) {
+        copied.add(jobs[k]);
+        const uintptr_t out = (uintptr_t)jobs[k].out, in = (uintptr_t)jobs[k].in, bytes = (uintptr_t)(jobs[k].rows * jobs[k].cols);
+        to.push_back(Span{out, out + bytes});
+        from.push_back(Span{in, in + bytes});
+    }
+    if (k == j) return 0;
+    const Span dst = hull(to), src = hull(from);
+    std::vector<Span> written[4];
+    for (int64_t t = i; t < j; t++) {
+        const mq_job& jb = jobs[t];
+        const uintptr_t size = jb.dtype == MQ_F32 ? 4 : 2, elements = (uintptr_t)(jb.rows * jb.cols), groups = elements / (uintptr_t)jb.p0;
+        const uintptr_t at[4] = {(uintptr_t)jb.out, (uintptr_t)jb.scale, (uintptr_t)jb.aux, (uintptr_t)jb.aux2};
+        const uintptr_t bytes[4] = {elements / 2, groups * size, groups, groups / 2};
+        if (!apart(Span{(uintptr_t)jb.in, (uintptr_t)jb.in + elements * size}, dst)) return 0;
+        for (int f = 0; f < (jb.kind == MQ_JOB_INT4_PACK_ASYM ? 4 : 2); f++) written[f].push_back(Span{at[f], at[f] + bytes[f]});
+    }
+    for (const std::vector<Span>& w : written) {
+        if (w.empty()) continue;
+        const Span h = hull(w);
+        if (!apart(h, dst) && !ascending_apart(w, to)) return 0;
+        if (!apart(h, src) && !ascending_apart(w, from)) return 0;
+    }
+    return k - j;
+}
 
 // per-tensor FP8 run [i, j): chunks of up to kMaxGroup tensors of similar size with the same floor and flags
 // (`table`: the device descriptors of jobs[0..), or null)
@@ -746,6 +803,17 @@ extern "C" int mq_run_jobs_tabled(const mq_job* jobs, int64_t n, const void* dev
             case MQ_JOB_MXFP4:
             case MQ_JOB_INT4_PACK:
             case MQ_JOB_INT4_PACK_ASYM: {
+                RiderArgs riders{};
+                CopyRun run[kMaxGroup];
+                if (head.kind == MQ_JOB_INT4_PACK || head.kind == MQ_JOB_INT4_PACK_ASYM) {
+                    const bool entries = tabled && cnt > kMaxGroup;
+                    riders.n = (int)int4_riders(jobs, n, i, j, entries ? kTableGroup : kMaxGroup);
+                    riders.entry = entries ? (const CopyTableEntry*)table + j : nullptr;
+                    riders.run = run;
+                    for (int t = 0; t < riders.n && !entries; t++)
+                        run[t] = CopyRun{(const uint8_t*)jobs[j + t].in, (uint8_t*)jobs[j + t].out, jobs[j + t].rows * jobs[j + t].cols};
+                    j += riders.n;
+                }
                 if (tabled && cnt > kMaxGroup) {        // small groups keep the kernel-argument form (no pointer chase)
                     int64_t zero_tiles = 0;
                     if (head.kind == MQ_JOB_INT4_PACK_ASYM)
@@ -755,8 +823,8 @@ extern "C" int mq_run_jobs_tabled(const mq_job* jobs, int64_t n, const void* dev
                         }
                     rc = head.kind == MQ_JOB_MXFP8       ? mq_mxfp8_launch_table(head.dtype, table + i, cnt, mx / 8, st)
                          : head.kind == MQ_JOB_MXFP4     ? mq_mxfp4_launch_table(head.dtype, table + i, cnt, mx / 8, st)
-                         : head.kind == MQ_JOB_INT4_PACK ? mq_int4_pack_launch_table(head.dtype, table + i, cnt, mx / 8, head.p0, st)
-                                                         : mq_int4_pack_asym_launch_table(head.dtype, table + i, cnt, mx / 8, zero_tiles, head.p0, st);
+                         : head.kind == MQ_JOB_INT4_PACK ? mq_int4_pack_launch_table(head.dtype, table + i, cnt, mx / 8, head.p0, riders, st)
+                                                         : mq_int4_pack_asym_launch_table(head.dtype, table + i, cnt, mx / 8, zero_tiles, head.p0, riders, st);
                     break;
                 }
                 FlatTable tab{};
@@ -764,8 +832,8 @@ extern "C" int mq_run_jobs_tabled(const mq_job* jobs, int64_t n, const void* dev
                 for (int t = 0; t < cnt; t++) tab.job[t] = flat_entry(jobs[i + t]);
                 rc = head.kind == MQ_JOB_MXFP8       ? mq_mxfp8_launch_group(head.dtype, tab, st)
                      : head.kind == MQ_JOB_MXFP4     ? mq_mxfp4_launch_group(head.dtype, tab, st)
-                     : head.kind == MQ_JOB_INT4_PACK ? mq_int4_pack_launch_group(head.dtype, tab, head.p0, st)
-                                                     : mq_int4_pack_asym_launch_group(head.dtype, tab, head.p0, st);
+                     : head.kind == MQ_JOB_INT4_PACK ? mq_int4_pack_launch_group(head.dtype, tab, head.p0, riders, st)
+                                                     : mq_int4_pack_asym_launch_group(head.dtype, tab, head.p0, riders, st);
                 break;
             }
             case MQ_JOB_FP8_TO_MXFP8: {
