@@ -63,6 +63,9 @@ __device__ __forceinline__ TilePick pick_tile(const TileRef& tab) {
     const int32_t tiles = ((job.M + kTile - 1) / kTile) * ((job.K + kTile - 1) / kTile);
     return TilePick{(int32_t)blockIdx.y, xcd_contiguous_item(tiles)};
 }
+// Tiles of a launch below which a lane issues its four loads at once.  Syncs, us, one then three / at once: 840 tiles 10.9 / 10.5,
+// 2400 22.0 / 21.8, 2800 26.2 / 25.9, 4500 38.6 / 38.4, 7500 61.2 / 61.3, 18500 143.1 / 144.4.
+constexpr uint32_t kShortLaunch = 4096;
 template <int MODE, class Table, int F16>
 __global__ __launch_bounds__(kTileThreads) void fp8_block128_kernel(const Table tab) {
     constexpr uint32_t kInfBits = F16 ? 0x7C00u : 0x7F80u;      // pattern of +inf; anything above is a NaN
@@ -96,6 +99,7 @@ __global__ __launch_bounds__(kTileThreads) void fp8_block128_kernel(const Table 
     const uint32_t t = threadIdx.x, r0 = t >> 4, c0 = (t & 15u) * 8u;
     const bool col_ok = full || c0 < cols_left;  // K % 8 == 0: an 8-wide segment is entirely inside or outside
     u32x4 v[kRowsPerThread];
+    const bool short_launch = gridDim.x * gridDim.y < kShortLaunch;
     if (full) {
         const uint32_t off = (r0 * ldw + c0) * 2u;
 #pragma unroll
@@ -104,7 +108,8 @@ __global__ __launch_bounds__(kTileThreads) void fp8_block128_kernel(const Table 
             // The first quarter of the tile is waited for before the other three are requested.  With all four loads
             // of every lane in flight at once the sync ran 0.5 - 1.2 % slower (alternating runs on one GPU): the
             // memory queues are full either way, and the narrower front of requests keeps more of them on open pages.
-            if (i == 0 && kRowsPerThread > 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            // A short launch has a memory latency less without the wait (kShortLaunch).
+            if (i == 0 && kRowsPerThread > 2 && !short_launch) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
     } else {
         const uint32_t c = col_ok ? c0 : 0u;
