@@ -301,11 +301,13 @@ __device__ __forceinline__ void nv_decode8(uint32_t word, float q[8]) {
 // with value * f32(scale) either zero or in 2^-10 .. 2688, so one test of the tensor amax covers every element:
 // nv_fast_division(amax) allows the sequence for the whole tensor, otherwise every quotient is the IEEE division.
 // 0: IEEE divisions; 1: the sequence; 2: the sequence, and the amax has at most 12 significant bits (the amax of a bf16 or
-// fp16 tensor has), so that value x f32(scale) x amax -- 2, 4 and 12 bits -- is exact in whatever order it is taken
+// fp16 tensor has), so that value x f32(scale) x amax -- 2, 4 and 12 bits -- is exact in whatever order it is taken, and it is
+// 2^-60 or more, so that a block maximum out of the range of div_by_shared (below 2^-91; S_enc is at most 2^72) has a scale of
+// zero whatever its sixth comes to in the last place
 __device__ __forceinline__ int nv_fast_division(float amax) {
     const uint32_t e = f2u(amax) & 0x7F800000u;
     if (!(e >= 0x17800000u /* 2^-80 */ && e <= 0x65800000u /* 2^76 */)) return 0;
-    return (f2u(amax) & 0xFFFu) == 0 ? 2 : 1;
+    return (f2u(amax) & 0xFFFu) == 0 && e >= 0x21800000u /* 2^-60 */ ? 2 : 1;
 }
 template <int FASTDIV>
 __device__ __forceinline__ float div_by_numer(float x, float d, float y) {
@@ -341,9 +343,10 @@ __device__ __forceinline__ void nv_error_terms(const float f[8], uint32_t word, 
 // order, takes sixteen additions in each lane of the pair.  The data is therefore regrouped first: a lane ends up with the
 // thirty-two bytes of one whole block, and the kernels are bound by vector instructions, not by memory.
 struct NvCandidate16 {
-    uint32_t sc;        // e4m3 byte
+    uint32_t at;        // eight times the e4m3 byte of the scale: where the table has its entry
     uint32_t lo, hi;    // codes of elements 0..7 and 8..15
     float a;            // RN(f32(sc) * amax / denom): what one unit of the code grid is worth (tensors that take the estimate)
+    __device__ __forceinline__ uint32_t sc() const { return at >> 3; }
 };
 // A candidate's block scale is one of 128 bytes, and what the quantizer needs of it -- the reciprocal
 // min(1 / (f32(byte) * S_dec), FLT_MAX) and, for the error estimate, RN(f32(byte) * amax / denom) -- depends on the byte
@@ -364,17 +367,18 @@ __device__ __forceinline__ void nv_fill_scale_table(NvScaleEntry* table, int t, 
         table[t] = e;
     }
 }
-__device__ __forceinline__ NvCandidate16 nv_candidate16(const float f[16], float s_hp, const NvScaleEntry* table) {
+__device__ __forceinline__ NvCandidate16 nv_candidate16(const float f[16], uint32_t at, const NvScaleEntry* table) {
     NvCandidate16 c;
-    c.sc = hw_e4m3x2<false>(__builtin_fminf(s_hp, kFp8Max), 0.0f, 0u) & 0xFFu;
-    const NvScaleEntry e = table[c.sc & 0x7Fu];      // s_hp is not negative: the byte has no sign bit
+    c.at = at;
+    const NvScaleEntry e = *reinterpret_cast<const NvScaleEntry*>(reinterpret_cast<const char*>(table) + at);
     const float inv = e.inv;
     c.a = e.a;
-    c.lo = hw_e2m1x2<0>(f[0] * inv, f[1] * inv, 0u);
+    asm("" : "=v"(c.lo), "=v"(c.hi));      // (four conversions write all of each)
+    c.lo = hw_e2m1x2<0>(f[0] * inv, f[1] * inv, c.lo);
     c.lo = hw_e2m1x2<1>(f[2] * inv, f[3] * inv, c.lo);
     c.lo = hw_e2m1x2<2>(f[4] * inv, f[5] * inv, c.lo);
     c.lo = hw_e2m1x2<3>(f[6] * inv, f[7] * inv, c.lo);
-    c.hi = hw_e2m1x2<0>(f[8] * inv, f[9] * inv, 0u);
+    c.hi = hw_e2m1x2<0>(f[8] * inv, f[9] * inv, c.hi);
     c.hi = hw_e2m1x2<1>(f[10] * inv, f[11] * inv, c.hi);
     c.hi = hw_e2m1x2<2>(f[12] * inv, f[13] * inv, c.hi);
     c.hi = hw_e2m1x2<3>(f[14] * inv, f[15] * inv, c.hi);
@@ -384,7 +388,7 @@ template <int EM, int FASTDIV>
 __device__ __forceinline__ float nv_block_error(const float f[16], const NvCandidate16& c, float amax, float enc, float denom,
                                                 float denom_inv) {
     float term[8], error = 0.0f;
-    const float s_f = hw_e4m3x2_decode<false>(c.sc).x;
+    const float s_f = hw_e4m3x2_decode<false>(c.sc()).x;
     nv_error_terms<EM, FASTDIV>(f, c.lo, s_f, amax, enc, denom, denom_inv, term);
 #pragma unroll
     for (int j = 0; j < 8; j++) error = error + term[j];
@@ -426,14 +430,23 @@ __device__ __forceinline__ float nv_block_error_estimate(const float f[16], cons
     }
     return sum;
 }
-template <int EM, int FASTDIV, bool F32 = false>
+// TRUSTED: bmax is a number not above amax, so that s6_hp is at most 448 (1 + 2^-22), which the conversion takes for 448
+template <int EM, int FASTDIV, bool F32 = false, bool TRUSTED = false>
 __device__ __forceinline__ NvCandidate16 nv_four_over_six16(const float f[16], float bmax, float amax, const NvScales& gs,
                                                             float denom, float denom_inv, const NvScaleEntry* table) {
-    const bool plain_bmax = shared_div_ok(bmax);
-    // (an fp32 block's maximum has more bits than the shared-divisor sequence takes)
-    const float s6_hp = (!F32 && __builtin_amdgcn_ballot_w64(!plain_bmax) == 0 ? div_by_shared(bmax, 6.0f, 0x1.555556p-3f) : bmax / 6.0f) * gs.enc;
-    const float s4_hp = s6_hp * 1.5f;
-    const NvCandidate16 c4 = nv_candidate16(f, s4_hp, table), c6 = nv_candidate16(f, s6_hp, table);
+    float sixth;
+    if (FASTDIV == 2) {
+        sixth = div_by_shared(bmax, 6.0f, 0x1.555556p-3f);
+    } else {
+        const bool plain_bmax = shared_div_ok(bmax);
+        // (an fp32 block's maximum has more bits than the shared-divisor sequence takes)
+        sixth = !F32 && __builtin_amdgcn_ballot_w64(!plain_bmax) == 0 ? div_by_shared(bmax, 6.0f, 0x1.555556p-3f) : bmax / 6.0f;
+    }
+    const float s6_hp = sixth * gs.enc, s4_hp = s6_hp * 1.5f;
+    uint32_t bytes;      // of both scales, which have no sign bit
+    asm("" : "=v"(bytes));
+    bytes = hw_e4m3x2<false>(__builtin_fminf(s4_hp, kFp8Max), TRUSTED ? s6_hp : __builtin_fminf(s6_hp, kFp8Max), bytes);
+    const NvCandidate16 c4 = nv_candidate16(f, (bytes << 3) & 0x3F8u, table), c6 = nv_candidate16(f, (bytes >> 5) & 0x3F8u, table);
     if ((EM == 0 || EM == 1) && FASTDIV == 2) {
         // (FASTDIV 2: f32(scale) * amax is exact and its quotient by denom comes correctly rounded from the sequence)
         const float a4 = c4.a, a6 = c6.a;
@@ -441,7 +454,7 @@ __device__ __forceinline__ NvCandidate16 nv_four_over_six16(const float f[16], f
         float guard;
         if (EM == 0) {
             // twice the bound's first part and four times its second: rounding in this line cannot bring it below the bound
-            guard = 0x1p-19f * (32.0f * (a4 + a6) + 4.0f * bmax + 4.0f * (g4 + g6));
+            guard = 0x1p-17f * (__builtin_fmaf(8.0f, a4 + a6, bmax) + (g4 + g6));
         } else {
             // twice the squared error's bound for both candidates, and more (the hardware square root is within one unit
             // in the last place; the small constant keeps a denormal sum from dropping out of it and is the floor below
@@ -452,7 +465,7 @@ __device__ __forceinline__ NvCandidate16 nv_four_over_six16(const float f[16], f
         }
         // (an all-zero block, or two candidates with one scale byte -- the block that holds the tensor's maximum, whose
         // scales both saturate: the candidates are the same, the tie goes to map-to-6, as g4 < g6 says; a NaN compares false)
-        const bool decided = __builtin_fabsf(g4 - g6) > guard || bmax == 0.0f || c4.sc == c6.sc;
+        const bool decided = __builtin_fabsf(g4 - g6) > guard || bmax == 0.0f || c4.at == c6.at;
         if (__builtin_amdgcn_ballot_w64(!decided) == 0) return g4 < g6 ? c4 : c6;
         // a wavefront with a block too close to call (a few blocks in 10 000, most of them exact ties) takes the exact sums below
     }
@@ -501,16 +514,19 @@ __device__ __forceinline__ u32x4 nv_scaled16(const float q[8], float scale) {
 constexpr int kFosRounds = MQ_NV_FOS_ROUNDS;
 // units a workgroup of the quantizer covers (FOS as in nvfp4_quant_units)
 constexpr int64_t nv_units_per_block(int fos) { return (int64_t)kNvThreads * kNvUnroll * (fos ? kFosRounds : 1); }
+// `trusted`: the amax is the maximum of these very elements, so that a tensor whose amax is a number has no NaN in it.
 template <int EM, int F16, bool QDQ, class Scales>
 __device__ __forceinline__ uint32_t nvfp4_fos_units(const FlatJob& job, const int64_t base, const int t, const float denom,
-                                                    const float inv_denom, Scales scales) {
+                                                    const float inv_denom, const bool trusted, Scales scales) {
     static_assert(kNvUnroll == 2, "the regrouping pairs the two units of a lane");
     constexpr uint32_t kPiece = kNvThreads * 2;
     __shared__ u32x4 stage[kPiece];
     __shared__ NvScaleEntry scale_table[128];
+    __shared__ float final_scale[QDQ ? 128 : 1];       // of the dequantized values, by the scale's byte
     const uint16_t* __restrict__ w = (const uint16_t*)job.w;
     uint32_t* __restrict__ q = (uint32_t*)job.q;
     uint8_t* __restrict__ s8 = (uint8_t*)job.s;
+    uint16_t* __restrict__ y0 = (uint16_t*)job.q + base * 8;
     const int64_t left = job.units - base;
     const uint32_t rem_all = left < kPiece * kFosRounds ? (uint32_t)left : kPiece * kFosRounds;
     const uint16_t* __restrict__ w0 = w + base * 8;
@@ -538,6 +554,7 @@ __device__ __forceinline__ uint32_t nvfp4_fos_units(const FlatJob& job, const in
     const float denom_inv = denom == 2688.0f ? kInv2688 : denom == 1536.0f ? kInv1536 : 1.0f / denom;
     // (a workgroup that comes here again, in the striding second pass, writes the same values over the table: one tensor)
     nv_fill_scale_table(scale_table, t, amax, gs.s_dec, fastdiv == 2 && EM < 2, denom, denom_inv);
+    if (QDQ && t < 128) final_scale[t] = (hw_e4m3x2_decode<false>((uint32_t)t).x * amax) * inv_denom;
     __syncthreads();
     uint32_t seen = 0;
 #pragma unroll
@@ -559,25 +576,37 @@ __device__ __forceinline__ uint32_t nvfp4_fos_units(const FlatJob& job, const in
         // (and the next piece's writes stay below these reads)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        const uint32_t m2 = max2_u16(max2_u16(max2_u16(abs2(lo.x), abs2(lo.y)), max2_u16(abs2(lo.z), abs2(lo.w))),
-                                     max2_u16(max2_u16(abs2(hi.x), abs2(hi.y)), max2_u16(abs2(hi.z), abs2(hi.w))));
-        const uint32_t mb = hmax_u16(m2);
-        seen = umax(seen, mb);
-        const float bmax = elem_lo<F16>(mb);
+        auto pattern_max = [&] {
+            return hmax_u16(max2_u16(max2_u16(max2_u16(abs2(lo.x), abs2(lo.y)), max2_u16(abs2(lo.z), abs2(lo.w))),
+                                     max2_u16(max2_u16(abs2(hi.x), abs2(hi.y)), max2_u16(abs2(hi.z), abs2(hi.w)))));
+        };
         const float f[16] = {elem_lo<F16>(lo.x), elem_hi<F16>(lo.x), elem_lo<F16>(lo.y), elem_hi<F16>(lo.y),
                              elem_lo<F16>(lo.z), elem_hi<F16>(lo.z), elem_lo<F16>(lo.w), elem_hi<F16>(lo.w),
                              elem_lo<F16>(hi.x), elem_hi<F16>(hi.x), elem_lo<F16>(hi.y), elem_hi<F16>(hi.y),
                              elem_lo<F16>(hi.z), elem_hi<F16>(hi.z), elem_lo<F16>(hi.w), elem_hi<F16>(hi.w)};
-        const NvCandidate16 c = fastdiv == 2   ? nv_four_over_six16<EM, 2>(f, bmax, amax, gs, denom, denom_inv, scale_table)
-                                : fastdiv == 1 ? nv_four_over_six16<EM, 1>(f, bmax, amax, gs, denom, denom_inv, scale_table)
-                                               : nv_four_over_six16<EM, 0>(f, bmax, amax, gs, denom, denom_inv, scale_table);
+        NvCandidate16 c;
+        if (trusted && fastdiv == 2) {
+            // (no NaN: the maximum of the numbers, three at a time)
+            float bmax = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(f[0]), __builtin_fabsf(f[1])), __builtin_fabsf(f[2]));
+#pragma unroll
+            for (int j = 3; j < 15; j += 2) bmax = __builtin_fmaxf(__builtin_fmaxf(bmax, __builtin_fabsf(f[j])), __builtin_fabsf(f[j + 1]));
+            bmax = __builtin_fmaxf(bmax, __builtin_fabsf(f[15]));
+            c = nv_four_over_six16<EM, 2, false, true>(f, bmax, amax, gs, denom, denom_inv, scale_table);
+        } else {
+            const uint32_t mb = pattern_max();
+            seen = umax(seen, mb);
+            const float bmax = elem_lo<F16>(mb);
+            c = fastdiv == 2   ? nv_four_over_six16<EM, 2>(f, bmax, amax, gs, denom, denom_inv, scale_table)
+                : fastdiv == 1 ? nv_four_over_six16<EM, 1>(f, bmax, amax, gs, denom, denom_inv, scale_table)
+                               : nv_four_over_six16<EM, 0>(f, bmax, amax, gs, denom, denom_inv, scale_table);
+        }
         if (QDQ) {
-            const float final_scale = (hw_e4m3x2_decode<false>(c.sc).x * amax) * inv_denom;
+            const float scale = final_scale[c.sc()];
             float y[8];
             nv_decode8(c.lo, y);
-            stage[first] = nv_scaled16<F16>(y, final_scale);
+            stage[first] = nv_scaled16<F16>(y, scale);
             nv_decode8(c.hi, y);
-            stage[first + 1] = nv_scaled16<F16>(y, final_scale);
+            stage[first + 1] = nv_scaled16<F16>(y, scale);
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -585,13 +614,13 @@ __device__ __forceinline__ uint32_t nvfp4_fos_units(const FlatJob& job, const in
             for (int i = 0; i < 2; i++) {
                 const uint32_t off = (uint32_t)t + i * kNvThreads;
                 const u32x4 o = stage[off];
-                if (off < rem) st16((uint16_t*)job.q + (base + r * kPiece + off) * 8, o);
+                if (off < rem) st16(y0 + (r * kPiece + off) * 8u, o);
             }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
         } else if (first < rem) {      // the tensor is whole blocks: both units of a block are inside or outside
             st8(q0 + r * kPiece + first, u32x2{c.lo, c.hi});      // `first` is even and `base` a multiple of the piece
-            s80[(r * kPiece + first) >> 1] = (uint8_t)c.sc;
+            s80[(r * kPiece + first) >> 1] = (uint8_t)c.sc();
         }
     }
     return seen;
@@ -637,10 +666,10 @@ __device__ __forceinline__ NvUnitCodes nvfp4_quant_unit(const u32x4 v, const NvS
 }
 
 // kNvThreads * kNvUnroll units starting at `base` of one tensor; returns the largest |element| this lane saw (bf16 bits)
-// FOS = 0: standard quantizer; FOS = 1 + error mode: Four Over Six
-template <int FOS, int F16, class Scales>
+// FOS = 0: standard quantizer; FOS = 1 + error mode: Four Over Six, which returns nothing of use where TRUSTED
+template <int FOS, int F16, bool TRUSTED, class Scales>
 __device__ __forceinline__ uint32_t nvfp4_quant_units(const FlatJob& job, const int64_t base, const int t, const float denom, Scales scales) {
-    if (FOS) return nvfp4_fos_units<(FOS > 0 ? FOS - 1 : 0), F16, false>(job, base, t, denom, 0.0f, scales);
+    if (FOS) return nvfp4_fos_units<(FOS > 0 ? FOS - 1 : 0), F16, false>(job, base, t, denom, 0.0f, TRUSTED, scales);
     const uint16_t* __restrict__ w = (const uint16_t*)job.w;
     uint32_t* __restrict__ q = (uint32_t*)job.q;
     uint8_t* __restrict__ s8 = (uint8_t*)job.s;
@@ -704,7 +733,7 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
         // an XCD takes a run of consecutive blocks in every trip of the grid, as the flat grids do (second pass 2 pct faster)
         const int64_t first = xcd_chunked_block(gridDim.x == kSectionWords ? kSectionWords / kXcds : tab.chunk);
         for (int64_t base = first * kPerBlock; base < job.units; base += (int64_t)gridDim.x * kPerBlock)
-            nvfp4_quant_units<FOS, F16>(job, base, t, denom, [&] { return nv_record_scales(job); });
+            nvfp4_quant_units<FOS, F16, true>(job, base, t, denom, [&] { return nv_record_scales(job); });
         return;
     }
     const int64_t base = flat_block(tab) * kPerBlock;
@@ -720,12 +749,12 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
             return a;
         };
         if (job.units == 0) fold();
-        else nvfp4_quant_units<FOS, F16>(job, base, t, denom, fold);
+        else nvfp4_quant_units<FOS, F16, true>(job, base, t, denom, fold);
         return;
     }
     if (base >= job.units) return;
     if (PASS == 3) {
-        nvfp4_quant_units<FOS, F16>(job, base, t, denom, [&] { return nv_record_scales(job); });
+        nvfp4_quant_units<FOS, F16, true>(job, base, t, denom, [&] { return nv_record_scales(job); });
         return;
     }
     uint32_t seen;
@@ -733,7 +762,7 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
         seen = 0;
         for (int64_t piece = base; piece < base + kPerBlock && piece < job.units; piece += kNvThreads * kNvUnroll)
             seen = umax(seen, nvfp4_amax_units(job, piece, t));
-    } else seen = nvfp4_quant_units<FOS, F16>(job, base, t, denom, [&] { return nv_record_scales(job); });
+    } else seen = nvfp4_quant_units<FOS, F16, false>(job, base, t, denom, [&] { return nv_record_scales(job); });
     if (PASS == 1) {
         __shared__ uint32_t wave_seen[kNvThreads / 64];
         seen = wave_max(seen);
@@ -939,7 +968,7 @@ __device__ __forceinline__ void nv_one_rest(const Table& tab, const uint32_t ten
     if ((got & kOneFull) == 0 && worker == 0 && t == 0) nv_publish_plain(job, a.amax, a.gs, numer, moved_counter);
     constexpr int64_t kPerBlock = nv_units_per_block(0);
     for (int64_t base = worker * kPerBlock; base < job.units; base += workers * kPerBlock)
-        nvfp4_quant_units<0, F16>(job, base, t, numer, [&] { return a; });
+        nvfp4_quant_units<0, F16, true>(job, base, t, numer, [&] { return a; });
 }
 // By a record's first workgroup, when it has nothing else to do: the record of a maximum that it has published, for all
 // tensors that share it; the slots, which nobody reads any more, are cleared for a carried run.
@@ -1099,7 +1128,7 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_f32_kernel(const Table
         if (t < rem) {
             ((uint32_t*)job.q + first)[2 * t] = c.lo;
             ((uint32_t*)job.q + first)[2 * t + 1] = c.hi;
-            ((uint8_t*)job.s + first / 2)[t] = (uint8_t)c.sc;
+            ((uint8_t*)job.s + first / 2)[t] = (uint8_t)c.sc();
         }
     } else {
         constexpr uint32_t kPerBlock = kNvThreads * kNvF32Loads;
@@ -1223,7 +1252,7 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_fake_kernel(const FlatTable 
     const int64_t base = flat_block(tab) * nv_units_per_block(FOS);
     if (base >= job.units) return;
     if constexpr (FOS != 0) {
-        nvfp4_fos_units<FOS - 1, F16, true>(job, base, t, numer, inv_numer, [&] { return nv_fake_scales(job, t, numer); });
+        nvfp4_fos_units<FOS - 1, F16, true>(job, base, t, numer, inv_numer, job.aux2 == nullptr, [&] { return nv_fake_scales(job, t, numer); });
     } else {
         const int64_t left = job.units - base;
         const uint32_t rem = left < kNvThreads * kNvUnroll ? (uint32_t)left : (uint32_t)(kNvThreads * kNvUnroll);
