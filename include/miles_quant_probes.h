@@ -48,7 +48,7 @@ int mqp_copy_bytes(const void* src, void* dst, int64_t nbytes, void* stream);
  *                  length K; both sides, the reads alone, the writes alone */
 enum { MQP_FLAT_2_1 = 0, MQP_FLAT_1_2 = 1, MQP_LOOP_2_1 = 2, MQP_TILE_2_1 = 3, MQP_TILE_READ = 4, MQP_TILE_WRITE = 5 };
 /* How the waits of the NVFP4 form that reads a list once end: runs it on n <= MQ_MAX_GROUP jobs (struct mq_job of miles_quant.h, kind
- * MQ_JOB_NVFP4: bf16 or fp16, standard block scaling, contiguous, 16-byte aligned and not empty, an amax record each, at most 512
+ * MQ_JOB_NVFP4: bf16 or fp16, one p1 without MQ_NVFP4_ERR_FP16, contiguous, 16-byte aligned and not empty, an amax record each, at most 512
  * workgroups of 64 KiB) with the given numbers of looks: of a record's first workgroup, and of those that watch its word. */
 struct mq_job;
 int mqp_nvfp4_one_pass(const struct mq_job* jobs, int n, int first_polls, int patience, void* stream);

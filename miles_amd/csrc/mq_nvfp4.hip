@@ -430,10 +430,12 @@ __device__ __forceinline__ float nv_block_error_estimate(const float f[16], cons
     }
     return sum;
 }
+struct NvCandidates16 {
+    NvCandidate16 c4, c6;
+};
 // TRUSTED: bmax is a number not above amax, so that s6_hp is at most 448 (1 + 2^-22), which the conversion takes for 448
-template <int EM, int FASTDIV, bool F32 = false, bool TRUSTED = false>
-__device__ __forceinline__ NvCandidate16 nv_four_over_six16(const float f[16], float bmax, float amax, const NvScales& gs,
-                                                            float denom, float denom_inv, const NvScaleEntry* table) {
+template <int FASTDIV, bool F32, bool TRUSTED>
+__device__ __forceinline__ NvCandidates16 nv_candidates16(const float f[16], float bmax, const NvScales& gs, const NvScaleEntry* table) {
     float sixth;
     if (FASTDIV == 2) {
         sixth = div_by_shared(bmax, 6.0f, 0x1.555556p-3f);
@@ -446,27 +448,41 @@ __device__ __forceinline__ NvCandidate16 nv_four_over_six16(const float f[16], f
     uint32_t bytes;      // of both scales, which have no sign bit
     asm("" : "=v"(bytes));
     bytes = hw_e4m3x2<false>(__builtin_fminf(s4_hp, kFp8Max), TRUSTED ? s6_hp : __builtin_fminf(s6_hp, kFp8Max), bytes);
-    const NvCandidate16 c4 = nv_candidate16(f, (bytes << 3) & 0x3F8u, table), c6 = nv_candidate16(f, (bytes >> 5) & 0x3F8u, table);
-    if ((EM == 0 || EM == 1) && FASTDIV == 2) {
-        // (FASTDIV 2: f32(scale) * amax is exact and its quotient by denom comes correctly rounded from the sequence)
-        const float a4 = c4.a, a6 = c6.a;
-        const float g4 = nv_block_error_estimate<EM == 1>(f, c4, a4), g6 = nv_block_error_estimate<EM == 1>(f, c6, a6);
-        float guard;
-        if (EM == 0) {
-            // twice the bound's first part and four times its second: rounding in this line cannot bring it below the bound
-            guard = 0x1p-17f * (__builtin_fmaf(8.0f, a4 + a6, bmax) + (g4 + g6));
-        } else {
-            // twice the squared error's bound for both candidates, and more (the hardware square root is within one unit
-            // in the last place; the small constant keeps a denormal sum from dropping out of it and is the floor below
-            // which two sums are too small to call)
-            const float e4 = 0x1p-24f * (25.0f * a4 + 2.0f * bmax), e6 = 0x1p-24f * (25.0f * a6 + 2.0f * bmax);
-            guard = 17.0f * (e4 * __builtin_amdgcn_sqrtf(g4 + 0x1p-100f) + e6 * __builtin_amdgcn_sqrtf(g6 + 0x1p-100f)) +
-                    33.0f * (e4 * e4 + e6 * e6) + 0x1p-17f * (g4 + g6) + 0x1p-100f;
-        }
-        // (an all-zero block, or two candidates with one scale byte -- the block that holds the tensor's maximum, whose
-        // scales both saturate: the candidates are the same, the tie goes to map-to-6, as g4 < g6 says; a NaN compares false)
-        const bool decided = __builtin_fabsf(g4 - g6) > guard || bmax == 0.0f || c4.at == c6.at;
-        if (__builtin_amdgcn_ballot_w64(!decided) == 0) return g4 < g6 ? c4 : c6;
+    return NvCandidates16{nv_candidate16(f, (bytes << 3) & 0x3F8u, table), nv_candidate16(f, (bytes >> 5) & 0x3F8u, table)};
+}
+// What the estimates say of two candidates (FASTDIV 2: f32(scale) * amax is exact and its quotient by denom comes correctly
+// rounded from the sequence).
+struct NvPick {
+    bool decided, four;
+};
+template <int EM>
+__device__ __forceinline__ NvPick nv_estimated_pick(const float f[16], float bmax, const NvCandidate16& c4, const NvCandidate16& c6) {
+    const float a4 = c4.a, a6 = c6.a;
+    const float g4 = nv_block_error_estimate<EM == 1>(f, c4, a4), g6 = nv_block_error_estimate<EM == 1>(f, c6, a6);
+    float guard;
+    if (EM == 0) {
+        // twice the bound's first part and four times its second: rounding in this line cannot bring it below the bound
+        guard = 0x1p-17f * (__builtin_fmaf(8.0f, a4 + a6, bmax) + (g4 + g6));
+    } else {
+        // twice the squared error's bound for both candidates, and more (the hardware square root is within one unit
+        // in the last place; the small constant keeps a denormal sum from dropping out of it and is the floor below
+        // which two sums are too small to call)
+        const float e4 = 0x1p-24f * (25.0f * a4 + 2.0f * bmax), e6 = 0x1p-24f * (25.0f * a6 + 2.0f * bmax);
+        guard = 17.0f * (e4 * __builtin_amdgcn_sqrtf(g4 + 0x1p-100f) + e6 * __builtin_amdgcn_sqrtf(g6 + 0x1p-100f)) +
+                33.0f * (e4 * e4 + e6 * e6) + 0x1p-17f * (g4 + g6) + 0x1p-100f;
+    }
+    // (an all-zero block, or two candidates with one scale byte -- the block that holds the tensor's maximum, whose
+    // scales both saturate: the candidates are the same, the tie goes to map-to-6, as g4 < g6 says; a NaN compares false)
+    return NvPick{__builtin_fabsf(g4 - g6) > guard || bmax == 0.0f || c4.at == c6.at, g4 < g6};
+}
+template <int EM, int FASTDIV, bool F32 = false, bool TRUSTED = false>
+__device__ __forceinline__ NvCandidate16 nv_four_over_six16(const float f[16], float bmax, float amax, const NvScales& gs,
+                                                            float denom, float denom_inv, const NvScaleEntry* table) {
+    const NvCandidates16 both = nv_candidates16<FASTDIV, F32, TRUSTED>(f, bmax, gs, table);
+    const NvCandidate16 c4 = both.c4, c6 = both.c6;
+    if constexpr ((EM == 0 || EM == 1) && FASTDIV == 2) {
+        const NvPick pick = nv_estimated_pick<EM>(f, bmax, c4, c6);
+        if (__builtin_amdgcn_ballot_w64(!pick.decided) == 0) return pick.four ? c4 : c6;
         // a wavefront with a block too close to call (a few blocks in 10 000, most of them exact ties) takes the exact sums below
     }
     const float e4 = nv_block_error<EM, FASTDIV>(f, c4, amax, gs.enc, denom, denom_inv);
@@ -498,6 +514,24 @@ __device__ __forceinline__ u32x4 nv_scaled16(const float q[8], float scale) {
         }
     }
     return u32x4{p[0], p[1], p[2], p[3]};
+}
+
+// the largest magnitude of sixteen numbers (no NaN), three at a time
+__device__ __forceinline__ float nv_numbers_max(const float f[16]) {
+    float m = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(f[0]), __builtin_fabsf(f[1])), __builtin_fabsf(f[2]));
+#pragma unroll
+    for (int j = 3; j < 15; j += 2) m = __builtin_fmaxf(__builtin_fmaxf(m, __builtin_fabsf(f[j])), __builtin_fabsf(f[j + 1]));
+    return __builtin_fmaxf(m, __builtin_fabsf(f[15]));
+}
+template <int F16>
+__device__ __forceinline__ void nv_unpack16(const u32x4 lo, const u32x4 hi, float f[16]) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        f[2 * k] = elem_lo<F16>(lo[k]);
+        f[2 * k + 1] = elem_hi<F16>(lo[k]);
+        f[8 + 2 * k] = elem_lo<F16>(hi[k]);
+        f[9 + 2 * k] = elem_hi<F16>(hi[k]);
+    }
 }
 
 // Four Over Six over kNvThreads * 2 units starting at `base`: loaded as the standard quantizer loads them (lane t takes
@@ -580,18 +614,11 @@ __device__ __forceinline__ uint32_t nvfp4_fos_units(const FlatJob& job, const in
             return hmax_u16(max2_u16(max2_u16(max2_u16(abs2(lo.x), abs2(lo.y)), max2_u16(abs2(lo.z), abs2(lo.w))),
                                      max2_u16(max2_u16(abs2(hi.x), abs2(hi.y)), max2_u16(abs2(hi.z), abs2(hi.w)))));
         };
-        const float f[16] = {elem_lo<F16>(lo.x), elem_hi<F16>(lo.x), elem_lo<F16>(lo.y), elem_hi<F16>(lo.y),
-                             elem_lo<F16>(lo.z), elem_hi<F16>(lo.z), elem_lo<F16>(lo.w), elem_hi<F16>(lo.w),
-                             elem_lo<F16>(hi.x), elem_hi<F16>(hi.x), elem_lo<F16>(hi.y), elem_hi<F16>(hi.y),
-                             elem_lo<F16>(hi.z), elem_hi<F16>(hi.z), elem_lo<F16>(hi.w), elem_hi<F16>(hi.w)};
+        float f[16];
+        nv_unpack16<F16>(lo, hi, f);
         NvCandidate16 c;
         if (trusted && fastdiv == 2) {
-            // (no NaN: the maximum of the numbers, three at a time)
-            float bmax = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(f[0]), __builtin_fabsf(f[1])), __builtin_fabsf(f[2]));
-#pragma unroll
-            for (int j = 3; j < 15; j += 2) bmax = __builtin_fmaxf(__builtin_fmaxf(bmax, __builtin_fabsf(f[j])), __builtin_fabsf(f[j + 1]));
-            bmax = __builtin_fmaxf(bmax, __builtin_fabsf(f[15]));
-            c = nv_four_over_six16<EM, 2, false, true>(f, bmax, amax, gs, denom, denom_inv, scale_table);
+            c = nv_four_over_six16<EM, 2, false, true>(f, nv_numbers_max(f), amax, gs, denom, denom_inv, scale_table);
         } else {
             const uint32_t mb = pattern_max();
             seen = umax(seen, mb);
@@ -806,6 +833,13 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
 // 209 us), where two units a lane stream at 6.9.  Two, four or six units a lane more, held in LDS, 222 to 234 us; four loads in flight
 // at a time 225 to 236; a tensor's units dealt to its workgroups in turn 222; plain stores 220; starting the first
 // workgroups of a CU one after the other, no difference.
+// Four Over Six (the error modes that have an estimate): a lane holds eight whole blocks, regrouped through LDS before the wait;
+// the last pair of units stays there, or 24 registers would go to scratch memory instead of five.  Blocks that were too close to
+// call are taken up again behind the others, in a loop with the one copy of the exact sums, which reads them again.  32 x
+// [2048, 7168]: 342 us in two passes, 298 this way, 48 x [1536, 2048] 111 and 95 (four workgroups per CU without the spills 319 and
+// 103; regrouped by lane exchange after the wait 308 and 100; the next block's table lookups ahead of this block's sums 309 and
+// 101).  Bound by the two hundred vector instructions of a block, which all workgroups of a tensor run at the same time: they
+// overlap with the loads of the next two tensors, half as well as in the second of two passes.
 constexpr int kOneThreads = 256, kOneUnits = 16, kOneWavesPerSimd = 5;
 constexpr int64_t kOnePerBlock = kOneThreads * kOneUnits;
 constexpr int kOneSlots = 2 * kSectionWords;         // 16-bit slots of a section
@@ -832,10 +866,12 @@ __global__ __launch_bounds__(256) void nvfp4_one_pass_clear_kernel(const Table t
     if (job.section == 0 && threadIdx.x < kOneWords) rec[kRecOne + threadIdx.x * kOneStride] = 0;
 }
 
-// maximum of the block that a lane's unit and its neighbour's make up (16-bit pattern)
-__device__ __forceinline__ uint32_t nv_block_max(const u32x4 v) {
-    return group_max2(hmax_u16(max2_u16(max2_u16(abs2(v.x), abs2(v.y)), max2_u16(abs2(v.z), abs2(v.w)))));
+// a unit's maxima of its even and of its odd elements (16-bit patterns)
+__device__ __forceinline__ uint32_t nv_unit_max(const u32x4 v) {
+    return max2_u16(max2_u16(abs2(v.x), abs2(v.y)), max2_u16(abs2(v.z), abs2(v.w)));
 }
+// maximum of the block that a lane's unit and its neighbour's make up (16-bit pattern)
+__device__ __forceinline__ uint32_t nv_block_max(const u32x4 v) { return group_max2(hmax_u16(nv_unit_max(v))); }
 // The scale byte and the factor of a block with finite elements, for 1 / S_enc in 2^-82 .. 2^81: a block scale is 0 or in
 // 2^-9 .. 448, so the divisor of every block with a scale is in the range of recip_shared.  For a divisor of zero that gives
 // NaN, and the minimum with the largest factor is that factor, as for 1 / 0.
@@ -932,8 +968,9 @@ __device__ __forceinline__ uint32_t nv_one_scan(const Table& tab, const uint32_t
 }
 // Tensors with an infinity or a NaN, or with a scale at the ends of the fp32 range, are left as well: the code behind
 // has the software forms, which here, in sixteen copies, were 8 700 instructions in the way of the 2 000 that run.
-template <int F16>
+template <int FOS, int F16>
 __device__ __forceinline__ bool nv_one_leaves(const uint32_t m, const NvScales& gs) {
+    if (FOS) return nv_fast_division(elem_lo<F16>(m)) != 2;
     const uint32_t dec = f2u(gs.s_dec);
     return m >= (F16 ? 0x7C00u : 0x7F80u) || !(dec >= 0x16800000u /* 2^-82 */ && dec <= 0x68000000u /* 2^81 */);
 }
@@ -942,7 +979,7 @@ __device__ __forceinline__ bool nv_one_leaves(const uint32_t m, const NvScales& 
 // when every workgroup of the tensors has, most of which are done, and of a record that is done there is its word to read.
 // The slots of a record whose first workgroup has given up, which every worker folds, are cleared by the last one to have read
 // them (a carried run would take their marks for kCarriedMark).
-template <int F16, class Table>
+template <int FOS, int F16, class Table>
 __device__ __forceinline__ void nv_one_rest(const Table& tab, const uint32_t tensors, const uint32_t workers, const int patience, const int t, float numer,
                                             uint32_t* moved_counter) {
     __shared__ uint32_t readers;
@@ -958,7 +995,7 @@ __device__ __forceinline__ void nv_one_rest(const Table& tab, const uint32_t ten
     if (__syncthreads_or(late)) m = nv_one_scan(tab, row - job.section, job.pad, t);
     const float amax = elem_lo<F16>(m);
     const NvAmaxScales a{amax, nv_scales(amax, numer)};
-    if ((got & kOneFull) != 0 && !nv_one_leaves<F16>(m, a.gs)) return;
+    if ((got & kOneFull) != 0 && !nv_one_leaves<FOS, F16>(m, a.gs)) return;
     if (gave_up) {
         if (t == 0) readers = atomicAdd(rec + kRecReaders, 1u);
         __syncthreads();
@@ -966,9 +1003,9 @@ __device__ __forceinline__ void nv_one_rest(const Table& tab, const uint32_t ten
             for (int k = 0; k < job.pad; k++) rec[k * kSectionWords + t] = 0;
     }
     if ((got & kOneFull) == 0 && worker == 0 && t == 0) nv_publish_plain(job, a.amax, a.gs, numer, moved_counter);
-    constexpr int64_t kPerBlock = nv_units_per_block(0);
+    constexpr int64_t kPerBlock = nv_units_per_block(FOS);
     for (int64_t base = worker * kPerBlock; base < job.units; base += workers * kPerBlock)
-        nvfp4_quant_units<0, F16, true>(job, base, t, numer, [&] { return a; });
+        nvfp4_quant_units<FOS, F16, true>(job, base, t, numer, [&] { return a; });
 }
 // By a record's first workgroup, when it has nothing else to do: the record of a maximum that it has published, for all
 // tensors that share it; the slots, which nobody reads any more, are cleared for a carried run.
@@ -982,14 +1019,77 @@ __device__ __forceinline__ void nv_one_settle(const Table& tab, const FlatJob& j
     for (int k = 0; k < job.pad; k++) nv_publish_plain(flat_job_at(tab, blockIdx.y + k), amax, gs, numer, moved_counter);
 }
 
+// Of the units of two loads, the even lane of a pair takes the block of the first one and the odd lane that of the second.
+__device__ __forceinline__ void nv_pair_blocks(u32x4* stage, u32x4& a, u32x4& b, const int t) {
+    stage[t] = a;
+    stage[kOneThreads + t] = b;
+    // (as in nvfp4_fos_units: a wavefront reads back what its own lanes wrote)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const uint32_t first = ((t & 1) ? (uint32_t)kOneThreads : 0u) + ((uint32_t)t & ~1u);
+    a = stage[first];
+    b = stage[first + 1];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+// The blocks of a lane of the one-pass kernel with Four Over Six, the last one in `stage`, for an amax that nv_fast_division puts at
+// 2; maxima: of the blocks, two to a register.
+template <int EM, int F16>
+__device__ __forceinline__ void nv_one_four_over_six(const FlatJob& job, const u32x4 (&v)[kOneUnits], const uint32_t (&maxima)[kOneUnits / 2], const u32x4* stage, const int64_t base, const uint32_t rem, const int t,
+                                                     const float amax, const NvScales& gs, const float denom) {
+    __shared__ NvScaleEntry scale_table[128];
+    constexpr float kInv2688 = 1.0f / 2688.0f, kInv1536 = 1.0f / 1536.0f;
+    const float denom_inv = denom == 2688.0f ? kInv2688 : denom == 1536.0f ? kInv1536 : 1.0f / denom;
+    nv_fill_scale_table(scale_table, t, amax, gs.s_dec, true, denom, denom_inv);
+    __syncthreads();
+    const uint32_t odd = (uint32_t)t & 1u;
+    uint32_t* __restrict__ q0 = (uint32_t*)job.q + base;
+    uint8_t* __restrict__ s80 = (uint8_t*)job.s + base / 2;
+    auto store = [&](const uint32_t load, const NvCandidate16& c) {
+        const uint32_t first = ((uint32_t)t & ~1u) + (load + odd) * kOneThreads;      // the block's first unit
+        if (first < rem) {
+            st8(q0 + first, u32x2{c.lo, c.hi});
+            s80[first >> 1] = (uint8_t)c.sc();
+        }
+    };
+    uint32_t open = 0;      // blocks too close to call
+#pragma unroll
+    for (int i = 0; i < kOneUnits; i += 2) {
+        float f[16];
+        const uint32_t held = odd * kOneThreads + ((uint32_t)t & ~1u);
+        if (i + 2 < kOneUnits) nv_unpack16<F16>(v[i], v[i + 1], f);
+        else nv_unpack16<F16>(stage[held], stage[held + 1], f);
+        const float bmax = i % 4 ? elem_hi<F16>(maxima[i / 4]) : elem_lo<F16>(maxima[i / 4]);
+        const NvCandidates16 c = nv_candidates16<2, false, true>(f, bmax, gs, scale_table);
+        const NvPick pick = nv_estimated_pick<EM>(f, bmax, c.c4, c.c6);
+        store(i, pick.four ? c.c4 : c.c6);
+        if (!pick.decided) open |= 1u << (i / 2);
+        __builtin_amdgcn_sched_barrier(0);      // a block at a time: more do not fit the registers
+    }
+    if (__builtin_amdgcn_ballot_w64(open != 0) == 0) return;
+#pragma unroll 1
+    for (uint32_t i = 0; i < kOneUnits; i += 2) {
+        if (__builtin_amdgcn_ballot_w64((open >> (i / 2)) & 1u) == 0) continue;
+        // (the block is read again: with every unit kept, 28 registers went to scratch memory)
+        const uint32_t first = ((uint32_t)t & ~1u) + (i + odd) * kOneThreads;
+        const uint16_t* __restrict__ w = (const uint16_t*)job.w + (base + (first < rem ? first : 0)) * 8;
+        float f[16];
+        nv_unpack16<F16>(ld16(w), ld16(w + 8), f);
+        const NvCandidates16 c = nv_candidates16<2, false, true>(f, nv_numbers_max(f), gs, scale_table);
+        const float e4 = nv_block_error<EM, 2>(f, c.c4, amax, gs.enc, denom, denom_inv), e6 = nv_block_error<EM, 2>(f, c.c6, amax, gs.enc, denom, denom_inv);
+        if ((open >> (i / 2)) & 1u) store(i, e4 < e6 ? c.c4 : c.c6);
+    }
+}
+
 // job as for the quantize pass: section = place of the tensor inside its record, pad = tensors sharing it (neighbours)
 // grid (workgroups of the largest tensor, tensors + rows behind)
-template <int F16, class Table>
+template <int FOS, int F16, class Table>
 __global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_kernel(const Table tab, float numer, int first_polls, int patience, uint32_t tensors,
                                                                                        uint32_t workers, uint32_t* moved_counter, uint32_t* moved_mirror) {
     const int t = threadIdx.x;
     if (blockIdx.y >= tensors) {
-        nv_one_rest<F16>(tab, tensors, workers, patience, t, numer, moved_counter);
+        nv_one_rest<FOS, F16>(tab, tensors, workers, patience, t, numer, moved_counter);
         return;
     }
     const FlatJob job = flat_job(tab);
@@ -1011,9 +1111,17 @@ __global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_
         }
     }
     // the block maxima, two to a register: what does not depend on the amax is done before the wait for it
+    __shared__ u32x4 stage[FOS ? 2 * kOneThreads : 1];
     uint32_t maxima[kOneUnits / 2], m2 = 0;
 #pragma unroll
     for (int i = 0; i < kOneUnits; i += 2) {
+        if constexpr (FOS != 0) {
+            nv_pair_blocks(stage, v[i], v[i + 1], t);
+            const uint32_t bmax = hmax_u16(max2_u16(nv_unit_max(v[i]), nv_unit_max(v[i + 1])));
+            maxima[i / 4] = i % 4 ? maxima[i / 4] | (bmax << 16) : bmax;
+            m2 = max2_u16(m2, bmax);
+            continue;
+        }
         maxima[i / 2] = nv_block_max(v[i]) | (nv_block_max(v[i + 1]) << 16);
         if constexpr (std::is_same<Table, FlatRef>::value) asm("" : "+v"(maxima[i / 2]));      // (else its halves are kept as well, in scratch memory)
         m2 = max2_u16(m2, maxima[i / 2]);
@@ -1041,8 +1149,10 @@ __global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_
     }
     const float amax = elem_lo<F16>(m);
     const NvScales scales = nv_scales(amax, numer), gs{uniform_f(scales.enc_sixth), uniform_f(scales.s_dec), uniform_f(scales.enc)};
-    const bool leaves = nv_one_leaves<F16>(m, gs);
-    if (!leaves) {
+    const bool leaves = nv_one_leaves<FOS, F16>(m, gs);
+    if constexpr (FOS != 0) {
+        if (!leaves) nv_one_four_over_six<FOS - 1, F16>(job, v, maxima, stage, base, rem, t, amax, gs, numer);
+    } else if (!leaves) {
         // Both lanes of a pair hold the maxima of the same blocks: of two units the even lane takes the first one's scale and the
         // odd lane the second one's, so that a scale is computed once and every lane stores a byte.
         const uint32_t odd = (uint32_t)t & 1u;
@@ -1475,7 +1585,7 @@ int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, in
     return nvfp4_quant_launch(dtype, ref, n, max_units * n, sections, e4m3_max, 0, mode, st);
 }
 
-// Whether a chunk of NVFP4 jobs (standard scaling, packed kernels, no carried amax) takes the one-pass form.  `slots` is the
+// Whether a chunk of NVFP4 jobs (packed kernels, no carried amax) takes the one-pass form.  `slots` is the
 // largest number of workgroups that share a record, `bytes` the input of the whole chunk.  All workgroups of a record
 // have to be on the chip together, and the records behind it should be loading meanwhile: half of what fits (640 workgroups,
 // 40 MB, on 256 CUs).  A pair of [2048, 7168] weights, 896 workgroups, gained less (313 -> 265 us for 16 pairs) and is one
@@ -1483,11 +1593,16 @@ int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, in
 // read in the memory-side cache, and the launch that clears the slots takes what is left of the gain (us, two passes / one): 4 x
 // [256, 1024] (2 MB) 6.5 / 8.8, 2 x [1024, 2048] 8.3 / 9.9, 4 of them (17 MB) 10.8 / 11.3, 1 x [2048, 4096] (17 MB) 11.5 / 11.1,
 // 4 x [1537, 2064] (25 MB) 14.2 / 13.3, 1 x [2048, 7168] (29 MB) 16.3 / 13.9, 8 x [1024, 2048] (34 MB) 16.2 / 14.8, 2 x [2048, 7168] (59 MB)
-// 24.0 / 19.0.
-constexpr int64_t kOneMinBytes = 24ll << 20;
-bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes) {
+// 24.0 / 19.0.  With Four Over Six the arithmetic of the first two tensors' loads and the last one's arithmetic have nothing beside them,
+// and a list pays from 170 to 230 MB on, the more workgroups its tensors have the later: 33 x [528, 3088] (108 MB) 44 / 48, 24 x [1536, 2048]
+// (151 MB) 59.5 / 57.3, 45 x [740, 1952] (130 MB) 53.4 / 54.3, 60 of them 68.2 / 65.6, 5 x [4096, 4096] (168 MB) 64.5 / 66.4, 6 x [2048, 7168] (176 MB)
+// 68.6 / 67.4, 8 of them 88.2 / 83.9, 7 x [4096, 4096] (235 MB) 88.0 / 87.1, 38 x [1536, 2048] (239 MB) 90.8 / 80.4.
+constexpr int64_t kOneMinBytes = 24ll << 20, kOneFosMinBytes = 200ll << 20;
+bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes, int flags) {
     int device = 0, cus = 0;
-    if (bytes < kOneMinBytes || max_units > kOneSlots * kOnePerBlock) return false;
+    const bool fos = (flags & MQ_NVFP4_4OVER6) != 0;
+    if (fos && nv_error_mode(flags) > 1) return false;       // (an error in fp16 has no estimate)
+    if (bytes < (fos ? kOneFosMinBytes : kOneMinBytes) || max_units > kOneSlots * kOnePerBlock) return false;
     if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
         (void)hipGetLastError();
         return false;
@@ -1499,42 +1614,51 @@ int64_t mq_nvfp4_one_pass_slots(int64_t units) { return (units + kOnePerBlock - 
 // workgroups behind the tensors' own, for each of n tensors of at most max_units: 64 of a list of 32 tensors (the launch has
 // 0.4 ns for one that finds nothing to do), and enough to fill half of the chip for one that is left
 constexpr int kOneWorkers = 2048;
-static uint32_t nv_one_workers(int n, int64_t max_units) {
-    const int64_t blocks = (max_units + nv_units_per_block(0) - 1) / nv_units_per_block(0);
+static uint32_t nv_one_workers(int n, int64_t max_units, int fos) {
+    const int64_t blocks = (max_units + nv_units_per_block(fos) - 1) / nv_units_per_block(fos);
     int64_t workers = kOneWorkers / n;
     workers = workers < 16 ? 16 : workers > kSectionWords ? kSectionWords : workers;
     return (uint32_t)(workers < blocks ? workers : blocks);
 }
 // descriptors as for mode 1
-template <class Table, int F16>
+template <class Table, int FOS, int F16>
 static int nvfp4_one_pass_launch_dtype(const Table& tab, int n, int64_t max_units, float numer, int first_polls, int patience, hipStream_t st) {
-    const uint32_t workers = nv_one_workers(n, max_units), blocks = (uint32_t)tab.max_blocks;
+    const uint32_t workers = nv_one_workers(n, max_units, FOS), blocks = (uint32_t)tab.max_blocks;
     const dim3 grid(blocks, (unsigned)(n + ((int64_t)n * workers + blocks - 1) / blocks));
     hipLaunchKernelGGL((nvfp4_one_pass_clear_kernel<Table>), dim3((unsigned)n), dim3(256), 0, st, tab);
-    hipLaunchKernelGGL((nvfp4_one_pass_kernel<F16, Table>), grid, dim3(kOneThreads), 0, st, tab, numer, first_polls, patience, (uint32_t)n, workers,
+    hipLaunchKernelGGL((nvfp4_one_pass_kernel<FOS, F16, Table>), grid, dim3(kOneThreads), 0, st, tab, numer, first_polls, patience, (uint32_t)n, workers,
                        mq_amax_feedback(), mq_amax_feedback_mirror());
     return mq_check_launch("nvfp4 quant (one pass)");
 }
 template <class Table>
-static int nvfp4_one_pass_launch(int dtype, const Table& tab, int n, int64_t max_units, int e4m3_max, int first_polls, int patience, hipStream_t st) {
+static int nvfp4_one_pass_launch(int dtype, const Table& tab, int n, int64_t max_units, int e4m3_max, int flags, int first_polls, int patience, hipStream_t st) {
     const float numer = (float)e4m3_max * 6.0f;
-    return dtype == MQ_F16 ? nvfp4_one_pass_launch_dtype<Table, 1>(tab, n, max_units, numer, first_polls, patience, st)
-                           : nvfp4_one_pass_launch_dtype<Table, 0>(tab, n, max_units, numer, first_polls, patience, st);
+    if constexpr (std::is_same<Table, FlatTable>::value) {
+        if (flags & MQ_NVFP4_4OVER6) {
+            const bool squared = nv_error_mode(flags) == 1;
+            if (dtype == MQ_F16) return squared ? nvfp4_one_pass_launch_dtype<Table, 2, 1>(tab, n, max_units, numer, first_polls, patience, st)
+                                                : nvfp4_one_pass_launch_dtype<Table, 1, 1>(tab, n, max_units, numer, first_polls, patience, st);
+            return squared ? nvfp4_one_pass_launch_dtype<Table, 2, 0>(tab, n, max_units, numer, first_polls, patience, st)
+                           : nvfp4_one_pass_launch_dtype<Table, 1, 0>(tab, n, max_units, numer, first_polls, patience, st);
+        }
+    }
+    return dtype == MQ_F16 ? nvfp4_one_pass_launch_dtype<Table, 0, 1>(tab, n, max_units, numer, first_polls, patience, st)
+                           : nvfp4_one_pass_launch_dtype<Table, 0, 0>(tab, n, max_units, numer, first_polls, patience, st);
 }
 static int nv_one_polls(int flags) { return (flags & MQ_NVFP4_NO_WAIT) ? 0 : kOnePolls; }
 // (with limits of its own for the waits: for the tests of how they end)
-int mq_nvfp4_one_pass_launch_waits(int dtype, FlatTable& tab, int64_t max_units, int e4m3_max, int first_polls, int patience, hipStream_t st) {
+int mq_nvfp4_one_pass_launch_waits(int dtype, FlatTable& tab, int64_t max_units, int e4m3_max, int flags, int first_polls, int patience, hipStream_t st) {
     if (!flat_grid(tab, kOnePerBlock)) return mq_fail(MQ_ERR_ARG, "tensor too large");
-    return nvfp4_one_pass_launch(dtype, tab, tab.n, max_units, e4m3_max, first_polls, patience, st);
+    return nvfp4_one_pass_launch(dtype, tab, tab.n, max_units, e4m3_max, flags, first_polls, patience, st);
 }
 int mq_nvfp4_one_pass_launch_group(int dtype, FlatTable& tab, int64_t max_units, int e4m3_max, int flags, hipStream_t st) {
-    return mq_nvfp4_one_pass_launch_waits(dtype, tab, max_units, e4m3_max, nv_one_polls(flags), kOnePatience, st);
+    return mq_nvfp4_one_pass_launch_waits(dtype, tab, max_units, e4m3_max, flags, nv_one_polls(flags), kOnePatience, st);
 }
 int mq_nvfp4_one_pass_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int e4m3_max, int flags,
                                    hipStream_t st) {
     FlatRef ref{device_jobs, 0, 0};
     if (!flat_grid(ref, max_units, kOnePerBlock)) return mq_fail(MQ_ERR_ARG, "tensor too large");
-    return nvfp4_one_pass_launch(dtype, ref, n, max_units, e4m3_max, nv_one_polls(flags), kOnePatience, st);
+    return nvfp4_one_pass_launch(dtype, ref, n, max_units, e4m3_max, flags, nv_one_polls(flags), kOnePatience, st);
 }
 
 extern "C" int mq_nvfp4_amax(const void* w, int dtype, int64_t numel, void* record, int section, void* stream) {

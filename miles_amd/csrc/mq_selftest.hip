@@ -98,7 +98,7 @@ extern "C" int mqp_selftest_convert(uint64_t* counts, void* stream) {
     return mqp_check_launch("selftest");
 }
 
-int mq_nvfp4_one_pass_launch_waits(int dtype, mq::FlatTable& tab, int64_t max_units, int e4m3_max, int first_polls, int patience, hipStream_t st);
+int mq_nvfp4_one_pass_launch_waits(int dtype, mq::FlatTable& tab, int64_t max_units, int e4m3_max, int flags, int first_polls, int patience, hipStream_t st);
 
 extern "C" int mqp_nvfp4_one_pass(const mq_job* jobs, int n, int first_polls, int patience, void* stream) {
     if (!jobs || n < 1 || n > mq::kMaxGroup || first_polls < 0 || patience < 0) return mqp_fail(MQP_ERR_ARG, "bad argument");
@@ -108,14 +108,14 @@ extern "C" int mqp_nvfp4_one_pass(const mq_job* jobs, int n, int first_polls, in
     for (int i = 0; i < n; i++) {
         const mq_job& j = jobs[i];
         const int64_t units = j.rows * j.cols / 8;
-        if (j.kind != MQ_JOB_NVFP4 || j.dtype != jobs[0].dtype || (j.dtype != MQ_BF16 && j.dtype != MQ_F16) || !j.in || !j.out || !j.scale || !j.aux ||
-            units <= 0 || units > 512 * 4096 || j.cols % 16 != 0 || (uintptr_t)j.in % 16 != 0 || (uintptr_t)j.out % 4 != 0)
+        if (j.kind != MQ_JOB_NVFP4 || j.p1 != jobs[0].p1 || (j.p1 & MQ_NVFP4_ERR_FP16) || j.dtype != jobs[0].dtype || (j.dtype != MQ_BF16 && j.dtype != MQ_F16) || !j.in || !j.out || !j.scale || !j.aux ||
+            units <= 0 || units > 512 * 4096 || j.cols % 16 != 0 || (uintptr_t)j.in % 16 != 0 || (uintptr_t)j.out % 8 != 0)
             return mqp_fail(MQP_ERR_ARG, "not a job of this form");
         for (int k = 0; k < i; k++)
             if (jobs[k].aux == j.aux) return mqp_fail(MQP_ERR_ARG, "a record of its own for every job");
         tab.job[i] = mq::FlatJob{j.in, j.out, j.scale, j.aux, units, j.aux2, 0, 1};
         max_units = units > max_units ? units : max_units;
     }
-    return mq_nvfp4_one_pass_launch_waits(jobs[0].dtype, tab, max_units, jobs[0].p0, first_polls, patience, (hipStream_t)stream) == MQ_OK
+    return mq_nvfp4_one_pass_launch_waits(jobs[0].dtype, tab, max_units, jobs[0].p0, jobs[0].p1, first_polls, patience, (hipStream_t)stream) == MQ_OK
                ? MQP_OK : mqp_fail(MQP_ERR_HIP, mq_last_error());
 }
