@@ -230,8 +230,9 @@ __global__ __launch_bounds__(kTileThreads) void fp8_block128_kernel(const Table 
 // own is written twice with one value.  Bound by the memory system, which takes unaligned rows at 4.9 TB/s (24 [4097, 4099] bf16 tensors, 3.3 with
 // non-temporal loads and 2.9 with non-temporal stores too) and aligned fp32 rows (LINES, non-temporal loads) at 6.1.  Twelve
 // [1545, 2563] bf16 tensors as one list: 779 us in the two-pass kernel below, one launch each; 72 us here, host included.
+// `aligned`: tensors that the fast kernel would take; a NaN's code and scale have that kernel's sign and payload.
 template <int MODE, int DT, bool LINES>
-__global__ __launch_bounds__(kTileThreads) void fp8_block128_any_kernel(const TileTable tab) {
+__global__ __launch_bounds__(kTileThreads) void fp8_block128_any_kernel(const TileTable tab, const bool aligned) {
     constexpr uint32_t kInfBits = DT == MQ_F32 ? 0x7F800000u : DT == MQ_F16 ? 0x7C00u : 0x7F80u;
     constexpr uint32_t kSize = DT == MQ_F32 ? 4u : 2u;
     constexpr int kF16 = DT == MQ_F16;
@@ -327,7 +328,7 @@ __global__ __launch_bounds__(kTileThreads) void fp8_block128_any_kernel(const Ti
     float s;
     if (MODE == 0) s = amax / kFp8Max;
     else if (MODE == 1) s = (amax > 1e-10f ? amax : 1e-10f) / kFp8Max;
-    else s = special ? amax : ceil_pow2_scale((amax > 1e-4f ? amax : 1e-4f) / kFp8Max);
+    else s = special ? (aligned && m > kInfBits ? u2f(0x7FC00000u) : amax) : ceil_pow2_scale((amax > 1e-4f ? amax : 1e-4f) / kFp8Max);
     const float y = 1.0f / s;
     if (t == 0) tile_scales[tile] = s;
     const bool zero_tile = MODE == 0 && !(amax > 0.0f) && amax == amax;       // 0 / 0: the negative NaN code
@@ -350,6 +351,10 @@ __global__ __launch_bounds__(kTileThreads) void fp8_block128_any_kernel(const Ti
 #pragma unroll
             for (uint32_t j = 0; j < kCols; j += 4)       // at most 448 (1 + 2^-22): rounds to 448 by itself
                 o[j / 4] = hw_e4m3x4(f[j], f[j + 1], f[j + 2], f[j + 3]);
+        } else if (MODE == 0 && DT != MQ_F32 && aligned) {
+#pragma unroll
+            for (uint32_t j = 0; j < kCols; j += 4)
+                o[j / 4] = hw_e4m3x4(element(i, j) / s, element(i, j + 1) / s, element(i, j + 2) / s, element(i, j + 3) / s);
         } else {
 #pragma unroll
             for (uint32_t j = 0; j < kCols; j++) {
@@ -908,11 +913,11 @@ static void tile_launch(int mode, bool f16, dim3 grid, hipStream_t st, const Tab
 // the memory system best unless a launch reads more lines at a time than it keeps open; see mq_fp8_tile_launch_group.
 constexpr unsigned kTwoPerCu = 56u << 10, kThreePerCu = 44u << 10;
 template <int DT, bool LINES>
-static void tile_any_launch(int mode, dim3 grid, unsigned lds, hipStream_t st, const TileTable& tab) {
+static void tile_any_launch(int mode, dim3 grid, unsigned lds, bool aligned, hipStream_t st, const TileTable& tab) {
     const dim3 blk(kTileThreads);
-    if (mode == 0) hipLaunchKernelGGL((fp8_block128_any_kernel<0, DT, LINES>), grid, blk, lds, st, tab);
-    else if (mode == 1) hipLaunchKernelGGL((fp8_block128_any_kernel<1, DT, LINES>), grid, blk, lds, st, tab);
-    else hipLaunchKernelGGL((fp8_block128_any_kernel<2, DT, LINES>), grid, blk, lds, st, tab);
+    if (mode == 0) hipLaunchKernelGGL((fp8_block128_any_kernel<0, DT, LINES>), grid, blk, lds, st, tab, aligned);
+    else if (mode == 1) hipLaunchKernelGGL((fp8_block128_any_kernel<1, DT, LINES>), grid, blk, lds, st, tab, aligned);
+    else hipLaunchKernelGGL((fp8_block128_any_kernel<2, DT, LINES>), grid, blk, lds, st, tab, aligned);
 }
 
 // n finished descriptors in device memory, all of one 16-bit dtype; max_tiles: the largest tensor's tile count
@@ -924,18 +929,34 @@ int mq_fp8_tile_launch_table(int mode, int dtype, const TileJob* device_jobs, in
     return mq_check_launch("fp8 block quant");
 }
 
+bool mq_fp8_tile_rows_share_lines(const void* w, int64_t ldw) { return (uintptr_t)w % 128 != 0 || ldw % 64 != 0; }
+// The most tiles of a launch for which the any-alignment kernel, with its temporal loads and stores, ends sooner whatever the
+// rows (us, fast kernel / that one): 64 tiles of [1024, 1024] 5.2 / 4.7, 128 of [1024, 2048] 5.4 / 5.0, 256 of [2048, 2048] 5.9 / 5.8,
+// 512 of [2048, 4096] 7.9 / 8.3.
+constexpr int64_t kAnyTiles = 256;
+
 // tab.job[i] filled by the caller (w, q, scale, ldw, M, K, row blocks), all of one dtype; fills the division constants
 // and `end`, launches.  `aligned`: every tensor passed mq_fp8_tile_fast_ok, otherwise mq_fp8_tile_any_ok.
+// Aligned tensors take the any-alignment kernel as well where most of their tiles have rows that begin inside a 128-byte line: two
+// tiles share the line at their border, and the fast kernel's non-temporal loads fetch it, and its partial stores write it,
+// once for each (us, fast / any): 64 x [768, 2056] 98.7 / 55.0, 64 x [768, 2080] 76.6 / 54.4, 12 x [1545, 2568] 40.6 / 28.1, 4 x [3000, 7184]
+// 67 / 45.8, 2 x [8192, 8200] 111.5 / 80.2, 4 x [1545, 2592] 14.7 / 13.8, 1 x [1545, 2592] 6.4 / 6.5; with rows of whole lines
+// 2 x [8192, 8192] 64.9 / 74.4, 12 x [1545, 2624] the fast one 28.2.
 int mq_fp8_tile_launch_group(int mode, int dtype, bool aligned, TileTable& tab, hipStream_t st) {
-    int64_t tiles = 0;
+    int64_t tiles = 0, shared = 0;     // tiles, and those of tensors whose rows share lines
+    bool blocked = false;
     for (int i = 0; i < tab.n; i++) {
-        tiles += mq_fp8_tile_job_finish(tab.job[i]);
+        TileJob& j = tab.job[i];
+        const int64_t own = mq_fp8_tile_job_finish(j);
+        tiles += own;
         if (tiles >= 0x7FFFFFF0) return mq_fail(MQ_ERR_ARG, "too many tiles");
         tab.end[i] = (int32_t)tiles;
+        blocked |= j.tiles_per_block != 0;
+        if (mq_fp8_tile_rows_share_lines(j.w, j.ldw)) shared += own;
     }
     if (tiles == 0) return MQ_OK;
     seal_table(tab);
-    if (aligned) {
+    if (aligned && (blocked || (shared * 2 <= tiles && tiles > kAnyTiles))) {      // (row blocks are the fast kernel's)
         tile_launch(mode, dtype == MQ_F16, dim3((unsigned)xcd_grid(tiles)), st, tab);
         return mq_check_launch("fp8 block quant");
     }
@@ -973,10 +994,10 @@ int mq_fp8_tile_launch_group(int mode, int dtype, bool aligned, TileTable& tab, 
         if (lines) lds = tiles >= 16384 && narrowest >= 32768 ? kTwoPerCu : 0u;
         else if (narrowest > kTile) lds = mib >= 160 && !slim ? kTwoPerCu : mib >= (narrowest <= 2 * kTile ? 48 : 96) ? kThreePerCu : 0u;
     }
-    if (dtype == MQ_BF16) tile_any_launch<MQ_BF16, false>(mode, grid, lds, st, tab);
-    else if (dtype == MQ_F16) tile_any_launch<MQ_F16, false>(mode, grid, lds, st, tab);
-    else if (lines) tile_any_launch<MQ_F32, true>(mode, grid, lds, st, tab);
-    else tile_any_launch<MQ_F32, false>(mode, grid, lds, st, tab);
+    if (dtype == MQ_BF16) tile_any_launch<MQ_BF16, false>(mode, grid, lds, aligned, st, tab);
+    else if (dtype == MQ_F16) tile_any_launch<MQ_F16, false>(mode, grid, lds, aligned, st, tab);
+    else if (lines) tile_any_launch<MQ_F32, true>(mode, grid, lds, aligned, st, tab);
+    else tile_any_launch<MQ_F32, false>(mode, grid, lds, aligned, st, tab);
     return mq_check_launch("fp8 block quant");
 }
 

@@ -24,6 +24,7 @@ bool mq_fp8_tile_fast_ok(const void* w, int dtype, int64_t sxm, int64_t sxn, con
 bool mq_fp8_tile_any_ok(const void* w, int dtype, int64_t sxm, int64_t sxn, int64_t M, int64_t K, int bm, int bk);
 int mq_fp8_tile_launch_group(int mode, int dtype, bool aligned, TileTable& tab, hipStream_t st);
 int64_t mq_fp8_tile_job_finish(TileJob& j);
+bool mq_fp8_tile_rows_share_lines(const void* w, int64_t ldw);
 int mq_fp8_tile_launch_table(int mode, int dtype, const TileJob* device_jobs, int n, int64_t max_tiles, hipStream_t st);
 bool mq_fp8_dequant_fast_ok(const void* x, const void* y, int64_t M, int64_t N, int block);
 bool mq_fp8_dequant_any_ok(const void* y, int64_t M, int64_t N, int block);
@@ -715,18 +716,22 @@ extern "C" int mq_run_jobs_tabled(const mq_job* jobs, int64_t n, const void* dev
             // tile jobs of similar tile counts (an MoE layer's experts) beyond what the kernel arguments hold: one launch
             // on a (largest tile count) x (tensors) grid; mixed shapes keep the searched form below, 64 tensors at a time
             int64_t j = i + 1, sum = tiles_of(head), mx = sum;
+            bool plain = head.rows_per_block == 0, lines = !mq_fp8_tile_rows_share_lines(head.in, head.ld);
             while (j < n && j - i < kTableGroup && same_group(head, jobs[j]) && job_fast(jobs[j]) && jobs[j].rows > 0 &&
                    jobs[j].cols > 0) {
                 const int64_t e = tiles_of(jobs[j]);
                 const int64_t nmx = e > mx ? e : mx;
                 if (nmx * (j - i + 1) * 4 > (sum + e) * 5) break;
+                plain &= jobs[j].rows_per_block == 0;
+                lines |= !mq_fp8_tile_rows_share_lines(jobs[j].in, jobs[j].ld);
                 sum += e;
                 mx = nmx;
                 j++;
             }
             j = tile_run_end(jobs, i, j, sum);
-            // (tensors of 256 tiles and more fill a searched launch of 64 well enough, and run 1-2 % faster in that form)
-            if (j - i > kMaxGroup && mx < 256) {
+            // (tensors of 256 tiles and more fill a searched launch of 64 well enough, and run 1-2 % faster in that form; those of
+            // 32 and more whose rows share lines as well, in the any-alignment kernel: 200 x [512, 1032] 124 and 79 us, 300 x [384, 776] 79.6 and 81.2)
+            if (j - i > kMaxGroup && mx < (plain && !lines ? 32 : 256)) {
                 const int mode = head.kind == MQ_JOB_FP8_BLOCK ? 0 : head.kind == MQ_JOB_FP8_BLOCKWISE_CAST ? 1 : 2;
                 int rc = mq_fp8_tile_launch_table(mode, head.dtype, (const TileJob*)table + i, (int)(j - i), mx, st);
                 if (rc) return rc;
