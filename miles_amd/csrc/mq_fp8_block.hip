@@ -1049,7 +1049,7 @@ extern "C" int mq_fp8_block_quant_pow2(const void* w, int dtype, int64_t ldw, vo
 // How the rows of a tensor are held (fp8_channel_kernel): lanes per row and units per lane, and whether the rows are whole
 // aligned units.  A wavefront per row while that leaves a lane no more than four units; sixteen units a lane are 64
 // registers.  0: rows of less than a unit or of more than 4096, which take the element-wise kernels.
-enum ChannelForm { kChannelNone = 0, kChannel64x4 = 1, kChannel256x4, kChannel256x8, kChannel256x16, kChannelLines = 8 };
+enum ChannelForm { kChannelNone = 0, kChannel64x4 = 1, kChannel64x8, kChannel256x4, kChannel256x8, kChannel256x16, kChannelLines = 8 };
 int mq_fp8_channel_form(const void* w, int dtype, int64_t ldw, const void* q, int64_t M, int64_t K) {
     if (dtype < MQ_BF16 || dtype > MQ_F32 || M <= 0 || M > 0x7FFFFFFF) return kChannelNone;
     const int64_t E = dtype == MQ_F32 ? 4 : 8, units = (K + E - 1) / E;
@@ -1059,22 +1059,41 @@ int mq_fp8_channel_form(const void* w, int dtype, int64_t ldw, const void* q, in
     const bool lines = K % E == 0 && ldw % E == 0 && (uintptr_t)w % 16 == 0 && (uintptr_t)q % E == 0;
     return (units <= 256 ? kChannel64x4 : units <= 1024 ? kChannel256x4 : units <= 2048 ? kChannel256x8 : kChannel256x16) | (lines ? kChannelLines : 0);
 }
-int64_t mq_fp8_channel_blocks(int form, int64_t M) { return (form & ~kChannelLines) == kChannel64x4 ? (M + 3) / 4 : M; }
+int64_t mq_fp8_channel_blocks(int form, int64_t M) { return (form & ~kChannelLines) <= kChannel64x8 ? (M + 3) / 4 : M; }
 template <int DT, bool LINES>
 static void channel_launch(int form, const ChannelTable& tab, hipStream_t st) {
     const dim3 grid((unsigned)tab.max_blocks, (unsigned)tab.n), blk(256);
     switch (form) {
         case kChannel64x4: hipLaunchKernelGGL((fp8_channel_kernel<64, DT, 4, LINES>), grid, blk, 0, st, tab); break;
+        case kChannel64x8: hipLaunchKernelGGL((fp8_channel_kernel<64, DT, 8, LINES>), grid, blk, 0, st, tab); break;
         case kChannel256x4: hipLaunchKernelGGL((fp8_channel_kernel<256, DT, 4, LINES>), grid, blk, 0, st, tab); break;
         case kChannel256x8: hipLaunchKernelGGL((fp8_channel_kernel<256, DT, 8, LINES>), grid, blk, 0, st, tab); break;
         default: hipLaunchKernelGGL((fp8_channel_kernel<256, DT, 16, LINES>), grid, blk, 0, st, tab); break;
     }
 }
+// The form of a whole list (neither with kChannelLines), rows of at most `units`.  Of 257 to 384 units half of the lanes of a 256-lane row
+// and more have nothing in their second unit: a wavefront per row from 8192 rows on (us, 256 lanes / 64; 18540 rows of 2056 bf16
+// 26.5 / 23.5, of 2560 28.2 / 25.4, of 2563 30.7 / 26.1, of 2880 30.2 / 28.7, of 3200 31.6 / 31.3, of 3584 33.4 / 34.9, of 1032 fp32
+// 23.4 / 20.1; 7470 rows of 2880 14.3 / 14.2, 1545 of 2560 4.8 / 5.3).  Few rows leave a wavefront alone with its row: 256 lanes
+// from 129 units on up to 2048 rows (64 lanes / 256; 64 rows of 2048 3.3 / 2.5, 512 4.3 / 3.2, 2048 5.0 / 4.6, 4096 6.4 / 7.2; of
+// 1024 64 rows 2.9 / 2.8, 1024 3.4 / 3.4).
+static int channel_list_form(int form, int64_t units, int64_t rows) {
+    if (form == kChannel64x4 && units > 128 && rows <= 2048) return kChannel256x4;
+    if (form == kChannel256x4 && units <= 384 && rows >= 8192) return kChannel64x8;
+    return form;
+}
 // n <= kMaxGroup tensors of one dtype and one form
 int mq_fp8_channel_launch_group(int dtype, int form, const MqScaledArgs* a, int n, hipStream_t st) {
     ChannelTable tab{};
     tab.n = n;
-    int64_t mx = 0;
+    const bool lines = (form & kChannelLines) != 0;
+    int64_t mx = 0, rows = 0, cols = 0;
+    for (int i = 0; i < n; i++) {
+        rows += a[i].M;
+        cols = a[i].K > cols ? a[i].K : cols;
+    }
+    const int64_t E = dtype == MQ_F32 ? 4 : 8;
+    form = channel_list_form(form & ~kChannelLines, (cols + E - 1) / E, rows);
     for (int i = 0; i < n; i++) {
         tab.job[i] = ChannelJob{a[i].w, (uint8_t*)a[i].q, a[i].scale, a[i].ldw, (int32_t)a[i].K, (int32_t)a[i].M, a[i].floor_v, 0};
         const int64_t blocks = mq_fp8_channel_blocks(form, a[i].M);
@@ -1082,8 +1101,6 @@ int mq_fp8_channel_launch_group(int dtype, int form, const MqScaledArgs* a, int 
     }
     tab.chunk = (int32_t)flat_chunk(mx);
     tab.max_blocks = (int32_t)flat_padded(mx, tab.chunk);
-    const bool lines = (form & kChannelLines) != 0;
-    form &= ~kChannelLines;
     if (dtype == MQ_F32) lines ? channel_launch<MQ_F32, true>(form, tab, st) : channel_launch<MQ_F32, false>(form, tab, st);
     else if (dtype == MQ_F16) lines ? channel_launch<MQ_F16, true>(form, tab, st) : channel_launch<MQ_F16, false>(form, tab, st);
     else lines ? channel_launch<MQ_BF16, true>(form, tab, st) : channel_launch<MQ_BF16, false>(form, tab, st);
