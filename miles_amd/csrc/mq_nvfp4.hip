@@ -1353,8 +1353,8 @@ __global__ __launch_bounds__(256) void nvfp4_quant_generic_kernel(const void* __
 // Nothing but x (and the amax, see nv_fake_scales) is read and nothing but y written.  job: w = x, q = y, units.
 // Standard blocks: two lanes own one 1x16 block.  Four Over Six: nvfp4_fos_units.
 // Both are bound by memory, the reads by the memory-side cache where the amax pass left its input there: sixteen [1536, 2048]
-// weights in one launch 28.4 us (33 from HBM; one launch per weight 4.6 us each), four [4096, 7168] with Four Over Six 67 us
-// (78 from HBM; 120 with two lanes per block and the exact error sums throughout, where vector instructions were the bound).
+// weights in one launch 28.4 us (33 from HBM; one launch per weight 4.6 us each), four [4096, 7168] with Four Over Six 66 us
+// (78 from HBM; 67 without the forms for an amax of the tensor's own; 120 with two lanes per block and the exact error sums throughout, where vector instructions were the bound).
 template <int FOS, int F16>
 __global__ __launch_bounds__(kNvThreads) void nvfp4_fake_kernel(const FlatTable tab, float numer, float inv_numer) {
     const FlatJob job = flat_job(tab);
@@ -1517,8 +1517,8 @@ static void launch_nvfp4_quant(int dtype, const Table& tab, int flags, float num
 //   gate and up in pairs, bf16: 2 x [2048, 7168] (59 MB) 25.1 / 25.6, 4 of them 44.3 / 43.7, 16 of them 168 / 158, 64 of them
 //     (1.9 GB) 646 / 615; fp32: 34 MB 16.6 / 17.3, 67 MB 26.8 / 27.0, 117 MB 42.1 / 41.2, 470 MB 156 / 148, 940 MB 314 / 293.
 //     (A pair folds two sections, a quarter of the bytes that a workgroup quantizes.)
-//   Four Over Six of 16-bit tensors, bound by vector instructions: 34 MB 19.7 / 20.9, 51 MB 25.7 / 26.0, 67 MB 34.5 / 34.1,
-//     134 MB 53.6 / 52.3, 268 MB 102.6 / 99.1, 470 MB 181 / 170, 1.9 GB 705 / 654.
+//   Four Over Six of 16-bit tensors, bound by vector instructions: 34 MB 19.8 / 20.3, 50 MB 25.6 / 26.0, 67 MB 31.5 / 31.4,
+//     134 MB 55.4 / 53.6, 189 MB 75.6 / 72.6 (longer lists are read once, or by the carried form).
 //   Four Over Six of fp32 tensors, as long as the second pass finds all of its input in the memory-side cache: 78 MB 34.1 / 34.8
 //     (in pairs 35.8 / 35.3), 117 MB 46.3 / 46.2 (47.6 / 46.3), 235 MB 85.4 / 83.9 (86.8 / 84.0), 268 MB 112 / 111; but 403 MB
 //     143.0 / 143.1, 470 MB 169 / 173 (170 / 173), 604 MB 207 / 211.
