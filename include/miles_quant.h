@@ -198,7 +198,8 @@ int mq_fp8_act_quant(const void* x, int dtype, void* y, void* scale, int64_t num
  * mq_nvfp4_quant: folds the record, then quantizes: w [M,K] contiguous, K % 16 == 0; q [M,K/2] (element 2i in
  *   the low nibble);
  *   block_scale [M,K/16] e4m3fn bytes; global_scale (may be NULL) receives weight_scale_2 =
- *   1 / min(e4m3_max*6/amax, FLT_MAX) as one fp32 (nvfp4.py:19-39).
+ *   1 / min(e4m3_max*6/amax, FLT_MAX) as one fp32 (nvfp4.py:19-39).  The record may hold another amax than that of w: block
+ *   scales stop at 448.
  * flags: MQ_NVFP4_4OVER6 selects Transformer Engine's Four Over Six block scaling (NVTE_NVFP4_4OVER6; restated in
  *   miles/kernels/quant/nvfp4_qdq.py:893-990): every block is quantized for a maximum of 6 and of 4 and keeps the
  *   candidate with the smaller error; MQ_NVFP4_ERR_MSE squares the error terms (NVTE_NVFP4_4OVER6_ERR_MODE=MSE),

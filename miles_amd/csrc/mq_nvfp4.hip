@@ -693,10 +693,10 @@ __device__ __forceinline__ NvUnitCodes nvfp4_quant_unit(const u32x4 v, const NvS
 }
 
 // kNvThreads * kNvUnroll units starting at `base` of one tensor; returns the largest |element| this lane saw (bf16 bits)
-// FOS = 0: standard quantizer; FOS = 1 + error mode: Four Over Six, which returns nothing of use where TRUSTED
-template <int FOS, int F16, bool TRUSTED, class Scales>
-__device__ __forceinline__ uint32_t nvfp4_quant_units(const FlatJob& job, const int64_t base, const int t, const float denom, Scales scales) {
-    if (FOS) return nvfp4_fos_units<(FOS > 0 ? FOS - 1 : 0), F16, false>(job, base, t, denom, 0.0f, TRUSTED, scales);
+// FOS = 0: standard quantizer; FOS = 1 + error mode: Four Over Six, which returns nothing of use where `trusted` (nvfp4_fos_units)
+template <int FOS, int F16, class Scales>
+__device__ __forceinline__ uint32_t nvfp4_quant_units(const FlatJob& job, const int64_t base, const int t, const float denom, const bool trusted, Scales scales) {
+    if (FOS) return nvfp4_fos_units<(FOS > 0 ? FOS - 1 : 0), F16, false>(job, base, t, denom, 0.0f, trusted, scales);
     const uint16_t* __restrict__ w = (const uint16_t*)job.w;
     uint32_t* __restrict__ q = (uint32_t*)job.q;
     uint8_t* __restrict__ s8 = (uint8_t*)job.s;
@@ -750,8 +750,10 @@ __device__ __forceinline__ uint32_t nvfp4_amax_units(const FlatJob& job, const i
 // PASS 0 is the second pass of the plain two-pass form (amax kernel, then this): every workgroup folds the partial maxima,
 // and the first one of each tensor publishes what comes of them, also for a tensor without elements.
 // PASS 3 is the same behind nvfp4_publish_kernel.
+// `own` (passes 0 and 3): the partial maxima are those of an amax pass over these very elements.  A caller of mq_nvfp4_quant
+// may hand over a record that holds another amax, below some elements or without the NaN among them.
 template <int FOS, int PASS, class Table, int F16>
-__global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Table tab, float denom, uint32_t* moved_counter, uint32_t* moved_mirror) {
+__global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Table tab, float denom, const bool own, uint32_t* moved_counter, uint32_t* moved_mirror) {
     const FlatJob job = flat_job(tab);       // a copy in registers: a descriptor in device memory must not be re-read after the stores
     const int t = threadIdx.x;
     constexpr int64_t kPerBlock = nv_units_per_block(FOS);
@@ -760,7 +762,7 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
         // an XCD takes a run of consecutive blocks in every trip of the grid, as the flat grids do (second pass 2 pct faster)
         const int64_t first = xcd_chunked_block(gridDim.x == kSectionWords ? kSectionWords / kXcds : tab.chunk);
         for (int64_t base = first * kPerBlock; base < job.units; base += (int64_t)gridDim.x * kPerBlock)
-            nvfp4_quant_units<FOS, F16, true>(job, base, t, denom, [&] { return nv_record_scales(job); });
+            nvfp4_quant_units<FOS, F16>(job, base, t, denom, true, [&] { return nv_record_scales(job); });
         return;
     }
     const int64_t base = flat_block(tab) * kPerBlock;
@@ -776,12 +778,12 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
             return a;
         };
         if (job.units == 0) fold();
-        else nvfp4_quant_units<FOS, F16, true>(job, base, t, denom, fold);
+        else nvfp4_quant_units<FOS, F16>(job, base, t, denom, own, fold);
         return;
     }
     if (base >= job.units) return;
     if (PASS == 3) {
-        nvfp4_quant_units<FOS, F16, true>(job, base, t, denom, [&] { return nv_record_scales(job); });
+        nvfp4_quant_units<FOS, F16>(job, base, t, denom, own, [&] { return nv_record_scales(job); });
         return;
     }
     uint32_t seen;
@@ -789,7 +791,7 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
         seen = 0;
         for (int64_t piece = base; piece < base + kPerBlock && piece < job.units; piece += kNvThreads * kNvUnroll)
             seen = umax(seen, nvfp4_amax_units(job, piece, t));
-    } else seen = nvfp4_quant_units<FOS, F16, false>(job, base, t, denom, [&] { return nv_record_scales(job); });
+    } else seen = nvfp4_quant_units<FOS, F16>(job, base, t, denom, false, [&] { return nv_record_scales(job); });
     if (PASS == 1) {
         __shared__ uint32_t wave_seen[kNvThreads / 64];
         seen = wave_max(seen);
@@ -1005,7 +1007,7 @@ __device__ __forceinline__ void nv_one_rest(const Table& tab, const uint32_t ten
     if ((got & kOneFull) == 0 && worker == 0 && t == 0) nv_publish_plain(job, a.amax, a.gs, numer, moved_counter);
     constexpr int64_t kPerBlock = nv_units_per_block(FOS);
     for (int64_t base = worker * kPerBlock; base < job.units; base += workers * kPerBlock)
-        nvfp4_quant_units<FOS, F16, true>(job, base, t, numer, [&] { return a; });
+        nvfp4_quant_units<FOS, F16>(job, base, t, numer, true, [&] { return a; });
 }
 // By a record's first workgroup, when it has nothing else to do: the record of a maximum that it has published, for all
 // tensors that share it; the slots, which nobody reads any more, are cleared for a carried run.
@@ -1463,20 +1465,20 @@ int mq_nvfp4_amax_launch_table(int dtype, const FlatJob* device_jobs, int n, int
 }
 
 template <int PASS, class Table, int F16>
-static void launch_nvfp4_quant_dtype(const Table& tab, int flags, float numer, bool counted, dim3 grid, hipStream_t st) {
+static void launch_nvfp4_quant_dtype(const Table& tab, int flags, float numer, bool own, bool counted, dim3 grid, hipStream_t st) {
     const dim3 blk(kNvThreads);
     uint32_t *const moved = counted ? mq_amax_feedback() : nullptr, *const mirror = mq_amax_feedback_mirror();
     // Four Over Six keeps to launches of kernel-argument tables (its five error modes are not built in the other form)
     const int fos = (flags & MQ_NVFP4_4OVER6) ? 1 + nv_error_mode(flags) : 0;
     if constexpr (std::is_same<Table, FlatRef>::value) {
-        hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<0, PASS, Table, F16>), grid, blk, 0, st, tab, numer, moved, mirror);
+        hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<0, PASS, Table, F16>), grid, blk, 0, st, tab, numer, own, moved, mirror);
     } else {
         switch (fos) {
-            case 0: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<0, PASS, Table, F16>), grid, blk, 0, st, tab, numer, moved, mirror); break;
-            case 1: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<1, PASS, Table, F16>), grid, blk, 0, st, tab, numer, moved, mirror); break;
-            case 2: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<2, PASS, Table, F16>), grid, blk, 0, st, tab, numer, moved, mirror); break;
-            case 3: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<3, PASS, Table, F16>), grid, blk, 0, st, tab, numer, moved, mirror); break;
-            default: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<4, PASS, Table, F16>), grid, blk, 0, st, tab, numer, moved, mirror); break;
+            case 0: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<0, PASS, Table, F16>), grid, blk, 0, st, tab, numer, own, moved, mirror); break;
+            case 1: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<1, PASS, Table, F16>), grid, blk, 0, st, tab, numer, own, moved, mirror); break;
+            case 2: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<2, PASS, Table, F16>), grid, blk, 0, st, tab, numer, own, moved, mirror); break;
+            case 3: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<3, PASS, Table, F16>), grid, blk, 0, st, tab, numer, own, moved, mirror); break;
+            default: hipLaunchKernelGGL((nvfp4_quant_bf16_kernel<4, PASS, Table, F16>), grid, blk, 0, st, tab, numer, own, moved, mirror); break;
         }
     }
 }
@@ -1497,9 +1499,9 @@ static void launch_nvfp4_quant_f32(const Table& tab, int flags, float numer, boo
         }
     }
 }
-// counted: pass 0 adds to the counters of the call's feedback (in a carried run the fold does)
+// own: see nvfp4_quant_bf16_kernel; counted: pass 0 adds to the counters of the call's feedback (in a carried run the fold does)
 template <int PASS, class Table>
-static void launch_nvfp4_quant(int dtype, const Table& tab, int flags, float numer, bool counted, dim3 grid, hipStream_t st) {
+static void launch_nvfp4_quant(int dtype, const Table& tab, int flags, float numer, bool own, bool counted, dim3 grid, hipStream_t st) {
     // (fp32 has no instances of passes 1 and 2: nvfp4_quant_launch refuses mode 2 for it)
     if constexpr (PASS == 0 || PASS == 3) {
         if (dtype == MQ_F32) {
@@ -1507,8 +1509,8 @@ static void launch_nvfp4_quant(int dtype, const Table& tab, int flags, float num
             return;
         }
     }
-    if (dtype == MQ_F16) launch_nvfp4_quant_dtype<PASS, Table, 1>(tab, flags, numer, counted, grid, st);
-    else launch_nvfp4_quant_dtype<PASS, Table, 0>(tab, flags, numer, counted, grid, st);
+    if (dtype == MQ_F16) launch_nvfp4_quant_dtype<PASS, Table, 1>(tab, flags, numer, own, counted, grid, st);
+    else launch_nvfp4_quant_dtype<PASS, Table, 0>(tab, flags, numer, own, counted, grid, st);
 }
 
 // Whether a plain run's amax is folded by a launch between the two passes (nvfp4_publish_kernel), or by every workgroup of the
@@ -1540,28 +1542,29 @@ static int nvfp4_quant_launch(int dtype, const Table& tab, int n, int64_t all_un
     const dim3 folds((unsigned)n), blk(256);
     const dim3 grid((unsigned)tab.max_blocks, (unsigned)n);
     if (mode == 2) {
-        if (tab.max_blocks > 0) launch_nvfp4_quant<1>(dtype, tab, flags, numer, false, grid, st);
+        if (tab.max_blocks > 0) launch_nvfp4_quant<1>(dtype, tab, flags, numer, false, false, grid, st);
         hipLaunchKernelGGL((nvfp4_fold_kernel<2, Table>), folds, blk, 0, st, tab, numer, mq_amax_feedback(), mq_amax_feedback_mirror());
         if (tab.max_blocks > 0) {
             const unsigned redo_blocks = tab.max_blocks < kSectionWords ? (unsigned)tab.max_blocks : (unsigned)kSectionWords;
-            launch_nvfp4_quant<2>(dtype, tab, flags, numer, false, dim3(redo_blocks, (unsigned)n), st);
+            launch_nvfp4_quant<2>(dtype, tab, flags, numer, true, false, dim3(redo_blocks, (unsigned)n), st);
         }
         return mq_check_launch("nvfp4 quant (carried-over amax)");
     }
     if (nv_published(dtype, (flags & MQ_NVFP4_4OVER6) != 0, sections, n, all_units * (dtype == MQ_F32 ? 32 : 16))) {
         hipLaunchKernelGGL((nvfp4_publish_kernel<Table>), dim3(1, (unsigned)n), dim3(kWave), 0, st, tab, numer,
                            mode == 1 ? mq_amax_feedback() : nullptr, mq_amax_feedback_mirror());
-        launch_nvfp4_quant<3>(dtype, tab, flags, numer, false, grid, st);
+        launch_nvfp4_quant<3>(dtype, tab, flags, numer, mode == 1, false, grid, st);
         return mq_check_launch("nvfp4 quant");
     }
     // (a list of empty tensors still has its scales published, by the first workgroup of each)
-    launch_nvfp4_quant<0>(dtype, tab, flags, numer, mode == 1, dim3(grid.x > 0 ? grid.x : 1u, grid.y), st);
+    launch_nvfp4_quant<0>(dtype, tab, flags, numer, mode == 1, mode == 1, dim3(grid.x > 0 ? grid.x : 1u, grid.y), st);
     return mq_check_launch("nvfp4 quant");
 }
 
 // tab.job[i]: w, q, s = block scales, aux = amax record, aux2 = fp32 global scale out (may be null), units = numel / 8.
 // section = place of the tensor inside its record, pad = tensors sharing the record (adjacent entries).
-// mode 0 (single calls) and 1 (job driver), after the amax pass: quantize; mode 1 is counted in the call's feedback.
+// mode 0 (single calls, whose record is the caller's) and 1 (job driver), after the amax pass: quantize; mode 1 is counted in
+//   the call's feedback.
 // (fp32 tensors take modes 0 and 1.)
 // mode 2 (job driver, carried-over amax): quantize with the record's old scales while collecting the new partial maxima,
 //   fold and compare, quantize again where they differ.

@@ -59,3 +59,38 @@ def test_amax_of_the_callers(oracle, top, err, fast):  # noqa: F811
             number = ~w.isnan()             # (a NaN's own code is the conversion's)
             _assert_same(got.cpu()[number].nan_to_num(nan=77.0), want[number].nan_to_num(nan=77.0), f"amax {amax}, specials {i}")
         w[3, 100], w[20, 7] = float("nan"), float("inf")
+
+
+@pytest.mark.parametrize("copies", [1, 1000])       # (from 64 MiB on the record is finished in a launch of its own)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("top, err, fast", MODES)
+def test_record_of_the_callers(oracle, top, err, fast, dtype, copies):  # noqa: F811
+    """mq_nvfp4_quant with a record that the caller has written: an amax of few bits below the elements, above them, and without
+    the NaN and the infinity among them."""
+    from miles_amd import _lib
+    from miles_amd.utils.nvfp4 import AMAX_RECORD_WORDS
+
+    flags = _lib.NVFP4_4OVER6 | (_lib.NVFP4_ERR_MSE if err == "MSE" else 0) | (_lib.NVFP4_ERR_FP16 if fast else 0)
+    w = _weight((33, 1040), 1.0, 78).to(dtype)
+    record = torch.zeros(AMAX_RECORD_WORDS, dtype=torch.int32, device=DEV)
+    rows, cols = w.shape
+    q = torch.empty((copies * rows, cols // 2), dtype=torch.uint8, device=DEV)
+    s = torch.empty((copies * rows, cols // 16), dtype=torch.uint8, device=DEV)
+    g = torch.empty((), device=DEV)
+    for i in range(2):
+        dev = w.to(DEV).repeat(copies, 1)
+        nan = w.isnan().view(rows, -1, 16).any(-1)      # blocks with a NaN: the largest scale, whose codes are the conversion's
+        number = ~nan.repeat_interleave(16, dim=1)
+        for amax in (0.125, 0.96875, 8.0):
+            record[7] = int(torch.tensor(amax).view(torch.int32))
+            _lib.check(_lib.load().mq_nvfp4_quant(dev.data_ptr(), _lib.DTYPE_CODE[dtype], record.data_ptr(), 1, q.data_ptr(), s.data_ptr(),
+                                                  g.data_ptr(), copies * rows, cols, top, flags, _lib.stream_ptr()))
+            q_o, s_o, g_o = oracle.nvfp4_quantize_1d(w, amax, top, flags)
+            s_o = torch.where(nan, 0x7E, s_o.view(torch.uint8))
+            nibbles = torch.stack((q & 15, q >> 4), -1).view(copies, rows, cols)
+            nibbles_o = torch.stack((q_o & 15, q_o >> 4), -1).view(rows, cols)
+            what = f"amax {amax}, specials {i}"
+            assert torch.equal(s.view(copies, rows, -1), s_o.to(DEV).expand(copies, -1, -1)), f"scales, {what}"
+            assert torch.equal(nibbles[:, number.to(DEV)], nibbles_o[number].to(DEV).expand(copies, -1)), f"codes, {what}"
+            _assert_same(g, g_o, f"global scale, {what}")
+        w[3, 100], w[20, 7] = float("nan"), float("inf")
