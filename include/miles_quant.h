@@ -188,7 +188,7 @@ int mq_fp8_act_quant(const void* x, int dtype, void* y, void* scale, int64_t num
 /* NVFP4                                              miles/utils/nvfp4.py:54-114
  * The global amax travels on the device in an "amax record": MQ_NVFP4_RECORD_WORDS uint32 words made of
  * MQ_NVFP4_SECTIONS sections of MQ_NVFP4_SECTION_WORDS partial maxima (float bit patterns; jobs that are read
- * once, see the note at mq_run_jobs, keep 16-bit patterns of their tensors' dtype there while they run).  Each tensor that
+ * once, see the note at mq_run_jobs, leave 16-bit patterns of their tensors' dtype there, with bit 15 set).  Each tensor that
  * shares the amax writes ONE whole section (no atomics, nothing to clear beforehand); the amax is the maximum
  * over the first n_sections sections.  A single tensor uses section 0 with n_sections = 1; a gate/up pair
  * uses sections 0 and 1 with n_sections = 2 (nvfp4.py:100-103).  The words after the last section hold the

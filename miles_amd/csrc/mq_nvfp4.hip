@@ -811,11 +811,12 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
 // 64 KiB in registers (16 units per lane, 93 VGPRs, five workgroups per CU: 80 MB on the chip), publishes their maximum,
 // waits for the tensor's other workgroups and quantizes what it holds.  While one tensor waits for its last loads, the
 // workgroups of the next two are already loading.
-//   exchange: a workgroup stores its maximum (with kOneFull, so that it is never zero) into a 16-bit slot of its tensor's
-//     section; the record's first workgroup alone watches the slots and publishes the maximum of all of them in
+//   exchange: a workgroup stores its maximum (with kOneFull, so that it is never zero) into a word of its own of the record's
+//     sections, its slot; the record's first workgroup alone watches the slots and publishes the maximum of all of them in
 //     kOneWords words, each a line of its own, one of which every other workgroup watches with one request at a time.
 //     (With every workgroup watching all slots the polling itself filled the memory channels that hold them: 496 us
-//     instead of 240 on 32 x [2048, 7168].)  No counters, so no atomic read-modify-writes.
+//     instead of 240 on 32 x [2048, 7168].)  No counters, so no atomic read-modify-writes.  What stays in the slots, however
+//     the waits ended, is nothing to a carried run: it has no kCarriedMark and is below every word that has.
 //   every wait ends: after kOnePolls looks the first workgroup of a record publishes that it has given up (kOneGaveUp) in place
 //     of the maximum, and every workgroup that reads it leaves: that happens when workgroups of one record cannot all be on
 //     the chip because something else occupies it; workgroups start in order of their ids, so otherwise the oldest
@@ -844,27 +845,35 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
 // overlap with the loads of the next two tensors, half as well as in the second of two passes.
 constexpr int kOneThreads = 256, kOneUnits = 16, kOneWavesPerSimd = 5;
 constexpr int64_t kOnePerBlock = kOneThreads * kOneUnits;
-constexpr int kOneSlots = 2 * kSectionWords;         // 16-bit slots of a section
+constexpr int kOneSlots = 2 * kSectionWords;         // the most workgroups of a tensor
+constexpr int kOneRecordSlots = kRecordSections * kSectionWords;     // of the tensors of a record
 constexpr uint32_t kOneFull = 0x8000u;               // marks a slot or word that holds a maximum
+static_assert((kOneFull & kCarriedMark) == 0, "no slot passes for what a carried run has collected");
 constexpr uint32_t kOneGaveUp = 0x10000u;            // in a word: the first workgroup has stopped waiting
 constexpr int kOneWords = 7, kOneStride = 32, kRecOne = kRecAmax + 32;     // the published maximum, 128 bytes apart
 static_assert(kRecOne + (kOneWords - 1) * kOneStride < MQ_NVFP4_RECORD_WORDS, "the published words lie inside the record");
-constexpr int kRecReaders = kRecMovedRuns + 1;       // workgroups of the rows behind that have read the slots of a record left to them
 constexpr int kOneLeaderSleep = 1, kOneSleep = 12;   // between two looks, in units of 64 cycles
 constexpr int kOnePolls = 256;                       // looks of a first workgroup, 0.25 ms or more; undisturbed, some 10 are enough
 constexpr int kOnePatience = 1 << 16;                // of those that watch its word, which it writes in any case, 60 ms or more
 
 __device__ __forceinline__ void agent_store(uint32_t* p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-__device__ __forceinline__ void agent_store16(uint16_t* p, uint16_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ uint32_t agent_load(const uint32_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-// one workgroup per tensor: no slot and no word written yet
+// workgroups of the `count` tensors from `row` on
+template <class Table>
+__device__ __forceinline__ uint32_t nv_one_slots(const Table& tab, const uint32_t row, const int count) {
+    uint32_t slots = 0;
+    for (int k = 0; k < count; k++) slots += (uint32_t)((tab.job[row + k].units + kOnePerBlock - 1) / kOnePerBlock);
+    return slots;
+}
+// one workgroup per tensor: no slot and no word written yet, and nothing in the sections of the record that a carried run would
+// take for its own
 template <class Table>
 __global__ __launch_bounds__(256) void nvfp4_one_pass_clear_kernel(const Table tab) {
-    const FlatJob& job = tab.job[blockIdx.x];
+    const FlatJob job = flat_job_at(tab, blockIdx.x);
     uint32_t* rec = (uint32_t*)job.aux;
-    rec[job.section * kSectionWords + threadIdx.x] = 0;
-    if (job.section == 0 && threadIdx.x == 0) rec[kRecReaders] = 0;
+    const uint32_t slots = nv_one_slots(tab, blockIdx.x - job.section, job.pad), sections = (uint32_t)(job.pad * kSectionWords);
+    for (uint32_t word = job.section * kSectionWords + threadIdx.x; word < sections || word < slots; word += sections) rec[word] = 0;
     if (job.section == 0 && threadIdx.x < kOneWords) rec[kRecOne + threadIdx.x * kOneStride] = 0;
 }
 
@@ -917,25 +926,23 @@ __device__ __forceinline__ uint32_t nv_one_max(uint32_t m, const int t) {
     for (int k = 0; k < kOneThreads / kWave; k++) m = umax(m, part[k]);
     return (uint32_t)__builtin_amdgcn_readfirstlane((int)m);
 }
-// What this lane sees of a record's slots, a word (two slots) of each section, as soon as they are all written; `late` if that
-// took more than `polls` looks.  row: of the record's first tensor.
+// What this lane sees of a record's slots, two at a time, as soon as they are all written; `late` if that took more than
+// `polls` looks.  row: of the record's first tensor.
 template <class Table>
 __device__ __forceinline__ uint32_t nv_one_collect(const Table& tab, const uint32_t row, const uint32_t* rec, const int tensors_of_it, const int t,
                                                    const int polls, bool& late) {
+    const uint32_t slots = nv_one_slots(tab, row, tensors_of_it);
     uint32_t m = 0;
-    for (int k = 0; k < tensors_of_it; k++) {
-        const int64_t units = tab.job[row + k].units;
-        const int slots = (int)((units + kOnePerBlock - 1) / kOnePerBlock);
-        for (int word = t; word * 2 < slots; word += kOneThreads) {
-            const uint32_t need = word * 2 + 1 < slots ? 0x80008000u : 0x8000u;
-            uint32_t got = agent_load(rec + k * kSectionWords + word);
-            for (int n = 0; (got & need) != need && n < polls; n++) {
-                __builtin_amdgcn_s_sleep(kOneLeaderSleep);
-                got = agent_load(rec + k * kSectionWords + word);
-            }
-            late |= (got & need) != need;
-            m = umax(m, hmax_u16(abs2(got)));
+    for (uint32_t slot = t; slot < slots; slot += 2 * kOneThreads) {
+        const uint32_t* other = rec + (slot + kOneThreads < slots ? slot + kOneThreads : slot);
+        uint32_t a = agent_load(rec + slot), b = agent_load(other);
+        for (int n = 0; (a & b & kOneFull) == 0 && n < polls; n++) {
+            __builtin_amdgcn_s_sleep(kOneLeaderSleep);
+            a = agent_load(rec + slot);
+            b = agent_load(other);
         }
+        late |= (a & b & kOneFull) == 0;
+        m = umax(m, umax(a & ~kOneFull, b & ~kOneFull));
     }
     return m;
 }
@@ -979,12 +986,10 @@ __device__ __forceinline__ bool nv_one_leaves(const uint32_t m, const NvScales& 
 
 // Rows behind the tensors', `workers` workgroups to a tensor: they quantize the records that were left.  They come to the chip
 // when every workgroup of the tensors has, most of which are done, and of a record that is done there is its word to read.
-// The slots of a record whose first workgroup has given up, which every worker folds, are cleared by the last one to have read
-// them (a carried run would take their marks for kCarriedMark).
+// Of a record whose first workgroup has given up every worker folds the slots.
 template <int FOS, int F16, class Table>
 __device__ __forceinline__ void nv_one_rest(const Table& tab, const uint32_t tensors, const uint32_t workers, const int patience, const int t, float numer,
                                             uint32_t* moved_counter) {
-    __shared__ uint32_t readers;
     const uint32_t id = (blockIdx.y - tensors) * gridDim.x + blockIdx.x, worker = id / tensors, row = id - worker * tensors;
     if (worker >= workers) return;
     const FlatJob job = flat_job_at(tab, row);
@@ -998,26 +1003,18 @@ __device__ __forceinline__ void nv_one_rest(const Table& tab, const uint32_t ten
     const float amax = elem_lo<F16>(m);
     const NvAmaxScales a{amax, nv_scales(amax, numer)};
     if ((got & kOneFull) != 0 && !nv_one_leaves<FOS, F16>(m, a.gs)) return;
-    if (gave_up) {
-        if (t == 0) readers = atomicAdd(rec + kRecReaders, 1u);
-        __syncthreads();
-        if (readers + 1 == workers * (uint32_t)job.pad)
-            for (int k = 0; k < job.pad; k++) rec[k * kSectionWords + t] = 0;
-    }
     if ((got & kOneFull) == 0 && worker == 0 && t == 0) nv_publish_plain(job, a.amax, a.gs, numer, moved_counter);
     constexpr int64_t kPerBlock = nv_units_per_block(FOS);
     for (int64_t base = worker * kPerBlock; base < job.units; base += workers * kPerBlock)
         nvfp4_quant_units<FOS, F16>(job, base, t, numer, true, [&] { return a; });
 }
 // By a record's first workgroup, when it has nothing else to do: the record of a maximum that it has published, for all
-// tensors that share it; the slots, which nobody reads any more, are cleared for a carried run.
+// tensors that share it.
 template <class Table>
 __device__ __forceinline__ void nv_one_settle(const Table& tab, const FlatJob& job, const int t, float amax, const NvScales& gs, float numer,
                                               const bool left, uint32_t* moved_counter) {
-    uint32_t* rec = (uint32_t*)job.aux;
-    for (int k = 0; k < job.pad; k++) rec[k * kSectionWords + t] = 0;
     if (t != 0) return;
-    rec[kRecRedo] = left;
+    ((uint32_t*)job.aux)[kRecRedo] = left;
     for (int k = 0; k < job.pad; k++) nv_publish_plain(flat_job_at(tab, blockIdx.y + k), amax, gs, numer, moved_counter);
 }
 
@@ -1130,7 +1127,7 @@ __global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_
     }
     uint32_t m = nv_one_max<0>(hmax_u16(m2), t);
     uint32_t* rec = (uint32_t*)job.aux;
-    if (t == 0) agent_store16((uint16_t*)(rec + job.section * kSectionWords) + block, (uint16_t)(kOneFull | m));
+    if (t == 0) agent_store(rec + nv_one_slots(tab, blockIdx.y - job.section, job.section) + block, kOneFull | m);
     const bool first = block == 0 && job.section == 0;
     if (first) {
         // the record's first workgroup waits for every other one
@@ -1610,7 +1607,7 @@ bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes, int f
         (void)hipGetLastError();
         return false;
     }
-    return slots * 2 <= (int64_t)cus * kOneWavesPerSimd;       // a workgroup is one wavefront per SIMD
+    return slots <= kOneRecordSlots && slots * 2 <= (int64_t)cus * kOneWavesPerSimd;       // a workgroup is one wavefront per SIMD
 }
 int64_t mq_nvfp4_one_pass_slots(int64_t units) { return (units + kOnePerBlock - 1) / kOnePerBlock; }
 

@@ -78,3 +78,33 @@ def test_workgroups_that_wait_for_nobody(n, rows, cols, first_polls):
     _probes.check(_probes.load().mqp_nvfp4_one_pass(ctypes.byref(batch.freeze()), n, first_polls, 0, stream))
     for i in range(n):
         _same(got[i], nvfp4_quantize_1d(x[i]), f"tensor {i}")
+
+
+@pytest.mark.parametrize("first_polls, patience", [(0, 0), (0, 256), (256, 0)])
+@pytest.mark.parametrize("n, rows, cols", [(1, 2048, 8192), (5, 512, 7216), (64, 3, 16384)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_records_serve_a_carried_run_however_the_waits_ended(dtype, n, rows, cols, first_polls, patience):
+    """Nothing that waits in vain may leave in a record what a carried run takes for its own."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = (torch.randn(n, rows, cols, generator=g, device="cuda") * 4.0).to(dtype)       # patterns with the exponent's top bit set
+    with launch.recording() as batch:
+        got = [nvfp4_quantize_1d(t) for t in x]
+    records = batch.amax_records()
+    for record in records:
+        record.fill_(-1)
+    stream = torch.cuda.current_stream().cuda_stream
+    _probes.check(_probes.load().mqp_nvfp4_one_pass(ctypes.byref(batch.freeze()), n, first_polls, patience, stream))
+    words = max(256, -(-rows * cols // (256 * 16 * 8)))
+    assert all(bool((r[:words] >= 0).all()) for r in records), "marked as words of a carried run are"
+    for r, t in zip(records, x):
+        assert r[_lib.RECORD_AMAX_WORD].view(torch.float32).item() == t.abs().max().float().item()
+    batch.carry_amax(adaptive=False)
+    for run in range(2):
+        for one in got:
+            for t in one:
+                t.view(torch.uint8).fill_(0xA5) if t.dim() else t.fill_(-1.0)
+        batch.run()
+        for i in {0, 1, n // 2, n - 1} & set(range(n)):
+            _same(got[i], nvfp4_quantize_1d(x[i]), f"run {run}, tensor {i}")
+            assert records[i][_lib.RECORD_REDO_WORD].item() == 0 or run > 0, "the amax has not moved"
+        x.mul_(0.125)
