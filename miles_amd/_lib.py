@@ -60,6 +60,7 @@ TABLE_ENTRY_BYTES, TABLE_GROUP = 56, 8192                 # MQ_JOB_TABLE_ENTRY_B
 NVFP4_4OVER6, NVFP4_ERR_MSE, NVFP4_ERR_FP16 = 1, 2, 4     # flags of mq_nvfp4_quant / mq_nvfp4_qdq
 NVFP4_CARRY_AMAX = 8                                      # MQ_NVFP4_CARRY_AMAX: NVFP4 jobs of a re-submitted list only
 NVFP4_NO_WAIT = 16                                        # MQ_NVFP4_NO_WAIT: NVFP4 jobs leave everything to the workgroups behind
+RECORD_WORDS = 1280                                       # MQ_NVFP4_RECORD_WORDS: of an amax record
 # words of an amax record behind its four sections of 256 partial maxima (MQ_NVFP4_RECORD_*_WORD)
 RECORD_AMAX_WORD, RECORD_REDO_WORD, RECORD_VOLATILE_WORD = 1024, 1028, 1029
 

@@ -179,12 +179,25 @@ class JobBatch:
         """The amax records of the NVFP4 and per-tensor FP8 jobs, one per tensor or gate/up pair, in job order (int32
         tensors; words `_lib.RECORD_AMAX_WORD`, `RECORD_REDO_WORD`, `RECORD_VOLATILE_WORD` hold the folded amax and
         the state of the carried-over amax after a run)."""
-        by_address = {t.data_ptr(): t for t in self._keep}
+        jobs = self._records        # (takes over what native code has recorded: before the tensors are looked at)
+        by_address, stacks = {}, []
+        for t in self._keep:
+            if t.dtype == torch.int32 and t.dim() == 2 and t.shape[1] == _lib.RECORD_WORDS:
+                stacks.append(t)        # (the records of a stack of matrices are held as one tensor)
+            else:
+                by_address[t.data_ptr()] = t
         seen, out = set(), []
-        for r in self._records:
-            if r[self.KIND] in (_lib.JOB_NVFP4, _lib.JOB_FP8_TENSOR) and r[self.AUX] not in seen:
-                seen.add(r[self.AUX])
-                out.append(by_address[r[self.AUX]])
+        for r in jobs:
+            address = r[self.AUX]
+            if r[self.KIND] in (_lib.JOB_NVFP4, _lib.JOB_FP8_TENSOR) and address not in seen:
+                seen.add(address)
+                record = by_address.get(address)
+                if record is None:
+                    stack = next((t for t in stacks if 0 <= address - t.data_ptr() < t.nbytes), None)
+                    if stack is None:
+                        raise KeyError(address)
+                    record = stack[(address - stack.data_ptr()) // (stack.element_size() * _lib.RECORD_WORDS)]
+                out.append(record)
         return out
 
     def hold(self, tensor: torch.Tensor) -> None:

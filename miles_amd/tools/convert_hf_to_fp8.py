@@ -51,7 +51,7 @@ def block_fp8(weight: torch.Tensor, block_size):
 _FLOORS = {dtype: int(torch.tensor(1e-12, dtype=dtype).float().view(torch.int32))
            for dtype in (torch.bfloat16, torch.float16, torch.float32)}
 _FLOOR_BITS = tuple(_FLOORS.values())
-_AMAX_RECORD_WORDS = 1280   # MQ_NVFP4_RECORD_WORDS: partial maxima of a tensor on the device, then its folded amax
+_AMAX_RECORD_WORDS = _lib.RECORD_WORDS   # partial maxima of a tensor on the device, then its folded amax
 
 
 def _scaled_fp8(weight: torch.Tensor, per_channel: bool):

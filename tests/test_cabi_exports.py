@@ -87,7 +87,7 @@ def test_python_constants_match_the_header():
     assert _lib.MAX_GROUP == int(defines["MQ_MAX_GROUP"])
     assert (_lib.TABLE_ENTRY_BYTES, _lib.TABLE_GROUP) == (int(defines["MQ_JOB_TABLE_ENTRY_BYTES"]), int(defines["MQ_TABLE_GROUP"]))
     words = int(defines["MQ_NVFP4_SECTION_WORDS"]) * (int(defines["MQ_NVFP4_SECTIONS"]) + 1)
-    assert AMAX_RECORD_WORDS == _AMAX_RECORD_WORDS == words
+    assert AMAX_RECORD_WORDS == _AMAX_RECORD_WORDS == _lib.RECORD_WORDS == words
     amax_word = int(defines["MQ_NVFP4_SECTION_WORDS"]) * int(defines["MQ_NVFP4_SECTIONS"])
     assert defines["MQ_NVFP4_RECORD_REDO_WORD"] == "(MQ_NVFP4_RECORD_AMAX_WORD + 4)"
     assert defines["MQ_NVFP4_RECORD_VOLATILE_WORD"] == "(MQ_NVFP4_RECORD_AMAX_WORD + 5)"

@@ -4,7 +4,7 @@ the native one hands a call back."""
 import pytest
 import torch
 
-from miles_amd import launch
+from miles_amd import _lib, launch
 from miles_amd.kernels.quant import int4_fake
 from miles_amd.megatron_to_hf.processors import quantizer_nvfp4
 from miles_amd.tools import convert_hf_to_fp8, convert_kimi_int4_to_bf16, convert_mxfp4_to_fp8, fp8_cast_bf16
@@ -148,3 +148,16 @@ def test_a_recording_keeps_the_python_jobs():
     batch.run()
     want = quantizer_nvfp4.quantize_nvfp4(stack)
     assert torch.equal(codes, want[0]) and torch.equal(published, want[2])
+
+
+@pytest.mark.parametrize("n", [1, 3])
+def test_records_of_a_deferred_stack(n):
+    """A block that is submitted at its end: the records of a stack, which are one tensor, and of what was recorded beside it."""
+    stack, single = _w(n * 16, 64).view(n, 16, 64), _w(8, 32)
+    with launch.deferred() as batch:
+        quantizer_nvfp4.quantize_nvfp4(stack)
+        quantizer_nvfp4.quantize_nvfp4(single)
+    records = batch.amax_records()
+    assert [tuple(r.shape) for r in records] == [(_lib.RECORD_WORDS,)] * (n + 1)
+    assert [r.data_ptr() for r in records] == [job[batch.AUX] for job in batch.records]
+    assert [r[_lib.RECORD_AMAX_WORD].view(torch.float32).item() for r in records] == [w.abs().max().float().item() for w in (*stack, single)]
