@@ -931,19 +931,27 @@ int mq_fp8_tile_launch_table(int mode, int dtype, const TileJob* device_jobs, in
 
 bool mq_fp8_tile_rows_share_lines(const void* w, int64_t ldw) { return (uintptr_t)w % 128 != 0 || ldw % 64 != 0; }
 // The most tiles of a launch for which the any-alignment kernel, with its temporal loads and stores, ends sooner whatever the
-// rows (us, fast kernel / that one): 64 tiles of [1024, 1024] 5.2 / 4.7, 128 of [1024, 2048] 5.4 / 5.0, 256 of [2048, 2048] 5.9 / 5.8,
-// 512 of [2048, 4096] 7.9 / 8.3.
-constexpr int64_t kAnyTiles = 256;
+// rows.  Inputs from HBM, us of a launch among others, fast kernel / that one (runs of one side differ by 0.05): block_fp8 32 tiles
+// 5.02 / 4.59, 64 5.13 / 4.67, 80 5.16 / 4.73, 96 5.22 / 5.10, 112 5.28 / 5.28, 128 5.31 / 5.67, 256 5.84 / 6.88; blockwise cast 64
+// 4.66 / 4.44, 80 4.71 / 4.49, 96 4.71 / 4.89, 128 4.83 / 5.50, 256 5.36 / 6.79.  (In a captured graph, where launches follow one another
+// sooner, the fast one is ahead by 0.3 throughout: 64 tiles 4.47 / 4.74; alone 7.5 / 7.4.)
+constexpr int64_t kAnyTiles = 80;
+// Where most tiles are of tensors whose rows begin inside a 128-byte line, two tiles share the line at their border: the fast
+// kernel's non-temporal loads fetch it, and its partial stores write it, once for each.  The temporal accesses of the other kernel
+// pay as soon as every compute unit has several tiles.  Inputs from HBM, us, fast / any (runs of one side differ by 0.1): rows of
+// 1032 elements 288 tiles 6.54 / 8.22, 576 9.95 / 10.8, 864 13.3 / 13.3, 1152 16.0 / 15.3, 1728 23.0 / 19.7, 6528 of 2056 97 / 60; of 8200 520
+// 9.4 / 9.9, 1040 15.0 / 15.0, 1560 20.9 / 19.6, 4160 54 / 45, 16640 244 / 159.  Rows of whole half lines have one border in two
+// on a line, and gain later: of 2592 1008 13.0 / 14.0, 1344 17.1 / 17.6 (blockwise cast 16.5 / 17.3), 1491 18.1 / 18.2, 2016 23.2 / 22.5,
+// 4032 44.4 / 39.1; of 2080 1207 15.2 / 15.8, 1496 18.0 / 18.1, 1802 20.9 / 20.7.  (Inputs that are still in the memory-side cache gain at
+// any number of tiles: 288 of 1032 5.9 / 5.2, 1152 13.9 / 11.4.)
+constexpr int64_t kSharedTiles = 1152, kHalfLineTiles = 1536;
 
 // tab.job[i] filled by the caller (w, q, scale, ldw, M, K, row blocks), all of one dtype; fills the division constants
 // and `end`, launches.  `aligned`: every tensor passed mq_fp8_tile_fast_ok, otherwise mq_fp8_tile_any_ok.
-// Aligned tensors take the any-alignment kernel as well where most of their tiles have rows that begin inside a 128-byte line: two
-// tiles share the line at their border, and the fast kernel's non-temporal loads fetch it, and its partial stores write it,
-// once for each (us, fast / any): 64 x [768, 2056] 98.7 / 55.0, 64 x [768, 2080] 76.6 / 54.4, 12 x [1545, 2568] 40.6 / 28.1, 4 x [3000, 7184]
-// 67 / 45.8, 2 x [8192, 8200] 111.5 / 80.2, 4 x [1545, 2592] 14.7 / 13.8, 1 x [1545, 2592] 6.4 / 6.5; with rows of whole lines
-// 2 x [8192, 8192] 64.9 / 74.4, 12 x [1545, 2624] the fast one 28.2.
+// Aligned tensors take the any-alignment kernel as well in short launches and where tiles share lines (kAnyTiles, kSharedTiles); with rows
+// of whole lines 2 x [8192, 8192] 64.9 / 74.4, 12 x [1545, 2624] the fast one 28.2.
 int mq_fp8_tile_launch_group(int mode, int dtype, bool aligned, TileTable& tab, hipStream_t st) {
-    int64_t tiles = 0, shared = 0;     // tiles, and those of tensors whose rows share lines
+    int64_t tiles = 0, shared = 0, halves = 0;     // tiles, those of tensors whose rows share lines, and share them at half a line
     bool blocked = false;
     for (int i = 0; i < tab.n; i++) {
         TileJob& j = tab.job[i];
@@ -952,11 +960,14 @@ int mq_fp8_tile_launch_group(int mode, int dtype, bool aligned, TileTable& tab, 
         if (tiles >= 0x7FFFFFF0) return mq_fail(MQ_ERR_ARG, "too many tiles");
         tab.end[i] = (int32_t)tiles;
         blocked |= j.tiles_per_block != 0;
-        if (mq_fp8_tile_rows_share_lines(j.w, j.ldw)) shared += own;
+        if (!mq_fp8_tile_rows_share_lines(j.w, j.ldw)) continue;
+        shared += own;
+        if ((uintptr_t)j.w % 64 == 0 && j.ldw % 32 == 0) halves += own;
     }
     if (tiles == 0) return MQ_OK;
     seal_table(tab);
-    if (aligned && (blocked || (shared * 2 <= tiles && tiles > kAnyTiles))) {      // (row blocks are the fast kernel's)
+    const bool sharing = shared * 2 > tiles && tiles >= (halves * 2 > shared ? kHalfLineTiles : kSharedTiles);
+    if (aligned && (blocked || (!sharing && tiles > kAnyTiles))) {      // (row blocks are the fast kernel's)
         tile_launch(mode, dtype == MQ_F16, dim3((unsigned)xcd_grid(tiles)), st, tab);
         return mq_check_launch("fp8 block quant");
     }

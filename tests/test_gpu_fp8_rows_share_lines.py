@@ -21,11 +21,19 @@ def _bytes_equal(got, want, what):
 @pytest.mark.parametrize("specials", [False, True])
 @pytest.mark.parametrize("shapes", [
     [(1, 8), (127, 72), (129, 136), (128, 128), (300, 264)],
-    [(2048, 2048)],                                  # 256 tiles: the last short list
+    [(1024, 1280)],                                  # 80 tiles: the last short list
+    [(1152, 1152)],
+    [(2048, 2048)],
     [(2049, 2048), (1, 8)],
     [(2049, 2056)],                                  # 289 tiles, rows that share lines
-    [(1025, 1032)] * 4 + [(1024, 2048)] * 2,         # mostly those, and mostly the others
-    [(1025, 1032)] * 2 + [(1024, 2048)] * 3,
+    [(16255, 1032)],                                 # 1143 of them
+    [(16255, 1032), (127, 1032)],                    # 1152
+    [(21759, 1056)],                                 # 1530, at half a line
+    [(21760, 1056), (5, 1056)],                      # 1539
+    [(1025, 1032)] * 4 + [(1024, 2048)] * 2,
+    [(4000, 1032)] * 4 + [(1024, 2048)] * 8,         # mostly those, and mostly the others
+    [(4000, 1032)] * 2 + [(1024, 2048)] * 8,
+    [(4000, 1032)] * 2 + [(4000, 1056)] * 3,
 ])
 def test_lists_against_oracle(oracle, shapes, dtype, specials):  # noqa: F811
     hosts = [_matrix(s, dtype, 700 + i, specials) for i, s in enumerate(shapes)]
