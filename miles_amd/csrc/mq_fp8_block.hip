@@ -1082,15 +1082,20 @@ static void channel_launch(int form, const ChannelTable& tab, hipStream_t st) {
         default: hipLaunchKernelGGL((fp8_channel_kernel<256, DT, 16, LINES>), grid, blk, 0, st, tab); break;
     }
 }
-// The form of a whole list (neither with kChannelLines), rows of at most `units`.  Of 257 to 384 units half of the lanes of a 256-lane row
-// and more have nothing in their second unit: a wavefront per row from 8192 rows on (us, 256 lanes / 64; 18540 rows of 2056 bf16
-// 26.5 / 23.5, of 2560 28.2 / 25.4, of 2563 30.7 / 26.1, of 2880 30.2 / 28.7, of 3200 31.6 / 31.3, of 3584 33.4 / 34.9, of 1032 fp32
-// 23.4 / 20.1; 7470 rows of 2880 14.3 / 14.2, 1545 of 2560 4.8 / 5.3).  Few rows leave a wavefront alone with its row: 256 lanes
-// from 129 units on up to 2048 rows (64 lanes / 256; 64 rows of 2048 3.3 / 2.5, 512 4.3 / 3.2, 2048 5.0 / 4.6, 4096 6.4 / 7.2; of
-// 1024 64 rows 2.9 / 2.8, 1024 3.4 / 3.4).
-static int channel_list_form(int form, int64_t units, int64_t rows) {
+// The form of a whole list (neither with kChannelLines), rows of at most `units`; inputs from HBM, us, runs of one side differ by
+// 0.05 to 0.2.  Of 257 to 384 units half of the lanes of a 256-lane row and more have nothing in their second unit: a wavefront per
+// row from 8192 rows on, which are one round of its workgroups (256 lanes / 64; 8192 rows of 2056 bf16 12.6 / 12.0, of 3072 15.4 / 14.9;
+// 18540 of 2056 25.6 / 24.2, of 2560 27.6 / 25.1, of 2563 31.2 / 29.8, of 2880 29.6 / 28.8, of 3072 30.4 / 30.1, of 3200 31.6 / 31.3, but of 3584 33.4 /
+// 34.9; of 1028 fp32 22.7 / 20.1; 6180 of 2880 12.0 / 12.6, 1545 of 2560 4.7 / 5.2).  A second round with hardly anything in it costs the wider rows
+// of 16-bit elements what that gives: 8300 rows of 2880 14.9 / 15.3, of 3072 15.5 / 15.6, 8600 15.8 / 15.7 (of 2560 14.1 / 13.4; of 1440 fp32
+// 12.8 / 12.5).
+// Few rows leave a wavefront alone with its row: 256 lanes from 129 units on up to 2048 rows (device time, 64 lanes / 256; 64 rows
+// of 1040 2.9 / 2.3, of 2048 3.6 / 2.6; 512 3.4 / 2.8 and 4.1 / 2.9, 1024 3.6 / 3.3 and 4.4 / 3.5, 2048 4.1 / 4.1 and 4.9 / 4.3, 2052 4.2 / 4.4 and 4.9 / 5.0).
+static int channel_list_form(int form, int dtype, int64_t units, int64_t rows) {
+    constexpr int64_t kRound = 8192, kThin = kRound + kRound / 32;
+    const int64_t widest = dtype != MQ_F32 && rows > kRound && rows <= kThin ? 320 : 384;
     if (form == kChannel64x4 && units > 128 && rows <= 2048) return kChannel256x4;
-    if (form == kChannel256x4 && units <= 384 && rows >= 8192) return kChannel64x8;
+    if (form == kChannel256x4 && units <= widest && rows >= kRound) return kChannel64x8;
     return form;
 }
 // n <= kMaxGroup tensors of one dtype and one form
@@ -1104,7 +1109,7 @@ int mq_fp8_channel_launch_group(int dtype, int form, const MqScaledArgs* a, int 
         cols = a[i].K > cols ? a[i].K : cols;
     }
     const int64_t E = dtype == MQ_F32 ? 4 : 8;
-    form = channel_list_form(form & ~kChannelLines, (cols + E - 1) / E, rows);
+    form = channel_list_form(form & ~kChannelLines, dtype, (cols + E - 1) / E, rows);
     for (int i = 0; i < n; i++) {
         tab.job[i] = ChannelJob{a[i].w, (uint8_t*)a[i].q, a[i].scale, a[i].ldw, (int32_t)a[i].K, (int32_t)a[i].M, a[i].floor_v, 0};
         const int64_t blocks = mq_fp8_channel_blocks(form, a[i].M);

@@ -14,12 +14,21 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("offset", [0, 1])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("rows, units", [
-    ((700, 3, 1345), (128, 129, 200)),          # 2048 rows, the widest of 200 units
-    ((700, 3, 1346), (128, 129, 256)),          # 2049
-    ((5, 1), (1, 128)),
-    ((5, 1), (129, 256)),
+    ((680, 684, 684), (128, 129, 200)),         # 2048 rows in one launch, the widest of 200 units
+    ((680, 684, 685), (128, 129, 256)),         # 2049
+    ((2048,), (129,)),
+    ((2048,), (256,)),
+    ((2049,), (129,)),
+    ((2049,), (256,)),
+    ((680, 684, 684), (1, 127, 128)),
+    ((8, 7), (1, 128)),
+    ((8, 7), (129, 256)),
     ((4001, 4190), (257, 384)),                 # 8191 rows of 257 to 384 units
     ((4001, 4191), (257, 384)),                 # 8192
+    ((4001, 4192), (257, 320)),                 # 8193: a second round, of 16-bit rows up to 320 units
+    ((4001, 4192), (257, 321)),
+    ((4001, 4447), (257, 384)),                 # 8448
+    ((4001, 4448), (257, 384)),
     ((4097, 4097), (257, 385)),
 ])
 def test_lists_against_oracle(oracle, rows, units, dtype, offset):  # noqa: F811
