@@ -1,6 +1,8 @@
 """Copies behind INT4 jobs in one list: those that depend on nothing share a launch with them, and whatever the order and the
 overlaps, memory ends as if the jobs had run one after the other."""
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -81,3 +83,54 @@ def test_as_if_one_after_the_other(dtype, symmetric, n, table, order):
         for mine in place:
             got[mine["aux"]:mine["aux"] + nbytes["aux"]] = want[mine["aux"]:mine["aux"] + nbytes["aux"]]
     assert np.array_equal(got, want)
+
+
+def _launches(batch):
+    """Kernels of one run, counted in a capture of it."""
+    nodes = _lib.load().hipGraphGetNodes        # (resolved in the HIP runtime that the library is linked against)
+    nodes.restype, nodes.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        batch.run()
+    count = ctypes.c_size_t()
+    assert nodes(graph.raw_cuda_graph(), None, ctypes.byref(count)) == 0
+    return count.value
+
+
+# 32768 workgroups of tensors and more have the copies behind them; grid rows far wider than the copies need
+@pytest.mark.parametrize("n, rows, table", [(15, 2048, False), (16, 2048, False), (17, 2048, False), (64, 1008, False), (70, 1008, True)])
+def test_copies_behind_a_long_launch(n, rows, table):
+    cols = 4096
+    g = torch.Generator(device=DEV).manual_seed(n)
+    w = torch.randn(n, rows, cols, device=DEV, generator=g).bfloat16()
+    lengths = [SIZES[i % len(SIZES)] for i in range(n)]
+    at, place = 0, []
+    for length in lengths:                              # codes, scales and a record of every tensor, as in a packed payload
+        mine = {}
+        for name, size in (("out", rows * cols // 2), ("scale", rows * cols // GROUP * 2), ("copy", length)):
+            mine[name], at = at, at + size + -size % 16
+        place.append(mine)
+    payload = torch.full((at,), 0xA5, dtype=torch.uint8, device=DEV)
+    sources = torch.randint(0, 256, (n, max(SIZES) + 1), dtype=torch.uint8, device=DEV, generator=g)
+    want = payload.clone()
+    for mine, length, one, source in zip(place, lengths, w, sources):
+        packed, scale, _ = pack_layer(one, GROUP)
+        for name, t in (("out", packed), ("scale", scale), ("copy", source[:length])):
+            t = t.reshape(-1).view(torch.uint8)
+            want[mine[name]:mine[name] + t.numel()] = t
+    with launch.recording() as batch:
+        pass
+    batch.device = payload.device
+    base = payload.data_ptr()
+    for mine, one in zip(place, w):
+        batch.add(_lib.JOB_INT4_PACK, _lib.DTYPE_CODE[torch.bfloat16], one.data_ptr(), base + mine["out"], base + mine["scale"], None, None,
+                  rows, cols, cols, GROUP, 0)
+    for mine, length, source in zip(place, lengths, sources):
+        batch.add(_lib.JOB_COPY, 0, source.data_ptr(), base + mine["copy"], None, None, None, 1, length, length, 0, 0)
+    batch.freeze()
+    assert (batch._table is not None) == table
+    torch.cuda.synchronize()
+    assert _launches(batch) == 1
+    payload.fill_(0xA5)
+    batch.run()
+    assert torch.equal(payload, want)

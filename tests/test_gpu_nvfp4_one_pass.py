@@ -46,14 +46,12 @@ def test_one_pass_equals_single_calls(n, rows, cols, dtype):
 
 @pytest.mark.parametrize("no_wait", [False, True])
 @pytest.mark.parametrize("pairs, rows, cols", [(12, 768, 2048), (40, 768, 2048), (3, 1300, 7168)])
-def test_pairs_second_pass_and_carried_run(pairs, rows, cols, no_wait):
-    """A pair waits for both of its tensors; with no waiting at all the second pass does what is left; either way the
+def test_pairs_what_is_left_and_a_carried_run(pairs, rows, cols, no_wait):
+    """A pair waits for both of its tensors; with no waiting at all the workgroups behind do what is left; either way the
     records serve a carried run.  (Pairs of [1300, 7168] are 570 workgroups, close to the most that share a record;
     40 pairs are submitted over a device table.)"""
     x = _stack(2 * pairs, rows, cols, torch.bfloat16)
-    if pairs * rows * cols * 4 < 64 << 20:
-        x = torch.cat([x, x * 3])
-        pairs *= 2
+    assert x.nbytes >= 24 << 20         # (shorter lists take two passes)
     with launch.recording() as batch:
         got = [t for i in range(pairs) for t in nvfp4_quantize_1d_pair(x[2 * i], x[2 * i + 1])]
     if no_wait:

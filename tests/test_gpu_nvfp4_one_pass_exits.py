@@ -12,7 +12,7 @@ PUBLISHED, GAVE_UP = 0x8000, 0x10000
 
 
 def _run(tensors, pairs, flag=0):
-    """Outputs, and of every record the words watched and the one that asks for the second pass."""
+    """Outputs, and of every record the words watched and the one that says it was left to the workgroups behind."""
     with launch.recording() as batch:
         if pairs:
             got = [t for i in range(0, len(tensors), 2) for t in nvfp4_quantize_1d_pair(tensors[i], tensors[i + 1])]
@@ -35,7 +35,7 @@ def _tensors(n, rows, cols):
 
 @pytest.mark.parametrize("n, rows, cols, pairs", [(5, 1024, 7168, False), (70, 1031, 1040, False), (24, 768, 2048, True), (6, 1300, 7168, True)])
 def test_a_first_workgroup_that_gives_up_says_so(n, rows, cols, pairs):
-    """Every word that the other workgroups watch names the end of the wait, and the second pass quantizes the record."""
+    """Every word that the other workgroups watch names the end of the wait, and the workgroups behind quantize the record."""
     x = _tensors(n, rows, cols)
     got, words, redo = _run(x, pairs, _lib.NVFP4_NO_WAIT)
     assert (words == words[:, :1]).all()
@@ -61,7 +61,7 @@ def test_lists_that_are_read_once(n, rows, cols, pairs, one_pass):
 
 
 def test_two_streams_at_once():
-    """Two lists whose workgroups compete for the chip: whoever waits in vain leaves its record to the second pass, and every
+    """Two lists whose workgroups compete for the chip: whoever waits in vain leaves its record to the workgroups behind, and every
     byte is that of a single call."""
     lists = [_tensors(12, 2048, 7168), [t * 3 for t in _tensors(9, 2048, 8192)]]
     streams = [torch.cuda.Stream() for _ in lists]

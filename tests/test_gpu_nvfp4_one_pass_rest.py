@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from miles_amd import _lib, _probes, launch
+from miles_amd.megatron_to_hf.processors.quantizer_nvfp4 import quantize_nvfp4
 from miles_amd.utils.nvfp4 import nvfp4_quantize_1d, nvfp4_quantize_1d_pair
 
 pytestmark = pytest.mark.gpu
@@ -22,7 +23,7 @@ def _same(got, want, what):
 @pytest.mark.parametrize("n, rows, cols, pairs", [
     (3, 1024, 11184, False),            # few tensors: as many workers as a section has words
     (9, 512, 7216, False),              # ragged last workgroup
-    (128, 16, 16384, False),            # more tensors than one launch of 64, workers bounded by a tensor's blocks
+    (128, 16, 16384, False),            # over a device table, workers bounded by a tensor's blocks
     (140, 257, 1040, False),            # over a device table
     (24, 768, 2048, True),
 ])
@@ -40,8 +41,6 @@ def test_what_is_left_and_the_records_behind_it(n, rows, cols, pairs, dtype, fla
         else:
             got = [nvfp4_quantize_1d(t) for t in x]
     batch.replace_records([r[:batch.P1] + (r[batch.P1] | flag,) + r[batch.P1 + 1:] for r in batch.records])
-    if n == 140:
-        batch.freeze()
     for record in batch.amax_records():
         record.fill_(-1)                                # whatever was in this memory
     for run in range(3):
@@ -108,3 +107,15 @@ def test_records_serve_a_carried_run_however_the_waits_ended(dtype, n, rows, col
             _same(got[i], nvfp4_quantize_1d(x[i]), f"run {run}, tensor {i}")
             assert records[i][_lib.RECORD_REDO_WORD].item() == 0 or run > 0, "the amax has not moved"
         x.mul_(0.125)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_a_stack_cut_into_launches(dtype):
+    """Without a device table a list is cut after 64 tensors, and each launch has the workers for its own number of them."""
+    g = torch.Generator(device="cuda").manual_seed(70)
+    x = (torch.randn(70, 1024, 2064, generator=g, device="cuda") * 0.02).to(dtype)      # 4 MiB and more: both launches read once
+    x[5, 1, 3] = float("inf")
+    x[69, 1023, 2063] = float("nan")
+    codes, scales, published = quantize_nvfp4(x)
+    for i in (0, 4, 5, 6, 63, 64, 65, 68, 69):
+        _same((codes[i], scales[i], published[i]), nvfp4_quantize_1d(x[i]), f"tensor {i}")

@@ -70,7 +70,7 @@ def test_read_once_then_smaller_weights(no_wait):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_read_once_with_extreme_tensors(dtype):
-    """What the kernel that reads a tensor once leaves to the launch behind it: scales at the ends of the fp32 range,
+    """What the kernel that reads a tensor once leaves to the workgroups behind: scales at the ends of the fp32 range,
     infinities, NaN.  Its neighbours in the list stay where they are."""
     g = torch.Generator(device="cuda").manual_seed(4)
     x = torch.randn(8, 1024, 7168, generator=g, device="cuda").to(dtype)
