@@ -821,15 +821,17 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
 //     of the maximum, and every workgroup that reads it leaves: that happens when workgroups of one record cannot all be on
 //     the chip because something else occupies it; workgroups start in order of their ids, so otherwise the oldest
 //     unfinished tensor always gets there.  A record that does not fit next to a busy neighbour so costs
-//     one wait, not one for each batch of its workgroups that comes to the chip.  32 x [2048, 7168] beside a stream of
-//     [8192, 8192] matrix products: 1.0 ms, of copies 0.37 (1.8 and 0.37 with what is left in a launch behind, which
-//     starts when the neighbour makes room).
+//     one wait, not one for each batch of its workgroups that comes to the chip.  Medians beside a stream that is never idle, two
+//     passes / this way: 32 x [2048, 7168] beside [8192, 8192] matrix products 1.8 / 1.0 ms (with what is left in a launch behind, which
+//     starts when the neighbour makes room, 1.8), beside copies 0.38 / 0.38; lists of 24 to 56 MiB beside [8192, 8192] products 1.6 / 0.8 ms,
+//     beside [4096, 4096] ones 0.20 / 0.10 to 0.17, beside copies 34 to 53 us / 35 to 45.
 //   what is left: rows of workgroups behind those of the tensors (nv_one_rest), which start when all of these have, read every
 //     record's word and quantize what its own workgroups did not.  (As a launch behind this one they cost 4.5 us.)
-// 32 x [2048, 7168] (940 MB of bf16, all launches together): 311 us in two passes, 214 us this way (5.6 TB/s; 217 with what
-// is left in a launch behind, where 28 x [528, 3088] took 32.5 us and now 29, 48 x [1536, 2048] 73 and now 68; 226 with a
+// 32 x [2048, 7168] (940 MB of bf16, all launches together): 313 us in two passes, 211 us this way (5.7 TB/s; 211.1 with slots that had
+// to be cleared again, where [2048, 7168] took 13.0 us and now 12.3, 28 x [528, 3088] 28.3 and now 27.8; 214 with what
+// is left in a launch behind, where 28 x [528, 3088] took 31.6 us, 48 x [1536, 2048] 73 and now 68).  Before, at 217: 226 with a
 // block's scale computed in both lanes that hold it and its byte stored under a mask, 234 with the block maxima taken after the
-// wait and a range test and a branch to the software forms in each unit).  24 units per lane at
+// wait and a range test and a branch to the software forms in each unit.  24 units per lane at
 // four workgroups per CU were 5 % slower, 8 units in 512 lanes 6 %, six workgroups per CU (20 registers spilled) 38 %; two
 // units stored together, eight bytes a lane, 2 % slower here and 2 % faster on 18 x [1420, 1520].
 // What bounds it: so many long-lived workgroups stream at 5.8 TB/s even if nobody waits for anybody (206 of the kernel's
@@ -853,18 +855,28 @@ constexpr uint32_t kOneGaveUp = 0x10000u;            // in a word: the first wor
 constexpr int kOneWords = 7, kOneStride = 32, kRecOne = kRecAmax + 32;     // the published maximum, 128 bytes apart
 static_assert(kRecOne + (kOneWords - 1) * kOneStride < MQ_NVFP4_RECORD_WORDS, "the published words lie inside the record");
 constexpr int kOneLeaderSleep = 1, kOneSleep = 12;   // between two looks, in units of 64 cycles
-constexpr int kOnePolls = 256;                       // looks of a first workgroup, 0.25 ms or more; undisturbed, some 10 are enough
-constexpr int kOnePatience = 1 << 16;                // of those that watch its word, which it writes in any case, 60 ms or more
+// Looks of a first workgroup at each pair of slots: 0.04 ms where nothing else uses the memory (0.15 us a look), 0.16 ms beside a stream
+// of copies (0.6); undisturbed, some 10 are enough.
+constexpr int kOnePolls = 256;
+// Looks of those that watch its word: 28 ms or 57 ms (0.43 or 0.87 us).  It has come to the chip before them and writes its word when its own
+// looks are spent, so this ends a wait only where that workgroup itself is held up.
+constexpr int kOnePatience = 1 << 16;
 
 __device__ __forceinline__ void agent_store(uint32_t* p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ uint32_t agent_load(const uint32_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-// workgroups of the `count` tensors from `row` on
+// slots of a record: the first one of the tensor in row `row`, and how many there are
+struct NvOneSlots {
+    uint32_t first, all;
+};
+__device__ __forceinline__ uint32_t nv_one_slots_of(const int64_t units) { return (uint32_t)((units + kOnePerBlock - 1) / kOnePerBlock); }
 template <class Table>
-__device__ __forceinline__ uint32_t nv_one_slots(const Table& tab, const uint32_t row, const int count) {
-    uint32_t slots = 0;
-    for (int k = 0; k < count; k++) slots += (uint32_t)((tab.job[row + k].units + kOnePerBlock - 1) / kOnePerBlock);
-    return slots;
+__device__ __forceinline__ NvOneSlots nv_one_slots(const Table& tab, const FlatJob& job, const uint32_t row) {
+    uint32_t first = 0;
+    for (int k = job.section; k > 0; k--) first += nv_one_slots_of(tab.job[row - k].units);
+    uint32_t all = first + nv_one_slots_of(job.units);
+    for (int k = job.section + 1; k < job.pad; k++) all += nv_one_slots_of(tab.job[row + (k - job.section)].units);
+    return NvOneSlots{first, all};
 }
 // one workgroup per tensor: no slot and no word written yet, and nothing in the sections of the record that a carried run would
 // take for its own
@@ -872,7 +884,7 @@ template <class Table>
 __global__ __launch_bounds__(256) void nvfp4_one_pass_clear_kernel(const Table tab) {
     const FlatJob job = flat_job_at(tab, blockIdx.x);
     uint32_t* rec = (uint32_t*)job.aux;
-    const uint32_t slots = nv_one_slots(tab, blockIdx.x - job.section, job.pad), sections = (uint32_t)(job.pad * kSectionWords);
+    const uint32_t slots = nv_one_slots(tab, job, blockIdx.x).all, sections = (uint32_t)(job.pad * kSectionWords);
     for (uint32_t word = job.section * kSectionWords + threadIdx.x; word < sections || word < slots; word += sections) rec[word] = 0;
     if (job.section == 0 && threadIdx.x < kOneWords) rec[kRecOne + threadIdx.x * kOneStride] = 0;
 }
@@ -927,11 +939,8 @@ __device__ __forceinline__ uint32_t nv_one_max(uint32_t m, const int t) {
     return (uint32_t)__builtin_amdgcn_readfirstlane((int)m);
 }
 // What this lane sees of a record's slots, two at a time, as soon as they are all written; `late` if that took more than
-// `polls` looks.  row: of the record's first tensor.
-template <class Table>
-__device__ __forceinline__ uint32_t nv_one_collect(const Table& tab, const uint32_t row, const uint32_t* rec, const int tensors_of_it, const int t,
-                                                   const int polls, bool& late) {
-    const uint32_t slots = nv_one_slots(tab, row, tensors_of_it);
+// `polls` looks.
+__device__ __forceinline__ uint32_t nv_one_collect(const uint32_t* rec, const uint32_t slots, const int t, const int polls, bool& late) {
     uint32_t m = 0;
     for (uint32_t slot = t; slot < slots; slot += 2 * kOneThreads) {
         const uint32_t* other = rec + (slot + kOneThreads < slots ? slot + kOneThreads : slot);
@@ -988,17 +997,14 @@ __device__ __forceinline__ bool nv_one_leaves(const uint32_t m, const NvScales& 
 // when every workgroup of the tensors has, most of which are done, and of a record that is done there is its word to read.
 // Of a record whose first workgroup has given up every worker folds the slots.
 template <int FOS, int F16, class Table>
-__device__ __forceinline__ void nv_one_rest(const Table& tab, const uint32_t tensors, const uint32_t workers, const int patience, const int t, float numer,
-                                            uint32_t* moved_counter) {
-    const uint32_t id = (blockIdx.y - tensors) * gridDim.x + blockIdx.x, worker = id / tensors, row = id - worker * tensors;
-    if (worker >= workers) return;
-    const FlatJob job = flat_job_at(tab, row);
+__device__ __forceinline__ void nv_one_rest(const Table& tab, const FlatJob& job, const uint32_t row, const uint32_t worker,
+                                            const uint32_t workers, const int patience, const int t, float numer, uint32_t* moved_counter) {
     uint32_t* rec = (uint32_t*)job.aux;
-    const uint32_t got = nv_one_watch(rec + kRecOne + (id % kOneWords) * kOneStride, t, patience);
+    const uint32_t got = nv_one_watch(rec + kRecOne + ((row + worker) % kOneWords) * kOneStride, t, patience);
     const bool gave_up = got == kOneGaveUp;
     uint32_t m = got & 0x7FFFu;
     bool late = got == 0;
-    if (gave_up) m = nv_one_max<1>(nv_one_collect(tab, row - job.section, rec, job.pad, t, patience, late), t);
+    if (gave_up) m = nv_one_max<1>(nv_one_collect(rec, nv_one_slots(tab, job, row).all, t, patience, late), t);
     if (__syncthreads_or(late)) m = nv_one_scan(tab, row - job.section, job.pad, t);
     const float amax = elem_lo<F16>(m);
     const NvAmaxScales a{amax, nv_scales(amax, numer)};
@@ -1087,11 +1093,24 @@ template <int FOS, int F16, class Table>
 __global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_kernel(const Table tab, float numer, int first_polls, int patience, uint32_t tensors,
                                                                                        uint32_t workers, uint32_t* moved_counter, uint32_t* moved_mirror) {
     const int t = threadIdx.x;
-    if (blockIdx.y >= tensors) {
-        nv_one_rest<FOS, F16>(tab, tensors, workers, patience, t, numer, moved_counter);
+    const bool behind = blockIdx.y >= tensors;
+    uint32_t row = blockIdx.y, worker = 0;
+    if (behind) {
+        const uint32_t id = (blockIdx.y - tensors) * gridDim.x + blockIdx.x;
+        worker = id / tensors;
+        row = id - worker * tensors;
+    }
+    // A descriptor of a device table is read before the branch: below one with stores the compiler takes its values to vector
+    // registers, and with them sixteen addresses of each lane; three of the sixteen loads then waited for the others
+    // (96 x [2048, 7168] 695 us, now 620; 200 x [768, 2048] 142 and now 132).
+    constexpr bool kRef = std::is_same<Table, FlatRef>::value;
+    FlatJob job;
+    if (kRef || !behind) job = flat_job_at(tab, row);
+    if (behind) {
+        if (!kRef) job = flat_job_at(tab, row);
+        if (worker < workers) nv_one_rest<FOS, F16>(tab, job, row, worker, workers, patience, t, numer, moved_counter);
         return;
     }
-    const FlatJob job = flat_job(tab);
     const int64_t block = flat_block(tab), base = block * kOnePerBlock;
     if (base >= job.units) return;
     const int64_t left = job.units - base;
@@ -1109,6 +1128,12 @@ __global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_
             v[i] = ld16(w0 + (off < rem ? off : (off & 1u)) * 8u);      // a lane past the end reads the first block again
         }
     }
+    // Every load before the first use, else the last one waits for most of the others, and the slots meanwhile (us, 32 x [2048, 7168] with
+    // Four Over Six 277 and 269, over a device table 96 of them 626 and 620; but standard blocks over kernel arguments 210 and 213).
+    constexpr bool kEarly = FOS != 0 || kRef;
+    const NvOneSlots early = kEarly ? nv_one_slots(tab, job, row) : NvOneSlots{};
+    auto slots = [&] { return kEarly ? early : nv_one_slots(tab, job, row); };
+    if constexpr (kEarly) __builtin_amdgcn_sched_barrier(0);
     // the block maxima, two to a register: what does not depend on the amax is done before the wait for it
     __shared__ u32x4 stage[FOS ? 2 * kOneThreads : 1];
     uint32_t maxima[kOneUnits / 2], m2 = 0;
@@ -1127,12 +1152,12 @@ __global__ __launch_bounds__(kOneThreads, kOneWavesPerSimd) void nvfp4_one_pass_
     }
     uint32_t m = nv_one_max<0>(hmax_u16(m2), t);
     uint32_t* rec = (uint32_t*)job.aux;
-    if (t == 0) agent_store(rec + nv_one_slots(tab, blockIdx.y - job.section, job.section) + block, kOneFull | m);
+    if (t == 0) agent_store(rec + slots().first + block, kOneFull | m);
     const bool first = block == 0 && job.section == 0;
     if (first) {
         // the record's first workgroup waits for every other one
         bool late = false;
-        m = nv_one_max<1>(nv_one_collect(tab, blockIdx.y, rec, job.pad, t, first_polls, late), t);
+        m = nv_one_max<1>(nv_one_collect(rec, slots().all, t, first_polls, late), t);
         const bool gave_up = __syncthreads_or(late);
         if (t < kOneWords) agent_store(rec + kRecOne + t * kOneStride, gave_up ? kOneGaveUp : kOneFull | m);
         if (blockIdx.y == 0) amax_feedback_folded(moved_counter, moved_mirror, tensors);
@@ -1590,13 +1615,15 @@ int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, in
 // have to be on the chip together, and the records behind it should be loading meanwhile: half of what fits (640 workgroups,
 // 40 MB, on 256 CUs).  A pair of [2048, 7168] weights, 896 workgroups, gained less (313 -> 265 us for 16 pairs) and is one
 // busy neighbour away from waiting in vain, so it keeps two passes.  Short lists keep them as well: they find their second
-// read in the memory-side cache, and the launch that clears the slots takes what is left of the gain (us, two passes / one): 4 x
-// [256, 1024] (2 MB) 6.5 / 8.8, 2 x [1024, 2048] 8.3 / 9.9, 4 of them (17 MB) 10.8 / 11.3, 1 x [2048, 4096] (17 MB) 11.5 / 11.1,
-// 4 x [1537, 2064] (25 MB) 14.2 / 13.3, 1 x [2048, 7168] (29 MB) 16.3 / 13.9, 8 x [1024, 2048] (34 MB) 16.2 / 14.8, 2 x [2048, 7168] (59 MB)
-// 24.0 / 19.0.  With Four Over Six the arithmetic of the first two tensors' loads and the last one's arithmetic have nothing beside them,
-// and a list pays from 170 to 230 MB on, the more workgroups its tensors have the later: 33 x [528, 3088] (108 MB) 44 / 48, 24 x [1536, 2048]
-// (151 MB) 59.5 / 57.3, 45 x [740, 1952] (130 MB) 53.4 / 54.3, 60 of them 68.2 / 65.6, 5 x [4096, 4096] (168 MB) 64.5 / 66.4, 6 x [2048, 7168] (176 MB)
-// 68.6 / 67.4, 8 of them 88.2 / 83.9, 7 x [4096, 4096] (235 MB) 88.0 / 87.1, 38 x [1536, 2048] (239 MB) 90.8 / 80.4.
+// read in the memory-side cache, and the launch that clears the slots takes what is left of the gain (us, two passes / one, runs of
+// one side differ by 0.1): 4 x [256, 1024] (2 MB) 6.3 / 8.7, 2 x [1024, 2048] 8.1 / 9.3, 4 of them (17 MB) 10.5 / 10.4, 1 x [2048, 4096] (17 MB)
+// 11.3 / 10.5, 4 x [1537, 2064] (25 MB) 13.8 / 12.2, 1 x [2048, 7168] (29 MB) 16.3 / 12.8, 8 x [1024, 2048] (34 MB) 16.0 / 14.0, 2 x [2048, 7168]
+// (59 MB) 23.8 / 18.1.  With Four Over Six the first two tensors' loads and the last one's arithmetic have nothing beside them,
+// and what a list gains depends on its tensors and its values (blocks too close to call are looked at again): with slots that had to be
+// cleared again, 33 x [528, 3088] (108 MB) 44 / 48, 45 x [740, 1952] (130 MB) 53.4 / 54.3, 24 x [1536, 2048]
+// (151 MB) 59.5 / 57.3, 5 x [4096, 4096] (168 MB) 64.5 / 66.4, 6 x [2048, 7168] (176 MB) 68.6 / 67.4, 7 x [4096, 4096] (235 MB) 88.0 / 87.1, 38 x [1536,
+// 2048] (239 MB) 90.8 / 80.4; weights N(0, 0.02^2) with the slots as they are 44.5 / 44.0, 51.5 / 49.4, 57.9 / 52.2, 62.3 / 61.6, 66.3 / 63.2, 85.3 / 80.3,
+// 88.5 / 72.7.  From 200 MiB on it is ahead for all of them.
 constexpr int64_t kOneMinBytes = 24ll << 20, kOneFosMinBytes = 200ll << 20;
 bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes, int flags) {
     int device = 0, cus = 0;
