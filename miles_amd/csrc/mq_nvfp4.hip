@@ -843,7 +843,7 @@ __global__ __launch_bounds__(kNvThreads) void nvfp4_quant_bf16_kernel(const Tabl
 // call are taken up again behind the others, in a loop with the one copy of the exact sums, which reads them again.  32 x
 // [2048, 7168]: 342 us in two passes, 298 this way, 48 x [1536, 2048] 111 and 95 (four workgroups per CU without the spills 319 and
 // 103; regrouped by lane exchange after the wait 308 and 100; the next block's table lookups ahead of this block's sums 309 and
-// 101).  Bound by the two hundred vector instructions of a block, which all workgroups of a tensor run at the same time: they
+// 101); of weights N(0, 0.02^2), with all loads first, 318 and 273, 105 and 86.  Bound by the two hundred vector instructions of a block, which all workgroups of a tensor run at the same time: they
 // overlap with the loads of the next two tensors, half as well as in the second of two passes.
 constexpr int kOneThreads = 256, kOneUnits = 16, kOneWavesPerSimd = 5;
 constexpr int64_t kOnePerBlock = kOneThreads * kOneUnits;
@@ -1616,14 +1616,14 @@ int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, in
 // 40 MB, on 256 CUs).  A pair of [2048, 7168] weights, 896 workgroups, gained less (313 -> 265 us for 16 pairs) and is one
 // busy neighbour away from waiting in vain, so it keeps two passes.  Short lists keep them as well: they find their second
 // read in the memory-side cache, and the launch that clears the slots takes what is left of the gain (us, two passes / one, runs of
-// one side differ by 0.1): 4 x [256, 1024] (2 MB) 6.3 / 8.7, 2 x [1024, 2048] 8.1 / 9.3, 4 of them (17 MB) 10.5 / 10.4, 1 x [2048, 4096] (17 MB)
-// 11.3 / 10.5, 4 x [1537, 2064] (25 MB) 13.8 / 12.2, 1 x [2048, 7168] (29 MB) 16.3 / 12.8, 8 x [1024, 2048] (34 MB) 16.0 / 14.0, 2 x [2048, 7168]
-// (59 MB) 23.8 / 18.1.  With Four Over Six the first two tensors' loads and the last one's arithmetic have nothing beside them,
+// one side differ by 0.1): 4 x [256, 1024] (2 MB) 6.4 / 8.9, 2 x [1024, 2048] 8.1 / 9.5, 4 of them (17 MB) 10.5 / 10.6, 1 x [2048, 4096] (17 MB)
+// 11.3 / 10.7, 4 x [1537, 2064] (25 MB) 13.9 / 12.2, 1 x [2048, 7168] (29 MB) 16.2 / 13.0, 8 x [1024, 2048] (34 MB) 16.1 / 14.0, 2 x [2048, 7168]
+// (59 MB) 23.8 / 18.3.  With Four Over Six the first two tensors' loads and the last one's arithmetic have nothing beside them,
 // and what a list gains depends on its tensors and its values (blocks too close to call are looked at again): with slots that had to be
 // cleared again, 33 x [528, 3088] (108 MB) 44 / 48, 45 x [740, 1952] (130 MB) 53.4 / 54.3, 24 x [1536, 2048]
 // (151 MB) 59.5 / 57.3, 5 x [4096, 4096] (168 MB) 64.5 / 66.4, 6 x [2048, 7168] (176 MB) 68.6 / 67.4, 7 x [4096, 4096] (235 MB) 88.0 / 87.1, 38 x [1536,
-// 2048] (239 MB) 90.8 / 80.4; weights N(0, 0.02^2) with the slots as they are 44.5 / 44.0, 51.5 / 49.4, 57.9 / 52.2, 62.3 / 61.6, 66.3 / 63.2, 85.3 / 80.3,
-// 88.5 / 72.7.  From 200 MiB on it is ahead for all of them.
+// 2048] (239 MB) 90.8 / 80.4; weights N(0, 0.02^2) with the slots as they are 44.8 / 44.0, 52.3 / 49.7, 58.1 / 52.8, 62.3 / 63.3, 66.4 / 63.7, 85.3 / 81.0,
+// 88.5 / 72.8.  From 200 MiB on it is ahead for all of them.
 constexpr int64_t kOneMinBytes = 24ll << 20, kOneFosMinBytes = 200ll << 20;
 bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes, int flags) {
     int device = 0, cus = 0;
