@@ -301,7 +301,8 @@ int mq_nvfp4_fake_quant(const mq_fake_quant_item* list, int64_t n, int dtype, vo
  * collects its amax and the second pass quantizes it (what the plain two-pass form costs), and it returns to the
  * single pass once its amax has stayed the same for one submission.
  * Without that flag, bf16 or fp16 tensors are read once as well when the tensors of a grouped launch are 24 MiB and more
- * (200 MiB with MQ_NVFP4_4OVER6, and not with MQ_NVFP4_ERR_FP16) and every record's tensors fit the chip's registers twice (640 workgroups of 64 KiB, 40 MB, on
+ * (and 384 KiB each on average, from 48 MiB on 320 KiB, from 64 MiB on any; 200 MiB with MQ_NVFP4_4OVER6, and not with
+ * MQ_NVFP4_ERR_FP16) and every record's tensors fit the chip's registers twice (640 workgroups of 64 KiB, 40 MB, on
  * 256 CUs; a single tensor 32 MB at most).  A grouped launch holds MQ_MAX_GROUP tensors, or with a device table
  * MQ_TABLE_GROUP.  The workgroups of a record keep their share and wait for each other's maxima, for a bounded time, after
  * which workgroups behind them in the same launch do what is left.  MQ_NVFP4_NO_WAIT in p1: a record's first workgroup, which

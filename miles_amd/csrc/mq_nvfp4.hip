@@ -1624,12 +1624,20 @@ int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, in
 // (151 MB) 59.5 / 57.3, 5 x [4096, 4096] (168 MB) 64.5 / 66.4, 6 x [2048, 7168] (176 MB) 68.6 / 67.4, 7 x [4096, 4096] (235 MB) 88.0 / 87.1, 38 x [1536,
 // 2048] (239 MB) 90.8 / 80.4; weights N(0, 0.02^2) with the slots as they are 44.8 / 44.0, 52.3 / 49.7, 58.1 / 52.8, 62.3 / 63.3, 66.4 / 63.7, 85.3 / 81.0,
 // 88.5 / 72.8.  From 200 MiB on it is ahead for all of them.
+// A list of many small tensors (over a device table; 64 tensors of 24 MiB have 384 KiB each) has a grid row and a wait for each, and two
+// passes have neither: us, two / one, 24 MiB in tensors of 64 KiB 13.9 / 34.2, of 256 KiB 13.3 / 15.9, of 320 KiB 13.2 / 14.7; 32 MiB of
+// 320 KiB 16.1 / 17.7, of 384 KiB 15.7 / 15.4; 50 MiB of 264 KiB 23.7 / 25.0, of 330 KiB 23.1 / 22.0; 64 MiB of 192 KiB 27.7 / 34.4, of 320 KiB
+// 27.4 / 26.4.  Lists of 64 MiB and more are read once whatever their tensors are, though two passes would be faster below 256 KiB a
+// tensor (400 MiB of 64 KiB 159 / 474, of 192 KiB 149 / 187, of 256 KiB 149 / 145).
 constexpr int64_t kOneMinBytes = 24ll << 20, kOneFosMinBytes = 200ll << 20;
-bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes, int flags) {
+constexpr int64_t kOneAnyTensors = 64ll << 20;
+static int64_t one_min_tensor(int64_t bytes) { return bytes >= kOneAnyTensors ? 0 : bytes >= (48ll << 20) ? 320 << 10 : 384 << 10; }
+// n: tensors of the chunk
+bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes, int64_t n, int flags) {
     int device = 0, cus = 0;
     const bool fos = (flags & MQ_NVFP4_4OVER6) != 0;
     if (fos && nv_error_mode(flags) > 1) return false;       // (an error in fp16 has no estimate)
-    if (bytes < (fos ? kOneFosMinBytes : kOneMinBytes) || max_units > kOneSlots * kOnePerBlock) return false;
+    if (bytes < (fos ? kOneFosMinBytes : kOneMinBytes) || max_units > kOneSlots * kOnePerBlock || bytes < n * one_min_tensor(bytes)) return false;
     if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
         (void)hipGetLastError();
         return false;

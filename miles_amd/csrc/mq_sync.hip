@@ -36,7 +36,7 @@ int mq_int4_pack_launch_group(int dtype, FlatTable& tab, int group, const RiderA
 bool mq_nvfp4_fast_ok(const void* w, int dtype, const void* q);
 int mq_nvfp4_amax_launch_group(int dtype, FlatTable& tab, hipStream_t st);
 int mq_nvfp4_quant_launch_group(int dtype, FlatTable& tab, int e4m3_max, int flags, int mode, hipStream_t st);
-bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes, int flags);
+bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes, int64_t n, int flags);
 int64_t mq_nvfp4_one_pass_slots(int64_t units);
 int mq_nvfp4_one_pass_launch_group(int dtype, FlatTable& tab, int64_t max_units, int e4m3_max, int flags, hipStream_t st);
 int mq_nvfp4_one_pass_launch_table(int dtype, const FlatJob* device_jobs, int n, int64_t max_units, int e4m3_max, int flags,
@@ -577,7 +577,7 @@ static int run_nvfp4(const mq_job* jobs, int64_t n_all, int64_t i, int64_t j, co
                 slots = (section[t] == 0 ? 0 : slots) + mq_nvfp4_one_pass_slots(u);
                 max_slots = slots > max_slots ? slots : max_slots;
             }
-            const bool one_pass = !carry && !empty && jobs[i].dtype != MQ_F32 && mq_nvfp4_one_pass_ok(max_units, max_slots, sum_units * 16, jobs[i].p1);
+            const bool one_pass = !carry && !empty && jobs[i].dtype != MQ_F32 && mq_nvfp4_one_pass_ok(max_units, max_slots, sum_units * 16, n, jobs[i].p1);
             if (from_table) {
                 if (one_pass) {
                     rc = mq_nvfp4_one_pass_launch_table(jobs[i].dtype, table + i, n, max_units, jobs[i].p0, jobs[i].p1, st);

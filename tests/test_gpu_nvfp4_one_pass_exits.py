@@ -83,3 +83,26 @@ def test_two_streams_at_once():
                     assert torch.equal(a.reshape(-1).view(torch.uint8), b.reshape(-1).view(torch.uint8))
                     a.reshape(-1).view(torch.uint8).fill_(0xA5)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("n, kib, one_pass", [
+    (66, 383, False), (66, 384, True),              # 24 MiB and more: 384 KiB a tensor
+    (127, 383, False), (128, 384, True),            # around 48 MiB
+    (160, 319, False), (160, 320, True),            # from 48 MiB on 320 KiB
+    (800, 64, False), (1024, 64, True),             # from 64 MiB on any
+])
+@pytest.mark.parametrize("pairs", [False, True])
+def test_lists_of_small_tensors(n, kib, one_pass, pairs):
+    """Over a device table: two passes for lists of many small tensors."""
+    if pairs and n % 2:
+        n += 1
+    x = _tensors(n, kib, 512)
+    x[n - 1][kib - 1, 511] = 3.0
+    got, words, redo = _run(x, pairs)
+    assert (((words & PUBLISHED) != 0) if one_pass else (words == 0)).all()
+    assert (redo == 0).all()
+    for i in (0, 2, n // 2 & ~1, n - 2):
+        want = nvfp4_quantize_1d_pair(x[i], x[i + 1]) if pairs else [nvfp4_quantize_1d(x[i]), nvfp4_quantize_1d(x[i + 1])]
+        for one, ref in zip(got[i:i + 2], want):
+            for a, b in zip(one, ref):
+                assert torch.equal(a.reshape(-1).view(torch.uint8), b.reshape(-1).view(torch.uint8))
