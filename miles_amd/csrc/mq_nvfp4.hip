@@ -1625,10 +1625,10 @@ int mq_nvfp4_quant_launch_table(int dtype, const FlatJob* device_jobs, int n, in
 // 2048] (239 MB) 90.8 / 80.4; weights N(0, 0.02^2) with the slots as they are 44.8 / 44.0, 52.3 / 49.7, 58.1 / 52.8, 62.3 / 63.3, 66.4 / 63.7, 85.3 / 81.0,
 // 88.5 / 72.8.  From 200 MiB on it is ahead for all of them.
 // A list of many small tensors (over a device table; 64 tensors of 24 MiB have 384 KiB each) has a grid row and a wait for each, and two
-// passes have neither: us, two / one, 24 MiB in tensors of 64 KiB 13.9 / 34.2, of 256 KiB 13.3 / 15.9, of 320 KiB 13.2 / 14.7; 32 MiB of
-// 320 KiB 16.1 / 17.7, of 384 KiB 15.7 / 15.4; 50 MiB of 264 KiB 23.7 / 25.0, of 330 KiB 23.1 / 22.0; 64 MiB of 192 KiB 27.7 / 34.4, of 320 KiB
-// 27.4 / 26.4.  Lists of 64 MiB and more are read once whatever their tensors are, though two passes would be faster below 256 KiB a
-// tensor (400 MiB of 64 KiB 159 / 474, of 192 KiB 149 / 187, of 256 KiB 149 / 145).
+// passes have neither: us, two / one, 24 MiB in tensors of 64 KiB 13.8 / 34.1, of 256 KiB 13.3 / 15.9, of 320 KiB 13.3 / 14.7; 32 MiB of
+// 320 KiB 16.1 / 17.7, of 384 KiB 15.7 / 15.4; 50 MiB of 264 KiB 23.7 / 25.0, of 330 KiB 23.1 / 21.9; 64 MiB of 192 KiB 27.6 / 33.0, of 320 KiB
+// 27.5 / 26.3.  Lists of 64 MiB and more are read once whatever their tensors are, though two passes would be faster up to 192 KiB a
+// tensor (400 MiB of 64 KiB 160 / 435, of 192 KiB 149 / 162, of 256 KiB 149 / 130).
 constexpr int64_t kOneMinBytes = 24ll << 20, kOneFosMinBytes = 200ll << 20;
 constexpr int64_t kOneAnyTensors = 64ll << 20;
 static int64_t one_min_tensor(int64_t bytes) { return bytes >= kOneAnyTensors ? 0 : bytes >= (48ll << 20) ? 320 << 10 : 384 << 10; }
@@ -1647,12 +1647,15 @@ bool mq_nvfp4_one_pass_ok(int64_t max_units, int64_t slots, int64_t bytes, int64
 int64_t mq_nvfp4_one_pass_slots(int64_t units) { return (units + kOnePerBlock - 1) / kOnePerBlock; }
 
 // workgroups behind the tensors' own, for each of n tensors of at most max_units: 64 of a list of 32 tensors (the launch has
-// 0.4 ns for one that finds nothing to do), and enough to fill half of the chip for one that is left
-constexpr int kOneWorkers = 2048;
+// 0.4 ns for one that finds nothing to do), and enough to fill half of the chip for one that is left.  A list of more than 128 has 16 for
+// each, or one for eight pieces of a smaller tensor: with 16, or one for each piece, 6400 x 64 KiB took 473 us, now 435, 2133 x 192 KiB 184 and 160,
+// 1066 x 384 KiB 112 and 103 (452, 177 and 122 before there were any); all tensors left, 1600 x 256 KiB 180 and 162, 204 x 640 KiB 48.2 and 49.3.
+constexpr int kOneWorkers = 2048, kOneFewest = 16, kOnePieces = 8;
 static uint32_t nv_one_workers(int n, int64_t max_units, int fos) {
     const int64_t blocks = (max_units + nv_units_per_block(fos) - 1) / nv_units_per_block(fos);
+    const int64_t few = (blocks + kOnePieces - 1) / kOnePieces, fewest = few < kOneFewest ? few : kOneFewest;
     int64_t workers = kOneWorkers / n;
-    workers = workers < 16 ? 16 : workers > kSectionWords ? kSectionWords : workers;
+    workers = workers < fewest ? fewest : workers > kSectionWords ? kSectionWords : workers;
     return (uint32_t)(workers < blocks ? workers : blocks);
 }
 // descriptors as for mode 1

@@ -106,3 +106,15 @@ def test_lists_of_small_tensors(n, kib, one_pass, pairs):
         for one, ref in zip(got[i:i + 2], want):
             for a, b in zip(one, ref):
                 assert torch.equal(a.reshape(-1).view(torch.uint8), b.reshape(-1).view(torch.uint8))
+
+
+@pytest.mark.parametrize("n, rows, cols", [(1100, 4, 8192), (1100, 2, 16400), (140, 60, 8192), (140, 5, 98320)])
+def test_few_workgroups_behind_small_tensors(n, rows, cols):
+    """One, two, 15 and 16 of them behind each tensor, whose last piece is whole or of a few blocks: they quantize the tensors whose
+    first workgroup gave up (a tensor of one workgroup has nothing to wait for)."""
+    x = _tensors(n, rows, cols)
+    got, words, redo = _run(x, False, _lib.NVFP4_NO_WAIT)
+    assert (words != 0).all()
+    for i in range(0, n, 7):
+        for a, b in zip(got[i], nvfp4_quantize_1d(x[i])):
+            assert torch.equal(a.reshape(-1).view(torch.uint8), b.reshape(-1).view(torch.uint8))
