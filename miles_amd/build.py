@@ -1,5 +1,6 @@
 """Builds libmiles_quant.so (the C-ABI HIP library) and libmq_probes.so (self-tests and streaming probes that only
-the GPU tests and bench.py load; not part of the product) for gfx950 with hipcc, in-tree.
+the GPU tests and bench.py load; not part of the product; linked to the product library, one of whose kernels a probe runs with
+limits of its own for its waits) for gfx950 with hipcc, in-tree.
 
     python -m miles_amd.build
 
